@@ -213,7 +213,7 @@ def dominant_kernel_traffic():
     m_hash = re.search(r"gemm_source_sha256:\s*([0-9a-f]{64})", text)
     if not m_bytes or not m_hash:
         return None
-    src = os.path.join(ROOT, "flexflow-train_amd", "csrc", "gemm.hip")
+    src = os.path.join(ROOT, "flexflow-train_amd", "csrc", "gemm_bf16.h")
     if hashlib.sha256(open(src, "rb").read()).hexdigest() != m_hash.group(1):
         return None
     return int(m_bytes.group(1))
