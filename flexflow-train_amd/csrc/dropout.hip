@@ -39,7 +39,8 @@ __global__ __launch_bounds__(kDropThreads) void dropout_vec_kernel(
   constexpr int V = VecIO<T>::kVec;
   int64_t const nvec = n / V;
   int64_t const stride = (int64_t)gridDim.x * kDropThreads;
-  for (int64_t i = (int64_t)blockIdx.x * kDropThreads + threadIdx.x; i < nvec; i += stride) {
+  int64_t i = (int64_t)blockIdx.x * kDropThreads + threadIdx.x;
+  for (; i < nvec; i += stride) {
     float x[V], y[V], aux[V];
     if (MODE == kDropPlain || MODE == kDropAfterGelu) {
       VecIO<T>::load(X + i * V, x);
@@ -69,14 +70,25 @@ __global__ __launch_bounds__(kDropThreads) void dropout_vec_kernel(
     }
     VecIO<T>::store(Y + i * V, y);
   }
+  // the last n % V elements, by the one thread whose vector would begin with them (a launch of
+  // their own is 3 us)
+  if (MODE == kDropPlain && i == nvec && n % V != 0) {
+    uint32_t w[4];
+    philox4x32_10((p.offset + (uint64_t)i * V) >> 3, p.key, w);
+    for (int64_t t = i * V; t < n; t++) {
+      float v = keep_dynamic(w, (uint32_t)((p.offset + (uint64_t)t) & 7), p) ? VecIO<T>::load1(X + t) * p.scale : 0.0f;
+      if (ACC) v += VecIO<T>::load1(Y + t);
+      VecIO<T>::store1(Y + t, v);
+    }
+  }
 }
 
-// Any offset / alignment / tail: one element per thread.
+// Any offset and alignment: one element per thread.
 template <typename T, bool ACC>
 __global__ __launch_bounds__(kDropThreads) void dropout_scalar_kernel(
-    T const *__restrict__ X, T *Y, int64_t first, int64_t n, DropoutParams p) {
+    T const *__restrict__ X, T *Y, int64_t n, DropoutParams p) {
   int64_t const stride = (int64_t)gridDim.x * kDropThreads;
-  for (int64_t i = first + (int64_t)blockIdx.x * kDropThreads + threadIdx.x; i < n; i += stride) {
+  for (int64_t i = (int64_t)blockIdx.x * kDropThreads + threadIdx.x; i < n; i += stride) {
     uint64_t const e = p.offset + (uint64_t)i;
     uint32_t w[4];
     philox4x32_10(e >> 3, p.key, w);
@@ -110,17 +122,12 @@ static int dropout_run(hipStream_t st, void const *x, void *y, int64_t n,
   constexpr int V = VecIO<T>::kVec;
   T const *X = static_cast<T const *>(x);
   T *Y = static_cast<T *>(y);
-  int64_t done = 0;
-  if ((p.offset & 7) == 0 && aligned16(x) && aligned16(y) && n >= V) {
-    int64_t nvec = n / V;
-    dropout_vec_kernel<T, ACC, kDropPlain><<<grid_for(nvec), kDropThreads, 0, st>>>(X, nullptr, Y, n, p);
-    FFK_CHECK_LAUNCH();
-    done = nvec * V;
+  if ((p.offset & 7) == 0 && aligned16(x) && aligned16(y)) {
+    dropout_vec_kernel<T, ACC, kDropPlain><<<grid_for(ceil_div(n, V)), kDropThreads, 0, st>>>(X, nullptr, Y, n, p);
+  } else {
+    dropout_scalar_kernel<T, ACC><<<grid_for(n), kDropThreads, 0, st>>>(X, Y, n, p);
   }
-  if (done < n) {
-    dropout_scalar_kernel<T, ACC><<<grid_for(n - done), kDropThreads, 0, st>>>(X, Y, done, n, p);
-    FFK_CHECK_LAUNCH();
-  }
+  FFK_CHECK_LAUNCH();
   return FFK_OK;
 }
 

@@ -157,6 +157,47 @@ struct VecIO<bf16> {
   }
 };
 
+// Accesses to rows of any length, whose elements are only known to be aligned to themselves.  The
+// vector memory unit takes 16 bytes from any such address; the packed types tell the compiler to
+// use that.
+template <typename T>
+struct __attribute__((packed, aligned(sizeof(T)))) AnyRaw16 { u32x4 v; };
+template <typename T>
+__device__ __forceinline__ u32x4 load_raw_any(T const *p) { return reinterpret_cast<AnyRaw16<T> const *>(p)->v; }
+template <typename T>
+__device__ __forceinline__ void store_raw_any(T *p, u32x4 v) { reinterpret_cast<AnyRaw16<T> *>(p)->v = v; }
+// The first n elements (fewer than 16 bytes of them), the others as zeros / left alone.
+__device__ __forceinline__ u32x4 load_raw_first(bf16 const *p, int n) {
+  uint16_t const *h = reinterpret_cast<uint16_t const *>(p);
+  u32x4 v = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int e = 0; e < 7; e++) {
+    if (e < n) v[e >> 1] |= (uint32_t)h[e] << (16 * (e & 1));
+  }
+  return v;
+}
+__device__ __forceinline__ u32x4 load_raw_first(float const *p, int n) {
+  u32x4 v = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int e = 0; e < 3; e++) {
+    if (e < n) v[e] = __float_as_uint(p[e]);
+  }
+  return v;
+}
+__device__ __forceinline__ void store_raw_first(bf16 *p, u32x4 v, int n) {
+  uint16_t *h = reinterpret_cast<uint16_t *>(p);
+#pragma unroll
+  for (int e = 0; e < 7; e++) {
+    if (e < n) h[e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+  }
+}
+__device__ __forceinline__ void store_raw_first(float *p, u32x4 v, int n) {
+#pragma unroll
+  for (int e = 0; e < 3; e++) {
+    if (e < n) p[e] = __uint_as_float(v[e]);
+  }
+}
+
 // Raw 16-byte streaming load, unpacked later: lets a kernel issue the loads of
 // its next row before it works on the current one.
 __device__ __forceinline__ u32x4 load_raw_stream(void const *p) {
@@ -173,6 +214,46 @@ __device__ __forceinline__ void unpack_raw(u32x4 r, float (&v)[8], bf16 const *)
     v[2 * i + 1] = __uint_as_float(r[i] & 0xffff0000u);
   }
 }
+__device__ __forceinline__ u32x4 pack_raw(float const (&v)[4], float const *) {
+  return u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
+}
+__device__ __forceinline__ u32x4 pack_raw(float const (&v)[8], bf16 const *) {
+  return u32x4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
+}
+
+// Vector v (kVec elements from v * kVec on) of a row of N elements, in the two kinds of rows there
+// are: whole aligned vectors, or (ANY) any N at any address, where the last vector may be partial:
+// its missing elements are read as zeros and not stored.
+template <typename T, bool ANY>
+struct RowVec {
+  static constexpr int V = VecIO<T>::kVec;
+  __host__ __device__ static __forceinline__ int count(int N) { return ANY ? (N + V - 1) / V : N / V; }
+  // how many of vector v's elements exist
+  __device__ static __forceinline__ int elems(int v, int N) { return ANY ? min(V, N - v * V) : V; }
+  __device__ static __forceinline__ u32x4 load_raw(T const *row, int v, int N, bool stream) {
+    T const *p = row + (int64_t)v * V;
+    if constexpr (ANY) return elems(v, N) == V ? load_raw_any(p) : load_raw_first(p, elems(v, N));
+    return stream ? __builtin_nontemporal_load(reinterpret_cast<u32x4 const *>(p)) : *reinterpret_cast<u32x4 const *>(p);
+  }
+  __device__ static __forceinline__ void load(T const *row, int v, int N, float (&x)[V], bool stream = false) {
+    unpack_raw(load_raw(row, v, N, stream), x, (T const *)nullptr);
+  }
+  __device__ static __forceinline__ void store(T *row, int v, int N, float const (&x)[V], bool stream = false) {
+    T *p = row + (int64_t)v * V;
+    u32x4 const r = pack_raw(x, (T const *)nullptr);
+    if constexpr (ANY) {
+      if (elems(v, N) == V) {
+        store_raw_any(p, r);
+      } else {
+        store_raw_first(p, r, elems(v, N));
+      }
+    } else if (stream) {
+      __builtin_nontemporal_store(r, reinterpret_cast<u32x4 *>(p));
+    } else {
+      *reinterpret_cast<u32x4 *>(p) = r;
+    }
+  }
+};
 
 // ---- GELU (exact erf form) shared by ElementUnary and the GEMM epilogue ----
 // erf by Abramowitz & Stegun 7.1.26 (|error| <= 1.5e-7), sharing exp(-z^2)

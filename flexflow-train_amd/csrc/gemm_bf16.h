@@ -73,33 +73,12 @@ inline char const *tf(bool b) { return b ? "true" : "false"; }
 // ---------------------------------------------------------------------------
 // bf16 MFMA kernel
 // ---------------------------------------------------------------------------
-// Accesses to rows of odd length, whose elements are only known to be 2-byte aligned.  The vector
-// memory unit takes 16 bytes from any address; the packed types tell the compiler to use that.
-struct __attribute__((packed, aligned(2))) Raw16 { u32x4 v; };
+// eight / the first few bytes of a row at any address
 struct __attribute__((packed, aligned(2))) Raw8 { u32x2 v; };
-__device__ __forceinline__ u32x4 load_any(bf16 const *p) { return reinterpret_cast<Raw16 const *>(p)->v; }
 __device__ __forceinline__ u32x2 load_any8(bf16 const *p) { return reinterpret_cast<Raw8 const *>(p)->v; }
-__device__ __forceinline__ void store_any(bf16 *p, u32x4 v) { reinterpret_cast<Raw16 *>(p)->v = v; }
-// the first n (below the vector's length) elements only
-__device__ __forceinline__ u32x4 load_first(bf16 const *p, int n) {
-  uint16_t const *h = reinterpret_cast<uint16_t const *>(p);
-  u32x4 v = {0u, 0u, 0u, 0u};
-#pragma unroll
-  for (int e = 0; e < 7; e++) {
-    if (e < n) v[e >> 1] |= (uint32_t)h[e] << (16 * (e & 1));
-  }
-  return v;
-}
 __device__ __forceinline__ u32x2 load_first4(bf16 const *p, int n) {
-  u32x4 const v = load_first(p, n);
+  u32x4 const v = load_raw_first(p, n);
   return u32x2{v[0], v[1]};
-}
-__device__ __forceinline__ void store_first(bf16 *p, u32x4 v, int n) {
-  uint16_t *h = reinterpret_cast<uint16_t *>(p);
-#pragma unroll
-  for (int e = 0; e < 7; e++) {
-    if (e < n) h[e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
-  }
 }
 
 constexpr int kBK = 64;        // K extent of one LDS tile
@@ -156,8 +135,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_kernel(
 
   // Elements [pos, pos + 8) of a row of `len` elements, those past its end as zeros.
   auto chunk = [](bf16 const *row, int pos, int len) __attribute__((always_inline)) -> u32x4 {
-    if (pos + 8 <= len) return load_any(row + pos);
-    return pos < len ? load_first(row + pos, len - pos) : u32x4{0u, 0u, 0u, 0u};
+    if (pos + 8 <= len) return load_raw_any(row + pos);
+    return pos < len ? load_raw_first(row + pos, len - pos) : u32x4{0u, 0u, 0u, 0u};
   };
   // One operand's next tile.  KC: the reduction index is contiguous; rows past the edge are read
   // from the last one (what they give is not stored).  INNER: the whole tile exists, which is
@@ -171,12 +150,12 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_kernel(
       if constexpr (KC) {
         int const row = c >> 3, k = k0 + (c & 7) * 8;
         bf16 const *const p = X + (int64_t)min(r0 + row, R - 1) * ld;
-        dst[i] = INNER ? load_any(p + k) : chunk(p, k, K);
+        dst[i] = INNER ? load_raw_any(p + k) : chunk(p, k, K);
       } else {
         int const k = k0 + c / (BR / 8), r = r0 + (c % (BR / 8)) * 8;
         bf16 const *const p = X + (int64_t)k * ld;
         if (INNER) {
-          dst[i] = load_any(p + r);
+          dst[i] = load_raw_any(p + r);
         } else {
           dst[i] = k < K ? chunk(p, r, R) : u32x4{0u, 0u, 0u, 0u};
         }
@@ -792,9 +771,9 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
     if constexpr (EDGE) {
       if (m >= M || n >= N) return;
       if (n + 8 <= N) {
-        store_any(to, v);
+        store_raw_any(to, v);
       } else {
-        store_first(to, v, N - n);
+        store_raw_first(to, v, N - n);
       }
     } else {
       *reinterpret_cast<u32x4 *>(to) = v;

@@ -21,7 +21,8 @@ namespace ffk {
 
 // PRE: the row normalised is residual + dropout(X), computed here, rounded to T where the two
 // separate operators would have stored it, and written to `summed` as well.
-template <typename T, int EPT, int WPR, bool PRE = false, bool STREAM = false>
+// ANY: any N, rows at any address (RowVec).
+template <typename T, int EPT, int WPR, bool PRE = false, bool STREAM = false, bool ANY = false>
 __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
     T const *__restrict__ X, T *__restrict__ Y, T const *__restrict__ gamma,
     T const *__restrict__ beta, float *__restrict__ mean,
@@ -29,11 +30,12 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
     T const *__restrict__ residual = nullptr, T *__restrict__ summed = nullptr,
     DropoutParams drop = DropoutParams{}) {
   constexpr int V = VecIO<T>::kVec;
+  using RV = RowVec<T, ANY>;
   constexpr int RPB = 4 / WPR;  // rows per workgroup
   constexpr int LANES = 64 * WPR;
   __shared__ float smem[2][4][2];
   RowReducer<WPR> red(smem);
-  int const nvec = N / V;
+  int const nvec = RV::count(N);
   int const lane = WPR == 1 ? (threadIdx.x & 63) : threadIdx.x;
   int64_t const row = (int64_t)blockIdx.x * RPB + (WPR == 1 ? (threadIdx.x >> 6) : 0);
   bool const row_ok = row < M;
@@ -55,8 +57,8 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
       b[j][e] = 0.0f;
     }
     if (v < nvec) {
-      if (gamma != nullptr) VecIO<T>::load(gamma + (int64_t)v * V, g[j]);
-      if (beta != nullptr) VecIO<T>::load(beta + (int64_t)v * V, b[j]);
+      if (gamma != nullptr) RV::load(gamma, v, N, g[j]);
+      if (beta != nullptr) RV::load(beta, v, N, b[j]);
     }
   };
   if constexpr (kEarly) {
@@ -67,11 +69,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
   for (int j = 0; j < EPT; j++) {
     int v = lane + j * LANES;
     if (v < nvec) {
-      if (STREAM) {
-        VecIO<T>::load_stream(xr + (int64_t)v * V, x[j]);
-      } else {
-        VecIO<T>::load(xr + (int64_t)v * V, x[j]);
-      }
+      RV::load(xr, v, N, x[j], STREAM);
       if constexpr (PRE) {
         static_assert(V == 4 || V == 8, "a lane's vector is a Philox block or half of one");
         if (row_ok) {
@@ -110,6 +108,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
 #pragma unroll
       for (int e = 0; e < V; e++) {
         float d = x[j][e] - mu;
+        if (ANY && e >= RV::elems(v, N)) d = 0.0f;
         q += d * d;
       }
     }
@@ -133,16 +132,12 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
         float xh = (x[j][e] - mu) * rs;
         y[e] = xh * g[j][e] + b[j][e];
       }
-      if (STREAM) {
-        VecIO<T>::store_stream(yr + (int64_t)v * V, y);
-      } else {
-        VecIO<T>::store(yr + (int64_t)v * V, y);
-      }
+      RV::store(yr, v, N, y, STREAM);
     }
   }
 }
 
-// Generic forward: any N, one workgroup per row, scalar accesses.
+// Generic forward: rows too long for registers, one workgroup per row, scalar accesses.
 template <typename T>
 __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_generic_kernel(
     T const *__restrict__ X, T *__restrict__ Y, T const *__restrict__ gamma,
@@ -177,7 +172,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_generic_kernel(
 // in registers until the workgroup is done.
 // DROP: dropout_backward(dX as stored) is written to `dropped` as well (the gradient entering
 // a dropout whose output fed the residual sum that this LayerNorm normalised).
-template <typename T, int EPT, int WPR, bool ACC, bool DROP = false>
+template <typename T, int EPT, int WPR, bool ACC, bool DROP = false, bool ANY = false>
 __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
     T const *__restrict__ dY, T const *__restrict__ X,
     float const *__restrict__ mean, float const *__restrict__ rstd,
@@ -190,11 +185,12 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
   // res to the stored gradient would give; without round_first the sum is rounded once, i.e.
   // what dX += gradient gives when dX holds a copy of res.
   constexpr int V = VecIO<T>::kVec;
+  using RV = RowVec<T, ANY>;
   constexpr int RPB = 4 / WPR;
   constexpr int LANES = 64 * WPR;
   __shared__ float smem[2][4][2];
   RowReducer<WPR> red(smem);
-  int const nvec = N / V;
+  int const nvec = RV::count(N);
   int const lane = WPR == 1 ? (threadIdx.x & 63) : threadIdx.x;
   int const sub = WPR == 1 ? (threadIdx.x >> 6) : 0;
   float const inv_n = 1.0f / (float)N;
@@ -210,7 +206,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
       db[j][e] = 0.0f;
     }
     if (gamma != nullptr && v < nvec) {
-      VecIO<T>::load(gamma + (int64_t)v * V, g[j]);
+      RV::load(gamma, v, N, g[j]);
     }
   }
 
@@ -235,8 +231,8 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
       for (int j = 0; j < EPT; j++) {
         int v = lane + j * LANES;
         if (v < nvec) {
-          rx[j] = load_raw_stream(X + r * (int64_t)N + (int64_t)v * V);
-          rdy[j] = load_raw_stream(dY + r * (int64_t)N + (int64_t)v * V);
+          rx[j] = RV::load_raw(X + r * (int64_t)N, v, N, true);
+          rdy[j] = RV::load_raw(dY + r * (int64_t)N, v, N, true);
         }
       }
     } else {
@@ -286,21 +282,15 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
         int v = lane + j * LANES;
         if (v < nvec) {
           float o[V];
-          T *dst = dX + row * (int64_t)N + (int64_t)v * V;
-          if (ACC) {
-            VecIO<T>::load(res != nullptr ? res + row * (int64_t)N + (int64_t)v * V : dst, o);
-          }
+          T *const dst = dX + row * (int64_t)N;
+          if (ACC) RV::load((res != nullptr ? res : dX) + row * (int64_t)N, v, N, o);
 #pragma unroll
           for (int e = 0; e < V; e++) {
             float val = fmaf(dy[j][e], rs, fmaf(x[j][e], c1, c0));
             if (ACC && res != nullptr && round_first) val = storage_round<T>(val);
             o[e] = ACC ? o[e] + val : val;
           }
-          if (stream_out) {
-            VecIO<T>::store_stream(dst, o);
-          } else {
-            VecIO<T>::store(dst, o);
-          }
+          RV::store(dst, v, N, o, stream_out);
           if constexpr (DROP) {
             static_assert(V == 4 || V == 8, "a lane's vector is a Philox block or half of one");
             int64_t const at = row * (int64_t)N + (int64_t)v * V;
@@ -354,6 +344,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
           for (int e = 0; e < V; e++) {
             float tot = (pass == 0 ? dg[j][e] : db[j][e]) + fold[0][lane][e] +
                         fold[1][lane][e] + fold[2][lane][e];
+            if (ANY && e >= RV::elems(v, N)) continue;
             (pass == 0 ? pg : pb)[(int64_t)v * V + e] = tot;
           }
         }
@@ -366,6 +357,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
       if (v < nvec) {
 #pragma unroll
         for (int e = 0; e < V; e++) {
+          if (ANY && e >= RV::elems(v, N)) continue;
           pg[(int64_t)v * V + e] = dg[j][e];
           pb[(int64_t)v * V + e] = db[j][e];
         }
@@ -374,8 +366,8 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
   }
 }
 
-// Generic backward: any N; one workgroup per row for dX, then a column kernel
-// for dgamma/dbeta that walks all rows (GammaBetaBackwardSimpleCUDAKernel
+// Generic backward: rows too long for registers; one workgroup per row for dX, then a column
+// kernel for dgamma/dbeta that walks all rows (GammaBetaBackwardSimpleCUDAKernel
 // style, layer_norm_kernels.cu:184-214).
 template <typename T>
 __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_generic_dx_kernel(
@@ -446,11 +438,12 @@ static int ln_forward(hipStream_t st, void const *x, void *y, void const *gamma,
   T const *G = static_cast<T const *>(gamma);
   T const *Bt = static_cast<T const *>(beta);
   int ept = 0, wpr = 0;
-  bool vec = (N % V == 0) && aligned16(x) && aligned16(y) &&
-             (gamma == nullptr || aligned16(gamma)) &&
-             (beta == nullptr || aligned16(beta)) &&
-             pick_row_config_small(N / V, ept, wpr);
-  if (vec) {
+  bool const vec = (N % V == 0) && aligned16(x) && aligned16(y) && (gamma == nullptr || aligned16(gamma)) &&
+                   (beta == nullptr || aligned16(beta));
+  if (!pick_row_config_small(ceil_div(N, V), ept, wpr)) {
+    layer_norm_fwd_generic_kernel<T><<<(unsigned)M, kRowThreads, 0, st>>>(
+        X, Y, G, Bt, mean, rstd, M, (int)N, eps);
+  } else if (vec) {
     int64_t blocks = ceil_div(M, 4 / wpr);
     bool const stream = stream_past_caches(M * N, sizeof(T));
 #define CALL(E, W)                                                             \
@@ -465,8 +458,12 @@ static int ln_forward(hipStream_t st, void const *x, void *y, void const *gamma,
     FFK_ROW_DISPATCH_SMALL(ept, wpr, CALL);
 #undef CALL
   } else {
-    layer_norm_fwd_generic_kernel<T><<<(unsigned)M, kRowThreads, 0, st>>>(
-        X, Y, G, Bt, mean, rstd, M, (int)N, eps);
+    // [3001, 1001] fp32: 11.3 us with the scalar kernel, which reads a row three times
+#define CALL(E, W)                                                                                             \
+  layer_norm_fwd_kernel<T, E, W, false, false, true><<<(unsigned)ceil_div(M, 4 / wpr), kRowThreads, 0, st>>>( \
+      X, Y, G, Bt, mean, rstd, M, (int)N, eps)
+    FFK_ROW_DISPATCH_SMALL(ept, wpr, CALL);
+#undef CALL
   }
   FFK_CHECK_LAUNCH();
   return FFK_OK;
@@ -491,14 +488,19 @@ static int ln_backward(hipStream_t st, void const *dy, void const *x,
   T const *G = static_cast<T const *>(gamma);
   T *DX = static_cast<T *>(dx);
   int ept = 0, wpr = 0;
-  bool vec = (N % V == 0) && aligned16(dy) && aligned16(x) &&
-             (dx == nullptr || aligned16(dx)) && aligned16(residual) &&
-             (gamma == nullptr || aligned16(gamma)) && pick_row_config_small(N / V, ept, wpr);
+  bool const fits = pick_row_config_small(ceil_div(N, V), ept, wpr);
+  bool const vec = (N % V == 0) && aligned16(dy) && aligned16(x) && (dx == nullptr || aligned16(dx)) &&
+                   aligned16(residual) && (gamma == nullptr || aligned16(gamma)) && fits;
   if (!vec && RES != nullptr) {
     return fail(FFK_ERR_UNSUPPORTED, "layer_norm_backward: residual form needs the vector kernel");
   }
-  if (vec) {
+  // Rows that are not whole aligned vectors run the same kernel with any-address accesses
+  // ([3001, 1001] fp32, dX and both parameter gradients: 796 us in two scalar kernels, the second
+  // of them one thread a column over all rows).  It needs the workspace, which they did not: a
+  // caller that brought none still gets them.
+  if (vec || (fits && workspace != nullptr && workspace_bytes >= 2 * (size_t)N * sizeof(float))) {
     int blocks = ln_bwd_blocks(M, wpr);
+    if (!vec) fit_blocks_to_workspace = true;
     size_t const per_block = 2 * (size_t)N * sizeof(float);
     if (fit_blocks_to_workspace && workspace_bytes / per_block < (size_t)blocks) {
       // fewer, longer-running workgroups: dX is unchanged, the parameter
@@ -515,7 +517,14 @@ static int ln_backward(hipStream_t st, void const *dy, void const *x,
     bool const stream = stream_past_caches(M * N, sizeof(T));
 #define CALL(E, W)                                                             \
   do {                                                                         \
-    if (dropped != nullptr) {                                                  \
+    if (!vec) {                                                                \
+      if (acc)                                                                 \
+        layer_norm_bwd_kernel<T, E, W, true, false, true><<<blocks, kRowThreads, 0, st>>>( \
+            DY, X, mean, rstd, G, DX, partials, M, (int)N, nullptr);           \
+      else                                                                     \
+        layer_norm_bwd_kernel<T, E, W, false, false, true><<<blocks, kRowThreads, 0, st>>>( \
+            DY, X, mean, rstd, G, DX, partials, M, (int)N, nullptr);           \
+    } else if (dropped != nullptr) {                                                  \
       if constexpr (sizeof(T) == 2)                                            \
         layer_norm_bwd_kernel<T, E, W, true, true><<<blocks, kRowThreads, 0, st>>>( \
             DY, X, mean, rstd, G, DX, partials, M, (int)N, RES,                \

@@ -11,15 +11,17 @@
 
 namespace ffk {
 
-template <typename T, int EPT, int WPR, bool STREAM>
+// ANY: any row length at any address (RowVec).
+template <typename T, int EPT, int WPR, bool STREAM, bool ANY = false>
 __global__ __launch_bounds__(kRowThreads) void softmax_fwd_kernel(
     T const *__restrict__ X, T *__restrict__ Y, int64_t rows, int N) {
   constexpr int V = VecIO<T>::kVec;
+  using RV = RowVec<T, ANY>;
   constexpr int RPB = 4 / WPR;
   constexpr int LANES = 64 * WPR;
   __shared__ float smem[2][4][2];
   RowReducer<WPR> red(smem);
-  int const nvec = N / V;
+  int const nvec = RV::count(N);
   int const lane = WPR == 1 ? (threadIdx.x & 63) : threadIdx.x;
   int64_t const row = (int64_t)blockIdx.x * RPB + (WPR == 1 ? (threadIdx.x >> 6) : 0);
   bool const row_ok = row < rows;
@@ -30,10 +32,10 @@ __global__ __launch_bounds__(kRowThreads) void softmax_fwd_kernel(
   for (int j = 0; j < EPT; j++) {
     int v = lane + j * LANES;
     if (v < nvec) {
-      if (STREAM) {
-        VecIO<T>::load_stream(xr + (int64_t)v * V, x[j]);
-      } else {
-        VecIO<T>::load(xr + (int64_t)v * V, x[j]);
+      RV::load(xr, v, N, x[j], STREAM);
+      if constexpr (ANY) {
+#pragma unroll
+        for (int e = 0; e < V; e++) x[j][e] = e < RV::elems(v, N) ? x[j][e] : -INFINITY;
       }
 #pragma unroll
       for (int e = 0; e < V; e++) mx = fmaxf(mx, x[j][e]);
@@ -64,25 +66,23 @@ __global__ __launch_bounds__(kRowThreads) void softmax_fwd_kernel(
       float y[V];
 #pragma unroll
       for (int e = 0; e < V; e++) y[e] = x[j][e] * inv;
-      if (STREAM) {
-        VecIO<T>::store_stream(yr + (int64_t)v * V, y);
-      } else {
-        VecIO<T>::store(yr + (int64_t)v * V, y);
-      }
+      RV::store(yr, v, N, y, STREAM);
     }
   }
 }
 
-template <typename T, int EPT, int WPR, bool STREAM>
+// ANY: any row length at any address (RowVec).
+template <typename T, int EPT, int WPR, bool STREAM, bool ANY = false>
 __global__ __launch_bounds__(kRowThreads) void softmax_bwd_kernel(
     T const *__restrict__ Y, T const *__restrict__ dY, T *__restrict__ dX,
     int64_t rows, int N) {
   constexpr int V = VecIO<T>::kVec;
+  using RV = RowVec<T, ANY>;
   constexpr int RPB = 4 / WPR;
   constexpr int LANES = 64 * WPR;
   __shared__ float smem[2][4][2];
   RowReducer<WPR> red(smem);
-  int const nvec = N / V;
+  int const nvec = RV::count(N);
   int const lane = WPR == 1 ? (threadIdx.x & 63) : threadIdx.x;
   int64_t const row = (int64_t)blockIdx.x * RPB + (WPR == 1 ? (threadIdx.x >> 6) : 0);
   bool const row_ok = row < rows;
@@ -94,8 +94,8 @@ __global__ __launch_bounds__(kRowThreads) void softmax_bwd_kernel(
     int v = lane + j * LANES;
     if (v < nvec) {
       // two input streams read once: cache-bypassing loads
-      VecIO<T>::load_stream(Y + r * (int64_t)N + (int64_t)v * V, y[j]);
-      VecIO<T>::load_stream(dY + r * (int64_t)N + (int64_t)v * V, dy[j]);
+      RV::load(Y + r * (int64_t)N, v, N, y[j], true);
+      RV::load(dY + r * (int64_t)N, v, N, dy[j], true);
 #pragma unroll
       for (int e = 0; e < V; e++) dot += y[j][e] * dy[j][e];
     }
@@ -109,11 +109,7 @@ __global__ __launch_bounds__(kRowThreads) void softmax_bwd_kernel(
       float o[V];
 #pragma unroll
       for (int e = 0; e < V; e++) o[e] = y[j][e] * (dy[j][e] - dot);
-      if (STREAM) {
-        VecIO<T>::store_stream(dX + row * (int64_t)N + (int64_t)v * V, o);
-      } else {
-        VecIO<T>::store(dX + row * (int64_t)N + (int64_t)v * V, o);
-      }
+      RV::store(dX + row * (int64_t)N, v, N, o, STREAM);
     }
   }
 }
@@ -205,12 +201,15 @@ static int softmax_fwd(hipStream_t st, void const *x, void *y, int64_t outer,
   T *Y = static_cast<T *>(y);
   if (inner == 1) {
     int ept = 0, wpr = 0;
-    if (dim % V == 0 && aligned16(x) && aligned16(y) && pick_row_config(dim / V, ept, wpr)) {
+    if (pick_row_config(ceil_div(dim, V), ept, wpr)) {
       int64_t blocks = ceil_div(outer, 4 / wpr);
+      bool const vec = dim % V == 0 && aligned16(x) && aligned16(y);
       bool const stream = stream_past_caches(outer * dim, sizeof(T));
 #define CALL(E, W)                                                             \
   do {                                                                         \
-    if (stream)                                                                \
+    if (!vec)                                                                  \
+      softmax_fwd_kernel<T, E, W, false, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(X, Y, outer, (int)dim); \
+    else if (stream)                                                           \
       softmax_fwd_kernel<T, E, W, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(X, Y, outer, (int)dim); \
     else                                                                       \
       softmax_fwd_kernel<T, E, W, false><<<(unsigned)blocks, kRowThreads, 0, st>>>(X, Y, outer, (int)dim); \
@@ -237,13 +236,15 @@ static int softmax_bwd(hipStream_t st, void const *y, void const *dy, void *dx,
   T *DX = static_cast<T *>(dx);
   if (inner == 1) {
     int ept = 0, wpr = 0;
-    if (dim % V == 0 && aligned16(y) && aligned16(dy) && aligned16(dx) &&
-        pick_row_config(dim / V, ept, wpr)) {
+    if (pick_row_config(ceil_div(dim, V), ept, wpr)) {
       int64_t blocks = ceil_div(outer, 4 / wpr);
+      bool const vec = dim % V == 0 && aligned16(y) && aligned16(dy) && aligned16(dx);
       bool const stream = stream_past_caches(outer * dim, sizeof(T));
 #define CALL(E, W)                                                             \
   do {                                                                         \
-    if (stream)                                                                \
+    if (!vec)                                                                  \
+      softmax_bwd_kernel<T, E, W, false, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(Y, DY, DX, outer, (int)dim); \
+    else if (stream)                                                           \
       softmax_bwd_kernel<T, E, W, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(Y, DY, DX, outer, (int)dim); \
     else                                                                       \
       softmax_bwd_kernel<T, E, W, false><<<(unsigned)blocks, kRowThreads, 0, st>>>(Y, DY, DX, outer, (int)dim); \
