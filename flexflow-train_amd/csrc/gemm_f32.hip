@@ -1,0 +1,423 @@
+// fp32 GEMM kernels for gfx950 (v_mfma_f32_32x32x2f32), behind gemm_dispatch.
+#include "gemm_bf16.h"
+#include "small_f32.h"
+
+namespace ffk {
+
+// ---------------------------------------------------------------------------
+// fp32 MFMA kernel (32x32x2), 64x64 block tile, bounds-checked everywhere.
+// ---------------------------------------------------------------------------
+template <bool TA, bool TB>
+__global__ __launch_bounds__(256) void gemm_f32_kernel(
+    float const *__restrict__ A, float const *__restrict__ B, float *C, int M,
+    int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
+    float const *__restrict__ bias, int act, int accumulate) {
+  constexpr int BM = 64, BN = 64, BKF = 16, LD = 68;
+  __shared__ float As[BKF][LD];  // [k][m]
+  __shared__ float Bs[BKF][LD];  // [k][n]
+  int const t = threadIdx.x;
+  int const lane = t & 63;
+  int const wave = t >> 6;
+  int const wm0 = (wave >> 1) * 32;
+  int const wn0 = (wave & 1) * 32;
+  int const nbn = (N + BN - 1) / BN;
+  int const m0 = (blockIdx.x / nbn) * BM;
+  int const n0 = (blockIdx.x % nbn) * BN;
+
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+
+  for (int k0 = 0; k0 < K; k0 += BKF) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      int m, k;
+      if (!TA) {  // A[M,K]: k fastest across lanes
+        k = t & 15;
+        m = (t >> 4) + 16 * i;
+      } else {  // A[K,M]: m fastest
+        m = t & 63;
+        k = (t >> 6) + 4 * i;
+      }
+      int gm = m0 + m, gk = k0 + k;
+      float v = 0.0f;
+      if (gm < M && gk < K) {
+        v = TA ? A[(int64_t)gk * lda + gm] : A[(int64_t)gm * lda + gk];
+      }
+      As[k][m] = v;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      int n, k;
+      if (TB) {  // B[N,K]: k fastest
+        k = t & 15;
+        n = (t >> 4) + 16 * i;
+      } else {  // B[K,N]: n fastest
+        n = t & 63;
+        k = (t >> 6) + 4 * i;
+      }
+      int gn = n0 + n, gk = k0 + k;
+      float v = 0.0f;
+      if (gn < N && gk < K) {
+        v = TB ? B[(int64_t)gn * ldb + gk] : B[(int64_t)gk * ldb + gn];
+      }
+      Bs[k][n] = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < BKF / 2; kk++) {
+      float a = As[2 * kk + (lane >> 5)][wm0 + (lane & 31)];
+      float b = Bs[2 * kk + (lane >> 5)][wn0 + (lane & 31)];
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
+    }
+    __syncthreads();
+  }
+
+  int const n = n0 + wn0 + (lane & 31);
+  if (n < N) {
+    float bv = bias != nullptr ? bias[n] : 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      int const m = m0 + wm0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+      if (m < M) {
+        float v = apply_activation(acc[r] + bv, act);
+        float *dst = C + (int64_t)m * ldc + n;
+        if (accumulate) {
+          v += *dst;
+        }
+        *dst = v;
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// fp32 MFMA kernel: BM x BN block tile (128 or 64 each), 2 x 2 waves of BM/2 x BN/2, reduction
+// tiles of 32, operands read 16 bytes at a time.
+// The next tile travels global -> registers while this one is multiplied and
+// goes to the other LDS buffer afterwards: one barrier per tile.  The fp32
+// MFMA (32x32x2, 64 cycles) is so slow next to its two one-register operands
+// that LDS and issue bandwidth are never short; what the kernel has to do is
+// keep loads in flight and the matrix pipe fed, which two workgroups per CU and
+// fragments read one step ahead take care of.
+//   An operand whose reduction index is contiguous in memory (A[M,K], B[N,K])
+// lies in LDS as [k / 2][row][k % 2], row stride 2 * rows + 4: a lane's four
+// consecutive k go out as two 8-byte writes, and the MFMA read -- lanes 0-31
+// one k, lanes 32-63 the next -- touches 64 consecutive floats.  The compiler
+// pairs a lane's reads for two 32-row blocks into one two-dword read, which is
+// served 32 lanes at a time: the pairs of odd blocks are stored swapped, so
+// that those 32 lanes take even banks for one block and odd banks for the
+// other (unswapped they met in the same banks: 2.6 conflict cycles per cycle
+// of LDS work, the matrix pipe 80% busy).  An operand
+// whose rows are contiguous (A[K,M], B[K,N]) lies as [k][row] with the two
+// 32-float halves of every odd k swapped, which does the same for the read
+// without padding.  Every element's products are added in ascending k, two per
+// MFMA, as in gemm_f32_kernel: the two kernels give the same bits.
+// Rows and columns past the edge are read from the last valid ones and never
+// stored; k past the end is zeroed when the tile is written to LDS.
+// ANY: lengths and row starts that are no multiple of four elements.  The 16-byte reads then start
+// at any element; a quad that straddles an edge is read element by element from clamped places --
+// of a k-contiguous operand only in the last k-tile, of the others only in the workgroups whose
+// tile reaches past the edge.
+// ---------------------------------------------------------------------------
+template <bool TA, bool TB, int BM, int BN, bool ANY>
+__global__ __launch_bounds__(256, 2) void gemm_f32_tiled_kernel(
+    float const *__restrict__ A, float const *__restrict__ B, float *C, int M, int N, int K, int64_t lda,
+    int64_t ldb, int64_t ldc, float const *__restrict__ bias, int act, int accumulate) {
+  constexpr int BKT = 32;
+  constexpr int TMW = BM / 64, TNW = BN / 64;  // 32-row / 32-column blocks per wave
+  constexpr bool A_KC = !TA, B_KC = TB;     // reduction index contiguous in memory
+  constexpr int A_CH = BM * BKT / 4 / 256, B_CH = BN * BKT / 4 / 256;  // 16-byte chunks per thread and tile
+  constexpr int A_SP = 2 * BM + 4, B_SP = 2 * BN + 4;                  // pair-layout row strides
+  constexpr int A_FLOATS = A_KC ? (BKT / 2) * A_SP : BKT * BM;
+  constexpr int B_FLOATS = B_KC ? (BKT / 2) * B_SP : BKT * BN;
+  __shared__ __attribute__((aligned(16))) float As[2][A_FLOATS];
+  __shared__ __attribute__((aligned(16))) float Bs[2][B_FLOATS];
+  int const t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  int const h = lane >> 5, l32 = lane & 31;
+  int const wm0 = (wave >> 1) * (BM / 2), wn0 = (wave & 1) * (BN / 2);
+  int tm, tn;
+  tile_coords(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN, tm, tn);
+  int const m0 = tm * BM, n0 = tn * BN;
+
+  // Chunk i of this thread: (row, k quad) of a k-contiguous operand, (k row, row quad) otherwise.
+  // Its address for k-tile 0 is kept and moved on by a constant per tile; only a tile that
+  // reaches past K (the last one of a ragged reduction) computes clamped addresses afresh.
+  constexpr int NCH = A_CH + B_CH;
+  f32x4 rgs[2][NCH];  // k-tile kt travels in set kt % 2, two tiles ahead of its use
+  float const *pg[NCH];
+#pragma unroll
+  for (int i = 0; i < A_CH; i++) {
+    int const c = t + i * 256;
+    pg[i] = A_KC ? A + (int64_t)min(m0 + c / 8, M - 1) * lda + 4 * (c % 8)
+                 : A + (int64_t)(c / (BM / 4)) * lda + (ANY ? m0 + 4 * (c % (BM / 4)) : min(m0 + 4 * (c % (BM / 4)), M - 4));
+  }
+#pragma unroll
+  for (int i = 0; i < B_CH; i++) {
+    int const c = t + i * 256;
+    pg[A_CH + i] = B_KC ? B + (int64_t)min(n0 + c / 8, N - 1) * ldb + 4 * (c % 8)
+                        : B + (int64_t)(c / (BN / 4)) * ldb + (ANY ? n0 + 4 * (c % (BN / 4)) : min(n0 + 4 * (c % (BN / 4)), N - 4));
+  }
+  int64_t const step_a = A_KC ? BKT : (int64_t)BKT * lda, step_b = B_KC ? BKT : (int64_t)BKT * ldb;
+  // load of chunk i of k-tile kt; pg[i] points at k-tile kt on entry and at kt + 1 on return
+  auto gload_chunk = [&](int kt, int i, f32x4 (&rg)[NCH]) __attribute__((always_inline)) {
+    int const k0 = kt * BKT;
+    bool const is_a = i < A_CH;
+    bool const kc = is_a ? A_KC : B_KC;
+    // this chunk's tile reaches past the edge along the operand's contiguous index
+    bool const straddles = ANY && (kc ? k0 + BKT > K : is_a ? m0 + BM > M : n0 + BN > N);  // uniform
+    if (straddles) {
+      int const c = t + (is_a ? i : i - A_CH) * 256;
+      int const row = (is_a ? BM : BN) / 4;
+      int const at = kc ? k0 + 4 * (c % 8) : (is_a ? m0 : n0) + 4 * (c % row);
+      int const len = kc ? K : is_a ? M : N;
+      // rows past K (of an operand lying [K][..]) are read from the last one
+      float const *const p = kc || k0 + c / row < K ? pg[i] : pg[i] - (int64_t)(k0 + c / row - (K - 1)) * (is_a ? lda : ldb);
+#pragma unroll
+      for (int j = 0; j < 4; j++) rg[i][j] = p[min(j, len - 1 - at)];
+    } else if (k0 + BKT <= K) {
+      rg[i] = ANY ? __builtin_bit_cast(f32x4, load_raw_any(pg[i])) : *reinterpret_cast<f32x4 const *>(pg[i]);
+    } else {
+      int const c = t + (is_a ? i : i - A_CH) * 256;
+      // how far this chunk's k lies past the last one it may read
+      if (is_a ? A_KC : B_KC) {
+        int const over = max(k0 + 4 * (c % 8) - (K - 4), 0);
+        rg[i] = *reinterpret_cast<f32x4 const *>(pg[i] - over);
+      } else {
+        int const over = max(k0 + c / ((is_a ? BM : BN) / 4) - (K - 1), 0);
+        float const *const p = pg[i] - (int64_t)over * (is_a ? lda : ldb);
+        rg[i] = ANY ? __builtin_bit_cast(f32x4, load_raw_any(p)) : *reinterpret_cast<f32x4 const *>(p);
+      }
+    }
+    pg[i] += is_a ? step_a : step_b;
+  };
+  auto gload = [&](int kt, f32x4 (&rg)[NCH]) {
+#pragma unroll
+    for (int i = 0; i < NCH; i++) gload_chunk(kt, i, rg);
+  };
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  // chunk i of k-tile kt from its registers into buffer buf, k past the end zeroed
+  auto lstore_chunk = [&](int buf, int kt, int i, f32x4 const (&rg)[NCH]) __attribute__((always_inline)) {
+    f32x4 const zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    int const k0 = kt * BKT;
+    bool const is_a = i < A_CH;
+    int const c = t + (is_a ? i : i - A_CH) * 256;
+    float *dst = is_a ? As[buf] : Bs[buf];
+    int const SP = is_a ? A_SP : B_SP, R = is_a ? BM : BN;
+    // (vector instructions between the MFMAs are not free: with two waves on a SIMD the masks
+    // and selects of this function, applied to every tile, cost 5-10% of the matrix pipe's time.
+    // The mask is for the one tile that reaches past K; which blocks are swapped is known per chunk.)
+    bool const whole = k0 + BKT <= K;  // uniform
+    if (is_a ? A_KC : B_KC) {
+      int const row = c / 8, kq = c % 8;
+      f32x4 v = rg[i];
+      if (!whole) {
+        asm volatile("" ::: "memory");  // a branch, not four selects on every tile
+        if constexpr (ANY) {
+#pragma unroll
+          for (int j = 0; j < 4; j++) v[j] = k0 + 4 * kq + j < K ? v[j] : 0.0f;
+        } else {
+          v = k0 + 4 * kq < K ? v : zero;
+        }
+      }
+      // odd 32-row blocks hold their k pairs swapped; row / 32 = chunk number (t / 8 < 32)
+      bool const odd = (((is_a ? i : i - A_CH) & 1) != 0);
+      *reinterpret_cast<f32x2 *>(&dst[(2 * kq) * SP + 2 * row]) = odd ? f32x2{v[1], v[0]} : f32x2{v[0], v[1]};
+      *reinterpret_cast<f32x2 *>(&dst[(2 * kq + 1) * SP + 2 * row]) = odd ? f32x2{v[3], v[2]} : f32x2{v[2], v[3]};
+    } else {
+      int const k = c / (R / 4), rq = c % (R / 4);
+      f32x4 v = rg[i];
+      if (!whole) {
+        asm volatile("" ::: "memory");
+        v = k0 + k < K ? v : zero;
+      }
+      *reinterpret_cast<f32x4 *>(&dst[k * R + ((4 * rq) ^ ((k & 1) * 32))]) = v;
+    }
+  };
+  // operand value of this lane for MFMA step kk (k = 2 kk + h) and its row
+  auto frag_a = [&](int buf, int kk, int row) -> float {
+    return A_KC ? As[buf][kk * A_SP + 2 * row + (h ^ ((row >> 5) & 1))] : As[buf][(2 * kk + h) * BM + (row ^ (h * 32))];
+  };
+  auto frag_b = [&](int buf, int kk, int row) -> float {
+    return B_KC ? Bs[buf][kk * B_SP + 2 * row + (h ^ ((row >> 5) & 1))] : Bs[buf][(2 * kk + h) * BN + (row ^ (h * 32))];
+  };
+
+  f32x16 acc[TMW][TNW];
+#pragma unroll
+  for (int i = 0; i < TMW; i++)
+#pragma unroll
+    for (int j = 0; j < TNW; j++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+
+  int const KT = (K + BKT - 1) / BKT;
+  gload(0, rgs[0]);
+  if (KT > 1) gload(1, rgs[1]);
+#pragma unroll
+  for (int i = 0; i < NCH; i++) lstore_chunk(0, 0, i, rgs[0]);
+  __syncthreads();
+  // One k-tile, kt, from buffer kt % 2.  AHEAD2: k-tile kt + 2 exists; its loads go out one per
+  // step in the first NCH steps (a burst of them holds the wave, and with it its MFMAs, for as
+  // long as the memory pipeline takes to accept them), into the register set that tile kt
+  // travelled in.  AHEAD1: k-tile kt + 1
+  // exists; it was asked for a tile ago and is written to the other buffer (which nobody reads
+  // during this tile) one chunk per step in the last NCH steps, under the MFMAs.  A wave sits
+  // at each MFMA until the pipe takes it, so whatever is placed between two of them costs
+  // nothing as long as it is short; the fences keep it there.
+  constexpr int KS = BKT / 2;
+  static_assert(NCH <= KS, "one chunk per step");
+  auto tile = [&](int kt, auto set_tag, auto ahead1_tag, auto ahead2_tag) {
+    constexpr int SET = decltype(set_tag)::value;  // = kt % 2
+    constexpr bool AHEAD1 = decltype(ahead1_tag)::value, AHEAD2 = decltype(ahead2_tag)::value;
+    float af[2][TMW], bfv[2][TNW];
+#pragma unroll
+    for (int i = 0; i < TMW; i++) af[0][i] = frag_a(SET, 0, wm0 + i * 32 + l32);
+#pragma unroll
+    for (int j = 0; j < TNW; j++) bfv[0][j] = frag_b(SET, 0, wn0 + j * 32 + l32);
+#pragma unroll
+    for (int kk = 0; kk < KS; kk++) {
+      int const c = kk & 1, nx = c ^ 1;
+      // the next step's fragments are asked for before this step's MFMAs are issued: reads
+      // issued behind them would start their round trip only when the last one has gone
+      if (kk + 1 < KS) {
+#pragma unroll
+        for (int i = 0; i < TMW; i++) af[nx][i] = frag_a(SET, kk + 1, wm0 + i * 32 + l32);
+#pragma unroll
+        for (int j = 0; j < TNW; j++) bfv[nx][j] = frag_b(SET, kk + 1, wn0 + j * 32 + l32);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[c][0], bfv[c][0], acc[0][0], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (AHEAD2 && kk < NCH) gload_chunk(kt + 2, kk, rgs[SET]);
+      if (AHEAD1 && kk >= KS - NCH) lstore_chunk(SET ^ 1, kt + 1, kk - (KS - NCH), rgs[SET ^ 1]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < TMW; i++)
+#pragma unroll
+        for (int j = 0; j < TNW; j++)
+          if (i + j > 0) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[c][i], bfv[c][j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+  };
+  using T0 = std::integral_constant<int, 0>;
+  using T1 = std::integral_constant<int, 1>;
+  int kt = 0;
+  for (; kt + 3 < KT; kt += 2) {  // both tiles of the pair have two successors
+    tile(kt, T0{}, std::true_type{}, std::true_type{});
+    tile(kt + 1, T1{}, std::true_type{}, std::true_type{});
+  }
+  // the last one to three tiles (kt is even)
+  if (kt + 2 < KT) {
+    tile(kt, T0{}, std::true_type{}, std::true_type{});
+    tile(kt + 1, T1{}, std::true_type{}, std::false_type{});
+    tile(kt + 2, T0{}, std::false_type{}, std::false_type{});
+  } else if (kt + 1 < KT) {
+    tile(kt, T0{}, std::true_type{}, std::false_type{});
+    tile(kt + 1, T1{}, std::false_type{}, std::false_type{});
+  } else {
+    tile(kt, T0{}, std::false_type{}, std::false_type{});
+  }
+
+  // accumulator element r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of its block
+#pragma unroll
+  for (int j = 0; j < TNW; j++) {
+    int const n = n0 + wn0 + j * 32 + l32;
+    if (n >= N) continue;
+    float const bv = bias != nullptr ? bias[n] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < TMW; i++) {
+      int const mb = m0 + wm0 + i * 32 + 4 * h;
+      float old[16];
+      if (accumulate) {  // what C holds, all loads in flight together
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          int const m = min(mb + 8 * (r >> 2) + (r & 3), M - 1);
+          old[r] = C[(int64_t)m * ldc + n];
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        int const m = mb + 8 * (r >> 2) + (r & 3);
+        float v = apply_activation(acc[i][j][r] + bv, act);
+        if (accumulate) v += old[r];
+        if (m < M) C[(int64_t)m * ldc + n] = v;
+      }
+    }
+  }
+}
+
+// A long reduction over few outputs: sixteen waves a 16 x 16 tile (small_f32.h), where block tiles
+// would leave most of the chip idle and walk the reduction alone ([25,1024] over 42 023: 1180 us with
+// sixteen workgroups of 64 x 64).
+template <bool TA, bool TB>
+__global__ __launch_bounds__(1024) void gemm_f32_deep_kernel(float const *__restrict__ A, float const *__restrict__ B, float *C,
+                                                             int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
+                                                             float const *__restrict__ bias, int act, int accumulate) {
+  constexpr int T = 16, WAVES = 16;
+  __shared__ SmallShared<T, WAVES> sm;
+  int const nbn = (N + T - 1) / T, tm = (int)blockIdx.x / nbn, tn = (int)blockIdx.x - tm * nbn;
+  SmallOperand<!TA, FFK_ACT_NONE> const a = {A, nullptr, lda, 0};
+  SmallOperand<TB, FFK_ACT_NONE> const b = {B, nullptr, ldb, 0};
+  auto store = [&](int m, int n, float v) {
+    v = apply_activation(v + (bias != nullptr ? bias[n] : 0.0f), act);
+    float *const to = C + (int64_t)m * ldc + n;
+    *to = accumulate ? *to + v : v;
+  };
+  small_tile<T, WAVES, WAVES>(a, b, M, N, K, tm * T, tn * T, true, nullptr, 0, store, false, [](int, float) {}, sm);
+}
+
+template <bool TA, bool TB, int BM, int BN, bool ANY>
+static void launch_tiled(hipStream_t st, int M, int N, int K, float const *A, int64_t lda, float const *B, int64_t ldb,
+                         float *C, int64_t ldc, GemmEpilogue const &ep) {
+  if (describe_only("gemm_f32_tiled_kernel<%s,%s,%d,%d,%s>", tf(TA), tf(TB), BM, BN, tf(ANY))) return;
+  gemm_f32_tiled_kernel<TA, TB, BM, BN, ANY><<<(int)(ceil_div(M, BM) * ceil_div(N, BN)), 256, 0, st>>>(
+      A, B, C, M, N, K, lda, ldb, ldc, static_cast<float const *>(ep.bias), ep.activation, ep.accumulate);
+}
+
+template <bool TA, bool TB>
+static void pick_f32(hipStream_t st, int M, int N, int K, float const *A, int64_t lda, float const *B, int64_t ldb,
+                     float *C, int64_t ldc, GemmEpilogue const &ep) {
+  // (64 x 64 tiles of the same output would reach a quarter of the CUs at most)
+  if (K >= 2048 && ceil_div(M, 64) * ceil_div(N, 64) <= kNumCU / 4) {
+    if (describe_only("gemm_f32_deep_kernel<%s,%s>", tf(TA), tf(TB))) return;
+    gemm_f32_deep_kernel<TA, TB><<<(int)(ceil_div(M, 16) * ceil_div(N, 16)), 1024, 0, st>>>(
+        A, B, C, M, N, K, lda, ldb, ldc, static_cast<float const *>(ep.bias), ep.activation, ep.accumulate);
+    return;
+  }
+  if ((int64_t)M * N < 128 * 128 || K < 4) {
+    if (describe_only("gemm_f32_kernel<%s,%s>", tf(TA), tf(TB))) return;
+    gemm_f32_kernel<TA, TB><<<(int)(ceil_div(M, 64) * ceil_div(N, 64)), 256, 0, st>>>(
+        A, B, C, M, N, K, lda, ldb, ldc, static_cast<float const *>(ep.bias), ep.activation, ep.accumulate);
+    return;
+  }
+  // 16-byte reads: aligned rows, and whole quads along whichever index is contiguous
+  bool const quads = aligned16(A) && aligned16(B) && lda % 4 == 0 && ldb % 4 == 0 && (TA ? M : K) % 4 == 0 && (TB ? K : N) % 4 == 0 &&
+                     M >= 4 && N >= 4;
+  // 128 x 128 tiles when they give every CU two workgroups, 128 x 64 when those reach three quarters
+  // of the CUs, 64 x 64 below and where half a 128-row tile would be empty
+  int const tile = M <= 64 ? 2 : ceil_div(M, 128) * ceil_div(N, 128) >= 2 * kNumCU ? 0 :
+                   ceil_div(M, 128) * ceil_div(N, 64) >= kNumCU * 3 / 4 ? 1 : 2;
+#define FFK_F32(BM_, BN_)                                                              \
+  do {                                                                                 \
+    if (quads)                                                                         \
+      launch_tiled<TA, TB, BM_, BN_, false>(st, M, N, K, A, lda, B, ldb, C, ldc, ep);  \
+    else                                                                               \
+      launch_tiled<TA, TB, BM_, BN_, true>(st, M, N, K, A, lda, B, ldb, C, ldc, ep);   \
+  } while (0)
+  if (tile == 0) FFK_F32(128, 128);
+  else if (tile == 1) FFK_F32(128, 64);
+  else FFK_F32(64, 64);
+#undef FFK_F32
+}
+
+hipError_t gemm_f32_launch(hipStream_t st, bool ta, bool tb, int M, int N, int K, float const *A, int64_t lda,
+                           float const *B, int64_t ldb, float *C, int64_t ldc, GemmEpilogue const &ep) {
+  if (!ta && !tb) pick_f32<false, false>(st, M, N, K, A, lda, B, ldb, C, ldc, ep);
+  else if (!ta && tb) pick_f32<false, true>(st, M, N, K, A, lda, B, ldb, C, ldc, ep);
+  else if (ta && !tb) pick_f32<true, false>(st, M, N, K, A, lda, B, ldb, C, ldc, ep);
+  else pick_f32<true, true>(st, M, N, K, A, lda, B, ldb, C, ldc, ep);
+  return tl_name_sink != nullptr ? hipSuccess : hipGetLastError();
+}
+
+}  // namespace ffk

@@ -12,6 +12,7 @@
 //           bias_grad (+)= column sums of g (linear_kernels.cu:249-334).
 #include "elementwise.h"
 #include "gemm.h"
+#include "small_f32.h"
 
 namespace ffk {
 
@@ -76,186 +77,64 @@ static hipError_t l2_reg_grad(hipStream_t st, void const *w, void *dw, int64_t n
 }
 
 // ---------------------------------------------------------------------------
-// The whole backward of a small fp32 Linear in ONE launch.  At sizes like the
-// reference's CPU-runnable case ([32,64] . [128,64]^T) every kernel is a few
-// microseconds of launch latency around almost no work, so the activation
-// gradient, the two products and the bias sums, which are independent given
-// (output, output_grad), run as jobs of one grid: workgroups [0, tiles_dx)
-// compute 64x64 tiles of input_grad, the next tiles_dw ones tiles of
-// weight_grad, the rest 64 columns of bias_grad each.  g = act'(output) *
-// output_grad is applied where an operand element is loaded, never stored.
+// Small fp32 Linear layers: ONE launch forward and ONE backward on the tiles of small_f32.h.  At
+// sizes like the reference's CPU-runnable case ([32,64] . [128,64]^T) a pass is one chain of
+// latencies around almost no work: 6.5 + 7.2 us with 64x64 tiles staged through LDS and one wave's
+// chain of 32 MFMAs, 2.4 + 2.9 us with these.
+// The backward's jobs -- tiles of input_grad, then tiles of weight_grad, the first column of which
+// also adds up bias_grad -- are independent given (output, output_grad): g = act'(output) *
+// output_grad is applied where an operand element is used, never stored.
 // ---------------------------------------------------------------------------
 struct SmallLinearBwd {
   float const *y, *dy, *x, *w;
   float *dx, *dw, *db;
   int batch, in_dim, out_dim;
-  int act, relu_mode, accumulate;  // accumulate: FFK_ACC_* bits
-  int tiles_dx, tiles_dw;
+  int relu_mode, accumulate;  // accumulate: FFK_ACC_* bits
+  int blocks_dx;
 };
-
-// ACT is a template argument of the kernel: a run-time switch here puts a branch and a wait
-// between every two loads of a thread, and the kernel's time is its round trips to memory.
-template <int ACT>
-__device__ __forceinline__ float small_act_grad(int mode, float y, float dy) {
-  if constexpr (ACT == FFK_ACT_RELU) {
-    return mode == 1 ? (dy > 0.0f ? 1.0f : 0.0f) : (y > 0.0f ? dy : 0.0f);
-  } else if constexpr (ACT == FFK_ACT_SIGMOID) {
-    return dy * y * (1.0f - y);
-  } else if constexpr (ACT == FFK_ACT_TANH) {
-    return dy * (1.0f - y * y);
-  } else {
-    return dy;
-  }
-}
-
-// One 64x64 tile of sum_k a(m, k) * b(k, n), handed element by element to store(m, n, value).  a
-// and b clamp their coordinates into the problem and return what lies there: rows and columns
-// past the edge give values that are never stored, k past the edge is zeroed here when the tile
-// is written to LDS (a select on a loaded value any earlier is a wait for that load).  A_KFAST: consecutive lanes walk k of the A operand (it
-// lies [M][K]); otherwise m; B_KFAST likewise for B lying [N][K].  A k-tile is 64 deep, all of a thread's 32 loads are issued
-// before the first is waited for, and the next k-tile's are issued before this one is multiplied: at these sizes the
-// time is the number of round trips to memory, not the arithmetic.
-constexpr int kSmallBK = 64;
-constexpr int kSmallMaxDepth = 1024;  // longest reduction the one-launch kernels take (16 k-tiles)
-// a returns what it loaded (a float, or the pair an activation gradient is made of) and av turns
-// that into the operand's value when the tile is written to LDS, one k-tile later: arithmetic on a
-// loaded value any earlier would make the wave wait for the load it is meant to run under.
-template <bool A_KFAST, bool B_KFAST, typename FA, typename FAV, typename FB, typename FS>
-__device__ __forceinline__ void small_f32_tile(FA a, FAV av, FB b, int M, int N, int K, int m0, int n0, FS store,
-                                               float (&As)[kSmallBK][68], float (&Bs)[kSmallBK][68],
-                                               float const *prior = nullptr, int64_t prior_ld = 0) {
-  int const t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  int const wm0 = (wave >> 1) * 32, wn0 = (wave & 1) * 32;
-  f32x16 acc;
-#pragma unroll
-  for (int r = 0; r < 16; r++) acc[r] = 0.0f;
-  decltype(a(0, 0)) ra[16];
-  float rb[16];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-      int const k = A_KFAST ? (t & 63) : (t >> 6) + 4 * i;
-      int const m = A_KFAST ? (t >> 6) + 4 * i : (t & 63);
-      int const kb = B_KFAST ? (t & 63) : (t >> 6) + 4 * i;
-      int const n = B_KFAST ? (t >> 6) + 4 * i : (t & 63);
-      ra[i] = a(m0 + m, k0 + k);
-      rb[i] = b(k0 + kb, n0 + n);
-    }
-  };
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += kSmallBK) {
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-      int const k = A_KFAST ? (t & 63) : (t >> 6) + 4 * i;
-      int const m = A_KFAST ? (t >> 6) + 4 * i : (t & 63);
-      int const kb = B_KFAST ? (t & 63) : (t >> 6) + 4 * i;
-      int const n = B_KFAST ? (t >> 6) + 4 * i : (t & 63);
-      As[k][m] = k0 + k < K ? av(ra[i]) : 0.0f;
-      Bs[kb][n] = k0 + kb < K ? rb[i] : 0.0f;
-    }
-    __syncthreads();
-    if (k0 + kSmallBK < K) fetch(k0 + kSmallBK);  // on its way while this tile is multiplied
-#pragma unroll
-    for (int kk = 0; kk < kSmallBK / 2; kk++) {
-      float const av = As[2 * kk + (lane >> 5)][wm0 + (lane & 31)];
-      float const bv = Bs[2 * kk + (lane >> 5)][wn0 + (lane & 31)];
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc, 0, 0, 0);
-    }
-    __syncthreads();
-  }
-  int const n = n0 + wn0 + (lane & 31);
-  if (n < N) {
-    if (prior != nullptr) {  // accumulating: what the destination holds, all 16 loads in flight together
-      float old[16];
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        int const m = m0 + wm0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        old[r] = prior[(int64_t)(m < M ? m : M - 1) * prior_ld + n];
-      }
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[r] = old[r] + acc[r];
-    }
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-      int const m = m0 + wm0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-      if (m < M) store(m, n, acc[r]);
-    }
-  }
-}
-
-template <int ACT>
-__global__ __launch_bounds__(256) void linear_small_bwd_f32_kernel(SmallLinearBwd p) {
-  __shared__ float As[kSmallBK][68], Bs[kSmallBK][68];
-  int const bid = blockIdx.x;
-  // g[batch, out] = act'(output) * output_grad, as the pair it is made of and as its value
-  auto g_raw = [&](int row, int col) -> float2 {
-    int const r = row < p.batch ? row : p.batch - 1, c = col < p.out_dim ? col : p.out_dim - 1;
-    int64_t const i = (int64_t)r * p.out_dim + c;
-    float yv = 0.0f;
-    if constexpr (ACT == FFK_ACT_RELU || ACT == FFK_ACT_SIGMOID || ACT == FFK_ACT_TANH) yv = p.y[i];
-    return make_float2(yv, p.dy[i]);
-  };
-  auto g_val = [&](float2 r) -> float { return small_act_grad<ACT>(p.relu_mode, r.x, r.y); };
-  if (bid < p.tiles_dx) {
-    // input_grad[batch, in] (+)= g[batch, out] . weight[out, in]
-    int const nbn = (p.in_dim + 63) / 64;
-    auto b = [&](int k, int n) -> float {
-      return p.w[(int64_t)(k < p.out_dim ? k : p.out_dim - 1) * p.in_dim + (n < p.in_dim ? n : p.in_dim - 1)];
-    };
-    bool const add = (p.accumulate & FFK_ACC_INPUT) != 0;
-    auto store = [&](int m, int n, float v) { p.dx[(int64_t)m * p.in_dim + n] = v; };
-    small_f32_tile<true, false>(g_raw, g_val, b, p.batch, p.in_dim, p.out_dim, (bid / nbn) * 64, (bid % nbn) * 64, store, As, Bs,
-                                add ? p.dx : nullptr, p.in_dim);
-  } else if (bid < p.tiles_dx + p.tiles_dw) {
-    // weight_grad[out, in] (+)= g[batch, out]^T . input[batch, in]
-    int const tb = bid - p.tiles_dx, nbn = (p.in_dim + 63) / 64;
-    auto a = [&](int m, int k) -> float2 { return g_raw(k, m); };
-    auto b = [&](int k, int n) -> float {
-      return p.x[(int64_t)(k < p.batch ? k : p.batch - 1) * p.in_dim + (n < p.in_dim ? n : p.in_dim - 1)];
-    };
-    bool const add = (p.accumulate & FFK_ACC_WEIGHT) != 0;
-    auto store = [&](int m, int n, float v) { p.dw[(int64_t)m * p.in_dim + n] = v; };
-    small_f32_tile<false, false>(a, g_val, b, p.out_dim, p.in_dim, p.batch, (tb / nbn) * 64, (tb % nbn) * 64, store, As, Bs,
-                                add ? p.dw : nullptr, p.in_dim);
-  } else {
-    // bias_grad[out] (+)= column sums of g: 64 columns, four row lanes that meet in LDS
-    int const col = (bid - p.tiles_dx - p.tiles_dw) * 64 + (threadIdx.x & 63);
-    int const ry = threadIdx.x >> 6;
-    float s = 0.0f;
-    for (int row = ry; row < p.batch; row += 32) {  // eight loads in flight, added in row order
-      float2 v[8];
-#pragma unroll
-      for (int i = 0; i < 8; i++) v[i] = g_raw(row + 4 * i, col);
-#pragma unroll
-      for (int i = 0; i < 8; i++) s += row + 4 * i < p.batch ? g_val(v[i]) : 0.0f;
-    }
-    As[ry][threadIdx.x & 63] = s;
-    __syncthreads();
-    if (ry == 0 && col < p.out_dim) {
-      float const v = (As[0][threadIdx.x] + As[1][threadIdx.x]) + (As[2][threadIdx.x] + As[3][threadIdx.x]);
-      p.db[col] = (p.accumulate & FFK_ACC_BIAS) != 0 ? p.db[col] + v : v;
-    }
-  }
-}
-
-// Forward of a small fp32 Linear: output = act(input . weight^T + bias), one 64x64 tile per
-// workgroup, the same 64-deep reduction tiles.
 struct SmallLinearFwd {
   float const *x, *w, *bias;
   float *y;
   int batch, in_dim, out_dim, act;
 };
 
+// WAVES waves a workgroup; a tile of input_grad (reduction out_dim) takes SX of them, a tile of
+// weight_grad (reduction batch) all: a long batch over a small weight needs many waves a tile.
+template <int T, int ACT, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void linear_small_bwd_f32_kernel(SmallLinearBwd p) {
+  __shared__ SmallShared<T, WAVES> sm;
+  constexpr int SX = 4;
+  int const bid = blockIdx.x;
+  int const nbn = (p.in_dim + T - 1) / T;
+  auto no_bias = [](int, float) {};
+  if (bid < p.blocks_dx) {
+    // input_grad[batch, in] (+)= g[batch, out] . weight[out, in]
+    int const tile = bid * (WAVES / SX) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / SX;
+    int const tm = tile / nbn;
+    SmallOperand<true, ACT> const a = {p.dy, p.y, p.out_dim, p.relu_mode};
+    SmallOperand<false, FFK_ACT_NONE> const b = {p.w, nullptr, p.in_dim, 0};
+    auto store = [&](int m, int n, float v) { p.dx[(int64_t)m * p.in_dim + n] = v; };
+    small_tile<T, SX, WAVES>(a, b, p.batch, p.in_dim, p.out_dim, tm * T, (tile - tm * nbn) * T, tm * T < p.batch,
+                             (p.accumulate & FFK_ACC_INPUT) != 0 ? p.dx : nullptr, p.in_dim, store, false, no_bias, sm);
+  } else {
+    // weight_grad[out, in] (+)= g[batch, out]^T . input[batch, in]; bias_grad[out] (+)= column sums of g
+    int const tb = bid - p.blocks_dx;
+    SmallOperand<false, ACT> const a = {p.dy, p.y, p.out_dim, p.relu_mode};
+    SmallOperand<false, FFK_ACT_NONE> const b = {p.x, nullptr, p.in_dim, 0};
+    auto store = [&](int m, int n, float v) { p.dw[(int64_t)m * p.in_dim + n] = v; };
+    auto store_bias = [&](int m, float v) { p.db[m] = (p.accumulate & FFK_ACC_BIAS) != 0 ? p.db[m] + v : v; };
+    small_tile<T, WAVES, WAVES>(a, b, p.out_dim, p.in_dim, p.batch, (tb / nbn) * T, (tb % nbn) * T, true,
+                                (p.accumulate & FFK_ACC_WEIGHT) != 0 ? p.dw : nullptr, p.in_dim, store,
+                                p.db != nullptr && tb % nbn == 0, store_bias, sm);
+  }
+}
+
+// output = act(input . weight^T + bias)
+template <int T>
 __global__ __launch_bounds__(256) void linear_small_fwd_f32_kernel(SmallLinearFwd p) {
-  __shared__ float As[kSmallBK][68], Bs[kSmallBK][68];
-  int const nbn = (p.out_dim + 63) / 64;
-  auto a = [&](int m, int k) -> float {
-    return p.x[(int64_t)(m < p.batch ? m : p.batch - 1) * p.in_dim + (k < p.in_dim ? k : p.in_dim - 1)];
-  };
-  // weight is [out, in]: b(k, n) = weight[n][k], k contiguous like the input's
-  auto b = [&](int k, int n) -> float {
-    return p.w[(int64_t)(n < p.out_dim ? n : p.out_dim - 1) * p.in_dim + (k < p.in_dim ? k : p.in_dim - 1)];
-  };
+  __shared__ SmallShared<T, 4> sm;
+  int const nbn = (p.out_dim + T - 1) / T;
+  SmallOperand<true, FFK_ACT_NONE> const a = {p.x, nullptr, p.in_dim, 0}, b = {p.w, nullptr, p.in_dim, 0};
   auto store = [&](int m, int n, float v) {
     v += p.bias != nullptr ? p.bias[n] : 0.0f;
     switch (p.act) {
@@ -267,21 +146,45 @@ __global__ __launch_bounds__(256) void linear_small_fwd_f32_kernel(SmallLinearFw
     }
     p.y[(int64_t)m * p.out_dim + n] = v;
   };
-  small_f32_tile<true, true>(a, [](float v) { return v; }, b, p.batch, p.out_dim, p.in_dim, (blockIdx.x / nbn) * 64, (blockIdx.x % nbn) * 64, store, As, Bs);
+  small_tile<T, 4, 4>(a, b, p.batch, p.out_dim, p.in_dim, ((int)blockIdx.x / nbn) * T, ((int)blockIdx.x % nbn) * T, true,
+                      nullptr, 0, store, false, [](int, float) {}, sm);
 }
 
-// Small enough that launches, not work, set the time: at most two workgroups per CU in all.
-static bool small_linear_bwd(int dtype, int64_t batch, int64_t in_dim, int64_t out_dim, bool bias, int &tiles_dx,
-                             int &tiles_dw, int &blocks) {
-  // a tile's reduction (out_dim for the input gradient, batch for the weight gradient) stays short
-  if (dtype != FFK_FLOAT || batch > kSmallMaxDepth || out_dim > kSmallMaxDepth || in_dim > (1 << 20)) return false;
-  int64_t const tdx = ceil_div(batch, 64) * ceil_div(in_dim, 64), tdw = ceil_div(out_dim, 64) * ceil_div(in_dim, 64);
-  int64_t const tb = bias ? ceil_div(out_dim, 64) : 0;
-  if (tdx + tdw + tb > 2 * kNumCU) return false;
-  tiles_dx = (int)tdx;
-  tiles_dw = (int)tdw;
-  blocks = (int)(tdx + tdw + tb);
-  return true;
+// The tile (16, 32, or 0: the general kernels) of the one-launch forward.  Measured against the 64x64
+// tiles of the general kernel: 512 x 256 -> 512 6.0 us (12.3), 1024 x 512 -> 512 12.6 (19.4); at
+// 1024 x 1024 -> 1024 the wave tiles' operand traffic loses, 41 (30).  A few rows over a wide weight
+// are bound by reading it and keep these tiles.
+static int small_linear_fwd_tile(int64_t batch, int64_t in_dim, int64_t out_dim) {
+  if (in_dim > 1024 || batch >= (1 << 20) || out_dim >= (1 << 20)) return 0;
+  int64_t const area = batch * out_dim;
+  if (area <= 16 * 16 * 1024) return 16;
+  if (area <= 32 * 32 * 640 || (batch <= 32 && area <= 32 * 32 * 4096)) return 32;
+  return 0;
+}
+// The tile and the waves a workgroup of the one-launch backward.  A long batch over a small weight has
+// few tiles of weight_grad and a long reduction: sixteen waves share a tile there (8000 x 64 -> 64
+// 39 us, 860 with one workgroup of four waves a 128 x 64 tile).
+struct SmallBwdShape { int tile, waves; };
+static SmallBwdShape small_linear_bwd_shape(int dtype, int64_t batch, int64_t in_dim, int64_t out_dim) {
+  if (dtype != FFK_FLOAT || batch > 16384 || out_dim > 1024 || in_dim > 16384) return {0, 0};
+  int64_t const weights = out_dim * in_dim, both = (batch + out_dim) * in_dim;
+  if (batch <= 512 && both <= 16 * 16 * 1024) return {16, 4};
+  if (batch > 512 && weights <= 16 * 16 * 256) return {16, 16};
+  if (batch <= 1024 && both <= 32 * 32 * 2048) return {32, 4};
+  if (batch > 1024 && weights <= 32 * 32 * 256) return {32, 16};
+  return {0, 0};
+}
+template <int T, int WAVES>
+static void small_linear_bwd_launch(hipStream_t st, int activation, SmallLinearBwd p) {
+  int64_t const nbn = ceil_div(p.in_dim, T);
+  p.blocks_dx = (int)ceil_div(ceil_div(p.batch, T) * nbn, WAVES / 4);
+  int const blocks = p.blocks_dx + (int)(ceil_div(p.out_dim, T) * nbn);
+  switch (activation) {
+    case FFK_ACT_RELU: linear_small_bwd_f32_kernel<T, FFK_ACT_RELU, WAVES><<<blocks, WAVES * 64, 0, st>>>(p); break;
+    case FFK_ACT_SIGMOID: linear_small_bwd_f32_kernel<T, FFK_ACT_SIGMOID, WAVES><<<blocks, WAVES * 64, 0, st>>>(p); break;
+    case FFK_ACT_TANH: linear_small_bwd_f32_kernel<T, FFK_ACT_TANH, WAVES><<<blocks, WAVES * 64, 0, st>>>(p); break;
+    default: linear_small_bwd_f32_kernel<T, FFK_ACT_NONE, WAVES><<<blocks, WAVES * 64, 0, st>>>(p); break;
+  }
 }
 
 }  // namespace ffk
@@ -314,13 +217,17 @@ extern "C" int ffk_linear_forward(ffk_stream_t stream, int dtype,
   FFK_REQUIRE(batch > 0 && in_dim > 0 && out_dim > 0,
               "linear_forward: non-positive dimension");
   FFK_REQUIRE(input && output && weight, "linear_forward: NULL tensor");
-  if (dtype == FFK_FLOAT && batch <= 8192 && ceil_div(batch, 64) * ceil_div(out_dim, 64) <= 2 * kNumCU &&
-      in_dim <= kSmallMaxDepth) {
+  int const tile = dtype == FFK_FLOAT ? small_linear_fwd_tile(batch, in_dim, out_dim) : 0;
+  if (tile != 0) {
     SmallLinearFwd p = {static_cast<float const *>(input), static_cast<float const *>(weight),
                         static_cast<float const *>(bias), static_cast<float *>(output),
                         (int)batch, (int)in_dim, (int)out_dim, activation};
-    unsigned const blocks = (unsigned)(ceil_div(batch, 64) * ceil_div(out_dim, 64));
-    linear_small_fwd_f32_kernel<<<blocks, 256, 0, as_stream(stream)>>>(p);
+    unsigned const blocks = (unsigned)(ceil_div(batch, tile) * ceil_div(out_dim, tile));
+    if (tile == 16) {
+      linear_small_fwd_f32_kernel<16><<<blocks, 256, 0, as_stream(stream)>>>(p);
+    } else {
+      linear_small_fwd_f32_kernel<32><<<blocks, 256, 0, as_stream(stream)>>>(p);
+    }
     FFK_CHECK_LAUNCH();
     return FFK_OK;
   }
@@ -354,10 +261,10 @@ static int linear_backward_impl(
     FFK_REQUIRE(output != nullptr, "linear_backward: output needed for activation");
   }
   // a small fp32 problem whose three gradients are all asked for: one launch, no scratch
-  int tiles_dx = 0, tiles_dw = 0, blocks = 0;
-  if (input_tail == nullptr && input_grad != nullptr && weight_grad != nullptr &&
-      small_linear_bwd(dtype, batch, in_dim, out_dim, bias_grad != nullptr, tiles_dx, tiles_dw, blocks)) {
-    SmallLinearBwd p;
+  SmallBwdShape const small = input_tail == nullptr && input_grad != nullptr && weight_grad != nullptr
+                                  ? small_linear_bwd_shape(dtype, batch, in_dim, out_dim) : SmallBwdShape{0, 0};
+  if (small.tile != 0) {
+    SmallLinearBwd p = {};
     p.y = static_cast<float const *>(output);
     p.dy = static_cast<float const *>(output_grad);
     p.x = static_cast<float const *>(input);
@@ -368,16 +275,16 @@ static int linear_backward_impl(
     p.batch = (int)batch;
     p.in_dim = (int)in_dim;
     p.out_dim = (int)out_dim;
-    p.act = activation;
     p.relu_mode = relu_grad_mode;
     p.accumulate = accumulate;
-    p.tiles_dx = tiles_dx;
-    p.tiles_dw = tiles_dw;
-    switch (activation) {
-      case FFK_ACT_RELU: linear_small_bwd_f32_kernel<FFK_ACT_RELU><<<blocks, 256, 0, st>>>(p); break;
-      case FFK_ACT_SIGMOID: linear_small_bwd_f32_kernel<FFK_ACT_SIGMOID><<<blocks, 256, 0, st>>>(p); break;
-      case FFK_ACT_TANH: linear_small_bwd_f32_kernel<FFK_ACT_TANH><<<blocks, 256, 0, st>>>(p); break;
-      default: linear_small_bwd_f32_kernel<FFK_ACT_NONE><<<blocks, 256, 0, st>>>(p); break;
+    if (small.tile == 16 && small.waves == 16) {
+      small_linear_bwd_launch<16, 16>(st, activation, p);
+    } else if (small.tile == 16) {
+      small_linear_bwd_launch<16, 4>(st, activation, p);
+    } else if (small.waves == 16) {
+      small_linear_bwd_launch<32, 16>(st, activation, p);
+    } else {
+      small_linear_bwd_launch<32, 4>(st, activation, p);
     }
     FFK_CHECK_LAUNCH();
     return FFK_OK;

@@ -95,3 +95,52 @@ def test_values_next_to_the_edge_stay_out(ffk):
         rows = torch.isinf(C).any(1)
         assert bool(rows[5]) and int(rows.sum()) == 1 and not bool(torch.isnan(C).any())
         assert bool((C[torch.arange(M, device="cuda") != 5] == K).all())
+
+
+# fp32: lengths that are no multiple of four around the 64 and 128 tiles, and reductions of thousands
+# over few outputs (sixteen waves a tile)
+F32_ANY = [(130, 129, 33), (257, 1001, 65), (63, 300, 7), (1100, 2051, 70)]
+F32_DEEP = [(25, 100, 5003), (1, 17, 2048), (250, 500, 2051), (16, 16, 4096)]
+
+
+@pytest.mark.parametrize("ta,tb", KINDS)
+@pytest.mark.parametrize("mnk", F32_ANY + F32_DEEP)
+def test_gemm_fp32_any_lengths(ffk, oracle, ta, tb, mnk):
+    M, N, K = mnk
+    print("gemm fp32 any lengths", mnk, "ta", ta, "tb", tb, flush=True)
+    assert ffk.gemm_kernel_name(ffk.FLOAT, ta, tb, M, N, K).startswith(
+        "gemm_f32_deep" if mnk in F32_DEEP else "gemm_f32_tiled" if M * N >= 128 * 128 else "gemm_f32_kernel")
+    g = rng(M * 7 + N * 3 + K)
+    A = g.standard_normal((K, M) if ta else (M, K)).astype(np.float32)
+    B = g.standard_normal((N, K) if tb else (K, N)).astype(np.float32)
+    want = oracle.gemm_f64(A, B, ta, tb)
+    buf = torch.full((M * N + 16,), 7.0, device="cuda")
+    C = buf[8:8 + M * N].view(M, N)
+    ffk.gemm(to_dev(A, torch), to_dev(B, torch), C, ta, tb)
+    assert_close(to_np(C), want, 1e-5, "C")
+    ffk.gemm(to_dev(A, torch), to_dev(B, torch), C, ta, tb, accumulate=True)
+    assert_close(to_np(C), 2 * want, 1e-5, "C accumulate")
+    assert bool((buf[:8] == 7.0).all()) and bool((buf[8 + M * N:] == 7.0).all())
+
+
+# one per tile and wave count of the one-launch Linear kernels, sizes off every multiple of theirs
+@pytest.mark.parametrize("shape", [(17, 33, 15), (3, 130, 77), (513, 41, 59), (1025, 65, 99), (601, 530, 501), (1030, 499, 510),
+                                   (31, 1000, 5001)])
+@pytest.mark.parametrize("act", [-1, 0, 2])
+def test_linear_fp32_small_tiles(ffk, oracle, shape, act):
+    batch, in_dim, out_dim = shape
+    print("linear fp32 small", shape, "act", act, flush=True)
+    g = rng(batch)
+    x = g.uniform(-1, 1, (batch, in_dim)).astype(np.float32)
+    w = (g.standard_normal((out_dim, in_dim)) * 0.2).astype(np.float32)
+    b = (g.standard_normal((out_dim,)) * 0.2).astype(np.float32)
+    dy = g.standard_normal((batch, out_dim)).astype(np.float32)
+    y_ref = oracle.linear_forward(x, w, b, activation=act)
+    xd, wd, bd, dyd = (to_dev(a, torch) for a in (x, w, b, dy))
+    y = ffk.linear_forward(xd, wd, bd, activation=act)
+    assert_close(to_np(y), y_ref, 1e-5, "y")
+    dx_ref, dw_ref, db_ref = oracle.linear_backward(y_ref, dy, x, w, activation=act)
+    got = [torch.full_like(t, 0.5) for t in (xd, wd, bd)]
+    ffk.linear_backward(to_dev(y_ref, torch), dyd, xd, wd, *got, activation=act, accumulate=True)
+    for t, want, name in zip(got, (dx_ref, dw_ref, db_ref), ("dx", "dw", "db")):
+        assert_close(to_np(t), want + 0.5, 1e-5, name)
