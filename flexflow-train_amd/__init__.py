@@ -11,6 +11,7 @@ The directory name contains a hyphen, so load it with
 (see ``tests/conftest.py``).
 """
 import ctypes
+import importlib.util
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -227,6 +228,30 @@ def check(rc):
         raise FFKError("ffk error %d: %s" % (rc, lib().ffk_last_error().decode()))
 
 
+class _Call:
+    """The entry points on tensors and the current stream (csrc/python_call.cc), loaded when the
+    first one is asked for: `_call.ffk_x(...)` takes ffk_x's arguments behind the stream, tensors and
+    descriptors as they are, and raises FFKError for a non-zero status.  Size queries return their
+    bytes.  No fallback: without the built module an entry point fails."""
+
+    def __getattr__(self, name):
+        lib()
+        _torch()
+        path = os.path.join(HERE, "_ffk_call.so")
+        if not os.path.exists(path):
+            raise FFKError("_ffk_call.so is missing at %s: build it with "
+                           "`python flexflow-train_amd/build.py` (there is no fallback path)" % path)
+        spec = importlib.util.spec_from_file_location("_ffk_call", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        module.set_error(FFKError)
+        self.__dict__.update({k: v for k, v in vars(module).items() if k.startswith("ffk_")})
+        return self.__dict__[name]
+
+
+_call = _Call()
+
+
 # --------------------------------------------------------------------------
 # torch-tensor helpers
 # --------------------------------------------------------------------------
@@ -236,12 +261,16 @@ def _torch():
     return torch
 
 
+_dtypes = {}
+
+
 def dtype_of(t):
-    torch = _torch()
-    table = {torch.float32: FLOAT, torch.bfloat16: BF16, torch.int32: INT32,
-             torch.int64: INT64, torch.float16: HALF, torch.float64: DOUBLE,
-             torch.bool: BOOL}
-    return table[t.dtype]
+    if not _dtypes:
+        torch = _torch()
+        _dtypes.update({torch.float32: FLOAT, torch.bfloat16: BF16, torch.int32: INT32,
+                        torch.int64: INT64, torch.float16: HALF, torch.float64: DOUBLE,
+                        torch.bool: BOOL})
+    return _dtypes[t.dtype]
 
 
 def ptr(t):
@@ -258,8 +287,7 @@ def current_stream():
 def probe_mfma_bf16(iterations, out, seed=1):
     """Launches the matrix-rate probe on the current stream; returns the flops of the launch."""
     flops = ctypes.c_double()
-    check(lib().ffk_probe_mfma_bf16(current_stream(), iterations, seed, ptr(out), out.numel() * out.element_size(),
-                                    ctypes.byref(flops)))
+    _call.ffk_probe_mfma_bf16(iterations, seed, out, out.numel() * out.element_size(), flops)
     return flops.value
 
 
@@ -269,8 +297,7 @@ def linear_forward(x, w, b=None, activation=ACT_NONE, out=None):
     out_dim = w.shape[0]
     if out is None:
         out = torch.empty((batch, out_dim), dtype=x.dtype, device=x.device)
-    check(lib().ffk_linear_forward(current_stream(), dtype_of(x), activation, ptr(x), ptr(out),
-                                   ptr(w), ptr(b), batch, in_dim, out_dim))
+    _call.ffk_linear_forward(dtype_of(x), activation, x, out, w, b, batch, in_dim, out_dim)
     return out
 
 
@@ -280,15 +307,12 @@ def linear_backward(y, dy, x, w, dx=None, dw=None, db=None, activation=ACT_NONE,
     batch, in_dim = x.shape
     out_dim = w.shape[0]
     if workspace is None:
-        need = lib().ffk_linear_backward_workspace_bytes(dtype_of(x), activation,
+        need = _call.ffk_linear_backward_workspace_bytes(dtype_of(x), activation,
                                                          int(db is not None), batch, out_dim)
         if need:
             workspace = torch.empty((need,), dtype=torch.uint8, device=x.device)
     ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    check(lib().ffk_linear_backward(current_stream(), dtype_of(x), activation, relu_grad_mode,
-                                    ptr(y), ptr(dy), ptr(x), ptr(dx), ptr(w), ptr(dw), ptr(db),
-                                    batch, in_dim, out_dim, ptr(workspace), ws_bytes,
-                                    7 if accumulate is True else int(accumulate)))
+    _call.ffk_linear_backward(dtype_of(x), activation, relu_grad_mode, y, dy, x, dx, w, dw, db, batch, in_dim, out_dim, workspace, ws_bytes, 7 if accumulate is True else int(accumulate))
     return dx, dw, db
 
 
@@ -301,7 +325,7 @@ def gemm_kernel_name(dtype, trans_a, trans_b, M, N, K, has_bias=False, activatio
 
 def linear_l2_regularizer_grad(w, dw, lam):
     """dw = dw + lam * w in place (the L2 regulariser's term of Linear's weight gradient)."""
-    check(lib().ffk_linear_l2_regularizer_grad(current_stream(), dtype_of(w), ptr(w), ptr(dw), w.numel(), lam))
+    _call.ffk_linear_l2_regularizer_grad(dtype_of(w), w, dw, w.numel(), lam)
     return dw
 
 
@@ -313,8 +337,7 @@ def linear_gelu_dropout_forward(x, w, b, rate, seed, offset=0):
     out_dim = w.shape[0]
     y = torch.empty((batch, out_dim), dtype=x.dtype, device=x.device)
     dropped = torch.empty_like(y)
-    check(lib().ffk_linear_gelu_dropout_forward(current_stream(), dtype_of(x), ptr(x), ptr(y), ptr(dropped),
-                                                ptr(w), ptr(b), batch, in_dim, out_dim, rate, seed, offset))
+    _call.ffk_linear_gelu_dropout_forward(dtype_of(x), x, y, dropped, w, b, batch, in_dim, out_dim, rate, seed, offset)
     return y, dropped
 
 
@@ -324,8 +347,7 @@ def linear_dropout_add_forward(x, residual, w, b, rate, seed, offset=0):
     batch, in_dim = x.shape
     out_dim = w.shape[0]
     y = torch.empty((batch, out_dim), dtype=x.dtype, device=x.device)
-    check(lib().ffk_linear_dropout_add_forward(current_stream(), dtype_of(x), ptr(x), ptr(residual), ptr(y),
-                                               ptr(w), ptr(b), batch, in_dim, out_dim, rate, seed, offset))
+    _call.ffk_linear_dropout_add_forward(dtype_of(x), x, residual, y, w, b, batch, in_dim, out_dim, rate, seed, offset)
     return y
 
 
@@ -335,11 +357,9 @@ def linear_backward_dropout_gelu(dy, x, gelu_input, w, rate, seed, offset=0, dw=
     batch, in_dim = x.shape
     out_dim = w.shape[0]
     dx = torch.empty_like(x)
-    need = lib().ffk_linear_backward_workspace_bytes(dtype_of(x), ACT_NONE, int(db is not None), batch, out_dim)
+    need = _call.ffk_linear_backward_workspace_bytes(dtype_of(x), ACT_NONE, int(db is not None), batch, out_dim)
     workspace = torch.empty((max(need, 1),), dtype=torch.uint8, device=x.device)
-    check(lib().ffk_linear_backward_dropout_gelu(current_stream(), dtype_of(x), ptr(dy), ptr(x), ptr(gelu_input),
-                                                 ptr(dx), ptr(w), ptr(dw), ptr(db), batch, in_dim, out_dim,
-                                                 ptr(workspace), need, int(accumulate), rate, seed, offset))
+    _call.ffk_linear_backward_dropout_gelu(dtype_of(x), dy, x, gelu_input, dx, w, dw, db, batch, in_dim, out_dim, workspace, need, int(accumulate), rate, seed, offset)
     return dx
 
 
@@ -350,14 +370,11 @@ def linear_backward_dropout_gelu_bias_grad(dy, x, gelu_input, w, rate, seed, gel
     batch, in_dim = x.shape
     out_dim = w.shape[0]
     dx = torch.empty_like(x)
-    need = lib().ffk_linear_backward_workspace_bytes(dtype_of(x), ACT_NONE, int(db is not None), batch, out_dim)
+    need = _call.ffk_linear_backward_workspace_bytes(dtype_of(x), ACT_NONE, int(db is not None), batch, out_dim)
     workspace = torch.empty((max(need, 1),), dtype=torch.uint8, device=x.device)
-    need2 = lib().ffk_dropout_backward_bias_grad_workspace_bytes(batch, in_dim)
+    need2 = _call.ffk_dropout_backward_bias_grad_workspace_bytes(batch, in_dim)
     workspace2 = torch.empty((need2,), dtype=torch.uint8, device=x.device)
-    check(lib().ffk_linear_backward_dropout_gelu_bias_grad(
-        current_stream(), dtype_of(x), ptr(dy), ptr(x), ptr(gelu_input), ptr(dx), ptr(w), ptr(dw), ptr(db), batch,
-        in_dim, out_dim, ptr(workspace), need, int(accumulate), rate, seed, offset, ptr(gelu_bias_grad),
-        int(accumulate_gelu_bias), ptr(workspace2), need2))
+    _call.ffk_linear_backward_dropout_gelu_bias_grad(dtype_of(x), dy, x, gelu_input, dx, w, dw, db, batch, in_dim, out_dim, workspace, need, int(accumulate), rate, seed, offset, gelu_bias_grad, int(accumulate_gelu_bias), workspace2, need2)
     return dx
 
 
@@ -366,19 +383,16 @@ def dropout_backward_bias_grad(dy, rate, seed, bias_grad, offset=0, accumulate_b
     torch = _torch()
     batch, out_dim = dy.shape
     dx = torch.empty_like(dy)
-    need = lib().ffk_dropout_backward_bias_grad_workspace_bytes(batch, out_dim)
+    need = _call.ffk_dropout_backward_bias_grad_workspace_bytes(batch, out_dim)
     workspace = torch.empty((need,), dtype=torch.uint8, device=dy.device)
-    check(lib().ffk_dropout_backward_bias_grad(current_stream(), dtype_of(dy), ptr(dy), ptr(dx), batch, out_dim,
-                                               ptr(bias_grad), int(accumulate_bias), ptr(workspace), need, rate, seed,
-                                               offset))
+    _call.ffk_dropout_backward_bias_grad(dtype_of(dy), dy, dx, batch, out_dim, bias_grad, int(accumulate_bias), workspace, need, rate, seed, offset)
     return dx
 
 
 def gemm(A, B, C, trans_a=False, trans_b=False, accumulate=False):
     M, N = C.shape
     K = A.shape[0] if trans_a else A.shape[1]
-    check(lib().ffk_gemm(current_stream(), dtype_of(A), int(trans_a), int(trans_b), M, N, K,
-                         ptr(A), ptr(B), ptr(C), int(accumulate)))
+    _call.ffk_gemm(dtype_of(A), int(trans_a), int(trans_b), M, N, K, A, B, C, int(accumulate))
     return C
 
 
@@ -386,14 +400,12 @@ def element_unary_forward(op, x, scalar=0.0, out=None):
     torch = _torch()
     if out is None:
         out = torch.empty_like(x)
-    check(lib().ffk_element_unary_forward(current_stream(), dtype_of(x), op, scalar, ptr(x),
-                                          ptr(out), x.numel()))
+    _call.ffk_element_unary_forward(dtype_of(x), op, scalar, x, out, x.numel())
     return out
 
 
 def element_unary_backward(op, y, dy, x, dx, scalar=0.0, accumulate=-1):
-    check(lib().ffk_element_unary_backward(current_stream(), dtype_of(x), op, scalar, ptr(y),
-                                           ptr(dy), ptr(x), ptr(dx), x.numel(), accumulate))
+    _call.ffk_element_unary_backward(dtype_of(x), op, scalar, y, dy, x, dx, x.numel(), accumulate)
     return dx
 
 
@@ -401,23 +413,18 @@ def element_binary_forward(op, l, r, out=None):
     torch = _torch()
     if out is None:
         out = torch.empty_like(l if l.numel() >= r.numel() else r)
-    check(lib().ffk_element_binary_forward(current_stream(), dtype_of(out), op, ptr(l), ptr(r),
-                                           ptr(out), out.numel(), l.numel(), r.numel()))
+    _call.ffk_element_binary_forward(dtype_of(out), op, l, r, out, out.numel(), l.numel(), r.numel())
     return out
 
 
 def element_binary_backward(op, g, l, r, dl, dr, accumulate=False):
-    check(lib().ffk_element_binary_backward(current_stream(), dtype_of(g), op, ptr(g), ptr(l),
-                                            ptr(r), ptr(dl), ptr(dr), g.numel(),
-                                            int(accumulate)))
+    _call.ffk_element_binary_backward(dtype_of(g), op, g, l, r, dl, dr, g.numel(), int(accumulate))
     return dl, dr
 
 
 def element_binary_backward_broadcast(op, g, l, r, dl, dr, accumulate=False):
     """Backward with operands that were broadcast over the leading dims; dl / dr may be None."""
-    check(lib().ffk_element_binary_backward_broadcast(
-        current_stream(), dtype_of(g), op, ptr(g), ptr(l), ptr(r), ptr(dl) if dl is not None else None,
-        ptr(dr) if dr is not None else None, g.numel(), l.numel(), r.numel(), int(accumulate)))
+    _call.ffk_element_binary_backward_broadcast(dtype_of(g), op, g, l, r, dl, dr, g.numel(), l.numel(), r.numel(), int(accumulate))
     return dl, dr
 
 
@@ -430,8 +437,7 @@ def layer_norm_forward(x, gamma, beta, eps, out=None, mean=None, rstd=None):
         mean = torch.empty((M,), dtype=torch.float32, device=x.device)
     if rstd is None:
         rstd = torch.empty((M,), dtype=torch.float32, device=x.device)
-    check(lib().ffk_layer_norm_forward(current_stream(), dtype_of(x), ptr(x), ptr(out),
-                                       ptr(gamma), ptr(beta), ptr(mean), ptr(rstd), M, N, eps))
+    _call.ffk_layer_norm_forward(dtype_of(x), x, out, gamma, beta, mean, rstd, M, N, eps)
     return out, mean, rstd
 
 
@@ -443,22 +449,17 @@ def layer_norm_backward(dy, x, mean, rstd, gamma, dx, dgamma, dbeta, accumulate=
                         workspace=None):
     torch = _torch()
     M, N = x.shape
-    need = lib().ffk_layer_norm_backward_workspace_bytes(M, N)
     if workspace is None:
+        need = _call.ffk_layer_norm_backward_workspace_bytes(M, N)
         workspace = torch.empty((need,), dtype=torch.uint8, device=x.device)
-    check(lib().ffk_layer_norm_backward(current_stream(), dtype_of(x), ptr(dy), ptr(x),
-                                        ptr(mean), ptr(rstd), ptr(gamma), ptr(dx), ptr(dgamma),
-                                        ptr(dbeta), M, N, ptr(workspace), workspace.numel(),
-                                        int(accumulate)))
+    _call.ffk_layer_norm_backward(dtype_of(x), dy, x, mean, rstd, gamma, dx, dgamma, dbeta, M, N, workspace, workspace.numel(), int(accumulate))
     return dx, dgamma, dbeta
 
 
 def layer_norm_backward_static(dy, x, mean, rstd, gamma, dx, dgamma, dbeta, accumulate=False):
     """ffk_layer_norm_backward without a workspace: the library's own per-device array."""
     M, N = x.shape
-    check(lib().ffk_layer_norm_backward_static(current_stream(), dtype_of(x), ptr(dy), ptr(x),
-                                               ptr(mean), ptr(rstd), ptr(gamma), ptr(dx),
-                                               ptr(dgamma), ptr(dbeta), M, N, int(accumulate)))
+    _call.ffk_layer_norm_backward_static(dtype_of(x), dy, x, mean, rstd, gamma, dx, dgamma, dbeta, M, N, int(accumulate))
     return dx, dgamma, dbeta
 
 
@@ -468,12 +469,9 @@ def layer_norm_backward_residual(dy, x, mean, rstd, gamma, residual, dx, dgamma,
     torch = _torch()
     M, N = x.shape
     if workspace is None:
-        workspace = torch.empty((lib().ffk_layer_norm_backward_workspace_bytes(M, N),), dtype=torch.uint8,
+        workspace = torch.empty((_call.ffk_layer_norm_backward_workspace_bytes(M, N),), dtype=torch.uint8,
                                 device=x.device)
-    check(lib().ffk_layer_norm_backward_residual(current_stream(), dtype_of(x), ptr(dy), ptr(x), ptr(mean), ptr(rstd),
-                                                 ptr(gamma), ptr(residual), ptr(dx), ptr(dgamma), ptr(dbeta), M, N,
-                                                 ptr(workspace), workspace.numel(), int(accumulate_params),
-                                                 ptr(dropped), rate, seed, offset))
+    _call.ffk_layer_norm_backward_residual(dtype_of(x), dy, x, mean, rstd, gamma, residual, dx, dgamma, dbeta, M, N, workspace, workspace.numel(), int(accumulate_params), dropped, rate, seed, offset)
     return dx, dgamma, dbeta
 
 
@@ -484,9 +482,7 @@ def dropout_add_layer_norm_forward(x, residual, gamma, beta, eps, rate, seed, of
     total, y = torch.empty_like(x), torch.empty_like(x)
     mean = torch.empty((M,), dtype=torch.float32, device=x.device)
     rstd = torch.empty((M,), dtype=torch.float32, device=x.device)
-    check(lib().ffk_dropout_add_layer_norm_forward(current_stream(), dtype_of(x), ptr(x), ptr(residual), ptr(total),
-                                                   ptr(y), ptr(gamma), ptr(beta), ptr(mean), ptr(rstd), M, N, eps,
-                                                   rate, seed, offset))
+    _call.ffk_dropout_add_layer_norm_forward(dtype_of(x), x, residual, total, y, gamma, beta, mean, rstd, M, N, eps, rate, seed, offset)
     return total, y, mean, rstd
 
 
@@ -494,8 +490,7 @@ def softmax_forward(x, outer, dim, inner, out=None):
     torch = _torch()
     if out is None:
         out = torch.empty_like(x)
-    check(lib().ffk_softmax_forward(current_stream(), dtype_of(x), ptr(x), ptr(out), outer, dim,
-                                    inner))
+    _call.ffk_softmax_forward(dtype_of(x), x, out, outer, dim, inner)
     return out
 
 
@@ -503,8 +498,7 @@ def softmax_backward(y, dy, outer, dim, inner, dx=None):
     torch = _torch()
     if dx is None:
         dx = torch.empty_like(y)
-    check(lib().ffk_softmax_backward(current_stream(), dtype_of(y), ptr(y), ptr(dy), ptr(dx),
-                                     outer, dim, inner))
+    _call.ffk_softmax_backward(dtype_of(y), y, dy, dx, outer, dim, inner)
     return dx
 
 
@@ -512,8 +506,7 @@ def softmax_backward_copy(dy, dx=None):
     torch = _torch()
     if dx is None:
         dx = torch.empty_like(dy)
-    check(lib().ffk_softmax_backward_copy(current_stream(), dtype_of(dy), ptr(dy), ptr(dx),
-                                          dy.numel()))
+    _call.ffk_softmax_backward_copy(dtype_of(dy), dy, dx, dy.numel())
     return dx
 
 
@@ -521,8 +514,7 @@ def dropout_forward(x, rate, seed, offset=0, out=None):
     torch = _torch()
     if out is None:
         out = torch.empty_like(x)
-    check(lib().ffk_dropout_forward(current_stream(), dtype_of(x), ptr(x), ptr(out), x.numel(),
-                                    rate, seed, offset))
+    _call.ffk_dropout_forward(dtype_of(x), x, out, x.numel(), rate, seed, offset)
     return out
 
 
@@ -530,38 +522,35 @@ def dropout_backward(dy, rate, seed, offset=0, dx=None, accumulate=False):
     torch = _torch()
     if dx is None:
         dx = torch.empty_like(dy)
-    check(lib().ffk_dropout_backward(current_stream(), dtype_of(dy), ptr(dy), ptr(dx),
-                                     dy.numel(), rate, seed, offset, int(accumulate)))
+    _call.ffk_dropout_backward(dtype_of(dy), dy, dx, dy.numel(), rate, seed, offset, int(accumulate))
     return dx
 
 
 def dropout_add_forward(x, residual, rate, seed, offset=0):
     """residual + dropout(x), one pass."""
     out = _torch().empty_like(x)
-    check(lib().ffk_dropout_add_forward(current_stream(), dtype_of(x), ptr(x), ptr(residual), ptr(out), x.numel(),
-                                        rate, seed, offset))
+    _call.ffk_dropout_add_forward(dtype_of(x), x, residual, out, x.numel(), rate, seed, offset)
     return out
 
 
 def gelu_dropout_forward(x, rate, seed, offset=0):
     """dropout(GELU(x)), one pass."""
     out = _torch().empty_like(x)
-    check(lib().ffk_gelu_dropout_forward(current_stream(), dtype_of(x), ptr(x), ptr(out), x.numel(), rate, seed, offset))
+    _call.ffk_gelu_dropout_forward(dtype_of(x), x, out, x.numel(), rate, seed, offset)
     return out
 
 
 def dropout_gelu_backward(dy, gelu_input, rate, seed, offset=0):
     """dropout_backward(dy) * GELU'(gelu_input), one pass."""
     dx = _torch().empty_like(dy)
-    check(lib().ffk_dropout_gelu_backward(current_stream(), dtype_of(dy), ptr(dy), ptr(gelu_input), ptr(dx),
-                                          dy.numel(), rate, seed, offset))
+    _call.ffk_dropout_gelu_backward(dtype_of(dy), dy, gelu_input, dx, dy.numel(), rate, seed, offset)
     return dx
 
 
 def dropout_mask(n, rate, seed, offset=0, device="cuda"):
     torch = _torch()
     m = torch.empty((n,), dtype=torch.uint8, device=device)
-    check(lib().ffk_dropout_mask(current_stream(), ptr(m), n, rate, seed, offset))
+    _call.ffk_dropout_mask(m, n, rate, seed, offset)
     return m
 
 
@@ -569,18 +558,14 @@ def sgd_update(weight, grad, lr, momentum=0.0, nesterov=False, weight_decay=0.0,
                num_replicas=1, weight_lowp=None):
     """In-place SGD step on fp32 `weight` (and `sgd_v`); grad is [num_replicas * n] fp32 or bf16."""
     n = weight.numel()
-    check(lib().ffk_sgd_update(current_stream(), dtype_of(grad), lr, momentum, int(nesterov),
-                               weight_decay, ptr(grad), n, num_replicas, ptr(weight), ptr(sgd_v),
-                               ptr(weight_lowp)))
+    _call.ffk_sgd_update(dtype_of(grad), lr, momentum, int(nesterov), weight_decay, grad, n, num_replicas, weight, sgd_v, weight_lowp)
     return weight
 
 
 def adam_update(weight, grad, adam_m, adam_v, alpha_t, beta1=0.9, beta2=0.999, weight_decay=0.0,
                 epsilon=1e-8, num_replicas=1, weight_lowp=None):
     n = weight.numel()
-    check(lib().ffk_adam_update(current_stream(), dtype_of(grad), alpha_t, beta1, beta2, weight_decay,
-                                epsilon, ptr(grad), n, num_replicas, ptr(weight), ptr(adam_v),
-                                ptr(adam_m), ptr(weight_lowp)))
+    _call.ffk_adam_update(dtype_of(grad), alpha_t, beta1, beta2, weight_decay, epsilon, grad, n, num_replicas, weight, adam_v, adam_m, weight_lowp)
     return weight
 
 
@@ -589,9 +574,7 @@ def sparse_categorical_crossentropy_loss_backward(logit, label, num_samples, num
     torch = _torch()
     if out is None:
         out = torch.empty_like(logit)
-    check(lib().ffk_sparse_categorical_crossentropy_loss_backward(
-        current_stream(), ptr(out), ptr(logit), ptr(label), logit.numel(), out.numel(), num_samples,
-        num_classes, k, scale_factor))
+    _call.ffk_sparse_categorical_crossentropy_loss_backward(out, logit, label, logit.numel(), out.numel(), num_samples, num_classes, k, scale_factor)
     return out
 
 
@@ -600,9 +583,7 @@ def difference_loss_backward(kind, logit, label, scale_factor, out=None):
     torch = _torch()
     if out is None:
         out = torch.empty_like(logit)
-    fn = getattr(lib(), "ffk_%s_loss_backward" % kind)
-    check(fn(current_stream(), ptr(out), ptr(logit), ptr(label), logit.numel(), out.numel(),
-             scale_factor))
+    getattr(_call, "ffk_%s_loss_backward" % kind)(out, logit, label, logit.numel(), out.numel(), scale_factor)
     return out
 
 
@@ -610,20 +591,17 @@ def identity_loss_backward(loss, scale_factor, out=None):
     torch = _torch()
     if out is None:
         out = torch.empty_like(loss)
-    check(lib().ffk_identity_loss_backward(current_stream(), ptr(out), ptr(loss), loss.numel(),
-                                           out.numel(), scale_factor))
+    _call.ffk_identity_loss_backward(out, loss, loss.numel(), out.numel(), scale_factor)
     return out
 
 
 def cast_forward(x, out):
-    check(lib().ffk_cast_forward(current_stream(), dtype_of(x), dtype_of(out), ptr(x), ptr(out),
-                                 x.numel()))
+    _call.ffk_cast_forward(dtype_of(x), dtype_of(out), x, out, x.numel())
     return out
 
 
 def cast_backward(out_grad, in_grad):
-    check(lib().ffk_cast_backward(current_stream(), dtype_of(out_grad), dtype_of(in_grad),
-                                  ptr(out_grad), ptr(in_grad), out_grad.numel()))
+    _call.ffk_cast_backward(dtype_of(out_grad), dtype_of(in_grad), out_grad, in_grad, out_grad.numel())
     return in_grad
 
 
@@ -637,9 +615,7 @@ def embedding_forward(indices, weight, aggr=AGGR_NONE, out_dtype=None):
         num_bags = indices.numel() // bag
     out_dtype = out_dtype or weight.dtype
     out = torch.empty((num_bags, D), dtype=out_dtype, device=weight.device)
-    check(lib().ffk_embedding_forward(current_stream(), dtype_of(indices), dtype_of(weight),
-                                      dtype_of(out), ptr(indices), ptr(out), ptr(weight), aggr,
-                                      num_bags, bag, D, V))
+    _call.ffk_embedding_forward(dtype_of(indices), dtype_of(weight), dtype_of(out), indices, out, weight, aggr, num_bags, bag, D, V)
     return out
 
 
@@ -657,13 +633,10 @@ def embedding_backward(indices, out_grad, weight_grad, aggr=AGGR_NONE, determini
     ws = None
     ws_bytes = 0
     if workspace or deterministic:
-        ws_bytes = lib().ffk_embedding_backward_workspace_bytes(num_bags * bag, V)
+        ws_bytes = _call.ffk_embedding_backward_workspace_bytes(num_bags * bag, V)
         if ws_bytes:
             ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=weight_grad.device)
-    check(lib().ffk_embedding_backward(current_stream(), dtype_of(indices), dtype_of(out_grad),
-                                       ptr(indices), ptr(out_grad), ptr(weight_grad), aggr,
-                                       num_bags, bag, D, V, int(deterministic), ptr(ws),
-                                       ws_bytes))
+    _call.ffk_embedding_backward(dtype_of(indices), dtype_of(out_grad), indices, out_grad, weight_grad, aggr, num_bags, bag, D, V, int(deterministic), ws, ws_bytes)
     return weight_grad
 
 
@@ -676,8 +649,7 @@ def embedding_backward_typed(indices, out_grad, weight_grad, aggr=AGGR_NONE):
     else:
         bag = indices.shape[-1]
         num_bags = indices.numel() // bag
-    check(lib().ffk_embedding_backward_typed(current_stream(), dtype_of(indices), dtype_of(out_grad), ptr(indices),
-                                             ptr(out_grad), ptr(weight_grad), aggr, num_bags, bag, D, V))
+    _call.ffk_embedding_backward_typed(dtype_of(indices), dtype_of(out_grad), indices, out_grad, weight_grad, aggr, num_bags, bag, D, V)
     return weight_grad
 
 
@@ -695,8 +667,7 @@ def attention_forward(q, k, v, scale, causal, desc=None):
     desc = desc or attention_desc_bshd(q, k, scale, causal, v)
     o = torch.empty(tuple(q.shape[:3]) + (v.shape[3],), dtype=q.dtype, device=q.device)
     lse = torch.empty((desc.batch, desc.heads, desc.seq_q), dtype=torch.float32, device=q.device)
-    check(lib().ffk_attention_forward(current_stream(), dtype_of(q), ctypes.byref(desc), ptr(q),
-                                      ptr(k), ptr(v), ptr(o), ptr(lse)))
+    _call.ffk_attention_forward(dtype_of(q), desc, q, k, v, o, lse)
     return o, lse
 
 
@@ -707,9 +678,7 @@ def attention_backward(q, k, v, o, d_o, lse, scale, causal, desc=None):
     dk = torch.empty_like(k)
     dv = torch.empty_like(v)
     delta = torch.empty_like(lse)
-    check(lib().ffk_attention_backward(current_stream(), dtype_of(q), ctypes.byref(desc), ptr(q),
-                                       ptr(k), ptr(v), ptr(o), ptr(d_o), ptr(lse), ptr(delta),
-                                       ptr(dq), ptr(dk), ptr(dv)))
+    _call.ffk_attention_backward(dtype_of(q), desc, q, k, v, o, d_o, lse, delta, dq, dk, dv)
     return dq, dk, dv
 
 
@@ -725,7 +694,7 @@ MHA_ACC_INPUT_GRADS, MHA_OVERWRITE_WEIGHT_GRAD = 1, 2
 
 def mha_reserve(desc, dtype, device="cuda"):
     torch = _torch()
-    n = lib().ffk_mha_reserve_bytes(ctypes.byref(desc), dtype)
+    n = _call.ffk_mha_reserve_bytes(desc, dtype)
     return torch.empty((n,), dtype=torch.uint8, device=device)
 
 
@@ -734,18 +703,13 @@ def mha_forward(desc, query, key, value, weight, reserve, out=None):
     if out is None:
         out = torch.empty((desc.num_samples, desc.qo_seq_length, desc.o_proj_size),
                           dtype=query.dtype, device=query.device)
-    check(lib().ffk_mha_forward(current_stream(), dtype_of(query), ctypes.byref(desc), ptr(query),
-                                ptr(key), ptr(value), ptr(weight), ptr(out), ptr(reserve),
-                                reserve.numel()))
+    _call.ffk_mha_forward(dtype_of(query), desc, query, key, value, weight, out, reserve, reserve.numel())
     return out
 
 
 def mha_backward(desc, query, dquery, key, dkey, value, dvalue, weight, dweight, out_grad,
                  reserve, accumulate=False):
-    check(lib().ffk_mha_backward(current_stream(), dtype_of(query), ctypes.byref(desc),
-                                 ptr(query), ptr(dquery), ptr(key), ptr(dkey), ptr(value),
-                                 ptr(dvalue), ptr(weight), ptr(dweight), ptr(out_grad),
-                                 ptr(reserve), reserve.numel(), int(accumulate)))
+    _call.ffk_mha_backward(dtype_of(query), desc, query, dquery, key, dkey, value, dvalue, weight, dweight, out_grad, reserve, reserve.numel(), int(accumulate))
     return dquery, dkey, dvalue, dweight
 
 
@@ -768,21 +732,17 @@ def encoder_layer_params(tensors):
 
 def encoder_layer_workspace(desc, dtype, device="cuda"):
     torch = _torch()
-    n = lib().ffk_encoder_layer_workspace_bytes(ctypes.byref(desc), dtype)
+    n = _call.ffk_encoder_layer_workspace_bytes(desc, dtype)
     return torch.empty((n,), dtype=torch.uint8, device=device)
 
 
 def encoder_layer_forward(desc, weights, x, y, workspace):
-    check(lib().ffk_encoder_layer_forward(current_stream(), dtype_of(x), ctypes.byref(desc),
-                                          ctypes.byref(weights), ptr(x), ptr(y), ptr(workspace),
-                                          workspace.numel()))
+    _call.ffk_encoder_layer_forward(dtype_of(x), desc, weights, x, y, workspace, workspace.numel())
     return y
 
 
 def encoder_layer_backward(desc, weights, grads, x, dy, dx, workspace):
-    check(lib().ffk_encoder_layer_backward(current_stream(), dtype_of(x), ctypes.byref(desc),
-                                           ctypes.byref(weights), ctypes.byref(grads), ptr(x),
-                                           ptr(dy), ptr(dx), ptr(workspace), workspace.numel()))
+    _call.ffk_encoder_layer_backward(dtype_of(x), desc, weights, grads, x, dy, dx, workspace, workspace.numel())
     return dx
 
 
@@ -815,16 +775,14 @@ def concat_forward(inputs, axis, out=None):
         shape = list(inputs[0].shape)
         shape[axis] = sum(t.shape[axis] for t in inputs)
         out = torch.empty(shape, dtype=inputs[0].dtype, device=inputs[0].device)
-    check(lib().ffk_concat_forward(current_stream(), dtype_of(out), ptr(out), ptrs, blks, len(inputs),
-                                   num_blocks))
+    _call.ffk_concat_forward(dtype_of(out), out, ptrs, blks, len(inputs), num_blocks)
     return out
 
 
 def concat_backward(out_grad, input_grads, axis, accumulate=True):
     """input_grads[i] (+)= the slice of out_grad that input i produced."""
     axis, num_blocks, ptrs, blks = _concat_args(input_grads, axis)
-    check(lib().ffk_concat_backward(current_stream(), dtype_of(out_grad), ptr(out_grad), ptrs, blks,
-                                    len(input_grads), num_blocks, int(accumulate)))
+    _call.ffk_concat_backward(dtype_of(out_grad), out_grad, ptrs, blks, len(input_grads), num_blocks, int(accumulate))
     return input_grads
 
 
@@ -836,7 +794,7 @@ def transpose_forward(x, perm, out=None):
     pm = (ctypes.c_int * x.dim())(*perm)
     if out is None:
         out = torch.empty([x.shape[p] for p in perm], dtype=x.dtype, device=x.device)
-    check(lib().ffk_transpose_forward(current_stream(), dtype_of(x), ptr(x), ptr(out), x.dim(), dims, pm))
+    _call.ffk_transpose_forward(dtype_of(x), x, out, x.dim(), dims, pm)
     return out
 
 
@@ -845,8 +803,7 @@ def transpose_backward(out_grad, in_grad, perm, accumulate=True):
     import ctypes
     dims = (ctypes.c_int64 * in_grad.dim())(*in_grad.shape)
     pm = (ctypes.c_int * in_grad.dim())(*perm)
-    check(lib().ffk_transpose_backward(current_stream(), dtype_of(out_grad), ptr(out_grad), ptr(in_grad),
-                                       in_grad.dim(), dims, pm, int(accumulate)))
+    _call.ffk_transpose_backward(dtype_of(out_grad), out_grad, in_grad, in_grad.dim(), dims, pm, int(accumulate))
     return in_grad
 
 
@@ -867,16 +824,14 @@ def gather_forward(x, index, dim, out=None):
     outer, ind, outd, stride = _gather_view(tuple(x.shape), tuple(index.shape), dim)
     if out is None:
         out = torch.empty(index.shape, dtype=x.dtype, device=x.device)
-    check(lib().ffk_gather_forward(current_stream(), dtype_of(x), dtype_of(index), ptr(x), ptr(index), ptr(out),
-                                   outer, ind, outd, stride))
+    _call.ffk_gather_forward(dtype_of(x), dtype_of(index), x, index, out, outer, ind, outd, stride)
     return out
 
 
 def gather_backward(out_grad, index, in_grad, dim):
     """in_grad[.., index, ..] += out_grad (fp32, atomics)."""
     outer, ind, outd, stride = _gather_view(tuple(in_grad.shape), tuple(index.shape), dim)
-    check(lib().ffk_gather_backward(current_stream(), dtype_of(index), ptr(out_grad), ptr(index), ptr(in_grad),
-                                    outer, ind, outd, stride))
+    _call.ffk_gather_backward(dtype_of(index), out_grad, index, in_grad, outer, ind, outd, stride)
     return in_grad
 
 
@@ -890,13 +845,12 @@ def split_forward(x, sizes, axis):
         shape[axis] = n
         outs.append(torch.empty(shape, dtype=x.dtype, device=x.device))
     _, num_blocks, ptrs, blks = _concat_args(outs, axis)
-    check(lib().ffk_split_forward(current_stream(), dtype_of(x), ptrs, ptr(x), blks, len(outs), num_blocks))
+    _call.ffk_split_forward(dtype_of(x), ptrs, x, blks, len(outs), num_blocks)
     return outs
 
 
 def split_backward(out_grads, in_grad, axis, accumulate=True):
     """in_grad (+)= the output gradients side by side along `axis`."""
     axis, num_blocks, ptrs, blks = _concat_args(out_grads, axis)
-    check(lib().ffk_split_backward(current_stream(), dtype_of(in_grad), ptr(in_grad), ptrs, blks,
-                                   len(out_grads), num_blocks, int(accumulate)))
+    _call.ffk_split_backward(dtype_of(in_grad), in_grad, ptrs, blks, len(out_grads), num_blocks, int(accumulate))
     return in_grad

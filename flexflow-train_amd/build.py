@@ -1,19 +1,24 @@
-"""Build recipe for libffk.so (the gfx950 operator-kernel library).
+"""Build recipe for libffk.so (the gfx950 operator-kernel library) and _ffk_call.so
+(its entry points as Python functions).
 
 Every ``csrc/*.hip`` file is compiled to an object with hipcc for gfx950 and
 the objects are linked into ``flexflow-train_amd/libffk.so`` next to this
 file.  hipcc cross-compiles without a GPU, so this runs anywhere the ROCm
-toolchain is installed.  Usage: ``python flexflow-train_amd/build.py [-j N]``.
+toolchain is installed.  ``csrc/python_call.cc`` is host code on the C API of
+Python and torch's tensor header.  Usage: ``python flexflow-train_amd/build.py [-j N]``.
 """
 import concurrent.futures
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "build")
 LIB_PATH = os.path.join(HERE, "libffk.so")
+CALL_PATH = os.path.join(HERE, "_ffk_call.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
@@ -81,12 +86,37 @@ def _compile_one(src, force):
     return obj, log
 
 
+def _compile_call(force):
+    """csrc/python_call.cc against this Python and this torch."""
+    src, obj = os.path.join(CSRC, "python_call.cc"), os.path.join(OBJ_DIR, "python_call.o")
+    if not force and os.path.exists(obj) and os.path.getmtime(obj) > max(os.path.getmtime(src), _headers_mtime()):
+        return obj
+    spec = importlib.util.find_spec("torch")
+    include = os.path.join(os.path.dirname(spec.origin), "include")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-isystem", include, "-isystem", sysconfig.get_paths()["include"],
+           "-c", src, "-o", obj]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError("g++ failed for %s:\n%s" % (src, proc.stdout + proc.stderr))
+    return obj
+
+
+def _link_call(obj):
+    torch_lib = os.path.join(os.path.dirname(importlib.util.find_spec("torch").origin), "lib")
+    cmd = ["g++", "-shared", "-o", CALL_PATH, obj, "-L" + HERE, "-lffk", "-Wl,-rpath,$ORIGIN", "-L" + torch_lib,
+           "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError("link failed:\n" + proc.stdout + proc.stderr)
+
+
 def build(jobs=8, force=True, verbose=False):
-    """Compile every kernel source and link libffk.so. Returns its path."""
+    """Compile every kernel source and link libffk.so and _ffk_call.so. Returns libffk.so's path."""
     os.makedirs(OBJ_DIR, exist_ok=True)
     srcs = _sources()
     objs = []
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
+        call_obj = pool.submit(_compile_call, force)
         for obj, log in pool.map(lambda s: _compile_one(s, force), srcs):
             objs.append(obj)
             if verbose and log.strip():
@@ -95,6 +125,7 @@ def build(jobs=8, force=True, verbose=False):
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError("link failed:\n" + proc.stdout + proc.stderr)
+    _link_call(call_obj.result())
     return LIB_PATH
 
 
