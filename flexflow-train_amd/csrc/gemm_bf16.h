@@ -81,6 +81,8 @@ __device__ __forceinline__ u32x2 load_first4(bf16 const *p, int n) {
   return u32x2{v[0], v[1]};
 }
 
+enum { kEdgeNone = 0, kEdgeOverlap = 1, kEdgeBounded = 2 };
+
 constexpr int kBK = 64;        // K extent of one LDS tile
 constexpr int kPadK = 8;       // row padding (elements) of a K-contiguous tile
 constexpr int kPadMN = 32;     // row padding of an M/N-contiguous tile
@@ -338,14 +340,23 @@ struct GemmSecondProblem {
 // pieces of the output tile on their way from LDS to memory.
 // PAIR: the launch carries two problems (no bias, no split-K).
 // EDGE: M, N and K need not be whole tiles (the operands still have to be readable 16 bytes at a
-// time).  Rows past the end of an operand panel and the k-rows past K lie past the bound of the
-// load's buffer descriptor and arrive as zeros; in the last k-tile of an operand whose k index is
-// contiguous the lanes whose 16 bytes lie past K ask for an offset beyond every bound.  Garbage in
-// columns past M or N only reaches outputs that are not stored.  The steady loop carries none of
-// this: it stops one tile earlier, so that it never asks for the last k-tile.
+// time).  Two ways:
+//   kEdgeOverlap (M >= BM, N >= BN): the last row and column of tiles begin early enough to lie inside
+//     the output, and do not store what their neighbours store.  No load needs a bound but those of a
+//     ragged last k-tile, whose lanes past K ask for an offset past the descriptor's bound and get
+//     zeros; the steady loop stops one tile earlier and is that of whole tiles.
+//   kEdgeBounded (any M, N): every load has a descriptor of its own, bounded by what is left of the
+//     operand behind its first row; what lies past it arrives as zeros, garbage in columns past M or N
+//     only reaches outputs that are not stored.  The descriptors cost 20% of the loop of a 128x128
+//     tile (4095 x 1024 over 4096: 39.0 us, 32.6 with 4096 rows) and nothing noticeable where a
+//     64x64 tile waits anyway.
+// KG: groups of waves that each take a part of the reduction (with LDS stages of their own) and add
+// up their accumulators at the end.  A 64x64 tile is 4 MFMAs a wave and k-tile, which a barrier, an
+// LDS round trip and the MFMAs' own dependence stretch to some 600 cycles; a second group fills them
+// where there are too few tiles for a second workgroup per CU.
 template <int BM, int BN, int WM, int WN, int BK, int STAGES, int PF, bool TA, bool TB, int TAIL = 0,
-          bool PAIR = false, bool EDGE = false>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_kernel(
+          bool PAIR = false, int EDGE = kEdgeNone, int KG = 1>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pipe_kernel(
     bf16 const *__restrict__ A, bf16 const *__restrict__ B, bf16 *C, int M,
     int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
     bf16 const *__restrict__ bias, int act, int accumulate,
@@ -379,7 +390,9 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
 
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
 
-  int const t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  static_assert(KG == 1 || (EDGE == kEdgeBounded && !PAIR), "written for these");
+  int const kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+  int const t = KG == 1 ? threadIdx.x : threadIdx.x % NT, lane = t & 63, wave = t >> 6;
   int const wm0 = (wave / (BN / WN)) * WM;
   int const wn0 = (wave % (BN / WN)) * WN;
   int tm, tn;
@@ -387,8 +400,11 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
   int const tiles = nbm * nbn;
   int const split = partial != nullptr ? bid / tiles : 0;
   tile_coords(partial != nullptr ? bid % tiles : bid, nbm, nbn, tm, tn);
-  int const m0 = tm * BM, n0 = tn * BN;
-  int const kt0 = split * k_tiles_per_split;  // first k-tile of this workgroup
+  // (kEdgeOverlap) what of the tile is this workgroup's to store begins at first_m, first_n
+  int const first_m = tm * BM, first_n = tn * BN;
+  int const m0 = EDGE == kEdgeOverlap ? min(first_m, M - BM) : first_m, n0 = EDGE == kEdgeOverlap ? min(first_n, N - BN) : first_n;
+  // first k-tile of this workgroup, or of this group of waves
+  int const kt0 = KG == 1 ? split * k_tiles_per_split : kg * (((K + BK - 1) / BK + KG - 1) / KG);
 
   // Per-lane offset of its first chunk inside the block's operand panel; the
   // chunk of load i lies a uniform number of rows further on, and the k-tile
@@ -442,11 +458,12 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
   bf16 const *const panel_a = TA ? A + m0 : A + (int64_t)m0 * lda;
   bf16 const *const panel_b = TBL ? B + n0 : B + (int64_t)n0 * ldb;
   // one past the last element of the operand that a workgroup may read, from its panel's start
-  int64_t const end_a = !EDGE ? 0 : TA ? (int64_t)(K - 1) * lda + (M - m0) : (int64_t)(min(BM, M - m0) - 1) * lda + K;
-  int64_t const end_b = !EDGE ? 0 : TBL ? (int64_t)(K - 1) * ldb + (N - n0) : (int64_t)(min(BN, N - n0) - 1) * ldb + K;
+  int64_t const end_a = EDGE != kEdgeBounded ? 0 : TA ? (int64_t)(K - 1) * lda + (M - m0) : (int64_t)(min(BM, M - m0) - 1) * lda + K;
+  int64_t const end_b = EDGE != kEdgeBounded ? 0 : TBL ? (int64_t)(K - 1) * ldb + (N - n0) : (int64_t)(min(BN, N - n0) - 1) * ldb + K;
 
   // LDS destinations of the direct loads are scalar byte addresses: base + stage + chunk row
-  unsigned const smem_addr = lds_address_of(smem);
+  bf16 *const stages = smem + (KG == 1 ? 0 : kg * (STAGES * STAGE_ELEMS));
+  unsigned const smem_addr = lds_address_of(stages);
   int const wave_s = __builtin_amdgcn_readfirstlane(wave);
   // Loads [first, first + count) of a k-tile's LPT direct loads (A's, then B's).
   // (first and count are constants once the caller's loops are unrolled)
@@ -454,9 +471,31 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
   auto issue_some = [&](int kt, int stage, int first, int count, bool maybe_last) __attribute__((always_inline)) {
     unsigned const sa = smem_addr + (unsigned)(stage * STAGE_ELEMS) * 2u;
     unsigned const sb = sa + (unsigned)A_ELEMS * 2u;
-    if constexpr (EDGE) {
-      bool const last = maybe_last && kt0 + kt == KT_all - 1;
-      unsigned const va = !TA && last ? voff_a_last : voff_a, vb = !TBL && last ? voff_b_last : voff_b;
+    if constexpr (EDGE == kEdgeOverlap) {
+      if (maybe_last && kt0 + kt == KT_all - 1 && K % BK != 0) {  // uniform over the launch's workgroups
+        i32x4 const ra = buffer_resource(panel_a + (TA ? (int64_t)(kt0 + kt) * BK * lda : (int64_t)(kt0 + kt) * BK), 0x80000000u);
+        i32x4 const rb = buffer_resource(panel_b + (TBL ? (int64_t)(kt0 + kt) * BK * ldb : (int64_t)(kt0 + kt) * BK), 0x80000000u);
+        int const left = K - (KT_all - 1) * BK;  // k's of this tile
+        int const c = wave * 64 + lane;
+#pragma unroll
+        for (int q = 0; q < LPT; q++) {
+          if (q < first || q >= first + count) continue;
+          if (q < A_LOADS) {
+            unsigned const va = !TA ? voff_a_last : c / (BM / 8) + q * (NT * 8 / BM) < left ? voff_a : 0x80000000u;
+            lds_dma16(ra, va, (unsigned)(q * step_a) * 2u, sa + (unsigned)(q * NW + wave_s) * 1024u);
+          } else {
+            int const i = q - A_LOADS;
+            unsigned const vb = !TBL ? voff_b_last : c / (BN / 8) + i * (NT * 8 / BN) < left ? voff_b : 0x80000000u;
+            lds_dma16(rb, vb, (unsigned)(i * step_b) * 2u, sb + (unsigned)(i * NW + wave_s) * 1024u);
+          }
+        }
+        return;
+      }
+    }
+    if constexpr (EDGE == kEdgeBounded) {
+      bool const last = maybe_last && kt0 + kt >= KT_all - 1;
+      unsigned va = !TA && last ? voff_a_last : voff_a, vb = !TBL && last ? voff_b_last : voff_b;
+      if (KG > 1 && maybe_last && kt0 + kt >= KT_all) va = vb = 0x80000000u;  // a group that ran out of k-tiles: zeros
       int64_t const at_a = TA ? (int64_t)(kt0 + kt) * BK * lda : (int64_t)(kt0 + kt) * BK;
       int64_t const at_b = TBL ? (int64_t)(kt0 + kt) * BK * ldb : (int64_t)(kt0 + kt) * BK;
       // a descriptor per load: its bound is what is left of the operand behind the load's first row
@@ -517,21 +556,23 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
   // Tile lying as [BK][cols]: lane reads rows kk*16 + 8 (l/32) + (l%16)/4 (+4),
   // columns col0 + 16 ((l/16)%2) + 4 (l%4); the 64-byte segment index is
   // XOR-ed with tr_swizzle(row), which touches only its two low bits (its one bit).
-  int tr_tab_a[4], tr_tab_b[4];
+  // One entry per 32-wide block of the wave's tile.
+  int tr_tab_a[TM], tr_tab_b[TN];
   {
     int const i16 = lane & 15;
     int const q = i16 >> 2;
     int const inseg = ((lane >> 4) & 1) * 16 + (i16 & 3) * 4;
     int const krow = (lane >> 5) * 8 + q;
+    auto offset = [&](int cols, int block) {
+      return krow * cols + (((block & 3) ^ tr_swizzle(q, cols)) << 5) + ((block & ~3) << 5) + inseg;
+    };
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-      tr_tab_a[c] = krow * BM + ((c ^ tr_swizzle(q, BM)) << 5) + inseg;
-      tr_tab_b[c] = krow * BN + ((c ^ tr_swizzle(q, BN)) << 5) + inseg;
-    }
+    for (int i = 0; i < TM; i++) tr_tab_a[i] = offset(BM, (wm0 >> 5) + i);
+#pragma unroll
+    for (int j = 0; j < TN; j++) tr_tab_b[j] = offset(BN, (wn0 >> 5) + j);
   }
-  auto frag_tr = [&](bf16 const *tile, int rowlen, int const (&tab)[4], int col0, int kk) -> bf16x8 {
-    int const seg = col0 >> 5;
-    bf16 const *p = tile + tab[seg & 3] + ((seg & ~3) << 5) + kk * 16 * rowlen;
+  auto frag_tr = [&](bf16 const *tile, int rowlen, int tab, int kk) -> bf16x8 {
+    bf16 const *p = tile + tab + kk * 16 * rowlen;
     typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
     s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p));
     s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p + 4 * rowlen));
@@ -552,7 +593,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
 #pragma unroll
       for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
 
-  int const KT = partial != nullptr ? (EDGE ? min(k_tiles_per_split, KT_all - kt0) : k_tiles_per_split) : KT_all;
+  int const KT = KG > 1 ? (KT_all + KG - 1) / KG : partial != nullptr ? (EDGE ? min(k_tiles_per_split, KT_all - kt0) : k_tiles_per_split) : KT_all;
   constexpr int NB = PF + 1;  // fragment buffers
   static_assert(KS % NB == 0, "buffer index must not depend on the tile");
   static_assert(STAGES >= 2, "one stage in use, at least one in flight");
@@ -582,15 +623,15 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
   // step) are already in flight.
   bf16x8 af[NB][TM], bfr[NB][TN];
   auto read_frags = [&](int buf, int stage, int kk) {
-    bf16 const *sa = smem + stage * STAGE_ELEMS;
+    bf16 const *sa = stages + stage * STAGE_ELEMS;
     bf16 const *sb = sa + A_ELEMS;
 #pragma unroll
     for (int i = 0; i < TM; i++) {
-      af[buf][i] = TA ? frag_tr(sa, BM, tr_tab_a, wm0 + i * 32, kk) : frag_kc(sa, wm0 + i * 32, kk);
+      af[buf][i] = TA ? frag_tr(sa, BM, tr_tab_a[i], kk) : frag_kc(sa, wm0 + i * 32, kk);
     }
 #pragma unroll
     for (int j = 0; j < TN; j++) {
-      bfr[buf][j] = TBL ? frag_tr(sb, BN, tr_tab_b, wn0 + j * 32, kk) : frag_kc(sb, wn0 + j * 32, kk);
+      bfr[buf][j] = TBL ? frag_tr(sb, BN, tr_tab_b[j], kk) : frag_kc(sb, wn0 + j * 32, kk);
     }
   };
   // Tile 0 must have landed (STAGES-1 younger tiles may still be in flight).
@@ -654,10 +695,10 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
             if (r * NS / NR != p || !reads) continue;
             if (r == 0 || r > TN) {
               int const i = r == 0 ? 0 : r - TN;
-              af[nxt][i] = TA ? frag_tr(ra, BM, tr_tab_a, wm0 + i * 32, rkk) : frag_kc(ra, wm0 + i * 32, rkk);
+              af[nxt][i] = TA ? frag_tr(ra, BM, tr_tab_a[i], rkk) : frag_kc(ra, wm0 + i * 32, rkk);
             } else {
               int const j = r - 1;
-              bfr[nxt][j] = TBL ? frag_tr(rb, BN, tr_tab_b, wn0 + j * 32, rkk) : frag_kc(rb, wn0 + j * 32, rkk);
+              bfr[nxt][j] = TBL ? frag_tr(rb, BN, tr_tab_b[j], rkk) : frag_kc(rb, wn0 + j * 32, rkk);
             }
           }
 #pragma unroll
@@ -712,7 +753,10 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
           // Every wave has all fragments of tile kt in registers once its LDS
           // counter drains, so after the barrier the stage is free.
           if (STEADY || kt + STAGES - 1 < KT) {
-            wait_vmcnt<(STAGES - 2) * LPT>();
+            // (PF = 3 reads the next tile one step before the last part of a refill goes out: of
+            // what is younger than the next tile's own last part, two parts are missing)
+            static_assert(!SPREAD || PF <= 2 || (PF == 3 && KS == 4), "count of younger loads");
+            wait_vmcnt<(STAGES - 2) * LPT - (SPREAD && PF == 3 ? 2 * PART : 0)>();
           } else {
             wait_vmcnt<0>();
           }
@@ -736,7 +780,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
   };
   using Dyn = std::integral_constant<int, -1>;
   int kt = 0;
-  int const KT_steady = EDGE ? KT - 1 : KT;  // the steady loop asks for no tile from here on
+  // the steady loop asks for no tile from here on (a group's own last k-tiles may lie past the others')
+  int const KT_steady = EDGE != kEdgeNone ? KT - KG : KT;
   if constexpr (!WIDE2 && (STAGES == 4 || STAGES == 2)) {
     for (; kt + 2 * STAGES - 1 < KT_steady; kt += STAGES) {  // kt % STAGES == 0, all STAGES tiles steady
       tile_step(kt, std::true_type{}, std::integral_constant<int, 0>{});
@@ -768,7 +813,10 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
   // Eight columns from column n of row m on (EDGE: those that exist).
   auto store8 = [&](int m, int n, u32x4 v) __attribute__((always_inline)) {
     bf16 *const to = C + (int64_t)m * ldc + n;
-    if constexpr (EDGE) {
+    if constexpr (EDGE == kEdgeOverlap) {
+      if (m < first_m || n + 8 <= first_n) return;
+      store_raw_any(to, v);
+    } else if constexpr (EDGE == kEdgeBounded) {
       if (m >= M || n >= N) return;
       if (n + 8 <= N) {
         store_raw_any(to, v);
@@ -781,12 +829,12 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
   };
   // Bias of four columns from n on.
   auto bias4 = [&](int n, float (&bv)[4]) __attribute__((always_inline)) {
-    if constexpr (EDGE) {
+    if constexpr (EDGE == kEdgeBounded) {
 #pragma unroll
       for (int e = 0; e < 4; e++) bv[e] = bias != nullptr && n + e < N ? VecIO<bf16>::load1(bias + n + e) : 0.0f;
     } else {
       u32x2 raw = {0u, 0u};
-      if (bias != nullptr) raw = *reinterpret_cast<u32x2 const *>(bias + n);
+      if (bias != nullptr) raw = EDGE != kEdgeNone ? load_any8(bias + n) : *reinterpret_cast<u32x2 const *>(bias + n);
       bv[0] = __uint_as_float(raw[0] << 16);
       bv[1] = __uint_as_float(raw[0] & 0xffff0000u);
       bv[2] = __uint_as_float(raw[1] << 16);
@@ -828,6 +876,39 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
     }
   }
   __syncthreads();  // all stages are free now: reuse them for the output tile
+  if constexpr (KG > 1) {
+    static_assert((KG - 1) * NW * TM * TN * 1024 <= (KG - 1) * STAGES * STAGE_ELEMS / 2, "partial tiles fit the groups' stages");
+    // group g's accumulators, 16 bytes a lane and access, in the stages that were group g's (the
+    // output tile is staged in group 0's)
+    f32x4 *const mine = reinterpret_cast<f32x4 *>(stages) + wave * (TM * TN * 4 * 64) + lane;
+    if (kg > 0) {
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int g = 0; g < 4; g++) {
+            mine[((i * TN + j) * 4 + g) * 64] =
+                f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+          }
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int o = 1; o < KG; o++) {
+      f32x4 const *const other = reinterpret_cast<f32x4 const *>(smem + o * (STAGES * STAGE_ELEMS)) + wave * (TM * TN * 4 * 64) + lane;
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int g = 0; g < 4; g++) {
+            f32x4 const v = other[((i * TN + j) * 4 + g) * 64];
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[i][j][4 * g + e] += v[e];
+          }
+    }
+  }
 
   // Each wave stages its own WM x WN tile and writes it out in 16-byte chunks.
   bf16 *cs = smem + wave * (WM * CS);
@@ -867,7 +948,9 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
             // add the old value in fp32 before the single rounding
             bf16 const *const from = dst + (int64_t)(m0 + wm0 + m) * ldc + n0 + wn0 + n;
             u32x2 old = {0u, 0u};
-            if constexpr (EDGE) {
+            if constexpr (EDGE == kEdgeOverlap) {
+              old = load_any8(from);
+            } else if constexpr (EDGE == kEdgeBounded) {
               int const left = m0 + wm0 + m < M ? N - (n0 + wn0 + n) : 0;  // columns of these four that exist
               old = left >= 4 ? load_any8(from) : left > 0 ? load_first4(from, left) : old;
             } else {
@@ -892,7 +975,10 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
       if constexpr (TAIL == GemmEpilogue::kTailNone) {
         store8(m0 + wm0 + row, n0 + wn0 + ch * 8, v);
       } else {
-        if constexpr (EDGE) {  // N is a multiple of 8 here: a piece is whole or not there
+        if constexpr (EDGE == kEdgeOverlap) {  // N is a multiple of 8 here: a piece is one workgroup's
+          if (m0 + wm0 + row < first_m || n0 + wn0 + ch * 8 < first_n) continue;
+        }
+        if constexpr (EDGE == kEdgeBounded) {  // ... or not there
           if (m0 + wm0 + row >= M || n0 + wn0 + ch * 8 >= N) {
             *reinterpret_cast<u32x4 *>(cs + row * CS + ch * 8) = u32x4{0u, 0u, 0u, 0u};  // for the column sums
             continue;
@@ -956,7 +1042,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
               run[q] = acc_rows;
             }
             int64_t const part = (m0 + wm0) / kColsumRowsPerBlock + blk;
-            if (EDGE && (part * kColsumRowsPerBlock >= M || n0 + wn0 + col >= N)) continue;
+            static_assert(EDGE != kEdgeOverlap || TAIL != GemmEpilogue::kTailDropoutGeluGrad, "blocks of 32 rows begin at multiples of 32");
+            if (EDGE == kEdgeBounded && (part * kColsumRowsPerBlock >= M || n0 + wn0 + col >= N)) continue;
             tail.colsum_partials[part * N + n0 + wn0 + col] = (run[0] + run[1]) + (run[2] + run[3]);
           }
         }
@@ -981,7 +1068,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_pipe_ker
 #pragma unroll
         for (int g = 0; g < 4; g++) {
           int const n = n0 + wn0 + j * 32 + 8 * g + 4 * (lane >> 5);
-          if (EDGE && (m >= M || n >= N)) continue;  // (N % 4 == 0 where a reduction is split)
+          if (EDGE == kEdgeBounded && (m >= M || n >= N)) continue;  // (N % 4 == 0 where a reduction is split)
           f32x4 v = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
           *reinterpret_cast<f32x4 *>(dst + m * N + n) = v;
         }
@@ -1041,26 +1128,29 @@ struct PipeCfg {
   static_assert(kLds <= 160 * 1024, "LDS budget");
 };
 
-template <int BM, int BN, int WM, int WN, int BK, int STAGES, int PF, bool TA, bool TB, int TAIL = 0, bool EDGE = false>
+template <int BM, int BN, int WM, int WN, int BK, int STAGES, int PF, bool TA, bool TB, int TAIL = 0, int EDGE = kEdgeNone,
+          int KG = 1>
 static hipError_t launch_pipe(hipStream_t st, bf16 const *A, bf16 const *B,
                               bf16 *C, int M, int N, int K, int64_t lda,
                               int64_t ldb, int64_t ldc, GemmEpilogue const &ep,
                               int splits = 1) {
   using Cfg = PipeCfg<BM, BN, WM, WN, BK, STAGES>;
-  constexpr int NT = Cfg::NW * 64;
-  if (describe_only("gemm_bf16_pipe_kernel<%d,%d,%d,%d,%d,%d,%d,%s,%s,%d,false%s>%s", BM, BN, WM, WN, BK, STAGES, PF,
-                    tf(TA), tf(TB), TAIL, EDGE ? ",true" : "", splits > 1 ? " (split-K) + splitk_reduce_kernel" : "")) {
+  constexpr int NT = Cfg::NW * 64 * KG;
+  constexpr size_t kLds = KG == 1 ? Cfg::kLds : KG * Cfg::kStageBytes;
+  static_assert(kLds <= 160 * 1024, "LDS budget");
+  if (describe_only("gemm_bf16_pipe_kernel<%d,%d,%d,%d,%d,%d,%d,%s,%s,%d,false%s%s>%s", BM, BN, WM, WN, BK, STAGES, PF,
+                    tf(TA), tf(TB), TAIL, EDGE == kEdgeNone ? "" : EDGE == kEdgeOverlap ? ",overlap" : ",bounded", KG == 1 ? "" : ",2", splits > 1 ? " (split-K) + splitk_reduce_kernel" : "")) {
     return hipSuccess;
   }
-  auto kern = gemm_bf16_pipe_kernel<BM, BN, WM, WN, BK, STAGES, PF, TA, TB, TAIL, false, EDGE>;
+  auto kern = gemm_bf16_pipe_kernel<BM, BN, WM, WN, BK, STAGES, PF, TA, TB, TAIL, false, EDGE, KG>;
   GemmTailArgs const tail = {static_cast<bf16 const *>(ep.tail_in), static_cast<bf16 *>(ep.tail_out),
                              ep.tail_dropout, ep.tail_colsum_partials};
   static LdsOptIn lds;  // per template instance
-  if (hipError_t e = lds.ensure(reinterpret_cast<void const *>(kern), (int)Cfg::kLds); e != hipSuccess) return e;
+  if (hipError_t e = lds.ensure(reinterpret_cast<void const *>(kern), (int)kLds); e != hipSuccess) return e;
   int const blocks = EDGE ? ((M + BM - 1) / BM) * ((N + BN - 1) / BN) : (M / BM) * (N / BN);
   if (splits > 1) {
     float *partial = static_cast<float *>(ep.splitk_ws);
-    kern<<<blocks * splits, NT, Cfg::kLds, st>>>(A, B, C, M, N, K, lda, ldb, ldc, nullptr,
+    kern<<<blocks * splits, NT, kLds, st>>>(A, B, C, M, N, K, lda, ldb, ldc, nullptr,
                                                 FFK_ACT_NONE, 0, partial, K / BK / splits, tail,
                                                 GemmSecondProblem{});
     hipError_t e = hipGetLastError();
@@ -1071,7 +1161,7 @@ static hipError_t launch_pipe(hipStream_t st, bf16 const *A, bf16 const *B,
         ep.accumulate);
     return hipGetLastError();
   }
-  kern<<<blocks, NT, Cfg::kLds, st>>>(A, B, C, M, N, K, lda, ldb, ldc,
+  kern<<<blocks, NT, kLds, st>>>(A, B, C, M, N, K, lda, ldb, ldc,
                                      static_cast<bf16 const *>(ep.bias), ep.activation,
                                      ep.accumulate, nullptr, 0, tail, GemmSecondProblem{});
   return hipGetLastError();
@@ -1158,18 +1248,32 @@ inline int pipe_tile_for(bf16 const *C, int M, int N, int K, int64_t lda, int64_
 // offsets reach.
 inline bool edge_operands_ok(int64_t lda, int64_t ldb) { return 2 * 256 * std::max(lda, ldb) < (int64_t(1) << 31); }
 
-// The tile for a problem none of the whole-tile rules takes.  256x256 (two waves per SIMD: with one,
-// the descriptors of the ragged loads sit between the MFMAs and cost 10-20%) once it reaches three
-// quarters of the CUs, 128x128 once it reaches half of them, 64x64 below.  Against the
-// register-staged 128x128 / 64x64 kernel that took these shapes before, us: [1379,2304] over 768
-// 10.8 (15.2), [1379,768] over 3072 22.4 (39.9), [4000,4000] over 4000 114 (181); and against one
-// thread an output, which took every weight gradient over a token count that is no multiple of 8:
-// [3072,768] over 1379 15.8 (1900).
-inline int edge_tile_for(int M, int N) {
-  int64_t const t256 = ceil_div(M, 256) * ceil_div(N, 256), t128 = ceil_div(M, 128) * ceil_div(N, 128);
-  if (t256 >= kNumCU * 3 / 4) return 256;
-  if (t128 >= kNumCU / 2) return 128;
-  return 64;
+// The tile for a problem none of the whole-tile rules takes: the one whose rounds over the chip take
+// the least time.  A round's time is its k-tiles (64 deep) times what one costs with that tile, in us,
+// measured over M 100-2500, N 256-2304, K 100-3072 in three transposes (the choice is within 10% of the
+// best tile on nearly all of them):
+//   64 x 64, two groups of waves that split the reduction, two workgroups a CU: 0.17 while there are
+//     at most as many tiles as CUs, 0.39 for two a CU; with four LDS stages a group and one workgroup
+//     a CU (deep) 0.21, for which a long reduction over one tile a CU is worth having
+//   128 x 64: 0.385, or 0.62 for two a CU        128 x 128: 0.46        256 x 256: 1.3
+// and about 1 us of fill and drain per round.
+enum EdgeTile { kTile64 = 64, kTile64Deep = 65, kTile128x64 = 70, kTile128 = 128, kTile256 = 256, kTile256Wide = 264 };
+inline EdgeTile edge_tile_for(int M, int N, int K, bool wide_ok) {
+  auto tiles = [&](int bm, int bn) { return (double)ceil_div(M, bm) * (double)ceil_div(N, bn); };
+  double const kt = (double)ceil_div(K, 64);
+  auto rounds = [&](double n, double per_round, double us) { return ceil(n / per_round) * (kt * us + 1.0); };
+  EdgeTile best = kTile64;
+  double const t64 = tiles(64, 64), t12 = tiles(128, 64);
+  double time = t64 <= kNumCU ? kt * 0.17 + 1.0 : rounds(t64, 2 * kNumCU, 0.39);
+  auto consider = [&](EdgeTile t, double us) {
+    if (us < time) best = t, time = us;
+  };
+  if (kt > 24) consider(kTile64Deep, t64 <= kNumCU ? kt * 0.16 : rounds(t64, kNumCU, 0.21));
+  consider(kTile128x64, t12 <= kNumCU ? kt * 0.385 + 1.0 : rounds(t12, 2 * kNumCU, 0.62));
+  consider(kTile128, rounds(tiles(128, 128), kNumCU, 0.46));
+  // one wave per SIMD where that kernel has what it takes, two otherwise
+  consider(wide_ok && K >= 1024 ? kTile256Wide : kTile256, rounds(tiles(256, 256), kNumCU, 1.3));
+  return best;
 }
 
 template <bool TA, bool TB>
@@ -1251,14 +1355,26 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
   }
   if (ep.tail != GemmEpilogue::kTailNone) return hipErrorInvalidValue;
   if (variant != 1 && edge_operands_ok(lda, ldb)) {
-    int const tile = variant == 64 || variant == 128 || variant == 256 ? variant : edge_tile_for(M, N);
-    if (tile == 256) {
-      return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB, 0, true>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+    EdgeTile tile = edge_tile_for(M, N, K, ep.activation == FFK_ACT_NONE && ldc % 8 == 0);
+    bool const forced = variant == 64 || variant == 65 || variant == 70 || variant == 128 || variant == 256 || variant == 264;
+    if (forced) tile = (EdgeTile)variant;
+    // tiles that begin early: the output has to hold one, and old values added by one workgroup only
+    int const bm = tile == kTile256 || tile == kTile256Wide ? 256 : 128, bn = tile == kTile128x64 ? 64 : bm;
+    if (tile != kTile64 && tile != kTile64Deep && (M < bm || N < bn || (ep.accumulate && N % 8 != 0))) tile = kTile64;
+    switch (tile) {
+      case kTile256Wide:
+        return launch_pipe<256, 256, 128, 128, 64, 2, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+      case kTile256:
+        return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+      case kTile128:
+        return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+      case kTile128x64:
+        return launch_pipe<128, 64, 32, 32, 64, 3, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+      case kTile64Deep:
+        return launch_pipe<64, 64, 32, 32, 64, 4, 3, TA, TB, 0, kEdgeBounded, 2>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+      case kTile64:
+        return launch_pipe<64, 64, 32, 32, 64, 2, 3, TA, TB, 0, kEdgeBounded, 2>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
     }
-    if (tile == 128) {
-      return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, 0, true>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
-    }
-    return launch_pipe<64, 64, 32, 32, 64, 4, 1, TA, TB, 0, true>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
   }
   // Largest tile that still gives every CU a workgroup.
   int64_t const b128 = ceil_div(M, 128) * ceil_div(N, 128);

@@ -11,7 +11,8 @@ BT = torch.bfloat16
 
 # M, N, K: one element short of and past a tile, one row, one column group, reductions of less than
 # one k-tile, of a whole one, and of a few with a remainder
-ALIGNED = [(8, 8, 8), (136, 264, 72), (256, 128, 64), (248, 120, 200), (512, 520, 328), (40, 1032, 136)]
+ALIGNED = [(8, 8, 8), (136, 264, 72), (256, 128, 64), (248, 120, 200), (512, 520, 328), (40, 1032, 136),
+           (264, 256, 1416)]
 ANY = [(1, 2111, 1000), (129, 257, 65), (255, 127, 191), (131, 509, 261), (513, 33, 127)]
 KINDS = [(False, True), (False, False), (True, False), (True, True)]
 
@@ -36,7 +37,7 @@ def product(ffk, oracle, mnk, ta, tb, accumulate):
 
 
 @pytest.mark.parametrize("ta,tb", KINDS)
-@pytest.mark.parametrize("variant", [64, 128, 256])
+@pytest.mark.parametrize("variant", [64, 65, 70, 128, 256, 264])
 @pytest.mark.parametrize("mnk", ALIGNED)
 def test_pipelined_tiles_with_ragged_edges(ffk, oracle, ta, tb, variant, mnk):
     print("gemm edges", mnk, "ta", ta, "tb", tb, "tile", variant, flush=True)
