@@ -54,13 +54,12 @@ int gemm_dispatch(hipStream_t stream, int dtype, bool trans_a, bool trans_b,
                   void const *B, int64_t ldb, void *C, int64_t ldc,
                   GemmEpilogue const &ep);
 
-// Two GEMMs of the same kind (same transposes, same reduction length K, no
-// bias or activation, same accumulate switch) in ONE launch: for two outputs
-// that each leave part of the chip idle (the two weight gradients of an
-// attention block).  Each problem's result is the bits of gemm_dispatch on it
-// alone with the 128x128 tile.  gemm_pair_supported says whether the pair
-// runs (BF16, outputs multiples of 128, K a multiple of 64, 16-byte aligned
-// operands); gemm_dispatch_pair fails otherwise.
+// Weight gradients that are collected and run as ONE launch: C = A^T . B, A [K, M], B [K, N], of
+// problems with the same reduction length K that each leave part of the chip idle.  While a group
+// is set on the calling thread, weight_grad_dispatch puts such problems into it instead of launching
+// them (their operands have to stay as they are until the flush), and launches all others as
+// gemm_dispatch would.
+constexpr int kMaxGemmGroup = 4;
 struct GemmProblem {
   int64_t M, N;
   void const *A;
@@ -70,10 +69,26 @@ struct GemmProblem {
   void *C;
   int64_t ldc;
 };
-bool gemm_pair_supported(int dtype, bool trans_a, bool trans_b, int64_t K, GemmProblem const &p0,
-                         GemmProblem const &p1);
-int gemm_dispatch_pair(hipStream_t stream, int dtype, bool trans_a, bool trans_b, int64_t K,
-                       GemmProblem const &p0, GemmProblem const &p1, bool accumulate);
+struct WeightGradGroup {
+  GemmProblem p[kMaxGemmGroup];
+  int count = 0;
+  int64_t K = 0;
+  bool accumulate = false;
+};
+inline thread_local WeightGradGroup *tl_weight_grads = nullptr;
+// Collects the calling thread's weight gradients for its lifetime (unless an outer one does).
+struct CollectWeightGrads {
+  WeightGradGroup group;
+  WeightGradGroup *const saved;
+  explicit CollectWeightGrads(bool on) : saved(tl_weight_grads) {
+    if (on && saved == nullptr) tl_weight_grads = &group;
+  }
+  ~CollectWeightGrads() { tl_weight_grads = saved; }
+};
+int weight_grad_dispatch(hipStream_t stream, int dtype, int64_t M, int64_t N, int64_t K, void const *A, int64_t lda,
+                         void const *B, int64_t ldb, void *C, int64_t ldc, GemmEpilogue const &ep);
+// Runs what was collected (nothing to do for an empty group) and empties it.
+int weight_grad_flush(hipStream_t stream, WeightGradGroup &group);
 
 // Scratch bytes with which a bf16 GEMM of this shape would split its reduction
 // (0: it would not).

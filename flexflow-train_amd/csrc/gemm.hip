@@ -26,13 +26,13 @@ hipError_t gemm_f32_launch(hipStream_t st, bool ta, bool tb, int M, int N, int K
 // instantiated in gemm_nn.hip, gemm_nt.hip, gemm_tn.hip, gemm_tt.hip
 #define FFK_EXTERN_BF16(TA_, TB_)                                                                                       \
   extern template hipError_t pick_bf16<TA_, TB_>(hipStream_t, bf16 const *, bf16 const *, bf16 *, int, int, int,        \
-                                                 int64_t, int64_t, int64_t, GemmEpilogue const &, bool);                \
-  extern template hipError_t launch_pipe_pair<TA_, TB_>(hipStream_t, GemmProblem const &, GemmProblem const &, int, bool)
+                                                 int64_t, int64_t, int64_t, GemmEpilogue const &, bool)
 FFK_EXTERN_BF16(false, false);
 FFK_EXTERN_BF16(false, true);
 FFK_EXTERN_BF16(true, false);
 FFK_EXTERN_BF16(true, true);
 #undef FFK_EXTERN_BF16
+extern template hipError_t pick_bf16_group<true, false>(hipStream_t, GemmProblem const *, int, int, bool);
 
 size_t gemm_splitk_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
   if (dtype != FFK_BF16 || M % 128 != 0 || N % 128 != 0) return 0;
@@ -248,33 +248,51 @@ int dropout_backward_colsum(hipStream_t st, int dtype, void const *dy, void *dx,
   return FFK_ERR_UNSUPPORTED;
 }
 
-static bool pair_member_ok(bool ta, bool tb, GemmProblem const &p, int64_t K) {
-  if (p.M <= 0 || p.N <= 0 || p.M % 128 != 0 || p.N % 128 != 0 || !p.A || !p.B || !p.C) return false;
-  if (p.M >= (1ll << 31) || p.N >= (1ll << 31)) return false;
-  if (p.lda < (ta ? p.M : K) || p.ldb < (tb ? K : p.N) || p.ldc < p.N) return false;
-  bool const vec_ok = (p.lda % 8 == 0) && (p.ldb % 8 == 0) && aligned16(p.A) && aligned16(p.B);
-  GemmEpilogue none;
-  return vec_ok && pipe_tile_for(static_cast<bf16 const *>(p.C), (int)p.M, (int)p.N, (int)K, p.lda, p.ldb, p.ldc, none,
-                                 128) == 128;
+// Whether a weight gradient joins a group: one that fills the chip twice over has better kernels of
+// its own, and the group's take operands readable 16 bytes at a time.
+static bool joins_group(int dtype, int64_t M, int64_t N, int64_t K, GemmProblem const &p, GemmEpilogue const &ep) {
+  if (dtype != FFK_BF16 || gemm_variant_override() != 0 || ep.bias != nullptr || ep.activation != FFK_ACT_NONE ||
+      ep.tail != GemmEpilogue::kTailNone) {
+    return false;
+  }
+  if (M <= 0 || N <= 0 || K <= 0 || M >= (1ll << 31) || N >= (1ll << 31) || K >= (1ll << 31)) return false;
+  if (!p.A || !p.B || !p.C || p.lda < M || p.ldb < N || p.ldc < N) return false;
+  if (ceil_div(M, 128) * ceil_div(N, 128) >= 2 * kNumCU) return false;
+  return M % 8 == 0 && N % 8 == 0 && p.lda % 8 == 0 && p.ldb % 8 == 0 && aligned16(p.A) && aligned16(p.B) &&
+         edge_operands_ok(p.lda, p.ldb);
 }
 
-bool gemm_pair_supported(int dtype, bool ta, bool tb, int64_t K, GemmProblem const &p0, GemmProblem const &p1) {
-  if (dtype != FFK_BF16 || K <= 0 || K % 64 != 0 || K >= (1ll << 31) || gemm_variant_override() != 0) return false;
-  if (!pair_member_ok(ta, tb, p0, K) || !pair_member_ok(ta, tb, p1, K)) return false;
-  // worth it when neither problem fills the chip on its own and the two together come closer
-  int64_t const t0 = (p0.M / 128) * (p0.N / 128), t1 = (p1.M / 128) * (p1.N / 128);
-  return t0 < 2 * kNumCU && t1 < 2 * kNumCU && t0 + t1 >= kNumCU / 2;
+int weight_grad_dispatch(hipStream_t st, int dtype, int64_t M, int64_t N, int64_t K, void const *A, int64_t lda,
+                         void const *B, int64_t ldb, void *C, int64_t ldc, GemmEpilogue const &ep) {
+  WeightGradGroup *const g = tl_weight_grads;
+  GemmProblem const p = {M, N, A, lda, B, ldb, C, ldc};
+  if (g != nullptr && g->count < kMaxGemmGroup && (g->count == 0 || (g->K == K && g->accumulate == ep.accumulate)) &&
+      joins_group(dtype, M, N, K, p, ep)) {
+    bool clash = false;  // two gradients into one tensor keep their order
+    for (int i = 0; i < g->count; i++) clash = clash || g->p[i].C == C;
+    if (!clash) {
+      g->p[g->count++] = p;
+      g->K = K;
+      g->accumulate = ep.accumulate;
+      return FFK_OK;
+    }
+    int const rc = weight_grad_flush(st, *g);
+    if (rc != FFK_OK) return rc;
+  }
+  return gemm_dispatch(st, dtype, true, false, M, N, K, A, lda, B, ldb, C, ldc, ep);
 }
 
-int gemm_dispatch_pair(hipStream_t st, int dtype, bool ta, bool tb, int64_t K, GemmProblem const &p0,
-                       GemmProblem const &p1, bool accumulate) {
-  FFK_REQUIRE(gemm_pair_supported(dtype, ta, tb, K, p0, p1),
-              "gemm: these two problems do not run as one launch (ask gemm_pair_supported first)");
-  hipError_t e;
-  if (!ta && !tb) e = launch_pipe_pair<false, false>(st, p0, p1, (int)K, accumulate);
-  else if (!ta && tb) e = launch_pipe_pair<false, true>(st, p0, p1, (int)K, accumulate);
-  else if (ta && !tb) e = launch_pipe_pair<true, false>(st, p0, p1, (int)K, accumulate);
-  else e = launch_pipe_pair<true, true>(st, p0, p1, (int)K, accumulate);
+int weight_grad_flush(hipStream_t st, WeightGradGroup &g) {
+  int const n = g.count;
+  g.count = 0;
+  if (n == 0) return FFK_OK;
+  if (n == 1) {
+    GemmProblem const &p = g.p[0];
+    GemmEpilogue ep;
+    ep.accumulate = g.accumulate;
+    return gemm_dispatch(st, FFK_BF16, true, false, p.M, p.N, g.K, p.A, p.lda, p.B, p.ldb, p.C, p.ldc, ep);
+  }
+  hipError_t const e = pick_bf16_group<true, false>(st, g.p, n, (int)g.K, g.accumulate);
   FFK_HIP(e);
   return FFK_OK;
 }

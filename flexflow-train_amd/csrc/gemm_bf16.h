@@ -326,19 +326,22 @@ struct GemmTailArgs {
   float *colsum_partials;
 };
 
-// A second GEMM of the same kind and reduction length run by the same launch:
-// workgroups from first_tiles on compute it.
-struct GemmSecondProblem {
-  bf16 const *A, *B;
-  bf16 *C;
-  int M, N;
-  int64_t lda, ldb, ldc;
-  int first_tiles;  // number of tiles (= workgroups) of the first problem
+// Further GEMMs of the same kind and reduction length run by the same launch: workgroups from
+// first_tile of a problem on compute it.
+struct GemmGroupArgs {
+  struct Problem {
+    bf16 const *A, *B;
+    bf16 *C;
+    int64_t lda, ldb, ldc;
+    int M, N;
+    int first_tile;  // number of tiles (= workgroups) of the problems before it
+  } p[kMaxGemmGroup - 1];
+  int count;  // of p
 };
 
 // TAIL (GemmEpilogue::Tail): element-wise operators applied to the 8-element
 // pieces of the output tile on their way from LDS to memory.
-// PAIR: the launch carries two problems (no bias, no split-K).
+// GROUP: the launch carries several problems (no bias, no split-K).
 // EDGE: M, N and K need not be whole tiles (the operands still have to be readable 16 bytes at a
 // time).  Two ways:
 //   kEdgeOverlap (M >= BM, N >= BN): the last row and column of tiles begin early enough to lie inside
@@ -355,19 +358,23 @@ struct GemmSecondProblem {
 // LDS round trip and the MFMAs' own dependence stretch to some 600 cycles; a second group fills them
 // where there are too few tiles for a second workgroup per CU.
 template <int BM, int BN, int WM, int WN, int BK, int STAGES, int PF, bool TA, bool TB, int TAIL = 0,
-          bool PAIR = false, int EDGE = kEdgeNone, int KG = 1>
+          bool GROUP = false, int EDGE = kEdgeNone, int KG = 1>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pipe_kernel(
     bf16 const *__restrict__ A, bf16 const *__restrict__ B, bf16 *C, int M,
     int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
     bf16 const *__restrict__ bias, int act, int accumulate,
-    float *__restrict__ partial, int k_tiles_per_split, GemmTailArgs tail, GemmSecondProblem second) {
+    float *__restrict__ partial, int k_tiles_per_split, GemmTailArgs tail, GemmGroupArgs group) {
   int bid = blockIdx.x;
-  if constexpr (PAIR) {
-    if (bid >= second.first_tiles) {  // uniform over the workgroup
-      bid -= second.first_tiles;
-      A = second.A, B = second.B, C = second.C;
-      M = second.M, N = second.N;
-      lda = second.lda, ldb = second.ldb, ldc = second.ldc;
+  if constexpr (GROUP) {
+    int const id = bid;
+#pragma unroll
+    for (int q = 0; q < kMaxGemmGroup - 1; q++) {
+      if (q < group.count && id >= group.p[q].first_tile) {  // uniform over the workgroup
+        bid = id - group.p[q].first_tile;
+        A = group.p[q].A, B = group.p[q].B, C = group.p[q].C;
+        M = group.p[q].M, N = group.p[q].N;
+        lda = group.p[q].lda, ldb = group.p[q].ldb, ldc = group.p[q].ldc;
+      }
     }
   }
   // partial != nullptr: split-K.  Workgroup (tile, split) reduces k-tiles
@@ -390,7 +397,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
 
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
 
-  static_assert(KG == 1 || (EDGE == kEdgeBounded && !PAIR), "written for these");
+  static_assert(KG == 1 || EDGE == kEdgeBounded, "written for this");
   int const kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
   int const t = KG == 1 ? threadIdx.x : threadIdx.x % NT, lane = t & 63, wave = t >> 6;
   int const wm0 = (wave / (BN / WN)) * WM;
@@ -1152,7 +1159,7 @@ static hipError_t launch_pipe(hipStream_t st, bf16 const *A, bf16 const *B,
     float *partial = static_cast<float *>(ep.splitk_ws);
     kern<<<blocks * splits, NT, kLds, st>>>(A, B, C, M, N, K, lda, ldb, ldc, nullptr,
                                                 FFK_ACT_NONE, 0, partial, K / BK / splits, tail,
-                                                GemmSecondProblem{});
+                                                GemmGroupArgs{});
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     int64_t const quads = (int64_t)M * N / 4;
@@ -1163,25 +1170,32 @@ static hipError_t launch_pipe(hipStream_t st, bf16 const *A, bf16 const *B,
   }
   kern<<<blocks, NT, kLds, st>>>(A, B, C, M, N, K, lda, ldb, ldc,
                                      static_cast<bf16 const *>(ep.bias), ep.activation,
-                                     ep.accumulate, nullptr, 0, tail, GemmSecondProblem{});
+                                     ep.accumulate, nullptr, 0, tail, GemmGroupArgs{});
   return hipGetLastError();
 }
 
-// Two GEMMs of the same kind and reduction length on 128x128 tiles in one launch.
-template <bool TA, bool TB>
-hipError_t launch_pipe_pair(hipStream_t st, GemmProblem const &p0, GemmProblem const &p1, int K,
-                                   bool accumulate) {
-  using Cfg = PipeCfg<128, 128, 64, 32, 64, 4>;
-  constexpr int NT = Cfg::NW * 64;
-  auto kern = gemm_bf16_pipe_kernel<128, 128, 64, 32, 64, 4, 1, TA, TB, 0, true>;
+// Several GEMMs of the same kind and reduction length in one launch.
+template <int BM, int BN, int WM, int WN, int STAGES, int PF, bool TA, bool TB, int EDGE, int KG>
+static hipError_t launch_pipe_group(hipStream_t st, GemmProblem const *p, int n, int K, bool accumulate) {
+  using Cfg = PipeCfg<BM, BN, WM, WN, 64, STAGES>;
+  constexpr int NT = Cfg::NW * 64 * KG;
+  constexpr size_t kLds = KG == 1 ? Cfg::kLds : KG * Cfg::kStageBytes;
+  auto kern = gemm_bf16_pipe_kernel<BM, BN, WM, WN, 64, STAGES, PF, TA, TB, 0, true, EDGE, KG>;
   static LdsOptIn lds;
-  if (hipError_t e = lds.ensure(reinterpret_cast<void const *>(kern), (int)Cfg::kLds); e != hipSuccess) return e;
-  int const t0 = (int)((p0.M / 128) * (p0.N / 128)), t1 = (int)((p1.M / 128) * (p1.N / 128));
-  GemmSecondProblem const second = {static_cast<bf16 const *>(p1.A), static_cast<bf16 const *>(p1.B),
-                                    static_cast<bf16 *>(p1.C), (int)p1.M, (int)p1.N, p1.lda, p1.ldb, p1.ldc, t0};
-  kern<<<t0 + t1, NT, Cfg::kLds, st>>>(static_cast<bf16 const *>(p0.A), static_cast<bf16 const *>(p0.B),
-                                       static_cast<bf16 *>(p0.C), (int)p0.M, (int)p0.N, K, p0.lda, p0.ldb, p0.ldc,
-                                       nullptr, FFK_ACT_NONE, accumulate ? 1 : 0, nullptr, 0, GemmTailArgs{}, second);
+  if (hipError_t e = lds.ensure(reinterpret_cast<void const *>(kern), (int)kLds); e != hipSuccess) return e;
+  GemmGroupArgs g = {};
+  int64_t tiles = 0;
+  for (int i = 0; i < n; i++) {
+    if (i > 0) {
+      g.p[i - 1] = {static_cast<bf16 const *>(p[i].A), static_cast<bf16 const *>(p[i].B), static_cast<bf16 *>(p[i].C),
+                    p[i].lda, p[i].ldb, p[i].ldc, (int)p[i].M, (int)p[i].N, (int)tiles};
+    }
+    tiles += ceil_div(p[i].M, BM) * ceil_div(p[i].N, BN);
+  }
+  g.count = n - 1;
+  kern<<<(unsigned)tiles, NT, kLds, st>>>(static_cast<bf16 const *>(p[0].A), static_cast<bf16 const *>(p[0].B),
+                                         static_cast<bf16 *>(p[0].C), (int)p[0].M, (int)p[0].N, K, p[0].lda, p[0].ldb,
+                                         p[0].ldc, nullptr, FFK_ACT_NONE, accumulate ? 1 : 0, nullptr, 0, GemmTailArgs{}, g);
   return hipGetLastError();
 }
 
@@ -1274,6 +1288,26 @@ inline EdgeTile edge_tile_for(int M, int N, int K, bool wide_ok) {
   // one wave per SIMD where that kernel has what it takes, two otherwise
   consider(wide_ok && K >= 1024 ? kTile256Wide : kTile256, rounds(tiles(256, 256), kNumCU, 1.3));
   return best;
+}
+
+// A group of problems that each leave part of the chip idle: 128x128 tiles or 64x64 ones, whichever
+// the model above gives less time for all of them together.
+template <bool TA, bool TB>
+hipError_t pick_bf16_group(hipStream_t st, GemmProblem const *p, int n, int K, bool accumulate) {
+  bool exact = K % 64 == 0, fits = true;
+  double t64 = 0, t128 = 0;
+  for (int i = 0; i < n; i++) {
+    exact = exact && p[i].M % 128 == 0 && p[i].N % 128 == 0 && p[i].ldc % 8 == 0 && aligned16(p[i].C);
+    fits = fits && p[i].M >= 128 && p[i].N >= 128 && !(accumulate && p[i].N % 8 != 0);
+    t64 += (double)(ceil_div(p[i].M, 64) * ceil_div(p[i].N, 64));
+    t128 += (double)(ceil_div(p[i].M, 128) * ceil_div(p[i].N, 128));
+  }
+  double const kt = (double)ceil_div(K, 64);
+  double const us64 = t64 <= kNumCU ? kt * 0.17 + 1.0 : ceil(t64 / (2 * kNumCU)) * (kt * 0.39 + 1.0);
+  double const us128 = ceil(t128 / kNumCU) * (kt * 0.46 + 1.0);
+  if (!fits || us64 < us128) return launch_pipe_group<64, 64, 32, 32, 2, 3, TA, TB, kEdgeBounded, 2>(st, p, n, K, accumulate);
+  if (exact) return launch_pipe_group<128, 128, 64, 32, 4, 1, TA, TB, kEdgeNone, 1>(st, p, n, K, accumulate);
+  return launch_pipe_group<128, 128, 64, 32, 4, 1, TA, TB, kEdgeOverlap, 1>(st, p, n, K, accumulate);
 }
 
 template <bool TA, bool TB>

@@ -4,5 +4,4 @@
 namespace ffk {
 template hipError_t pick_bf16<false, true>(hipStream_t, bf16 const *, bf16 const *, bf16 *, int, int, int, int64_t, int64_t,
                                       int64_t, GemmEpilogue const &, bool);
-template hipError_t launch_pipe_pair<false, true>(hipStream_t, GemmProblem const &, GemmProblem const &, int, bool);
 }  // namespace ffk

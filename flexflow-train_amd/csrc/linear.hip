@@ -325,8 +325,7 @@ static int linear_backward_impl(
   if (weight_grad != nullptr) {
     ep.accumulate = (accumulate & FFK_ACC_WEIGHT) != 0;
     // weight_grad[out,in] = g[batch,out]^T . input[batch,in]
-    rc = gemm_dispatch(st, dtype, true, false, out_dim, in_dim, batch, g, out_dim,
-                       input, in_dim, weight_grad, in_dim, ep);
+    rc = weight_grad_dispatch(st, dtype, out_dim, in_dim, batch, g, out_dim, input, in_dim, weight_grad, in_dim, ep);
     if (rc != FFK_OK) return rc;
   }
   if (bias_grad != nullptr) {

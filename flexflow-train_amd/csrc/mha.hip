@@ -210,24 +210,19 @@ extern "C" int ffk_mha_backward(ffk_stream_t stream, int dtype,
   rc = gemm_dispatch(st, dtype, false, false, L.TQ, HDv, d->o_proj_size, output_grad,
                      d->o_proj_size, w + L.wo * es, HDv, dctx, HDv, over);
   if (rc != FFK_OK) return rc;
-  // The two weight gradients of a self-attention block (output projection and
-  // folded Q/K/V projection) have the same reduction length and each leaves
-  // part of the chip idle: where the library can, they run as ONE launch after
-  // the core's backward.
+  // The two weight gradients of a self-attention block (output projection and folded Q/K/V
+  // projection) have the same reduction length and each leaves part of the chip idle: they run as
+  // one launch after the core's backward (or later, with those of the layer around it).
   bool const folded = aliased && key_grad == nullptr && value_grad == nullptr;
-  GemmProblem const wo_grad = {d->o_proj_size, HDv, output_grad, d->o_proj_size, ctx, HDv,
-                               dw != nullptr ? dw + L.wo * es : nullptr, HDv};
-  GemmProblem const wqkv_grad = {row, d->q_size, dqkv, row, query, d->q_size,
-                                 dw != nullptr ? dw + L.wq * es : nullptr, d->q_size};
-  bool const paired = dw != nullptr && folded && gemm_pair_supported(dtype, true, false, L.TQ, wqkv_grad, wo_grad);
-  if (dw != nullptr && !paired) {
+  CollectWeightGrads collect(folded);
+  if (dw != nullptr) {
     // d(QKV projections) is not written before the core's backward: until
     // then it serves as split-K scratch for this small-output, long-K GEMM.
     GemmEpilogue acc_o = acc;
     acc_o.splitk_ws = dqkv;
     acc_o.splitk_ws_bytes = L.total - L.off_dqkv;
-    rc = gemm_dispatch(st, dtype, true, false, d->o_proj_size, HDv, L.TQ, output_grad,
-                       d->o_proj_size, ctx, HDv, dw + L.wo * es, HDv, acc_o);
+    rc = weight_grad_dispatch(st, dtype, d->o_proj_size, HDv, L.TQ, output_grad,
+                              d->o_proj_size, ctx, HDv, dw + L.wo * es, HDv, acc_o);
     if (rc != FFK_OK) return rc;
   }
 
@@ -254,15 +249,12 @@ extern "C" int ffk_mha_backward(ffk_stream_t stream, int dtype,
                          w + L.wq * es, d->q_size, query_grad, d->q_size, in_ep);
       if (rc != FFK_OK) return rc;
     }
-    if (paired) {
-      return gemm_dispatch_pair(st, dtype, true, false, L.TQ, wqkv_grad, wo_grad, acc.accumulate);
-    }
     if (dw != nullptr) {
-      rc = gemm_dispatch(st, dtype, true, false, row, d->q_size, L.TQ, dqkv, row, query,
-                         d->q_size, dw + L.wq * es, d->q_size, acc);
+      rc = weight_grad_dispatch(st, dtype, row, d->q_size, L.TQ, dqkv, row, query,
+                                d->q_size, dw + L.wq * es, d->q_size, acc);
       if (rc != FFK_OK) return rc;
     }
-    return FFK_OK;
+    return weight_grad_flush(st, collect.group);
   }
   struct Part {
     void const *x; void *dx; void const *dp; int64_t T, size, woff, HD;
