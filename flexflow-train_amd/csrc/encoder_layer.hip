@@ -153,28 +153,46 @@ extern "C" int ffk_encoder_layer_forward(ffk_stream_t st, int dtype,
     ffn_in = ws + L.h2;
   } else {
     // h1 = attn + x ; x1 = LN1(h1)
-    FFK_TRY(ffk_element_binary_forward(st, dtype, FFK_OP_EW_ADD, attn_res, x, ws + L.h1, T * E, T * E, T * E));
-    FFK_TRY(ffk_layer_norm_forward(st, dtype, ws + L.h1, ws + L.x1, w->ln1_gamma, w->ln1_beta,
-                                   mean(L.mean1), mean(L.rstd1), T, E, d->ln_eps));
+    int rc = FFK_ERR_UNSUPPORTED;
+    if (layer_fusion_enabled()) {  // the sum inside the LayerNorm: its dropout at a rate of zero
+      rc = dropout_add_layer_norm_forward(as_stream(st), dtype, attn_res, x, ws + L.h1, ws + L.x1, w->ln1_gamma, w->ln1_beta,
+                                          mean(L.mean1), mean(L.rstd1), T, E, d->ln_eps, 0.0f, 0, 0);
+      if (rc != FFK_OK && rc != FFK_ERR_UNSUPPORTED) return rc;
+    }
+    if (rc == FFK_ERR_UNSUPPORTED) {
+      FFK_TRY(ffk_element_binary_forward(st, dtype, FFK_OP_EW_ADD, attn_res, x, ws + L.h1, T * E, T * E, T * E));
+      FFK_TRY(ffk_layer_norm_forward(st, dtype, ws + L.h1, ws + L.x1, w->ln1_gamma, w->ln1_beta,
+                                     mean(L.mean1), mean(L.rstd1), T, E, d->ln_eps));
+    }
     ffn_in = ws + L.x1;
   }
   // dense(d_ff, activation) -> dropout -> dense(d_model) -> dropout
-  if (gelu) {
-    // (The GEMM could apply GELU and the dropout while it stores its tile --
-    // linear_gelu_dropout_forward -- but every CU reaches the store of its one
-    // tile at the same time, nothing overlaps the extra arithmetic, and the
-    // launch measured 55.6 us against 37.7 + 15.1 us for the two kernels here.)
-    FFK_TRY(ffk_linear_forward(st, dtype, FFK_ACT_NONE, ffn_in, ws + L.f1, w->w1, w->b1, T, E, F));
-  } else {
-    FFK_TRY(ffk_linear_forward(st, dtype, FFK_ACT_RELU, ffn_in, ws + L.act1, w->w1, w->b1, T, E, F));
+  int act_rc = FFK_ERR_UNSUPPORTED;
+  if (layer_fusion_enabled()) {
+    // The activation and the dropout on the GEMM's tile store: ReLU's at every size, GELU's where
+    // the GEMM runs on small tiles.  (On one large tile a CU every CU reaches its store at the same
+    // time and nothing overlaps the arithmetic: 55.6 us against 37.7 + 15.1 us for the two kernels
+    // at 4096 x 1024 -> 4096.)
+    act_rc = gelu ? linear_gelu_dropout_forward(as_stream(st), dtype, ffn_in, ws + L.f1, ws + L.act1_drop, w->w1, w->b1, T, E,
+                                                F, p, d->seed + 1, 0, true)
+                  : linear_relu_dropout_forward(as_stream(st), dtype, ffn_in, ws + L.act1, ws + L.act1_drop, w->w1, w->b1, T,
+                                                E, F, p, d->seed + 1, 0);
+    if (act_rc != FFK_OK && act_rc != FFK_ERR_UNSUPPORTED) return act_rc;
   }
-  if (gelu && layer_fusion_enabled() &&
-      dropout_fusable(dtype, ws + L.f1, nullptr, ws + L.act1_drop, T * F, 0)) {
-    // GELU's own output is not needed again: backward reads the pre-activation
-    FFK_TRY(gelu_dropout_forward(as_stream(st), dtype, ws + L.f1, ws + L.act1_drop, T * F, p, d->seed + 1, 0));
-  } else {
-    if (gelu) FFK_TRY(ffk_element_unary_forward(st, dtype, FFK_OP_GELU, 0.0f, ws + L.f1, ws + L.act1, T * F));
-    FFK_TRY(ffk_dropout_forward(st, dtype, ws + L.act1, ws + L.act1_drop, T * F, p, d->seed + 1, 0));
+  if (act_rc != FFK_OK) {
+    if (gelu) {
+      FFK_TRY(ffk_linear_forward(st, dtype, FFK_ACT_NONE, ffn_in, ws + L.f1, w->w1, w->b1, T, E, F));
+    } else {
+      FFK_TRY(ffk_linear_forward(st, dtype, FFK_ACT_RELU, ffn_in, ws + L.act1, w->w1, w->b1, T, E, F));
+    }
+    if (gelu && layer_fusion_enabled() &&
+        dropout_fusable(dtype, ws + L.f1, nullptr, ws + L.act1_drop, T * F, 0)) {
+      // GELU's own output is not needed again: backward reads the pre-activation
+      FFK_TRY(gelu_dropout_forward(as_stream(st), dtype, ws + L.f1, ws + L.act1_drop, T * F, p, d->seed + 1, 0));
+    } else {
+      if (gelu) FFK_TRY(ffk_element_unary_forward(st, dtype, FFK_OP_GELU, 0.0f, ws + L.f1, ws + L.act1, T * F));
+      FFK_TRY(ffk_dropout_forward(st, dtype, ws + L.act1, ws + L.act1_drop, T * F, p, d->seed + 1, 0));
+    }
   }
   // x1 + dropout(dense(d_model)): the dropout and the addition ride on the GEMM's tile store
   // where that kernel exists (backward reads neither the Linear's nor the dropout's output)
@@ -182,7 +200,7 @@ extern "C" int ffk_encoder_layer_forward(ffk_stream_t st, int dtype,
   int sum_rc = FFK_ERR_UNSUPPORTED;
   if (layer_fusion_enabled()) {
     sum_rc = linear_dropout_add_forward(as_stream(st), dtype, ws + L.act1_drop, ws + L.x1, ffn_sum, w->w2, w->b2,
-                                        T, F, E, p, d->seed + 2, 0);
+                                        T, F, E, p, d->seed + 2, 0, true);
     if (sum_rc != FFK_OK && sum_rc != FFK_ERR_UNSUPPORTED) return sum_rc;
   }
   if (sum_rc != FFK_OK) {
@@ -264,44 +282,53 @@ extern "C" int ffk_encoder_layer_backward(ffk_stream_t st, int dtype,
   int g_f1_rc = FFK_ERR_UNSUPPORTED;
   bool b1_done = false;  // the first Linear's bias gradient already computed
   void const *ffn_in = d->pre_layer_norm ? ws + L.h2 : ws + L.x1;
-  if (gelu && layer_fusion_enabled()) {
-    // the dropout's and GELU's backward ride on the tile store of the input-gradient GEMM
+  // what the activation's gradient is taken from: GELU's input, ReLU's output
+  void const *act_saved = gelu ? ws + L.f1 : ws + L.act1;
+  if (layer_fusion_enabled()) {
+    // the dropout's and the activation's backward ride on the tile store of the input-gradient GEMM
     // (52.7 us against 37.7 + 18.4 us: the separate kernel moves three tensors, this one adds one read)
     // ... and so do the column sums of what it stores, the first Linear's bias gradient
     if (g->b1 != nullptr) {
-      g_f1_rc = linear_backward_dropout_gelu(as_stream(st), dtype, ws + L.g_f2, ws + L.act1_drop, ws + L.f1,
+      g_f1_rc = linear_backward_dropout_gelu(as_stream(st), dtype, ws + L.g_f2, ws + L.act1_drop, act_saved,
                                              ws + L.g_f1, w->w2, g->w2, b2_grad, T, F, E, ws + L.lin_ws,
                                              lin_ws_bytes, wacc, p, d->seed + 1, 0, g->b1,
-                                             reinterpret_cast<float *>(ws + L.lin_ws_b), (wacc & FFK_ACC_BIAS) != 0);
+                                             reinterpret_cast<float *>(ws + L.lin_ws_b), (wacc & FFK_ACC_BIAS) != 0, true, !gelu);
       b1_done = g_f1_rc == FFK_OK;
     }
     if (g_f1_rc == FFK_ERR_UNSUPPORTED) {
-      g_f1_rc = linear_backward_dropout_gelu(as_stream(st), dtype, ws + L.g_f2, ws + L.act1_drop, ws + L.f1,
+      g_f1_rc = linear_backward_dropout_gelu(as_stream(st), dtype, ws + L.g_f2, ws + L.act1_drop, act_saved,
                                              ws + L.g_f1, w->w2, g->w2, b2_grad, T, F, E, ws + L.lin_ws,
-                                             lin_ws_bytes, wacc, p, d->seed + 1, 0);
+                                             lin_ws_bytes, wacc, p, d->seed + 1, 0, nullptr, nullptr, false, true, !gelu);
     }
     if (g_f1_rc != FFK_OK && g_f1_rc != FFK_ERR_UNSUPPORTED) return g_f1_rc;
   }
-  bool const g_f1_ready = g_f1_rc == FFK_OK;
+  bool g_f1_ready = g_f1_rc == FFK_OK;
   if (!g_f1_ready) {
     FFK_TRY(ffk_linear_backward(st, dtype, FFK_ACT_NONE, 0, ws + L.f2, ws + L.g_f2, ws + L.act1_drop,
                                 ws + L.g_act1_drop, w->w2, g->w2, b2_grad, T, F, E, ws + L.lin_ws, lin_ws_bytes,
                                 wacc));
-  }
-  bool const fuse_gelu_bwd = g_f1_ready || (gelu && layer_fusion_enabled() &&
-                             dropout_fusable(dtype, ws + L.g_act1_drop, ws + L.f1, ws + L.g_f1, T * F, 0));
-  if (g_f1_ready) {
-  } else if (fuse_gelu_bwd) {
-    FFK_TRY(dropout_backward_gelu_backward(as_stream(st), dtype, ws + L.g_act1_drop, ws + L.f1, ws + L.g_f1,
-                                           T * F, p, d->seed + 1, 0));
-  } else {
-    FFK_TRY(ffk_dropout_backward(st, dtype, ws + L.g_act1_drop, ws + L.g_act1, T * F, p, d->seed + 1, 0, 0));
-  }
-  if (gelu) {
-    if (!fuse_gelu_bwd) {
-      FFK_TRY(ffk_element_unary_backward(st, dtype, FFK_OP_GELU, 0.0f, ws + L.act1, ws + L.g_act1, ws + L.f1,
-                                         ws + L.g_f1, T * F, 0));
+    if (gelu && layer_fusion_enabled() && dropout_fusable(dtype, ws + L.g_act1_drop, ws + L.f1, ws + L.g_f1, T * F, 0)) {
+      FFK_TRY(dropout_backward_gelu_backward(as_stream(st), dtype, ws + L.g_act1_drop, ws + L.f1, ws + L.g_f1,
+                                             T * F, p, d->seed + 1, 0));
+      g_f1_ready = true;
+    } else {
+      FFK_TRY(ffk_dropout_backward(st, dtype, ws + L.g_act1_drop, ws + L.g_act1, T * F, p, d->seed + 1, 0, 0));
+      if (gelu) {
+        FFK_TRY(ffk_element_unary_backward(st, dtype, FFK_OP_GELU, 0.0f, ws + L.act1, ws + L.g_act1, ws + L.f1,
+                                           ws + L.g_f1, T * F, 0));
+        g_f1_ready = true;
+      }
     }
+  }
+  // post-LN: the gradient reaching x1 is g_h2 + g_sum, the sum on the GEMM's tile store where it can be
+  int x1_rc = FFK_ERR_UNSUPPORTED;
+  if (!d->pre_layer_norm && g_f1_ready && layer_fusion_enabled()) {
+    x1_rc = linear_backward_add_residual(as_stream(st), dtype, ws + L.g_f1, ffn_in, g_sum, ws + L.g_x1, w->w1, g->w1,
+                                         b1_done ? nullptr : g->b1, T, E, F, ws + L.lin_ws_b, lin_ws_bytes, wacc);
+    if (x1_rc != FFK_OK && x1_rc != FFK_ERR_UNSUPPORTED) return x1_rc;
+  }
+  if (x1_rc == FFK_OK) {
+  } else if (g_f1_ready) {
     FFK_TRY(ffk_linear_backward(st, dtype, FFK_ACT_NONE, 0, ws + L.f1, ws + L.g_f1, ffn_in, ws + L.g_h2,
                                 w->w1, g->w1, b1_done ? nullptr : g->b1, T, E, F,
                                 ws + L.lin_ws_b, lin_ws_bytes, wacc));
@@ -329,7 +356,7 @@ extern "C" int ffk_encoder_layer_backward(ffk_stream_t st, int dtype,
                                       ws + L.g_x1, g->ln2_gamma, g->ln2_beta, T, E, ws + L.ln_ws, ln_ws_bytes, ln_mode));
       FFK_TRY(ffk_element_binary_forward(st, dtype, FFK_OP_EW_ADD, ws + L.g_x1, dy, ws + L.g_x1, T * E, T * E, T * E));
     }
-  } else {
+  } else if (x1_rc != FFK_OK) {
     FFK_TRY(ffk_element_binary_forward(st, dtype, FFK_OP_EW_ADD, ws + L.g_h2, g_sum, ws + L.g_x1, T * E, T * E, T * E));
   }
   // ---- attention block backward
@@ -357,9 +384,11 @@ extern "C" int ffk_encoder_layer_backward(ffk_stream_t st, int dtype,
     FFK_TRY(ffk_layer_norm_backward(st, dtype, ws + L.g_x1, ws + L.h1, mean(L.mean1), mean(L.rstd1), w->ln1_gamma,
                                     ws + L.g_attn, g->ln1_gamma, g->ln1_beta, T, E, ws + L.ln_ws_b, ln_ws_bytes, ln_mode));
     g_attn_res = ws + L.g_attn;
-    FFK_TRY(ffk_mha_backward(st, dtype, &m, x, dx, x, nullptr, x, nullptr, w->attn_weight, g->attn_weight,
-                             g_attn_res, ws + L.mha_reserve, L.ln_ws - L.mha_reserve, mha_mode));
-    FFK_TRY(ffk_element_binary_forward(st, dtype, FFK_OP_EW_ADD, dx, g_attn_res, dx, T * E, T * E, T * E));
+    bool added = false;
+    FFK_TRY(mha_backward_add_residual(as_stream(st), dtype, &m, x, dx, layer_fusion_enabled() ? g_attn_res : nullptr, &added,
+                                      w->attn_weight, g->attn_weight, g_attn_res, ws + L.mha_reserve,
+                                      L.ln_ws - L.mha_reserve, mha_mode));
+    if (!added) FFK_TRY(ffk_element_binary_forward(st, dtype, FFK_OP_EW_ADD, dx, g_attn_res, dx, T * E, T * E, T * E));
   }
   FFK_TRY(weight_grad_flush(as_stream(st), weight_grads.group));
   FFK_HIP(colreduce_flush(as_stream(st), reductions));

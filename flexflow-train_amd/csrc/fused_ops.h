@@ -35,6 +35,12 @@ int gelu_dropout_forward(hipStream_t st, int dtype, void const *x, void *y,
 int linear_gelu_dropout_forward(hipStream_t st, int dtype, void const *input, void *output,
                                 void *dropped, void const *weight, void const *bias, int64_t batch,
                                 int64_t in_dim, int64_t out_dim, float rate, uint64_t seed,
+                                uint64_t offset, bool any_size = false);
+
+// output = relu(input . weight^T + bias) (stored), dropped = dropout(output), as above.
+int linear_relu_dropout_forward(hipStream_t st, int dtype, void const *input, void *output,
+                                void *dropped, void const *weight, void const *bias, int64_t batch,
+                                int64_t in_dim, int64_t out_dim, float rate, uint64_t seed,
                                 uint64_t offset);
 
 // output = residual + dropout(input . weight^T + bias); Linear's own output
@@ -42,7 +48,7 @@ int linear_gelu_dropout_forward(hipStream_t st, int dtype, void const *input, vo
 int linear_dropout_add_forward(hipStream_t st, int dtype, void const *input, void const *residual,
                                void *output, void const *weight, void const *bias, int64_t batch,
                                int64_t in_dim, int64_t out_dim, float rate, uint64_t seed,
-                               uint64_t offset);
+                               uint64_t offset, bool any_size = false);
 
 // Linear backward (no activation) whose input gradient is
 // dropout_backward(output_grad . weight) * GELU'(gelu_input): the gradient of
@@ -59,7 +65,24 @@ int linear_backward_dropout_gelu(hipStream_t st, int dtype, void const *output_g
                                  // colsum_partials_elems(batch, in_dim) that nothing else uses until the
                                  // sums are complete
                                  void *input_grad_colsum = nullptr, float *colsum_partials = nullptr,
-                                 bool colsum_accumulate = false);
+                                 bool colsum_accumulate = false, bool any_size = false,
+                                 // the operator in front of the dropout was a ReLU whose output is
+                                 // gelu_input, not a GELU with that input
+                                 bool relu = false);
+
+// Linear backward (no activation) whose input gradient is residual + output_grad . weight, the product
+// rounded to the storage type first: what a separate element-wise add of the stored gradient gives.
+// FFK_ERR_UNSUPPORTED as above, before any launch.
+int linear_backward_add_residual(hipStream_t st, int dtype, void const *output_grad, void const *input, void const *residual,
+                                 void *input_grad, void const *weight, void *weight_grad, void *bias_grad, int64_t batch,
+                                 int64_t in_dim, int64_t out_dim, void *workspace, size_t workspace_bytes, int accumulate);
+
+// ffk_mha_backward of a self-attention block (one tensor as query, key and value) whose query_grad is
+// residual + the block's input gradient, rounded as above; *added says whether it is (false: query_grad is
+// the plain gradient).
+int mha_backward_add_residual(hipStream_t st, int dtype, ffk_mha_desc_t const *d, void const *x, void *x_grad,
+                              void const *residual, bool *added, void const *weight, void *weight_grad,
+                              void const *output_grad, void *reserve, size_t reserve_bytes, int accumulate);
 
 // summed = residual + dropout(in); y = LayerNorm(summed), statistics kept as the separate
 // LayerNorm would.  Returns FFK_ERR_UNSUPPORTED (without setting an error

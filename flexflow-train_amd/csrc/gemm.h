@@ -23,14 +23,20 @@ struct GemmEpilogue {
   //                        plain result is not stored
   //   kTailDropoutAdd      C = tail_in + dropout(result); the plain result is
   //                        not stored
+  //   kTailDropoutReluGrad C = dropout_backward(result) where tail_in > 0, else 0
+  //   kTailActDropout      C = act(result), tail_out = dropout(C)
   // tail_in / tail_out are dense [M, N] tensors, the dropout stream is indexed
   // by m * N + n from tail_dropout.offset.
-  enum Tail { kTailNone = 0, kTailGeluDropout = 1, kTailDropoutGeluGrad = 2, kTailDropoutAdd = 3 };
+  enum Tail { kTailNone = 0, kTailGeluDropout = 1, kTailDropoutGeluGrad = 2, kTailDropoutAdd = 3,
+              kTailDropoutReluGrad = 4, kTailActDropout = 5 };
   int tail = kTailNone;
+  // also sizes that are no whole tiles, or fewer than fill the chip (the encoder layer; the entry
+  // points keep to the sizes they document)
+  bool tail_any_size = false;
   void const *tail_in = nullptr;
   void *tail_out = nullptr;
   DropoutParams tail_dropout = {};
-  // kTailDropoutGeluGrad, optional: the GEMM also leaves the partial column
+  // kTailDropout*Grad, optional: the GEMM also leaves the partial column
   // sums of what it stores (colsum_partials_elems(M, N) floats, the partials
   // colsum_dispatch would compute from the stored tensor); colsum_finish adds
   // them up into the column sums (+)= out.

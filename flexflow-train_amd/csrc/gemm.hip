@@ -32,6 +32,10 @@ FFK_EXTERN_BF16(false, true);
 FFK_EXTERN_BF16(true, false);
 FFK_EXTERN_BF16(true, true);
 #undef FFK_EXTERN_BF16
+extern template hipError_t pick_bf16_tail<false, false>(hipStream_t, bf16 const *, bf16 const *, bf16 *, int, int, int, int64_t,
+                                                        int64_t, int64_t, GemmEpilogue const &);
+extern template hipError_t pick_bf16_tail<false, true>(hipStream_t, bf16 const *, bf16 const *, bf16 *, int, int, int, int64_t,
+                                                       int64_t, int64_t, GemmEpilogue const &);
 extern template hipError_t pick_bf16_group<true, false>(hipStream_t, GemmProblem const *, int, int, bool);
 
 size_t gemm_splitk_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
@@ -165,9 +169,9 @@ static int64_t colsum_rows_per_split(int64_t M) {
 
 int colsum_finish(hipStream_t st, int dtype, float const *partials, int64_t M, int64_t N, void *out,
                   bool accumulate) {
-  FFK_REQUIRE(dtype == FFK_BF16 && M % kColsumRowsPerBlock == 0 && colsum_rows_per_split(M) == kColsumRowsPerBlock,
+  FFK_REQUIRE(dtype == FFK_BF16 && colsum_rows_per_split(M) == kColsumRowsPerBlock,
               "colsum_finish: partials of this shape do not come from a GEMM tail");
-  FFK_HIP(colreduce_launch<bf16>(st, partials, (int)(M / kColsumRowsPerBlock), (int)N, (int)N,
+  FFK_HIP(colreduce_launch<bf16>(st, partials, (int)ceil_div(M, kColsumRowsPerBlock), (int)N, (int)N,
                                  static_cast<bf16 *>(out), nullptr, accumulate));
   return FFK_OK;
 }
@@ -303,20 +307,36 @@ bool gemm_tail_supported(int dtype, bool ta, bool tb, int64_t M, int64_t N, int6
   if (dtype != FFK_BF16 || ta || ep.accumulate || ldc != N || M <= 0 || N <= 0 || K <= 0) return false;
   if (M >= (1ll << 31) || N >= (1ll << 31) || K >= (1ll << 31)) return false;
   if ((ep.tail_dropout.offset & 7) != 0) return false;
-  if (ep.tail == GemmEpilogue::kTailGeluDropout) {
-    if (!tb || ep.tail_out == nullptr || !aligned16(ep.tail_out)) return false;
-  } else if (ep.tail == GemmEpilogue::kTailDropoutGeluGrad) {
-    if (tb || ep.tail_in == nullptr || !aligned16(ep.tail_in)) return false;
-    if (ep.tail_colsum_partials != nullptr && colsum_rows_per_split(M) != kColsumRowsPerBlock) return false;
-  } else if (ep.tail == GemmEpilogue::kTailDropoutAdd) {
-    if (!tb || ep.tail_in == nullptr || !aligned16(ep.tail_in)) return false;
-  } else {
-    return false;
+  bool sums = false;
+  switch (ep.tail) {
+    case GemmEpilogue::kTailGeluDropout:
+    case GemmEpilogue::kTailActDropout:
+      if (!tb || ep.tail_out == nullptr || !aligned16(ep.tail_out)) return false;
+      break;
+    case GemmEpilogue::kTailDropoutGeluGrad:
+    case GemmEpilogue::kTailDropoutReluGrad:
+      if (tb || ep.tail_in == nullptr || !aligned16(ep.tail_in)) return false;
+      sums = true;
+      if (ep.tail_colsum_partials != nullptr && colsum_rows_per_split(M) != kColsumRowsPerBlock) return false;
+      break;
+    case GemmEpilogue::kTailDropoutAdd:
+      if (ep.tail_in == nullptr || !aligned16(ep.tail_in) || (!tb && !ep.tail_any_size)) return false;
+      break;
+    default: return false;
   }
+  int const variant = gemm_variant_override();
   bool const vec_ok = (K % 8 == 0) && (lda % 8 == 0) && (ldb % 8 == 0) && aligned16(A) && aligned16(B) &&
                       (tb || N % 8 == 0);
-  return vec_ok && pipe_tile_for(static_cast<bf16 const *>(C), (int)M, (int)N, (int)K, lda, ldb, ldc, ep,
-                                 gemm_variant_override()) != 0;
+  if (!vec_ok) return false;
+  if (pipe_tile_for(static_cast<bf16 const *>(C), (int)M, (int)N, (int)K, lda, ldb, ldc, ep, variant) != 0) {
+    // with one 256x256 or 128x128 tile a CU every CU reaches its store at the same time and nothing
+    // overlaps GELU's arithmetic: two kernels are as soon done
+    return !(ep.tail_any_size && ep.tail == GemmEpilogue::kTailGeluDropout);
+  }
+  if (!ep.tail_any_size || variant != 0 || N % 8 != 0 || !aligned16(C) || !edge_operands_ok(lda, ldb)) return false;
+  bool const splits = edge_splits_reduction((int)M, (int)N, (int)K, ep);
+  if (ep.tail == GemmEpilogue::kTailGeluDropout) return splits;
+  return splits || sums || (M >= 128 && N >= 128);
 }
 
 int gemm_dispatch(hipStream_t st, int dtype, bool ta, bool tb, int64_t M,
@@ -355,6 +375,9 @@ int gemm_dispatch(hipStream_t st, int dtype, bool ta, bool tb, int64_t M,
           a, b, c, (int)M, (int)N, (int)K, lda, ldb, ldc, ta, tb,
           static_cast<bf16 const *>(ep.bias), ep.activation, ep.accumulate);
       e = hipGetLastError();
+    } else if (ep.tail != GemmEpilogue::kTailNone) {
+      e = tb ? pick_bf16_tail<false, true>(st, a, b, c, (int)M, (int)N, (int)K, lda, ldb, ldc, ep)
+             : pick_bf16_tail<false, false>(st, a, b, c, (int)M, (int)N, (int)K, lda, ldb, ldc, ep);
     } else if (!ta && !tb) {
       e = pick_bf16<false, false>(st, a, b, c, (int)M, (int)N, (int)K, lda, ldb, ldc, ep, vec_ok);
     } else if (!ta && tb) {

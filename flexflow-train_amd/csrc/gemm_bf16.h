@@ -1,6 +1,6 @@
 // The bf16 MFMA kernels behind gemm.hip, and the rules that choose among them.  A template of the
-// transposes that gemm_nn.hip, gemm_nt.hip, gemm_tn.hip and gemm_tt.hip each instantiate once (the
-// kernels take minutes to compile; four files compile side by side).
+// transposes that gemm_nn.hip, gemm_nt.hip, gemm_tn.hip, gemm_tt.hip and gemm_tail_*.hip instantiate
+// (the kernels take minutes to compile; these files compile side by side).
 #pragma once
 #include "lds_dma.h"
 #include "gemm.h"
@@ -321,7 +321,7 @@ struct GemmTailArgs {
   bf16 const *in;
   bf16 *out;
   DropoutParams dropout;
-  // kTailDropoutGeluGrad only, optional: [M / 32][N] sums of 32-row blocks of
+  // kTailDropout*Grad only, optional: [M / 32][N] sums of 32-row blocks of
   // what the tail stores, added up in colsum_partial_vec_kernel's order
   float *colsum_partials;
 };
@@ -920,6 +920,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   // Each wave stages its own WM x WN tile and writes it out in 16-byte chunks.
   bf16 *cs = smem + wave * (WM * CS);
   constexpr int CCH = WM * WN / 8 / 64;  // 16-byte chunks per lane
+  constexpr bool kColsums = TAIL == GemmEpilogue::kTailDropoutGeluGrad || TAIL == GemmEpilogue::kTailDropoutReluGrad;
   // The activation is a compile-time functor here: a per-element switch inside
   // the unrolled loops made the epilogue several times longer than the GEMM's
   // own store traffic.
@@ -993,10 +994,12 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
         }
         // ldc == N here: `at` is the element's index in the dense tensor, and
         // the piece is one block of the dropout stream
-        uint32_t w[4];
-        philox4x32_10((tail.dropout.offset + (uint64_t)at) >> 3, tail.dropout.key, w);
+        uint32_t w[4] = {0u, 0u, 0u, 0u};
+        if (tail.dropout.threshold != 0) {  // (uniform: at a rate of zero everything is kept)
+          philox4x32_10((tail.dropout.offset + (uint64_t)at) >> 3, tail.dropout.key, w);
+        }
         u32x4 aux = {0u, 0u, 0u, 0u};
-        if constexpr (TAIL == GemmEpilogue::kTailGeluDropout) {
+        if constexpr (TAIL == GemmEpilogue::kTailGeluDropout || TAIL == GemmEpilogue::kTailActDropout) {
           *reinterpret_cast<u32x4 *>(dst + at) = v;
         } else {
           aux = *reinterpret_cast<u32x4 const *>(tail.in + at);
@@ -1015,22 +1018,25 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
             if constexpr (TAIL == GemmEpilogue::kTailDropoutGeluGrad) {
               x[h] = storage_round<bf16>(x[h]) * gelu_derivative(a[h]);
             }
+            if constexpr (TAIL == GemmEpilogue::kTailDropoutReluGrad) {
+              x[h] = a[h] > 0.0f ? x[h] : 0.0f;
+            }
             if constexpr (TAIL == GemmEpilogue::kTailDropoutAdd) {
               x[h] = storage_round<bf16>(x[h]) + a[h];
             }
           }
           r[q] = pack_bf16x2(x[0], x[1]);
         }
-        bf16 *const to = TAIL == GemmEpilogue::kTailGeluDropout ? tail.out : dst;
+        bf16 *const to = TAIL == GemmEpilogue::kTailGeluDropout || TAIL == GemmEpilogue::kTailActDropout ? tail.out : dst;
         *reinterpret_cast<u32x4 *>(to + at) = r;
-        if constexpr (TAIL == GemmEpilogue::kTailDropoutGeluGrad) {
+        if constexpr (kColsums) {
           // kept for the column sums below (the lane's own piece: no other lane reads it before the barrier)
           if (tail.colsum_partials != nullptr) *reinterpret_cast<u32x4 *>(cs + row * CS + ch * 8) = r;
         }
       }
     }
     }  // half
-    if constexpr (TAIL == GemmEpilogue::kTailDropoutGeluGrad) {
+    if constexpr (kColsums) {
       if (tail.colsum_partials != nullptr) {  // uniform over the launch
         __syncthreads();
         // A lane owns a column of the wave's tile; per block of 32 rows: four
@@ -1049,7 +1055,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
               run[q] = acc_rows;
             }
             int64_t const part = (m0 + wm0) / kColsumRowsPerBlock + blk;
-            static_assert(EDGE != kEdgeOverlap || TAIL != GemmEpilogue::kTailDropoutGeluGrad, "blocks of 32 rows begin at multiples of 32");
+            static_assert(EDGE != kEdgeOverlap, "blocks of 32 rows begin at multiples of 32");
             if (EDGE == kEdgeBounded && (part * kColsumRowsPerBlock >= M || n0 + wn0 + col >= N)) continue;
             tail.colsum_partials[part * N + n0 + wn0 + col] = (run[0] + run[1]) + (run[2] + run[3]);
           }
@@ -1290,6 +1296,53 @@ inline EdgeTile edge_tile_for(int M, int N, int K, bool wide_ok) {
   return best;
 }
 
+// Whether the plain kernel for this ragged or small problem is one of the two 64x64 ones, whose waves
+// split the reduction (an epilogue's tail then has to run on that tile too for the same bits), and not
+// one of the larger ones, which all add up in the same order.
+inline bool edge_splits_reduction(int M, int N, int K, GemmEpilogue const &ep) {
+  EdgeTile const t = edge_tile_for(M, N, K, ep.activation == FFK_ACT_NONE);
+  int const bm = t == kTile256 || t == kTile256Wide ? 256 : 128, bn = t == kTile128x64 ? 64 : bm;
+  return t == kTile64 || t == kTile64Deep || M < bm || N < bn;
+}
+
+// A GEMM with element-wise operators on its tile store.  gemm_tail_supported has been asked.
+template <int TAIL, bool TA, bool TB>
+static hipError_t launch_tail(hipStream_t st, bf16 const *A, bf16 const *B, bf16 *C, int M, int N, int K, int64_t lda,
+                              int64_t ldb, int64_t ldc, GemmEpilogue const &ep) {
+  int const tile = pipe_tile_for(C, M, N, K, lda, ldb, ldc, ep, gemm_variant_override());
+  if (tile == 256) return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB, TAIL>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+  if (tile == 128) return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, TAIL>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+  if (edge_splits_reduction(M, N, K, ep)) {
+    return launch_pipe<64, 64, 32, 32, 64, 2, 3, TA, TB, TAIL, kEdgeBounded, 2>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+  }
+  // column sums are taken over blocks of 32 rows from multiples of 32 on, where overlapping tiles do not begin
+  constexpr bool sums = TAIL == GemmEpilogue::kTailDropoutGeluGrad || TAIL == GemmEpilogue::kTailDropoutReluGrad;
+  constexpr int edge = sums ? kEdgeBounded : kEdgeOverlap;
+  if (!sums && (M < 128 || N < 128)) return hipErrorInvalidValue;
+  return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, TAIL, edge>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+}
+template <bool TA, bool TB>
+hipError_t pick_bf16_tail(hipStream_t st, bf16 const *A, bf16 const *B, bf16 *C, int M, int N, int K, int64_t lda,
+                          int64_t ldb, int64_t ldc, GemmEpilogue const &ep) {
+  switch (ep.tail) {
+    case GemmEpilogue::kTailDropoutAdd:
+      return launch_tail<GemmEpilogue::kTailDropoutAdd, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+    case GemmEpilogue::kTailGeluDropout:
+      if constexpr (TB) return launch_tail<GemmEpilogue::kTailGeluDropout, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+      break;
+    case GemmEpilogue::kTailActDropout:
+      if constexpr (TB) return launch_tail<GemmEpilogue::kTailActDropout, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+      break;
+    case GemmEpilogue::kTailDropoutGeluGrad:
+      if constexpr (!TB) return launch_tail<GemmEpilogue::kTailDropoutGeluGrad, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+      break;
+    case GemmEpilogue::kTailDropoutReluGrad:
+      if constexpr (!TB) return launch_tail<GemmEpilogue::kTailDropoutReluGrad, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+      break;
+  }
+  return hipErrorInvalidValue;
+}
+
 // A group of problems that each leave part of the chip idle: 128x128 tiles or 64x64 ones, whichever
 // the model above gives less time for all of them together.
 template <bool TA, bool TB>
@@ -1319,35 +1372,6 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
   {
     bool const fits128 = M % 128 == 0 && N % 128 == 0;
     bool const use256 = pipe_tile == 256, use128 = pipe_tile == 128;
-    if (ep.tail != GemmEpilogue::kTailNone) {
-      // gemm_tail_supported() has been asked: one of the two tiles fits
-      if constexpr (!TA && TB) {
-        constexpr int kTail = GemmEpilogue::kTailGeluDropout;
-        if (ep.tail == kTail && use256) {
-          return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB, kTail>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
-        }
-        if (ep.tail == kTail && use128) {
-          return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, kTail>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
-        }
-        constexpr int kAdd = GemmEpilogue::kTailDropoutAdd;
-        if (ep.tail == kAdd && use256) {
-          return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB, kAdd>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
-        }
-        if (ep.tail == kAdd && use128) {
-          return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, kAdd>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
-        }
-      }
-      if constexpr (!TA && !TB) {
-        constexpr int kTail = GemmEpilogue::kTailDropoutGeluGrad;
-        if (ep.tail == kTail && use256) {
-          return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB, kTail>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
-        }
-        if (ep.tail == kTail && use128) {
-          return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, kTail>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
-        }
-      }
-      return hipErrorInvalidValue;
-    }
     // An output that 256x256 tiles cover in a ragged last round but 256x192 tiles cover in whole
     // rounds of the chip (the attention block's fused Q/K/V projection: [4096, 3072] is 192 tiles of
     // the first kind on 256 CUs, 256 of the second): one wave per SIMD on 128x96 wave tiles.  Only
@@ -1387,7 +1411,6 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
       return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
     }
   }
-  if (ep.tail != GemmEpilogue::kTailNone) return hipErrorInvalidValue;
   if (variant != 1 && edge_operands_ok(lda, ldb)) {
     EdgeTile tile = edge_tile_for(M, N, K, ep.activation == FFK_ACT_NONE && ldc % 8 == 0);
     bool const forced = variant == 64 || variant == 65 || variant == 70 || variant == 128 || variant == 256 || variant == 264;

@@ -12,6 +12,7 @@
 //           bias_grad (+)= column sums of g (linear_kernels.cu:249-334).
 #include "elementwise.h"
 #include "gemm.h"
+#include "fused_ops.h"
 #include "small_f32.h"
 
 namespace ffk {
@@ -363,12 +364,13 @@ namespace ffk {
 int linear_gelu_dropout_forward(hipStream_t st, int dtype, void const *input, void *output,
                                 void *dropped, void const *weight, void const *bias, int64_t batch,
                                 int64_t in_dim, int64_t out_dim, float rate, uint64_t seed,
-                                uint64_t offset) {
+                                uint64_t offset, bool any_size) {
   FFK_REQUIRE(input && output && dropped && weight, "linear_gelu_dropout_forward: NULL tensor");
   FFK_REQUIRE(batch > 0 && in_dim > 0 && out_dim > 0, "linear_gelu_dropout_forward: non-positive dimension");
   GemmEpilogue ep;
   ep.bias = bias;
   ep.tail = GemmEpilogue::kTailGeluDropout;
+  ep.tail_any_size = any_size;
   ep.tail_out = dropped;
   int const prc = make_dropout_params("linear_gelu_dropout_forward", rate, seed, offset, ep.tail_dropout);
   if (prc != FFK_OK) return prc;
@@ -380,15 +382,33 @@ int linear_gelu_dropout_forward(hipStream_t st, int dtype, void const *input, vo
                        output, out_dim, ep);
 }
 
+int linear_relu_dropout_forward(hipStream_t st, int dtype, void const *input, void *output, void *dropped,
+                                void const *weight, void const *bias, int64_t batch, int64_t in_dim, int64_t out_dim,
+                                float rate, uint64_t seed, uint64_t offset) {
+  GemmEpilogue ep;
+  ep.bias = bias;
+  ep.activation = FFK_ACT_RELU;
+  ep.tail = GemmEpilogue::kTailActDropout;
+  ep.tail_any_size = true;
+  ep.tail_out = dropped;
+  int const prc = make_dropout_params("linear_relu_dropout_forward", rate, seed, offset, ep.tail_dropout);
+  if (prc != FFK_OK) return prc;
+  if (!gemm_tail_supported(dtype, false, true, batch, out_dim, in_dim, input, in_dim, weight, in_dim, output, out_dim, ep)) {
+    return FFK_ERR_UNSUPPORTED;
+  }
+  return gemm_dispatch(st, dtype, false, true, batch, out_dim, in_dim, input, in_dim, weight, in_dim, output, out_dim, ep);
+}
+
 int linear_dropout_add_forward(hipStream_t st, int dtype, void const *input, void const *residual,
                                void *output, void const *weight, void const *bias, int64_t batch,
                                int64_t in_dim, int64_t out_dim, float rate, uint64_t seed,
-                               uint64_t offset) {
+                               uint64_t offset, bool any_size) {
   FFK_REQUIRE(input && residual && output && weight, "linear_dropout_add_forward: NULL tensor");
   FFK_REQUIRE(batch > 0 && in_dim > 0 && out_dim > 0, "linear_dropout_add_forward: non-positive dimension");
   GemmEpilogue ep;
   ep.bias = bias;
   ep.tail = GemmEpilogue::kTailDropoutAdd;
+  ep.tail_any_size = any_size;
   ep.tail_in = residual;
   int const prc = make_dropout_params("linear_dropout_add_forward", rate, seed, offset, ep.tail_dropout);
   if (prc != FFK_OK) return prc;
@@ -405,7 +425,8 @@ int linear_backward_dropout_gelu(hipStream_t st, int dtype, void const *output_g
                                  void *weight_grad, void *bias_grad, int64_t batch, int64_t in_dim,
                                  int64_t out_dim, void *workspace, size_t workspace_bytes,
                                  int accumulate, float rate, uint64_t seed, uint64_t offset,
-                                 void *input_grad_colsum, float *colsum_partials, bool colsum_accumulate) {
+                                 void *input_grad_colsum, float *colsum_partials, bool colsum_accumulate,
+                                 bool any_size, bool relu) {
   FFK_REQUIRE(output_grad && input && gelu_input && input_grad && weight,
               "linear_backward_dropout_gelu: NULL tensor");
   FFK_REQUIRE(input_grad_colsum == nullptr || colsum_partials != nullptr,
@@ -413,7 +434,8 @@ int linear_backward_dropout_gelu(hipStream_t st, int dtype, void const *output_g
   FFK_REQUIRE((accumulate & FFK_ACC_INPUT) == 0,
               "linear_backward_dropout_gelu: the input gradient is stored, not added");
   GemmEpilogue tail;
-  tail.tail = GemmEpilogue::kTailDropoutGeluGrad;
+  tail.tail = relu ? GemmEpilogue::kTailDropoutReluGrad : GemmEpilogue::kTailDropoutGeluGrad;
+  tail.tail_any_size = any_size;
   tail.tail_in = gelu_input;
   tail.tail_colsum_partials = input_grad_colsum != nullptr ? colsum_partials : nullptr;
   int const prc = make_dropout_params("linear_backward_dropout_gelu", rate, seed, offset, tail.tail_dropout);
@@ -423,6 +445,20 @@ int linear_backward_dropout_gelu(hipStream_t st, int dtype, void const *output_g
                                       accumulate, &tail);
   if (rc != FFK_OK || input_grad_colsum == nullptr) return rc;
   return colsum_finish(st, dtype, colsum_partials, batch, in_dim, input_grad_colsum, colsum_accumulate);
+}
+
+int linear_backward_add_residual(hipStream_t st, int dtype, void const *output_grad, void const *input, void const *residual,
+                                 void *input_grad, void const *weight, void *weight_grad, void *bias_grad, int64_t batch,
+                                 int64_t in_dim, int64_t out_dim, void *workspace, size_t workspace_bytes, int accumulate) {
+  GemmEpilogue tail;
+  tail.tail = GemmEpilogue::kTailDropoutAdd;  // at a rate of zero
+  tail.tail_any_size = true;
+  tail.tail_in = residual;
+  int const prc = make_dropout_params("linear_backward_add_residual", 0.0f, 0, 0, tail.tail_dropout);
+  if (prc != FFK_OK) return prc;
+  return linear_backward_impl(st, dtype, FFK_ACT_NONE, 0, nullptr, output_grad, input, input_grad, weight, weight_grad,
+                              bias_grad, batch, in_dim, out_dim, workspace, workspace_bytes, accumulate & ~FFK_ACC_INPUT,
+                              &tail);
 }
 
 }  // namespace ffk

@@ -16,6 +16,7 @@
 // Reserve space layout (bytes, each region 256-byte aligned):
 //   QKV projections | context | lse | delta | d(context) | d(QKV projections)
 #include "gemm.h"
+#include "fused_ops.h"
 
 namespace ffk {
 
@@ -170,14 +171,12 @@ extern "C" int ffk_mha_forward(ffk_stream_t stream, int dtype,
                        w + L.wo * es, HDv, output, d->o_proj_size, ep);
 }
 
-extern "C" int ffk_mha_backward(ffk_stream_t stream, int dtype,
-                                ffk_mha_desc_t const *d, void const *query,
-                                void *query_grad, void const *key,
-                                void *key_grad, void const *value,
-                                void *value_grad, void const *weight,
-                                void *weight_grad, void const *output_grad,
-                                void *reserve, size_t reserve_bytes,
-                                int accumulate) {
+// residual != nullptr (self-attention on one tensor): query_grad = residual + gradient where the library
+// has that kernel (*added says so).
+static int mha_backward_impl(ffk_stream_t stream, int dtype, ffk_mha_desc_t const *d, void const *query, void *query_grad,
+                             void const *key, void *key_grad, void const *value, void *value_grad, void const *weight,
+                             void *weight_grad, void const *output_grad, void *reserve, size_t reserve_bytes, int accumulate,
+                             void const *residual, bool *added) {
   int rc = check_mha("mha_backward", dtype, d);
   if (rc != FFK_OK) return rc;
   FFK_REQUIRE(query && key && value && weight && output_grad, "mha_backward: NULL tensor");
@@ -245,6 +244,17 @@ extern "C" int ffk_mha_backward(ffk_stream_t stream, int dtype,
   if (folded) {
     // dX (+)= dQKV[T,row] . [W_Q; W_K; W_V]  and  dW_QKV += dQKV^T . X
     if (query_grad != nullptr) {
+      if (residual != nullptr && !in_ep.accumulate) {
+        GemmEpilogue tail;
+        tail.tail = GemmEpilogue::kTailDropoutAdd;  // at a rate of zero
+        tail.tail_any_size = true;
+        tail.tail_in = residual;
+        rc = make_dropout_params("mha_backward", 0.0f, 0, 0, tail.tail_dropout);
+        if (rc != FFK_OK) return rc;
+        *added = gemm_tail_supported(dtype, false, false, L.TQ, d->q_size, row, dqkv, row, w + L.wq * es, d->q_size,
+                                     query_grad, d->q_size, tail);
+        if (*added) in_ep = tail;
+      }
       rc = gemm_dispatch(st, dtype, false, false, L.TQ, d->q_size, row, dqkv, row,
                          w + L.wq * es, d->q_size, query_grad, d->q_size, in_ep);
       if (rc != FFK_OK) return rc;
@@ -279,3 +289,23 @@ extern "C" int ffk_mha_backward(ffk_stream_t stream, int dtype,
   }
   return FFK_OK;
 }
+
+extern "C" int ffk_mha_backward(ffk_stream_t stream, int dtype, ffk_mha_desc_t const *d, void const *query,
+                                void *query_grad, void const *key, void *key_grad, void const *value,
+                                void *value_grad, void const *weight, void *weight_grad, void const *output_grad,
+                                void *reserve, size_t reserve_bytes, int accumulate) {
+  return mha_backward_impl(stream, dtype, d, query, query_grad, key, key_grad, value, value_grad, weight, weight_grad,
+                           output_grad, reserve, reserve_bytes, accumulate, nullptr, nullptr);
+}
+
+namespace ffk {
+
+int mha_backward_add_residual(hipStream_t st, int dtype, ffk_mha_desc_t const *d, void const *x, void *x_grad,
+                              void const *residual, bool *added, void const *weight, void *weight_grad,
+                              void const *output_grad, void *reserve, size_t reserve_bytes, int accumulate) {
+  *added = false;
+  return mha_backward_impl(st, dtype, d, x, x_grad, x, nullptr, x, nullptr, weight, weight_grad, output_grad, reserve,
+                           reserve_bytes, accumulate, residual, added);
+}
+
+}  // namespace ffk
