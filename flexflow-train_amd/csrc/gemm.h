@@ -6,12 +6,27 @@
 
 namespace ffk {
 
+// The gradient before a Linear's activation, from its output y and output gradient dy.
+template <int ACT>
+__device__ __forceinline__ float activation_grad(int relu_mode, float y, float dy) {
+  if (ACT == FFK_ACT_NONE) return dy;
+  if (ACT == FFK_ACT_RELU) {
+    if (relu_mode == 1) return dy > 0.0f ? 1.0f : 0.0f;  // linear_kernels_cpu.cc:46-52,69-71
+    return y > 0.0f ? dy : 0.0f;                         // cuda_helper.cu:60-64
+  }
+  if (ACT == FFK_ACT_SIGMOID) return dy * y * (1.0f - y);  // cuda_helper.cu:87-91
+  return dy * (1.0f - y * y);                              // tanh
+}
+
 struct GemmEpilogue {
   void const *bias = nullptr;  // [N] in the GEMM dtype, added to every row
   int activation = FFK_ACT_NONE;
   bool accumulate = false;     // C += result instead of C = result
-  // Optional fp32 scratch for split-K (used when the output has too few tiles
-  // to occupy the chip); gemm_splitk_workspace_bytes() says how much helps.
+  // A's rows (M or K elements) are followed by zeros up to the next multiple of 8 elements, which
+  // belong to its memory (bf16, trans_b == false): it is read 16 bytes at a time whatever the length
+  bool a_padded = false;
+  // Optional scratch for split-K, used when the output has too few tiles to occupy the chip: as many
+  // splits as it has room for fp32 copies of the output, and as help.
   void *splitk_ws = nullptr;
   size_t splitk_ws_bytes = 0;
   // Optional element-wise operators applied to the output tile while it is
@@ -96,10 +111,6 @@ int weight_grad_dispatch(hipStream_t stream, int dtype, int64_t M, int64_t N, in
 // Runs what was collected (nothing to do for an empty group) and empties it.
 int weight_grad_flush(hipStream_t stream, WeightGradGroup &group);
 
-// Scratch bytes with which a bf16 GEMM of this shape would split its reduction
-// (0: it would not).
-size_t gemm_splitk_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K);
-
 // out[N] (+)= sum over the M rows of X[M,N] (ldx row stride); `partials` is
 // fp32 scratch of colsum_partials_elems(M, N) floats.
 int64_t colsum_partials_elems(int64_t M, int64_t N);
@@ -111,6 +122,11 @@ int64_t colsum_partials_elems(int64_t M, int64_t N);
 int dropout_backward_colsum(hipStream_t stream, int dtype, void const *dy, void *dx, int64_t M,
                             int64_t N, void *colsum, bool accumulate, float *partials,
                             DropoutParams const &drop);
+// g[M,N] = act'(y) * dy (activation none: a copy) with rows of ldg elements, and colsum (+)= the column
+// sums of what is stored (nullptr: not wanted), one pass over dy and y; the columns of g from N to the
+// next whole 16 bytes, if ldg has them, become zeros.
+int linear_grad(hipStream_t stream, int dtype, int activation, int relu_mode, void const *y, void const *dy, void *g,
+                int64_t ldg, int64_t M, int64_t N, void *colsum, bool accumulate, float *partials);
 int colsum_dispatch(hipStream_t stream, int dtype, void const *X, int64_t ldx,
                     int64_t M, int64_t N, void *out, bool accumulate,
                     float *partials);

@@ -38,12 +38,6 @@ extern template hipError_t pick_bf16_tail<false, true>(hipStream_t, bf16 const *
                                                        int64_t, int64_t, GemmEpilogue const &);
 extern template hipError_t pick_bf16_group<true, false>(hipStream_t, GemmProblem const *, int, int, bool);
 
-size_t gemm_splitk_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
-  if (dtype != FFK_BF16 || M % 128 != 0 || N % 128 != 0) return 0;
-  int const s = splitk_splits(M, N, K, ~(size_t)0);
-  return s > 1 ? (size_t)s * (size_t)(M * N) * sizeof(float) : 0;
-}
-
 // ---------------------------------------------------------------------------
 // Plain kernel for bf16 shapes the tiled kernel cannot take.
 // ---------------------------------------------------------------------------
@@ -70,88 +64,103 @@ __global__ __launch_bounds__(256) void gemm_bf16_plain_kernel(
 // ---------------------------------------------------------------------------
 // Column sums (bias gradient): out[n] (+)= sum_m X[m,n]
 // ---------------------------------------------------------------------------
+// First pass: a thread reads 16 bytes (8 bf16 / 4 fp32 columns) of kColsumRowsPerLane rows, all
+// loads independent; 64 threads span the columns, the 4 row lanes of the workgroup meet in LDS.
+// What is summed, and on the way written to G, is given by OP:
+//   kSumOnly   X itself (nothing written)
+//   kSumDrop   the dropout's backward of X, rounded as stored (dense, ldx == N: a lane's V elements
+//              are a Philox block or half of one)
+//   kSumAct    act'(Y) * X, rounded as stored: the gradient before a Linear's activation (for an
+//              activation of "none" a copy).  ldg may be longer than a row: the columns behind it up
+//              to the next whole 16 bytes become zeros, for readers that take 16 bytes at a time.
+// ANY: rows of any length at any address.
+// Memory bound.  [2048, 50257] bf16 at odd addresses: the copy with its sums 83 us (5 TB/s); the
+// sums alone took 95 us one element at a time.
+enum ColsumOp { kSumOnly = 0, kSumDrop = 1, kSumAct = 2 };
 template <typename T>
-__global__ __launch_bounds__(256) void colsum_partial_kernel(
-    T const *__restrict__ X, int64_t ldx, int M, int N, int rows_per_split,
-    float *__restrict__ partials) {
-  __shared__ float red[4][64];
-  int const cx = threadIdx.x & 63;
-  int const ry = threadIdx.x >> 6;
-  int const n = blockIdx.x * 64 + cx;
-  int const r0 = blockIdx.y * rows_per_split;
-  int const r1 = min(M, r0 + rows_per_split);
-  float s = 0.0f;
-  if (n < N) {
-    for (int m = r0 + ry; m < r1; m += 4) {
-      s += VecIO<T>::load1(X + (int64_t)m * ldx + n);
-    }
-  }
-  red[ry][cx] = s;
-  __syncthreads();
-  if (ry == 0 && n < N) {
-    partials[(int64_t)blockIdx.y * N + n] =
-        red[0][cx] + red[1][cx] + red[2][cx] + red[3][cx];
-  }
-}
-
-// Vectorised first pass: a thread reads 16 bytes (8 bf16 / 4 fp32 columns) of
-// kColsumRowsPerLane rows, all loads independent; 64 threads span the columns,
-// the 4 row lanes of the workgroup meet in LDS.
-
-// DROP: X is the gradient of a dropout's output; what is summed is the
-// dropout's backward of it, rounded as stored, which is also written to G
-// (dense, ldx == N: a lane's V elements are a Philox block or half of one).
-template <typename T, bool DROP>
-__global__ __launch_bounds__(256) void colsum_partial_vec_kernel(
-    T const *__restrict__ X, int64_t ldx, int M, int N, int rows_per_split,
-    float *__restrict__ partials, T *__restrict__ G, DropoutParams drop) {
+struct ColsumArgs {
+  T const *X, *Y;
+  T *G;
+  int64_t ldx, ldg;
+  int M, N, rows_per_split;
+  float *partials;  // nullptr: no sums wanted
+  DropoutParams drop;
+  int relu_mode;
+};
+template <typename T, int OP, int ACT, bool ANY>
+__global__ __launch_bounds__(256) void colsum_partial_vec_kernel(ColsumArgs<T> a) {
   constexpr int V = VecIO<T>::kVec;
   __shared__ float red[4][64][V + 1];
   int const cx = threadIdx.x & 63;
   int const ry = threadIdx.x >> 6;
   int const n = (blockIdx.x * 64 + cx) * V;
-  int const r0 = blockIdx.y * rows_per_split;
-  int const r1 = min(M, r0 + rows_per_split);
+  int const r0 = blockIdx.y * a.rows_per_split;
+  int const r1 = min(a.M, r0 + a.rows_per_split);
+  int const N = a.N;
+  int const exist = ANY ? min(V, N - n) : V;  // of this thread's columns
   float s[V];
 #pragma unroll
   for (int e = 0; e < V; e++) s[e] = 0.0f;
+  auto load = [&](T const *p) -> u32x4 {
+    if constexpr (ANY) return exist == V ? load_raw_any(p) : load_raw_first(p, exist);
+    return load_raw_stream(p);
+  };
   if (n < N) {
     for (int m0 = r0 + ry * kColsumRowsPerLane; m0 < r1; m0 += kColsumRowsPerBlock) {
-      float v[kColsumRowsPerLane][V];
+      u32x4 x[kColsumRowsPerLane], y[kColsumRowsPerLane];
 #pragma unroll
       for (int i = 0; i < kColsumRowsPerLane; i++) {
-        int const m = min(m0 + i, r1 - 1);  // clamped rows are masked below
-        VecIO<T>::load_stream(X + (int64_t)m * ldx + n, v[i]);
+        int64_t const m = min(m0 + i, r1 - 1);  // clamped rows are masked below
+        x[i] = load(a.X + m * a.ldx + n);
+        if constexpr (OP == kSumAct && ACT != FFK_ACT_NONE) y[i] = load(a.Y + m * a.ldx + n);
       }
 #pragma unroll
       for (int i = 0; i < kColsumRowsPerLane; i++) {
         if (m0 + i < r1) {
-          if constexpr (DROP) {
-            uint64_t const e0 = drop.offset + (uint64_t)(m0 + i) * (uint64_t)N + (uint64_t)n;
+          float v[V];
+          unpack_raw(x[i], v, (T const *)nullptr);
+          if constexpr (OP == kSumDrop) {
+            uint64_t const e0 = a.drop.offset + (uint64_t)(m0 + i) * (uint64_t)N + (uint64_t)n;
             uint32_t w[4];
-            philox4x32_10(e0 >> 3, drop.key, w);
+            philox4x32_10(e0 >> 3, a.drop.key, w);
             if (V == 4 && (e0 & 4)) {  // upper half of the block
               w[0] = w[2];
               w[1] = w[3];
             }
 #pragma unroll
-            for (int e = 0; e < V; e++) v[i][e] = storage_round<T>(keep(w, e, drop) ? v[i][e] * drop.scale : 0.0f);
-            VecIO<T>::store(G + (int64_t)(m0 + i) * ldx + n, v[i]);
+            for (int e = 0; e < V; e++) v[e] = storage_round<T>(keep(w, e, a.drop) ? v[e] * a.drop.scale : 0.0f);
+            VecIO<T>::store(a.G + (int64_t)(m0 + i) * a.ldg + n, v);
+          }
+          if constexpr (OP == kSumAct) {
+            if constexpr (ACT != FFK_ACT_NONE) {
+              float out[V];
+              unpack_raw(y[i], out, (T const *)nullptr);
+#pragma unroll
+              for (int e = 0; e < V; e++) v[e] = storage_round<T>(activation_grad<ACT>(a.relu_mode, out[e], v[e]));
+            }
+            T *const to = a.G + (int64_t)(m0 + i) * a.ldg + n;
+            u32x4 const raw = pack_raw(v, (T const *)nullptr);
+            if (!ANY || n + V <= a.ldg) {
+              store_raw_any(to, raw);
+            } else {
+              store_raw_first(to, raw, exist);
+            }
           }
 #pragma unroll
-          for (int e = 0; e < V; e++) s[e] += v[i][e];
+          for (int e = 0; e < V; e++) s[e] += v[e];
         }
       }
     }
   }
+  if (a.partials == nullptr) return;  // uniform over the launch
 #pragma unroll
   for (int e = 0; e < V; e++) red[ry][cx][e] = s[e];
   __syncthreads();
   if (ry == 0 && n < N) {
 #pragma unroll
     for (int e = 0; e < V; e++) {
-      partials[(int64_t)blockIdx.y * N + n + e] =
-          (red[0][cx][e] + red[1][cx][e]) + (red[2][cx][e] + red[3][cx][e]);
+      if (ANY && e >= exist) break;
+      a.partials[(int64_t)blockIdx.y * N + n + e] = (red[0][cx][e] + red[1][cx][e]) + (red[2][cx][e] + red[3][cx][e]);
     }
   }
 }
@@ -180,46 +189,66 @@ int64_t colsum_partials_elems(int64_t M, int64_t N) {
   return (int64_t)colsum_splits(M) * N;
 }
 
-// dropped != nullptr: the sums are taken over dropout_backward(X), which is
-// written to dropped; vector shapes only (FFK_ERR_UNSUPPORTED otherwise, before
-// any launch).
-template <typename T>
-static int colsum_typed(hipStream_t st, T const *X, int64_t ldx, int64_t M,
-                        int64_t N, T *out, bool accumulate, float *partials,
-                        T *dropped = nullptr, DropoutParams const *drop = nullptr) {
-  constexpr int V = VecIO<T>::kVec;
-  int const splits = colsum_splits(M);
-  int rows_per_split = (int)ceil_div(M, splits);
-  bool const vec = (N % V == 0) && (ldx % V == 0) && aligned16(X);
-  if (dropped != nullptr) {
-    if (!vec || ldx != N || !aligned16(dropped) || (drop->offset & 7) != 0 || M >= (1ll << 31) || N >= (1ll << 31)) {
-      return FFK_ERR_UNSUPPORTED;
-    }
-    rows_per_split = (int)(ceil_div(rows_per_split, kColsumRowsPerBlock) * kColsumRowsPerBlock);
-    int const used = (int)ceil_div(M, rows_per_split);
-    dim3 grid((unsigned)ceil_div(N, 64 * V), (unsigned)used);
-    colsum_partial_vec_kernel<T, true><<<grid, 256, 0, st>>>(X, ldx, (int)M, (int)N, rows_per_split, partials,
-                                                            dropped, *drop);
-    FFK_CHECK_LAUNCH();
-    FFK_HIP(colreduce_launch<T>(st, partials, used, (int)N, (int)N, out, nullptr, accumulate));
-    return FFK_OK;
-  }
-  if (vec) {
-    // whole row blocks per split so that only the last split has a ragged end
-    rows_per_split = (int)(ceil_div(rows_per_split, kColsumRowsPerBlock) * kColsumRowsPerBlock);
-    int const used = (int)ceil_div(M, rows_per_split);
-    dim3 grid((unsigned)ceil_div(N, 64 * V), (unsigned)used);
-    colsum_partial_vec_kernel<T, false><<<grid, 256, 0, st>>>(X, ldx, (int)M, (int)N, rows_per_split, partials,
-                                                             nullptr, DropoutParams{});
-    FFK_CHECK_LAUNCH();
-    FFK_HIP(colreduce_launch<T>(st, partials, used, (int)N, (int)N, out, nullptr, accumulate));
-    return FFK_OK;
-  }
-  dim3 grid((unsigned)ceil_div(N, 64), (unsigned)splits);
-  colsum_partial_kernel<T><<<grid, 256, 0, st>>>(X, ldx, (int)M, (int)N, rows_per_split, partials);
+// The launch of one kernel of the first pass and, where sums are wanted, of the second.
+template <int OP, int ACT, bool ANY, typename T>
+static int colsum_launch(hipStream_t st, ColsumArgs<T> a, T *out, bool accumulate) {
+  // whole row blocks per split so that only the last split has a ragged end
+  a.rows_per_split = (int)colsum_rows_per_split(a.M);
+  int const used = (int)ceil_div(a.M, a.rows_per_split);
+  dim3 grid((unsigned)ceil_div(a.N, 64 * VecIO<T>::kVec), (unsigned)used);
+  colsum_partial_vec_kernel<T, OP, ACT, ANY><<<grid, 256, 0, st>>>(a);
   FFK_CHECK_LAUNCH();
-  FFK_HIP(colreduce_launch<T>(st, partials, splits, (int)N, (int)N, out, nullptr, accumulate));
+  if (out != nullptr) FFK_HIP(colreduce_launch<T>(st, a.partials, used, a.N, a.N, out, nullptr, accumulate));
   return FFK_OK;
+}
+
+template <typename T>
+static int colsum_typed(hipStream_t st, T const *X, int64_t ldx, int64_t M, int64_t N, T *out, bool accumulate,
+                        float *partials) {
+  ColsumArgs<T> const a = {X, nullptr, nullptr, ldx, 0, (int)M, (int)N, 0, partials, {}, 0};
+  bool const vec = N % VecIO<T>::kVec == 0 && ldx % VecIO<T>::kVec == 0 && aligned16(X);
+  return vec ? colsum_launch<kSumOnly, FFK_ACT_NONE, false>(st, a, out, accumulate)
+             : colsum_launch<kSumOnly, FFK_ACT_NONE, true>(st, a, out, accumulate);
+}
+
+template <typename T>
+static int dropout_backward_colsum_typed(hipStream_t st, T const *dy, T *dx, int64_t M, int64_t N, T *out, bool accumulate,
+                                         float *partials, DropoutParams const &drop) {
+  if (N % VecIO<T>::kVec != 0 || !aligned16(dy) || !aligned16(dx) || (drop.offset & 7) != 0 || M >= (1ll << 31) ||
+      N >= (1ll << 31)) {
+    return FFK_ERR_UNSUPPORTED;  // before any launch
+  }
+  ColsumArgs<T> const a = {dy, nullptr, dx, N, N, (int)M, (int)N, 0, partials, drop, 0};
+  return colsum_launch<kSumDrop, FFK_ACT_NONE, false>(st, a, out, accumulate);
+}
+
+template <int ACT, typename T>
+static int linear_grad_act(hipStream_t st, ColsumArgs<T> const &a, T *out, bool accumulate) {
+  constexpr int V = VecIO<T>::kVec;
+  bool const vec = a.N % V == 0 && a.ldg % V == 0 && aligned16(a.X) && aligned16(a.Y) && aligned16(a.G);
+  return vec ? colsum_launch<kSumAct, ACT, false>(st, a, out, accumulate) : colsum_launch<kSumAct, ACT, true>(st, a, out, accumulate);
+}
+template <typename T>
+static int linear_grad_typed(hipStream_t st, int act, int relu_mode, T const *y, T const *dy, T *g, int64_t ldg, int64_t M,
+                             int64_t N, T *colsum, bool accumulate, float *partials) {
+  ColsumArgs<T> const a = {dy, y, g, N, ldg, (int)M, (int)N, 0, colsum != nullptr ? partials : nullptr, {}, relu_mode};
+  switch (act) {
+    case FFK_ACT_NONE: return linear_grad_act<FFK_ACT_NONE>(st, a, colsum, accumulate);
+    case FFK_ACT_RELU: return linear_grad_act<FFK_ACT_RELU>(st, a, colsum, accumulate);
+    case FFK_ACT_SIGMOID: return linear_grad_act<FFK_ACT_SIGMOID>(st, a, colsum, accumulate);
+    default: return linear_grad_act<FFK_ACT_TANH>(st, a, colsum, accumulate);
+  }
+}
+
+int linear_grad(hipStream_t st, int dtype, int act, int relu_mode, void const *y, void const *dy, void *g, int64_t ldg,
+                int64_t M, int64_t N, void *colsum, bool accumulate, float *partials) {
+  FFK_REQUIRE(M < (1ll << 31) && N < (1ll << 31), "linear_grad: dimension exceeds 2^31");
+  if (dtype == FFK_FLOAT) {
+    return linear_grad_typed(st, act, relu_mode, static_cast<float const *>(y), static_cast<float const *>(dy),
+                             static_cast<float *>(g), ldg, M, N, static_cast<float *>(colsum), accumulate, partials);
+  }
+  return linear_grad_typed(st, act, relu_mode, static_cast<bf16 const *>(y), static_cast<bf16 const *>(dy),
+                           static_cast<bf16 *>(g), ldg, M, N, static_cast<bf16 *>(colsum), accumulate, partials);
 }
 
 int colsum_dispatch(hipStream_t st, int dtype, void const *X, int64_t ldx,
@@ -242,12 +271,12 @@ int dropout_backward_colsum(hipStream_t st, int dtype, void const *dy, void *dx,
   FFK_REQUIRE(dy && dx && colsum && partials, "dropout_backward_colsum: NULL operand");
   FFK_REQUIRE(M > 0 && N > 0, "dropout_backward_colsum: non-positive dimension");
   if (dtype == FFK_FLOAT) {
-    return colsum_typed<float>(st, static_cast<float const *>(dy), N, M, N, static_cast<float *>(colsum),
-                               accumulate, partials, static_cast<float *>(dx), &drop);
+    return dropout_backward_colsum_typed(st, static_cast<float const *>(dy), static_cast<float *>(dx), M, N,
+                                         static_cast<float *>(colsum), accumulate, partials, drop);
   }
   if (dtype == FFK_BF16) {
-    return colsum_typed<bf16>(st, static_cast<bf16 const *>(dy), N, M, N, static_cast<bf16 *>(colsum),
-                              accumulate, partials, static_cast<bf16 *>(dx), &drop);
+    return dropout_backward_colsum_typed(st, static_cast<bf16 const *>(dy), static_cast<bf16 *>(dx), M, N,
+                                         static_cast<bf16 *>(colsum), accumulate, partials, drop);
   }
   return FFK_ERR_UNSUPPORTED;
 }
@@ -334,7 +363,7 @@ bool gemm_tail_supported(int dtype, bool ta, bool tb, int64_t M, int64_t N, int6
     return !(ep.tail_any_size && ep.tail == GemmEpilogue::kTailGeluDropout);
   }
   if (!ep.tail_any_size || variant != 0 || N % 8 != 0 || !aligned16(C) || !edge_operands_ok(lda, ldb)) return false;
-  bool const splits = edge_splits_reduction((int)M, (int)N, (int)K, ep);
+  bool const splits = gemm_splits_reduction((int)M, (int)N, (int)K, ep);
   if (ep.tail == GemmEpilogue::kTailGeluDropout) return splits;
   return splits || sums || (M >= 128 && N >= 128);
 }
@@ -363,8 +392,8 @@ int gemm_dispatch(hipStream_t st, int dtype, bool ta, bool tb, int64_t M,
     bf16 const *b = static_cast<bf16 const *>(B);
     bf16 *c = static_cast<bf16 *>(C);
     // 16-byte chunks: the contiguous extent of each operand (K, or M / N) must be a multiple of 8
-    // elements, rows 16-byte aligned.
-    bool vec_ok = (ta ? M % 8 == 0 : K % 8 == 0) && (tb ? K % 8 == 0 : N % 8 == 0) && (lda % 8 == 0) &&
+    // elements, or padded to one, rows 16-byte aligned.
+    bool vec_ok = ((ta ? M % 8 == 0 : K % 8 == 0) || (ep.a_padded && !tb)) && (tb ? K % 8 == 0 : N % 8 == 0) && (lda % 8 == 0) &&
                   (ldb % 8 == 0) && aligned16(A) && aligned16(B) && K > 0;
     // Operands that are not: the register-staged kernel, but for products of so few elements that
     // one thread an output is over as soon.

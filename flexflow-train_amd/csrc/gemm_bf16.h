@@ -31,16 +31,16 @@ __device__ __forceinline__ float apply_activation(float v, int act) {
 // Block -> tile mapping.  Workgroups are dealt round-robin to the 8 XCDs, each
 // with its own L2; regroup ids so that one XCD works on a compact patch of the
 // output (tiles that share A rows / B columns), then walk the patch in groups
-// of kGroupM tile rows.
+// of kGroupM tile rows.  (xcds: how many of them share these tiles.)
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void tile_coords(int pid, int nbm, int nbn, int &tm,
-                                            int &tn) {
+                                            int &tn, int xcds = kNumXCD) {
   int const total = nbm * nbn;
   {
     // XCD x gets a contiguous run of total / 8 tiles, the first total % 8 of them one more
-    int const xcd = pid % kNumXCD;
-    int const local = pid / kNumXCD;
-    pid = xcd * (total / kNumXCD) + min(xcd, total % kNumXCD) + local;
+    int const xcd = pid % xcds;
+    int const local = pid / xcds;
+    pid = xcd * (total / xcds) + min(xcd, total % xcds) + local;
   }
   constexpr int kGroupM = 8;
   int const group_size = kGroupM * nbn;
@@ -405,11 +405,22 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   int tm, tn;
   int const nbm = EDGE ? (M + BM - 1) / BM : M / BM, nbn = EDGE ? (N + BN - 1) / BN : N / BN;
   int const tiles = nbm * nbn;
-  int const split = partial != nullptr ? bid / tiles : 0;
-  tile_coords(partial != nullptr ? bid % tiles : bid, nbm, nbn, tm, tn);
+  int split = 0;
+  if (partial == nullptr) {
+    tile_coords(bid, nbm, nbn, tm, tn);
+  } else {
+    // an XCD's workgroups take the same split: its part of the operands then passes through that
+    // L2 alone
+    int const splits = gridDim.x / tiles;
+    split = bid % splits;
+    tile_coords(bid / splits, nbm, nbn, tm, tn, splits < kNumXCD ? kNumXCD / splits : 1);
+  }
   // (kEdgeOverlap) what of the tile is this workgroup's to store begins at first_m, first_n
   int const first_m = tm * BM, first_n = tn * BN;
-  int const m0 = EDGE == kEdgeOverlap ? min(first_m, M - BM) : first_m, n0 = EDGE == kEdgeOverlap ? min(first_n, N - BN) : first_n;
+  // (an operand whose contiguous index is M may be padded to whole 16-byte chunks: rows past M are
+  // loaded then, and not stored)
+  int const M_loads = TA && EDGE ? (M + 7) & ~7 : M, K_loads = !TA && EDGE ? (K + 7) & ~7 : K;
+  int const m0 = EDGE == kEdgeOverlap ? min(first_m, M_loads - BM) : first_m, n0 = EDGE == kEdgeOverlap ? min(first_n, N - BN) : first_n;
   // first k-tile of this workgroup, or of this group of waves
   int const kt0 = KG == 1 ? split * k_tiles_per_split : kg * (((K + BK - 1) / BK + KG - 1) / KG);
 
@@ -465,7 +476,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   bf16 const *const panel_a = TA ? A + m0 : A + (int64_t)m0 * lda;
   bf16 const *const panel_b = TBL ? B + n0 : B + (int64_t)n0 * ldb;
   // one past the last element of the operand that a workgroup may read, from its panel's start
-  int64_t const end_a = EDGE != kEdgeBounded ? 0 : TA ? (int64_t)(K - 1) * lda + (M - m0) : (int64_t)(min(BM, M - m0) - 1) * lda + K;
+  int64_t const end_a = EDGE != kEdgeBounded ? 0 : TA ? (int64_t)(K - 1) * lda + (M_loads - m0) : (int64_t)(min(BM, M - m0) - 1) * lda + K_loads;
   int64_t const end_b = EDGE != kEdgeBounded ? 0 : TBL ? (int64_t)(K - 1) * ldb + (N - n0) : (int64_t)(min(BN, N - n0) - 1) * ldb + K;
 
   // LDS destinations of the direct loads are scalar byte addresses: base + stage + chunk row
@@ -821,7 +832,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   auto store8 = [&](int m, int n, u32x4 v) __attribute__((always_inline)) {
     bf16 *const to = C + (int64_t)m * ldc + n;
     if constexpr (EDGE == kEdgeOverlap) {
-      if (m < first_m || n + 8 <= first_n) return;
+      if (m < first_m || n + 8 <= first_n || (TA && m >= M)) return;
       store_raw_any(to, v);
     } else if constexpr (EDGE == kEdgeBounded) {
       if (m >= M || n >= N) return;
@@ -957,7 +968,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
             bf16 const *const from = dst + (int64_t)(m0 + wm0 + m) * ldc + n0 + wn0 + n;
             u32x2 old = {0u, 0u};
             if constexpr (EDGE == kEdgeOverlap) {
-              old = load_any8(from);
+              if (!TA || m0 + wm0 + m < M) old = load_any8(from);
             } else if constexpr (EDGE == kEdgeBounded) {
               int const left = m0 + wm0 + m < M ? N - (n0 + wn0 + n) : 0;  // columns of these four that exist
               old = left >= 4 ? load_any8(from) : left > 0 ? load_first4(from, left) : old;
@@ -1063,14 +1074,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
       }
     }
   };
-  // One wave per SIMD with a 128x128 wave tile keeps 256 accumulator registers: only the plain
-  // epilogue (bias, no activation, no split-K) is compiled for it, so that nothing outside the
-  // loop competes for registers.
-  if constexpr (WIDE2) {
-    finish([](float v) { return v; });
-    return;
-  }
-  if (partial != nullptr) {
+  if (!WIDE2 && partial != nullptr) {
     // raw accumulators, 16 bytes (4 consecutive columns) per store
     float *dst = partial + (int64_t)split * M * N;
 #pragma unroll
@@ -1081,12 +1085,19 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
 #pragma unroll
         for (int g = 0; g < 4; g++) {
           int const n = n0 + wn0 + j * 32 + 8 * g + 4 * (lane >> 5);
-          if (EDGE == kEdgeBounded && (m >= M || n >= N)) continue;  // (N % 4 == 0 where a reduction is split)
+          if (EDGE != kEdgeNone && m >= M) continue;
+          if (EDGE == kEdgeBounded && n >= N) continue;  // (N % 4 == 0 where a reduction is split)
           f32x4 v = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
           *reinterpret_cast<f32x4 *>(dst + m * N + n) = v;
         }
       }
     }
+    return;
+  }
+  // One wave per SIMD with a 128x128 wave tile keeps 256 accumulator registers: neither an activation
+  // nor a split reduction is compiled for it, so that nothing outside the loop competes for registers.
+  if constexpr (WIDE2) {
+    finish([](float v) { return v; });
     return;
   }
   if (act == FFK_ACT_NONE) {
@@ -1163,9 +1174,10 @@ static hipError_t launch_pipe(hipStream_t st, bf16 const *A, bf16 const *B,
   int const blocks = EDGE ? ((M + BM - 1) / BM) * ((N + BN - 1) / BN) : (M / BM) * (N / BN);
   if (splits > 1) {
     float *partial = static_cast<float *>(ep.splitk_ws);
-    kern<<<blocks * splits, NT, kLds, st>>>(A, B, C, M, N, K, lda, ldb, ldc, nullptr,
-                                                FFK_ACT_NONE, 0, partial, K / BK / splits, tail,
-                                                GemmGroupArgs{});
+    int const k_tiles = (K + BK - 1) / BK, per_split = (k_tiles + splits - 1) / splits;
+    splits = (k_tiles + per_split - 1) / per_split;  // none is empty
+    kern<<<blocks * splits, NT, kLds, st>>>(A, B, C, M, N, K, lda, ldb, ldc, nullptr, FFK_ACT_NONE, 0, partial, per_split,
+                                            tail, GemmGroupArgs{});
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     int64_t const quads = (int64_t)M * N / 4;
@@ -1222,20 +1234,6 @@ static hipError_t launch_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
 // register-staged kernel); 0 = the heuristic.  For tuning runs and tests.
 inline int gemm_variant_override() { return option(FFK_OPTION_GEMM_VARIANT); }
 
-// Number of K splits for an M x N output of 128x128 tiles: enough to give
-// every CU a workgroup, each split at least 8 k-tiles of 64 long, and no more
-// than the caller's scratch (splits * M * N floats) allows.
-inline int splitk_splits(int64_t M, int64_t N, int64_t K, size_t ws_bytes) {
-  int64_t const tiles = (M / 128) * (N / 128);
-  if (tiles <= 0 || tiles >= kNumCU / 2 || K % 64 != 0) return 1;
-  int s = 1;
-  while (s * 2 * tiles <= kNumCU && s < 8 && (K / 64) % (s * 2) == 0 && K / (s * 2) >= 512 &&
-         (size_t)(s * 2) * (size_t)(M * N) * sizeof(float) <= ws_bytes) {
-    s *= 2;
-  }
-  return s;
-}
-
 // What every pipelined kernel asks of the operands, whatever its tile.
 inline bool pipe_operands_ok(bf16 const *C, int K, int64_t lda, int64_t ldb, int64_t ldc, GemmEpilogue const &ep) {
   bool const c_vec = (ldc % 8 == 0) && aligned16(C);
@@ -1268,41 +1266,98 @@ inline int pipe_tile_for(bf16 const *C, int M, int N, int K, int64_t lda, int64_
 // offsets reach.
 inline bool edge_operands_ok(int64_t lda, int64_t ldb) { return 2 * 256 * std::max(lda, ldb) < (int64_t(1) << 31); }
 
-// The tile for a problem none of the whole-tile rules takes: the one whose rounds over the chip take
-// the least time.  A round's time is its k-tiles (64 deep) times what one costs with that tile, in us,
-// measured over M 100-2500, N 256-2304, K 100-3072 in three transposes (the choice is within 10% of the
-// best tile on nearly all of them):
-//   64 x 64, two groups of waves that split the reduction, two workgroups a CU: 0.17 while there are
-//     at most as many tiles as CUs, 0.39 for two a CU; with four LDS stages a group and one workgroup
-//     a CU (deep) 0.21, for which a long reduction over one tile a CU is worth having
-//   128 x 64: 0.385, or 0.62 for two a CU        128 x 128: 0.46        256 x 256: 1.3
-// and about 1 us of fill and drain per round.
+// The time of a bf16 product on each of the tiles, in us, from which its tile is chosen.  Measured on
+// products of M and N 128-4096, K 256-4096 (within 10% there, for whole tiles and overlapping ones,
+// the transposes within a further 10% of each other):
+//  - a round over the chip costs its 64-deep k-tiles times what one takes with so many CUs busy
+//    (memory and LDS are shared, the clock too), and a constant of filling, draining and storing
+//  - 64 x 64, two groups of waves that split the reduction, two workgroups a CU
+//    64 x 64 deep: four LDS stages a group, one workgroup a CU: holds its rate where the operands
+//    come from behind L2, as they do in reductions longer than 2048
+//    128 x 64: eight waves, two workgroups a CU; 128 x 128; 256 x 256; wide: the latter with one wave
+//    per SIMD
 enum EdgeTile { kTile64 = 64, kTile64Deep = 65, kTile128x64 = 70, kTile128 = 128, kTile256 = 256, kTile256Wide = 264 };
-inline EdgeTile edge_tile_for(int M, int N, int K, bool wide_ok) {
-  auto tiles = [&](int bm, int bn) { return (double)ceil_div(M, bm) * (double)ceil_div(N, bn); };
-  double const kt = (double)ceil_div(K, 64);
-  auto rounds = [&](double n, double per_round, double us) { return ceil(n / per_round) * (kt * us + 1.0); };
-  EdgeTile best = kTile64;
-  double const t64 = tiles(64, 64), t12 = tiles(128, 64);
-  double time = t64 <= kNumCU ? kt * 0.17 + 1.0 : rounds(t64, 2 * kNumCU, 0.39);
-  auto consider = [&](EdgeTile t, double us) {
-    if (us < time) best = t, time = us;
+inline double gemm_tile_us(EdgeTile t, double m, double n, double k, double splits = 1) {
+  int const bm = t == kTile64 || t == kTile64Deep ? 64 : t == kTile128x64 || t == kTile128 ? 128 : 256;
+  int const bn = t == kTile128x64 ? 64 : bm;
+  double const tiles = ceil(m / bm) * ceil(n / bn) * splits, kt = ceil(ceil(k / 64) / splits);
+  auto round_us = [&](double count) {  // of `count` workgroups at a time
+    double const f = count / kNumCU;
+    switch (t) {
+      case kTile64: return f <= 1 ? kt * 0.166 + 1.8 : kt * 0.36 + 2.4;
+      case kTile64Deep: return kt * 0.175 + 2.1;
+      case kTile128x64: return f <= 1 ? kt * (0.29 + 0.08 * f) + 1.6 : kt * 0.54 + 2.0;
+      case kTile128: return kt * std::max(0.31, 0.10 + 0.37 * f) + 2.0;
+      case kTile256: return kt * std::max(1.09, 0.35 + 1.25 * f) + 5.5 + 2.0 * f;
+      default: return kt * std::max(0.96, 0.25 + 1.19 * f) + 5.5 + 3.0 * f;
+    }
   };
-  if (kt > 24) consider(kTile64Deep, t64 <= kNumCU ? kt * 0.16 : rounds(t64, kNumCU, 0.21));
-  consider(kTile128x64, t12 <= kNumCU ? kt * 0.385 + 1.0 : rounds(t12, 2 * kNumCU, 0.62));
-  consider(kTile128, rounds(tiles(128, 128), kNumCU, 0.46));
-  // one wave per SIMD where that kernel has what it takes, two otherwise
-  consider(wide_ok && K >= 1024 ? kTile256Wide : kTile256, rounds(tiles(256, 256), kNumCU, 1.3));
+  double const a_round = t == kTile64 || t == kTile128x64 ? 2 * kNumCU : kNumCU;
+  double const full = floor(tiles / a_round), last = tiles - full * a_round;
+  double us = full * round_us(a_round) + (last > 0 ? round_us(last) : 0.0);
+  // the rounds of 128 x 128 tiles overlap less than the first one's fill suggests
+  if (t == kTile128) us += 2.0 * (ceil(tiles / a_round) - 1);
+  if (t == kTile64 && kt > 32) us += 0.2 * (kt - 32) * ceil(tiles / a_round);
+  if (splits > 1) us += 4.0 + splits * m * n * 8 / 4.0e6;  // the partial sums: written and read at 4 TB/s
+  return us;
+}
+inline EdgeTile gemm_tile_for(int M, int N, int K, bool wide_ok, double *time = nullptr) {
+  EdgeTile best = kTile64;
+  double least = gemm_tile_us(kTile64, M, N, K);
+  for (EdgeTile const t : {kTile64Deep, kTile128x64, kTile128, kTile256, kTile256Wide}) {
+    if ((t == kTile256Wide) != (wide_ok && K >= 1024) && (t == kTile256Wide || t == kTile256)) continue;
+    double const us = gemm_tile_us(t, M, N, K);
+    if (us < least) best = t, least = us;
+  }
+  if (time != nullptr) *time = least;
   return best;
 }
 
-// Whether the plain kernel for this ragged or small problem is one of the two 64x64 ones, whose waves
-// split the reduction (an epilogue's tail then has to run on that tile too for the same bits), and not
-// one of the larger ones, which all add up in the same order.
-inline bool edge_splits_reduction(int M, int N, int K, GemmEpilogue const &ep) {
-  EdgeTile const t = edge_tile_for(M, N, K, ep.activation == FFK_ACT_NONE);
+// Whether the plain kernel for this problem is one of the two 64x64 ones, whose waves split the
+// reduction (an epilogue's tail then has to run on that tile too for the same bits), and not one of
+// the larger ones, which all add up in the same order.
+inline bool gemm_splits_reduction(int M, int N, int K, GemmEpilogue const &ep) {
+  EdgeTile const t = gemm_tile_for(M, N, K, ep.activation == FFK_ACT_NONE);
   int const bm = t == kTile256 || t == kTile256Wide ? 256 : 128, bn = t == kTile128x64 ? 64 : bm;
   return t == kTile64 || t == kTile64Deep || M < bm || N < bn;
+}
+
+// Splitting the reduction over workgroups, where there is scratch for it: 128 x 128 or 256 x 256 tiles
+// in as many splits as make the product fastest.  1: none does.  (Reductions worth splitting stream
+// their operands from memory, which 256 x 256 tiles read half as often: [2048, 50257] . [50257, 1024]
+// takes 446 us unsplit, 290 us on 128 x 128 tiles and 2 splits, 210 us on 256 x 256 tiles and 8.)
+inline int gemm_splits_for(int M, int N, int K, size_t scratch, double unsplit_us, EdgeTile &tile) {
+  int best = 1;
+  double least = unsplit_us;
+  for (EdgeTile const t : {kTile128, kTile256}) {
+    if (M < t || N < t) continue;
+    for (int s = 2; s <= 16 && ceil_div(K, 64) >= 8 * s && (size_t)s * M * N * sizeof(float) <= scratch; s *= 2) {
+      double const us = gemm_tile_us(t, M, N, K, s) * (t == kTile128 ? 1.2 : 1.0);
+      if (us < least) best = s, least = us, tile = t;
+    }
+  }
+  return best;
+}
+
+// A product whose last round of 256 x 256 tiles is nearly empty: the rows (along_m) or columns that make
+// whole rounds go first, the others as a product of their own on the tile that suits them.  How many
+// rows or columns the first one takes, 0 if one launch is as soon done.  ([2048, 1024] . [50257, 1024]^T
+// is 1576 tiles, six rounds and 40 more: 238 us, 214 in two launches.)
+inline int gemm_whole_rounds(int M, int N, int K, bool wide_ok, double one_launch_us, bool &along_m) {
+  EdgeTile const t = wide_ok && K >= 1024 ? kTile256Wide : kTile256;
+  int64_t const nbm = ceil_div(M, 256), nbn = ceil_div(N, 256), full = nbm * nbn / kNumCU * kNumCU;
+  if (full == 0 || full == nbm * nbn) return 0;
+  int first = 0;
+  double least = one_launch_us - 2.0;
+  for (bool const m : {false, true}) {
+    int64_t const lines = full / (m ? nbn : nbm) * 256;
+    if (lines == 0 || lines >= (m ? M : N)) continue;
+    double rest = 0;
+    gemm_tile_for(m ? M - (int)lines : M, m ? N : N - (int)lines, K, wide_ok, &rest);
+    double const us = gemm_tile_us(t, m ? (double)lines : M, m ? N : (double)lines, K) + rest + 3.0;
+    if (us < least) first = (int)lines, along_m = m, least = us;
+  }
+  return first;
 }
 
 // A GEMM with element-wise operators on its tile store.  gemm_tail_supported has been asked.
@@ -1312,7 +1367,7 @@ static hipError_t launch_tail(hipStream_t st, bf16 const *A, bf16 const *B, bf16
   int const tile = pipe_tile_for(C, M, N, K, lda, ldb, ldc, ep, gemm_variant_override());
   if (tile == 256) return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB, TAIL>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
   if (tile == 128) return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, TAIL>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
-  if (edge_splits_reduction(M, N, K, ep)) {
+  if (gemm_splits_reduction(M, N, K, ep)) {
     return launch_pipe<64, 64, 32, 32, 64, 2, 3, TA, TB, TAIL, kEdgeBounded, 2>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
   }
   // column sums are taken over blocks of 32 rows from multiples of 32 on, where overlapping tiles do not begin
@@ -1368,62 +1423,67 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
                             bf16 *C, int M, int N, int K, int64_t lda,
                             int64_t ldb, int64_t ldc, GemmEpilogue const &ep, bool vec) {
   int const variant = vec ? gemm_variant_override() : 1;  // 1: the register-staged kernel, whose loads take any address
-  int const pipe_tile = pipe_tile_for(C, M, N, K, lda, ldb, ldc, ep, variant);
-  {
-    bool const fits128 = M % 128 == 0 && N % 128 == 0;
-    bool const use256 = pipe_tile == 256, use128 = pipe_tile == 128;
-    // An output that 256x256 tiles cover in a ragged last round but 256x192 tiles cover in whole
-    // rounds of the chip (the attention block's fused Q/K/V projection: [4096, 3072] is 192 tiles of
-    // the first kind on 256 CUs, 256 of the second): one wave per SIMD on 128x96 wave tiles.  Only
-    // with both operands K-contiguous: a [K][192] panel does not divide into whole direct loads.
-    if constexpr (!TA && TB) {
-      bool const fits192 = M % 256 == 0 && N % 192 == 0;
-      int64_t const t256 = M % 256 == 0 && N % 256 == 0 ? (int64_t)(M / 256) * (N / 256) : 0;
-      int64_t const t192 = fits192 ? (int64_t)(M / 256) * (N / 192) : 0;
-      bool const whole_rounds = t192 > 0 && t192 % kNumCU == 0 && t256 % kNumCU != 0;
-      if (pipe_operands_ok(C, K, lda, ldb, ldc, ep) && variant != 1 && ep.activation == FFK_ACT_NONE && K >= 1024 &&
-          (variant == 192 ? fits192 : (variant == 0 && whole_rounds))) {
-        return launch_pipe<256, 192, 128, 96, 64, 2, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
-      }
-    }
-    // Reductions from 1024 on without an activation: one wave per SIMD on 128x128 wave tiles, two
-    // 64-deep stages, every instruction of the loop placed by hand.  (Below that the eight-wave
-    // kernel's shorter prologue weighs more than the faster loop.)
-    if (use256 && ep.activation == FFK_ACT_NONE && (variant == 264 || (variant == 0 && K >= 1024))) {
-      return launch_pipe<256, 256, 128, 128, 64, 2, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
-    }
-    if (use256) {
-      return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
-    }
-    if (use128) {
-      return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
-    }
-    // Few output tiles and a long reduction: split K so every CU has a tile.
-    bool const pipe_ok = pipe_tile_for(C, M, N, K, lda, ldb, ldc, ep, 128) == 128;  // but for the tile count
-    int const splits = fits128 && pipe_ok ? splitk_splits(M, N, K, ep.splitk_ws_bytes) : 1;
-    if (variant == 0 && splits > 1 && ep.splitk_ws != nullptr && aligned16(ep.splitk_ws)) {
-      return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep, splits);
-    }
-    // No scratch to split the reduction with: from 32 tiles and a reduction of 2048 on, the
-    // pipelined tile on the CUs it reaches is still ahead of the register-staged 64x64 kernel on
-    // four times as many ([1024,1024] over 4096 rows, 64 tiles: 30.5 against 34.5 us).
-    if (variant == 0 && pipe_ok && fits128 && (int64_t)(M / 128) * (N / 128) >= kNumCU / 8 && K >= 2048) {
-      return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+  // An output that 256x256 tiles cover in a ragged last round but 256x192 tiles cover in whole
+  // rounds of the chip (the attention block's fused Q/K/V projection: [4096, 3072] is 192 tiles of
+  // the first kind on 256 CUs, 256 of the second): one wave per SIMD on 128x96 wave tiles.  Only
+  // with both operands K-contiguous: a [K][192] panel does not divide into whole direct loads.
+  if constexpr (!TA && TB) {
+    bool const fits192 = M % 256 == 0 && N % 192 == 0;
+    int64_t const t256 = M % 256 == 0 && N % 256 == 0 ? (int64_t)(M / 256) * (N / 256) : 0;
+    int64_t const t192 = fits192 ? (int64_t)(M / 256) * (N / 192) : 0;
+    bool const whole_rounds = t192 > 0 && t192 % kNumCU == 0 && t256 % kNumCU != 0;
+    if (pipe_operands_ok(C, K, lda, ldb, ldc, ep) && variant != 1 && ep.activation == FFK_ACT_NONE && K >= 1024 &&
+        (variant == 192 ? fits192 : (variant == 0 && whole_rounds))) {
+      return launch_pipe<256, 192, 128, 96, 64, 2, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
     }
   }
   if (variant != 1 && edge_operands_ok(lda, ldb)) {
-    EdgeTile tile = edge_tile_for(M, N, K, ep.activation == FFK_ACT_NONE && ldc % 8 == 0);
+    bool const wide_ok = ep.activation == FFK_ACT_NONE && ldc % 8 == 0;
+    double us;
+    EdgeTile tile = gemm_tile_for(M, N, K, wide_ok, &us);
     bool const forced = variant == 64 || variant == 65 || variant == 70 || variant == 128 || variant == 256 || variant == 264;
-    if (forced) tile = (EdgeTile)variant;
+    bool const whole128 = M % 128 == 0 && N % 128 == 0 && pipe_operands_ok(C, K, lda, ldb, ldc, ep);
+    if (forced) {
+      tile = variant == kTile256Wide && ep.activation != FFK_ACT_NONE ? kTile256 : (EdgeTile)variant;
+    } else {
+      if (ep.splitk_ws != nullptr && aligned16(ep.splitk_ws) && aligned16(C) && N % 8 == 0 && ldc % 8 == 0) {
+        EdgeTile split_tile = tile;
+        int const splits = gemm_splits_for(M, N, K, ep.splitk_ws_bytes, us, split_tile);
+        if (splits > 1) {
+          if (split_tile == kTile256) {
+            return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep, splits);
+          }
+          if (whole128) return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep, splits);
+          return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep, splits);
+        }
+      }
+      // (a long reduction over whole tiles has been on this tile, by name, since before there were 64-wide ones)
+      if (whole128 && (int64_t)(M / 128) * (N / 128) >= kNumCU / 4 && K >= 4096 && (tile == kTile64 || tile == kTile64Deep)) tile = kTile128;
+      bool along_m = false;
+      int const first = M >= 256 && N >= 256 ? gemm_whole_rounds(M, N, K, wide_ok, us, along_m) : 0;
+      if (first > 0) {
+        GemmEpilogue rest = ep;
+        int const m = along_m ? first : 0, n = along_m ? 0 : first;
+        if (ep.bias != nullptr) rest.bias = static_cast<bf16 const *>(ep.bias) + n;
+        hipError_t const e = pick_bf16<TA, TB>(st, A + (TA ? (int64_t)m : m * lda), B + (TB ? n * ldb : (int64_t)n), C + m * ldc + n,
+                                               M - m, N - n, K, lda, ldb, ldc, rest, vec);
+        if (e != hipSuccess) return e;
+        return pick_bf16<TA, TB>(st, A, B, C, along_m ? first : M, along_m ? N : first, K, lda, ldb, ldc, ep, vec);
+      }
+    }
     // tiles that begin early: the output has to hold one, and old values added by one workgroup only
     int const bm = tile == kTile256 || tile == kTile256Wide ? 256 : 128, bn = tile == kTile128x64 ? 64 : bm;
     if (tile != kTile64 && tile != kTile64Deep && (M < bm || N < bn || (ep.accumulate && N % 8 != 0))) tile = kTile64;
+    bool const whole = M % bm == 0 && N % bn == 0 && pipe_operands_ok(C, K, lda, ldb, ldc, ep);
     switch (tile) {
       case kTile256Wide:
+        if (whole) return launch_pipe<256, 256, 128, 128, 64, 2, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
         return launch_pipe<256, 256, 128, 128, 64, 2, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
       case kTile256:
+        if (whole) return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
         return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
       case kTile128:
+        if (whole) return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
         return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
       case kTile128x64:
         return launch_pipe<128, 64, 32, 32, 64, 3, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);

@@ -17,44 +17,6 @@
 
 namespace ffk {
 
-// in = (output, output_grad); out = g
-template <int ACT, int MODE>
-struct ActGrad {
-  __device__ __forceinline__ void operator()(float const (&in)[2],
-                                             float (&out)[1]) const {
-    float y = in[0], dy = in[1];
-    float g;
-    if (ACT == FFK_ACT_RELU) {
-      if (MODE == 1) {
-        g = dy > 0.0f ? 1.0f : 0.0f;  // linear_kernels_cpu.cc:46-52,69-71
-      } else {
-        g = y > 0.0f ? dy : 0.0f;     // cuda_helper.cu:60-64
-      }
-    } else if (ACT == FFK_ACT_SIGMOID) {
-      g = dy * y * (1.0f - y);        // cuda_helper.cu:87-91
-    } else {
-      g = dy * (1.0f - y * y);        // tanh
-    }
-    out[0] = g;
-  }
-};
-
-template <typename T>
-static hipError_t act_grad(hipStream_t st, int act, int mode, void const *y,
-                           void const *dy, void *g, int64_t n) {
-  EwArgs<T, 2, 1> a;
-  a.in[0] = static_cast<T const *>(y);
-  a.in[1] = static_cast<T const *>(dy);
-  a.in_elems[0] = n;
-  a.in_elems[1] = n;
-  a.out[0] = static_cast<T *>(g);
-  a.n = n;
-  if (act == FFK_ACT_RELU && mode == 1) return ew_launch<T, 2, 1>(st, a, ActGrad<FFK_ACT_RELU, 1>{});
-  if (act == FFK_ACT_RELU) return ew_launch<T, 2, 1>(st, a, ActGrad<FFK_ACT_RELU, 0>{});
-  if (act == FFK_ACT_SIGMOID) return ew_launch<T, 2, 1>(st, a, ActGrad<FFK_ACT_SIGMOID, 0>{});
-  return ew_launch<T, 2, 1>(st, a, ActGrad<FFK_ACT_TANH, 0>{});
-}
-
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // in = (weight, weight_grad); out = weight_grad + lambda * weight
@@ -192,13 +154,21 @@ static void small_linear_bwd_launch(hipStream_t st, int activation, SmallLinearB
 
 using namespace ffk;
 
+// bf16 gradient rows of no whole 16 bytes (a vocabulary's 50257): the products then could only be
+// read an element's address at a time, which costs them half their rate ([2048, 50257] . [50257, 1024]
+// 636 us so).  The pass that sums the bias gradient also writes g with rows that are.
+static bool linear_pads_grad(int dtype, int64_t out_dim) { return dtype == FFK_BF16 && out_dim % 8 != 0; }
+static int64_t linear_grad_ld(int dtype, int64_t out_dim) {
+  return linear_pads_grad(dtype, out_dim) ? (out_dim + 63) / 64 * 64 : out_dim;
+}
+
 extern "C" size_t ffk_linear_backward_workspace_bytes(int dtype, int activation,
                                                       int use_bias,
                                                       int64_t batch,
                                                       int64_t out_dim) {
   size_t bytes = 0;
-  if (activation != FFK_ACT_NONE) {
-    bytes += align256((size_t)batch * (size_t)out_dim * dtype_size(dtype));
+  if (activation != FFK_ACT_NONE || linear_pads_grad(dtype, out_dim)) {
+    bytes += align256((size_t)batch * (size_t)linear_grad_ld(dtype, out_dim) * dtype_size(dtype));
   }
   if (use_bias) {
     bytes += align256((size_t)colsum_partials_elems(batch, out_dim) * sizeof(float));
@@ -290,46 +260,61 @@ static int linear_backward_impl(
     FFK_CHECK_LAUNCH();
     return FFK_OK;
   }
-  size_t need = ffk_linear_backward_workspace_bytes(dtype, activation,
-                                                    bias_grad != nullptr, batch, out_dim);
-  if (need > 0 && (workspace == nullptr || workspace_bytes < need)) {
-    return fail(FFK_ERR_WORKSPACE,
-                "linear_backward: workspace of %zu bytes needed, %zu given", need,
-                workspace_bytes);
+  bool const act = activation != FFK_ACT_NONE;
+  bool const sums = bias_grad != nullptr;
+  // rows padded to whole 16 bytes, if the products can read the other operands so and there is a pass
+  // over g anyway or the products are large enough to pay for one
+  bool pad = linear_pads_grad(dtype, out_dim) && in_dim % 8 == 0 && input_tail == nullptr && aligned16(weight) &&
+             aligned16(input) && (input_grad != nullptr || weight_grad != nullptr) &&
+             (sums || act || batch * in_dim * out_dim >= (int64_t(1) << 26));
+  size_t const partial_bytes = sums ? align256((size_t)colsum_partials_elems(batch, out_dim) * sizeof(float)) : 0;
+  auto grad_bytes = [&](int64_t ld) { return align256((size_t)batch * (size_t)ld * dtype_size(dtype)); };
+  size_t const least = partial_bytes + (act ? grad_bytes(out_dim) : 0);
+  if (least > 0 && (workspace == nullptr || workspace_bytes < least)) {
+    return fail(FFK_ERR_WORKSPACE, "linear_backward: workspace of %zu bytes needed, %zu given", least, workspace_bytes);
+  }
+  // (a caller that knows the sizes without padding keeps working)
+  if (pad && (workspace == nullptr || !aligned16(workspace) ||
+              workspace_bytes < partial_bytes + grad_bytes(linear_grad_ld(dtype, out_dim)))) {
+    pad = false;
   }
   uint8_t *ws = static_cast<uint8_t *>(workspace);
   void const *g = output_grad;
-  if (activation != FFK_ACT_NONE) {
-    int64_t n = batch * out_dim;
-    hipError_t e = dtype == FFK_FLOAT
-                       ? act_grad<float>(st, activation, relu_grad_mode, output, output_grad, ws, n)
-                       : act_grad<bf16>(st, activation, relu_grad_mode, output, output_grad, ws, n);
-    FFK_HIP(e);
+  int64_t const ldg = pad ? linear_grad_ld(dtype, out_dim) : out_dim;
+  int rc;
+  if (act || pad) {
+    rc = linear_grad(st, dtype, activation, relu_grad_mode, output, output_grad, ws, ldg, batch, out_dim, bias_grad,
+                     (accumulate & FFK_ACC_BIAS) != 0, reinterpret_cast<float *>(ws + grad_bytes(ldg)));
+    if (rc != FFK_OK) return rc;
     g = ws;
-    ws += align256((size_t)n * dtype_size(dtype));
   }
   GemmEpilogue ep;
-  int rc;
+  ep.a_padded = pad;
   if (input_grad != nullptr) {
     GemmEpilogue dx = input_tail != nullptr ? *input_tail : ep;
     dx.accumulate = (accumulate & FFK_ACC_INPUT) != 0;
+    // what the weight gradient will overwrite serves as scratch until then: a reduction over a
+    // vocabulary is longer than its few output tiles keep the chip busy with
+    if (input_tail == nullptr && weight_grad != nullptr && (accumulate & FFK_ACC_WEIGHT) == 0) {
+      dx.splitk_ws = weight_grad;
+      dx.splitk_ws_bytes = (size_t)in_dim * (size_t)out_dim * dtype_size(dtype);
+    }
     // input_grad[batch,in] = g[batch,out] . weight[out,in]
     if (input_tail != nullptr &&
         !gemm_tail_supported(dtype, false, false, batch, in_dim, out_dim, g, out_dim, weight, in_dim,
                              input_grad, in_dim, dx)) {
       return FFK_ERR_UNSUPPORTED;  // before anything is launched: the caller runs the separate operators
     }
-    rc = gemm_dispatch(st, dtype, false, false, batch, in_dim, out_dim, g, out_dim,
-                       weight, in_dim, input_grad, in_dim, dx);
+    rc = gemm_dispatch(st, dtype, false, false, batch, in_dim, out_dim, g, ldg, weight, in_dim, input_grad, in_dim, dx);
     if (rc != FFK_OK) return rc;
   }
   if (weight_grad != nullptr) {
     ep.accumulate = (accumulate & FFK_ACC_WEIGHT) != 0;
     // weight_grad[out,in] = g[batch,out]^T . input[batch,in]
-    rc = weight_grad_dispatch(st, dtype, out_dim, in_dim, batch, g, out_dim, input, in_dim, weight_grad, in_dim, ep);
+    rc = weight_grad_dispatch(st, dtype, out_dim, in_dim, batch, g, ldg, input, in_dim, weight_grad, in_dim, ep);
     if (rc != FFK_OK) return rc;
   }
-  if (bias_grad != nullptr) {
+  if (sums && !act && !pad) {
     rc = colsum_dispatch(st, dtype, g, out_dim, batch, out_dim, bias_grad,
                          (accumulate & FFK_ACC_BIAS) != 0, reinterpret_cast<float *>(ws));
     if (rc != FFK_OK) return rc;

@@ -11,23 +11,10 @@
 
 namespace ffk {
 
-// ACT is a template argument of the kernel: a run-time switch here puts a branch and a wait
-// between every two loads of a thread, and the kernel's time is its round trips to memory.
-template <int ACT>
-__device__ __forceinline__ float small_act_grad(int mode, float y, float dy) {
-  if constexpr (ACT == FFK_ACT_RELU) {
-    return mode == 1 ? (dy > 0.0f ? 1.0f : 0.0f) : (y > 0.0f ? dy : 0.0f);
-  } else if constexpr (ACT == FFK_ACT_SIGMOID) {
-    return dy * y * (1.0f - y);
-  } else if constexpr (ACT == FFK_ACT_TANH) {
-    return dy * (1.0f - y * y);
-  } else {
-    return dy;
-  }
-}
-
 // An operand's element (r, k): KC: p[r * ld + k]; otherwise p[k * ld + r].  ACT: the element is
-// act'(y) * p with y laid out like p (FFK_ACT_NONE: p alone).
+// act'(y) * p with y laid out like p (FFK_ACT_NONE: p alone).  ACT is a template argument of the
+// kernel: a run-time switch puts a branch and a wait between every two loads of a thread, and the
+// kernel's time is its round trips to memory.
 template <bool KC, int ACT>
 struct SmallOperand {
   float const *p, *y;
@@ -59,7 +46,7 @@ struct SmallOperand {
     if constexpr (kPair) raw.y = four(y, ld, r, k, last, whole);
   }
   __device__ __forceinline__ float value(Raw const &raw, int j) const {
-    return small_act_grad<ACT>(mode, kPair ? raw.y[j] : 0.0f, raw.v[j]);
+    return activation_grad<ACT>(mode, kPair ? raw.y[j] : 0.0f, raw.v[j]);
   }
 };
 
