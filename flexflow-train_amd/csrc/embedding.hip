@@ -12,6 +12,7 @@
 // out of bounds for them).
 #include "ffk_common.h"
 #include "radix_sort.h"
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 #include <cstring>
@@ -275,16 +276,20 @@ __global__ __launch_bounds__(kEmbThreads) void embedding_bwd_atomic_kernel(
 // that cross a chunk border (at most two per walker) go through atomics.
 constexpr int kEmbChunk = 16;  // sorted positions per walker
 
-template <typename GT>
-__device__ __forceinline__ void load_grad4(GT const *p, float (&v)[4]);
-template <>
-__device__ __forceinline__ void load_grad4<float>(float const *p, float (&v)[4]) {
-  f32x4 r = __builtin_nontemporal_load(reinterpret_cast<f32x4 const *>(p));
+// STREAM: the row is read once (one lookup per gradient row), so it need not stay in the caches.
+template <typename V, bool STREAM>
+__device__ __forceinline__ V load_grad_vec(void const *p) {
+  if constexpr (STREAM) return __builtin_nontemporal_load(reinterpret_cast<V const *>(p));
+  else return *reinterpret_cast<V const *>(p);
+}
+template <bool STREAM>
+__device__ __forceinline__ void load_grad4(float const *p, float (&v)[4]) {
+  f32x4 r = load_grad_vec<f32x4, STREAM>(p);
   v[0] = r[0]; v[1] = r[1]; v[2] = r[2]; v[3] = r[3];
 }
-template <>
-__device__ __forceinline__ void load_grad4<bf16>(bf16 const *p, float (&v)[4]) {
-  u32x2 r = __builtin_nontemporal_load(reinterpret_cast<u32x2 const *>(p));
+template <bool STREAM>
+__device__ __forceinline__ void load_grad4(bf16 const *p, float (&v)[4]) {
+  u32x2 r = load_grad_vec<u32x2, STREAM>(p);
   v[0] = __uint_as_float(r[0] << 16);
   v[1] = __uint_as_float(r[0] & 0xffff0000u);
   v[2] = __uint_as_float(r[1] << 16);
@@ -325,7 +330,7 @@ __global__ __launch_bounds__(256) void embedding_bwd_sorted_kernel(
       for (int k = 0; k < CPL; k++) {
         int64_t const c = cbase + ((int64_t)k * LPR + wl) * 4;
         if (c < dim) {
-          load_grad4<GT>(row + c, v[k]);
+          load_grad4<true>(row + c, v[k]);
         } else {
           v[k][0] = v[k][1] = v[k][2] = v[k][3] = 0.0f;
         }
@@ -381,206 +386,190 @@ __global__ __launch_bounds__(256) void embedding_bwd_sorted_kernel(
   }
 }
 
-// The non-deterministic sorted path: a workgroup of 1024 threads owns
-// (1024 / LPR) * kEmbChunk consecutive sorted positions.  Walkers add runs that
-// lie inside their chunk straight to memory; the partial sums of runs that
-// cross a walker border meet in LDS and are merged by the workgroup, so only
-// runs that cross a WORKGROUP border reach memory as atomics.  A row looked up
+// The non-deterministic sorted path: a wave walks `chunk` consecutive sorted positions, a
+// workgroup sixteen such chunks.  Walkers add runs that lie inside their chunk straight to memory;
+// the partial sums of runs that cross a walker border meet in LDS and are merged by the workgroup,
+// so only runs that cross a WORKGROUP border reach memory as atomics.  A row looked up
 // thousands of times (Zipf-distributed tokens) then costs one atomic per
 // element per workgroup instead of one per walker, which matters because
 // atomics to one address are retired one after the other.
+// A walker is a whole wave whatever the row length (VPL columns per lane; blockIdx.y takes the next
+// 256 columns of longer rows): ids, row addresses and the run logic are then scalar work beside the loads.  With two
+// walkers to a wave (dim 128) every position took about a hundred vector instructions, and
+// they, not memory, were the bound (524 288 lookups in bags of 32, 1 M rows of 128
+// floats: 78 -> 58 us; 65 536 lookups of 1024 bf16 columns, which had a wave to a walker before: 62-64 both ways).
 constexpr int kEmbBlockThreads = 1024;
+constexpr int kEmbWalkers = kEmbBlockThreads / 64;
+constexpr int kEmbMaxChunk = 64;  // one (row id, lookup) pair per lane
 
-// CPL column chunks of 4 per lane and pass (more bytes in flight per walker
-// step: the walk is latency-bound otherwise).  LDS: 2 * WPB border partials of
-// LPR * 4 * CPL floats, passed as dynamic shared memory.
-template <typename GT, int LPR, int CPL>
-__global__ __launch_bounds__(kEmbBlockThreads) void embedding_bwd_sorted_block_kernel(
-    uint32_t const *__restrict__ keys, uint32_t const *__restrict__ vals,
-    GT const *__restrict__ dY, float *dW, int64_t n, int bag, int64_t dim,
-    uint32_t invalid_key, float scale) {
-  constexpr int WPB = kEmbBlockThreads / LPR;  // walkers per workgroup
-  constexpr int PW = LPR * 4 * CPL;            // columns per pass
-  extern __shared__ __attribute__((aligned(16))) float emb_part[];  // [2 * WPB][PW]
-  __shared__ uint32_t part_id[2 * WPB];
-  __shared__ int part_valid[2 * WPB];
-  int const w = threadIdx.x / LPR, wl = threadIdx.x % LPR;
-  int64_t const block0 = (int64_t)blockIdx.x * WPB * kEmbChunk;
-  int64_t const block1 = min(block0 + (int64_t)WPB * kEmbChunk, n);
-  int64_t const p0 = block0 + (int64_t)w * kEmbChunk;
-  int64_t const p1 = min(p0 + (int64_t)kEmbChunk, n);
-  // The walker's 16 (row id, lookup) pairs are fetched once, one pair per lane, and handed round
-  // with lane shuffles.  What the walk would otherwise wait for at every position -- the
-  // gradient row of the lookup and, where a run ends, the weight-gradient row it is added to --
-  // is then asked for two positions ahead.  (Walkers of cold rows, where every position ends a
-  // run, set the pace of their workgroup: each of their positions used to cost two dependent
-  // memory round trips.)
-  int const cnt = (int)max((int64_t)0, min((int64_t)kEmbChunk, n - p0));  // positions that exist
-  bool const active = cnt > 0;
-  static_assert(LPR >= kEmbChunk, "one pair per lane");
-  uint32_t my_key = invalid_key, my_val = 0;
-  if (wl < cnt) {
-    my_key = keys[p0 + wl];
-    my_val = vals[p0 + wl];
-    // what the walk needs of a lookup is the gradient row it reads: its bag.  Divided once here,
-    // by the lane that holds the pair, not at every position by every lane of the walker.
-    if (bag != 1) my_val /= (uint32_t)bag;
+template <int VPL, bool STREAM>
+__device__ __forceinline__ void load_grad_piece(float const *p, float (&v)[VPL]) {
+  using vec = typename std::conditional<VPL == 4, f32x4, typename std::conditional<VPL == 2, f32x2, float>::type>::type;
+  vec const r = load_grad_vec<vec, STREAM>(p);
+  if constexpr (VPL == 1) {
+    v[0] = r;
+  } else {
+#pragma unroll
+    for (int e = 0; e < VPL; e++) v[e] = r[e];
   }
-  int const wbase = ((threadIdx.x & 63) / LPR) * LPR;  // the walker's first lane in its wave
-  uint32_t const key_before = active && p0 > 0 ? keys[p0 - 1] : invalid_key;
-  uint32_t const key_after = active && p1 < n ? keys[p1] : invalid_key;
-  // every lane of the wave takes part in a shuffle, whatever its walker has to do
-  auto key_at = [&](int j) { return (uint32_t)__shfl((int)my_key, wbase + (j < kEmbChunk ? j : kEmbChunk - 1), 64); };
-  auto lookup_at = [&](int j) { return (uint32_t)__shfl((int)my_val, wbase + (j < kEmbChunk ? j : kEmbChunk - 1), 64); };
-  bool const head_shared = active && p0 > 0 && key_before == key_at(0);
-  auto add_row = [&](uint32_t id, int64_t cbase, float const (&acc)[CPL][4], bool atomic) {
-#pragma unroll
-    for (int k = 0; k < CPL; k++) {
-      int64_t const c = cbase + ((int64_t)k * LPR + wl) * 4;
-      if (c < dim) {
-        float *dst = dW + (int64_t)id * dim + c;
-        if (atomic) {
-#pragma unroll
-          for (int e = 0; e < 4; e++) atomicAdd(dst + e, acc[k][e] * scale);
-        } else {
-          f32x4 old = *reinterpret_cast<f32x4 const *>(dst);
-          f32x4 upd = {old[0] + acc[k][0] * scale, old[1] + acc[k][1] * scale,
-                       old[2] + acc[k][2] * scale, old[3] + acc[k][3] * scale};
-          *reinterpret_cast<f32x4 *>(dst) = upd;
-        }
-      }
-    }
+}
+template <int VPL, bool STREAM>
+__device__ __forceinline__ void load_grad_piece(bf16 const *p, float (&v)[VPL]) {
+  using word = typename std::conditional<VPL == 4, u32x2, typename std::conditional<VPL == 2, uint32_t, uint16_t>::type>::type;
+  word const r = load_grad_vec<word, STREAM>(p);
+  if constexpr (VPL == 1) {
+    v[0] = __uint_as_float((uint32_t)r << 16);
+  } else if constexpr (VPL == 2) {
+    v[0] = __uint_as_float(r << 16);
+    v[1] = __uint_as_float(r & 0xffff0000u);
+  } else {
+    v[0] = __uint_as_float(r[0] << 16);
+    v[1] = __uint_as_float(r[0] & 0xffff0000u);
+    v[2] = __uint_as_float(r[1] << 16);
+    v[3] = __uint_as_float(r[1] & 0xffff0000u);
+  }
+}
+
+// DEPTH positions in flight, as many as fit the registers that let two workgroups share a CU.
+// BAGGED: bags of several entries, whose gradient row the walkers read once per entry: cached loads.
+template <typename GT, int VPL, bool BAGGED>
+__global__ __launch_bounds__(kEmbBlockThreads, 8) void embedding_bwd_sorted_block_kernel(
+    uint32_t const *__restrict__ keys, uint32_t const *__restrict__ vals,
+    GT const *__restrict__ dY, float *dW, int64_t n, int chunk, int bag, int dim,
+    uint32_t invalid_key, float scale) {
+  constexpr int PW = 64 * VPL;  // columns of a workgroup
+  constexpr int DEPTH = VPL == 4 ? 4 : 8;
+  __shared__ float emb_part[2 * kEmbWalkers * PW];  // border partials
+  __shared__ uint32_t part_id[2 * kEmbWalkers];
+  __shared__ int part_valid[2 * kEmbWalkers];
+  int const lane = threadIdx.x & 63;
+  int const w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int64_t const block0 = (int64_t)blockIdx.x * kEmbWalkers * chunk;
+  int64_t const block1 = min(block0 + (int64_t)kEmbWalkers * chunk, n);
+  int64_t const p0 = block0 + (int64_t)w * chunk;
+  int64_t const p1 = min(p0 + (int64_t)chunk, n);
+  // The walker's (row id, lookup) pairs are fetched once, one pair per lane, and read back as
+  // scalars.  What the walk would otherwise wait for at every position -- the gradient row of the
+  // lookup and, where a run ends, the weight-gradient row it is added to -- is then asked for
+  // DEPTH positions ahead.
+  int const cnt = (int)max((int64_t)0, min((int64_t)chunk, n - p0));  // positions that exist
+  uint32_t my_key = invalid_key, my_val = 0;
+  if (lane < cnt) {
+    my_key = keys[p0 + lane];
+    my_val = vals[p0 + lane];
+    // what the walk needs of a lookup is the gradient row it reads: its bag
+    if (BAGGED) my_val /= (uint32_t)bag;
+  }
+  uint32_t const key_before = cnt > 0 && p0 > 0 ? keys[p0 - 1] : invalid_key;
+  uint32_t const key_after = cnt > 0 && p1 < n ? keys[p1] : invalid_key;
+  auto key_at = [&](int j) { return (uint32_t)__builtin_amdgcn_readlane((int)my_key, j); };  // j < cnt
+  auto next_key = [&](int j) { return j + 1 < cnt ? key_at(j + 1) : key_after; };
+  bool const head_shared = cnt > 0 && p0 > 0 && key_before == key_at(0);
+
+  // this lane's columns, and those it reads instead where the row ends before them
+  uint32_t const col = blockIdx.y * PW + lane * VPL;
+  uint32_t const safe = col < (uint32_t)dim ? col : blockIdx.y * PW;
+  auto store_piece = [&](float *row, float const (&v)[VPL]) {
+    if (col >= (uint32_t)dim) return;
+    if constexpr (VPL == 4) *reinterpret_cast<f32x4 *>(row + col) = f32x4{v[0], v[1], v[2], v[3]};
+    else if constexpr (VPL == 2) *reinterpret_cast<f32x2 *>(row + col) = f32x2{v[0], v[1]};
+    else row[col] = v[0];
   };
-  for (int64_t cbase = 0; cbase < dim; cbase += PW) {
-    if (wl == 0) {
-      part_valid[2 * w] = 0;
-      part_valid[2 * w + 1] = 0;
-    }
-    {
-      float acc[CPL][4], rows[2][CPL][4];
-      f32x4 old[2][CPL];
-      // position j's gradient row, and the weight-gradient row of its id if a run of this
-      // walker alone ends there (nobody else touches that row during the kernel)
-      auto prefetch = [&](int j, uint32_t id, uint32_t next_id, uint32_t l, float (&v)[CPL][4], f32x4 (&o)[CPL]) {
-        if (j >= cnt) return;
-        GT const *row = dY + (int64_t)l * dim;  // l: the lookup's bag (see my_val)
-        bool const ends = j + 1 >= cnt || next_id != id;
+  if (lane == 0) {
+    part_valid[2 * w] = 0;
+    part_valid[2 * w + 1] = 0;
+  }
+  {
+    float acc[VPL], rows[DEPTH][VPL], old[DEPTH][VPL];
+    // position j's gradient row, and the weight-gradient row of its id if a run of this
+    // walker alone ends there (nobody else touches that row during the kernel)
+    auto prefetch = [&](int j, float (&v)[VPL], float (&o)[VPL]) {
+      if (j >= cnt) return;
+      uint32_t const id = key_at(j);
+      GT const *row = dY + (int64_t)(uint32_t)__builtin_amdgcn_readlane((int)my_val, j) * dim;
+      load_grad_piece<VPL, !BAGGED>(row + safe, v);
+      if (next_key(j) != id && id != invalid_key) {
+        float const *dst = dW + (int64_t)id * dim;
+        load_grad_piece<VPL, false>(dst + safe, o);
+      }
+    };
+    bool shared_run = head_shared;
+    auto step = [&](int j, float (&v)[VPL], float (&o)[VPL]) {
+      if (j >= cnt) return;
+      uint32_t const id = key_at(j);
 #pragma unroll
-        for (int k = 0; k < CPL; k++) {
-          int64_t const c = cbase + ((int64_t)k * LPR + wl) * 4;
-          if (c < dim) {
-            load_grad4<GT>(row + c, v[k]);
-            if (ends && id != invalid_key) o[k] = *reinterpret_cast<f32x4 const *>(dW + (int64_t)id * dim + c);
-          } else {
-            v[k][0] = v[k][1] = v[k][2] = v[k][3] = 0.0f;
-          }
-        }
-      };
+      for (int e = 0; e < VPL; e++) acc[e] += v[e];
+      bool const tail_shared = j + 1 == cnt && p1 < n && key_after == id;
+      if (tail_shared || j + 1 == cnt || next_key(j) != id) {
+        if (id != invalid_key) {
+          if (shared_run || tail_shared) {
+            // slot 2w: run shared with the previous walker (or both sides);
+            // slot 2w+1: run shared with the next walker only
+            int const slot = shared_run ? 2 * w : 2 * w + 1;
 #pragma unroll
-      for (int k = 0; k < CPL; k++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) acc[k][e] = 0.0f;
-      bool shared_run = head_shared;
-      // the ids around position j: id_j, id_{j+1}, id_{j+2}, id_{j+3} slide along with j
-      uint32_t id0 = key_at(0), id1 = key_at(1), id2 = key_at(2), l0 = lookup_at(0), l1 = lookup_at(1);
-      prefetch(0, id0, id1, l0, rows[0], old[0]);
-      prefetch(1, id1, id2, l1, rows[1], old[1]);
-      auto step = [&](int j, float (&v)[CPL][4], f32x4 (&o)[CPL]) {
-        // shuffles first, by every lane
-        uint32_t const id3 = key_at(j + 3);
-        uint32_t const l2 = lookup_at(j + 2);
-        if (j < cnt) {
-          uint32_t const id = id0;
-#pragma unroll
-          for (int k = 0; k < CPL; k++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[k][e] += v[k][e];
-          bool const more = j + 1 < cnt;
-          uint32_t const next_id = j + 1 < kEmbChunk ? id1 : key_after;
-          if (!more || next_id != id) {
-            bool const tail_shared = !more && p1 < n && key_after == id;
-            if (id != invalid_key) {
-              if (shared_run || tail_shared) {
-                // slot 2w: run shared with the previous walker (or both sides);
-                // slot 2w+1: run shared with the next walker only
-                int const slot = shared_run ? 2 * w : 2 * w + 1;
-#pragma unroll
-                for (int k = 0; k < CPL; k++) {
-                  f32x4 pv = {acc[k][0], acc[k][1], acc[k][2], acc[k][3]};
-                  *reinterpret_cast<f32x4 *>(emb_part + slot * PW + (k * LPR + wl) * 4) = pv;
-                }
-                if (wl == 0) {
-                  part_id[slot] = id;
-                  // 1: a border partial; 2 / 4: its run also extends before /
-                  // beyond the workgroup's positions
-                  part_valid[slot] = 1 | ((shared_run && p0 == block0) ? 2 : 0) |
-                                     ((tail_shared && p1 == block1) ? 4 : 0);
-                }
-              } else {
-#pragma unroll
-                for (int k = 0; k < CPL; k++) {
-                  int64_t const c = cbase + ((int64_t)k * LPR + wl) * 4;
-                  if (c < dim) {
-                    f32x4 upd = {o[k][0] + acc[k][0] * scale, o[k][1] + acc[k][1] * scale,
-                                 o[k][2] + acc[k][2] * scale, o[k][3] + acc[k][3] * scale};
-                    *reinterpret_cast<f32x4 *>(dW + (int64_t)id * dim + c) = upd;
-                  }
-                }
-              }
+            for (int e = 0; e < VPL; e++) emb_part[slot * PW + e * 64 + lane] = acc[e];
+            if (lane == 0) {
+              part_id[slot] = id;
+              // 1: a border partial; 2 / 4: its run also extends before /
+              // beyond the workgroup's positions
+              part_valid[slot] = 1 | ((shared_run && p0 == block0) ? 2 : 0) |
+                                 ((tail_shared && p1 == block1) ? 4 : 0);
             }
-            shared_run = false;
+          } else {
+            float *dst = dW + (int64_t)id * dim;
+            float u[VPL];
 #pragma unroll
-            for (int k = 0; k < CPL; k++)
-#pragma unroll
-              for (int e = 0; e < 4; e++) acc[k][e] = 0.0f;
+            for (int e = 0; e < VPL; e++) u[e] = o[e] + acc[e] * scale;
+            store_piece(dst, u);
           }
         }
-        // this slot is free now: position j + 2 goes into it
-        prefetch(j + 2, id2, j + 3 < kEmbChunk ? id3 : key_after, l2, v, o);
-        id0 = id1;
-        id1 = id2;
-        id2 = id3;
-      };
+        shared_run = false;
+#pragma unroll
+        for (int e = 0; e < VPL; e++) acc[e] = 0.0f;
+      }
+      // this slot is free now: position j + DEPTH goes into it
+      prefetch(j + DEPTH, v, o);
+    };
+#pragma unroll
+    for (int e = 0; e < VPL; e++) acc[e] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < DEPTH; j++) prefetch(j, rows[j], old[j]);
 #pragma unroll 1
-      for (int j = 0; j < kEmbChunk; j += 2) {
-        step(j, rows[0], old[0]);
-        step(j + 1, rows[1], old[1]);
-      }
+    for (int j = 0; j < cnt; j += DEPTH) {
+#pragma unroll
+      for (int u = 0; u < DEPTH; u++) step(j + u, rows[u], old[u]);
     }
-    __syncthreads();
-    // merge the border partials in position order (first LPR threads, their column chunks)
-    if (threadIdx.x < LPR) {
-      float acc[CPL][4];
+  }
+  __syncthreads();
+  // Merge the border partials.  A run that crosses walkers has one partial per walker: the one
+  // it starts in (slot 2w+1, or slot 0 if it comes from the workgroup before) and slot 2w of
+  // each walker it reaches.  The walker of the first adds them up in position order, all runs
+  // side by side.
+  for (int sidx = w == 0 ? 0 : 2 * w + 1; sidx <= 2 * w + 1; sidx++) {
+    int flags = __builtin_amdgcn_readfirstlane(part_valid[sidx]);
+    if (flags == 0) continue;
+    uint32_t const id = (uint32_t)__builtin_amdgcn_readfirstlane((int)part_id[sidx]);
+    float acc[VPL];
 #pragma unroll
-      for (int k = 0; k < CPL; k++)
+    for (int e = 0; e < VPL; e++) acc[e] = emb_part[sidx * PW + e * 64 + lane];
+    for (int nxt = (sidx | 1) + 1; nxt < 2 * kEmbWalkers && part_valid[nxt] != 0 && part_id[nxt] == id; nxt += 2) {
+      flags |= part_valid[nxt];
 #pragma unroll
-        for (int e = 0; e < 4; e++) acc[k][e] = 0.0f;
-      uint32_t cur_id = invalid_key;
-      int flags = 0;
-      for (int sidx = 0; sidx < 2 * WPB; sidx++) {
-        int const v = part_valid[sidx];
-        if (v == 0) continue;
-        uint32_t const id = part_id[sidx];
-        if (id != cur_id) {
-          if (cur_id != invalid_key) add_row(cur_id, cbase, acc, (flags & 6) != 0);
-          cur_id = id;
-          flags = 0;
-#pragma unroll
-          for (int k = 0; k < CPL; k++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[k][e] = 0.0f;
-        }
-        flags |= v;
-#pragma unroll
-        for (int k = 0; k < CPL; k++) {
-          f32x4 pv = *reinterpret_cast<f32x4 const *>(emb_part + sidx * PW + (k * LPR + wl) * 4);
-#pragma unroll
-          for (int e = 0; e < 4; e++) acc[k][e] += pv[e];
-        }
-      }
-      if (cur_id != invalid_key) add_row(cur_id, cbase, acc, (flags & 6) != 0);
+      for (int e = 0; e < VPL; e++) acc[e] += emb_part[nxt * PW + e * 64 + lane];
     }
-    __syncthreads();
+    float *dst = dW + (int64_t)id * dim;
+    if ((flags & 6) != 0) {
+      if (col < (uint32_t)dim) {
+#pragma unroll
+        for (int e = 0; e < VPL; e++) atomicAdd(dst + col + e, acc[e] * scale);
+      }
+    } else {
+      float u[VPL];
+      load_grad_piece<VPL, false>(dst + safe, u);
+#pragma unroll
+      for (int e = 0; e < VPL; e++) u[e] += acc[e] * scale;
+      store_piece(dst, u);
+    }
   }
 }
 
@@ -654,7 +643,7 @@ static int emb_backward(hipStream_t st, void const *indices, void const *dy,
                         size_t workspace_bytes, bool deterministic) {
   int64_t const lookups = num_bags * bag;
   EmbSortLayout L;
-  bool const sorted = workspace != nullptr && dim % 4 == 0 &&
+  bool const sorted = workspace != nullptr && dim % 4 == 0 && dim <= 65535 * 256 &&
                       reinterpret_cast<uintptr_t>(dy) % 16 == 0 &&
                       reinterpret_cast<uintptr_t>(dw) % 16 == 0 &&
                       reinterpret_cast<uintptr_t>(workspace) % 256 == 0 &&
@@ -667,28 +656,36 @@ static int emb_backward(hipStream_t st, void const *indices, void const *dy,
                                    reinterpret_cast<uint32_t *>(ws + L.vals_a), reinterpret_cast<uint32_t *>(ws + L.vals_b),
                                    reinterpret_cast<uint32_t *>(ws + L.table), &keys_out, &vals_out));
     GT const *G = static_cast<GT const *>(dy);
-    int64_t const walkers = ceil_div(lookups, kEmbChunk);
+    if (deterministic) {
+      int64_t const walkers = ceil_div(lookups, kEmbChunk);
 #define FFK_EMB_SORTED(LPR_, CPL_)                                             \
+  embedding_bwd_sorted_kernel<GT, LPR_, CPL_, true><<<(unsigned)ceil_div(walkers * LPR_, 256), 256, 0, st>>>( \
+      keys_out, vals_out, G, dw, lookups, (int)bag, dim, (uint32_t)num_entries, scale)
+      if (dim > 512) FFK_EMB_SORTED(64, 4);
+      else if (dim > 256) FFK_EMB_SORTED(64, 2);
+      else if (dim > 128) FFK_EMB_SORTED(64, 1);
+      else if (dim > 64) FFK_EMB_SORTED(32, 1);
+      else FFK_EMB_SORTED(16, 1);
+#undef FFK_EMB_SORTED
+      FFK_CHECK_LAUNCH();
+      return FFK_OK;
+    }
+    // Longer chunks mean fewer border partials and fewer atomics on hot rows; 16384 walkers are
+    // two for every wave the chip holds.
+    int64_t const groups = ceil_div(dim, 256);
+    int const chunk =
+        (int)std::min<int64_t>(kEmbMaxChunk, std::max<int64_t>(kEmbChunk, ceil_div(lookups * groups, 16384)));
+    dim3 const blocks((unsigned)ceil_div(lookups, (int64_t)kEmbWalkers * chunk), (unsigned)groups);
+#define FFK_EMB_SORTED(VPL_)                                                   \
   do {                                                                         \
-    if (deterministic) {                                                       \
-      unsigned const blocks = (unsigned)ceil_div(walkers * LPR_, 256);         \
-      embedding_bwd_sorted_kernel<GT, LPR_, CPL_, true><<<blocks, 256, 0, st>>>( \
-          keys_out, vals_out, G, dw, lookups, (int)bag, dim, (uint32_t)num_entries, scale); \
-    } else {                                                                   \
-      unsigned const blocks = (unsigned)ceil_div(walkers * LPR_, kEmbBlockThreads); \
-      auto kern = embedding_bwd_sorted_block_kernel<GT, LPR_, CPL_>;           \
-      int const lds = 2 * (kEmbBlockThreads / LPR_) * LPR_ * 4 * CPL_ * (int)sizeof(float); \
-      FFK_HIP(hipFuncSetAttribute(reinterpret_cast<void const *>(kern),        \
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds)); \
-      kern<<<blocks, kEmbBlockThreads, lds, st>>>(                             \
-          keys_out, vals_out, G, dw, lookups, (int)bag, dim, (uint32_t)num_entries, scale); \
-    }                                                                          \
+    auto kern = bag > 1 ? embedding_bwd_sorted_block_kernel<GT, VPL_, true>    \
+                        : embedding_bwd_sorted_block_kernel<GT, VPL_, false>;  \
+    kern<<<blocks, kEmbBlockThreads, 0, st>>>(keys_out, vals_out, G, dw, lookups, chunk, (int)bag, (int)dim, \
+                                              (uint32_t)num_entries, scale);   \
   } while (0)
-    if (dim > 512) FFK_EMB_SORTED(64, 4);
-    else if (dim > 256) FFK_EMB_SORTED(64, 2);
-    else if (dim > 128) FFK_EMB_SORTED(64, 1);
-    else if (dim > 64) FFK_EMB_SORTED(32, 1);
-    else FFK_EMB_SORTED(16, 1);
+    if (dim > 128) FFK_EMB_SORTED(4);
+    else if (dim > 64) FFK_EMB_SORTED(2);
+    else FFK_EMB_SORTED(1);
 #undef FFK_EMB_SORTED
     FFK_CHECK_LAUNCH();
     return FFK_OK;

@@ -13,15 +13,16 @@
 //              ranking the keys of a step among their peers with the same digit
 //              by ballots, so equal digits keep their input order (stable) and
 //              the result does not depend on timing (no atomics decide a place).
-// Up to kSortFusedTiles tiles (131 072 lookups) a pass is ONE launch: the scan
-// moves into the scatter kernel (every workgroup adds up the counts of the
-// tiles before its own and the totals of the digits below, straight from a
-// table that is only a few tens of kilobytes), and the scatter counts the NEXT
-// pass's digits of the keys it places, per destination tile, with integer
-// atomics (a count does not depend on the order of the additions; the counts
-// are gathered in LDS first, since under a skewed id distribution thousands of
-// a workgroup's keys share one counter).  A sort of
-// the token table's lookups is then 3 launches instead of 7.
+// Up to 524 288 lookups a pass is ONE launch: the scan moves into the scatter
+// kernel (every workgroup adds up the counts of the tiles before its own and the
+// totals of the digits below, straight from a table of at most 128 KB), and the
+// scatter counts the NEXT pass's digits of the keys it places, per destination
+// tile, with integer atomics (a count does not depend on the order of the
+// additions; the counts are gathered in LDS first, since under a skewed id
+// distribution thousands of a workgroup's keys share one counter), or beyond
+// 131 072 lookups a histogram launch does.  Digits are as
+// narrow as the number of passes allows (three of 7 bits for a million rows).  Up
+// to 4096 lookups the whole sort is one workgroup and one launch.
 // The first pass reads the caller's index tensor directly (int32 or int64,
 // ids outside the table become the key `invalid_key`, which sorts behind every
 // row) and numbers the lookups itself, so no pass exists only to build keys.
@@ -171,148 +172,339 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// The one-launch-per-pass form for few tiles.  Tables are [tile][digit], one per
-// pass (pass p's is filled by the histogram kernel for p = 0 and by pass p-1's
-// scatter otherwise; each kernel clears the table that the kernel after it adds
-// into, so no launch exists only to clear).
+// One launch per pass, up to kSortFusedTiles tiles of 1024 threads with ITEMS
+// keys each.  Tables are [tile][digit], one per pass (pass p's is filled by the
+// histogram kernel for p = 0 and by pass p-1's scatter otherwise; each kernel
+// clears the table that the kernel after it adds into, so no launch exists only
+// to clear).  Bound by the latency of one workgroup's chain (keys, ranks, table,
+// places), not by bandwidth, hence sixteen waves with at most four steps each,
+// the ranking under the table's loads, and digits no wider than the passes need.
+// Sort of 65 536 token ids below 50 257: 23 -> 18 us (tiles of 2048 keys and four
+// waves before); 524 288 ids below a million: 63 -> 51 us (three launches a pass
+// before); 1000 ids: three launches and 20 us less for the whole gradient.
 // ---------------------------------------------------------------------------
-constexpr int kSortFusedTiles = 48;  // a workgroup keeps its next-pass counts [tiles][256] in LDS
+constexpr int kSortFusedThreads = 1024;
+constexpr int kSortFusedWaves = kSortFusedThreads / 64;
+constexpr int kSortFusedTiles = 128;
+constexpr int kSortFusedItems = 4;  // the most keys per thread
 
-template <typename IT>
-__global__ __launch_bounds__(kSortThreads) void radix_hist0_fused_kernel(IT const *__restrict__ idx,
-                                                                        uint32_t *__restrict__ table0,
-                                                                        uint32_t *__restrict__ table1, int64_t n,
-                                                                        int64_t num_entries) {
-  __shared__ uint32_t cnt[kSortRadix];
-  cnt[threadIdx.x] = 0;
-  __syncthreads();
-  int64_t const base = (int64_t)blockIdx.x * kSortTile;
-#pragma unroll
-  for (int k = 0; k < kSortItems; k++) {
-    int64_t const i = base + k * kSortThreads + threadIdx.x;
-    if (i < n) {
-      uint32_t const key = sort_key_at<IT, true>(idx, nullptr, i, num_entries);
-      atomicAdd(&cnt[key & (kSortRadix - 1)], 1u);
-    }
+// A step's lanes with this lane's digit (all of them take part; `valid` lanes only are counted).
+__device__ __forceinline__ uint64_t sort_peers(bool valid, uint32_t digit, int bits) {
+  uint64_t peers = __ballot(valid);
+  for (int bit = 0; bit < bits; bit++) {
+    uint64_t const m = __ballot((digit >> bit) & 1u);
+    peers &= ((digit >> bit) & 1u) ? m : ~m;
   }
-  __syncthreads();
-  table0[(int64_t)blockIdx.x * kSortRadix + threadIdx.x] = cnt[threadIdx.x];
-  if (table1 != nullptr) table1[(int64_t)blockIdx.x * kSortRadix + threadIdx.x] = 0;
+  return peers;
 }
 
-// table: this pass's counts; next: the next pass's table (nullptr on the last pass), added
-// into here; after: the table of the pass after that (nullptr if none), cleared here.
-template <typename IT, bool FIRST>
-__global__ __launch_bounds__(kSortThreads) void radix_scatter_fused_kernel(
-    IT const *__restrict__ idx, uint32_t const *__restrict__ keys_in, uint32_t const *__restrict__ vals_in,
-    uint32_t *__restrict__ keys_out, uint32_t *__restrict__ vals_out, uint32_t const *__restrict__ table,
-    uint32_t *__restrict__ next, uint32_t *__restrict__ after, int64_t n, int ntiles, int shift, int64_t num_entries) {
-  __shared__ uint32_t wave_off[4][kSortRadix];
-  __shared__ uint32_t wsum[4];
-  __shared__ uint32_t next_cnt[kSortFusedTiles][kSortRadix];  // this workgroup's share of the next pass's table
-  int const t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  for (int d = lane; d < kSortRadix; d += 64) wave_off[wave][d] = 0;
-  if (next != nullptr) {
-    for (int r = 0; r < ntiles; r++) next_cnt[r][t] = 0;
-  }
-  int64_t const first = (int64_t)blockIdx.x * kSortTile + (int64_t)wave * kSortWaveKeys;
-  constexpr int STEPS = kSortWaveKeys / 64;
-  uint32_t key[STEPS], val[STEPS];
+// Place of each of a wave's keys among the wave's keys with the same digit, in
+// input order; leaves the wave's digit counts in `count` (cleared by the caller).
+template <int ITEMS>
+__device__ __forceinline__ void sort_rank_wave(uint32_t const (&digit)[ITEMS], bool const (&valid)[ITEMS], int bits,
+                                               int lane, uint32_t *count, uint32_t (&rank)[ITEMS]) {
+  uint64_t const below = ((uint64_t)1 << lane) - 1;
 #pragma unroll
-  for (int c = 0; c < STEPS; c++) {
-    int64_t const i = first + c * 64 + lane;
-    key[c] = 0;
-    val[c] = 0;
-    if (i < n) {
-      key[c] = sort_key_at<IT, FIRST>(idx, keys_in, i, num_entries);
-      val[c] = FIRST ? (uint32_t)i : vals_in[i];
-      atomicAdd(&wave_off[wave][(key[c] >> shift) & (kSortRadix - 1)], 1u);
+  for (int c = 0; c < ITEMS; c++) {
+    uint64_t const peers = sort_peers(valid[c], digit[c], bits);
+    rank[c] = 0;
+    if (valid[c]) {
+      uint32_t const seen = count[digit[c]];
+      uint32_t const r = (uint32_t)__popcll(peers & below);
+      rank[c] = seen + r;
+      // LDS operations of a wave complete in program order: every peer has read `seen`
+      // before the first of them moves it on for the next step
+      if (r == 0) count[digit[c]] = seen + (uint32_t)__popcll(peers);
     }
+    __builtin_amdgcn_wave_barrier();  // the compiler keeps the next step's reads behind this
   }
-  // thread d: the keys with digit d in the tiles before this one, and in all tiles
-  uint32_t before_tiles = 0, all_tiles = 0;
-  {
-    int const tile = blockIdx.x;
-    for (int t0 = 0; t0 < ntiles; t0 += 8) {
-      uint32_t v[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = t0 + u < ntiles ? table[(int64_t)(t0 + u) * kSortRadix + t] : 0u;
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        all_tiles += v[u];
-        before_tiles += t0 + u < tile ? v[u] : 0u;
-      }
-    }
-  }
-  if (after != nullptr) after[(int64_t)blockIdx.x * kSortRadix + t] = 0;
-  // exclusive scan of all_tiles over the digits: the keys with a smaller digit
-  uint32_t incl = all_tiles;
+}
+
+// Exclusive prefix sum of v over the threads below `bins` (at most 256; the others pass 0).
+// Every thread calls it; it synchronises the workgroup once, on the way.
+__device__ __forceinline__ uint32_t sort_scan_bins(uint32_t v, int t, int lane, uint32_t *wsum) {
+  uint32_t incl = v;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
     uint32_t const up = __shfl_up(incl, off, 64);
     if (lane >= off) incl += up;
   }
-  if (lane == 63) wsum[wave] = incl;
-  __syncthreads();  // also orders the wave_off counts above before their use below
-  uint32_t smaller = incl - all_tiles;
+  if (lane == 63 && t < kSortRadix) wsum[t >> 6] = incl;
+  __syncthreads();
+  uint32_t excl = incl - v;
 #pragma unroll
-  for (int w = 0; w < 4; w++) smaller += w < wave ? wsum[w] : 0u;
+  for (int w = 0; w < kSortRadix / 64; w++) excl += w < (t >> 6) && t < kSortRadix ? wsum[w] : 0u;
+  return excl;
+}
+
+template <typename IT, bool FIRST>
+__global__ __launch_bounds__(kSortFusedThreads) void radix_hist_fused_kernel(IT const *__restrict__ idx,
+                                                                            uint32_t const *__restrict__ keys_in,
+                                                                            uint32_t *__restrict__ table0,
+                                                                            uint32_t *__restrict__ table1, int64_t n,
+                                                                            int items, int shift, int bits,
+                                                                            int64_t num_entries) {
+  __shared__ uint32_t cnt[kSortRadix];
+  int const t = threadIdx.x, bins = 1 << bits;
+  if (t < kSortRadix) cnt[t] = 0;
+  __syncthreads();
+  int64_t const base = (int64_t)blockIdx.x * kSortFusedThreads * items;
+#pragma unroll
+  for (int k = 0; k < kSortFusedItems; k++) {
+    int64_t const i = base + k * kSortFusedThreads + t;
+    if (k < items && i < n) {
+      uint32_t const key = sort_key_at<IT, FIRST>(idx, keys_in, i, num_entries);
+      atomicAdd(&cnt[(key >> shift) & (bins - 1)], 1u);  // LDS; a count does not depend on order
+    }
+  }
+  __syncthreads();
+  if (t < bins) {
+    table0[(int64_t)blockIdx.x * bins + t] = cnt[t];
+    if (table1 != nullptr) table1[(int64_t)blockIdx.x * bins + t] = 0;
+  }
+}
+
+// table: this pass's counts; next: the next pass's table (nullptr on the last pass), added
+// into here; after: the table of the pass after that (nullptr if none), cleared here.
+// Dynamic LDS: the workgroup's share of the next table, 16-bit counters in pairs (a workgroup
+// counts its own keys there, at most 4096).
+template <typename IT, bool FIRST, int ITEMS>
+__global__ __launch_bounds__(kSortFusedThreads) void radix_scatter_fused_kernel(
+    IT const *__restrict__ idx, uint32_t const *__restrict__ keys_in, uint32_t const *__restrict__ vals_in,
+    uint32_t *__restrict__ keys_out, uint32_t *__restrict__ vals_out, uint32_t const *__restrict__ table,
+    uint32_t *__restrict__ next, uint32_t *__restrict__ after, int64_t n, int ntiles, int shift, int bits,
+    int64_t num_entries) {
+  constexpr int TILE = kSortFusedThreads * ITEMS;
+  extern __shared__ uint32_t next_cnt[];
+  __shared__ uint32_t wave_off[kSortFusedWaves][kSortRadix];
+  __shared__ uint32_t part_all[kSortFusedThreads], part_before[kSortFusedThreads];
+  __shared__ uint32_t wsum[kSortRadix / 64];
+  int const t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  int const bins = 1 << bits, mask = bins - 1;
+  int const next_words = next != nullptr ? (ntiles * bins + 1) / 2 : 0;
+  for (int d = lane; d < bins; d += 64) wave_off[wave][d] = 0;
+  for (int i = t; i < next_words; i += kSortFusedThreads) next_cnt[i] = 0;
+  int64_t const first = (int64_t)blockIdx.x * TILE + wave * (64 * ITEMS);
+  uint32_t key[ITEMS], val[ITEMS], digit[ITEMS], rank[ITEMS];
+  bool valid[ITEMS];
+#pragma unroll
+  for (int c = 0; c < ITEMS; c++) {
+    int64_t const i = first + c * 64 + lane;
+    valid[c] = i < n;
+    key[c] = 0;
+    val[c] = 0;
+    if (valid[c]) {
+      key[c] = sort_key_at<IT, FIRST>(idx, keys_in, i, num_entries);
+      val[c] = FIRST ? (uint32_t)i : vals_in[i];
+    }
+  }
+  // the keys with digit d in the tiles before this one, and in all tiles: 1024 / bins threads a digit
   {
-    uint32_t run = smaller + before_tiles;
+    int const d = t & mask, part = t >> bits, parts = kSortFusedThreads >> bits, tile = blockIdx.x;
+    uint32_t before_tiles = 0, all_tiles = 0;
+    for (int t0 = part; t0 < ntiles; t0 += 8 * parts) {
+      uint32_t v[8];
 #pragma unroll
-    for (int w = 0; w < 4; w++) {
+      for (int u = 0; u < 8; u++) v[u] = t0 + u * parts < ntiles ? table[(int64_t)(t0 + u * parts) * bins + d] : 0u;
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        all_tiles += v[u];
+        before_tiles += t0 + u * parts < tile ? v[u] : 0u;
+      }
+    }
+    part_all[t] = all_tiles;
+    part_before[t] = before_tiles;
+  }
+  if (after != nullptr && t < bins) after[(int64_t)blockIdx.x * bins + t] = 0;
+#pragma unroll
+  for (int c = 0; c < ITEMS; c++) digit[c] = (key[c] >> shift) & mask;
+  sort_rank_wave<ITEMS>(digit, valid, bits, lane, wave_off[wave], rank);
+  __syncthreads();
+  uint32_t all = 0, before = 0;
+  if (t < bins) {
+    for (int p = t; p < kSortFusedThreads; p += bins) {
+      all += part_all[p];
+      before += part_before[p];
+    }
+  }
+  uint32_t const smaller = sort_scan_bins(all, t, lane, wsum);
+  if (t < bins) {
+    uint32_t run = smaller + before;
+#pragma unroll
+    for (int w = 0; w < kSortFusedWaves; w++) {
       uint32_t const c = wave_off[w][t];
       wave_off[w][t] = run;
       run += c;
     }
   }
   __syncthreads();
-  uint64_t const below = ((uint64_t)1 << lane) - 1;
 #pragma unroll
-  for (int c = 0; c < STEPS; c++) {
-    bool const valid = first + c * 64 + lane < n;
-    uint32_t const digit = (key[c] >> shift) & (kSortRadix - 1);
-    uint64_t peers = __ballot(valid);
-#pragma unroll
-    for (int bit = 0; bit < 8; bit++) {
-      uint64_t const m = __ballot((digit >> bit) & 1u);
-      peers &= ((digit >> bit) & 1u) ? m : ~m;
-    }
-    if (valid) {
-      uint32_t const start = wave_off[wave][digit];
-      uint32_t const rank = (uint32_t)__popcll(peers & below);
-      uint32_t const pos = start + rank;
+  for (int c = 0; c < ITEMS; c++) {
+    if (valid[c]) {
+      uint32_t const pos = wave_off[wave][digit[c]] + rank[c];
       keys_out[pos] = key[c];
       vals_out[pos] = val[c];
       // the next pass's count of this key, in the tile it has just been placed in
-      if (next != nullptr) atomicAdd(&next_cnt[pos / kSortTile][(key[c] >> (shift + 8)) & (kSortRadix - 1)], 1u);
-      if (rank == 0) wave_off[wave][digit] = start + (uint32_t)__popcll(peers);
+      if (next != nullptr) {
+        uint32_t const nd = (pos / TILE) * bins + ((key[c] >> (shift + bits)) & mask);
+        atomicAdd(&next_cnt[nd >> 1], 1u << (16 * (nd & 1u)));
+      }
     }
   }
   if (next != nullptr) {
     __syncthreads();
-    for (int r = 0; r < ntiles; r++) {
-      uint32_t const c = next_cnt[r][t];
-      if (c != 0) atomicAdd(&next[(int64_t)r * kSortRadix + t], c);
+    for (int i = t; i < next_words; i += kSortFusedThreads) {
+      uint32_t const c = next_cnt[i];
+      if ((c & 0xffffu) != 0) atomicAdd(&next[2 * (int64_t)i], c & 0xffffu);
+      if ((c >> 16) != 0) atomicAdd(&next[2 * (int64_t)i + 1], c >> 16);
+    }
+  }
+}
+
+// Up to 4096 lookups: the whole sort in one workgroup, pairs handed round through LDS.
+template <typename IT, int ITEMS>
+__global__ __launch_bounds__(kSortFusedThreads) void radix_sort_block_kernel(IT const *__restrict__ idx,
+                                                                            uint32_t *__restrict__ keys_out,
+                                                                            uint32_t *__restrict__ vals_out, int n,
+                                                                            int passes, int bits, int64_t num_entries) {
+  __shared__ uint32_t ks[kSortFusedThreads * ITEMS], vs[kSortFusedThreads * ITEMS];
+  __shared__ uint32_t wave_off[kSortFusedWaves][kSortRadix];
+  __shared__ uint32_t wsum[kSortRadix / 64];
+  int const t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  int const bins = 1 << bits, mask = bins - 1;
+  int const first = wave * (64 * ITEMS) + lane;
+  uint32_t key[ITEMS], val[ITEMS], digit[ITEMS], rank[ITEMS];
+  bool valid[ITEMS];
+#pragma unroll
+  for (int c = 0; c < ITEMS; c++) {
+    int const i = first + c * 64;
+    valid[c] = i < n;
+    key[c] = valid[c] ? sort_key_at<IT, true>(idx, nullptr, i, num_entries) : 0u;
+    val[c] = (uint32_t)i;
+  }
+  for (int pass = 0; pass < passes; pass++) {
+    for (int d = lane; d < bins; d += 64) wave_off[wave][d] = 0;
+#pragma unroll
+    for (int c = 0; c < ITEMS; c++) digit[c] = (key[c] >> (pass * bits)) & mask;
+    sort_rank_wave<ITEMS>(digit, valid, bits, lane, wave_off[wave], rank);
+    __syncthreads();
+    uint32_t all = 0;
+    if (t < bins) {
+#pragma unroll
+      for (int w = 0; w < kSortFusedWaves; w++) all += wave_off[w][t];
+    }
+    uint32_t run = sort_scan_bins(all, t, lane, wsum);
+    if (t < bins) {
+#pragma unroll
+      for (int w = 0; w < kSortFusedWaves; w++) {
+        uint32_t const c = wave_off[w][t];
+        wave_off[w][t] = run;
+        run += c;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < ITEMS; c++) {
+      if (valid[c]) {
+        uint32_t const pos = wave_off[wave][digit[c]] + rank[c];
+        ks[pos] = key[c];
+        vs[pos] = val[c];
+      }
+    }
+    __syncthreads();
+    // every key is read before the next pass's places are written: two barriers lie between
+#pragma unroll
+    for (int c = 0; c < ITEMS; c++) {
+      if (valid[c]) {
+        key[c] = ks[first + c * 64];
+        val[c] = vs[first + c * 64];
+      }
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < ITEMS; c++) {
+    if (valid[c]) {
+      keys_out[first + c * 64] = key[c];
+      vals_out[first + c * 64] = val[c];
     }
   }
 }
 
 struct RadixSortPlan {
   int passes;
+  int bits;            // of a digit
   int ntiles;
-  bool fused;          // one launch per pass (few tiles)
-  size_t table_bytes;  // fused: one [ntiles][256] table per pass; otherwise one [256][ntiles] table, then the digit totals [passes][256]
+  int items;           // fused: keys per thread
+  bool fused;          // one launch per pass, or (one tile) one launch in all
+  size_t table_bytes;  // fused: one [ntiles][bins] table per pass; otherwise one [256][ntiles] table, then the digit totals [passes][256]
 };
 
 static inline RadixSortPlan radix_sort_plan(int64_t n, unsigned key_bits) {
   RadixSortPlan p;
   p.passes = (int)((key_bits + 7) / 8);
-  p.ntiles = (int)ceil_div(n, kSortTile);
-  p.fused = p.ntiles <= kSortFusedTiles;
-  p.table_bytes = p.fused ? (size_t)kSortRadix * (size_t)p.ntiles * (size_t)p.passes * sizeof(uint32_t)
-                          : (size_t)kSortRadix * ((size_t)p.ntiles + (size_t)p.passes) * sizeof(uint32_t);
+  p.bits = 8;
+  // Fused while the tables a workgroup reads and counts into stay small (128 tiles: 64 KB of LDS).
+  // More keys than that take the three launches a pass, whose cost per key is lower.
+  p.fused = n <= (int64_t)kSortFusedTiles * kSortFusedThreads * kSortFusedItems;
+  p.items = 0;
+  if (p.fused) {
+    p.bits = (int)((key_bits + p.passes - 1) / p.passes);
+    // one tile as long as four keys per thread cover everything; then as few keys per thread as the tile limit allows
+    p.items = n <= kSortFusedThreads ? 1 : kSortFusedItems;
+    if (n > (int64_t)kSortFusedThreads * kSortFusedItems) {
+      p.items = 1;
+      while (n > (int64_t)kSortFusedTiles * kSortFusedThreads * p.items) p.items *= 2;
+    }
+    p.ntiles = (int)ceil_div(n, (int64_t)kSortFusedThreads * p.items);
+    p.table_bytes = ((size_t)p.ntiles << p.bits) * (size_t)p.passes * sizeof(uint32_t);
+  } else {
+    p.ntiles = (int)ceil_div(n, kSortTile);
+    p.table_bytes = (size_t)kSortRadix * ((size_t)p.ntiles + (size_t)p.passes) * sizeof(uint32_t);
+  }
   return p;
+}
+
+template <typename IT, int ITEMS>
+static inline hipError_t radix_sort_fused(hipStream_t st, IT const *idx, int64_t n, int64_t num_entries,
+                                          RadixSortPlan const &plan, uint32_t *keys_a, uint32_t *keys_b,
+                                          uint32_t *vals_a, uint32_t *vals_b, uint32_t *table,
+                                          uint32_t **keys_sorted, uint32_t **vals_sorted) {
+  size_t const tsz = (size_t)plan.ntiles << plan.bits;
+  unsigned const blocks = (unsigned)plan.ntiles;
+  // Counting the next pass's digits while placing costs an atomic for nearly every (tile, digit)
+  // pair of every workgroup: cheaper than a launch up to one key per thread, several times
+  // dearer beyond (524 288 keys: 13-21 us a pass against 5 for the launch and 12 without the counting).
+  constexpr bool kCountAhead = ITEMS == 1;
+  auto tab = [&](int pass) -> uint32_t * { return pass < plan.passes ? table + (size_t)pass * tsz : nullptr; };
+  auto ahead = [&](int pass) -> uint32_t * { return kCountAhead ? tab(pass) : nullptr; };
+  uint32_t *kin = nullptr, *vin = nullptr, *kout = keys_a, *vout = vals_a;
+  for (int pass = 0; pass < plan.passes; pass++) {
+    if (pass == 0) {
+      radix_hist_fused_kernel<IT, true><<<blocks, kSortFusedThreads, 0, st>>>(idx, nullptr, tab(0), ahead(1), n, ITEMS,
+                                                                             0, plan.bits, num_entries);
+    } else if (!kCountAhead) {
+      radix_hist_fused_kernel<IT, false><<<blocks, kSortFusedThreads, 0, st>>>(
+          idx, kin, tab(pass), nullptr, n, ITEMS, plan.bits * pass, plan.bits, num_entries);
+    }
+    auto kern = pass == 0 ? radix_scatter_fused_kernel<IT, true, ITEMS> : radix_scatter_fused_kernel<IT, false, ITEMS>;
+    size_t const lds = ahead(pass + 1) != nullptr ? (tsz + 1) / 2 * sizeof(uint32_t) : 0;
+    if (lds > 32 * 1024) {  // with the static part, more than a launch may ask for by default
+      hipError_t const e = hipFuncSetAttribute(reinterpret_cast<void const *>(kern),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (e != hipSuccess) return e;
+    }
+    kern<<<blocks, kSortFusedThreads, lds, st>>>(idx, kin, vin, kout, vout, tab(pass), ahead(pass + 1), ahead(pass + 2), n,
+                                                 plan.ntiles, plan.bits * pass, plan.bits, num_entries);
+    hipError_t const e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    kin = kout;
+    vin = vout;
+    kout = kin == keys_a ? keys_b : keys_a;
+    vout = vin == vals_a ? vals_b : vals_a;
+  }
+  *keys_sorted = kin;
+  *vals_sorted = vin;
+  return hipSuccess;
 }
 
 // Sorts the n lookups of `idx` by row id.  bufs: two key arrays and two value
@@ -323,32 +515,28 @@ static inline hipError_t radix_sort_lookups(hipStream_t st, IT const *idx, int64
                                             RadixSortPlan const &plan, uint32_t *keys_a, uint32_t *keys_b,
                                             uint32_t *vals_a, uint32_t *vals_b, uint32_t *table,
                                             uint32_t **keys_sorted, uint32_t **vals_sorted) {
-  uint32_t *kin = nullptr, *vin = nullptr, *kout = keys_a, *vout = vals_a;
   if (plan.fused) {
-    unsigned const blocks = (unsigned)plan.ntiles;
-    size_t const tsz = (size_t)kSortRadix * plan.ntiles;
-    auto tab = [&](int pass) -> uint32_t * { return pass < plan.passes ? table + (size_t)pass * tsz : nullptr; };
-    radix_hist0_fused_kernel<IT><<<blocks, kSortThreads, 0, st>>>(idx, tab(0), tab(1), n, num_entries);
-    for (int pass = 0; pass < plan.passes; pass++) {
-      int const shift = 8 * pass;
-      if (pass == 0) {
-        radix_scatter_fused_kernel<IT, true><<<blocks, kSortThreads, 0, st>>>(
-            idx, nullptr, nullptr, kout, vout, tab(0), tab(1), tab(2), n, plan.ntiles, shift, num_entries);
+    if (plan.ntiles == 1) {
+      if (plan.items == 1) {
+        radix_sort_block_kernel<IT, 1><<<1, kSortFusedThreads, 0, st>>>(idx, keys_a, vals_a, (int)n, plan.passes,
+                                                                        plan.bits, num_entries);
       } else {
-        radix_scatter_fused_kernel<IT, false><<<blocks, kSortThreads, 0, st>>>(
-            idx, kin, vin, kout, vout, tab(pass), tab(pass + 1), tab(pass + 2), n, plan.ntiles, shift, num_entries);
+        radix_sort_block_kernel<IT, kSortFusedItems><<<1, kSortFusedThreads, 0, st>>>(
+            idx, keys_a, vals_a, (int)n, plan.passes, plan.bits, num_entries);
       }
-      hipError_t const e = hipGetLastError();
-      if (e != hipSuccess) return e;
-      kin = kout;
-      vin = vout;
-      kout = kin == keys_a ? keys_b : keys_a;
-      vout = vin == vals_a ? vals_b : vals_a;
+      *keys_sorted = keys_a;
+      *vals_sorted = vals_a;
+      return hipGetLastError();
     }
-    *keys_sorted = kin;
-    *vals_sorted = vin;
-    return hipSuccess;
+#define FFK_SORT_FUSED(ITEMS_)                                                                              \
+  return radix_sort_fused<IT, ITEMS_>(st, idx, n, num_entries, plan, keys_a, keys_b, vals_a, vals_b, table, \
+                                      keys_sorted, vals_sorted)
+    if (plan.items == 1) FFK_SORT_FUSED(1);
+    if (plan.items == 2) FFK_SORT_FUSED(2);
+    FFK_SORT_FUSED(4);
+#undef FFK_SORT_FUSED
   }
+  uint32_t *kin = nullptr, *vin = nullptr, *kout = keys_a, *vout = vals_a;
   uint32_t *const totals_all = table + (size_t)kSortRadix * plan.ntiles;
   radix_zero_kernel<<<plan.passes, 256, 0, st>>>(totals_all, plan.passes * kSortRadix);
   for (int pass = 0; pass < plan.passes; pass++) {
