@@ -21,10 +21,10 @@
 // (lib/op-attrs/src/op-attrs/ops/attention.cc:23-37).  DP is the larger of
 // the two rounded up to 32, 64, 128 or 256; the missing columns of either
 // kind are read as zeros.  At DP = 256 a wave's operands and accumulators no
-// longer fit its 512 registers in one pass: tiles are then loaded without a
-// register prefetch and dK and dV are produced by two launches of the dK/dV
-// kernel (WHAT = 1: dV only, needs K; WHAT = 2: dK only, needs K and V).
+// longer fit its 512 registers in one pass of the backward: there two waves
+// share their rows (the pair kernels), and tiles go straight to LDS.
 #include "ffk_common.h"
+#include "lds_dma.h"
 
 namespace ffk {
 
@@ -54,6 +54,27 @@ struct AttnF32Cfg {
   // next tile fetched into registers while this one is computed on (not at DP = 256: no room)
   static constexpr bool kPrefetch = DP <= 128;
 };
+
+// DP = 256: the next tile goes straight to LDS while this one is computed on, a row (64 lanes of 16
+// bytes) per instruction.  With one wave per SIMD nothing else covers the loads: without it every
+// 32-row tile waited for its rows (batch 8 x 8 heads x 512: forward 176 -> 172 us).
+// `rsrc`: the operand's rows of this (batch, head); lanes beyond its head size D read zeros (their
+// offset lies past any bound).  Row offsets fit 31 bits (checked on the host).
+constexpr unsigned kRowsBound = 0x80000000u;
+__device__ __forceinline__ unsigned row_lane_offset(int lane, int D) {
+  return lane * 4 < D ? (unsigned)lane * 16u : kRowsBound;
+}
+template <int STRIDE>
+__device__ __forceinline__ void tile_dma(i32x4 rsrc, unsigned lane_off, int64_t row_stride, int row0, int last_row,
+                                         int wave, float *tile) {
+  unsigned const lds = lds_address_of(tile);
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    int const row = wave * 8 + i;
+    lds_dma16(rsrc, lane_off, (unsigned)min(row0 + row, last_row) * (unsigned)(row_stride * 4),
+              lds + (unsigned)(row * STRIDE * 4));
+  }
+}
 
 __device__ __forceinline__ f32x4 load4_or_zero(float const *row, int d0, int D) {
   f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -97,22 +118,73 @@ __device__ __forceinline__ void tile_lstore(float *tile, int t, f32x4 const (&r)
 
 // acc (+)= T . owned^T over d: rows = the tile's rows, columns = the owned rows
 // of this wave (one per lane and half).  tile_lane = tile + (l%32)*stride + h*DP/2.
+// Both contractions read the LDS fragments of a group of matrix instructions under the group before
+// it (at least four of 64 cycles each), held there by scheduling barriers: with one or two waves to
+// a SIMD nothing else covers the LDS latency, and the compiler left alone puts every read right in
+// front of the two instructions that use it.  Head size 256, batch 8 x 8 heads x 512: forward 172 -> 167
+// us, dK/dV 359 -> 345, dQ 278 -> 273.
 template <int DP>
 __device__ __forceinline__ void contract_d(float const *tile_lane, float const (&owned)[DP / 2], f32x16 &acc) {
+  constexpr int N = DP / 8, G = 2;
+  f32x4 a[2][G];
 #pragma unroll
-  for (int c = 0; c < DP / 8; c++) {
-    f32x4 const a = *reinterpret_cast<f32x4 const *>(tile_lane + 4 * c);
+  for (int g = 0; g < G; g++) a[0][g] = *reinterpret_cast<f32x4 const *>(tile_lane + 4 * g);
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], owned[4 * c + e], acc, 0, 0, 0);
+  for (int c = 0; c < N; c += G) {
+    if (c + G < N) {
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        a[(c / G + 1) & 1][g] = *reinterpret_cast<f32x4 const *>(tile_lane + 4 * (c + G + g));
+      }
     }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < G; g++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[(c / G) & 1][g][e], owned[4 * (c + g) + e], acc, 0, 0, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// acc[i] += (columns 32 i .. of the tile's rows) x (score tile), over the tile's 32 rows.  The score
+// tile is an accumulator's 16 elements per lane; step r takes the rows 8*(r/4) + 4*h + r%4.
+// tile_lane = tile + 4*h*STRIDE + l%32.  TILE_A: the tile is the A operand (rows of the result =
+// its columns), otherwise the B operand.
+template <int N, int STRIDE, bool TILE_A>
+__device__ __forceinline__ void contract_rows(float const *tile_lane, float const (&score)[16], f32x16 (&acc)[N]) {
+  constexpr int G = N >= 8 ? 1 : N >= 4 ? 2 : 4;
+  float f[2][G][N];
+  auto read = [&](int r0, float (&d)[G][N]) {
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      int const row = 8 * ((r0 + g) >> 2) + ((r0 + g) & 3);
+#pragma unroll
+      for (int i = 0; i < N; i++) d[g][i] = tile_lane[row * STRIDE + i * 32];
+    }
+  };
+  read(0, f[0]);
+#pragma unroll
+  for (int r = 0; r < 16; r += G) {
+    if (r + G < 16) read(r + G, f[(r / G + 1) & 1]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < G; g++)
+#pragma unroll
+      for (int i = 0; i < N; i++) {
+        float const t = f[(r / G) & 1][g][i];
+        acc[i] = TILE_A ? __builtin_amdgcn_mfma_f32_32x32x2f32(t, score[r + g], acc[i], 0, 0, 0)
+                        : __builtin_amdgcn_mfma_f32_32x32x2f32(score[r + g], t, acc[i], 0, 0, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
 // --------------------------------------------------------------------------
 // forward: workgroup = 128 query rows of one (batch, head), 32 per wave
 // --------------------------------------------------------------------------
-template <int DP>
+template <int DP, bool DMA>
 __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(AttnF32Params p) {
   using C = AttnF32Cfg<DP>;
   __shared__ __attribute__((aligned(16))) float Ks[2][C::kTile * C::kStrideA];
@@ -144,22 +216,40 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(AttnF32Params p) {
   float m_run = -INFINITY, l_run = 0.0f;
 
   f32x4 rk[C::kChunks], rv[C::kChunks];
-  auto fetch = [&](int kv0) {
-    tile_gload<DP>(kp, p.k_ss, kv0, p.Skv - 1, p.Dq, t, rk);
-    tile_gload<DP>(vp, p.v_ss, kv0, p.Skv - 1, p.Dv, t, rv);
+  i32x4 k_rsrc, v_rsrc;
+  unsigned k_lane = 0, v_lane = 0;
+  if constexpr (DMA) {
+    k_rsrc = buffer_resource(kp, kRowsBound);
+    v_rsrc = buffer_resource(vp, kRowsBound);
+    k_lane = row_lane_offset(lane, p.Dq);
+    v_lane = row_lane_offset(lane, p.Dv);
+  }
+  auto fetch = [&](int kv0, int buf) {
+    if constexpr (DMA) {
+      tile_dma<C::kStrideA>(k_rsrc, k_lane, p.k_ss, kv0, p.Skv - 1, wave, Ks[buf]);
+      tile_dma<C::kStrideB>(v_rsrc, v_lane, p.v_ss, kv0, p.Skv - 1, wave, Vs[buf]);
+    } else {
+      tile_gload<DP>(kp, p.k_ss, kv0, p.Skv - 1, p.Dq, t, rk);
+      tile_gload<DP>(vp, p.v_ss, kv0, p.Skv - 1, p.Dv, t, rv);
+    }
   };
   auto stash = [&](int buf) {
-    tile_lstore<DP, C::kStrideA>(Ks[buf], t, rk);
-    tile_lstore<DP, C::kStrideB>(Vs[buf], t, rv);
+    if constexpr (DMA) {
+      wait_vmcnt<0>();
+    } else {
+      tile_lstore<DP, C::kStrideA>(Ks[buf], t, rk);
+      tile_lstore<DP, C::kStrideB>(Vs[buf], t, rv);
+    }
   };
-  fetch(0);
+  fetch(0, 0);
   stash(0);
+  if constexpr (DMA) wait_all_vmem_known_to_compiler();
   __syncthreads();
   int cur = 0;
   for (int it = 0; it < ntiles; it++) {
     int const kv0 = it * C::kTile;
     bool const more = it + 1 < ntiles;
-    if (C::kPrefetch && more) fetch(kv0 + C::kTile);
+    if ((DMA || C::kPrefetch) && more) fetch(kv0 + C::kTile, cur ^ 1);
     // a wave whose rows all lie before this tile (causal) has nothing to add
     bool const active = !p.causal || kv0 <= q0 + wave * 32 + 31;
     if (active) {
@@ -200,18 +290,10 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(AttnF32Params p) {
           for (int r = 0; r < 16; r++) oacc[i][r] *= alpha;
       }
       // O^T += V^T P^T: A = V^T (row d), B = P^T (column = query), reduction over keys
-      float const *vt = Vs[cur] + (4 * h32) * C::kStrideB + l32;
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        int const krow = 8 * (r >> 2) + (r & 3);
-#pragma unroll
-        for (int i = 0; i < DP / 32; i++) {
-          oacc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(vt[krow * C::kStrideB + i * 32], pv[r], oacc[i], 0, 0, 0);
-        }
-      }
+      contract_rows<DP / 32, C::kStrideB, true>(Vs[cur] + (4 * h32) * C::kStrideB + l32, pv, oacc);
     }
     if (more) {
-      if (!C::kPrefetch) fetch(kv0 + C::kTile);
+      if (!DMA && !C::kPrefetch) fetch(kv0 + C::kTile, cur ^ 1);
       stash(cur ^ 1);
     }
     __syncthreads();
@@ -267,13 +349,11 @@ __global__ __launch_bounds__(256) void attn_f32_delta_kernel(AttnF32Params p) {
 
 // --------------------------------------------------------------------------
 // backward (A): dK, dV.  Workgroup owns 128 key rows, streams query tiles.
-// WHAT: bit 0 = produce dV, bit 1 = produce dK.
+// Head sizes up to 128 (attn_f32_bwd_dkdv_pair_kernel beyond).
 // --------------------------------------------------------------------------
-template <int DP, int WHAT>
+template <int DP>
 __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_kernel(AttnF32Params p) {
   using C = AttnF32Cfg<DP>;
-  constexpr bool kDV = (WHAT & 1) != 0, kDK = (WHAT & 2) != 0;
-  // dV needs the dO tile as an operand, dK needs it for dP: both
   __shared__ __attribute__((aligned(16))) float Qs[2][C::kTile * C::kStrideB];
   __shared__ __attribute__((aligned(16))) float Gs[2][C::kTile * C::kStrideB];  // dO
   __shared__ __attribute__((aligned(16))) float Ls[2][C::kTile], Ds[2][C::kTile];
@@ -290,19 +370,17 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_kernel(AttnF32Params p)
   float const *lsep = p.lse + ((int64_t)b * p.H + head) * p.Sq;
   float const *delp = p.delta + ((int64_t)b * p.H + head) * p.Sq;
 
-  float kf[DP / 2];
-  float vf[kDK ? DP / 2 : 1];
+  float kf[DP / 2], vf[DP / 2];
   load_owned_row<DP>(kp + (int64_t)min(kvrow, p.Skv - 1) * p.k_ss, p.Dq, h32, kf);
-  if constexpr (kDK) load_owned_row<DP>(vp + (int64_t)min(kvrow, p.Skv - 1) * p.v_ss, p.Dv, h32, vf);
-  f32x16 dk[kDK ? DP / 32 : 1], dv[kDV ? DP / 32 : 1];
+  load_owned_row<DP>(vp + (int64_t)min(kvrow, p.Skv - 1) * p.v_ss, p.Dv, h32, vf);
+  f32x16 dk[DP / 32], dv[DP / 32];
 #pragma unroll
-  for (int i = 0; i < (kDK ? DP / 32 : 1); i++)
+  for (int i = 0; i < DP / 32; i++)
 #pragma unroll
-    for (int r = 0; r < 16; r++) dk[i][r] = 0.0f;
-#pragma unroll
-  for (int i = 0; i < (kDV ? DP / 32 : 1); i++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) dv[i][r] = 0.0f;
+    for (int r = 0; r < 16; r++) {
+      dk[i][r] = 0.0f;
+      dv[i][r] = 0.0f;
+    }
 
   int const q_begin = p.causal ? (kv0 / C::kTile) * C::kTile : 0;
   int const ntiles = q_begin < p.Sq ? (p.Sq - q_begin + C::kTile - 1) / C::kTile : 0;
@@ -333,7 +411,7 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_kernel(AttnF32Params p)
   for (int it = 0; it < ntiles; it++) {
     int const qt0 = q_begin + it * C::kTile;
     bool const more = it + 1 < ntiles;
-    if (C::kPrefetch && more) gload(qt0 + C::kTile);
+    if (more) gload(qt0 + C::kTile);
     // a wave whose keys all lie after this query tile (causal) contributes nothing
     bool const active = !p.causal || kv0 + wave * 32 <= qt0 + C::kTile - 1;
     if (active) {
@@ -345,7 +423,7 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_kernel(AttnF32Params p)
         dp[r] = 0.0f;
       }
       contract_d<DP>(Qs[cur] + l32 * C::kStrideB + h32 * (DP / 2), kf, s);
-      if constexpr (kDK) contract_d<DP>(Gs[cur] + l32 * C::kStrideB + h32 * (DP / 2), vf, dp);
+      contract_d<DP>(Gs[cur] + l32 * C::kStrideB + h32 * (DP / 2), vf, dp);
       float pv[16], dsv[16];
 #pragma unroll
       for (int r = 0; r < 16; r++) {
@@ -359,24 +437,10 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_kernel(AttnF32Params p)
       }
       // dV += P^T dO, dK += dS^T Q: A = the accumulator (row = key), B = dO / Q rows of the
       // matching query, reduction over the tile's queries
-      float const *gt = Gs[cur] + (4 * h32) * C::kStrideB + l32;
-      float const *qt = Qs[cur] + (4 * h32) * C::kStrideB + l32;
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        int const qr = 8 * (r >> 2) + (r & 3);
-#pragma unroll
-        for (int i = 0; i < DP / 32; i++) {
-          if constexpr (kDV) {
-            dv[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(pv[r], gt[qr * C::kStrideB + i * 32], dv[i], 0, 0, 0);
-          }
-          if constexpr (kDK) {
-            dk[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(dsv[r], qt[qr * C::kStrideB + i * 32], dk[i], 0, 0, 0);
-          }
-        }
-      }
+      contract_rows<DP / 32, C::kStrideB, false>(Gs[cur] + (4 * h32) * C::kStrideB + l32, pv, dv);
+      contract_rows<DP / 32, C::kStrideB, false>(Qs[cur] + (4 * h32) * C::kStrideB + l32, dsv, dk);
     }
     if (more) {
-      if (!C::kPrefetch) gload(qt0 + C::kTile);
       lstore(cur ^ 1);
     }
     __syncthreads();
@@ -394,19 +458,16 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_kernel(AttnF32Params p)
     for (int r = 0; r < 16; r++) {
       int const grow = kv0 + wave * 32 + 8 * (r >> 2) + 4 * h32 + (r & 3);
       if (grow < p.Skv) {
-        if constexpr (kDK) {
-          if (d < p.Dq) dkp[(int64_t)grow * p.k_ss + d] = dk[i][r];
-        }
-        if constexpr (kDV) {
-          if (d < p.Dv) dvp[(int64_t)grow * p.v_ss + d] = dv[i][r];
-        }
+        if (d < p.Dq) dkp[(int64_t)grow * p.k_ss + d] = dk[i][r];
+        if (d < p.Dv) dvp[(int64_t)grow * p.v_ss + d] = dv[i][r];
       }
     }
   }
 }
 
 // --------------------------------------------------------------------------
-// backward (B): dQ.  Workgroup owns 128 query rows, streams key tiles.
+// backward (B): dQ.  Workgroup owns 128 query rows, streams key tiles.  Head
+// sizes up to 128 (attn_f32_bwd_dq_pair_kernel beyond).
 // --------------------------------------------------------------------------
 template <int DP>
 __global__ __launch_bounds__(256) void attn_f32_bwd_dq_kernel(AttnF32Params p) {
@@ -458,7 +519,7 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dq_kernel(AttnF32Params p) {
   for (int it = 0; it < ntiles; it++) {
     int const kt0 = it * C::kTile;
     bool const more = it + 1 < ntiles;
-    if (C::kPrefetch && more) fetch(kt0 + C::kTile);
+    if (more) fetch(kt0 + C::kTile);
     bool const active = !p.causal || kt0 <= q0 + wave * 32 + 31;
     if (active) {
       // S^T = K Q^T, dP^T = V dO^T: rows = keys of the tile, column = this lane's query
@@ -479,18 +540,9 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dq_kernel(AttnF32Params p) {
         dsv[r] = masked ? 0.0f : e * __builtin_fmaf(dp[r], p.scale, -delta_s);
       }
       // dQ^T += K^T dS^T: A = K^T (row d), B = dS^T, reduction over the tile's keys
-      float const *kt = Ks[cur] + (4 * h32) * C::kStrideB + l32;
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        int const krow = 8 * (r >> 2) + (r & 3);
-#pragma unroll
-        for (int i = 0; i < DP / 32; i++) {
-          dq[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(kt[krow * C::kStrideB + i * 32], dsv[r], dq[i], 0, 0, 0);
-        }
-      }
+      contract_rows<DP / 32, C::kStrideB, true>(Ks[cur] + (4 * h32) * C::kStrideB + l32, dsv, dq);
     }
     if (more) {
-      if (!C::kPrefetch) fetch(kt0 + C::kTile);
       stash(cur ^ 1);
     }
     __syncthreads();
@@ -513,13 +565,312 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dq_kernel(AttnF32Params p) {
   }
 }
 
+// --------------------------------------------------------------------------
+// Head sizes beyond 128: two waves share 32 owned rows, so that what a wave
+// holds (one owned operand, at most one whole accumulator) stays in registers
+// with room to spare, and exchange score tiles through LDS.  A workgroup owns
+// 64 rows; wave w works on rows 32 * (w % 2) in role w / 2.  Bound by the fp32
+// matrix pipe.  With a wave on its own, dK and dV took two launches (the scores
+// computed in both) and dQ spilled: batch 8 x 8 heads x 512 at
+// head size 256, dK and dV 498 -> 345 us, dQ 309 -> 273.
+// --------------------------------------------------------------------------
+struct PairTile {
+  f32x4 v[4][64];  // elements 4g .. 4g+3 of each lane's accumulator
+};
+__device__ __forceinline__ void pair_put(PairTile &x, int lane, float const (&e)[16]) {
+#pragma unroll
+  for (int g = 0; g < 4; g++) x.v[g][lane] = f32x4{e[4 * g], e[4 * g + 1], e[4 * g + 2], e[4 * g + 3]};
+}
+__device__ __forceinline__ void pair_get(PairTile const &x, int lane, float (&e)[16]) {
+#pragma unroll
+  for (int g = 0; g < 4; g++) {
+    f32x4 const v = x.v[g][lane];
+#pragma unroll
+    for (int i = 0; i < 4; i++) e[4 * g + i] = v[i];
+  }
+}
+// the waves' LDS writes before it are visible after it; direct loads in flight stay in flight
+__device__ __forceinline__ void pair_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Streams two operands' 32-row tiles into two buffers each: direct loads one tile ahead (DMA), or
+// loads and LDS writes between barriers.
+template <bool DMA, int STRIDE0, int STRIDE1>
+struct PairStream {
+  float const *base[2];
+  int64_t ss[2];
+  int D[2];
+  int last, t, lane, wave;
+  i32x4 rsrc[2];
+  unsigned lane_off[2];
+  __device__ __forceinline__ void init() {
+    if constexpr (DMA) {
+#pragma unroll
+      for (int o = 0; o < 2; o++) {
+        rsrc[o] = buffer_resource(base[o], kRowsBound);
+        lane_off[o] = row_lane_offset(lane, D[o]);
+      }
+    }
+  }
+  __device__ __forceinline__ void load(int row0, float *t0, float *t1) const {
+    if constexpr (DMA) {
+      tile_dma<STRIDE0>(rsrc[0], lane_off[0], ss[0], row0, last, wave, t0);
+      tile_dma<STRIDE1>(rsrc[1], lane_off[1], ss[1], row0, last, wave, t1);
+    } else {
+      f32x4 r[AttnF32Cfg<256>::kChunks];
+      tile_gload<256>(base[0], ss[0], row0, last, D[0], t, r);
+      tile_lstore<256, STRIDE0>(t0, t, r);
+      tile_gload<256>(base[1], ss[1], row0, last, D[1], t, r);
+      tile_lstore<256, STRIDE1>(t1, t, r);
+    }
+  }
+};
+
+// dK and dV: role 0 computes S and P, hands P over and produces dV; role 1 computes dP and from
+// it and P dS, and produces dK.
+template <bool DMA>
+__global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Params p) {
+  constexpr int DP = 256;
+  using C = AttnF32Cfg<DP>;
+  __shared__ __attribute__((aligned(16))) float Qs[2][C::kTile * C::kStrideB];
+  __shared__ __attribute__((aligned(16))) float Gs[2][C::kTile * C::kStrideB];  // dO
+  __shared__ PairTile Ps[2];
+  __shared__ __attribute__((aligned(16))) float Ls[2][C::kTile], Ds[2][C::kTile];
+  int const t = threadIdx.x, lane = t & 63, h32 = lane >> 5, l32 = lane & 31;
+  int const wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  int const blk = wave & 1, role = wave >> 1;
+  int const hb = blockIdx.x % (p.H * p.B);
+  int const head = hb % p.H, b = hb / p.H;
+  int const kv0 = (blockIdx.x / (p.H * p.B)) * 64 + blk * 32;  // this wave's first key
+  int const kvg = (blockIdx.x / (p.H * p.B)) * 64;             // the workgroup's
+  int const kvrow = kv0 + l32;
+  float const *lsep = p.lse + ((int64_t)b * p.H + head) * p.Sq;
+  float const *delp = p.delta + ((int64_t)b * p.H + head) * p.Sq;
+
+  float own[DP / 2];  // role 0: the row of K, role 1: of V
+  {
+    int const r = min(kvrow, p.Skv - 1);
+    if (role == 0) load_owned_row<DP>(p.k + (int64_t)b * p.k_bs + (int64_t)head * p.Dq + (int64_t)r * p.k_ss, p.Dq, h32, own);
+    else load_owned_row<DP>(p.v + (int64_t)b * p.v_bs + (int64_t)head * p.Dv + (int64_t)r * p.v_ss, p.Dv, h32, own);
+  }
+  f32x16 acc[DP / 32];  // role 0: dV, role 1: dK
+#pragma unroll
+  for (int i = 0; i < DP / 32; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[i][r] = 0.0f;
+
+  int const q_begin = p.causal ? (kvg / C::kTile) * C::kTile : 0;
+  int const ntiles = q_begin < p.Sq ? (p.Sq - q_begin + C::kTile - 1) / C::kTile : 0;
+  PairStream<DMA, C::kStrideB, C::kStrideB> st;
+  st.base[0] = p.q + (int64_t)b * p.q_bs + (int64_t)head * p.Dq;
+  st.base[1] = p.d_o + (int64_t)b * p.o_bs + (int64_t)head * p.Dv;
+  st.ss[0] = p.q_ss; st.ss[1] = p.o_ss;
+  st.D[0] = p.Dq; st.D[1] = p.Dv;
+  st.last = p.Sq - 1; st.t = t; st.lane = lane; st.wave = wave;
+  st.init();
+  float rl = 0.0f, rd = 0.0f;
+  auto load_row_terms = [&](int qt0) {
+    int const gr = min(qt0 + (t & (C::kTile - 1)), p.Sq - 1);
+    rl = lsep[gr];
+    rd = delp[gr];
+  };
+  auto store_row_terms = [&](int buf) {
+    if (t < C::kTile) {
+      Ls[buf][t] = rl * kLog2eF;
+      Ds[buf][t] = rd * p.scale;
+    }
+  };
+  if (ntiles > 0) {
+    load_row_terms(q_begin);
+    st.load(q_begin, Qs[0], Gs[0]);
+    store_row_terms(0);
+  }
+  if constexpr (DMA) {
+    wait_vmcnt<0>();
+    wait_all_vmem_known_to_compiler();
+  }
+  __syncthreads();
+  int cur = 0;
+  for (int it = 0; it < ntiles; it++) {
+    int const qt0 = q_begin + it * C::kTile;
+    bool const more = it + 1 < ntiles;
+    if (more) {
+      load_row_terms(qt0 + C::kTile);
+      if (DMA) st.load(qt0 + C::kTile, Qs[cur ^ 1], Gs[cur ^ 1]);
+    }
+    // waves whose keys all lie after this query tile (causal) contribute nothing
+    bool const active = !p.causal || kv0 <= qt0 + C::kTile - 1;
+    float ex[16];  // role 0: P, role 1: dS
+    f32x16 s;
+    if (active) {
+      // S = Q K^T or dP = dO V^T: rows = queries of the tile, column = this lane's key
+#pragma unroll
+      for (int r = 0; r < 16; r++) s[r] = 0.0f;
+      contract_d<DP>((role == 0 ? Qs[cur] : Gs[cur]) + l32 * C::kStrideB + h32 * (DP / 2), own, s);
+      if (role == 0) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          int const ql = 8 * (r >> 2) + 4 * h32 + (r & 3);
+          int const qg = qt0 + ql;
+          float const e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], p.scale_log2, -Ls[cur][ql]));
+          bool const masked = qg >= p.Sq || kvrow >= p.Skv || (p.causal && kvrow > qg);
+          ex[r] = masked ? 0.0f : e;
+        }
+        pair_put(Ps[blk], lane, ex);
+      }
+    }
+    pair_barrier();
+    if (active) {
+      if (role == 1) {
+        pair_get(Ps[blk], lane, ex);
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          int const ql = 8 * (r >> 2) + 4 * h32 + (r & 3);
+          int const qg = qt0 + ql;
+          bool const masked = qg >= p.Sq || kvrow >= p.Skv || (p.causal && kvrow > qg);
+          // dS = P (dP - delta) scale; Ds holds delta * scale
+          float const ds = ex[r] * __builtin_fmaf(s[r], p.scale, -Ds[cur][ql]);
+          ex[r] = masked ? 0.0f : ds;
+        }
+      }
+      // dV += P^T dO or dK += dS^T Q: A = the accumulator (row = key), B = rows of the
+      // matching query, reduction over the tile's queries
+      contract_rows<DP / 32, C::kStrideB, false>((role == 0 ? Gs[cur] : Qs[cur]) + (4 * h32) * C::kStrideB + l32, ex, acc);
+    }
+    if (more) {
+      if (DMA) wait_vmcnt<0>();
+      else st.load(qt0 + C::kTile, Qs[cur ^ 1], Gs[cur ^ 1]);
+      store_row_terms(cur ^ 1);
+    }
+    __syncthreads();
+    cur ^= 1;
+  }
+
+  // accumulator element r: key row 8*(r/4) + 4*h + r%4 of this wave's 32, column d = i*32 + l%32
+  float *op = role == 0 ? p.dv + (int64_t)b * p.v_bs + (int64_t)head * p.Dv : p.dk + (int64_t)b * p.k_bs + (int64_t)head * p.Dq;
+  int64_t const oss = role == 0 ? p.v_ss : p.k_ss;
+  int const D = role == 0 ? p.Dv : p.Dq;
+#pragma unroll
+  for (int i = 0; i < DP / 32; i++) {
+    int const d = i * 32 + l32;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      int const grow = kv0 + 8 * (r >> 2) + 4 * h32 + (r & 3);
+      if (grow < p.Skv && d < D) op[(int64_t)grow * oss + d] = acc[i][r];
+    }
+  }
+}
+
+// dQ: role 0 computes S and P, role 1 dP; each hands the other its tile, both form dS, and each
+// produces half of dQ's columns.
+template <bool DMA>
+__global__ __launch_bounds__(256) void attn_f32_bwd_dq_pair_kernel(AttnF32Params p) {
+  constexpr int DP = 256;
+  using C = AttnF32Cfg<DP>;
+  __shared__ __attribute__((aligned(16))) float Ks[2][C::kTile * C::kStrideB];
+  __shared__ __attribute__((aligned(16))) float Vs[2][C::kTile * C::kStrideA];
+  __shared__ PairTile Xs[2][2];
+  int const t = threadIdx.x, lane = t & 63, h32 = lane >> 5, l32 = lane & 31;
+  int const wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  int const blk = wave & 1, role = wave >> 1;
+  int const nqb = (p.Sq + 63) / 64;
+  int const hb = blockIdx.x % (p.H * p.B);
+  int const qb = nqb - 1 - blockIdx.x / (p.H * p.B);
+  int const head = hb % p.H, b = hb / p.H;
+  int const q0 = qb * 64 + blk * 32;  // this wave's first query
+  int const qrow = q0 + l32;
+  int const rq = min(qrow, p.Sq - 1);
+  float own[DP / 2];  // role 0: the row of Q, role 1: of dO
+  if (role == 0) load_owned_row<DP>(p.q + (int64_t)b * p.q_bs + (int64_t)head * p.Dq + (int64_t)rq * p.q_ss, p.Dq, h32, own);
+  else load_owned_row<DP>(p.d_o + (int64_t)b * p.o_bs + (int64_t)head * p.Dv + (int64_t)rq * p.o_ss, p.Dv, h32, own);
+  float const lse2 = p.lse[((int64_t)b * p.H + head) * p.Sq + rq] * kLog2eF;
+  float const delta_s = p.delta[((int64_t)b * p.H + head) * p.Sq + rq] * p.scale;
+  f32x16 dq[DP / 64];
+#pragma unroll
+  for (int i = 0; i < DP / 64; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) dq[i][r] = 0.0f;
+
+  int kv_end = p.Skv;
+  if (p.causal) kv_end = min(p.Skv, qb * 64 + 64);
+  int const ntiles = (kv_end + C::kTile - 1) / C::kTile;
+  PairStream<DMA, C::kStrideB, C::kStrideA> st;
+  st.base[0] = p.k + (int64_t)b * p.k_bs + (int64_t)head * p.Dq;
+  st.base[1] = p.v + (int64_t)b * p.v_bs + (int64_t)head * p.Dv;
+  st.ss[0] = p.k_ss; st.ss[1] = p.v_ss;
+  st.D[0] = p.Dq; st.D[1] = p.Dv;
+  st.last = p.Skv - 1; st.t = t; st.lane = lane; st.wave = wave;
+  st.init();
+  st.load(0, Ks[0], Vs[0]);
+  if constexpr (DMA) {
+    wait_vmcnt<0>();
+    wait_all_vmem_known_to_compiler();
+  }
+  __syncthreads();
+  int cur = 0;
+  for (int it = 0; it < ntiles; it++) {
+    int const kt0 = it * C::kTile;
+    bool const more = it + 1 < ntiles;
+    if (DMA && more) st.load(kt0 + C::kTile, Ks[cur ^ 1], Vs[cur ^ 1]);
+    bool const active = !p.causal || kt0 <= q0 + 31;
+    float ex[16];  // role 0: P, role 1: (dP - delta) scale
+    if (active) {
+      // S^T = K Q^T or dP^T = V dO^T: rows = keys of the tile, column = this lane's query
+      f32x16 s;
+#pragma unroll
+      for (int r = 0; r < 16; r++) s[r] = 0.0f;
+      contract_d<DP>(role == 0 ? Ks[cur] + l32 * C::kStrideB + h32 * (DP / 2) : Vs[cur] + l32 * C::kStrideA + h32 * (DP / 2),
+                     own, s);
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        int const kv = kt0 + 8 * (r >> 2) + 4 * h32 + (r & 3);
+        bool const masked = kv >= p.Skv || (p.causal && kv > qrow);
+        // both sides of a masked product are 0
+        ex[r] = masked ? 0.0f
+                       : (role == 0 ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], p.scale_log2, -lse2))
+                                    : __builtin_fmaf(s[r], p.scale, -delta_s));
+      }
+      pair_put(Xs[blk][role], lane, ex);
+    }
+    pair_barrier();
+    if (active) {
+      float other[16];
+      pair_get(Xs[blk][role ^ 1], lane, other);
+#pragma unroll
+      for (int r = 0; r < 16; r++) ex[r] *= other[r];
+      // dQ^T += K^T dS^T: A = K^T (row d), B = dS^T, reduction over the tile's keys
+      contract_rows<DP / 64, C::kStrideB, true>(Ks[cur] + (4 * h32) * C::kStrideB + role * (DP / 2) + l32, ex, dq);
+    }
+    if (more) {
+      if (DMA) wait_vmcnt<0>();
+      else st.load(kt0 + C::kTile, Ks[cur ^ 1], Vs[cur ^ 1]);
+    }
+    __syncthreads();
+    cur ^= 1;
+  }
+
+  if (qrow < p.Sq) {
+    float *dqp = p.dq + (int64_t)b * p.q_bs + (int64_t)qrow * p.q_ss + (int64_t)head * p.Dq;
+#pragma unroll
+    for (int i = 0; i < DP / 64; i++) {
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        int const d = role * (DP / 2) + i * 32 + 8 * g + 4 * h32;
+        if (d < p.Dq) {
+          f32x4 w = {dq[i][4 * g], dq[i][4 * g + 1], dq[i][4 * g + 2], dq[i][4 * g + 3]};
+          *reinterpret_cast<f32x4 *>(dqp + d) = w;
+        }
+      }
+    }
+  }
+}
+
 static int check_desc_f32(char const *who, ffk_attention_desc_t const *d) {
   int64_t const dq = d->head_dim, dv = d->v_head_dim > 0 ? d->v_head_dim : d->head_dim;
   FFK_REQUIRE(dq > 0 && dq <= 256 && dq % 4 == 0 && dv <= 256 && dv % 4 == 0,
               "%s: fp32 head_dim %lld / v_head_dim %lld not supported (multiples of 4 up to 256)", who,
               (long long)dq, (long long)dv);
   FFK_REQUIRE(d->batch > 0 && d->heads > 0 && d->seq_q > 0 && d->seq_kv > 0, "%s: bad shape", who);
-  FFK_REQUIRE(d->batch * d->heads * ((d->seq_q > d->seq_kv ? d->seq_q : d->seq_kv) / 128 + 1) < (1ll << 31),
+  FFK_REQUIRE(d->batch * d->heads * ((d->seq_q > d->seq_kv ? d->seq_q : d->seq_kv) / 64 + 1) < (1ll << 32),
               "%s: too many workgroups", who);
   FFK_REQUIRE(d->seq_q < (1ll << 30) && d->seq_kv < (1ll << 30), "%s: sequence too long", who);
   FFK_REQUIRE(d->q_seq_stride % 4 == 0 && d->k_seq_stride % 4 == 0 && d->v_seq_stride % 4 == 0 &&
@@ -547,12 +898,19 @@ static AttnF32Params make_params(ffk_attention_desc_t const *d) {
   return p;
 }
 
+// Rows of every operand within 31 bits of their (batch, head)'s first element: direct loads reach them.
+static bool rows_fit_dma(AttnF32Params const &p) {
+  auto fits = [](int64_t rows, int64_t stride) { return stride < (1 << 28) && rows * stride * 4 < (int64_t)kRowsBound; };
+  return fits(p.Sq, p.q_ss) && fits(p.Skv, p.k_ss) && fits(p.Skv, p.v_ss) && fits(p.Sq, p.o_ss);
+}
+
 #define FFK_ATTN_F32_DISPATCH(D_, CALL)                                        \
   do {                                                                         \
-    if ((D_) <= 32) { CALL(32); }                                              \
-    else if ((D_) <= 64) { CALL(64); }                                         \
-    else if ((D_) <= 128) { CALL(128); }                                       \
-    else { CALL(256); }                                                        \
+    if ((D_) <= 32) { CALL(32, false); }                                       \
+    else if ((D_) <= 64) { CALL(64, false); }                                  \
+    else if ((D_) <= 128) { CALL(128, false); }                                \
+    else if (rows_fit_dma(p)) { CALL(256, true); }                             \
+    else { CALL(256, false); }                                                 \
   } while (0)
 
 int attention_f32_forward(hipStream_t st, ffk_attention_desc_t const *d, void const *q, void const *k,
@@ -567,23 +925,26 @@ int attention_f32_forward(hipStream_t st, ffk_attention_desc_t const *d, void co
   p.lse = lse;
   unsigned const grid = (unsigned)(ceil_div(p.Sq, 128) * p.H * p.B);
   int const dmax = p.Dq > p.Dv ? p.Dq : p.Dv;
-#define CALL(DP_) attn_f32_fwd_kernel<DP_><<<grid, 256, 0, st>>>(p)
+#define CALL(DP_, DMA_) attn_f32_fwd_kernel<DP_, DMA_><<<grid, 256, 0, st>>>(p)
   FFK_ATTN_F32_DISPATCH(dmax, CALL);
 #undef CALL
   FFK_CHECK_LAUNCH();
   return FFK_OK;
 }
 
-template <int DP>
-static void launch_f32_backward(hipStream_t st, AttnF32Params const &p, int64_t rows, unsigned gkv, unsigned gq) {
+template <int DP, bool DMA>
+static void launch_f32_backward(hipStream_t st, AttnF32Params const &p, int64_t rows) {
   attn_f32_delta_kernel<DP><<<(unsigned)ceil_div(rows, 4 * (64 / (DP / 4))), 256, 0, st>>>(p);
+  int64_t const own = DP <= 128 ? 128 : 64;
+  unsigned const gkv = (unsigned)(ceil_div(p.Skv, own) * p.H * p.B);
+  unsigned const gq = (unsigned)(ceil_div(p.Sq, own) * p.H * p.B);
   if constexpr (DP <= 128) {
-    attn_f32_bwd_dkdv_kernel<DP, 3><<<gkv, 256, 0, st>>>(p);
+    attn_f32_bwd_dkdv_kernel<DP><<<gkv, 256, 0, st>>>(p);
+    attn_f32_bwd_dq_kernel<DP><<<gq, 256, 0, st>>>(p);
   } else {
-    attn_f32_bwd_dkdv_kernel<DP, 1><<<gkv, 256, 0, st>>>(p);
-    attn_f32_bwd_dkdv_kernel<DP, 2><<<gkv, 256, 0, st>>>(p);
+    attn_f32_bwd_dkdv_pair_kernel<DMA><<<gkv, 256, 0, st>>>(p);
+    attn_f32_bwd_dq_pair_kernel<DMA><<<gq, 256, 0, st>>>(p);
   }
-  attn_f32_bwd_dq_kernel<DP><<<gq, 256, 0, st>>>(p);
 }
 
 int attention_f32_backward(hipStream_t st, ffk_attention_desc_t const *d, void const *q, void const *k,
@@ -603,10 +964,8 @@ int attention_f32_backward(hipStream_t st, ffk_attention_desc_t const *d, void c
   p.dk = static_cast<float *>(dk);
   p.dv = static_cast<float *>(dv);
   int64_t const rows = (int64_t)p.B * p.H * p.Sq;
-  unsigned const gkv = (unsigned)(ceil_div(p.Skv, 128) * p.H * p.B);
-  unsigned const gq = (unsigned)(ceil_div(p.Sq, 128) * p.H * p.B);
   int const dmax = p.Dq > p.Dv ? p.Dq : p.Dv;
-#define CALL(DP_) launch_f32_backward<DP_>(st, p, rows, gkv, gq)
+#define CALL(DP_, DMA_) launch_f32_backward<DP_, DMA_>(st, p, rows)
   FFK_ATTN_F32_DISPATCH(dmax, CALL);
 #undef CALL
   FFK_CHECK_LAUNCH();
