@@ -349,7 +349,7 @@ __global__ __launch_bounds__(256) void attn_f32_delta_kernel(AttnF32Params p) {
 
 // --------------------------------------------------------------------------
 // backward (A): dK, dV.  Workgroup owns 128 key rows, streams query tiles.
-// Head sizes up to 128 (attn_f32_bwd_dkdv_pair_kernel beyond).
+// Where the pair kernels are not taken (launch_f32_backward).
 // --------------------------------------------------------------------------
 template <int DP>
 __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_kernel(AttnF32Params p) {
@@ -466,8 +466,8 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_kernel(AttnF32Params p)
 }
 
 // --------------------------------------------------------------------------
-// backward (B): dQ.  Workgroup owns 128 query rows, streams key tiles.  Head
-// sizes up to 128 (attn_f32_bwd_dq_pair_kernel beyond).
+// backward (B): dQ.  Workgroup owns 128 query rows, streams key tiles.
+// Where the pair kernels are not taken (launch_f32_backward).
 // --------------------------------------------------------------------------
 template <int DP>
 __global__ __launch_bounds__(256) void attn_f32_bwd_dq_kernel(AttnF32Params p) {
@@ -566,7 +566,8 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dq_kernel(AttnF32Params p) {
 }
 
 // --------------------------------------------------------------------------
-// Head sizes beyond 128: two waves share 32 owned rows, so that what a wave
+// Two waves share 32 owned rows (head sizes beyond 128, and where
+// launch_f32_backward says so), so that what a wave
 // holds (one owned operand, at most one whole accumulator) stays in registers
 // with room to spare, and exchange score tiles through LDS.  A workgroup owns
 // 64 rows; wave w works on rows 32 * (w % 2) in role w / 2.  Bound by the fp32
@@ -592,9 +593,9 @@ __device__ __forceinline__ void pair_get(PairTile const &x, int lane, float (&e)
 // the waves' LDS writes before it are visible after it; direct loads in flight stay in flight
 __device__ __forceinline__ void pair_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// Streams two operands' 32-row tiles into two buffers each: direct loads one tile ahead (DMA), or
-// loads and LDS writes between barriers.
-template <bool DMA, int STRIDE0, int STRIDE1>
+// Streams two operands' 32-row tiles into two buffers each, one tile ahead: by direct loads (DMA), or
+// through registers.
+template <int DP, bool DMA, int STRIDE0, int STRIDE1>
 struct PairStream {
   float const *base[2];
   int64_t ss[2];
@@ -602,6 +603,7 @@ struct PairStream {
   int last, t, lane, wave;
   i32x4 rsrc[2];
   unsigned lane_off[2];
+  f32x4 r0[DMA ? 1 : AttnF32Cfg<DP>::kChunks], r1[DMA ? 1 : AttnF32Cfg<DP>::kChunks];
   __device__ __forceinline__ void init() {
     if constexpr (DMA) {
 #pragma unroll
@@ -611,25 +613,29 @@ struct PairStream {
       }
     }
   }
-  __device__ __forceinline__ void load(int row0, float *t0, float *t1) const {
+  __device__ __forceinline__ void fetch(int row0, float *t0, float *t1) {
     if constexpr (DMA) {
       tile_dma<STRIDE0>(rsrc[0], lane_off[0], ss[0], row0, last, wave, t0);
       tile_dma<STRIDE1>(rsrc[1], lane_off[1], ss[1], row0, last, wave, t1);
     } else {
-      f32x4 r[AttnF32Cfg<256>::kChunks];
-      tile_gload<256>(base[0], ss[0], row0, last, D[0], t, r);
-      tile_lstore<256, STRIDE0>(t0, t, r);
-      tile_gload<256>(base[1], ss[1], row0, last, D[1], t, r);
-      tile_lstore<256, STRIDE1>(t1, t, r);
+      tile_gload<DP>(base[0], ss[0], row0, last, D[0], t, r0);
+      tile_gload<DP>(base[1], ss[1], row0, last, D[1], t, r1);
+    }
+  }
+  __device__ __forceinline__ void land(float *t0, float *t1) const {
+    if constexpr (DMA) {
+      wait_vmcnt<0>();
+    } else {
+      tile_lstore<DP, STRIDE0>(t0, t, r0);
+      tile_lstore<DP, STRIDE1>(t1, t, r1);
     }
   }
 };
 
 // dK and dV: role 0 computes S and P, hands P over and produces dV; role 1 computes dP and from
 // it and P dS, and produces dK.
-template <bool DMA>
+template <int DP, bool DMA>
 __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Params p) {
-  constexpr int DP = 256;
   using C = AttnF32Cfg<DP>;
   __shared__ __attribute__((aligned(16))) float Qs[2][C::kTile * C::kStrideB];
   __shared__ __attribute__((aligned(16))) float Gs[2][C::kTile * C::kStrideB];  // dO
@@ -660,7 +666,7 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Para
 
   int const q_begin = p.causal ? (kvg / C::kTile) * C::kTile : 0;
   int const ntiles = q_begin < p.Sq ? (p.Sq - q_begin + C::kTile - 1) / C::kTile : 0;
-  PairStream<DMA, C::kStrideB, C::kStrideB> st;
+  PairStream<DP, DMA, C::kStrideB, C::kStrideB> st;
   st.base[0] = p.q + (int64_t)b * p.q_bs + (int64_t)head * p.Dq;
   st.base[1] = p.d_o + (int64_t)b * p.o_bs + (int64_t)head * p.Dv;
   st.ss[0] = p.q_ss; st.ss[1] = p.o_ss;
@@ -681,13 +687,11 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Para
   };
   if (ntiles > 0) {
     load_row_terms(q_begin);
-    st.load(q_begin, Qs[0], Gs[0]);
+    st.fetch(q_begin, Qs[0], Gs[0]);
+    st.land(Qs[0], Gs[0]);
     store_row_terms(0);
   }
-  if constexpr (DMA) {
-    wait_vmcnt<0>();
-    wait_all_vmem_known_to_compiler();
-  }
+  if constexpr (DMA) wait_all_vmem_known_to_compiler();
   __syncthreads();
   int cur = 0;
   for (int it = 0; it < ntiles; it++) {
@@ -695,7 +699,7 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Para
     bool const more = it + 1 < ntiles;
     if (more) {
       load_row_terms(qt0 + C::kTile);
-      if (DMA) st.load(qt0 + C::kTile, Qs[cur ^ 1], Gs[cur ^ 1]);
+      st.fetch(qt0 + C::kTile, Qs[cur ^ 1], Gs[cur ^ 1]);
     }
     // waves whose keys all lie after this query tile (causal) contribute nothing
     bool const active = !p.causal || kv0 <= qt0 + C::kTile - 1;
@@ -737,8 +741,7 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Para
       contract_rows<DP / 32, C::kStrideB, false>((role == 0 ? Gs[cur] : Qs[cur]) + (4 * h32) * C::kStrideB + l32, ex, acc);
     }
     if (more) {
-      if (DMA) wait_vmcnt<0>();
-      else st.load(qt0 + C::kTile, Qs[cur ^ 1], Gs[cur ^ 1]);
+      st.land(Qs[cur ^ 1], Gs[cur ^ 1]);
       store_row_terms(cur ^ 1);
     }
     __syncthreads();
@@ -762,9 +765,8 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Para
 
 // dQ: role 0 computes S and P, role 1 dP; each hands the other its tile, both form dS, and each
 // produces half of dQ's columns.
-template <bool DMA>
+template <int DP, bool DMA>
 __global__ __launch_bounds__(256) void attn_f32_bwd_dq_pair_kernel(AttnF32Params p) {
-  constexpr int DP = 256;
   using C = AttnF32Cfg<DP>;
   __shared__ __attribute__((aligned(16))) float Ks[2][C::kTile * C::kStrideB];
   __shared__ __attribute__((aligned(16))) float Vs[2][C::kTile * C::kStrideA];
@@ -793,24 +795,22 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dq_pair_kernel(AttnF32Params
   int kv_end = p.Skv;
   if (p.causal) kv_end = min(p.Skv, qb * 64 + 64);
   int const ntiles = (kv_end + C::kTile - 1) / C::kTile;
-  PairStream<DMA, C::kStrideB, C::kStrideA> st;
+  PairStream<DP, DMA, C::kStrideB, C::kStrideA> st;
   st.base[0] = p.k + (int64_t)b * p.k_bs + (int64_t)head * p.Dq;
   st.base[1] = p.v + (int64_t)b * p.v_bs + (int64_t)head * p.Dv;
   st.ss[0] = p.k_ss; st.ss[1] = p.v_ss;
   st.D[0] = p.Dq; st.D[1] = p.Dv;
   st.last = p.Skv - 1; st.t = t; st.lane = lane; st.wave = wave;
   st.init();
-  st.load(0, Ks[0], Vs[0]);
-  if constexpr (DMA) {
-    wait_vmcnt<0>();
-    wait_all_vmem_known_to_compiler();
-  }
+  st.fetch(0, Ks[0], Vs[0]);
+  st.land(Ks[0], Vs[0]);
+  if constexpr (DMA) wait_all_vmem_known_to_compiler();
   __syncthreads();
   int cur = 0;
   for (int it = 0; it < ntiles; it++) {
     int const kt0 = it * C::kTile;
     bool const more = it + 1 < ntiles;
-    if (DMA && more) st.load(kt0 + C::kTile, Ks[cur ^ 1], Vs[cur ^ 1]);
+    if (more) st.fetch(kt0 + C::kTile, Ks[cur ^ 1], Vs[cur ^ 1]);
     bool const active = !p.causal || kt0 <= q0 + 31;
     float ex[16];  // role 0: P, role 1: (dP - delta) scale
     if (active) {
@@ -840,10 +840,7 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dq_pair_kernel(AttnF32Params
       // dQ^T += K^T dS^T: A = K^T (row d), B = dS^T, reduction over the tile's keys
       contract_rows<DP / 64, C::kStrideB, true>(Ks[cur] + (4 * h32) * C::kStrideB + role * (DP / 2) + l32, ex, dq);
     }
-    if (more) {
-      if (DMA) wait_vmcnt<0>();
-      else st.load(kt0 + C::kTile, Ks[cur ^ 1], Vs[cur ^ 1]);
-    }
+    if (more) st.land(Ks[cur ^ 1], Vs[cur ^ 1]);
     __syncthreads();
     cur ^= 1;
   }
@@ -935,15 +932,22 @@ int attention_f32_forward(hipStream_t st, ffk_attention_desc_t const *d, void co
 template <int DP, bool DMA>
 static void launch_f32_backward(hipStream_t st, AttnF32Params const &p, int64_t rows) {
   attn_f32_delta_kernel<DP><<<(unsigned)ceil_div(rows, 4 * (64 / (DP / 4))), 256, 0, st>>>(p);
-  int64_t const own = DP <= 128 ? 128 : 64;
-  unsigned const gkv = (unsigned)(ceil_div(p.Skv, own) * p.H * p.B);
-  unsigned const gq = (unsigned)(ceil_div(p.Sq, own) * p.H * p.B);
-  if constexpr (DP <= 128) {
-    attn_f32_bwd_dkdv_kernel<DP><<<gkv, 256, 0, st>>>(p);
-    attn_f32_bwd_dq_kernel<DP><<<gq, 256, 0, st>>>(p);
-  } else {
-    attn_f32_bwd_dkdv_pair_kernel<DMA><<<gkv, 256, 0, st>>>(p);
-    attn_f32_bwd_dq_pair_kernel<DMA><<<gq, 256, 0, st>>>(p);
+  int64_t const heads = (int64_t)p.H * p.B;
+  // Pairs always at 256 (see above) and at 64, where they leave registers for twice the waves (batch 6 x 32
+  // heads x 700, causal: dK/dV 358 -> 297 us, dQ 235 -> 212); at 128 while workgroups of 128 rows do not fill
+  // the chip (8 heads, 138 x 58, head size 80: dK/dV 56 -> 35 us; 2 x 32 heads x 469: 173 -> 196, so not there).
+  auto pairs = [&](int64_t rows_owned) {
+    return DP >= 64 && (DP != 128 || ceil_div(rows_owned, 128) * heads < kNumCU);
+  };
+  if constexpr (DP >= 64) {
+    if (pairs(p.Skv)) {
+      attn_f32_bwd_dkdv_pair_kernel<DP, DMA><<<(unsigned)(ceil_div(p.Skv, 64) * heads), 256, 0, st>>>(p);
+    }
+    if (pairs(p.Sq)) attn_f32_bwd_dq_pair_kernel<DP, DMA><<<(unsigned)(ceil_div(p.Sq, 64) * heads), 256, 0, st>>>(p);
+  }
+  if constexpr (DP == 32 || DP == 128) {
+    if (!pairs(p.Skv)) attn_f32_bwd_dkdv_kernel<DP><<<(unsigned)(ceil_div(p.Skv, 128) * heads), 256, 0, st>>>(p);
+    if (!pairs(p.Sq)) attn_f32_bwd_dq_kernel<DP><<<(unsigned)(ceil_div(p.Sq, 128) * heads), 256, 0, st>>>(p);
   }
 }
 

@@ -41,19 +41,25 @@ extern template hipError_t pick_bf16_group<true, false>(hipStream_t, GemmProblem
 // ---------------------------------------------------------------------------
 // Plain kernel for bf16 shapes the tiled kernel cannot take.
 // ---------------------------------------------------------------------------
+// LANES lanes an output share its reduction: a wave from 64 terms on (one thread walking 841 terms
+// took 95 us for 17 x 43 outputs, its loads one behind the other; a wave 5).
+template <int LANES>
 __global__ __launch_bounds__(256) void gemm_bf16_plain_kernel(
     bf16 const *__restrict__ A, bf16 const *__restrict__ B, bf16 *C, int M,
     int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int ta, int tb,
     bf16 const *__restrict__ bias, int act, int accumulate) {
-  int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (int64_t)M * N) return;
+  int64_t idx = ((int64_t)blockIdx.x * 256 + threadIdx.x) / LANES;
+  if (idx >= (int64_t)M * N) return;  // uniform over the LANES lanes
   int m = (int)(idx / N), n = (int)(idx % N);
   float acc = 0.0f;
-  for (int k = 0; k < K; k++) {
+  for (int k = threadIdx.x % LANES; k < K; k += LANES) {
     float a = VecIO<bf16>::load1(ta ? A + (int64_t)k * lda + m : A + (int64_t)m * lda + k);
     float b = VecIO<bf16>::load1(tb ? B + (int64_t)n * ldb + k : B + (int64_t)k * ldb + n);
     acc += a * b;
   }
+#pragma unroll
+  for (int off = LANES / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  if (threadIdx.x % LANES != 0) return;
   if (bias != nullptr) acc += VecIO<bf16>::load1(bias + n);
   acc = apply_activation(acc, act);
   bf16 *dst = C + (int64_t)m * ldc + n;
@@ -396,11 +402,12 @@ int gemm_dispatch(hipStream_t st, int dtype, bool ta, bool tb, int64_t M,
     bool vec_ok = ((ta ? M % 8 == 0 : K % 8 == 0) || (ep.a_padded && !tb)) && (tb ? K % 8 == 0 : N % 8 == 0) && (lda % 8 == 0) &&
                   (ldb % 8 == 0) && aligned16(A) && aligned16(B) && K > 0;
     // Operands that are not: the register-staged kernel, but for products of so few elements that
-    // one thread an output is over as soon.
+    // one thread, or one wave, an output is over as soon.
     if (!vec_ok && (K == 0 || M * N * K < (1 << 21))) {
-      int64_t total = M * N;
+      int64_t const total = M * N * (K >= 64 ? 64 : 1);
       if (describe_only("gemm_bf16_plain_kernel")) return FFK_OK;
-      gemm_bf16_plain_kernel<<<(unsigned)ceil_div(total, 256), 256, 0, st>>>(
+      auto kern = K >= 64 ? gemm_bf16_plain_kernel<64> : gemm_bf16_plain_kernel<1>;
+      kern<<<(unsigned)ceil_div(total, 256), 256, 0, st>>>(
           a, b, c, (int)M, (int)N, (int)K, lda, ldb, ldc, ta, tb,
           static_cast<bf16 const *>(ep.bias), ep.activation, ep.accumulate);
       e = hipGetLastError();

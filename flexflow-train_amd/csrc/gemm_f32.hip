@@ -347,14 +347,14 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiled_kernel(
   }
 }
 
-// A long reduction over few outputs: sixteen waves a 16 x 16 tile (small_f32.h), where block tiles
-// would leave most of the chip idle and walk the reduction alone ([25,1024] over 42 023: 1180 us with
-// sixteen workgroups of 64 x 64).
-template <bool TA, bool TB>
-__global__ __launch_bounds__(1024) void gemm_f32_deep_kernel(float const *__restrict__ A, float const *__restrict__ B, float *C,
+// Few outputs, or a long reduction over few: four or sixteen waves a tile of 16 x 16 or 32 x 32
+// (small_f32.h), where block tiles would leave most of the chip idle and walk the reduction alone
+// ([25,1024] over 42 023: 1180 us with sixteen workgroups of 64 x 64; 138 x 640 over 640, a short
+// sequence's projections: 20 us with thirty, 8-10 so).
+template <bool TA, bool TB, int T, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void gemm_f32_small_kernel(float const *__restrict__ A, float const *__restrict__ B, float *C,
                                                              int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
                                                              float const *__restrict__ bias, int act, int accumulate) {
-  constexpr int T = 16, WAVES = 16;
   __shared__ SmallShared<T, WAVES> sm;
   int const nbn = (N + T - 1) / T, tm = (int)blockIdx.x / nbn, tn = (int)blockIdx.x - tm * nbn;
   SmallOperand<!TA, FFK_ACT_NONE> const a = {A, nullptr, lda, 0};
@@ -378,13 +378,22 @@ static void launch_tiled(hipStream_t st, int M, int N, int K, float const *A, in
 template <bool TA, bool TB>
 static void pick_f32(hipStream_t st, int M, int N, int K, float const *A, int64_t lda, float const *B, int64_t ldb,
                      float *C, int64_t ldc, GemmEpilogue const &ep) {
+#define FFK_F32_SMALL(T_, WAVES_)                                                                                 \
+  do {                                                                                                           \
+    if (describe_only(WAVES_ == 16 ? "gemm_f32_deep_kernel<%s,%s>" : "gemm_f32_small_kernel<%s,%s>", tf(TA), tf(TB))) return; \
+    gemm_f32_small_kernel<TA, TB, T_, WAVES_><<<(int)(ceil_div(M, T_) * ceil_div(N, T_)), WAVES_ * 64, 0, st>>>( \
+        A, B, C, M, N, K, lda, ldb, ldc, static_cast<float const *>(ep.bias), ep.activation, ep.accumulate);     \
+    return;                                                                                                      \
+  } while (0)
   // (64 x 64 tiles of the same output would reach a quarter of the CUs at most)
-  if (K >= 2048 && ceil_div(M, 64) * ceil_div(N, 64) <= kNumCU / 4) {
-    if (describe_only("gemm_f32_deep_kernel<%s,%s>", tf(TA), tf(TB))) return;
-    gemm_f32_deep_kernel<TA, TB><<<(int)(ceil_div(M, 16) * ceil_div(N, 16)), 1024, 0, st>>>(
-        A, B, C, M, N, K, lda, ldb, ldc, static_cast<float const *>(ep.bias), ep.activation, ep.accumulate);
-    return;
+  if (K >= 2048 && ceil_div(M, 64) * ceil_div(N, 64) <= kNumCU / 4) FFK_F32_SMALL(16, 16);
+  // the areas up to which the small Linear's forward keeps these tiles
+  int64_t const area = (int64_t)M * N;
+  if (K >= 128 && K <= 1024 && M < (1 << 20) && N < (1 << 20) && area >= 128 * 128) {
+    if (area <= 16 * 16 * 1024) FFK_F32_SMALL(16, 4);
+    if (area <= 32 * 32 * 640) FFK_F32_SMALL(32, 4);
   }
+#undef FFK_F32_SMALL
   if ((int64_t)M * N < 128 * 128 || K < 4) {
     if (describe_only("gemm_f32_kernel<%s,%s>", tf(TA), tf(TB))) return;
     gemm_f32_kernel<TA, TB><<<(int)(ceil_div(M, 64) * ceil_div(N, 64)), 256, 0, st>>>(
