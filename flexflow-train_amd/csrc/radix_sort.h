@@ -13,9 +13,9 @@
 //              ranking the keys of a step among their peers with the same digit
 //              by ballots, so equal digits keep their input order (stable) and
 //              the result does not depend on timing (no atomics decide a place).
-// Up to 524 288 lookups a pass is ONE launch: the scan moves into the scatter
+// Up to 1 048 576 lookups a pass is one or two launches: the scan moves into the scatter
 // kernel (every workgroup adds up the counts of the tiles before its own and the
-// totals of the digits below, straight from a table of at most 128 KB), and the
+// totals of the digits below, straight from a table of at most 256 KB), and the
 // scatter counts the NEXT pass's digits of the keys it places, per destination
 // tile, with integer atomics (a count does not depend on the order of the
 // additions; the counts are gathered in LDS first, since under a skewed id
@@ -180,12 +180,13 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
 // places), not by bandwidth, hence sixteen waves with at most four steps each,
 // the ranking under the table's loads, and digits no wider than the passes need.
 // Sort of 65 536 token ids below 50 257: 23 -> 18 us (tiles of 2048 keys and four
-// waves before); 524 288 ids below a million: 63 -> 51 us (three launches a pass
+// waves before); 524 288 ids below a million: 63 -> 50 us (three launches a pass
 // before); 1000 ids: three launches and 20 us less for the whole gradient.
 // ---------------------------------------------------------------------------
 constexpr int kSortFusedThreads = 1024;
 constexpr int kSortFusedWaves = kSortFusedThreads / 64;
-constexpr int kSortFusedTiles = 128;
+constexpr int kSortAheadTiles = 128;  // up to these a scatter counts the next pass's digits
+constexpr int kSortFusedTiles = 256;
 constexpr int kSortFusedItems = 4;  // the most keys per thread
 
 // A step's lanes with this lane's digit (all of them take part; `valid` lanes only are counted).
@@ -267,7 +268,7 @@ __global__ __launch_bounds__(kSortFusedThreads) void radix_hist_fused_kernel(IT 
 // table: this pass's counts; next: the next pass's table (nullptr on the last pass), added
 // into here; after: the table of the pass after that (nullptr if none), cleared here.
 // Dynamic LDS: the workgroup's share of the next table, 16-bit counters in pairs (a workgroup
-// counts its own keys there, at most 4096).
+// counts its own keys there, at most 4096; only up to kSortAheadTiles tiles).
 template <typename IT, bool FIRST, int ITEMS>
 __global__ __launch_bounds__(kSortFusedThreads) void radix_scatter_fused_kernel(
     IT const *__restrict__ idx, uint32_t const *__restrict__ keys_in, uint32_t const *__restrict__ vals_in,
@@ -278,7 +279,8 @@ __global__ __launch_bounds__(kSortFusedThreads) void radix_scatter_fused_kernel(
   extern __shared__ uint32_t next_cnt[];
   __shared__ uint32_t wave_off[kSortFusedWaves][kSortRadix];
   __shared__ uint32_t part_all[kSortFusedThreads], part_before[kSortFusedThreads];
-  __shared__ uint32_t wsum[kSortRadix / 64];
+  __shared__ uint32_t wsum[kSortRadix / 64], delta[ITEMS > 1 ? kSortRadix : 1];
+  __shared__ uint32_t ks[ITEMS > 1 ? TILE : 1], vs[ITEMS > 1 ? TILE : 1];
   int const t = threadIdx.x, lane = t & 63, wave = t >> 6;
   int const bins = 1 << bits, mask = bins - 1;
   int const next_words = next != nullptr ? (ntiles * bins + 1) / 2 : 0;
@@ -302,12 +304,12 @@ __global__ __launch_bounds__(kSortFusedThreads) void radix_scatter_fused_kernel(
   {
     int const d = t & mask, part = t >> bits, parts = kSortFusedThreads >> bits, tile = blockIdx.x;
     uint32_t before_tiles = 0, all_tiles = 0;
-    for (int t0 = part; t0 < ntiles; t0 += 8 * parts) {
-      uint32_t v[8];
+    for (int t0 = part; t0 < ntiles; t0 += 16 * parts) {
+      uint32_t v[16];
 #pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = t0 + u * parts < ntiles ? table[(int64_t)(t0 + u * parts) * bins + d] : 0u;
+      for (int u = 0; u < 16; u++) v[u] = t0 + u * parts < ntiles ? table[(int64_t)(t0 + u * parts) * bins + d] : 0u;
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
+      for (int u = 0; u < 16; u++) {
         all_tiles += v[u];
         before_tiles += t0 + u * parts < tile ? v[u] : 0u;
       }
@@ -328,26 +330,70 @@ __global__ __launch_bounds__(kSortFusedThreads) void radix_scatter_fused_kernel(
     }
   }
   uint32_t const smaller = sort_scan_bins(all, t, lane, wsum);
-  if (t < bins) {
-    uint32_t run = smaller + before;
+  if constexpr (ITEMS == 1) {
+    if (t < bins) {
+      uint32_t run = smaller + before;
 #pragma unroll
-    for (int w = 0; w < kSortFusedWaves; w++) {
-      uint32_t const c = wave_off[w][t];
-      wave_off[w][t] = run;
-      run += c;
+      for (int w = 0; w < kSortFusedWaves; w++) {
+        uint32_t const c = wave_off[w][t];
+        wave_off[w][t] = run;
+        run += c;
+      }
     }
-  }
-  __syncthreads();
+    __syncthreads();
 #pragma unroll
-  for (int c = 0; c < ITEMS; c++) {
-    if (valid[c]) {
-      uint32_t const pos = wave_off[wave][digit[c]] + rank[c];
-      keys_out[pos] = key[c];
-      vals_out[pos] = val[c];
-      // the next pass's count of this key, in the tile it has just been placed in
-      if (next != nullptr) {
-        uint32_t const nd = (pos / TILE) * bins + ((key[c] >> (shift + bits)) & mask);
-        atomicAdd(&next_cnt[nd >> 1], 1u << (16 * (nd & 1u)));
+    for (int c = 0; c < ITEMS; c++) {
+      if (valid[c]) {
+        uint32_t const pos = wave_off[wave][digit[c]] + rank[c];
+        keys_out[pos] = key[c];
+        vals_out[pos] = val[c];
+        // the next pass's count of this key, in the tile it has just been placed in
+        if (next != nullptr) {
+          uint32_t const nd = (pos / TILE) * bins + ((key[c] >> (shift + bits)) & mask);
+          atomicAdd(&next_cnt[nd >> 1], 1u << (16 * (nd & 1u)));
+        }
+      }
+    }
+  } else {
+    __syncthreads();
+    // The pairs are put in order in LDS first and leave from there: a wave's stores then go to a few
+    // runs of consecutive places instead of 64 lines (524 288 ids: 14 -> 12 us a pass; with one key a thread
+    // the two more barriers cost more, 5.7 -> 7.3 us for 65 536).
+    uint32_t mine = 0;
+    if (t < bins) {
+#pragma unroll
+      for (int w = 0; w < kSortFusedWaves; w++) mine += wave_off[w][t];
+    }
+    uint32_t const local = sort_scan_bins(mine, t, lane, wsum);
+    if (t < bins) {
+      delta[t] = smaller + before - local;  // from a pair's place in LDS to its place in the output
+      uint32_t run = local;
+#pragma unroll
+      for (int w = 0; w < kSortFusedWaves; w++) {
+        uint32_t const c = wave_off[w][t];
+        wave_off[w][t] = run;
+        run += c;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < ITEMS; c++) {
+      if (valid[c]) {
+        uint32_t const at = wave_off[wave][digit[c]] + rank[c];
+        ks[at] = key[c];
+        vs[at] = val[c];
+      }
+    }
+    __syncthreads();
+    int const here = (int)min((int64_t)TILE, n - (int64_t)blockIdx.x * TILE);
+#pragma unroll
+    for (int c = 0; c < ITEMS; c++) {
+      int const at = c * kSortFusedThreads + t;
+      if (at < here) {
+        uint32_t const k = ks[at];
+        uint32_t const pos = (uint32_t)at + delta[(k >> shift) & mask];
+        keys_out[pos] = k;
+        vals_out[pos] = vs[at];
       }
     }
   }
@@ -443,8 +489,8 @@ static inline RadixSortPlan radix_sort_plan(int64_t n, unsigned key_bits) {
   RadixSortPlan p;
   p.passes = (int)((key_bits + 7) / 8);
   p.bits = 8;
-  // Fused while the tables a workgroup reads and counts into stay small (128 tiles: 64 KB of LDS).
-  // More keys than that take the three launches a pass, whose cost per key is lower.
+  // Fused while a CU each holds every tile: the table a workgroup reads grows with their number.  More
+  // keys than that take the three launches a pass.
   p.fused = n <= (int64_t)kSortFusedTiles * kSortFusedThreads * kSortFusedItems;
   p.items = 0;
   if (p.fused) {
@@ -452,8 +498,7 @@ static inline RadixSortPlan radix_sort_plan(int64_t n, unsigned key_bits) {
     // one tile as long as four keys per thread cover everything; then as few keys per thread as the tile limit allows
     p.items = n <= kSortFusedThreads ? 1 : kSortFusedItems;
     if (n > (int64_t)kSortFusedThreads * kSortFusedItems) {
-      p.items = 1;
-      while (n > (int64_t)kSortFusedTiles * kSortFusedThreads * p.items) p.items *= 2;
+      p.items = n <= (int64_t)kSortAheadTiles * kSortFusedThreads ? 1 : n <= (int64_t)kSortFusedTiles * kSortFusedThreads * 2 ? 2 : 4;
     }
     p.ntiles = (int)ceil_div(n, (int64_t)kSortFusedThreads * p.items);
     p.table_bytes = ((size_t)p.ntiles << p.bits) * (size_t)p.passes * sizeof(uint32_t);
@@ -473,7 +518,7 @@ static inline hipError_t radix_sort_fused(hipStream_t st, IT const *idx, int64_t
   unsigned const blocks = (unsigned)plan.ntiles;
   // Counting the next pass's digits while placing costs an atomic for nearly every (tile, digit)
   // pair of every workgroup: cheaper than a launch up to one key per thread, several times
-  // dearer beyond (524 288 keys: 13-21 us a pass against 5 for the launch and 12 without the counting).
+  // dearer beyond (524 288 keys: 15-21 us a pass against 5 for the launch and 12 without the counting).
   constexpr bool kCountAhead = ITEMS == 1;
   auto tab = [&](int pass) -> uint32_t * { return pass < plan.passes ? table + (size_t)pass * tsz : nullptr; };
   auto ahead = [&](int pass) -> uint32_t * { return kCountAhead ? tab(pass) : nullptr; };

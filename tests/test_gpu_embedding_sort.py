@@ -1,6 +1,6 @@
 """Sorted scatter-add of the embedding gradient at the sizes where its sort changes form: one
-workgroup (up to 4096 lookups), one launch per pass with 1, 2 or 4 keys per thread (up to 524 288),
-three launches per pass beyond.  Gradients are small whole numbers, so every sum is exact in fp32 in
+workgroup (up to 4096 lookups), 1, 2 or 4 keys per thread (up to 131 072, 524 288, 1 048 576), three
+launches per pass beyond.  Gradients are small whole numbers, so every sum is exact in fp32 in
 any order and the results are compared bit for bit with a float64 sum on the CPU."""
 import pytest
 import torch
@@ -32,9 +32,11 @@ def _case(ffk, n, bag, vocab, dim, index_dtype, grad_dtype, deterministic, skew,
     (1365, 3, 70000, 320),    # 4095 lookups: one short of the workgroup; three passes
     (4097, 1, 70000, 64),     # two launches' worth: a last tile of one key
     (26215, 5, 1000, 64),     # 131 075: two keys per thread
-    (131073, 2, 30000, 16),   # 262 146: four keys per thread
-    (16384, 32, 50000, 128),  # 524 288: every tile of the fused form full
-    (524289, 1, 300, 16),     # beyond it
+    (131072, 1, 60000, 16),   # one key per thread, every tile full
+    (131073, 2, 30000, 16),   # 262 146
+    (16384, 32, 50000, 128),  # 524 288: two keys per thread, every tile full
+    (524289, 1, 300, 16),     # four keys per thread
+    (1048577, 1, 300, 16),    # beyond it
 ])
 @pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])
 def test_sizes_where_the_sort_changes_form(ffk, n, bag, vocab, dim, index_dtype):
