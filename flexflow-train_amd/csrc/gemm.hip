@@ -403,7 +403,10 @@ int gemm_dispatch(hipStream_t st, int dtype, bool ta, bool tb, int64_t M,
                   (ldb % 8 == 0) && aligned16(A) && aligned16(B) && K > 0;
     // Operands that are not: the register-staged kernel, but for products of so few elements that
     // one thread, or one wave, an output is over as soon.
-    if (!vec_ok && (K == 0 || M * N * K < (1 << 21))) {
+    // (A reduction of thousands over a few 64 x 64 tiles would be walked by as many workgroups: 52 x 37 over
+    // 1907 51 us so, 13 with a wave an output.)
+    bool const few = K >= 512 && M * N <= 4 * 64 * 64 && M * N * K < (1 << 23);
+    if (!vec_ok && (K == 0 || M * N * K < (1 << 21) || (few && ep.tail == GemmEpilogue::kTailNone))) {
       int64_t const total = M * N * (K >= 64 ? 64 : 1);
       if (describe_only("gemm_bf16_plain_kernel")) return FFK_OK;
       auto kern = K >= 64 ? gemm_bf16_plain_kernel<64> : gemm_bf16_plain_kernel<1>;

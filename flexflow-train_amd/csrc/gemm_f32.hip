@@ -1,4 +1,5 @@
 // fp32 GEMM kernels for gfx950 (v_mfma_f32_32x32x2f32), behind gemm_dispatch.
+#include <algorithm>
 #include "gemm_bf16.h"
 #include "small_f32.h"
 
@@ -351,20 +352,47 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiled_kernel(
 // (small_f32.h), where block tiles would leave most of the chip idle and walk the reduction alone
 // ([25,1024] over 42 023: 1180 us with sixteen workgroups of 64 x 64; 138 x 640 over 640, a short
 // sequence's projections: 20 us with thirty, 8-10 so).
+// partial != nullptr: workgroup row y takes the k's from y * k_per_split on and leaves its sums in
+// partial[y][M][N], which gemm_f32_splits_kernel adds up.
 template <bool TA, bool TB, int T, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void gemm_f32_small_kernel(float const *__restrict__ A, float const *__restrict__ B, float *C,
                                                              int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
-                                                             float const *__restrict__ bias, int act, int accumulate) {
+                                                             float const *__restrict__ bias, int act, int accumulate,
+                                                             float *partial, int k_per_split) {
   __shared__ SmallShared<T, WAVES> sm;
   int const nbn = (N + T - 1) / T, tm = (int)blockIdx.x / nbn, tn = (int)blockIdx.x - tm * nbn;
+  if (partial != nullptr) {
+    int const k0 = (int)blockIdx.y * k_per_split;
+    K = min(K - k0, k_per_split);
+    A += TA ? (int64_t)k0 * lda : k0;
+    B += TB ? k0 : (int64_t)k0 * ldb;
+    partial += (int64_t)blockIdx.y * M * N;
+  }
   SmallOperand<!TA, FFK_ACT_NONE> const a = {A, nullptr, lda, 0};
   SmallOperand<TB, FFK_ACT_NONE> const b = {B, nullptr, ldb, 0};
   auto store = [&](int m, int n, float v) {
+    if (partial != nullptr) {
+      partial[(int64_t)m * N + n] = v;
+      return;
+    }
     v = apply_activation(v + (bias != nullptr ? bias[n] : 0.0f), act);
     float *const to = C + (int64_t)m * ldc + n;
     *to = accumulate ? *to + v : v;
   };
   small_tile<T, WAVES, WAVES>(a, b, M, N, K, tm * T, tn * T, true, nullptr, 0, store, false, [](int, float) {}, sm);
+}
+
+__global__ __launch_bounds__(256) void gemm_f32_splits_kernel(float const *__restrict__ partial, float *C, int M, int N,
+                                                              int64_t ldc, float const *__restrict__ bias, int act,
+                                                              int accumulate, int splits) {
+  int64_t const at = (int64_t)blockIdx.x * 256 + threadIdx.x, total = (int64_t)M * N;
+  if (at >= total) return;
+  int const m = (int)(at / N), n = (int)(at - (int64_t)m * N);
+  float v = 0.0f;
+  for (int s = 0; s < splits; s++) v += partial[s * total + at];
+  v = apply_activation(v + (bias != nullptr ? bias[n] : 0.0f), act);
+  float *const to = C + (int64_t)m * ldc + n;
+  *to = accumulate ? *to + v : v;
 }
 
 template <bool TA, bool TB, int BM, int BN, bool ANY>
@@ -382,14 +410,32 @@ static void pick_f32(hipStream_t st, int M, int N, int K, float const *A, int64_
   do {                                                                                                           \
     if (describe_only(WAVES_ == 16 ? "gemm_f32_deep_kernel<%s,%s>" : "gemm_f32_small_kernel<%s,%s>", tf(TA), tf(TB))) return; \
     gemm_f32_small_kernel<TA, TB, T_, WAVES_><<<(int)(ceil_div(M, T_) * ceil_div(N, T_)), WAVES_ * 64, 0, st>>>( \
-        A, B, C, M, N, K, lda, ldb, ldc, static_cast<float const *>(ep.bias), ep.activation, ep.accumulate);     \
+        A, B, C, M, N, K, lda, ldb, ldc, static_cast<float const *>(ep.bias), ep.activation, ep.accumulate, nullptr, 0); \
     return;                                                                                                      \
   } while (0)
   // (64 x 64 tiles of the same output would reach a quarter of the CUs at most)
-  if (K >= 2048 && ceil_div(M, 64) * ceil_div(N, 64) <= kNumCU / 4) FFK_F32_SMALL(16, 16);
+  if (K >= 2048 && ceil_div(M, 64) * ceil_div(N, 64) <= kNumCU / 4) {
+    // Two workgroups a CU: with scratch at hand, reductions of thousands are split over workgroups until
+    // there are ([476, 58] over 40 305: 147 us with 120 workgroups,
+    // 102 with 600 and the 5 of adding up; [128, 45] over 21 856: 72 and 14 + 7).
+    int64_t const tiles = ceil_div(M, 16) * ceil_div(N, 16);
+    int64_t const most = std::min<int64_t>(K / 1024, (int64_t)(ep.splitk_ws_bytes / sizeof(float)) / ((int64_t)M * N));
+    int64_t const want = std::min<int64_t>(ceil_div(2 * kNumCU, tiles), most);
+    if (ep.splitk_ws != nullptr && want > 1) {
+      if (describe_only("gemm_f32_deep_kernel<%s,%s> (split-K)", tf(TA), tf(TB))) return;
+      int const per = (int)(ceil_div(ceil_div(K, want), 64) * 64), splits = (int)ceil_div(K, per);
+      float *const partial = static_cast<float *>(ep.splitk_ws);
+      gemm_f32_small_kernel<TA, TB, 16, 16><<<dim3((unsigned)tiles, (unsigned)splits), 1024, 0, st>>>(
+          A, B, C, M, N, K, lda, ldb, ldc, nullptr, FFK_ACT_NONE, 0, partial, per);
+      gemm_f32_splits_kernel<<<(unsigned)ceil_div((int64_t)M * N, 256), 256, 0, st>>>(
+          partial, C, M, N, ldc, static_cast<float const *>(ep.bias), ep.activation, ep.accumulate, splits);
+      return;
+    }
+    FFK_F32_SMALL(16, 16);
+  }
   // the areas up to which the small Linear's forward keeps these tiles
   int64_t const area = (int64_t)M * N;
-  if (K >= 128 && K <= 1024 && M < (1 << 20) && N < (1 << 20) && area >= 128 * 128) {
+  if (K >= 256 && K <= 1024 && M < (1 << 20) && N < (1 << 20) && area >= 128 * 128) {
     if (area <= 16 * 16 * 1024) FFK_F32_SMALL(16, 4);
     if (area <= 32 * 32 * 640) FFK_F32_SMALL(32, 4);
   }

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
-@pytest.mark.parametrize("mnk", [(138, 640, 640), (129, 130, 128), (1023, 255, 1024), (17, 15000, 131), (799, 801, 1021)])
+@pytest.mark.parametrize("mnk", [(138, 640, 640), (129, 130, 256), (1023, 255, 1024), (17, 15000, 259), (799, 801, 1021)])
 def test_gemm_fp32_small_tiles(ffk, ta, tb, mnk):
     M, N, K = mnk
     print("gemm fp32 small", mnk, ta, tb, flush=True)
@@ -28,7 +28,7 @@ def test_gemm_fp32_small_tiles(ffk, ta, tb, mnk):
 
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
-@pytest.mark.parametrize("mnk", [(17, 43, 841), (1, 1, 64), (51, 131, 251), (43, 841, 17), (9, 7, 63), (3, 5, 20001)])
+@pytest.mark.parametrize("mnk", [(17, 43, 841), (1, 1, 64), (51, 131, 251), (43, 841, 17), (9, 7, 63), (3, 5, 20001), (52, 37, 1907), (129, 127, 513)])
 def test_gemm_bf16_few_outputs(ffk, ta, tb, mnk):
     M, N, K = mnk
     print("gemm bf16 few outputs", mnk, ta, tb, flush=True)
@@ -40,6 +40,18 @@ def test_gemm_bf16_few_outputs(ffk, ta, tb, mnk):
     ffk.gemm(A.cuda(), B.cuda(), C, ta, tb)
     # one rounding to bf16 of an fp32 sum: half a unit in the last of 8 bits
     assert_close(to_np(C.float()), want, 2.0 ** -8, "C")
+
+
+@pytest.mark.parametrize("shape", [(37, 61, 9001), (5, 17, 4097), (128, 45, 20001), (300, 40, 2048)])
+def test_linear_fp32_backward_split_reduction(ffk, shape):
+    """The input gradient's reduction over thousands of outputs, split in the weight gradient's memory."""
+    B, I, O = shape
+    gen = torch.Generator().manual_seed(B + I + O)
+    x, w, dy, y = (torch.randn(s, generator=gen) for s in ((B, I), (O, I), (B, O), (B, O)))
+    dx, dw, db = (torch.full(s, 3.0, device="cuda") for s in ((B, I), (O, I), (O,)))
+    ffk.linear_backward(y.cuda(), dy.cuda(), x.cuda(), w.cuda(), dx, dw, db, activation=ffk.ACT_NONE)
+    for t, want, name in ((dx, dy.double() @ w.double(), "dx"), (dw, dy.double().t() @ x.double(), "dw"), (db, dy.double().sum(0), "db")):
+        assert_close(to_np(t), to_np(want), 1e-5, name)
 
 
 @pytest.mark.parametrize("shape", [(1, 2, 1, 9, 64), (1, 3, 65, 33, 128), (2, 8, 138, 58, 80), (16, 16, 70, 70, 64),
