@@ -1,4 +1,4 @@
-"""Products and attention whose kernels are chosen for few elements: fp32 products on register-fed tiles,
+"""Products, attention and updates whose kernels are chosen for few elements: fp32 products on register-fed tiles,
 bf16 products of unaligned rows with a wave to an output, and the fp32 attention backward on both sides of the
 size where two waves stop sharing their rows.  References are float64 on the CPU."""
 import pytest
@@ -80,3 +80,19 @@ def test_attention_fp32_backward_both_forms(ffk, shape, causal):
     got = ffk.attention_backward(qd, kd, vd, o, dod, lse, scale, causal)
     for t, w, name in zip(got, want, ("dQ", "dK", "dV")):
         assert_close(to_np(t), to_np(w.transpose(1, 2).contiguous()), 1e-5, name)
+
+
+@pytest.mark.parametrize("n", [8388609, 8389631])
+def test_adam_past_the_caches(ffk, oracle, n):
+    """Parameters from where the update bypasses the caches on, with a last workgroup of few."""
+    gen = torch.Generator().manual_seed(n)
+    w0, grad, m0 = (torch.randn(n, generator=gen) for _ in range(3))
+    v0 = torch.rand(n, generator=gen)
+    args = dict(alpha_t=1e-2, beta1=0.9, beta2=0.99, weight_decay=0.05, epsilon=1e-6)
+    want = oracle.adam_update(w0.numpy().copy(), grad.numpy().copy(), m0.numpy().copy(), v0.numpy().copy(), **args)
+    w, m, v = w0.cuda(), m0.cuda(), v0.cuda()
+    low = torch.empty(n, device="cuda", dtype=torch.bfloat16)
+    ffk.adam_update(w, grad.cuda(), m, v, weight_lowp=low, **args)
+    for got, ref in zip((w, m, v), want):
+        assert torch.equal(got.cpu(), torch.from_numpy(ref))
+    assert torch.equal(low, w.to(torch.bfloat16))
