@@ -643,7 +643,8 @@ static int emb_backward(hipStream_t st, void const *indices, void const *dy,
                         size_t workspace_bytes, bool deterministic) {
   int64_t const lookups = num_bags * bag;
   EmbSortLayout L;
-  bool const sorted = workspace != nullptr && dim % 4 == 0 && dim <= 65535 * 256 &&
+  bool const sorted = workspace != nullptr && dim % 4 == 0 &&
+                      (deterministic || dim <= 65535 * 256) &&  // the walk's grid takes 256 columns a row
                       reinterpret_cast<uintptr_t>(dy) % 16 == 0 &&
                       reinterpret_cast<uintptr_t>(dw) % 16 == 0 &&
                       reinterpret_cast<uintptr_t>(workspace) % 256 == 0 &&
