@@ -397,7 +397,7 @@ __global__ __launch_bounds__(256) void embedding_bwd_sorted_kernel(
 // 256 columns of longer rows): ids, row addresses and the run logic are then scalar work beside the loads.  With two
 // walkers to a wave (dim 128) every position took about a hundred vector instructions, and
 // they, not memory, were the bound (524 288 lookups in bags of 32, 1 M rows of 128
-// floats: 78 -> 58 us; 65 536 lookups of 1024 bf16 columns, which had a wave to a walker before: 62-64 both ways).
+// floats: 78 -> 56 us; 65 536 lookups of 1024 bf16 columns, which had a wave to a walker before: 64 -> 58).
 constexpr int kEmbBlockThreads = 1024;
 constexpr int kEmbWalkers = kEmbBlockThreads / 64;
 constexpr int kEmbMaxChunk = 64;  // one (row id, lookup) pair per lane
@@ -671,11 +671,12 @@ static int emb_backward(hipStream_t st, void const *indices, void const *dy,
       FFK_CHECK_LAUNCH();
       return FFK_OK;
     }
-    // Longer chunks mean fewer border partials and fewer atomics on hot rows; 16384 walkers are
-    // two for every wave the chip holds.
+    // Longer chunks mean fewer border partials and fewer atomics on hot rows; 8192 walkers are every
+    // wave the chip holds (sort and walk of 524 288 x 128: 96.8 us, 99 with 16384 walkers, 109 with 32768;
+    // of 65 536 x 1024 bf16: 77, 81.6, 81.5).
     int64_t const groups = ceil_div(dim, 256);
     int const chunk =
-        (int)std::min<int64_t>(kEmbMaxChunk, std::max<int64_t>(kEmbChunk, ceil_div(lookups * groups, 16384)));
+        (int)std::min<int64_t>(kEmbMaxChunk, std::max<int64_t>(kEmbChunk, ceil_div(lookups * groups, 8192)));
     dim3 const blocks((unsigned)ceil_div(lookups, (int64_t)kEmbWalkers * chunk), (unsigned)groups);
 #define FFK_EMB_SORTED(VPL_)                                                   \
   do {                                                                         \
