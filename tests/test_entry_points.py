@@ -47,3 +47,47 @@ with FakeTensorMode():
     refused("vmap", RuntimeError, lambda: torch.vmap(lambda t: %s)(x))
 """ % call)
     assert out.strip() == "refused vmap RuntimeError"
+
+
+def test_host_memory_where_the_device_reads():
+    """An array of the host or a bare address, where a kernel would read it, is no tensor of the device."""
+    out = run("""
+import ctypes
+import numpy as np
+ints = (ctypes.c_int * 4)()
+with FakeTensorMode():
+    x, w = torch.empty((4, 8), device="cuda"), torch.empty((16, 8), device="cuda")
+    y, host = torch.empty((4, 16), device="cuda"), torch.empty((16,))
+    for b in (np.zeros(16, np.float32), bytearray(64), b"\\0" * 64, 1 << 20, (ctypes.c_float * 16)(), ctypes.c_void_p(1 << 20)):
+        refused(type(b).__name__, TypeError, lambda: ffk.linear_forward(x, w, b, out=y))
+    refused("cpu", AssertionError, lambda: ffk.linear_forward(x, w, host, out=y))
+    refused("strided", AssertionError, lambda: ffk.linear_forward(x, w.t(), out=torch.empty((4, 8), device="cuda")))
+    for label in (np.zeros(4, np.int32), ints):
+        refused(type(label).__name__, TypeError,
+                lambda: ffk.sparse_categorical_crossentropy_loss_backward(y, label, 4, 16, 1, 1.0))
+""")
+    assert out.split().count("refused") == 10, out
+
+
+def test_descriptors_and_lists():
+    """A descriptor is the structure of its entry point and a list has elements of its type."""
+    out = run("""
+import ctypes
+mha = ffk.mha_desc(1, 1, 8, 8, 8, 8, 8, 8, 8, 4, 4)
+layer = ffk.EncoderLayerDesc(1, 4, 8, 1, 8)
+assert ffk._call.ffk_mha_reserve_bytes(mha, ffk.FLOAT) == ffk.lib().ffk_mha_reserve_bytes(ctypes.byref(mha), ffk.FLOAT)
+assert ffk._call.ffk_encoder_layer_workspace_bytes(layer, ffk.BF16) > 0
+for what in (layer, None, b"short", ctypes.pointer(mha)):
+    refused(type(what).__name__, TypeError, lambda: ffk._call.ffk_mha_reserve_bytes(what, ffk.FLOAT))
+refused("MHADesc", TypeError, lambda: ffk._call.ffk_encoder_layer_workspace_bytes(mha, ffk.BF16))
+refused("float", TypeError, lambda: ffk._call.ffk_mha_reserve_bytes(mha, 4.0))
+refused("count", TypeError, lambda: ffk._call.ffk_mha_reserve_bytes(mha))
+with FakeTensorMode():
+    x, y = torch.empty((4, 8), device="cuda"), torch.empty((8, 4), device="cuda")
+    sizes, perm = (ctypes.c_int64 * 2)(4, 8), (ctypes.c_int * 2)(1, 0)
+    refused("sizes", TypeError, lambda: ffk._call.ffk_transpose_forward(ffk.FLOAT, x, y, 2, perm, perm))
+    refused("perm", TypeError, lambda: ffk._call.ffk_transpose_forward(ffk.FLOAT, x, y, 2, sizes, sizes))
+    refused("tensor", TypeError, lambda: ffk._call.ffk_transpose_forward(ffk.FLOAT, x, y, 2, x, perm))
+    refused("pointers", TypeError, lambda: ffk._call.ffk_concat_forward(ffk.FLOAT, y, perm, sizes, 2, 1))
+""")
+    assert out.split().count("refused") == 11, out
