@@ -212,7 +212,10 @@ static int mha_backward_impl(ffk_stream_t stream, int dtype, ffk_mha_desc_t cons
   // The two weight gradients of a self-attention block (output projection and folded Q/K/V
   // projection) have the same reduction length and each leaves part of the chip idle: they run as
   // one launch after the core's backward (or later, with those of the layer around it).
+  // A query_grad in output_grad's memory is written in between, and then dW_O cannot wait.
   bool const folded = aliased && key_grad == nullptr && value_grad == nullptr;
+  uint8_t const *const dout = static_cast<uint8_t const *>(output_grad), *const dx = static_cast<uint8_t const *>(query_grad);
+  bool const in_place = dx != nullptr && dx < dout + L.TQ * d->o_proj_size * es && dout < dx + L.TQ * d->q_size * es;
   CollectWeightGrads collect(folded);
   if (dw != nullptr) {
     // d(QKV projections) is not written before the core's backward: until
@@ -220,8 +223,10 @@ static int mha_backward_impl(ffk_stream_t stream, int dtype, ffk_mha_desc_t cons
     GemmEpilogue acc_o = acc;
     acc_o.splitk_ws = dqkv;
     acc_o.splitk_ws_bytes = L.total - L.off_dqkv;
-    rc = weight_grad_dispatch(st, dtype, d->o_proj_size, HDv, L.TQ, output_grad,
-                              d->o_proj_size, ctx, HDv, dw + L.wo * es, HDv, acc_o);
+    auto const dispatch = [&](auto... args) {
+      return in_place ? gemm_dispatch(st, dtype, true, false, args...) : weight_grad_dispatch(st, dtype, args...);
+    };
+    rc = dispatch(d->o_proj_size, HDv, L.TQ, output_grad, d->o_proj_size, ctx, HDv, dw + L.wo * es, HDv, acc_o);
     if (rc != FFK_OK) return rc;
   }
 

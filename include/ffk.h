@@ -627,7 +627,8 @@ int ffk_attention_backward(ffk_stream_t stream, int dtype,
  *   weight_grad is accumulated into (CUDNN_WGRAD_MODE_ADD).  `accumulate` is
  *   0 / 1 as just described, optionally or-ed with
  *   FFK_MHA_OVERWRITE_WEIGHT_GRAD to store the weight gradient instead of
- *   adding it (a caller that would otherwise clear it first).                */
+ *   adding it (a caller that would otherwise clear it first).
+ *   query_grad may lie in output_grad's memory (output_grad is then gone).    */
 /* ------------------------------------------------------------------------ */
 typedef struct {
   int64_t num_samples, num_heads;

@@ -463,6 +463,29 @@ def test_mha_separate_grads_when_aliased(ffk, oracle):
     assert_close(to_np(dv), dv_ref, BF16_RTOL, "dv")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("shape", [(7, 197, 2, 64), (1, 16, 2, 64), (4, 64, 2, 64), (2, 512, 8, 64)])  # B, S, H, Dh
+def test_mha_input_gradient_in_place(ffk, dtype, shape):
+    """query_grad in output_grad's memory: the gradients of a call with two tensors."""
+    B, S, H, Dh = shape
+    E = H * Dh
+    say("mha input gradient in place", shape, dtype)
+    gen = torch.Generator().manual_seed(B * S)
+    desc = ffk.mha_desc(B, H, E, E, E, Dh, Dh, Dh, E, S, S, Dh ** -0.5, False)
+    x, dout = (torch.randn((B, S, E), generator=gen).to("cuda", dtype) for _ in range(2))
+    w = (torch.randn(4 * E * E, generator=gen) * 0.1).to("cuda", dtype)
+    reserve = ffk.mha_reserve(desc, ffk.dtype_of(x))
+    ffk.mha_forward(desc, x, x, x, w, reserve)
+    kept = reserve.clone()
+    dx, dw = torch.empty_like(x), torch.zeros_like(w)
+    ffk.mha_backward(desc, x, dx, x, None, x, None, w, dw, dout, reserve)
+    both, dw2 = dout.clone(), torch.zeros_like(w)
+    ffk.mha_backward(desc, x, both, x, None, x, None, w, dw2, both, kept)
+    assert torch.equal(dx, both)
+    # the weight gradients' sums of B * S products may be taken in another order: fp32, and one rounding
+    assert_close(to_np(dw2), to_np(dw), 2.0 ** -8 if dtype == BT else FP32_RTOL, "dW")
+
+
 def test_mha_errors(ffk):
     desc = ffk.mha_desc(1, 2, 64, 64, 64, 64, 64, 64, 64, 8, 8)
     x = torch.zeros((1, 8, 64), dtype=BT, device="cuda")
