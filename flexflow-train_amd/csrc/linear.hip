@@ -162,6 +162,20 @@ static int64_t linear_grad_ld(int dtype, int64_t out_dim) {
   return linear_pads_grad(dtype, out_dim) ? (out_dim + 63) / 64 * 64 : out_dim;
 }
 
+// Room for the partial sums of an input gradient whose reduction over out_dim is split over workgroups:
+// it lies at the end of the workspace, where it overlaps neither g nor column sums that wait there, and
+// it depends on nothing else the call asks for, so that the input gradient has the same bits whatever
+// becomes of the weights'.  in_dim is not known here; what the splits can use is bounded all the same.
+//  fp32: 16 x 16 tiles on two workgroups a CU at most, fewer than 1024 tiles of 1 KB (gemm_f32.hip).
+//  bf16: one round of 256 x 256 tiles in fp32, 64 MB ([2048, 50257] . [50257, 1024] takes all of it: 8
+//  splits, 210 us, 446 without), 16 splits of 2048 columns for few rows.  Shorter reductions, and rows
+//  fewer than a tile's, are not split (gemm_splits_for).
+static size_t linear_split_bytes(int dtype, int64_t batch, int64_t out_dim) {
+  if (dtype == FFK_FLOAT) return out_dim >= 2048 ? size_t(1) << 20 : 0;
+  if (dtype != FFK_BF16 || out_dim <= 63 * 64 || batch < 128) return 0;
+  return batch >= 512 ? size_t(64) << 20 : (size_t)batch << 17;
+}
+
 extern "C" size_t ffk_linear_backward_workspace_bytes(int dtype, int activation,
                                                       int use_bias,
                                                       int64_t batch,
@@ -173,7 +187,7 @@ extern "C" size_t ffk_linear_backward_workspace_bytes(int dtype, int activation,
   if (use_bias) {
     bytes += align256((size_t)colsum_partials_elems(batch, out_dim) * sizeof(float));
   }
-  return bytes;
+  return bytes + linear_split_bytes(dtype, batch, out_dim);
 }
 
 extern "C" int ffk_linear_forward(ffk_stream_t stream, int dtype,
@@ -273,7 +287,7 @@ static int linear_backward_impl(
   if (least > 0 && (workspace == nullptr || workspace_bytes < least)) {
     return fail(FFK_ERR_WORKSPACE, "linear_backward: workspace of %zu bytes needed, %zu given", least, workspace_bytes);
   }
-  // (a caller that knows the sizes without padding keeps working)
+  // (a caller that knows the sizes without padding and splits keeps working)
   if (pad && (workspace == nullptr || !aligned16(workspace) ||
               workspace_bytes < partial_bytes + grad_bytes(linear_grad_ld(dtype, out_dim)))) {
     pad = false;
@@ -293,11 +307,13 @@ static int linear_backward_impl(
   if (input_grad != nullptr) {
     GemmEpilogue dx = input_tail != nullptr ? *input_tail : ep;
     dx.accumulate = (accumulate & FFK_ACC_INPUT) != 0;
-    // what the weight gradient will overwrite serves as scratch until then: a reduction over a
-    // vocabulary is longer than its few output tiles keep the chip busy with
-    if (input_tail == nullptr && weight_grad != nullptr && (accumulate & FFK_ACC_WEIGHT) == 0) {
-      dx.splitk_ws = weight_grad;
-      dx.splitk_ws_bytes = (size_t)in_dim * (size_t)out_dim * dtype_size(dtype);
+    size_t const used = partial_bytes + (act || pad ? grad_bytes(ldg) : 0), split = linear_split_bytes(dtype, batch, out_dim);
+    if (input_tail == nullptr && split > 0 && aligned16(workspace) && workspace_bytes >= used + split) {
+      dx.splitk_ws = ws + ((workspace_bytes - split) & ~(size_t)255);
+      // ... of no more partial sums than there are weights: beyond that it depends (4000 x 20 over 2048 in fp32
+      // 20 us unsplit, 23 in two; in bf16 2048 x 696 over 24566 130 us in two, 142 in eight, but 2048 x 432 over
+      // 50895 230 us in four, 198 in sixteen)
+      dx.splitk_ws_bytes = std::min(split, (size_t)in_dim * (size_t)out_dim * dtype_size(dtype));
     }
     // input_grad[batch,in] = g[batch,out] . weight[out,in]
     if (input_tail != nullptr &&

@@ -173,8 +173,14 @@ int ffk_get_option(int which, int *value);
  *   linear_kernels.cu:262,311,334; 0 = the reference CPU path, which
  *   overwrites, linear_kernels_cpu.cc:80-93).
  *   workspace: device scratch of ffk_linear_backward_workspace_bytes(...)
- *   bytes (holds g when there is an activation, and the partial column sums
- *   of the bias gradient); may be NULL when that size is 0.                  */
+ *   bytes; may be NULL when that size is 0.  It holds, one behind the other,
+ *   g when there is an activation or when out_dim is no multiple of 8 in bf16
+ *   (then with rows padded to whole 16 bytes); the partial column sums of the
+ *   bias gradient; and at its end the partial sums of an input_grad whose
+ *   reduction over out_dim is split over workgroups.  An activation's g and the
+ *   column sums are needed (FFK_ERR_WORKSPACE); without the size of the query,
+ *   or 16-byte alignment, the padding and the splits are left out, which costs
+ *   time and gives the sums another order, so other last bits.                */
 /* ------------------------------------------------------------------------ */
 int ffk_linear_forward(ffk_stream_t stream, int dtype, int activation,
                        void const *input, void *output, void const *weight,

@@ -1,6 +1,6 @@
 """bf16 Linear backward where a gradient row is no whole number of 16 bytes: the pass that pads it, sums
 the bias gradient and applies the activation, the products that read the padded rows, the reduction
-split over workgroups in the weight gradient's memory, and a product whose last round goes as its own."""
+split over workgroups, and a product whose last round goes as its own."""
 import numpy as np
 import pytest
 import torch

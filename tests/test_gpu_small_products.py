@@ -44,7 +44,7 @@ def test_gemm_bf16_few_outputs(ffk, ta, tb, mnk):
 
 @pytest.mark.parametrize("shape", [(37, 61, 9001), (5, 17, 4097), (128, 45, 20001), (300, 40, 2048)])
 def test_linear_fp32_backward_split_reduction(ffk, shape):
-    """The input gradient's reduction over thousands of outputs, split in the weight gradient's memory."""
+    """The input gradient's reduction over thousands of outputs, split over workgroups."""
     B, I, O = shape
     gen = torch.Generator().manual_seed(B + I + O)
     x, w, dy, y = (torch.randn(s, generator=gen) for s in ((B, I), (O, I), (B, O), (B, O)))
