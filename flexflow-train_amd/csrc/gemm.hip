@@ -43,7 +43,7 @@ extern template hipError_t pick_bf16_group<true, false>(hipStream_t, GemmProblem
 // ---------------------------------------------------------------------------
 // LANES lanes an output share its reduction: a wave from 64 terms on (one thread walking 841 terms
 // took 95 us for 17 x 43 outputs, its loads one behind the other; a wave 5).
-template <int LANES>
+template <int LANES = 64>
 __global__ __launch_bounds__(256) void gemm_bf16_plain_kernel(
     bf16 const *__restrict__ A, bf16 const *__restrict__ B, bf16 *C, int M,
     int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int ta, int tb,
@@ -408,7 +408,7 @@ int gemm_dispatch(hipStream_t st, int dtype, bool ta, bool tb, int64_t M,
     bool const few = K >= 512 && M * N <= 4 * 64 * 64 && M * N * K < (1 << 23);
     if (!vec_ok && (K == 0 || M * N * K < (1 << 21) || (few && ep.tail == GemmEpilogue::kTailNone))) {
       int64_t const total = M * N * (K >= 64 ? 64 : 1);
-      if (describe_only("gemm_bf16_plain_kernel")) return FFK_OK;
+      if (describe_only(K >= 64 ? "gemm_bf16_plain_kernel" : "gemm_bf16_plain_kernel<1>")) return FFK_OK;
       auto kern = K >= 64 ? gemm_bf16_plain_kernel<64> : gemm_bf16_plain_kernel<1>;
       kern<<<(unsigned)ceil_div(total, 256), 256, 0, st>>>(
           a, b, c, (int)M, (int)N, (int)K, lda, ldb, ldc, ta, tb,

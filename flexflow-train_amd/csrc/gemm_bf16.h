@@ -6,6 +6,8 @@
 #include "gemm.h"
 #include <algorithm>
 #include <stdarg.h>
+#include <stdio.h>
+#include <string.h>
 #include <type_traits>
 
 namespace ffk {
@@ -54,17 +56,19 @@ __device__ __forceinline__ void tile_coords(int pid, int nbm, int nbn, int &tm,
 
 // ---------------------------------------------------------------------------
 // Asking instead of launching: while this thread's name sink is set (by
-// ffk_gemm_kernel_name), every launch site below writes the kernel it would
-// have launched into the sink and returns without touching the device.
+// ffk_gemm_kernel_name), every launch site below adds the kernel it would
+// have launched to the sink and returns without touching the device.
 // ---------------------------------------------------------------------------
 inline thread_local char *tl_name_sink = nullptr;
 inline thread_local size_t tl_name_sink_bytes = 0;
 inline bool describe_only(char const *fmt, ...) __attribute__((format(printf, 1, 2)));
 inline bool describe_only(char const *fmt, ...) {
   if (tl_name_sink == nullptr) return false;
+  size_t used = strlen(tl_name_sink);
+  if (used > 0 && used + 4 < tl_name_sink_bytes) used += strlen(strcpy(tl_name_sink + used, " + "));
   va_list ap;
   va_start(ap, fmt);
-  vsnprintf(tl_name_sink, tl_name_sink_bytes, fmt, ap);
+  vsnprintf(tl_name_sink + used, tl_name_sink_bytes - used, fmt, ap);
   va_end(ap);
   return true;
 }
@@ -1165,8 +1169,11 @@ static hipError_t launch_pipe(hipStream_t st, bf16 const *A, bf16 const *B,
   constexpr int NT = Cfg::NW * 64 * KG;
   constexpr size_t kLds = KG == 1 ? Cfg::kLds : KG * Cfg::kStageBytes;
   static_assert(kLds <= 160 * 1024, "LDS budget");
-  if (describe_only("gemm_bf16_pipe_kernel<%d,%d,%d,%d,%d,%d,%d,%s,%s,%d,false%s%s>%s", BM, BN, WM, WN, BK, STAGES, PF,
-                    tf(TA), tf(TB), TAIL, EDGE == kEdgeNone ? "" : EDGE == kEdgeOverlap ? ",overlap" : ",bounded", KG == 1 ? "" : ",2", splits > 1 ? " (split-K) + splitk_reduce_kernel" : "")) {
+  static_assert(KG <= 2, "the names below");
+  constexpr char const *edge = KG == 1 ? (EDGE == 0 ? "" : EDGE == 1 ? ",1" : ",2")  // unless they have their default
+                                       : (EDGE == 0 ? ",0,2" : EDGE == 1 ? ",1,2" : ",2,2");
+  if (describe_only("gemm_bf16_pipe_kernel<%d,%d,%d,%d,%d,%d,%d,%s,%s,%d,false%s>", BM, BN, WM, WN, BK, STAGES, PF, tf(TA),
+                    tf(TB), TAIL, edge)) {
     return hipSuccess;
   }
   auto kern = gemm_bf16_pipe_kernel<BM, BN, WM, WN, BK, STAGES, PF, TA, TB, TAIL, false, EDGE, KG>;

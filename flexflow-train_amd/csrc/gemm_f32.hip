@@ -348,19 +348,41 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiled_kernel(
   }
 }
 
-// Few outputs, or a long reduction over few: four or sixteen waves a tile of 16 x 16 or 32 x 32
-// (small_f32.h), where block tiles would leave most of the chip idle and walk the reduction alone
-// ([25,1024] over 42 023: 1180 us with sixteen workgroups of 64 x 64; 138 x 640 over 640, a short
-// sequence's projections: 20 us with thirty, 8-10 so).
+// Few outputs, or a long reduction over few: four waves a tile of 16 x 16 or 32 x 32, sixteen where the
+// reduction is long (small_f32.h), where block tiles would leave most of the chip idle and walk the
+// reduction alone ([25,1024] over 42 023: 1180 us with sixteen workgroups of 64 x 64; 138 x 640 over 640, a
+// short sequence's projections: 20 us with thirty, 8-10 so).
+template <bool TA, bool TB, int T, int WAVES, typename Store>
+__device__ __forceinline__ void f32_small_tile(float const *A, float const *B, int M, int N, int K, int64_t lda, int64_t ldb,
+                                               Store const &store) {
+  __shared__ SmallShared<T, WAVES> sm;
+  int const nbn = (N + T - 1) / T, tm = (int)blockIdx.x / nbn, tn = (int)blockIdx.x - tm * nbn;
+  SmallOperand<!TA, FFK_ACT_NONE> const a = {A, nullptr, lda, 0};
+  SmallOperand<TB, FFK_ACT_NONE> const b = {B, nullptr, ldb, 0};
+  small_tile<T, WAVES, WAVES>(a, b, M, N, K, tm * T, tn * T, true, nullptr, 0, store, false, [](int, float) {}, sm);
+}
+__device__ __forceinline__ void f32_epilogue(float *C, int64_t ldc, float const *bias, int act, int accumulate, int m, int n,
+                                             float v) {
+  v = apply_activation(v + (bias != nullptr ? bias[n] : 0.0f), act);
+  float *const to = C + (int64_t)m * ldc + n;
+  *to = accumulate ? *to + v : v;
+}
+
+template <bool TA, bool TB, int T>
+__global__ __launch_bounds__(256) void gemm_f32_small_kernel(float const *__restrict__ A, float const *__restrict__ B, float *C,
+                                                             int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
+                                                             float const *__restrict__ bias, int act, int accumulate) {
+  f32_small_tile<TA, TB, T, 4>(A, B, M, N, K, lda, ldb,
+                               [&](int m, int n, float v) { f32_epilogue(C, ldc, bias, act, accumulate, m, n, v); });
+}
+
 // partial != nullptr: workgroup row y takes the k's from y * k_per_split on and leaves its sums in
 // partial[y][M][N], which gemm_f32_splits_kernel adds up.
-template <bool TA, bool TB, int T, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void gemm_f32_small_kernel(float const *__restrict__ A, float const *__restrict__ B, float *C,
+template <bool TA, bool TB>
+__global__ __launch_bounds__(1024) void gemm_f32_deep_kernel(float const *__restrict__ A, float const *__restrict__ B, float *C,
                                                              int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
                                                              float const *__restrict__ bias, int act, int accumulate,
                                                              float *partial, int k_per_split) {
-  __shared__ SmallShared<T, WAVES> sm;
-  int const nbn = (N + T - 1) / T, tm = (int)blockIdx.x / nbn, tn = (int)blockIdx.x - tm * nbn;
   if (partial != nullptr) {
     int const k0 = (int)blockIdx.y * k_per_split;
     K = min(K - k0, k_per_split);
@@ -368,18 +390,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_small_kernel(float const 
     B += TB ? k0 : (int64_t)k0 * ldb;
     partial += (int64_t)blockIdx.y * M * N;
   }
-  SmallOperand<!TA, FFK_ACT_NONE> const a = {A, nullptr, lda, 0};
-  SmallOperand<TB, FFK_ACT_NONE> const b = {B, nullptr, ldb, 0};
-  auto store = [&](int m, int n, float v) {
+  f32_small_tile<TA, TB, 16, 16>(A, B, M, N, K, lda, ldb, [&](int m, int n, float v) {
     if (partial != nullptr) {
       partial[(int64_t)m * N + n] = v;
-      return;
+    } else {
+      f32_epilogue(C, ldc, bias, act, accumulate, m, n, v);
     }
-    v = apply_activation(v + (bias != nullptr ? bias[n] : 0.0f), act);
-    float *const to = C + (int64_t)m * ldc + n;
-    *to = accumulate ? *to + v : v;
-  };
-  small_tile<T, WAVES, WAVES>(a, b, M, N, K, tm * T, tn * T, true, nullptr, 0, store, false, [](int, float) {}, sm);
+  });
 }
 
 __global__ __launch_bounds__(256) void gemm_f32_splits_kernel(float const *__restrict__ partial, float *C, int M, int N,
@@ -390,9 +407,7 @@ __global__ __launch_bounds__(256) void gemm_f32_splits_kernel(float const *__res
   int const m = (int)(at / N), n = (int)(at - (int64_t)m * N);
   float v = 0.0f;
   for (int s = 0; s < splits; s++) v += partial[s * total + at];
-  v = apply_activation(v + (bias != nullptr ? bias[n] : 0.0f), act);
-  float *const to = C + (int64_t)m * ldc + n;
-  *to = accumulate ? *to + v : v;
+  f32_epilogue(C, ldc, bias, act, accumulate, m, n, v);
 }
 
 template <bool TA, bool TB, int BM, int BN, bool ANY>
@@ -406,13 +421,7 @@ static void launch_tiled(hipStream_t st, int M, int N, int K, float const *A, in
 template <bool TA, bool TB>
 static void pick_f32(hipStream_t st, int M, int N, int K, float const *A, int64_t lda, float const *B, int64_t ldb,
                      float *C, int64_t ldc, GemmEpilogue const &ep) {
-#define FFK_F32_SMALL(T_, WAVES_)                                                                                 \
-  do {                                                                                                           \
-    if (describe_only(WAVES_ == 16 ? "gemm_f32_deep_kernel<%s,%s>" : "gemm_f32_small_kernel<%s,%s>", tf(TA), tf(TB))) return; \
-    gemm_f32_small_kernel<TA, TB, T_, WAVES_><<<(int)(ceil_div(M, T_) * ceil_div(N, T_)), WAVES_ * 64, 0, st>>>( \
-        A, B, C, M, N, K, lda, ldb, ldc, static_cast<float const *>(ep.bias), ep.activation, ep.accumulate, nullptr, 0); \
-    return;                                                                                                      \
-  } while (0)
+  float const *const bias = static_cast<float const *>(ep.bias);
   // (64 x 64 tiles of the same output would reach a quarter of the CUs at most)
   if (K >= 2048 && ceil_div(M, 64) * ceil_div(N, 64) <= kNumCU / 4) {
     // Two workgroups a CU: with scratch at hand, reductions of thousands are split over workgroups until
@@ -421,25 +430,32 @@ static void pick_f32(hipStream_t st, int M, int N, int K, float const *A, int64_
     int64_t const tiles = ceil_div(M, 16) * ceil_div(N, 16);
     int64_t const most = std::min<int64_t>(K / 1024, (int64_t)(ep.splitk_ws_bytes / sizeof(float)) / ((int64_t)M * N));
     int64_t const want = std::min<int64_t>(ceil_div(2 * kNumCU, tiles), most);
+    if (describe_only("gemm_f32_deep_kernel<%s,%s>", tf(TA), tf(TB))) return;
     if (ep.splitk_ws != nullptr && want > 1) {
-      if (describe_only("gemm_f32_deep_kernel<%s,%s> (split-K)", tf(TA), tf(TB))) return;
       int const per = (int)(ceil_div(ceil_div(K, want), 64) * 64), splits = (int)ceil_div(K, per);
       float *const partial = static_cast<float *>(ep.splitk_ws);
-      gemm_f32_small_kernel<TA, TB, 16, 16><<<dim3((unsigned)tiles, (unsigned)splits), 1024, 0, st>>>(
+      gemm_f32_deep_kernel<TA, TB><<<dim3((unsigned)tiles, (unsigned)splits), 1024, 0, st>>>(
           A, B, C, M, N, K, lda, ldb, ldc, nullptr, FFK_ACT_NONE, 0, partial, per);
-      gemm_f32_splits_kernel<<<(unsigned)ceil_div((int64_t)M * N, 256), 256, 0, st>>>(
-          partial, C, M, N, ldc, static_cast<float const *>(ep.bias), ep.activation, ep.accumulate, splits);
+      gemm_f32_splits_kernel<<<(unsigned)ceil_div((int64_t)M * N, 256), 256, 0, st>>>(partial, C, M, N, ldc, bias, ep.activation,
+                                                                                     ep.accumulate, splits);
       return;
     }
-    FFK_F32_SMALL(16, 16);
+    gemm_f32_deep_kernel<TA, TB><<<(unsigned)tiles, 1024, 0, st>>>(A, B, C, M, N, K, lda, ldb, ldc, bias, ep.activation,
+                                                                   ep.accumulate, nullptr, 0);
+    return;
   }
   // the areas up to which the small Linear's forward keeps these tiles
   int64_t const area = (int64_t)M * N;
   if (K >= 256 && K <= 1024 && M < (1 << 20) && N < (1 << 20) && area >= 128 * 128) {
-    if (area <= 16 * 16 * 1024) FFK_F32_SMALL(16, 4);
-    if (area <= 32 * 32 * 640) FFK_F32_SMALL(32, 4);
+    int const t = area <= 16 * 16 * 1024 ? 16 : 32;
+    if (area <= 32 * 32 * 640) {
+      if (describe_only("gemm_f32_small_kernel<%s,%s,%d>", tf(TA), tf(TB), t)) return;
+      auto kern = t == 16 ? gemm_f32_small_kernel<TA, TB, 16> : gemm_f32_small_kernel<TA, TB, 32>;
+      kern<<<(unsigned)(ceil_div(M, t) * ceil_div(N, t)), 256, 0, st>>>(A, B, C, M, N, K, lda, ldb, ldc, bias, ep.activation,
+                                                                        ep.accumulate);
+      return;
+    }
   }
-#undef FFK_F32_SMALL
   if ((int64_t)M * N < 128 * 128 || K < 4) {
     if (describe_only("gemm_f32_kernel<%s,%s>", tf(TA), tf(TB))) return;
     gemm_f32_kernel<TA, TB><<<(int)(ceil_div(M, 64) * ceil_div(N, 64)), 256, 0, st>>>(

@@ -218,12 +218,17 @@ int ffk_gemm(ffk_stream_t stream, int dtype, int trans_a, int trans_b,
              int64_t M, int64_t N, int64_t K, void const *A, void const *B,
              void *C, int accumulate);
 
-/* Which kernel ffk_gemm / ffk_linear_forward would launch for a dense problem of
- * this data type, kind, shape and epilogue (bias, FFK_ACT_*), as the kernel's
- * template instance, e.g. "gemm_bf16_pipe_kernel<256,256,128,128,64,2,1,false,
- * true,0,false>".  Nothing is launched and no device is touched: the dispatch
- * runs with a name sink in place of the launch.  For reports that must name
- * the kernel they measured; no counterpart in the reference.                  */
+/* Which kernel ffk_gemm, or another operator's product of this data type, kind,
+ * shape and epilogue (bias, FFK_ACT_*), launches for dense operands, as the
+ * kernel's template instance, e.g. "gemm_bf16_pipe_kernel<256,256,128,128,64,2,
+ * 1,false,true,0,false>": arguments at the end that have their default are left
+ * out (here the kind of edge, 0, and the groups of waves, 1, which a profiler
+ * prints as well).  A product that runs in two launches gives both names,
+ * joined by " + ".  (ffk_linear_forward is such a product, but for fp32 layers so
+ * small that they have kernels of their own.)  Nothing is launched and no device
+ * is touched: the dispatch runs with a name sink in place of the launch.  For
+ * reports that must name the kernel they measured; no counterpart in the
+ * reference.                                                                  */
 int ffk_gemm_kernel_name(int dtype, int trans_a, int trans_b, int64_t M,
                          int64_t N, int64_t K, int has_bias, int activation,
                          char *name, size_t name_bytes);

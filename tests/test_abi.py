@@ -2,7 +2,9 @@
 (no compute calls: runs without a GPU)."""
 import ctypes
 import os
+import random
 import re
+import subprocess
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -52,3 +54,43 @@ def test_gemm_kernel_name_needs_no_device(ffk):
         assert ffk.gemm_kernel_name(ffk.BF16, False, True, 4096, 4096, 1024, True).startswith("gemm_bf16_pipe_kernel<128,128,")
     finally:
         ffk.set_option(ffk.OPTION_GEMM_VARIANT, 0)
+
+
+def _kernels(path):
+    """The kernels in the library: name -> the template argument lists it is instantiated with."""
+    symbols = subprocess.run(["nm", "-C", path], capture_output=True, text=True, check=True).stdout
+    found = {}
+    for name, args in re.findall(r" V (?:void )?ffk::(gemm_\w+_kernel)(?:<([^>]*)>)?\(", symbols):
+        found.setdefault(name, set()).add(tuple(args.replace(" ", "").split(",")))
+    # what the demangler does not know (_Float16's kin): its literals by hand
+    for name, args in re.findall(r" V _ZN3ffk\d+(gemm_\w+_kernel)I((?:L[bi]\d+E)+)E", symbols):
+        literals = re.findall(r"L([bi])(\d+)E", args)
+        found.setdefault(name, set()).add(tuple(v if t == "i" else ("false", "true")[int(v)] for t, v in literals))
+    return found
+
+
+def test_gemm_kernel_names_are_kernels_of_the_library(ffk):
+    """Every name is an instance in the library, arguments left out at the end having their default."""
+    have = _kernels(ffk.LIB_PATH)
+    defaults = {"gemm_bf16_pipe_kernel": ("0", "1"), "gemm_bf16_plain_kernel": ("64",)}
+    rng, seen, launches = random.Random(0), set(), set()
+    sizes = [1, 8, 63, 64, 128, 200, 256, 500, 768, 1024, 1379, 2048, 4096, 5000, 8457]
+    shapes = [tuple(rng.choice(sizes) for _ in range(3)) for _ in range(400)] + [(2048, 8457, 1024), (4096, 3072, 1024), (51, 131, 9)]
+    for dtype in (ffk.FLOAT, ffk.BF16):
+        for M, N, K in shapes:
+            for ta, tb in ((False, False), (False, True), (True, False), (True, True)):
+                names = ffk.gemm_kernel_name(dtype, ta, tb, M, N, K).split(" + ")
+                launches.add(len(names))
+                for full in names:
+                    name, _, args = full.rstrip(">").partition("<")
+                    args = tuple(args.split(",")) if args else ()
+                    kernel = have.get(name)
+                    assert kernel, full
+                    n = len(next(iter(kernel)))
+                    fill = defaults.get(name, ())
+                    args += fill[len(fill) - (n - len(args)):] if n > len(args) else ()
+                    assert args in kernel, (full, args)
+                    seen.add(name)
+    assert launches == {1, 2}
+    assert seen == {"gemm_bf16_pipe_kernel", "gemm_bf16_kernel", "gemm_bf16_plain_kernel", "gemm_f32_kernel",
+                    "gemm_f32_tiled_kernel", "gemm_f32_small_kernel", "gemm_f32_deep_kernel"}
