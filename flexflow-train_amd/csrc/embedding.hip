@@ -298,11 +298,11 @@ __device__ __forceinline__ void load_grad4(bf16 const *p, float (&v)[4]) {
 
 // LPR lanes share a row, 4 columns per lane and CPL such chunks per lane in
 // one pass (columns c = ((k * LPR) + lane) * 4, k < CPL).
-// DET: a walker owns every run that STARTS in its chunk and follows it to its
+// A walker owns every run that STARTS in its chunk and follows it to its
 // end, however far; no run is shared, nothing is atomic, and every row is
 // summed in ascending lookup order, so the result is bit-reproducible (a very
 // popular row is then summed by a single walker, which is slow).
-template <typename GT, int LPR, int CPL, bool DET>
+template <typename GT, int LPR, int CPL>
 __global__ __launch_bounds__(256) void embedding_bwd_sorted_kernel(
     uint32_t const *__restrict__ keys, uint32_t const *__restrict__ vals,
     GT const *__restrict__ dY, float *dW, int64_t n, int bag, int64_t dim,
@@ -313,14 +313,10 @@ __global__ __launch_bounds__(256) void embedding_bwd_sorted_kernel(
   if (p0 >= n) return;
   int64_t const p1 = min(p0 + (int64_t)kEmbChunk, n);
   int64_t start = p0;
-  if (DET) {
-    while (start < p1 && start > 0 && keys[start - 1] == keys[start]) start++;
-    if (start >= p1) return;
-  }
+  while (start < p1 && start > 0 && keys[start - 1] == keys[start]) start++;
+  if (start >= p1) return;
   // is position p part of this walker's work?
-  auto mine = [&](int64_t p) {
-    return p < p1 || (DET && p < n && keys[p] == keys[p - 1]);
-  };
+  auto mine = [&](int64_t p) { return p < p1 || (p < n && keys[p] == keys[p - 1]); };
   for (int64_t cbase = 0; cbase < dim; cbase += (int64_t)LPR * 4 * CPL) {
     float acc[CPL][4], cur[CPL][4], nxt[CPL][4];
     auto fetch = [&](int64_t p, float (&v)[CPL][4]) {
@@ -340,8 +336,6 @@ __global__ __launch_bounds__(256) void embedding_bwd_sorted_kernel(
     for (int k = 0; k < CPL; k++)
 #pragma unroll
       for (int e = 0; e < 4; e++) acc[k][e] = 0.0f;
-    // a run that began in the previous chunk is shared with that walker
-    bool shared_run = !DET && p0 > 0 && keys[p0 - 1] == keys[p0];
     fetch(start, cur);
     for (int64_t p = start; mine(p); p++) {
       bool const more = mine(p + 1);
@@ -351,28 +345,20 @@ __global__ __launch_bounds__(256) void embedding_bwd_sorted_kernel(
       for (int k = 0; k < CPL; k++)
 #pragma unroll
         for (int e = 0; e < 4; e++) acc[k][e] += cur[k][e];
-      bool const run_end = !more || keys[p + 1] != id;
-      if (run_end) {
-        if (!DET && !more && p + 1 < n && keys[p + 1] == id) shared_run = true;  // continues next door
+      if (!more || keys[p + 1] != id) {  // the run's end
         if (id != invalid_key) {
 #pragma unroll
           for (int k = 0; k < CPL; k++) {
             int64_t const c = cbase + ((int64_t)k * LPR + wl) * 4;
             if (c < dim) {
               float *dst = dW + (int64_t)id * dim + c;
-              if (shared_run) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) atomicAdd(dst + e, acc[k][e] * scale);
-              } else {
-                f32x4 old = *reinterpret_cast<f32x4 const *>(dst);
-                f32x4 upd = {old[0] + acc[k][0] * scale, old[1] + acc[k][1] * scale,
-                             old[2] + acc[k][2] * scale, old[3] + acc[k][3] * scale};
-                *reinterpret_cast<f32x4 *>(dst) = upd;
-              }
+              f32x4 old = *reinterpret_cast<f32x4 const *>(dst);
+              f32x4 upd = {old[0] + acc[k][0] * scale, old[1] + acc[k][1] * scale,
+                           old[2] + acc[k][2] * scale, old[3] + acc[k][3] * scale};
+              *reinterpret_cast<f32x4 *>(dst) = upd;
             }
           }
         }
-        shared_run = false;
 #pragma unroll
         for (int k = 0; k < CPL; k++)
 #pragma unroll
@@ -660,7 +646,7 @@ static int emb_backward(hipStream_t st, void const *indices, void const *dy,
     if (deterministic) {
       int64_t const walkers = ceil_div(lookups, kEmbChunk);
 #define FFK_EMB_SORTED(LPR_, CPL_)                                             \
-  embedding_bwd_sorted_kernel<GT, LPR_, CPL_, true><<<(unsigned)ceil_div(walkers * LPR_, 256), 256, 0, st>>>( \
+  embedding_bwd_sorted_kernel<GT, LPR_, CPL_><<<(unsigned)ceil_div(walkers * LPR_, 256), 256, 0, st>>>( \
       keys_out, vals_out, G, dw, lookups, (int)bag, dim, (uint32_t)num_entries, scale)
       if (dim > 512) FFK_EMB_SORTED(64, 4);
       else if (dim > 256) FFK_EMB_SORTED(64, 2);

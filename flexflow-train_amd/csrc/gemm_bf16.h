@@ -1380,20 +1380,24 @@ static hipError_t launch_tail(hipStream_t st, bf16 const *A, bf16 const *B, bf16
   if (gemm_splits_reduction(M, N, K, ep)) {
     return launch_pipe<64, 64, 32, 32, 64, 2, 3, TA, TB, TAIL, kEdgeBounded, 2>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
   }
-  // column sums are taken over blocks of 32 rows from multiples of 32 on, where overlapping tiles do not begin
-  constexpr bool sums = TAIL == GemmEpilogue::kTailDropoutGeluGrad || TAIL == GemmEpilogue::kTailDropoutReluGrad;
-  constexpr int edge = sums ? kEdgeBounded : kEdgeOverlap;
-  if (!sums && (M < 128 || N < 128)) return hipErrorInvalidValue;
-  // 128 x 64 where the plain product takes it (1379 x 3072 over 768 with ReLU and dropout: 24.4 -> 21.6 us), and
-  // where a round holds them all: the operators on the store are then spread over twice the CUs (1379 x 768
-  // over 3072 with dropout and add: 25.7 -> 22.7).
-  if constexpr (!sums) {
-    if (gemm_tile_for(M, N, K, ep.activation == FFK_ACT_NONE) == kTile128x64 ||
-        ceil_div(M, 128) * ceil_div(N, 64) <= kNumCU) {
-      return launch_pipe<128, 64, 32, 32, 64, 3, 1, TA, TB, TAIL, edge>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+  if constexpr (TAIL == GemmEpilogue::kTailGeluDropout) {
+    return hipErrorInvalidValue;  // (one large tile a CU: gemm_tail_supported has refused it)
+  } else {
+    // column sums are taken over blocks of 32 rows from multiples of 32 on, where overlapping tiles do not begin
+    constexpr bool sums = TAIL == GemmEpilogue::kTailDropoutGeluGrad || TAIL == GemmEpilogue::kTailDropoutReluGrad;
+    constexpr int edge = sums ? kEdgeBounded : kEdgeOverlap;
+    if (!sums && (M < 128 || N < 128)) return hipErrorInvalidValue;
+    // 128 x 64 where the plain product takes it (1379 x 3072 over 768 with ReLU and dropout: 24.4 -> 21.6 us), and
+    // where a round holds them all: the operators on the store are then spread over twice the CUs (1379 x 768
+    // over 3072 with dropout and add: 25.7 -> 22.7).
+    if constexpr (!sums) {
+      if (gemm_tile_for(M, N, K, ep.activation == FFK_ACT_NONE) == kTile128x64 ||
+          ceil_div(M, 128) * ceil_div(N, 64) <= kNumCU) {
+        return launch_pipe<128, 64, 32, 32, 64, 3, 1, TA, TB, TAIL, edge>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+      }
     }
+    return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, TAIL, edge>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
   }
-  return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, TAIL, edge>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
 }
 template <bool TA, bool TB>
 hipError_t pick_bf16_tail(hipStream_t st, bf16 const *A, bf16 const *B, bf16 *C, int M, int N, int K, int64_t lda,
