@@ -212,6 +212,38 @@ def test_attention_strided_views(ffk, oracle):
     assert_close(d[:, :, 2], dv_ref, BF16_RTOL, "dV")
 
 
+@pytest.mark.parametrize("D,Dv", [(256, 256), (132, 200)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_attention_fp32_rows_past_31_bits(ffk, D, Dv, causal):
+    """fp32 head sizes beyond 128 with rows so far apart that direct loads do not reach them: the tiles come
+    through registers, the same arithmetic and bits as on dense tensors."""
+    say("attention fp32, wide rows", D, Dv, causal)
+    H, S, step = 2, 70, 1 << 23  # floats between two rows: 70 of them span 2.3 GB
+    gen = torch.Generator(device="cuda").manual_seed(D)
+    q, k, v, do = (torch.randn((1, S, H, d), generator=gen, device="cuda") for d in (D, D, Dv, Dv))
+    scale = D ** -0.5
+    o, lse = ffk.attention_forward(q, k, v, scale, causal)
+    dq, dk, dv = ffk.attention_backward(q, k, v, o, do, lse, scale, causal)
+    # the eight tensors side by side in one buffer, row after row
+    buf = torch.empty(((S - 1) * step + 8 * H * max(D, Dv),), device="cuda")
+    wide = [buf.as_strided((1, S, H, d), (S * step, step, d, 1), i * H * max(D, Dv))
+            for i, d in enumerate((D, D, Dv, Dv, Dv, D, D, Dv))]
+    wq, wk, wv, wdo, wo, wdq, wdk, wdv = wide
+    for t, src in ((wq, q), (wk, k), (wv, v), (wdo, do)):
+        t.copy_(src)
+    desc = ffk.AttentionDesc(1, H, S, S, D, *(S * step, step) * 4, scale, int(causal), Dv)
+    lse2, delta = torch.empty_like(lse), torch.empty_like(lse)
+    st = ffk.current_stream()
+    ffk.check(ffk.lib().ffk_attention_forward(st, ffk.FLOAT, desc, wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), wo.data_ptr(),
+                                              lse2.data_ptr()))
+    assert torch.equal(wo, o) and torch.equal(lse2, lse)
+    ffk.check(ffk.lib().ffk_attention_backward(st, ffk.FLOAT, desc, wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), wo.data_ptr(),
+                                               wdo.data_ptr(), lse2.data_ptr(), delta.data_ptr(), wdq.data_ptr(),
+                                               wdk.data_ptr(), wdv.data_ptr()))
+    for got, want, name in ((wdq, dq, "dQ"), (wdk, dk, "dK"), (wdv, dv, "dV")):
+        assert torch.equal(got, want), name
+
+
 def test_attention_errors(ffk):
     q = torch.zeros((1, 8, 2, 264), dtype=BT, device="cuda")
     with pytest.raises(ffk.FFKError, match="head_dim"):

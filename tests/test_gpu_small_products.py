@@ -59,8 +59,7 @@ def test_linear_fp32_backward_split_reduction(ffk, shape):
 @pytest.mark.parametrize("causal", [False, True])
 def test_attention_fp32_backward_both_forms(ffk, shape, causal):
     B, H, Sq, Skv, D = shape
-    if causal and Sq != Skv:
-        pytest.skip("causal masks are tested on equal lengths")
+    # causal with Sq != Skv: key j is visible to query i iff j <= i
     print("attention fp32", shape, causal, flush=True)
     gen = torch.Generator().manual_seed(Sq + D)
     q, k, v, do = (torch.randn((B, s, H, D), generator=gen) for s in (Sq, Skv, Skv, Sq))
@@ -78,8 +77,14 @@ def test_attention_fp32_backward_both_forms(ffk, shape, causal):
     o, lse = ffk.attention_forward(qd, kd, vd, scale, causal)
     assert_close(to_np(o), to_np(o_ref.transpose(1, 2).contiguous()), 1e-5, "O")
     got = ffk.attention_backward(qd, kd, vd, o, dod, lse, scale, causal)
+    # where the only query sees one key, of dQ and dK nothing is left but the rounding of dP - delta: 1e-5 of
+    # these two, times the other factor
+    rest = 1e-5 * float(dp.abs().max()) * scale * max(float(t.abs().max()) for t in (qt, kt)) if causal and Sq == 1 else 0.0
     for t, w, name in zip(got, want, ("dQ", "dK", "dV")):
-        assert_close(to_np(t), to_np(w.transpose(1, 2).contiguous()), 1e-5, name)
+        if rest > 0 and name != "dV":
+            assert float(t.abs().max()) <= rest, name
+        else:
+            assert_close(to_np(t), to_np(w.transpose(1, 2).contiguous()), 1e-5, name)
 
 
 @pytest.mark.parametrize("n", [8388609, 8389631])
