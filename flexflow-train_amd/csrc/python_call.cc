@@ -5,7 +5,7 @@
 //
 // Why not ctypes: a call of ten arguments is 0.65 us there, a tensor's pointer with its two checks
 // 0.2 us and torch.cuda.current_stream() 2.9 us, next to 2.6 us for the kernel launch itself: 8.0 us
-// for a Linear forward, of which this leaves 3.3.
+// for a Linear forward, of which this leaves 3.8.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <exception>
