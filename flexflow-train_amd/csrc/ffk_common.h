@@ -223,22 +223,32 @@ __device__ __forceinline__ u32x4 pack_raw(float const (&v)[8], bf16 const *) {
 
 // Vector v (kVec elements from v * kVec on) of a row of N elements, in the two kinds of rows there
 // are: whole aligned vectors, or (ANY) any N at any address, where the last vector may be partial:
-// its missing elements are read as zeros and not stored.
+// its missing elements are read as zeros and not stored.  STREAM: past the caches (whole vectors only).
+// It is a template argument because of two accesses to one address that differ in nothing but the hint
+// the compiler makes one, without the hint, also where the choice between them is a constant.
 template <typename T, bool ANY>
 struct RowVec {
   static constexpr int V = VecIO<T>::kVec;
   __host__ __device__ static __forceinline__ int count(int N) { return ANY ? (N + V - 1) / V : N / V; }
   // how many of vector v's elements exist
   __device__ static __forceinline__ int elems(int v, int N) { return ANY ? min(V, N - v * V) : V; }
-  __device__ static __forceinline__ u32x4 load_raw(T const *row, int v, int N, bool stream) {
+  template <bool STREAM = false>
+  __device__ static __forceinline__ u32x4 load_raw(T const *row, int v, int N) {
     T const *p = row + (int64_t)v * V;
-    if constexpr (ANY) return elems(v, N) == V ? load_raw_any(p) : load_raw_first(p, elems(v, N));
-    return stream ? __builtin_nontemporal_load(reinterpret_cast<u32x4 const *>(p)) : *reinterpret_cast<u32x4 const *>(p);
+    if constexpr (ANY) {
+      return elems(v, N) == V ? load_raw_any(p) : load_raw_first(p, elems(v, N));
+    } else if constexpr (STREAM) {
+      return load_raw_stream(p);
+    } else {
+      return *reinterpret_cast<u32x4 const *>(p);
+    }
   }
-  __device__ static __forceinline__ void load(T const *row, int v, int N, float (&x)[V], bool stream = false) {
-    unpack_raw(load_raw(row, v, N, stream), x, (T const *)nullptr);
+  template <bool STREAM = false>
+  __device__ static __forceinline__ void load(T const *row, int v, int N, float (&x)[V]) {
+    unpack_raw(load_raw<STREAM>(row, v, N), x, (T const *)nullptr);
   }
-  __device__ static __forceinline__ void store(T *row, int v, int N, float const (&x)[V], bool stream = false) {
+  template <bool STREAM = false>
+  __device__ static __forceinline__ void store(T *row, int v, int N, float const (&x)[V]) {
     T *p = row + (int64_t)v * V;
     u32x4 const r = pack_raw(x, (T const *)nullptr);
     if constexpr (ANY) {
@@ -247,7 +257,7 @@ struct RowVec {
       } else {
         store_raw_first(p, r, elems(v, N));
       }
-    } else if (stream) {
+    } else if constexpr (STREAM) {
       __builtin_nontemporal_store(r, reinterpret_cast<u32x4 *>(p));
     } else {
       *reinterpret_cast<u32x4 *>(p) = r;
@@ -364,6 +374,12 @@ static inline FastDiv make_fast_div(uint32_t d) {
 // tensors keep ordinary accesses so the next kernel finds them in cache.
 static inline bool stream_past_caches(int64_t elems, size_t elem_size) {
   return (size_t)elems * elem_size > ((size_t)128 << 20);
+}
+// The same for a row-wise backward, two such tensors read and one written: past the caches where the three do
+// not fit them together.  LayerNorm backward in bf16, read past the caches / through them: [16384, 4096] 76 / 85
+// us, [8192, 2048] 31 / 26, [4096, 1024] 11.4 / 11.2; Softmax's 71 / 76, 18.6 / 16.3, 3.6 / 3.6.
+static inline bool three_past_caches(int64_t elems, size_t elem_size) {
+  return 3 * (size_t)elems * elem_size > ((size_t)256 << 20);
 }
 
 // A kernel that uses more than 64 KB of dynamic LDS has to be given leave, once on every device

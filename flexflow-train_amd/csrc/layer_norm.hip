@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
   for (int j = 0; j < EPT; j++) {
     int v = lane + j * LANES;
     if (v < nvec) {
-      RV::load(xr, v, N, x[j], STREAM);
+      RV::template load<STREAM>(xr, v, N, x[j]);
       if constexpr (PRE) {
         static_assert(V == 4 || V == 8, "a lane's vector is a Philox block or half of one");
         if (row_ok) {
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
         float xh = (x[j][e] - mu) * rs;
         y[e] = xh * g[j][e] + b[j][e];
       }
-      RV::store(yr, v, N, y, STREAM);
+      RV::template store<STREAM>(yr, v, N, y);
     }
   }
 }
@@ -172,14 +172,14 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_generic_kernel(
 // in registers until the workgroup is done.
 // DROP: dropout_backward(dX as stored) is written to `dropped` as well (the gradient entering
 // a dropout whose output fed the residual sum that this LayerNorm normalised).
-template <typename T, int EPT, int WPR, bool ACC, bool DROP = false, bool ANY = false>
+// STREAM: dY and X are read past the caches.
+template <typename T, int EPT, int WPR, bool ACC, bool DROP = false, bool ANY = false, bool STREAM = false>
 __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
     T const *__restrict__ dY, T const *__restrict__ X,
     float const *__restrict__ mean, float const *__restrict__ rstd,
     T const *__restrict__ gamma, T *dX, float *__restrict__ partials,
     int64_t M, int N, T const *res, T *__restrict__ dropped = nullptr,
-    DropoutParams drop = DropoutParams{}, bool stream_out = false, bool round_first = true) {
-  // stream_out: dX is too large to be found in cache by its reader; store it past the caches.
+    DropoutParams drop = DropoutParams{}, bool round_first = true) {
   // ACC with res == nullptr: dX += gradient (one rounding).  ACC with res set and round_first:
   // dX = res + gradient rounded to the storage type, i.e. what a separate element-wise add of
   // res to the stored gradient would give; without round_first the sum is rounded once, i.e.
@@ -231,8 +231,8 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
       for (int j = 0; j < EPT; j++) {
         int v = lane + j * LANES;
         if (v < nvec) {
-          rx[j] = RV::load_raw(X + r * (int64_t)N, v, N, true);
-          rdy[j] = RV::load_raw(dY + r * (int64_t)N, v, N, true);
+          rx[j] = RV::template load_raw<STREAM>(X + r * (int64_t)N, v, N);
+          rdy[j] = RV::template load_raw<STREAM>(dY + r * (int64_t)N, v, N);
         }
       }
     } else {
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
             if (ACC && res != nullptr && round_first) val = storage_round<T>(val);
             o[e] = ACC ? o[e] + val : val;
           }
-          RV::store(dst, v, N, o, stream_out);
+          RV::store(dst, v, N, o);
           if constexpr (DROP) {
             static_assert(V == 4 || V == 8, "a lane's vector is a Philox block or half of one");
             int64_t const at = row * (int64_t)N + (int64_t)v * V;
@@ -514,7 +514,14 @@ static int ln_backward(hipStream_t st, void const *dy, void const *x,
                   need, workspace_bytes);
     }
     float *partials = static_cast<float *>(workspace);
-    bool const stream = stream_past_caches(M * N, sizeof(T));
+    bool const stream = three_past_caches(M * N, sizeof(T));
+#define LAUNCH(...)                                                            \
+  do {                                                                         \
+    auto kern = stream ? layer_norm_bwd_kernel<__VA_ARGS__, false, true>       \
+                       : layer_norm_bwd_kernel<__VA_ARGS__, false, false>;     \
+    kern<<<blocks, kRowThreads, 0, st>>>(DY, X, mean, rstd, G, DX, partials, M, (int)N, RES, static_cast<T *>(dropped), \
+                                         drop != nullptr ? *drop : DropoutParams{}, round_first); \
+  } while (0)
 #define CALL(E, W)                                                             \
   do {                                                                         \
     if (!vec) {                                                                \
@@ -524,20 +531,17 @@ static int ln_backward(hipStream_t st, void const *dy, void const *x,
       else                                                                     \
         layer_norm_bwd_kernel<T, E, W, false, false, true><<<blocks, kRowThreads, 0, st>>>( \
             DY, X, mean, rstd, G, DX, partials, M, (int)N, nullptr);           \
-    } else if (dropped != nullptr) {                                                  \
-      if constexpr (sizeof(T) == 2)                                            \
-        layer_norm_bwd_kernel<T, E, W, true, true><<<blocks, kRowThreads, 0, st>>>( \
-            DY, X, mean, rstd, G, DX, partials, M, (int)N, RES,                \
-            static_cast<T *>(dropped), *drop, stream, round_first);            \
-    } else if (acc)                                                            \
-      layer_norm_bwd_kernel<T, E, W, true><<<blocks, kRowThreads, 0, st>>>(    \
-          DY, X, mean, rstd, G, DX, partials, M, (int)N, RES, nullptr, DropoutParams{}, stream, round_first); \
-    else                                                                       \
-      layer_norm_bwd_kernel<T, E, W, false><<<blocks, kRowThreads, 0, st>>>(   \
-          DY, X, mean, rstd, G, DX, partials, M, (int)N, nullptr, nullptr, DropoutParams{}, stream); \
+    } else if (dropped != nullptr) {                                           \
+      if constexpr (sizeof(T) == 2) LAUNCH(T, E, W, true, true);               \
+    } else if (acc) {                                                          \
+      LAUNCH(T, E, W, true, false);                                            \
+    } else {                                                                   \
+      LAUNCH(T, E, W, false, false);                                           \
+    }                                                                          \
   } while (0)
     FFK_ROW_DISPATCH_SMALL(ept, wpr, CALL);
 #undef CALL
+#undef LAUNCH
     FFK_CHECK_LAUNCH();
     if (dgamma != nullptr || dbeta != nullptr) {
       // partials are [blocks][2][N]: gamma sums in columns [0, N), beta after

@@ -32,7 +32,7 @@ __global__ __launch_bounds__(kRowThreads) void softmax_fwd_kernel(
   for (int j = 0; j < EPT; j++) {
     int v = lane + j * LANES;
     if (v < nvec) {
-      RV::load(xr, v, N, x[j], STREAM);
+      RV::template load<STREAM>(xr, v, N, x[j]);
       if constexpr (ANY) {
 #pragma unroll
         for (int e = 0; e < V; e++) x[j][e] = e < RV::elems(v, N) ? x[j][e] : -INFINITY;
@@ -66,7 +66,7 @@ __global__ __launch_bounds__(kRowThreads) void softmax_fwd_kernel(
       float y[V];
 #pragma unroll
       for (int e = 0; e < V; e++) y[e] = x[j][e] * inv;
-      RV::store(yr, v, N, y, STREAM);
+      RV::template store<STREAM>(yr, v, N, y);
     }
   }
 }
@@ -93,9 +93,8 @@ __global__ __launch_bounds__(kRowThreads) void softmax_bwd_kernel(
   for (int j = 0; j < EPT; j++) {
     int v = lane + j * LANES;
     if (v < nvec) {
-      // two input streams read once: cache-bypassing loads
-      RV::load(Y + r * (int64_t)N, v, N, y[j], true);
-      RV::load(dY + r * (int64_t)N, v, N, dy[j], true);
+      RV::template load<STREAM>(Y + r * (int64_t)N, v, N, y[j]);
+      RV::template load<STREAM>(dY + r * (int64_t)N, v, N, dy[j]);
 #pragma unroll
       for (int e = 0; e < V; e++) dot += y[j][e] * dy[j][e];
     }
@@ -109,7 +108,7 @@ __global__ __launch_bounds__(kRowThreads) void softmax_bwd_kernel(
       float o[V];
 #pragma unroll
       for (int e = 0; e < V; e++) o[e] = y[j][e] * (dy[j][e] - dot);
-      RV::store(dX + row * (int64_t)N, v, N, o, STREAM);
+      RV::template store<STREAM>(dX + row * (int64_t)N, v, N, o);
     }
   }
 }
@@ -239,7 +238,7 @@ static int softmax_bwd(hipStream_t st, void const *y, void const *dy, void *dx,
     if (pick_row_config(ceil_div(dim, V), ept, wpr)) {
       int64_t blocks = ceil_div(outer, 4 / wpr);
       bool const vec = dim % V == 0 && aligned16(y) && aligned16(dy) && aligned16(dx);
-      bool const stream = stream_past_caches(outer * dim, sizeof(T));
+      bool const stream = three_past_caches(outer * dim, sizeof(T));
 #define CALL(E, W)                                                             \
   do {                                                                         \
     if (!vec)                                                                  \
