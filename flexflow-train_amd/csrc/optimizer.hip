@@ -15,9 +15,14 @@
 namespace ffk {
 
 constexpr int kOptThreads = 256;
-// Adam: vectors per thread.  Past the caches one, with more workgroups taking turns (bf16 gradients: 12.6 M
-// parameters 62.2 -> 60.1 us, 50 M 245 -> 241); within them two (3 M 13.2 us, 13.9 with one).
-constexpr int adam_unroll(bool stream) { return stream ? 1 : 2; }
+// Adam: vectors per thread.  Within the caches two (3 M parameters 13.2 us, 13.9 with one).  Past them one, with
+// more workgroups taking turns, and without a bf16 copy written out two again from a size on.  us, one / two,
+// fp32 and bf16 gradients: 12.6 M parameters 59 / 61 and 54 / 57; 25 M 123 / 119 and 107 / 111; 50 M 246 / 240
+// and 228 / 223.  (With the copy 12.6 M 64 / 68 and 58 / 63, 25 M 133 / 132 and 116 / 123; 67 M 371 / 364 and 344 /
+// 336, or 342 / 353 and 311 / 322, by where the arrays lie.)
+static int adam_unroll(bool past_caches, int64_t n, int grad_dtype, bool lowp) {
+  return past_caches && (lowp || n <= (grad_dtype == FFK_BF16 ? 2 << 24 : 5 << 22)) ? 1 : 2;
+}
 
 // 16-byte accesses; STREAM: past the caches (parameter sets larger than the last-level cache
 // are touched once per step and never found there again)
@@ -139,11 +144,10 @@ __device__ __forceinline__ void adam_step(float g, float &w, float &m, float &v,
   w = w - q;
 }
 
-template <typename GT, bool STREAM>
+template <typename GT, bool STREAM, int UNROLL>
 __global__ __launch_bounds__(kOptThreads) void adam_update_kernel(
     GT const *__restrict__ grad, float *W, float *M, float *V, bf16 *W_lowp,
     int64_t n, int replicas, AdamParams p) {
-  constexpr int UNROLL = adam_unroll(STREAM);
   // UNROLL vectors of 4 parameters per thread, a workgroup's vectors interleaved: all loads
   // of a thread are issued before the first arithmetic, which keeps more bytes in flight
   int64_t const first = ((int64_t)blockIdx.x * kOptThreads * UNROLL + threadIdx.x) * 4;
@@ -253,15 +257,20 @@ extern "C" int ffk_adam_update(ffk_stream_t stream, int grad_dtype, float alpha_
   AdamParams p{alpha_t, beta1, beta2, weight_decay, epsilon};
   hipStream_t st = as_stream(stream);
   bool const past_caches = stream_past_caches(num_elements, 16);
-  unsigned const blocks = (unsigned)ceil_div(ceil_div(num_elements, 4), kOptThreads * adam_unroll(past_caches));
-#define FFK_ADAM(GT_, S_)                                                      \
-  adam_update_kernel<GT_, S_><<<blocks, kOptThreads, 0, st>>>(                 \
+  int const unroll = adam_unroll(past_caches, num_elements, grad_dtype, weight_lowp != nullptr);
+  unsigned const blocks = (unsigned)ceil_div(ceil_div(num_elements, 4), kOptThreads * unroll);
+#define FFK_ADAM(GT_, S_, U_)                                                  \
+  adam_update_kernel<GT_, S_, U_><<<blocks, kOptThreads, 0, st>>>(             \
       static_cast<GT_ const *>(weight_grad), weight, adam_m, adam_v, static_cast<bf16 *>(weight_lowp), \
       num_elements, num_replicas, p)
   if (grad_dtype == FFK_FLOAT) {
-    if (past_caches) FFK_ADAM(float, true); else FFK_ADAM(float, false);
+    if (!past_caches) FFK_ADAM(float, false, 2);
+    else if (unroll == 1) FFK_ADAM(float, true, 1);
+    else FFK_ADAM(float, true, 2);
   } else {
-    if (past_caches) FFK_ADAM(bf16, true); else FFK_ADAM(bf16, false);
+    if (!past_caches) FFK_ADAM(bf16, false, 2);
+    else if (unroll == 1) FFK_ADAM(bf16, true, 1);
+    else FFK_ADAM(bf16, true, 2);
   }
 #undef FFK_ADAM
   FFK_CHECK_LAUNCH();

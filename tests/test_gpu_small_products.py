@@ -87,17 +87,21 @@ def test_attention_fp32_backward_both_forms(ffk, shape, causal):
             assert_close(to_np(t), to_np(w.transpose(1, 2).contiguous()), 1e-5, name)
 
 
-@pytest.mark.parametrize("n", [8388609, 8389631])
-def test_adam_past_the_caches(ffk, oracle, n):
-    """Parameters from where the update bypasses the caches on, with a last workgroup of few."""
+@pytest.mark.parametrize("n,dtype,copy", [(8388609, torch.float32, True), (8389631, torch.float32, True),
+                                          (20971520, torch.float32, False), (20972543, torch.float32, False),
+                                          (33554433, torch.bfloat16, False)])
+def test_adam_past_the_caches(ffk, oracle, n, dtype, copy):
+    """Parameters from where the update bypasses the caches on, with a last workgroup of few, on both sides of the
+    sizes from which a thread takes two vectors again."""
     gen = torch.Generator().manual_seed(n)
     w0, grad, m0 = (torch.randn(n, generator=gen) for _ in range(3))
+    grad = grad.to(dtype)
     v0 = torch.rand(n, generator=gen)
     args = dict(alpha_t=1e-2, beta1=0.9, beta2=0.99, weight_decay=0.05, epsilon=1e-6)
-    want = oracle.adam_update(w0.numpy().copy(), grad.numpy().copy(), m0.numpy().copy(), v0.numpy().copy(), **args)
+    want = oracle.adam_update(w0.numpy().copy(), grad.float().numpy().copy(), m0.numpy().copy(), v0.numpy().copy(), **args)
     w, m, v = w0.cuda(), m0.cuda(), v0.cuda()
-    low = torch.empty(n, device="cuda", dtype=torch.bfloat16)
+    low = torch.empty(n, device="cuda", dtype=torch.bfloat16) if copy else None
     ffk.adam_update(w, grad.cuda(), m, v, weight_lowp=low, **args)
     for got, ref in zip((w, m, v), want):
         assert torch.equal(got.cpu(), torch.from_numpy(ref))
-    assert torch.equal(low, w.to(torch.bfloat16))
+    assert low is None or torch.equal(low, w.to(torch.bfloat16))
