@@ -1,8 +1,9 @@
 """Python plumbing over libffk.so, the gfx950 operator-kernel library.
 
-This module only loads the C-ABI library (``include/ffk.h``) with ctypes and
-offers thin helpers that pass ``torch`` tensors' device pointers and the
-current HIP stream to it.  PyTorch is used for device memory and streams only;
+This module only loads the C-ABI library (``include/ffk.h``) and offers thin
+helpers that pass ``torch`` tensors and the current HIP stream to its entry
+points, through functions generated from their prototypes
+(``csrc/python_call.cc``); every symbol is bound with ctypes beside them.  PyTorch is used for device memory and streams only;
 no arithmetic here is done by torch.  If ``libffk.so`` is missing the import of
 any entry point fails loudly -- there is no fallback path.
 
