@@ -4,6 +4,7 @@
 #pragma once
 #include "lds_dma.h"
 #include "gemm.h"
+#include "gemm_any.h"
 #include <algorithm>
 #include <stdarg.h>
 #include <stdio.h>
@@ -87,217 +88,31 @@ __device__ __forceinline__ u32x2 load_first4(bf16 const *p, int n) {
 
 enum { kEdgeNone = 0, kEdgeOverlap = 1, kEdgeBounded = 2 };
 
-constexpr int kBK = 64;        // K extent of one LDS tile
-constexpr int kPadK = 8;       // row padding (elements) of a K-contiguous tile
-constexpr int kPadMN = 32;     // row padding of an M/N-contiguous tile
-
-template <int ROWS, bool TRANS>
-struct TileGeom {
-  // TRANS == false: tile held as [ROWS][kBK] (reduction dim contiguous)
-  // TRANS == true : tile held as [kBK][ROWS] (as it lies in memory)
-  static constexpr int kStride = TRANS ? (ROWS + kPadMN) : (kBK + kPadK);
-  static constexpr int kElems = TRANS ? kBK * kStride : ROWS * kStride;
-};
-
+// The register-staged kernel: operands at any address with any row stride (the tile and what it costs are
+// in gemm_any.h).
 template <int BM, int BN, int WM, int WN, bool TA, bool TB>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16_kernel(
     bf16 const *__restrict__ A, bf16 const *__restrict__ B, bf16 *C, int M,
     int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
     bf16 const *__restrict__ bias, int act, int accumulate) {
-  constexpr int NW = (BM / WM) * (BN / WN);
-  constexpr int NT = NW * 64;
-  constexpr int TM = WM / 32;  // MFMA tiles per wave along M
-  constexpr int TN = WN / 32;
-  using GA = TileGeom<BM, TA>;
-  using GB = TileGeom<BN, TB == false>;  // B is "transposed" when it is [K,N]
-  constexpr bool TBL = (TB == false);    // B tile lies as [kBK][BN]
-  constexpr int A_CHUNKS = BM * kBK / 8 / NT;  // 16-byte chunks per thread
-  constexpr int B_CHUNKS = BN * kBK / 8 / NT;
-  static_assert(BM * kBK / 8 % NT == 0 && BN * kBK / 8 % NT == 0, "tile/threads");
-
-  __shared__ __attribute__((aligned(16))) bf16 As[2][GA::kElems];
-  __shared__ __attribute__((aligned(16))) bf16 Bs[2][GB::kElems];
-
-  int const t = threadIdx.x;
-  int const lane = t & 63;
-  int const wave = t >> 6;
-  int const wm0 = (wave / (BN / WN)) * WM;
-  int const wn0 = (wave % (BN / WN)) * WN;
-
+  using Tile = AnyTile<BM, BN, WM, WN, !TA, TB>;
+  __shared__ __attribute__((aligned(16))) bf16 smem[2 * Tile::kBufElems];
   int tm, tn;
   tile_coords(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN, tm, tn);
-  int const m0 = tm * BM;
-  int const n0 = tn * BN;
-
-  f32x16 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; i++)
-#pragma unroll
-    for (int j = 0; j < TN; j++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-
-  u32x4 ra[A_CHUNKS], rb[B_CHUNKS];
-
-  // Elements [pos, pos + 8) of a row of `len` elements, those past its end as zeros.
-  auto chunk = [](bf16 const *row, int pos, int len) __attribute__((always_inline)) -> u32x4 {
-    if (pos + 8 <= len) return load_raw_any(row + pos);
-    return pos < len ? load_raw_first(row + pos, len - pos) : u32x4{0u, 0u, 0u, 0u};
-  };
-  // One operand's next tile.  KC: the reduction index is contiguous; rows past the edge are read
-  // from the last one (what they give is not stored).  INNER: the whole tile exists, which is
-  // decided once for the workgroup and keeps the loads free of branches.
-  auto gload_one = [&](auto inner, auto kc_tag, auto br_tag, bf16 const *X, int64_t ld, int r0, int R, int k0, u32x4 *dst) __attribute__((always_inline)) {
-    constexpr bool INNER = decltype(inner)::value, KC = decltype(kc_tag)::value;
-    constexpr int BR = decltype(br_tag)::value;
-#pragma unroll
-    for (int i = 0; i < BR * kBK / 8 / NT; i++) {
-      int const c = t + i * NT;
-      if constexpr (KC) {
-        int const row = c >> 3, k = k0 + (c & 7) * 8;
-        bf16 const *const p = X + (int64_t)min(r0 + row, R - 1) * ld;
-        dst[i] = INNER ? load_raw_any(p + k) : chunk(p, k, K);
-      } else {
-        int const k = k0 + c / (BR / 8), r = r0 + (c % (BR / 8)) * 8;
-        bf16 const *const p = X + (int64_t)k * ld;
-        if (INNER) {
-          dst[i] = load_raw_any(p + r);
-        } else {
-          dst[i] = k < K ? chunk(p, r, R) : u32x4{0u, 0u, 0u, 0u};
-        }
-      }
-    }
-  };
-  using KcA = std::integral_constant<bool, !TA>;
-  using KcB = std::integral_constant<bool, !TBL>;
-  using BmT = std::integral_constant<int, BM>;
-  using BnT = std::integral_constant<int, BN>;
-  bool const inner_mn = m0 + BM <= M && n0 + BN <= N;
-  auto gload = [&](int k0) {
-    if (inner_mn && k0 + kBK <= K) {
-      gload_one(std::true_type{}, KcA{}, BmT{}, A, lda, m0, M, k0, ra);
-      gload_one(std::true_type{}, KcB{}, BnT{}, B, ldb, n0, N, k0, rb);
-    } else {
-      gload_one(std::false_type{}, KcA{}, BmT{}, A, lda, m0, M, k0, ra);
-      gload_one(std::false_type{}, KcB{}, BnT{}, B, ldb, n0, N, k0, rb);
-    }
-  };
-
-  auto lstore = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < A_CHUNKS; i++) {
-      int c = t + i * NT;
-      int idx;
-      if (!TA) {
-        idx = (c >> 3) * GA::kStride + (c & 7) * 8;
-      } else {
-        idx = (c / (BM / 8)) * GA::kStride + (c % (BM / 8)) * 8;
-      }
-      *reinterpret_cast<u32x4 *>(&As[buf][idx]) = ra[i];
-    }
-#pragma unroll
-    for (int i = 0; i < B_CHUNKS; i++) {
-      int c = t + i * NT;
-      int idx;
-      if (!TBL) {
-        idx = (c >> 3) * GB::kStride + (c & 7) * 8;
-      } else {
-        idx = (c / (BN / 8)) * GB::kStride + (c % (BN / 8)) * 8;
-      }
-      *reinterpret_cast<u32x4 *>(&Bs[buf][idx]) = rb[i];
-    }
-  };
-
-  // Operand fragment for one 32-row MFMA tile and one 16-wide k step.
-  // Lane l supplies row (l % 32), k = 8 * (l / 32) .. + 7.
-  auto frag = [&](bf16 const *tile, int stride, bool trans, int row0,
-                  int kk) -> bf16x8 {
-    if (!trans) {
-      bf16 const *p = tile + (row0 + (lane & 31)) * stride + kk * 16 + (lane >> 5) * 8;
-      return *reinterpret_cast<bf16x8 const *>(p);
-    }
-    // Transposing load: within each 16-lane group, lane i points at 4 elements
-    // of row k_(i/4), columns 4*(i%4)..+3, and receives column i of the four
-    // rows.  Two loads give 8 consecutive k for this lane's row.
-    int const i16 = lane & 15;
-    int const col = row0 + ((lane >> 4) & 1) * 16 + (i16 & 3) * 4;
-    int const kbase = kk * 16 + (lane >> 5) * 8 + (i16 >> 2);
-    typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
-    s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (lds_s16x4_ptr)(tile + kbase * stride + col));
-    s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (lds_s16x4_ptr)(tile + (kbase + 4) * stride + col));
-    union {
-      s16x4 h[2];
-      bf16x8 v;
-    } u;
-    u.h[0] = lo;
-    u.h[1] = hi;
-    return u.v;
-  };
-
-  int const KT = (K + kBK - 1) / kBK;
-  gload(0);
-  lstore(0);
-  __syncthreads();
-  int cur = 0;
-  for (int kt = 0; kt < KT; kt++) {
-    bool const more = kt + 1 < KT;
-    if (more) {
-      gload((kt + 1) * kBK);
-    }
-#pragma unroll
-    for (int kk = 0; kk < kBK / 16; kk++) {
-      bf16x8 af[TM], bfr[TN];
-#pragma unroll
-      for (int i = 0; i < TM; i++) {
-        af[i] = frag(As[cur], GA::kStride, TA, wm0 + i * 32, kk);
-      }
-#pragma unroll
-      for (int j = 0; j < TN; j++) {
-        bfr[j] = frag(Bs[cur], GB::kStride, TBL, wn0 + j * 32, kk);
-      }
-#pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], bfr[j],
-                                                             acc[i][j], 0, 0, 0);
-    }
-    if (more) {
-      lstore(cur ^ 1);
-    }
-    __syncthreads();
-    cur ^= 1;
-  }
-
-  // Epilogue: accumulator element r of lane l is row 8*(r/4) + 4*(l/32) + r%4,
-  // column l % 32 of its 32x32 tile.
-#pragma unroll
-  for (int j = 0; j < TN; j++) {
-    int const n = n0 + wn0 + j * 32 + (lane & 31);
-    bool const n_ok = n < N;
-    float bv = 0.0f;
-    if (bias != nullptr && n_ok) {
-      bv = VecIO<bf16>::load1(bias + n);
-    }
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        int const m = m0 + wm0 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (n_ok && m < M) {
-          float v = acc[i][j][r] + bv;
-          v = apply_activation(v, act);
-          bf16 *dst = C + (int64_t)m * ldc + n;
-          if (accumulate) {
-            v += VecIO<bf16>::load1(dst);
-          }
-          VecIO<bf16>::store1(dst, v);
-        }
-      }
-    }
-  }
+  int const m0 = tm * BM, n0 = tn * BN;
+  typename Tile::OpA a;
+  typename Tile::OpB b;
+  a.init(A, nullptr, lda, M, K, 0, m0, threadIdx.x);
+  b.init(B, nullptr, ldb, N, K, 0, n0, threadIdx.x);
+  Tile tile;
+  tile.template reduce<false>(a, b, K, 0, (K + kBK - 1) / kBK, smem);
+  tile.store(m0, n0, M, N, [&](int m, int n, float v) {
+    if (bias != nullptr) v += VecIO<bf16>::load1(bias + n);
+    v = apply_activation(v, act);
+    bf16 *const dst = C + (int64_t)m * ldc + n;
+    if (accumulate) v += VecIO<bf16>::load1(dst);
+    VecIO<bf16>::store1(dst, v);
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -1530,10 +1345,13 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
         return launch_pipe<64, 64, 32, 32, 64, 2, 3, TA, TB, 0, kEdgeBounded, 2>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
     }
   }
-  // Largest tile that still gives every CU a workgroup.
-  int64_t const b128 = ceil_div(M, 128) * ceil_div(N, 128);
-  if (b128 >= kNumCU) {
-    return launch_bf16<128, 128, 64, 64, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+  // By what a k-tile takes of a CU: on a 64x64 tile 0.42 us among others and 0.62 alone, on a 128x128 one 0.85
+  // and 1.0 ([2560, 2479] . [1324, 2479]^T 60 us on the first, 51 on the second; [1024, 1023] . [1023, 1023] 16 on
+  // the first, with a quarter of the chip in use on the second).
+  double const per_cu64 = (double)(ceil_div(M, 64) * ceil_div(N, 64)) / kNumCU;
+  double const rounds128 = ceil((double)(ceil_div(M, 128) * ceil_div(N, 128)) / kNumCU);
+  if (std::max(1.0, 0.85 * rounds128) < std::max(0.62, 0.42 * per_cu64)) {
+    return launch_bf16<128, 128, 64, 32, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
   }
   return launch_bf16<64, 64, 32, 32, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
 }

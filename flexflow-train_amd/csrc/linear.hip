@@ -14,6 +14,8 @@
 #include "gemm.h"
 #include "fused_ops.h"
 #include "small_f32.h"
+#include "colreduce.h"
+#include "linear_any.h"
 
 namespace ffk {
 
@@ -162,18 +164,44 @@ static int64_t linear_grad_ld(int dtype, int64_t out_dim) {
   return linear_pads_grad(dtype, out_dim) ? (out_dim + 63) / 64 * 64 : out_dim;
 }
 
-// Room for the partial sums of an input gradient whose reduction over out_dim is split over workgroups:
-// it lies at the end of the workspace, where it overlaps neither g nor column sums that wait there, and
-// it depends on nothing else the call asks for, so that the input gradient has the same bits whatever
-// becomes of the weights'.  in_dim is not known here; what the splits can use is bounded all the same.
+// Room for the partial sums of reductions that are split over workgroups: it lies at the end of the
+// workspace, where it overlaps neither g nor column sums that wait there, and it depends on nothing else
+// the call asks for, so that each gradient has the same bits whatever becomes of the others.
+// in_dim is not known here; what the splits can use is bounded all the same.
 //  fp32: 16 x 16 tiles on two workgroups a CU at most, fewer than 1024 tiles of 1 KB (gemm_f32.hip).
-//  bf16: one round of 256 x 256 tiles in fp32, 64 MB ([2048, 50257] . [50257, 1024] takes all of it: 8
+//  bf16: the jobs of linear_any.hip, on outputs so few that parts of their reductions have to fill the
+//  chip: 512 tiles of 64 x 64 at 16 KB, where a reduction has 512 terms and more.  The input gradient
+//  alone: one round of 256 x 256 tiles in fp32, 64 MB ([2048, 50257] . [50257, 1024] takes all of it: 8
 //  splits, 210 us, 446 without), 16 splits of 2048 columns for few rows.  Shorter reductions, and rows
 //  fewer than a tile's, are not split (gemm_splits_for).
 static size_t linear_split_bytes(int dtype, int64_t batch, int64_t out_dim) {
   if (dtype == FFK_FLOAT) return out_dim >= 2048 ? size_t(1) << 20 : 0;
-  if (dtype != FFK_BF16 || out_dim <= 63 * 64 || batch < 128) return 0;
-  return batch >= 512 ? size_t(64) << 20 : (size_t)batch << 17;
+  if (dtype != FFK_BF16) return 0;
+  size_t const any = batch >= 512 || out_dim >= 512 ? size_t(8) << 20 : 0;
+  if (out_dim <= 63 * 64 || batch < 128) return any;
+  return std::max(any, batch >= 512 ? size_t(64) << 20 : (size_t)batch << 17);
+}
+
+// Whether the two tensors share memory.
+static bool overlap(void const *a, int64_t a_elems, void const *b, int64_t b_elems, size_t size) {
+  uintptr_t const p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+  return a != nullptr && b != nullptr && p < q + (size_t)b_elems * size && q < p + (size_t)a_elems * size;
+}
+
+// Whether the backward runs as the jobs of one launch (linear_any.hip).  aligned: the input and the weight
+// can be read 16 bytes at a time, so that the sequence below has the pipelined products, which overtake the
+// register-staged ones where there is enough to multiply.  Whole backward, this against the sequence, with
+// the forward's share: 7616 x 2176 -> 44 (8046 tiles of 64 deep k's in the two products) 47 and 71 us; 6976 x
+// 576 -> 384 (11 772) 57 and 57; 1280 x 2688 -> 768 (20 160) 43 and 43; 4181 x 2560 -> 247 (21 120) 96 and 81;
+// 2689 x 1728 -> 1024 114 and 69.  The sequence's tiles are wider than 128 columns: 1537 x 128 -> 48518 229 and
+// 265, 832 x 64 -> 41672 109 and 239.
+// Other operands gain at all sizes: 57 x 56 -> 64 9 and 21 us, 2944 x 3446 -> 1488 194 and 479.
+static bool linear_any_takes(int64_t batch, int64_t in_dim, int64_t out_dim, bool aligned) {
+  if (!aligned) return true;
+  // whole tiles that fill half the chip: the fused operators of the encoder layer promise the bits of this sequence
+  if (batch % 128 == 0 && in_dim % 128 == 0 && out_dim % 64 == 0 && (batch / 128) * (in_dim / 128) >= kNumCU / 2) return false;
+  int64_t const k_tiles = ceil_div(batch, 64) * ceil_div(in_dim, 64) * ceil_div(out_dim, 64);
+  return k_tiles <= (in_dim <= 128 ? 40000 : 8000);
 }
 
 extern "C" size_t ffk_linear_backward_workspace_bytes(int dtype, int activation,
@@ -276,6 +304,37 @@ static int linear_backward_impl(
   }
   bool const act = activation != FFK_ACT_NONE;
   bool const sums = bias_grad != nullptr;
+  if (dtype == FFK_BF16 && input_tail == nullptr && std::max(std::max(batch, in_dim), out_dim) < (1 << 30) && (input_grad != nullptr || weight_grad != nullptr) &&
+      tl_weight_grads == nullptr && option(FFK_OPTION_GEMM_VARIANT) == 0 && option(FFK_OPTION_LAYER_UNFUSED) == 0 &&
+      linear_any_takes(batch, in_dim, out_dim, in_dim % 8 == 0 && aligned16(weight) && aligned16(input))) {
+    size_t const split = linear_split_bytes(dtype, batch, out_dim);
+    LinearAnyPlan const plan = linear_any_plan(batch, in_dim, out_dim, split);
+    bool const room = plan.scratch == 0 || (workspace != nullptr && aligned16(workspace) && workspace_bytes >= split);
+    // one launch reads what it writes elsewhere: a gradient over one of the operands takes the sequence below
+    void const *const out[3] = {input_grad, weight_grad, bias_grad};
+    int64_t const out_elems[3] = {batch * in_dim, out_dim * in_dim, out_dim};
+    void const *const in[4] = {output, output_grad, input, weight};
+    int64_t const in_elems[4] = {act ? batch * out_dim : 0, batch * out_dim, batch * in_dim, out_dim * in_dim};
+    bool apart = true;
+    for (int o = 0; o < 3; o++)
+      for (int i = 0; i < 4; i++) apart = apart && !overlap(out[o], out_elems[o], in[i], in_elems[i], 2);
+    if (room && apart) {
+      // the bias gradient is written here and now: a collected job that writes it comes first
+      if (ColreduceBatch *const waiting = tl_colreduce_batch; waiting != nullptr && sums) {
+        bool clash = false;
+        for (int k = 0; k < waiting->count; k++) clash = clash || waiting->job[k].out0 == bias_grad || waiting->job[k].out1 == bias_grad;
+        if (clash) FFK_HIP(colreduce_flush(st, *waiting));
+      }
+      LinearAnyArgs const a = {static_cast<bf16 const *>(output), static_cast<bf16 const *>(output_grad),
+                               static_cast<bf16 const *>(input), static_cast<bf16 const *>(weight),
+                               static_cast<bf16 *>(input_grad), static_cast<bf16 *>(weight_grad),
+                               static_cast<bf16 *>(bias_grad), (int)batch, (int)in_dim, (int)out_dim, relu_grad_mode,
+                               accumulate};
+      void *const scratch = plan.scratch == 0 ? nullptr : static_cast<uint8_t *>(workspace) + ((workspace_bytes - split) & ~(size_t)255);
+      FFK_HIP(linear_any_backward(st, activation, a, plan, scratch));
+      return FFK_OK;
+    }
+  }
   // rows padded to whole 16 bytes, if the products can read the other operands so and there is a pass
   // over g anyway or the products are large enough to pay for one
   bool pad = linear_pads_grad(dtype, out_dim) && in_dim % 8 == 0 && input_tail == nullptr && aligned16(weight) &&
