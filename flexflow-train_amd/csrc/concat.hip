@@ -53,7 +53,24 @@ __global__ __launch_bounds__(kConcatThreads) void concat_kernel(char *cat, Conca
   char *const p0 = part[lo] + (byte - offset[lo]);
   char *const c0 = cat + byte;
   int64_t const step = (int64_t)gridDim.y * rows_per_wg;
-  for (int64_t row = (int64_t)blockIdx.y * rows_per_wg + r_local; row < a.num_blocks; row += step) {
+  int64_t row = (int64_t)blockIdx.y * rows_per_wg + r_local;
+  if constexpr (MODE == kGather || MODE == kScatter) {
+    constexpr int kRows = 4;  // in flight
+    for (; row + (kRows - 1) * step < a.num_blocks; row += kRows * step) {
+      U v[kRows];
+#pragma unroll
+      for (int k = 0; k < kRows; k++) {
+        int64_t const r = row + k * step;
+        v[k] = *reinterpret_cast<U const *>(MODE == kGather ? p0 + r * part_row : c0 + r * cat_row);
+      }
+#pragma unroll
+      for (int k = 0; k < kRows; k++) {
+        int64_t const r = row + k * step;
+        *reinterpret_cast<U *>(MODE == kGather ? c0 + r * cat_row : p0 + r * part_row) = v[k];
+      }
+    }
+  }
+  for (; row < a.num_blocks; row += step) {
     U *const pp = reinterpret_cast<U *>(p0 + row * part_row);
     U *const cp = reinterpret_cast<U *>(c0 + row * cat_row);
     if (MODE == kGather) {
@@ -91,7 +108,17 @@ __global__ __launch_bounds__(kConcatThreads) void concat_kernel(char *cat, Conca
 template <typename U, int MODE>
 static hipError_t concat_launch(hipStream_t st, char *cat, ConcatArgs &a, int64_t window_bytes) {
   a.units_per_row = window_bytes / (int64_t)sizeof(U);
-  a.cols_per_wg = (int)(a.units_per_row < kConcatThreads ? a.units_per_row : kConcatThreads);
+  // The columns of a workgroup, of which it takes as many rows as it has threads for, so that as few of its
+  // threads as can be are left over (288 columns of 16 bytes, nine parts of 128 floats: 9 x 32, where 256 + 32 had
+  // every other workgroup work with 32 threads; [16384, 9 x 128] 39 us, with four rows of a thread in flight 30,
+  // a copy of that size 25).
+  a.cols_per_wg = 1;
+  int64_t most = 0;
+  for (int cols = (int)(a.units_per_row < kConcatThreads ? a.units_per_row : kConcatThreads); cols >= 1; cols--) {
+    // of 2^20 threads, those with an element
+    int64_t const used = a.units_per_row * (kConcatThreads / cols * cols) * 4096 / (ceil_div(a.units_per_row, cols) * cols);
+    if (used > most + most / 32) most = used, a.cols_per_wg = cols;  // (a few more for shorter pieces of a row are not worth it)
+  }
   int const rows_per_wg = kConcatThreads / a.cols_per_wg;
   int64_t const gx = ceil_div(a.units_per_row, a.cols_per_wg);
   int64_t gy = ceil_div(a.num_blocks, rows_per_wg);

@@ -90,3 +90,19 @@ def test_split_is_concat_read_the_other_way(ffk, oracle, dtype):
         ffk.split_backward([to_dev(d, torch, dtype) for d in douts], din, 1, accumulate=accumulate)
         want = oracle.concat_forward(douts, 1) + (old if accumulate else 0.0)
         assert np.array_equal(to_np(din), rnd(want.astype(np.float32)))
+
+
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 1023, 16385])
+@pytest.mark.parametrize("blocks", [[128] * 9, [128, 4, 512, 36], [1, 3, 2], [1028]])
+def test_columns_and_rows_of_a_workgroup(ffk, blocks, rows):
+    """Rows that leave threads of a workgroup over (288, 170, 6 and 257 units), and rows short of and past what one has in flight."""
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    parts = [torch.randn((rows, b), generator=gen, device="cuda") for b in blocks]
+    want = torch.cat(parts, 1)
+    buf = torch.full((want.numel() + 16,), 7.0, device="cuda")
+    out = buf[8:8 + want.numel()].view(want.shape)
+    ffk.concat_forward(parts, 1, out=out)
+    assert torch.equal(out, want) and bool((buf[:8] == 7.0).all()) and bool((buf[8 + want.numel():] == 7.0).all())
+    back = [torch.empty_like(p) for p in parts]
+    ffk.concat_backward(out, back, 1, accumulate=False)
+    assert all(torch.equal(a, b) for a, b in zip(back, parts))
