@@ -13,7 +13,7 @@
 //              ranking the keys of a step among their peers with the same digit
 //              by ballots, so equal digits keep their input order (stable) and
 //              the result does not depend on timing (no atomics decide a place).
-// Up to 1 048 576 lookups a pass is one or two launches: the scan moves into the scatter
+// Up to 1 048 576 lookups a pass is one to three launches: the scan moves into the scatter
 // kernel (every workgroup adds up the counts of the tiles before its own and the
 // totals of the digits below, straight from a table of at most 256 KB), and the
 // scatter counts the NEXT pass's digits of the keys it places, per destination
@@ -21,8 +21,8 @@
 // additions; the counts are gathered in LDS first, since under a skewed id
 // distribution thousands of a workgroup's keys share one counter), or beyond
 // 131 072 lookups a histogram launch does.  Digits are as
-// narrow as the number of passes allows (three of 7 bits for a million rows).  Up
-// to 4096 lookups the whole sort is one workgroup and one launch.
+// narrow as the number of passes allows, and up to ten bits wide where that saves a
+// pass (radix_sort_plan).  Up to 4096 lookups the whole sort is one workgroup and one launch.
 // The first pass reads the caller's index tensor directly (int32 or int64,
 // ids outside the table become the key `invalid_key`, which sorts behind every
 // row) and numbers the lookups itself, so no pass exists only to build keys.
@@ -181,13 +181,15 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
 // the ranking under the table's loads, and digits no wider than the passes need.
 // Sort of 65 536 token ids below 50 257: 23 -> 18 us (tiles of 2048 keys and four
 // waves before); 524 288 ids below a million: 63 -> 50 us (three launches a pass
-// before); 1000 ids: three launches and 20 us less for the whole gradient.
+// before), 40 in two passes of ten bits with a scan launch each; 1000 ids: three launches and 20 us less for the whole gradient.
 // ---------------------------------------------------------------------------
 constexpr int kSortFusedThreads = 1024;
 constexpr int kSortFusedWaves = kSortFusedThreads / 64;
 constexpr int kSortAheadTiles = 128;  // up to these a scatter counts the next pass's digits
 constexpr int kSortFusedTiles = 256;
 constexpr int kSortFusedItems = 4;  // the most keys per thread
+constexpr int kSortWideRadix = 1024;
+constexpr int kSortWideTiles = 16;
 
 // A step's lanes with this lane's digit (all of them take part; `valid` lanes only are counted).
 __device__ __forceinline__ uint64_t sort_peers(bool valid, uint32_t digit, int bits) {
@@ -221,8 +223,9 @@ __device__ __forceinline__ void sort_rank_wave(uint32_t const (&digit)[ITEMS], b
   }
 }
 
-// Exclusive prefix sum of v over the threads below `bins` (at most 256; the others pass 0).
+// Exclusive prefix sum of v over the threads below `bins` (at most BINS; the others pass 0).
 // Every thread calls it; it synchronises the workgroup once, on the way.
+template <int BINS>
 __device__ __forceinline__ uint32_t sort_scan_bins(uint32_t v, int t, int lane, uint32_t *wsum) {
   uint32_t incl = v;
 #pragma unroll
@@ -230,24 +233,24 @@ __device__ __forceinline__ uint32_t sort_scan_bins(uint32_t v, int t, int lane, 
     uint32_t const up = __shfl_up(incl, off, 64);
     if (lane >= off) incl += up;
   }
-  if (lane == 63 && t < kSortRadix) wsum[t >> 6] = incl;
+  if (lane == 63 && t < BINS) wsum[t >> 6] = incl;
   __syncthreads();
   uint32_t excl = incl - v;
 #pragma unroll
-  for (int w = 0; w < kSortRadix / 64; w++) excl += w < (t >> 6) && t < kSortRadix ? wsum[w] : 0u;
+  for (int w = 0; w < BINS / 64; w++) excl += w < (t >> 6) && t < BINS ? wsum[w] : 0u;
   return excl;
 }
 
-template <typename IT, bool FIRST>
+template <typename IT, bool FIRST, int BINS>
 __global__ __launch_bounds__(kSortFusedThreads) void radix_hist_fused_kernel(IT const *__restrict__ idx,
                                                                             uint32_t const *__restrict__ keys_in,
                                                                             uint32_t *__restrict__ table0,
                                                                             uint32_t *__restrict__ table1, int64_t n,
                                                                             int items, int shift, int bits,
                                                                             int64_t num_entries) {
-  __shared__ uint32_t cnt[kSortRadix];
+  __shared__ uint32_t cnt[BINS];
   int const t = threadIdx.x, bins = 1 << bits;
-  if (t < kSortRadix) cnt[t] = 0;
+  if (t < BINS) cnt[t] = 0;
   __syncthreads();
   int64_t const base = (int64_t)blockIdx.x * kSortFusedThreads * items;
 #pragma unroll
@@ -265,22 +268,54 @@ __global__ __launch_bounds__(kSortFusedThreads) void radix_hist_fused_kernel(IT 
   }
 }
 
+// table[tile][digit], counts, become the number of the digit's keys in the tiles before; totals[digit].
+// A workgroup takes 64 digits, sixteen threads to each.
+__global__ __launch_bounds__(kSortFusedThreads) void radix_scan_fused_kernel(uint32_t *table, uint32_t *__restrict__ totals,
+                                                                            int ntiles, int bits) {
+  constexpr int kParts = kSortFusedThreads / 64, kEach = kSortFusedTiles / kParts;
+  __shared__ uint32_t part_sum[kParts][64];
+  int const lane = threadIdx.x & 63, part = threadIdx.x >> 6, d = blockIdx.x * 64 + lane;
+  uint32_t v[kEach], sum = 0;
+#pragma unroll
+  for (int k = 0; k < kEach; k++) {
+    int const tile = part * kEach + k;
+    v[k] = tile < ntiles ? table[((int64_t)tile << bits) + d] : 0u;
+  }
+#pragma unroll
+  for (int k = 0; k < kEach; k++) sum += v[k];
+  part_sum[part][lane] = sum;
+  __syncthreads();
+  uint32_t run = 0;
+#pragma unroll
+  for (int q = 0; q < kParts; q++) run += q < part ? part_sum[q][lane] : 0u;
+#pragma unroll
+  for (int k = 0; k < kEach; k++) {
+    int const tile = part * kEach + k;
+    if (tile < ntiles) table[((int64_t)tile << bits) + d] = run;
+    run += v[k];
+  }
+  if (part == kParts - 1) totals[d] = run;
+}
+
 // table: this pass's counts; next: the next pass's table (nullptr on the last pass), added
 // into here; after: the table of the pass after that (nullptr if none), cleared here.
+// SCANNED: radix_scan_fused_kernel has been over the table, its totals behind it.
 // Dynamic LDS: the workgroup's share of the next table, 16-bit counters in pairs (a workgroup
 // counts its own keys there, at most 4096; only up to kSortAheadTiles tiles).
-template <typename IT, bool FIRST, int ITEMS>
+template <typename IT, bool FIRST, int ITEMS, int BINS, bool SCANNED>
 __global__ __launch_bounds__(kSortFusedThreads) void radix_scatter_fused_kernel(
     IT const *__restrict__ idx, uint32_t const *__restrict__ keys_in, uint32_t const *__restrict__ vals_in,
     uint32_t *__restrict__ keys_out, uint32_t *__restrict__ vals_out, uint32_t const *__restrict__ table,
     uint32_t *__restrict__ next, uint32_t *__restrict__ after, int64_t n, int ntiles, int shift, int bits,
     int64_t num_entries) {
   constexpr int TILE = kSortFusedThreads * ITEMS;
+  // pairs leave through LDS in order, where that makes runs of them
+  constexpr bool kOrdered = ITEMS > 1 && BINS == kSortRadix;
   extern __shared__ uint32_t next_cnt[];
-  __shared__ uint32_t wave_off[kSortFusedWaves][kSortRadix];
+  __shared__ uint32_t wave_off[kSortFusedWaves][BINS];
   __shared__ uint32_t part_all[kSortFusedThreads], part_before[kSortFusedThreads];
-  __shared__ uint32_t wsum[kSortRadix / 64], delta[ITEMS > 1 ? kSortRadix : 1];
-  __shared__ uint32_t ks[ITEMS > 1 ? TILE : 1], vs[ITEMS > 1 ? TILE : 1];
+  __shared__ uint32_t wsum[BINS / 64], delta[kOrdered ? BINS : 1];
+  __shared__ uint32_t ks[kOrdered ? TILE : 1], vs[kOrdered ? TILE : 1];
   int const t = threadIdx.x, lane = t & 63, wave = t >> 6;
   int const bins = 1 << bits, mask = bins - 1;
   int const next_words = next != nullptr ? (ntiles * bins + 1) / 2 : 0;
@@ -301,7 +336,10 @@ __global__ __launch_bounds__(kSortFusedThreads) void radix_scatter_fused_kernel(
     }
   }
   // the keys with digit d in the tiles before this one, and in all tiles: 1024 / bins threads a digit
-  {
+  if constexpr (SCANNED) {
+    part_before[t] = t < bins ? table[((int64_t)blockIdx.x << bits) + t] : 0u;
+    part_all[t] = t < bins ? table[((int64_t)ntiles << bits) + t] : 0u;
+  } else {
     int const d = t & mask, part = t >> bits, parts = kSortFusedThreads >> bits, tile = blockIdx.x;
     uint32_t before_tiles = 0, all_tiles = 0;
     for (int t0 = part; t0 < ntiles; t0 += 16 * parts) {
@@ -329,8 +367,8 @@ __global__ __launch_bounds__(kSortFusedThreads) void radix_scatter_fused_kernel(
       before += part_before[p];
     }
   }
-  uint32_t const smaller = sort_scan_bins(all, t, lane, wsum);
-  if constexpr (ITEMS == 1) {
+  uint32_t const smaller = sort_scan_bins<BINS>(all, t, lane, wsum);
+  if constexpr (!kOrdered) {
     if (t < bins) {
       uint32_t run = smaller + before;
 #pragma unroll
@@ -364,7 +402,7 @@ __global__ __launch_bounds__(kSortFusedThreads) void radix_scatter_fused_kernel(
 #pragma unroll
       for (int w = 0; w < kSortFusedWaves; w++) mine += wave_off[w][t];
     }
-    uint32_t const local = sort_scan_bins(mine, t, lane, wsum);
+    uint32_t const local = sort_scan_bins<BINS>(mine, t, lane, wsum);
     if (t < bins) {
       delta[t] = smaller + before - local;  // from a pair's place in LDS to its place in the output
       uint32_t run = local;
@@ -408,14 +446,14 @@ __global__ __launch_bounds__(kSortFusedThreads) void radix_scatter_fused_kernel(
 }
 
 // Up to 4096 lookups: the whole sort in one workgroup, pairs handed round through LDS.
-template <typename IT, int ITEMS>
+template <typename IT, int ITEMS, int BINS>
 __global__ __launch_bounds__(kSortFusedThreads) void radix_sort_block_kernel(IT const *__restrict__ idx,
                                                                             uint32_t *__restrict__ keys_out,
                                                                             uint32_t *__restrict__ vals_out, int n,
                                                                             int passes, int bits, int64_t num_entries) {
   __shared__ uint32_t ks[kSortFusedThreads * ITEMS], vs[kSortFusedThreads * ITEMS];
-  __shared__ uint32_t wave_off[kSortFusedWaves][kSortRadix];
-  __shared__ uint32_t wsum[kSortRadix / 64];
+  __shared__ uint32_t wave_off[kSortFusedWaves][BINS];
+  __shared__ uint32_t wsum[BINS / 64];
   int const t = threadIdx.x, lane = t & 63, wave = t >> 6;
   int const bins = 1 << bits, mask = bins - 1;
   int const first = wave * (64 * ITEMS) + lane;
@@ -439,7 +477,7 @@ __global__ __launch_bounds__(kSortFusedThreads) void radix_sort_block_kernel(IT 
 #pragma unroll
       for (int w = 0; w < kSortFusedWaves; w++) all += wave_off[w][t];
     }
-    uint32_t run = sort_scan_bins(all, t, lane, wsum);
+    uint32_t run = sort_scan_bins<BINS>(all, t, lane, wsum);
     if (t < bins) {
 #pragma unroll
       for (int w = 0; w < kSortFusedWaves; w++) {
@@ -481,27 +519,39 @@ struct RadixSortPlan {
   int bits;            // of a digit
   int ntiles;
   int items;           // fused: keys per thread
-  bool fused;          // one launch per pass, or (one tile) one launch in all
-  size_t table_bytes;  // fused: one [ntiles][bins] table per pass; otherwise one [256][ntiles] table, then the digit totals [passes][256]
+  bool fused;          // the launches below, or (one tile) one launch in all
+  bool wide;           // fused: digits of up to 10 bits instead of 8
+  bool scanned;        // fused: a scan launch between a pass's histogram and its scatter
+  size_t table_bytes;  // fused: one [ntiles][bins] table per pass (scanned: one table and its totals); otherwise one [256][ntiles] table, then the digit totals [passes][256]
 };
 
 static inline RadixSortPlan radix_sort_plan(int64_t n, unsigned key_bits) {
-  RadixSortPlan p;
+  RadixSortPlan p = {};
   p.passes = (int)((key_bits + 7) / 8);
   p.bits = 8;
   // Fused while a CU each holds every tile: the table a workgroup reads grows with their number.  More
   // keys than that take the three launches a pass.
   p.fused = n <= (int64_t)kSortFusedTiles * kSortFusedThreads * kSortFusedItems;
-  p.items = 0;
   if (p.fused) {
-    p.bits = (int)((key_bits + p.passes - 1) / p.passes);
     // one tile as long as four keys per thread cover everything; then as few keys per thread as the tile limit allows
     p.items = n <= kSortFusedThreads ? 1 : kSortFusedItems;
     if (n > (int64_t)kSortFusedThreads * kSortFusedItems) {
       p.items = n <= (int64_t)kSortAheadTiles * kSortFusedThreads ? 1 : n <= (int64_t)kSortFusedTiles * kSortFusedThreads * 2 ? 2 : 4;
     }
     p.ntiles = (int)ceil_div(n, (int64_t)kSortFusedThreads * p.items);
-    p.table_bytes = ((size_t)p.ntiles << p.bits) * (size_t)p.passes * sizeof(uint32_t);
+    // Digits of ten bits where they save a pass (a million rows, 20 bits: two instead of three): up to 16
+    // tiles the table is still small enough for every workgroup to add up (6089 ids below 71 797 29 -> 25 us
+    // with gather and walk; at 28 tiles the counts ahead cost more, 42 -> 47 us for 28 474 ids); beyond 131 072
+    // lookups, where each pass has a histogram launch of its own, a third launch adds it up once (524 288 ids
+    // below a million: two passes of 18-21 us instead of three of 17).  In between, neither pays.
+    int const wide_passes = (int)((key_bits + 9) / 10);
+    p.wide = wide_passes < p.passes && (p.ntiles <= kSortWideTiles || p.items > 1);
+    if (p.wide) p.passes = wide_passes;
+    p.scanned = p.wide && p.items > 1 && p.ntiles > 1;
+    p.bits = (int)((key_bits + p.passes - 1) / p.passes);
+    if (p.scanned && p.bits < 6) p.bits = 6;  // the scan's workgroups take 64 digits
+    p.table_bytes = p.scanned ? ((size_t)(p.ntiles + 1) << p.bits) * sizeof(uint32_t)
+                              : ((size_t)p.ntiles << p.bits) * (size_t)p.passes * sizeof(uint32_t);
   } else {
     p.ntiles = (int)ceil_div(n, kSortTile);
     p.table_bytes = (size_t)kSortRadix * ((size_t)p.ntiles + (size_t)p.passes) * sizeof(uint32_t);
@@ -509,7 +559,7 @@ static inline RadixSortPlan radix_sort_plan(int64_t n, unsigned key_bits) {
   return p;
 }
 
-template <typename IT, int ITEMS>
+template <typename IT, int ITEMS, int BINS>
 static inline hipError_t radix_sort_fused(hipStream_t st, IT const *idx, int64_t n, int64_t num_entries,
                                           RadixSortPlan const &plan, uint32_t *keys_a, uint32_t *keys_b,
                                           uint32_t *vals_a, uint32_t *vals_b, uint32_t *table,
@@ -519,21 +569,25 @@ static inline hipError_t radix_sort_fused(hipStream_t st, IT const *idx, int64_t
   // Counting the next pass's digits while placing costs an atomic for nearly every (tile, digit)
   // pair of every workgroup: cheaper than a launch up to one key per thread, several times
   // dearer beyond (524 288 keys: 15-21 us a pass against 5 for the launch and 12 without the counting).
-  constexpr bool kCountAhead = ITEMS == 1;
-  auto tab = [&](int pass) -> uint32_t * { return pass < plan.passes ? table + (size_t)pass * tsz : nullptr; };
+  constexpr bool kCountAhead = ITEMS == 1, kScanned = ITEMS > 1 && BINS > kSortRadix;
+  auto tab = [&](int pass) -> uint32_t * { return pass < plan.passes ? table + (kScanned ? 0 : (size_t)pass * tsz) : nullptr; };
   auto ahead = [&](int pass) -> uint32_t * { return kCountAhead ? tab(pass) : nullptr; };
   uint32_t *kin = nullptr, *vin = nullptr, *kout = keys_a, *vout = vals_a;
   for (int pass = 0; pass < plan.passes; pass++) {
     if (pass == 0) {
-      radix_hist_fused_kernel<IT, true><<<blocks, kSortFusedThreads, 0, st>>>(idx, nullptr, tab(0), ahead(1), n, ITEMS,
-                                                                             0, plan.bits, num_entries);
+      radix_hist_fused_kernel<IT, true, BINS><<<blocks, kSortFusedThreads, 0, st>>>(
+          idx, nullptr, tab(0), ahead(1), n, ITEMS, 0, plan.bits, num_entries);
     } else if (!kCountAhead) {
-      radix_hist_fused_kernel<IT, false><<<blocks, kSortFusedThreads, 0, st>>>(
+      radix_hist_fused_kernel<IT, false, BINS><<<blocks, kSortFusedThreads, 0, st>>>(
           idx, kin, tab(pass), nullptr, n, ITEMS, plan.bits * pass, plan.bits, num_entries);
     }
-    auto kern = pass == 0 ? radix_scatter_fused_kernel<IT, true, ITEMS> : radix_scatter_fused_kernel<IT, false, ITEMS>;
+    if (kScanned) {
+      radix_scan_fused_kernel<<<(1u << plan.bits) / 64, kSortFusedThreads, 0, st>>>(table, table + tsz, plan.ntiles, plan.bits);
+    }
+    auto kern = pass == 0 ? radix_scatter_fused_kernel<IT, true, ITEMS, BINS, kScanned>
+                          : radix_scatter_fused_kernel<IT, false, ITEMS, BINS, kScanned>;
     size_t const lds = ahead(pass + 1) != nullptr ? (tsz + 1) / 2 * sizeof(uint32_t) : 0;
-    if (lds > 32 * 1024) {  // with the static part, more than a launch may ask for by default
+    if (lds > (BINS > kSortRadix ? 0 : 32 * 1024)) {  // with the static part, more than a launch may ask for by default
       hipError_t const e = hipFuncSetAttribute(reinterpret_cast<void const *>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       if (e != hipSuccess) return e;
@@ -562,20 +616,19 @@ static inline hipError_t radix_sort_lookups(hipStream_t st, IT const *idx, int64
                                             uint32_t **keys_sorted, uint32_t **vals_sorted) {
   if (plan.fused) {
     if (plan.ntiles == 1) {
-      if (plan.items == 1) {
-        radix_sort_block_kernel<IT, 1><<<1, kSortFusedThreads, 0, st>>>(idx, keys_a, vals_a, (int)n, plan.passes,
-                                                                        plan.bits, num_entries);
-      } else {
-        radix_sort_block_kernel<IT, kSortFusedItems><<<1, kSortFusedThreads, 0, st>>>(
-            idx, keys_a, vals_a, (int)n, plan.passes, plan.bits, num_entries);
-      }
+      auto kern = plan.items == 1 ? (plan.wide ? radix_sort_block_kernel<IT, 1, kSortWideRadix> : radix_sort_block_kernel<IT, 1, kSortRadix>)
+                                  : (plan.wide ? radix_sort_block_kernel<IT, kSortFusedItems, kSortWideRadix>
+                                               : radix_sort_block_kernel<IT, kSortFusedItems, kSortRadix>);
+      kern<<<1, kSortFusedThreads, 0, st>>>(idx, keys_a, vals_a, (int)n, plan.passes, plan.bits, num_entries);
       *keys_sorted = keys_a;
       *vals_sorted = vals_a;
       return hipGetLastError();
     }
-#define FFK_SORT_FUSED(ITEMS_)                                                                              \
-  return radix_sort_fused<IT, ITEMS_>(st, idx, n, num_entries, plan, keys_a, keys_b, vals_a, vals_b, table, \
-                                      keys_sorted, vals_sorted)
+#define FFK_SORT_FUSED(ITEMS_)                                                                                      \
+  return plan.wide ? radix_sort_fused<IT, ITEMS_, kSortWideRadix>(st, idx, n, num_entries, plan, keys_a, keys_b, vals_a, \
+                                                                  vals_b, table, keys_sorted, vals_sorted)          \
+                   : radix_sort_fused<IT, ITEMS_, kSortRadix>(st, idx, n, num_entries, plan, keys_a, keys_b, vals_a, vals_b, \
+                                                              table, keys_sorted, vals_sorted)
     if (plan.items == 1) FFK_SORT_FUSED(1);
     if (plan.items == 2) FFK_SORT_FUSED(2);
     FFK_SORT_FUSED(4);
