@@ -11,6 +11,7 @@
 // Indices outside [0, num_entries) are skipped (the reference reads or writes
 // out of bounds for them).
 #include "ffk_common.h"
+#include "embedding_walk.h"
 #include "radix_sort.h"
 #include <algorithm>
 #include <cstdlib>
@@ -372,7 +373,8 @@ __global__ __launch_bounds__(256) void embedding_bwd_sorted_kernel(
   }
 }
 
-// The non-deterministic sorted path: a wave walks `chunk` consecutive sorted positions, a
+// The non-deterministic sorted path of tensors of 4 GB and more, which the walk's 32-bit offsets
+// (embedding_walk.h) do not reach: a wave walks `chunk` consecutive sorted positions, a
 // workgroup sixteen such chunks.  Walkers add runs that lie inside their chunk straight to memory;
 // the partial sums of runs that cross a walker border meet in LDS and are merged by the workgroup,
 // so only runs that cross a WORKGROUP border reach memory as atomics.  A row looked up
@@ -655,6 +657,13 @@ static int emb_backward(hipStream_t st, void const *indices, void const *dy,
       else FFK_EMB_SORTED(16, 1);
 #undef FFK_EMB_SORTED
       FFK_CHECK_LAUNCH();
+      return FFK_OK;
+    }
+    // 32-bit byte offsets reach all of both tensors
+    if ((uint64_t)num_entries * dim * 4 <= kWalkNowhere && (uint64_t)num_bags * dim * sizeof(GT) <= kWalkNowhere) {
+      WalkArgs const a = {keys_out, vals_out, lookups, 0, (int)bag, (int)dim, (uint32_t)num_entries, scale,
+                          (uint32_t)(num_bags * dim * (int64_t)sizeof(GT)), (uint32_t)(num_entries * dim * 4)};
+      FFK_HIP(embedding_walk<GT>(st, a, G, dw));
       return FFK_OK;
     }
     // Longer chunks mean fewer border partials and fewer atomics on hot rows; 8192 walkers are every
