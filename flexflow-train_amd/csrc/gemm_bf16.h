@@ -169,11 +169,10 @@ struct GemmGroupArgs {
 //     the output, and do not store what their neighbours store.  No load needs a bound but those of a
 //     ragged last k-tile, whose lanes past K ask for an offset past the descriptor's bound and get
 //     zeros; the steady loop stops one tile earlier and is that of whole tiles.
-//   kEdgeBounded (any M, N): every load has a descriptor of its own, bounded by what is left of the
-//     operand behind its first row; what lies past it arrives as zeros, garbage in columns past M or N
-//     only reaches outputs that are not stored.  The descriptors cost 20% of the loop of a 128x128
-//     tile (4095 x 1024 over 4096: 39.0 us, 32.6 with 4096 rows) and nothing noticeable where a
-//     64x64 tile waits anyway.
+//   kEdgeBounded (any M, N): lanes whose rows or columns lie past the operand ask for an offset past the
+//     descriptor's bound and get zeros, for which each load of a K-contiguous panel keeps lane offsets of
+//     its own.  (A descriptor per load, bounded by what is left of the operand, took 20% of the loop of a
+//     128x128 tile, 4095 x 1024 over 4096: 39.0 us, 32.6 with 4096 rows, and 8% of a 64x64 one.)
 // KG: groups of waves that each take a part of the reduction (with LDS stages of their own) and add
 // up their accumulators at the end.  A 64x64 tile is 4 MFMAs a wave and k-tile, which a barrier, an
 // LDS round trip and the MFMAs' own dependence stretch to some 600 cycles; a second group fills them
@@ -240,7 +239,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   int const first_m = tm * BM, first_n = tn * BN;
   // (an operand whose contiguous index is M may be padded to whole 16-byte chunks: rows past M are
   // loaded then, and not stored)
-  int const M_loads = TA && EDGE ? (M + 7) & ~7 : M, K_loads = !TA && EDGE ? (K + 7) & ~7 : K;
+  int const M_loads = TA && EDGE ? (M + 7) & ~7 : M;
   int const m0 = EDGE == kEdgeOverlap ? min(first_m, M_loads - BM) : first_m, n0 = EDGE == kEdgeOverlap ? min(first_n, N - BN) : first_n;
   // first k-tile of this workgroup, or of this group of waves
   int const kt0 = KG == 1 ? split * k_tiles_per_split : kg * (((K + BK - 1) / BK + KG - 1) / KG);
@@ -283,22 +282,33 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
     }
   }
   int const KT_all = EDGE ? (K + BK - 1) / BK : K / BK;  // k-tiles of the whole reduction
-  // the same offsets for the last k-tile (EDGE): lanes past K ask for what no descriptor covers
-  unsigned voff_a_last = voff_a, voff_b_last = voff_b;
-  if constexpr (EDGE) {
-    int const c = wave * 64 + lane, row = c / CPRK;
-    int const k = ((c % CPRK) ^ ((row / RPW) & (CPRK - 1))) * 8;
-    bool const past = k >= K - (KT_all - 1) * BK;
-    if (!TA && past) voff_a_last = 0x80000000u;
-    if (!TBL && past) voff_b_last = 0x80000000u;
-  }
   int64_t const step_a = TA ? (int64_t)(NT * 8 / BM) * lda : (int64_t)ROWS_PER_LOAD_KC * lda;
   int64_t const step_b = TBL ? (int64_t)(NT * 8 / BN) * ldb : (int64_t)ROWS_PER_LOAD_KC * ldb;
   bf16 const *const panel_a = TA ? A + m0 : A + (int64_t)m0 * lda;
   bf16 const *const panel_b = TBL ? B + n0 : B + (int64_t)n0 * ldb;
-  // one past the last element of the operand that a workgroup may read, from its panel's start
-  int64_t const end_a = EDGE != kEdgeBounded ? 0 : TA ? (int64_t)(K - 1) * lda + (M_loads - m0) : (int64_t)(min(BM, M - m0) - 1) * lda + K_loads;
-  int64_t const end_b = EDGE != kEdgeBounded ? 0 : TBL ? (int64_t)(K - 1) * ldb + (N - n0) : (int64_t)(min(BN, N - n0) - 1) * ldb + K;
+  // (kEdgeBounded) lanes whose rows or columns lie past the operand ask for what no descriptor covers and get
+  // zeros: of a K-contiguous panel each load has rows of its own, of one lying [BK][cols] all have the lane's columns
+  constexpr bool ROWS_A = EDGE == kEdgeBounded && !TA, ROWS_B = EDGE == kEdgeBounded && !TBL;
+  unsigned off_a[ROWS_A ? A_LOADS : 1], off_b[ROWS_B ? B_LOADS : 1];
+  {
+    int const c = wave * 64 + lane;
+    auto columns_from = [&](int cols) {  // of the lane's pieces (see the swizzle above)
+      int const krow = c / (cols / 8), pc = c % (cols / 8);
+      return (((pc >> 2) ^ tr_swizzle(krow, cols)) << 5) | ((pc & 3) << 3);
+    };
+#pragma unroll
+    for (int q = 0; q < (ROWS_A ? A_LOADS : 1); q++) {
+      bool const there = EDGE != kEdgeBounded || (TA ? m0 + columns_from(BM) < M_loads : m0 + c / CPRK + q * ROWS_PER_LOAD_KC < M);
+      off_a[q] = there ? voff_a : 0x80000000u;
+    }
+#pragma unroll
+    for (int q = 0; q < (ROWS_B ? B_LOADS : 1); q++) {
+      bool const there = EDGE != kEdgeBounded || (TBL ? n0 + columns_from(BN) < N : n0 + c / CPRK + q * ROWS_PER_LOAD_KC < N);
+      off_b[q] = there ? voff_b : 0x80000000u;
+    }
+  }
+  auto lane_a = [&](int q) __attribute__((always_inline)) { return off_a[ROWS_A ? q : 0]; };
+  auto lane_b = [&](int q) __attribute__((always_inline)) { return off_b[ROWS_B ? q : 0]; };
 
   // LDS destinations of the direct loads are scalar byte addresses: base + stage + chunk row
   bf16 *const stages = smem + (KG == 1 ? 0 : kg * (STAGES * STAGE_ELEMS));
@@ -310,63 +320,40 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   auto issue_some = [&](int kt, int stage, int first, int count, bool maybe_last) __attribute__((always_inline)) {
     unsigned const sa = smem_addr + (unsigned)(stage * STAGE_ELEMS) * 2u;
     unsigned const sb = sa + (unsigned)A_ELEMS * 2u;
-    if constexpr (EDGE == kEdgeOverlap) {
-      if (maybe_last && kt0 + kt == KT_all - 1 && K % BK != 0) {  // uniform over the launch's workgroups
+    unsigned const bound = EDGE == kEdgeBounded ? 0x80000000u : 0xffffffffu;
+    if constexpr (EDGE != kEdgeNone) {
+      if (maybe_last && kt0 + kt >= KT_all - 1 && (K % BK != 0 || kt0 + kt >= KT_all)) {  // uniform over the wave
         i32x4 const ra = buffer_resource(panel_a + (TA ? (int64_t)(kt0 + kt) * BK * lda : (int64_t)(kt0 + kt) * BK), 0x80000000u);
         i32x4 const rb = buffer_resource(panel_b + (TBL ? (int64_t)(kt0 + kt) * BK * ldb : (int64_t)(kt0 + kt) * BK), 0x80000000u);
-        int const left = K - (KT_all - 1) * BK;  // k's of this tile
+        // k's of this tile, none for a group of waves that ran out of k-tiles
+        int const left = kt0 + kt >= KT_all ? 0 : K - (KT_all - 1) * BK;
         int const c = wave * 64 + lane;
+        bool const past = ((c % CPRK) ^ ((c / CPRK / RPW) & (CPRK - 1))) * 8 >= left;  // this lane's k's of a K-contiguous panel
 #pragma unroll
         for (int q = 0; q < LPT; q++) {
           if (q < first || q >= first + count) continue;
           if (q < A_LOADS) {
-            unsigned const va = !TA ? voff_a_last : c / (BM / 8) + q * (NT * 8 / BM) < left ? voff_a : 0x80000000u;
-            lds_dma16(ra, va, (unsigned)(q * step_a) * 2u, sa + (unsigned)(q * NW + wave_s) * 1024u);
+            bool const there = !TA ? !past : c / (BM / 8) + q * (NT * 8 / BM) < left;
+            lds_dma16(ra, there ? lane_a(q) : 0x80000000u, (unsigned)(q * step_a) * 2u, sa + (unsigned)(q * NW + wave_s) * 1024u);
           } else {
             int const i = q - A_LOADS;
-            unsigned const vb = !TBL ? voff_b_last : c / (BN / 8) + i * (NT * 8 / BN) < left ? voff_b : 0x80000000u;
-            lds_dma16(rb, vb, (unsigned)(i * step_b) * 2u, sb + (unsigned)(i * NW + wave_s) * 1024u);
+            bool const there = !TBL ? !past : c / (BN / 8) + i * (NT * 8 / BN) < left;
+            lds_dma16(rb, there ? lane_b(i) : 0x80000000u, (unsigned)(i * step_b) * 2u, sb + (unsigned)(i * NW + wave_s) * 1024u);
           }
         }
         return;
       }
     }
-    if constexpr (EDGE == kEdgeBounded) {
-      bool const last = maybe_last && kt0 + kt >= KT_all - 1;
-      unsigned va = !TA && last ? voff_a_last : voff_a, vb = !TBL && last ? voff_b_last : voff_b;
-      if (KG > 1 && maybe_last && kt0 + kt >= KT_all) va = vb = 0x80000000u;  // a group that ran out of k-tiles: zeros
-      int64_t const at_a = TA ? (int64_t)(kt0 + kt) * BK * lda : (int64_t)(kt0 + kt) * BK;
-      int64_t const at_b = TBL ? (int64_t)(kt0 + kt) * BK * ldb : (int64_t)(kt0 + kt) * BK;
-      // a descriptor per load: its bound is what is left of the operand behind the load's first row
-      // (the row offset must not go into the scalar offset: a scalar offset past the bound wraps)
-      auto bytes_left = [](int64_t elems) {
-        int64_t const b = elems * 2;
-        return (unsigned)(b < 0 ? 0 : b > 0x7fffffff ? 0x7fffffff : b);
-      };
-#pragma unroll
-      for (int q = 0; q < LPT; q++) {
-        if (q < first || q >= first + count) continue;
-        if (q < A_LOADS) {
-          int64_t const at = at_a + q * step_a;
-          lds_dma16(buffer_resource(panel_a + at, bytes_left(end_a - at)), va, 0u, sa + (unsigned)(q * NW + wave_s) * 1024u);
-        } else {
-          int const i = q - A_LOADS;
-          int64_t const at = at_b + i * step_b;
-          lds_dma16(buffer_resource(panel_b + at, bytes_left(end_b - at)), vb, 0u, sb + (unsigned)(i * NW + wave_s) * 1024u);
-        }
-      }
-      return;
-    }
-    i32x4 const ra = buffer_resource(panel_a + (TA ? (int64_t)(kt0 + kt) * BK * lda : (int64_t)(kt0 + kt) * BK));
-    i32x4 const rb = buffer_resource(panel_b + (TBL ? (int64_t)(kt0 + kt) * BK * ldb : (int64_t)(kt0 + kt) * BK));
+    i32x4 const ra = buffer_resource(panel_a + (TA ? (int64_t)(kt0 + kt) * BK * lda : (int64_t)(kt0 + kt) * BK), bound);
+    i32x4 const rb = buffer_resource(panel_b + (TBL ? (int64_t)(kt0 + kt) * BK * ldb : (int64_t)(kt0 + kt) * BK), bound);
 #pragma unroll
     for (int q = 0; q < LPT; q++) {
       if (q < first || q >= first + count) continue;
       if (q < A_LOADS) {
-        lds_dma16(ra, voff_a, (unsigned)(q * step_a) * 2u, sa + (unsigned)(q * NW + wave_s) * 1024u);
+        lds_dma16(ra, lane_a(q), (unsigned)(q * step_a) * 2u, sa + (unsigned)(q * NW + wave_s) * 1024u);
       } else {
         int const i = q - A_LOADS;
-        lds_dma16(rb, voff_b, (unsigned)(i * step_b) * 2u, sb + (unsigned)(i * NW + wave_s) * 1024u);
+        lds_dma16(rb, lane_b(i), (unsigned)(i * step_b) * 2u, sb + (unsigned)(i * NW + wave_s) * 1024u);
       }
     }
   };
