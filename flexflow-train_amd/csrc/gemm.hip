@@ -369,7 +369,7 @@ bool gemm_tail_supported(int dtype, bool ta, bool tb, int64_t M, int64_t N, int6
     return !(ep.tail_any_size && ep.tail == GemmEpilogue::kTailGeluDropout);
   }
   if (!ep.tail_any_size || variant != 0 || N % 8 != 0 || !aligned16(C) || !edge_operands_ok(lda, ldb)) return false;
-  bool const splits = gemm_splits_reduction((int)M, (int)N, (int)K, ep);
+  bool const splits = gemm_split_tile((int)M, (int)N, (int)K, ep) != 0;
   if (ep.tail == GemmEpilogue::kTailGeluDropout) return splits;
   return splits || sums || (M >= 128 && N >= 128);
 }

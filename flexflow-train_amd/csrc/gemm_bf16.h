@@ -177,6 +177,11 @@ struct GemmGroupArgs {
 // up their accumulators at the end.  A 64x64 tile is 4 MFMAs a wave and k-tile, which a barrier, an
 // LDS round trip and the MFMAs' own dependence stretch to some 600 cycles; a second group fills them
 // where there are too few tiles for a second workgroup per CU.
+// With four groups of one wave a 32x32 tile, no barrier stands in the loop.  Where the tiles leave CUs idle,
+// a workgroup's time is the bytes it reads over what its LDS stages can have in flight for the some 800 ns
+// they take to come: a quarter of the tile reads half the bytes and there are four times the workgroups
+// (405 x 512 over 2048 8.8 -> 6.3 us, 63 x 768 over 3072 10.2 -> 6.7, 756 x 256 over 768 5.5 -> 4.5), and the
+// output's operators are spread over all of its waves (96 x 256 over 128 with GELU and dropout 7.3 -> 4.9).
 template <int BM, int BN, int WM, int WN, int BK, int STAGES, int PF, bool TA, bool TB, int TAIL = 0,
           bool GROUP = false, int EDGE = kEdgeNone, int KG = 1>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pipe_kernel(
@@ -203,6 +208,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   // applies the epilogue.
   constexpr int NW = (BM / WM) * (BN / WN);
   constexpr int NT = NW * 64;
+  // a group is one wave: nobody but the wave itself reads its stages, and no barrier stands in its loop
+  constexpr bool ALONE = NW == 1 && KG > 1;
   constexpr int TM = WM / 32, TN = WN / 32;
   constexpr bool TBL = (TB == false);  // B tile lies as [BK][BN]
   constexpr int A_ELEMS = BM * BK, B_ELEMS = BN * BK;
@@ -251,8 +258,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   // K-contiguous tile [rows][BK]: physical chunk pc of a row holds logical
   // chunk pc ^ ((row / RPW) % CPRK).  Tile lying as [BK][cols]: the 64-byte
   // segment s of row k sits at segment s ^ (k % 4) (with 64 columns, whose rows are
-  // half a bank window, at s ^ ((k / 2) % 2)).
-  auto tr_swizzle = [](int krow, int cols) { return cols == 64 ? (krow >> 1) & 1 : krow & 3; };
+  // half a bank window, at s ^ ((k / 2) % 2); with 32 there is one).
+  auto tr_swizzle = [](int krow, int cols) { return cols == 32 ? 0 : cols == 64 ? (krow >> 1) & 1 : krow & 3; };
   constexpr int ROWS_PER_LOAD_KC = NT / CPRK;     // rows covered by one load of all threads
   static_assert((ROWS_PER_LOAD_KC / RPW) % CPRK == 0, "swizzle must repeat per load");
   static_assert((!TA || (NT * 8 % BM == 0 && (NT * 8 / BM) % 4 == 0)) && (!TBL || (NT * 8 % BN == 0 && (NT * 8 / BN) % 4 == 0)),
@@ -468,7 +475,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   }
   // Barrier without a memory fence: a fence would wait for every direct load
   // still in flight; the vmcnt waits already cover the tile that is needed.
-  asm volatile("s_barrier" ::: "memory");
+  if constexpr (!ALONE) asm volatile("s_barrier" ::: "memory");
 #pragma unroll
   for (int kk = 0; kk < PF; kk++) read_frags(kk, 0, kk);
   // One k-tile.  STEADY: every condition of the generic body is known true
@@ -586,7 +593,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
           } else {
             wait_vmcnt<0>();
           }
-          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          if constexpr (ALONE) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          else asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
           if (STEADY || kt + STAGES < KT) {
             issue_some(kt + STAGES, stage, 0, PART, !STEADY);
           }
@@ -701,8 +709,153 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
       return;
     }
   }
+  // Column sums of a staged tile of `rows` x `cols` from row m, column n on.  A thread owns a column; per block of
+  // 32 rows: four runs of 8 rows summed in row order, then (0 + 1) + (2 + 3).
+  auto column_sums = [&](bf16 const *staged, int stride, int rows, int cols, int m, int n, int first, int threads) __attribute__((always_inline)) {
+    for (int i = first; i < cols * (rows / kColsumRowsPerBlock); i += threads) {
+      int const col = i % cols, blk = i / cols;
+      float run[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        float acc_rows = 0.0f;
+#pragma unroll
+        for (int r = 0; r < kColsumRowsPerLane; r++) {
+          acc_rows += VecIO<bf16>::load1(staged + (blk * kColsumRowsPerBlock + q * kColsumRowsPerLane + r) * stride + col);
+        }
+        run[q] = acc_rows;
+      }
+      int64_t const part = m / kColsumRowsPerBlock + blk;
+      if (EDGE == kEdgeBounded && (part * kColsumRowsPerBlock >= M || n + col >= N)) continue;
+      tail.colsum_partials[part * N + n + col] = (run[0] + run[1]) + (run[2] + run[3]);
+    }
+  };
+  constexpr bool kColsums = TAIL == GemmEpilogue::kTailDropoutGeluGrad || TAIL == GemmEpilogue::kTailDropoutReluGrad;
+  static_assert(!kColsums || EDGE != kEdgeOverlap, "blocks of 32 rows begin at multiples of 32");
+  // Eight results from column n of row m on, rounded, to memory through the tail's operators.  kept: the
+  // piece's place in the staged tile.
+  auto put_piece = [&](int m, int n, u32x4 v, bf16 *kept) __attribute__((always_inline)) {
+    int64_t const at = (int64_t)m * ldc + n;
+    if constexpr (TAIL == GemmEpilogue::kTailNone) {
+      store8(m, n, v);
+    } else {
+      if constexpr (EDGE == kEdgeOverlap) {  // N is a multiple of 8 here: a piece is one workgroup's
+        if (m < first_m || n < first_n) return;
+      }
+      if constexpr (EDGE == kEdgeBounded) {  // ... or not there
+        if (m >= M || n >= N) {
+          *reinterpret_cast<u32x4 *>(kept) = u32x4{0u, 0u, 0u, 0u};  // for the column sums
+          return;
+        }
+      }
+      // ldc == N here: `at` is the element's index in the dense tensor, and
+      // the piece is one block of the dropout stream
+      uint32_t w[4] = {0u, 0u, 0u, 0u};
+      // At a rate of zero everything is kept, whatever the stream says.  Only the residual add of a
+      // backward (always rate zero) asks: the branch keeps the pieces' loads from running under one
+      // another (forward of 4096 x 4096 -> 1024 with dropout and add: 45 us with it, 42 without).
+      if (!(TAIL == GemmEpilogue::kTailDropoutAdd && !TB) || tail.dropout.threshold != 0) {
+        philox4x32_10((tail.dropout.offset + (uint64_t)at) >> 3, tail.dropout.key, w);
+      }
+      u32x4 aux = {0u, 0u, 0u, 0u};
+      if constexpr (TAIL == GemmEpilogue::kTailGeluDropout || TAIL == GemmEpilogue::kTailActDropout) {
+        *reinterpret_cast<u32x4 *>(C + at) = v;
+      } else {
+        aux = *reinterpret_cast<u32x4 const *>(tail.in + at);
+      }
+      u32x4 r;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        float x[2] = {__uint_as_float(v[q] << 16), __uint_as_float(v[q] & 0xffff0000u)};
+        float const a[2] = {__uint_as_float(aux[q] << 16), __uint_as_float(aux[q] & 0xffff0000u)};
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          if constexpr (TAIL == GemmEpilogue::kTailGeluDropout) {
+            x[h] = storage_round<bf16>(gelu_forward(x[h]));
+          }
+          x[h] = keep(w, 2 * q + h, tail.dropout) ? x[h] * tail.dropout.scale : 0.0f;
+          if constexpr (TAIL == GemmEpilogue::kTailDropoutGeluGrad) {
+            x[h] = storage_round<bf16>(x[h]) * gelu_derivative(a[h]);
+          }
+          if constexpr (TAIL == GemmEpilogue::kTailDropoutReluGrad) {
+            x[h] = a[h] > 0.0f ? x[h] : 0.0f;
+          }
+          if constexpr (TAIL == GemmEpilogue::kTailDropoutAdd) {
+            x[h] = storage_round<bf16>(x[h]) + a[h];
+          }
+        }
+        r[q] = pack_bf16x2(x[0], x[1]);
+      }
+      bf16 *const to = TAIL == GemmEpilogue::kTailGeluDropout || TAIL == GemmEpilogue::kTailActDropout ? tail.out : C;
+      *reinterpret_cast<u32x4 *>(to + at) = r;
+      if constexpr (kColsums) {
+        // kept for the column sums below (the lane's own piece: no other lane reads it before the barrier)
+        if (tail.colsum_partials != nullptr) *reinterpret_cast<u32x4 *>(kept) = r;
+      }
+    }
+  };
+  if constexpr (ALONE) {
+    // Every wave lays down its sums in its own stages, 16 bytes a lane and access (66 lanes' room for each 64:
+    // what eight lanes read side by side below then lies in different banks); then all threads add up pieces
+    // of eight columns over the waves, in their order, and finish them.
+    static_assert(TM * TN * 4 * 66 * 8 <= STAGES * STAGE_ELEMS, "a tile's sums fit a wave's stages");
+    f32x4 *const mine = reinterpret_cast<f32x4 *>(stages) + lane;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          mine[((i * TN + j) * 4 + g) * 66] = f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+        }
+    __syncthreads();
+    constexpr int AS = BN + 8;
+    bf16 *const tile_kept = smem + KG * (STAGES * STAGE_ELEMS);
+    auto pieces = [&](auto actf) __attribute__((always_inline)) {
+      for (int c = threadIdx.x; c < BM * BN / 8; c += KG * 64) {
+        int const row = c / (BN / 8), ch = c % (BN / 8), m = m0 + row, n = n0 + ch * 8;
+        int const at = (((row >> 5) * TN + (ch >> 2)) * 4 + (ch & 3)) * 66 + (row & 31);
+        f32x4 lo = {0.0f, 0.0f, 0.0f, 0.0f}, hi = lo;
+#pragma unroll
+        for (int o = 0; o < KG; o++) {
+          f32x4 const *const part = reinterpret_cast<f32x4 const *>(smem + o * (STAGES * STAGE_ELEMS)) + at;
+          lo += part[0];
+          hi += part[32];
+        }
+        float v[8], old[8];
+        float bv[2][4];
+        bias4(n, bv[0]);
+        bias4(n + 4, bv[1]);
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = actf((e < 4 ? lo[e & 3] : hi[e & 3]) + bv[e >> 2][e & 3]);
+        if (accumulate != 0 && m < M && n < N) {
+          // add the old value in fp32 before the single rounding
+          bf16 const *const from = C + (int64_t)m * ldc + n;
+          unpack_raw(n + 8 <= N ? load_raw_any(from) : load_raw_first(from, N - n), old, (bf16 const *)nullptr);
+#pragma unroll
+          for (int e = 0; e < 8; e++) v[e] += old[e];
+        }
+        put_piece(m, n, pack_raw(v, (bf16 const *)nullptr), tile_kept + row * AS + ch * 8);
+      }
+    };
+    if (act == FFK_ACT_NONE) {
+      pieces([](float v) { return v; });
+    } else if (act == FFK_ACT_GELU) {
+      pieces([](float v) { return gelu_forward(v); });
+    } else if (act == FFK_ACT_RELU) {
+      pieces([](float v) { return v >= 0.0f ? v : 0.0f; });
+    } else {
+      pieces([act](float v) { return apply_activation(v, act); });
+    }
+    if constexpr (kColsums) {
+      if (tail.colsum_partials != nullptr) {  // uniform over the launch
+        __syncthreads();
+        column_sums(tile_kept, AS, BM, BN, m0, n0, (int)threadIdx.x, KG * 64);
+      }
+    }
+    return;
+  }
   __syncthreads();  // all stages are free now: reuse them for the output tile
-  if constexpr (KG > 1) {
+  if constexpr (KG > 1 && !ALONE) {
     static_assert((KG - 1) * NW * TM * TN * 1024 <= (KG - 1) * STAGES * STAGE_ELEMS / 2, "partial tiles fit the groups' stages");
     // group g's accumulators, 16 bytes a lane and access, in the stages that were group g's (the
     // output tile is staged in group 0's)
@@ -739,7 +892,6 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   // Each wave stages its own WM x WN tile and writes it out in 16-byte chunks.
   bf16 *cs = smem + wave * (WM * CS);
   constexpr int CCH = WM * WN / 8 / 64;  // 16-byte chunks per lane
-  constexpr bool kColsums = TAIL == GemmEpilogue::kTailDropoutGeluGrad || TAIL == GemmEpilogue::kTailDropoutReluGrad;
   // The activation is a compile-time functor here: a per-element switch inside
   // the unrolled loops made the epilogue several times longer than the GEMM's
   // own store traffic.
@@ -798,90 +950,13 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
       int c = lane + i * 64;
       int row = c / (WN / 8), ch = c % (WN / 8);
       u32x4 v = *reinterpret_cast<u32x4 const *>(cs + row * CS + ch * 8);
-      int64_t const at = (int64_t)(m0 + wm0 + row) * ldc + n0 + wn0 + ch * 8;
-      if constexpr (TAIL == GemmEpilogue::kTailNone) {
-        store8(m0 + wm0 + row, n0 + wn0 + ch * 8, v);
-      } else {
-        if constexpr (EDGE == kEdgeOverlap) {  // N is a multiple of 8 here: a piece is one workgroup's
-          if (m0 + wm0 + row < first_m || n0 + wn0 + ch * 8 < first_n) continue;
-        }
-        if constexpr (EDGE == kEdgeBounded) {  // ... or not there
-          if (m0 + wm0 + row >= M || n0 + wn0 + ch * 8 >= N) {
-            *reinterpret_cast<u32x4 *>(cs + row * CS + ch * 8) = u32x4{0u, 0u, 0u, 0u};  // for the column sums
-            continue;
-          }
-        }
-        // ldc == N here: `at` is the element's index in the dense tensor, and
-        // the piece is one block of the dropout stream
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
-        // At a rate of zero everything is kept, whatever the stream says.  Only the residual add of a
-        // backward (always rate zero) asks: the branch keeps the pieces' loads from running under one
-        // another (forward of 4096 x 4096 -> 1024 with dropout and add: 45 us with it, 42 without).
-        if (!(TAIL == GemmEpilogue::kTailDropoutAdd && !TB) || tail.dropout.threshold != 0) {
-          philox4x32_10((tail.dropout.offset + (uint64_t)at) >> 3, tail.dropout.key, w);
-        }
-        u32x4 aux = {0u, 0u, 0u, 0u};
-        if constexpr (TAIL == GemmEpilogue::kTailGeluDropout || TAIL == GemmEpilogue::kTailActDropout) {
-          *reinterpret_cast<u32x4 *>(dst + at) = v;
-        } else {
-          aux = *reinterpret_cast<u32x4 const *>(tail.in + at);
-        }
-        u32x4 r;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          float x[2] = {__uint_as_float(v[q] << 16), __uint_as_float(v[q] & 0xffff0000u)};
-          float const a[2] = {__uint_as_float(aux[q] << 16), __uint_as_float(aux[q] & 0xffff0000u)};
-#pragma unroll
-          for (int h = 0; h < 2; h++) {
-            if constexpr (TAIL == GemmEpilogue::kTailGeluDropout) {
-              x[h] = storage_round<bf16>(gelu_forward(x[h]));
-            }
-            x[h] = keep(w, 2 * q + h, tail.dropout) ? x[h] * tail.dropout.scale : 0.0f;
-            if constexpr (TAIL == GemmEpilogue::kTailDropoutGeluGrad) {
-              x[h] = storage_round<bf16>(x[h]) * gelu_derivative(a[h]);
-            }
-            if constexpr (TAIL == GemmEpilogue::kTailDropoutReluGrad) {
-              x[h] = a[h] > 0.0f ? x[h] : 0.0f;
-            }
-            if constexpr (TAIL == GemmEpilogue::kTailDropoutAdd) {
-              x[h] = storage_round<bf16>(x[h]) + a[h];
-            }
-          }
-          r[q] = pack_bf16x2(x[0], x[1]);
-        }
-        bf16 *const to = TAIL == GemmEpilogue::kTailGeluDropout || TAIL == GemmEpilogue::kTailActDropout ? tail.out : dst;
-        *reinterpret_cast<u32x4 *>(to + at) = r;
-        if constexpr (kColsums) {
-          // kept for the column sums below (the lane's own piece: no other lane reads it before the barrier)
-          if (tail.colsum_partials != nullptr) *reinterpret_cast<u32x4 *>(cs + row * CS + ch * 8) = r;
-        }
-      }
+      put_piece(m0 + wm0 + row, n0 + wn0 + ch * 8, v, cs + row * CS + ch * 8);
     }
     }  // half
     if constexpr (kColsums) {
       if (tail.colsum_partials != nullptr) {  // uniform over the launch
         __syncthreads();
-        // A lane owns a column of the wave's tile; per block of 32 rows: four
-        // runs of 8 rows summed in row order, then (0 + 1) + (2 + 3).
-        for (int col = lane; col < WN; col += 64) {
-#pragma unroll
-          for (int blk = 0; blk < WM / kColsumRowsPerBlock; blk++) {
-            float run[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-              float acc_rows = 0.0f;
-#pragma unroll
-              for (int r = 0; r < kColsumRowsPerLane; r++) {
-                acc_rows += VecIO<bf16>::load1(cs + (blk * kColsumRowsPerBlock + q * kColsumRowsPerLane + r) * CS + col);
-              }
-              run[q] = acc_rows;
-            }
-            int64_t const part = (m0 + wm0) / kColsumRowsPerBlock + blk;
-            static_assert(EDGE != kEdgeOverlap, "blocks of 32 rows begin at multiples of 32");
-            if (EDGE == kEdgeBounded && (part * kColsumRowsPerBlock >= M || n0 + wn0 + col >= N)) continue;
-            tail.colsum_partials[part * N + n0 + wn0 + col] = (run[0] + run[1]) + (run[2] + run[3]);
-          }
-        }
+        column_sums(cs, CS, WM, WN, m0 + wm0, n0 + wn0, lane, 64);
       }
     }
   };
@@ -961,6 +1036,11 @@ struct PipeCfg {
   static constexpr size_t kOutBytes = (size_t)NW * WM * (WN + 8) * sizeof(bf16);
   static constexpr size_t kLds = kStageBytes > kOutBytes ? kStageBytes : kOutBytes;
   static_assert(kLds <= 160 * 1024, "LDS budget");
+  // of KG groups of waves; groups of one wave keep the output tile behind their stages
+  template <int KG>
+  static constexpr size_t groups() {
+    return KG == 1 ? kLds : KG * kStageBytes + (NW == 1 ? (size_t)BM * (BN + 8) * sizeof(bf16) : 0);
+  }
 };
 
 template <int BM, int BN, int WM, int WN, int BK, int STAGES, int PF, bool TA, bool TB, int TAIL = 0, int EDGE = kEdgeNone,
@@ -971,13 +1051,14 @@ static hipError_t launch_pipe(hipStream_t st, bf16 const *A, bf16 const *B,
                               int splits = 1) {
   using Cfg = PipeCfg<BM, BN, WM, WN, BK, STAGES>;
   constexpr int NT = Cfg::NW * 64 * KG;
-  constexpr size_t kLds = KG == 1 ? Cfg::kLds : KG * Cfg::kStageBytes;
+  constexpr size_t kLds = Cfg::template groups<KG>();
   static_assert(kLds <= 160 * 1024, "LDS budget");
-  static_assert(KG <= 2, "the names below");
-  constexpr char const *edge = KG == 1 ? (EDGE == 0 ? "" : EDGE == 1 ? ",1" : ",2")  // unless they have their default
-                                       : (EDGE == 0 ? ",0,2" : EDGE == 1 ? ",1,2" : ",2,2");
-  if (describe_only("gemm_bf16_pipe_kernel<%d,%d,%d,%d,%d,%d,%d,%s,%s,%d,false%s>", BM, BN, WM, WN, BK, STAGES, PF, tf(TA),
-                    tf(TB), TAIL, edge)) {
+  if (tl_name_sink != nullptr) {
+    char rest[16] = "";  // EDGE and KG unless they have their default
+    if (KG != 1) snprintf(rest, sizeof rest, ",%d,%d", EDGE, KG);
+    else if (EDGE != kEdgeNone) snprintf(rest, sizeof rest, ",%d", EDGE);
+    describe_only("gemm_bf16_pipe_kernel<%d,%d,%d,%d,%d,%d,%d,%s,%s,%d,false%s>", BM, BN, WM, WN, BK, STAGES, PF, tf(TA), tf(TB),
+                  TAIL, rest);
     return hipSuccess;
   }
   auto kern = gemm_bf16_pipe_kernel<BM, BN, WM, WN, BK, STAGES, PF, TA, TB, TAIL, false, EDGE, KG>;
@@ -1007,12 +1088,12 @@ static hipError_t launch_pipe(hipStream_t st, bf16 const *A, bf16 const *B,
 }
 
 // Several GEMMs of the same kind and reduction length in one launch.
-template <int BM, int BN, int WM, int WN, int STAGES, int PF, bool TA, bool TB, int EDGE, int KG>
+template <int BM, int BN, int WM, int WN, int BK, int STAGES, int PF, bool TA, bool TB, int EDGE, int KG>
 static hipError_t launch_pipe_group(hipStream_t st, GemmProblem const *p, int n, int K, bool accumulate) {
-  using Cfg = PipeCfg<BM, BN, WM, WN, 64, STAGES>;
+  using Cfg = PipeCfg<BM, BN, WM, WN, BK, STAGES>;
   constexpr int NT = Cfg::NW * 64 * KG;
-  constexpr size_t kLds = KG == 1 ? Cfg::kLds : KG * Cfg::kStageBytes;
-  auto kern = gemm_bf16_pipe_kernel<BM, BN, WM, WN, 64, STAGES, PF, TA, TB, 0, true, EDGE, KG>;
+  constexpr size_t kLds = Cfg::template groups<KG>();
+  auto kern = gemm_bf16_pipe_kernel<BM, BN, WM, WN, BK, STAGES, PF, TA, TB, 0, true, EDGE, KG>;
   static LdsOptIn lds;
   if (hipError_t e = lds.ensure(reinterpret_cast<void const *>(kern), (int)kLds); e != hipSuccess) return e;
   GemmGroupArgs g = {};
@@ -1086,19 +1167,21 @@ inline bool edge_operands_ok(int64_t lda, int64_t ldb) { return 2 * 256 * std::m
 // launch to launch (median 1.4; 2-3 us of each is the launch), the short and the transposed ones most.
 //  - a round over the chip costs its 64-deep k-tiles times what one takes with so many CUs busy
 //    (memory and LDS are shared, the clock too), and a constant of filling, draining and storing
-//  - 64 x 64, two groups of waves that split the reduction, two workgroups a CU
+//  - 32 x 32, four waves that split the reduction, two workgroups a CU
+//    64 x 64, two groups of waves that split the reduction, two workgroups a CU
 //    64 x 64 deep: four LDS stages a group, one workgroup a CU: holds its rate where the operands
 //    come from behind L2, as they do in reductions longer than 2048
 //    128 x 64: eight waves, two workgroups a CU; 128 x 128; 256 x 256; wide: the latter with one wave
 //    per SIMD
-enum EdgeTile { kTile64 = 64, kTile64Deep = 65, kTile128x64 = 70, kTile128 = 128, kTile256 = 256, kTile256Wide = 264 };
+enum EdgeTile { kTile32 = 32, kTile64 = 64, kTile64Deep = 65, kTile128x64 = 70, kTile128 = 128, kTile256 = 256, kTile256Wide = 264 };
 inline double gemm_tile_us(EdgeTile t, double m, double n, double k, double splits = 1) {
-  int const bm = t == kTile64 || t == kTile64Deep ? 64 : t == kTile128x64 || t == kTile128 ? 128 : 256;
+  int const bm = t == kTile32 ? 32 : t == kTile64 || t == kTile64Deep ? 64 : t == kTile128x64 || t == kTile128 ? 128 : 256;
   int const bn = t == kTile128x64 ? 64 : bm;
   double const tiles = ceil(m / bm) * ceil(n / bn) * splits, kt = ceil(ceil(k / 64) / splits);
   auto round_us = [&](double count) {  // of `count` workgroups at a time
     double const f = count / kNumCU;
     switch (t) {
+      case kTile32: return f <= 1 ? kt * 0.11 + 1.9 : kt * 0.40 + 2.4;
       case kTile64: return f <= 1 ? kt * 0.166 + 1.8 : kt * 0.36 + 2.4;
       case kTile64Deep: return kt * 0.175 + 2.1;
       case kTile128x64: return f <= 1 ? kt * (0.29 + 0.08 * f) + 1.6 : kt * 0.54 + 2.0;
@@ -1107,7 +1190,7 @@ inline double gemm_tile_us(EdgeTile t, double m, double n, double k, double spli
       default: return kt * std::max(0.96, 0.25 + 1.19 * f) + 5.5 + 3.0 * f;
     }
   };
-  double const a_round = t == kTile64 || t == kTile128x64 ? 2 * kNumCU : kNumCU;
+  double const a_round = t == kTile32 || t == kTile64 || t == kTile128x64 ? 2 * kNumCU : kNumCU;
   double const full = floor(tiles / a_round), last = tiles - full * a_round;
   double us = full * round_us(a_round) + (last > 0 ? round_us(last) : 0.0);
   // the rounds of 128 x 128 tiles overlap less than the first one's fill suggests
@@ -1119,7 +1202,7 @@ inline double gemm_tile_us(EdgeTile t, double m, double n, double k, double spli
 inline EdgeTile gemm_tile_for(int M, int N, int K, bool wide_ok, double *time = nullptr) {
   EdgeTile best = kTile64;
   double least = gemm_tile_us(kTile64, M, N, K);
-  for (EdgeTile const t : {kTile64Deep, kTile128x64, kTile128, kTile256, kTile256Wide}) {
+  for (EdgeTile const t : {kTile32, kTile64Deep, kTile128x64, kTile128, kTile256, kTile256Wide}) {
     if ((t == kTile256Wide) != (wide_ok && K >= 1024) && (t == kTile256Wide || t == kTile256)) continue;
     double const us = gemm_tile_us(t, M, N, K);
     if (us < least) best = t, least = us;
@@ -1128,13 +1211,14 @@ inline EdgeTile gemm_tile_for(int M, int N, int K, bool wide_ok, double *time = 
   return best;
 }
 
-// Whether the plain kernel for this problem is one of the two 64x64 ones, whose waves split the
-// reduction (an epilogue's tail then has to run on that tile too for the same bits), and not one of
-// the larger ones, which all add up in the same order.
-inline bool gemm_splits_reduction(int M, int N, int K, GemmEpilogue const &ep) {
+// The tile of the plain kernel for this problem if it is one of those whose waves split the reduction (an
+// epilogue's tail then has to run on that tile too for the same bits), 0 if it is one of the larger ones,
+// which all add up in the same order.
+inline int gemm_split_tile(int M, int N, int K, GemmEpilogue const &ep) {
   EdgeTile const t = gemm_tile_for(M, N, K, ep.activation == FFK_ACT_NONE);
+  if (t == kTile32 || t == kTile64 || t == kTile64Deep) return t;
   int const bm = t == kTile256 || t == kTile256Wide ? 256 : 128, bn = t == kTile128x64 ? 64 : bm;
-  return t == kTile64 || t == kTile64Deep || M < bm || N < bn;
+  return M < bm || N < bn ? kTile64 : 0;
 }
 
 // Splitting the reduction over workgroups, where there is scratch for it: 128 x 128 or 256 x 256 tiles
@@ -1182,8 +1266,10 @@ static hipError_t launch_tail(hipStream_t st, bf16 const *A, bf16 const *B, bf16
   int const tile = pipe_tile_for(C, M, N, K, lda, ldb, ldc, ep, gemm_variant_override());
   if (tile == 256) return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB, TAIL>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
   if (tile == 128) return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, TAIL>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
-  if (gemm_splits_reduction(M, N, K, ep)) {
-    return launch_pipe<64, 64, 32, 32, 64, 2, 3, TA, TB, TAIL, kEdgeBounded, 2>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+  switch (gemm_split_tile(M, N, K, ep)) {
+    case kTile32: return launch_pipe<32, 32, 32, 32, 32, 4, 1, TA, TB, TAIL, kEdgeBounded, 4>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+    case kTile64: return launch_pipe<64, 64, 32, 32, 64, 2, 3, TA, TB, TAIL, kEdgeBounded, 2>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+    case kTile64Deep: return launch_pipe<64, 64, 32, 32, 64, 4, 3, TA, TB, TAIL, kEdgeBounded, 2>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
   }
   if constexpr (TAIL == GemmEpilogue::kTailGeluDropout) {
     return hipErrorInvalidValue;  // (one large tile a CU: gemm_tail_supported has refused it)
@@ -1226,34 +1312,37 @@ hipError_t pick_bf16_tail(hipStream_t st, bf16 const *A, bf16 const *B, bf16 *C,
   return hipErrorInvalidValue;
 }
 
-// A group of problems that each leave part of the chip idle: 128x128 tiles or 64x64 ones, whichever
-// takes less for all of them together by two formulas of the group's own, rounds times k-tiles.  They
-// rank the two and do not predict: 432 tiles of 128 x 128 over 1379 rows (the gradients of a 768-wide
+// A group of problems that each leave part of the chip idle: 128x128 tiles, 64x64 or 32x32 ones, whichever
+// takes less for all of them together by formulas of the group's own, rounds times k-tiles.  They
+// rank the three and do not predict: 432 tiles of 128 x 128 over 1379 rows (the gradients of a 768-wide
 // layer) 37 us, 22 by the formula.
 template <bool TA, bool TB>
 hipError_t pick_bf16_group(hipStream_t st, GemmProblem const *p, int n, int K, bool accumulate) {
   bool exact = K % 64 == 0, fits = true, exact256 = true;
-  double t64 = 0, t128 = 0;
+  double t32 = 0, t64 = 0, t128 = 0;
   for (int i = 0; i < n; i++) {
     exact = exact && p[i].M % 128 == 0 && p[i].N % 128 == 0 && p[i].ldc % 8 == 0 && aligned16(p[i].C);
     exact256 = exact256 && p[i].M % 256 == 0 && p[i].N % 256 == 0;
     fits = fits && p[i].M >= 128 && p[i].N >= 128 && !(accumulate && p[i].N % 8 != 0);
+    t32 += (double)(ceil_div(p[i].M, 32) * ceil_div(p[i].N, 32));
     t64 += (double)(ceil_div(p[i].M, 64) * ceil_div(p[i].N, 64));
     t128 += (double)(ceil_div(p[i].M, 128) * ceil_div(p[i].N, 128));
   }
   double const kt = (double)ceil_div(K, 64);
   double const us64 = t64 <= kNumCU ? kt * 0.17 + 1.0 : ceil(t64 / (2 * kNumCU)) * (kt * 0.39 + 1.0);
   double const us128 = ceil(t128 / kNumCU) * (kt * 0.46 + 1.0);
-  if (!fits || us64 < us128) return launch_pipe_group<64, 64, 32, 32, 2, 3, TA, TB, kEdgeBounded, 2>(st, p, n, K, accumulate);
+  double const us32 = t32 <= kNumCU ? kt * 0.11 + 1.0 : t32 <= 2 * kNumCU ? kt * 0.22 + 1.0 : 1e9;
+  if (us32 < us64 && (us32 < us128 || !fits)) return launch_pipe_group<32, 32, 32, 32, 32, 4, 1, TA, TB, kEdgeBounded, 4>(st, p, n, K, accumulate);
+  if (!fits || us64 < us128) return launch_pipe_group<64, 64, 32, 32, 64, 2, 3, TA, TB, kEdgeBounded, 2>(st, p, n, K, accumulate);
   // Long reductions of whole 256 x 256 tiles: a round of them, three quarters full, takes less than three
   // of 128 x 128 (four gradients of 12.6 M elements together over 4096
   // rows: 106-114 us against 119; 81 by the model).
   if (exact && exact256 && K >= 1024 &&
       gemm_tile_us(kTile256Wide, 64 * t128, 256, K) < gemm_tile_us(kTile128, 128 * t128, 128, K)) {
-    return launch_pipe_group<256, 256, 128, 128, 2, 1, TA, TB, kEdgeNone, 1>(st, p, n, K, accumulate);
+    return launch_pipe_group<256, 256, 128, 128, 64, 2, 1, TA, TB, kEdgeNone, 1>(st, p, n, K, accumulate);
   }
-  if (exact) return launch_pipe_group<128, 128, 64, 32, 4, 1, TA, TB, kEdgeNone, 1>(st, p, n, K, accumulate);
-  return launch_pipe_group<128, 128, 64, 32, 4, 1, TA, TB, kEdgeOverlap, 1>(st, p, n, K, accumulate);
+  if (exact) return launch_pipe_group<128, 128, 64, 32, 64, 4, 1, TA, TB, kEdgeNone, 1>(st, p, n, K, accumulate);
+  return launch_pipe_group<128, 128, 64, 32, 64, 4, 1, TA, TB, kEdgeOverlap, 1>(st, p, n, K, accumulate);
 }
 
 template <bool TA, bool TB>
@@ -1279,7 +1368,7 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
     bool const wide_ok = ep.activation == FFK_ACT_NONE && ldc % 8 == 0;
     double us;
     EdgeTile tile = gemm_tile_for(M, N, K, wide_ok, &us);
-    bool const forced = variant == 64 || variant == 65 || variant == 70 || variant == 128 || variant == 256 || variant == 264;
+    bool const forced = variant == 32 || variant == 64 || variant == 65 || variant == 70 || variant == 128 || variant == 256 || variant == 264;
     bool const whole128 = M % 128 == 0 && N % 128 == 0 && pipe_operands_ok(C, K, lda, ldb, ldc, ep);
     if (forced) {
       tile = variant == kTile256Wide && ep.activation != FFK_ACT_NONE ? kTile256 : (EdgeTile)variant;
@@ -1312,7 +1401,7 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
     }
     // tiles that begin early: the output has to hold one, and old values added by one workgroup only
     int const bm = tile == kTile256 || tile == kTile256Wide ? 256 : 128, bn = tile == kTile128x64 ? 64 : bm;
-    if (tile != kTile64 && tile != kTile64Deep && (M < bm || N < bn || (ep.accumulate && N % 8 != 0))) tile = kTile64;
+    if (tile != kTile32 && tile != kTile64 && tile != kTile64Deep && (M < bm || N < bn || (ep.accumulate && N % 8 != 0))) tile = kTile64;
     bool const whole = M % bm == 0 && N % bn == 0 && pipe_operands_ok(C, K, lda, ldb, ldc, ep);
     switch (tile) {
       case kTile256Wide:
@@ -1328,6 +1417,8 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
         return launch_pipe<128, 64, 32, 32, 64, 3, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
       case kTile64Deep:
         return launch_pipe<64, 64, 32, 32, 64, 4, 3, TA, TB, 0, kEdgeBounded, 2>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+      case kTile32:
+        return launch_pipe<32, 32, 32, 32, 32, 4, 1, TA, TB, 0, kEdgeBounded, 4>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
       case kTile64:
         return launch_pipe<64, 64, 32, 32, 64, 2, 3, TA, TB, 0, kEdgeBounded, 2>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
     }
