@@ -221,50 +221,6 @@ __device__ __forceinline__ u32x4 pack_raw(float const (&v)[8], bf16 const *) {
   return u32x4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
 }
 
-// Vector v (kVec elements from v * kVec on) of a row of N elements, in the two kinds of rows there
-// are: whole aligned vectors, or (ANY) any N at any address, where the last vector may be partial:
-// its missing elements are read as zeros and not stored.  STREAM: past the caches (whole vectors only).
-// It is a template argument because of two accesses to one address that differ in nothing but the hint
-// the compiler makes one, without the hint, also where the choice between them is a constant.
-template <typename T, bool ANY>
-struct RowVec {
-  static constexpr int V = VecIO<T>::kVec;
-  __host__ __device__ static __forceinline__ int count(int N) { return ANY ? (N + V - 1) / V : N / V; }
-  // how many of vector v's elements exist
-  __device__ static __forceinline__ int elems(int v, int N) { return ANY ? min(V, N - v * V) : V; }
-  template <bool STREAM = false>
-  __device__ static __forceinline__ u32x4 load_raw(T const *row, int v, int N) {
-    T const *p = row + (int64_t)v * V;
-    if constexpr (ANY) {
-      return elems(v, N) == V ? load_raw_any(p) : load_raw_first(p, elems(v, N));
-    } else if constexpr (STREAM) {
-      return load_raw_stream(p);
-    } else {
-      return *reinterpret_cast<u32x4 const *>(p);
-    }
-  }
-  template <bool STREAM = false>
-  __device__ static __forceinline__ void load(T const *row, int v, int N, float (&x)[V]) {
-    unpack_raw(load_raw<STREAM>(row, v, N), x, (T const *)nullptr);
-  }
-  template <bool STREAM = false>
-  __device__ static __forceinline__ void store(T *row, int v, int N, float const (&x)[V]) {
-    T *p = row + (int64_t)v * V;
-    u32x4 const r = pack_raw(x, (T const *)nullptr);
-    if constexpr (ANY) {
-      if (elems(v, N) == V) {
-        store_raw_any(p, r);
-      } else {
-        store_raw_first(p, r, elems(v, N));
-      }
-    } else if constexpr (STREAM) {
-      __builtin_nontemporal_store(r, reinterpret_cast<u32x4 *>(p));
-    } else {
-      *reinterpret_cast<u32x4 *>(p) = r;
-    }
-  }
-};
-
 // ---- GELU (exact erf form) shared by ElementUnary and the GEMM epilogue ----
 // erf by Abramowitz & Stegun 7.1.26 (|error| <= 1.5e-7), sharing exp(-z^2)
 // with the caller: returns erf(z) given e = exp(-z*z).
@@ -318,19 +274,30 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_read(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
+// swaps the odd 16-lane rows of the first operand with the even rows of the second: with the
+// same value in both, the results hold rows {0,0,2,2} and {1,1,3,3}
 template <typename F>
+__device__ __forceinline__ float swap_rows(float v, F f) {
+  auto const a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+// the same for the two 32-lane halves
+template <typename F>
+__device__ __forceinline__ float swap_halves(float v, F f) {
+  auto const b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+// LANES: over aligned groups of 16 or 32 lanes instead, which leave out the last swaps.
+template <int LANES = 64, typename F>
 __device__ __forceinline__ float wave_reduce(float v, F f) {
+  static_assert(LANES == 16 || LANES == 32 || LANES == 64, "rows of lanes");
   v = f(v, dpp_read<0xB1>(v));   // quad_perm [1,0,3,2]
   v = f(v, dpp_read<0x4E>(v));   // quad_perm [2,3,0,1]
   v = f(v, dpp_read<0x141>(v));  // row_half_mirror
   v = f(v, dpp_read<0x140>(v));  // row_mirror
-  // swaps the odd 16-lane rows of the first operand with the even rows of the second: with the
-  // same value in both, the results hold rows {0,0,2,2} and {1,1,3,3}
-  auto const a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  // the same for the two 32-lane halves
-  auto const b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+  if constexpr (LANES >= 32) v = swap_rows(v, f);
+  if constexpr (LANES == 64) v = swap_halves(v, f);
+  return v;
 }
 __device__ __forceinline__ float wave_sum(float v) {
   return wave_reduce(v, [](float a, float b) { return a + b; });

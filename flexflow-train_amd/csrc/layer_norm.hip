@@ -21,8 +21,8 @@ namespace ffk {
 
 // PRE: the row normalised is residual + dropout(X), computed here, rounded to T where the two
 // separate operators would have stored it, and written to `summed` as well.
-// ANY: any N, rows at any address (RowVec).
-template <typename T, int EPT, int WPR, bool PRE = false, bool STREAM = false, bool ANY = false>
+// ANY: any N, rows at any address (LaneRow).
+template <typename T, int EPT, int LANES, bool PRE = false, bool STREAM = false, bool ANY = false>
 __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
     T const *__restrict__ X, T *__restrict__ Y, T const *__restrict__ gamma,
     T const *__restrict__ beta, float *__restrict__ mean,
@@ -30,14 +30,12 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
     T const *__restrict__ residual = nullptr, T *__restrict__ summed = nullptr,
     DropoutParams drop = DropoutParams{}) {
   constexpr int V = VecIO<T>::kVec;
-  using RV = RowVec<T, ANY>;
-  constexpr int RPB = 4 / WPR;  // rows per workgroup
-  constexpr int LANES = 64 * WPR;
+  using RV = LaneRow<T, ANY, EPT, LANES>;
   __shared__ float smem[2][4][2];
-  RowReducer<WPR> red(smem);
+  RowReducer<LANES> red(smem);
   int const nvec = RV::count(N);
-  int const lane = WPR == 1 ? (threadIdx.x & 63) : threadIdx.x;
-  int64_t const row = (int64_t)blockIdx.x * RPB + (WPR == 1 ? (threadIdx.x >> 6) : 0);
+  int const lane = threadIdx.x % LANES;
+  int64_t const row = (int64_t)blockIdx.x * (kRowThreads / LANES) + threadIdx.x / LANES;
   bool const row_ok = row < M;
   T const *xr = X + (row_ok ? row : 0) * (int64_t)N;
 
@@ -56,7 +54,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
       g[j][e] = 1.0f;
       b[j][e] = 0.0f;
     }
-    if (v < nvec) {
+    if (ANY || v < nvec) {
       if (gamma != nullptr) RV::load(gamma, v, N, g[j]);
       if (beta != nullptr) RV::load(beta, v, N, b[j]);
     }
@@ -68,7 +66,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
 #pragma unroll
   for (int j = 0; j < EPT; j++) {
     int v = lane + j * LANES;
-    if (v < nvec) {
+    if (ANY || v < nvec) {
       RV::template load<STREAM>(xr, v, N, x[j]);
       if constexpr (PRE) {
         static_assert(V == 4 || V == 8, "a lane's vector is a Philox block or half of one");
@@ -92,23 +90,23 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
         }
       }
 #pragma unroll
-      for (int e = 0; e < V; e++) s += x[j][e];
+      for (int e = 0; e < V; e++) s += RV::ragged(j, N) && e < RV::spare(v, N) ? 0.0f : x[j][e];
     } else {
 #pragma unroll
       for (int e = 0; e < V; e++) x[j][e] = 0.0f;
     }
   }
   float const inv_n = 1.0f / (float)N;
-  float const mu = red.sum(s) * inv_n;
+  float mu = red.sum(s) * inv_n;
+  asm("" : "+v"(mu));  // rounded once: x - mu is not to become a fused operation in one place and not in another
   float q = 0.0f;
 #pragma unroll
   for (int j = 0; j < EPT; j++) {
     int v = lane + j * LANES;
-    if (v < nvec) {
+    if (ANY || v < nvec) {
 #pragma unroll
       for (int e = 0; e < V; e++) {
-        float d = x[j][e] - mu;
-        if (ANY && e >= RV::elems(v, N)) d = 0.0f;
+        float const d = RV::ragged(j, N) && e < RV::spare(v, N) ? 0.0f : x[j][e] - mu;
         q += d * d;
       }
     }
@@ -144,7 +142,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_generic_kernel(
     T const *__restrict__ beta, float *__restrict__ mean,
     float *__restrict__ rstd, int64_t M, int N, float eps) {
   __shared__ float smem[2][4][2];
-  RowReducer<4> red(smem);
+  RowReducer<256> red(smem);
   int64_t const row = blockIdx.x;
   T const *xr = X + row * (int64_t)N;
   float s = 0.0f;
@@ -173,8 +171,13 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_generic_kernel(
 // DROP: dropout_backward(dX as stored) is written to `dropped` as well (the gradient entering
 // a dropout whose output fed the residual sum that this LayerNorm normalised).
 // STREAM: dY and X are read past the caches.
-template <typename T, int EPT, int WPR, bool ACC, bool DROP = false, bool ANY = false, bool STREAM = false>
-__global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
+// Eight waves a workgroup where a lane holds one vector: the grid is bounded by what its partial sums may cost,
+// and with four it has too few loads in flight on short rows ([7990, 410] bf16: 13.3 us, 7.6 so; the partial
+// sums leave as whole vectors: [335, 7107], a row a workgroup, 29 us element by element and 15 so).
+__host__ __device__ constexpr int ln_bwd_threads(int ept, int lanes) { return ept == 1 && lanes <= 64 ? 512 : kRowThreads; }
+
+template <typename T, int EPT, int LANES, bool ACC, bool DROP = false, bool ANY = false, bool STREAM = false>
+__global__ __launch_bounds__(ln_bwd_threads(EPT, LANES)) void layer_norm_bwd_kernel(
     T const *__restrict__ dY, T const *__restrict__ X,
     float const *__restrict__ mean, float const *__restrict__ rstd,
     T const *__restrict__ gamma, T *dX, float *__restrict__ partials,
@@ -185,14 +188,13 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
   // res to the stored gradient would give; without round_first the sum is rounded once, i.e.
   // what dX += gradient gives when dX holds a copy of res.
   constexpr int V = VecIO<T>::kVec;
-  using RV = RowVec<T, ANY>;
-  constexpr int RPB = 4 / WPR;
-  constexpr int LANES = 64 * WPR;
+  using RV = LaneRow<T, ANY, EPT, LANES>;
+  constexpr int THREADS = ln_bwd_threads(EPT, LANES), RPB = THREADS / LANES;  // rows per workgroup
   __shared__ float smem[2][4][2];
-  RowReducer<WPR> red(smem);
+  RowReducer<LANES> red(smem);
   int const nvec = RV::count(N);
-  int const lane = WPR == 1 ? (threadIdx.x & 63) : threadIdx.x;
-  int const sub = WPR == 1 ? (threadIdx.x >> 6) : 0;
+  int const lane = threadIdx.x % LANES;
+  int const sub = threadIdx.x / LANES;
   float const inv_n = 1.0f / (float)N;
 
   float g[EPT][V], dg[EPT][V], db[EPT][V];
@@ -205,7 +207,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
       dg[j][e] = 0.0f;
       db[j][e] = 0.0f;
     }
-    if (gamma != nullptr && v < nvec) {
+    if (gamma != nullptr && (ANY || v < nvec)) {
       RV::load(gamma, v, N, g[j]);
     }
   }
@@ -230,7 +232,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
 #pragma unroll
       for (int j = 0; j < EPT; j++) {
         int v = lane + j * LANES;
-        if (v < nvec) {
+        if (ANY || v < nvec) {
           rx[j] = RV::template load_raw<STREAM>(X + r * (int64_t)N, v, N);
           rdy[j] = RV::template load_raw<STREAM>(dY + r * (int64_t)N, v, N);
         }
@@ -265,8 +267,9 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
         float xh = (x[j][e] - mu) * rs;
         float const dyv = dy[j][e];
         float dyg = dyv * g[j][e];
-        s1 += dyg;
-        s2 += dyg * xh;
+        float const own = RV::ragged(j, N) && e < RV::spare(lane + j * LANES, N) ? 0.0f : dyg;
+        s1 += own;
+        s2 += own * xh;
         x[j][e] = xh;
         dg[j][e] += dyv * xh;
         db[j][e] += dyv;
@@ -290,7 +293,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
             if (ACC && res != nullptr && round_first) val = storage_round<T>(val);
             o[e] = ACC ? o[e] + val : val;
           }
-          RV::store(dst, v, N, o);
+          RV::template store<false, ACC>(dst, v, N, o);
           if constexpr (DROP) {
             static_assert(V == 4 || V == 8, "a lane's vector is a Philox block or half of one");
             int64_t const at = row * (int64_t)N + (int64_t)v * V;
@@ -321,47 +324,62 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_kernel(
     }
   }
 
-  // Workgroup partial: with WPR == 1 the four waves hold different rows of the
-  // same columns; fold them through LDS first.
+  // Workgroup partial: where its waves, and groups of lanes, hold different rows of the same columns they
+  // are folded first.
   float *pg = partials + (int64_t)blockIdx.x * 2 * N;
   float *pb = pg + N;
-  if (WPR == 1) {
-    __shared__ float fold[3][64][V + 1];
+  auto put = [&](float *to, int v, float const (&x)[V]) {
+    if (v >= nvec) return;
+    if (ANY && N < V) {
+#pragma unroll
+      for (int e = 0; e < V; e++) {
+        if (e >= RV::spare(v, N)) to[v * V + e - RV::spare(v, N)] = x[e];
+      }
+      return;
+    }
+    float *const p = to + (ANY ? min(v * V, N - V) : v * V);
+#pragma unroll
+    for (int e = 0; e < V; e += 4) {
+      store_raw_any(p + e, u32x4{__float_as_uint(x[e]), __float_as_uint(x[e + 1]), __float_as_uint(x[e + 2]),
+                                 __float_as_uint(x[e + 3])});
+    }
+  };
+  if constexpr (LANES <= 64) {
+    constexpr int WAVES = THREADS / 64;
+    __shared__ float fold[WAVES - 1][LANES][V + 1];
+    int const wave = threadIdx.x >> 6;
+    bool const first = (threadIdx.x & 63) < LANES;  // the group of lanes that speaks for its wave
 #pragma unroll
     for (int j = 0; j < EPT; j++) {
-      int v = lane + j * LANES;
       for (int pass = 0; pass < 2; pass++) {
-        __syncthreads();
-        if (sub > 0) {
+        float tot[V];
 #pragma unroll
-          for (int e = 0; e < V; e++) {
-            fold[sub - 1][lane][e] = pass == 0 ? dg[j][e] : db[j][e];
-          }
+        for (int e = 0; e < V; e++) {
+          tot[e] = pass == 0 ? dg[j][e] : db[j][e];
+          if (LANES == 16) tot[e] = swap_rows(tot[e], [](float a, float b) { return a + b; });
+          if (LANES <= 32) tot[e] = swap_halves(tot[e], [](float a, float b) { return a + b; });
         }
         __syncthreads();
-        if (sub == 0 && v < nvec) {
+        if (wave > 0 && first) {
 #pragma unroll
-          for (int e = 0; e < V; e++) {
-            float tot = (pass == 0 ? dg[j][e] : db[j][e]) + fold[0][lane][e] +
-                        fold[1][lane][e] + fold[2][lane][e];
-            if (ANY && e >= RV::elems(v, N)) continue;
-            (pass == 0 ? pg : pb)[(int64_t)v * V + e] = tot;
+          for (int e = 0; e < V; e++) fold[wave - 1][lane][e] = tot[e];
+        }
+        __syncthreads();
+        if (wave == 0 && first) {
+#pragma unroll
+          for (int w = 0; w < WAVES - 1; w++) {
+#pragma unroll
+            for (int e = 0; e < V; e++) tot[e] += fold[w][lane][e];
           }
+          put(pass == 0 ? pg : pb, lane + j * LANES, tot);
         }
       }
     }
   } else {
 #pragma unroll
     for (int j = 0; j < EPT; j++) {
-      int v = lane + j * LANES;
-      if (v < nvec) {
-#pragma unroll
-        for (int e = 0; e < V; e++) {
-          if (ANY && e >= RV::elems(v, N)) continue;
-          pg[(int64_t)v * V + e] = dg[j][e];
-          pb[(int64_t)v * V + e] = db[j][e];
-        }
-      }
+      put(pg, lane + j * LANES, dg[j]);
+      put(pb, lane + j * LANES, db[j]);
     }
   }
 }
@@ -375,7 +393,7 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_bwd_generic_dx_kernel(
     float const *__restrict__ mean, float const *__restrict__ rstd,
     T const *__restrict__ gamma, T *dX, int64_t M, int N, int acc) {
   __shared__ float smem[2][4][2];
-  RowReducer<4> red(smem);
+  RowReducer<256> red(smem);
   int64_t const row = blockIdx.x;
   float const mu = mean[row], rs = rstd[row];
   float s1 = 0.0f, s2 = 0.0f;
@@ -422,9 +440,8 @@ __global__ __launch_bounds__(256) void layer_norm_bwd_generic_param_kernel(
 // kernel that adds them up cost more than the extra requests in flight gain (80 and 92 us).
 constexpr int kLnBwdMaxBlocks = 2 * kNumCU;
 
-static int ln_bwd_blocks(int64_t M, int wpr) {
-  int64_t rpb = 4 / wpr;
-  int64_t b = ceil_div(M, rpb);
+static int ln_bwd_blocks(int64_t M, int ept, int lanes) {
+  int64_t b = ceil_div(M, ln_bwd_threads(ept, lanes) / lanes);
   return (int)(b < kLnBwdMaxBlocks ? b : kLnBwdMaxBlocks);
 }
 
@@ -437,32 +454,32 @@ static int ln_forward(hipStream_t st, void const *x, void *y, void const *gamma,
   T *Y = static_cast<T *>(y);
   T const *G = static_cast<T const *>(gamma);
   T const *Bt = static_cast<T const *>(beta);
-  int ept = 0, wpr = 0;
+  int ept = 0, lanes = 0;
   bool const vec = (N % V == 0) && aligned16(x) && aligned16(y) && (gamma == nullptr || aligned16(gamma)) &&
                    (beta == nullptr || aligned16(beta));
-  if (!pick_row_config_small(ceil_div(N, V), ept, wpr)) {
+  if (!pick_row_config_small(ceil_div(N, V), ept, lanes)) {
     layer_norm_fwd_generic_kernel<T><<<(unsigned)M, kRowThreads, 0, st>>>(
         X, Y, G, Bt, mean, rstd, M, (int)N, eps);
   } else if (vec) {
-    int64_t blocks = ceil_div(M, 4 / wpr);
+    int64_t blocks = ceil_div(M, kRowThreads / lanes);
     bool const stream = stream_past_caches(M * N, sizeof(T));
-#define CALL(E, W)                                                             \
+#define CALL(E, L)                                                             \
   do {                                                                         \
     if (stream)                                                                \
-      layer_norm_fwd_kernel<T, E, W, false, true><<<(unsigned)blocks, kRowThreads, 0, st>>>( \
+      layer_norm_fwd_kernel<T, E, L, false, true><<<(unsigned)blocks, kRowThreads, 0, st>>>( \
           X, Y, G, Bt, mean, rstd, M, (int)N, eps);                            \
     else                                                                       \
-      layer_norm_fwd_kernel<T, E, W><<<(unsigned)blocks, kRowThreads, 0, st>>>( \
+      layer_norm_fwd_kernel<T, E, L><<<(unsigned)blocks, kRowThreads, 0, st>>>( \
           X, Y, G, Bt, mean, rstd, M, (int)N, eps);                            \
   } while (0)
-    FFK_ROW_DISPATCH_SMALL(ept, wpr, CALL);
+    FFK_ROW_DISPATCH_SMALL(ept, lanes, CALL);
 #undef CALL
   } else {
     // [3001, 1001] fp32: 11.3 us with the scalar kernel, which reads a row three times
-#define CALL(E, W)                                                                                             \
-  layer_norm_fwd_kernel<T, E, W, false, false, true><<<(unsigned)ceil_div(M, 4 / wpr), kRowThreads, 0, st>>>( \
+#define CALL(E, L)                                                                                             \
+  layer_norm_fwd_kernel<T, E, L, false, false, true><<<(unsigned)ceil_div(M, kRowThreads / lanes), kRowThreads, 0, st>>>( \
       X, Y, G, Bt, mean, rstd, M, (int)N, eps)
-    FFK_ROW_DISPATCH_SMALL(ept, wpr, CALL);
+    FFK_ROW_DISPATCH_SMALL(ept, lanes, CALL);
 #undef CALL
   }
   FFK_CHECK_LAUNCH();
@@ -487,8 +504,8 @@ static int ln_backward(hipStream_t st, void const *dy, void const *x,
   T const *X = static_cast<T const *>(x);
   T const *G = static_cast<T const *>(gamma);
   T *DX = static_cast<T *>(dx);
-  int ept = 0, wpr = 0;
-  bool const fits = pick_row_config_small(ceil_div(N, V), ept, wpr);
+  int ept = 0, lanes = 0;
+  bool const fits = pick_row_config_small(ceil_div(N, V), ept, lanes);
   bool const vec = (N % V == 0) && aligned16(dy) && aligned16(x) && (dx == nullptr || aligned16(dx)) &&
                    aligned16(residual) && (gamma == nullptr || aligned16(gamma)) && fits;
   if (!vec && RES != nullptr) {
@@ -499,7 +516,7 @@ static int ln_backward(hipStream_t st, void const *dy, void const *x,
   // of them one thread a column over all rows).  It needs the workspace, which they did not: a
   // caller that brought none still gets them.
   if (vec || (fits && workspace != nullptr && workspace_bytes >= 2 * (size_t)N * sizeof(float))) {
-    int blocks = ln_bwd_blocks(M, wpr);
+    int blocks = ln_bwd_blocks(M, ept, lanes);
     if (!vec) fit_blocks_to_workspace = true;
     size_t const per_block = 2 * (size_t)N * sizeof(float);
     if (fit_blocks_to_workspace && workspace_bytes / per_block < (size_t)blocks) {
@@ -519,27 +536,27 @@ static int ln_backward(hipStream_t st, void const *dy, void const *x,
   do {                                                                         \
     auto kern = stream ? layer_norm_bwd_kernel<__VA_ARGS__, false, true>       \
                        : layer_norm_bwd_kernel<__VA_ARGS__, false, false>;     \
-    kern<<<blocks, kRowThreads, 0, st>>>(DY, X, mean, rstd, G, DX, partials, M, (int)N, RES, static_cast<T *>(dropped), \
+    kern<<<blocks, ln_bwd_threads(ept, lanes), 0, st>>>(DY, X, mean, rstd, G, DX, partials, M, (int)N, RES, static_cast<T *>(dropped), \
                                          drop != nullptr ? *drop : DropoutParams{}, round_first); \
   } while (0)
-#define CALL(E, W)                                                             \
+#define CALL(E, L)                                                             \
   do {                                                                         \
     if (!vec) {                                                                \
       if (acc)                                                                 \
-        layer_norm_bwd_kernel<T, E, W, true, false, true><<<blocks, kRowThreads, 0, st>>>( \
+        layer_norm_bwd_kernel<T, E, L, true, false, true><<<blocks, ln_bwd_threads(ept, lanes), 0, st>>>( \
             DY, X, mean, rstd, G, DX, partials, M, (int)N, nullptr);           \
       else                                                                     \
-        layer_norm_bwd_kernel<T, E, W, false, false, true><<<blocks, kRowThreads, 0, st>>>( \
+        layer_norm_bwd_kernel<T, E, L, false, false, true><<<blocks, ln_bwd_threads(ept, lanes), 0, st>>>( \
             DY, X, mean, rstd, G, DX, partials, M, (int)N, nullptr);           \
     } else if (dropped != nullptr) {                                           \
-      if constexpr (sizeof(T) == 2) LAUNCH(T, E, W, true, true);               \
+      if constexpr (sizeof(T) == 2) LAUNCH(T, E, L, true, true);               \
     } else if (acc) {                                                          \
-      LAUNCH(T, E, W, true, false);                                            \
+      LAUNCH(T, E, L, true, false);                                            \
     } else {                                                                   \
-      LAUNCH(T, E, W, false, false);                                           \
+      LAUNCH(T, E, L, false, false);                                           \
     }                                                                          \
   } while (0)
-    FFK_ROW_DISPATCH_SMALL(ept, wpr, CALL);
+    FFK_ROW_DISPATCH_SMALL(ept, lanes, CALL);
 #undef CALL
 #undef LAUNCH
     FFK_CHECK_LAUNCH();
@@ -571,18 +588,18 @@ static int ln_forward_pre(hipStream_t st, void const *in, void const *residual, 
                           void const *gamma, void const *beta, float *mean, float *rstd, int64_t M, int64_t N,
                           float eps, DropoutParams const &drop) {
   constexpr int V = VecIO<T>::kVec;
-  int ept = 0, wpr = 0;
+  int ept = 0, lanes = 0;
   bool vec = (N % 8 == 0) && (drop.offset & 7) == 0 && aligned16(in) && aligned16(residual) && aligned16(summed) &&
              aligned16(y) && (gamma == nullptr || aligned16(gamma)) && (beta == nullptr || aligned16(beta)) &&
-             pick_row_config_small(N / V, ept, wpr);
+             pick_row_config_small(N / V, ept, lanes);
   if (!vec) return FFK_ERR_UNSUPPORTED;
-  int64_t blocks = ceil_div(M, 4 / wpr);
-#define CALL(E, W)                                                                                  \
-  layer_norm_fwd_kernel<T, E, W, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(                  \
+  int64_t blocks = ceil_div(M, kRowThreads / lanes);
+#define CALL(E, L)                                                                                  \
+  layer_norm_fwd_kernel<T, E, L, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(                  \
       static_cast<T const *>(in), static_cast<T *>(y), static_cast<T const *>(gamma),             \
       static_cast<T const *>(beta), mean, rstd, M, (int)N, eps, static_cast<T const *>(residual), \
       static_cast<T *>(summed), drop)
-  FFK_ROW_DISPATCH_SMALL(ept, wpr, CALL);
+  FFK_ROW_DISPATCH_SMALL(ept, lanes, CALL);
 #undef CALL
   FFK_CHECK_LAUNCH();
   return FFK_OK;

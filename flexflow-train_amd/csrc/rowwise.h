@@ -1,9 +1,10 @@
 // Row-wise reduction scaffolding shared by LayerNorm and Softmax.
 //
-// A row of N elements is owned either by one wavefront (WPR == 1: no LDS, no
-// barrier, four independent rows per 256-thread workgroup) or by the four
-// wavefronts of a workgroup (WPR == 4).  Each lane keeps EPT 16-byte vectors
-// of the row in registers, so every element is read from HBM exactly once.
+// A row of N elements is owned by LANES lanes: by 16 or 32 where that many 16-byte vectors hold it (four or
+// two rows a wavefront: the instructions of a row, which are what such kernels are bound by, are issued for
+// all of them at once; [236881, 254] bf16, LayerNorm forward and backward, with a wavefront a row 249 and 469
+// us, so and with the last vector below 58 and 69; Softmax 130 and 188, 38 and 60), by one wavefront (no LDS, no barrier), or by the four wavefronts of a workgroup (256).  Each lane
+// keeps EPT vectors of the row in registers, so every element is read from HBM exactly once.
 #pragma once
 #include "ffk_common.h"
 
@@ -11,17 +12,20 @@ namespace ffk {
 
 constexpr int kRowThreads = 256;
 
-template <int WPR>
+template <int LANES>
 struct RowReducer {
   // smem: 2 phases x 4 waves x 2 values
   float (*smem)[4][2];
   int phase;
   __device__ __forceinline__ RowReducer(float (*s)[4][2]) : smem(s), phase(0) {}
 
+  __device__ __forceinline__ static float lanes_sum(float v) {
+    return wave_reduce<LANES < 64 ? LANES : 64>(v, [](float a, float b) { return a + b; });
+  }
   __device__ __forceinline__ void sum2(float &a, float &b) {
-    a = wave_sum(a);
-    b = wave_sum(b);
-    if (WPR > 1) {
+    a = lanes_sum(a);
+    b = lanes_sum(b);
+    if (LANES > 64) {
       int const wave = threadIdx.x >> 6;
       if ((threadIdx.x & 63) == 0) {
         smem[phase][wave][0] = a;
@@ -39,8 +43,8 @@ struct RowReducer {
     return a;
   }
   __device__ __forceinline__ float max(float a) {
-    a = wave_max(a);
-    if (WPR > 1) {
+    a = wave_reduce<LANES < 64 ? LANES : 64>(a, [](float x, float y) { return fmaxf(x, y); });
+    if (LANES > 64) {
       int const wave = threadIdx.x >> 6;
       if ((threadIdx.x & 63) == 0) {
         smem[phase][wave][0] = a;
@@ -54,62 +58,138 @@ struct RowReducer {
   }
 };
 
-// Picks (EPT, WPR) for a row of `nvec` 16-byte vectors; returns false when the
+// Vector v of a row of N elements in a kernel that gives every lane one, also lanes past the row's end.
+// Rows of whole aligned vectors (ANY false) are read by the lanes that have a vector, the others hold zeros.
+// Otherwise a vector that would reach past the end is the row's last 16 bytes instead, so that a load is one
+// instruction without a branch (element by element it is a chain of guarded loads, which every wave waits for:
+// [17225, 127] bf16, LayerNorm backward 26 us and 8): its first spare() elements belong to the vector before, hold the same values
+// there, and are left out of sums.  They may be stored by both, which write the same bits, but not where the
+// store adds to what is there.
+// STREAM: past the caches (whole vectors only).  It is a template argument because of two accesses to one
+// address that differ in nothing but the hint the compiler makes one, without the hint, also where the choice
+// between them is a constant.
+template <typename T, bool ANY, int EPT, int LANES>
+struct LaneRow {
+  static constexpr int V = VecIO<T>::kVec;
+  // only the narrowest form is chosen for rows shorter than a vector
+  static constexpr bool kMayBeShort = ANY && EPT == 1 && LANES == 16;
+  __host__ __device__ static __forceinline__ int count(int N) { return ANY ? (N + V - 1) / V : N / V; }
+  __device__ static __forceinline__ int spare(int v, int N) { return min(max((v + 1) * V - N, 0), V); }
+  // whether some lane's vector j may have spare elements (the same in every lane)
+  __device__ static __forceinline__ bool ragged(int j, int N) { return ANY && (EPT == 1 || (j + 1) * LANES * V > N); }
+  // (v >= 0; ANY needs N >= V unless kMayBeShort)
+  template <bool STREAM = false>
+  __device__ static __forceinline__ u32x4 load_raw(T const *row, int v, int N) {
+    if constexpr (ANY) {
+      if (kMayBeShort && N < V) {
+        float x[V];
+#pragma unroll
+        for (int e = 0; e < V; e++) x[e] = e >= V - N ? VecIO<T>::load1(row + e - (V - N)) : 0.0f;
+        return pack_raw(x, (T const *)nullptr);
+      }
+      return load_raw_any(row + min(v * V, N - V));
+    } else {
+      u32x4 r = {0u, 0u, 0u, 0u};
+      if (v < N / V) {
+        if constexpr (STREAM) {
+          r = load_raw_stream(row + (int64_t)v * V);
+        } else {
+          r = *reinterpret_cast<u32x4 const *>(row + (int64_t)v * V);
+        }
+      }
+      return r;
+    }
+  }
+  template <bool STREAM = false>
+  __device__ static __forceinline__ void load(T const *row, int v, int N, float (&x)[V]) {
+    unpack_raw(load_raw<STREAM>(row, v, N), x, (T const *)nullptr);
+  }
+  // OWN: not the spare elements
+  template <bool STREAM = false, bool OWN = false>
+  __device__ static __forceinline__ void store(T *row, int v, int N, float const (&x)[V]) {
+    if (v >= count(N)) return;
+    if constexpr (ANY) {
+      if (OWN || (kMayBeShort && N < V)) {
+        int const s = spare(v, N);
+#pragma unroll
+        for (int e = 0; e < V; e++) {
+          if (e >= s) VecIO<T>::store1(row + v * V + e - s, x[e]);
+        }
+      } else {
+        store_raw_any(row + min(v * V, N - V), pack_raw(x, (T const *)nullptr));
+      }
+    } else if constexpr (STREAM) {
+      __builtin_nontemporal_store(pack_raw(x, (T const *)nullptr), reinterpret_cast<u32x4 *>(row + (int64_t)v * V));
+    } else {
+      *reinterpret_cast<u32x4 *>(row + (int64_t)v * V) = pack_raw(x, (T const *)nullptr);
+    }
+  }
+};
+
+// Picks (EPT, LANES) for a row of `nvec` 16-byte vectors; returns false when the
 // row does not fit in registers (nvec > 256 * 8).
-static inline bool pick_row_config(int64_t nvec, int &ept, int &wpr) {
+static inline bool pick_row_config(int64_t nvec, int &ept, int &lanes) {
   if (nvec <= 64 * 8) {
-    wpr = 1;
+    lanes = nvec <= 16 ? 16 : nvec <= 32 ? 32 : 64;
     ept = nvec <= 64 ? 1 : nvec <= 128 ? 2 : nvec <= 256 ? 4 : 8;
     return true;
   }
   if (nvec <= 256 * 8) {
-    wpr = 4;
+    lanes = 256;
     ept = nvec <= 256 * 4 ? 4 : 8;
     return true;
   }
   return false;
 }
 
-// Row configuration used by the kernels: one wave per row up to 128 vectors,
+// The LayerNorm kernels': at most one wave per row up to 128 vectors,
 // one workgroup per row beyond (few vectors per lane keeps register use low and
 // measured 76% vs 59% of HBM peak for a [16384, 4096] bf16 LayerNorm forward).
-static inline bool pick_row_config_small(int64_t nvec, int &ept, int &wpr) {
+static inline bool pick_row_config_small(int64_t nvec, int &ept, int &lanes) {
   if (nvec <= 128) {
-    wpr = 1;
+    lanes = nvec <= 16 ? 16 : nvec <= 32 ? 32 : 64;
     ept = nvec <= 64 ? 1 : 2;
     return true;
   }
   if (nvec <= 256 * 8) {
-    wpr = 4;
+    lanes = 256;
     ept = nvec <= 256 ? 1 : nvec <= 512 ? 2 : nvec <= 1024 ? 4 : 8;
     return true;
   }
   return false;
 }
 
-#define FFK_ROW_DISPATCH_SMALL(EPT_, WPR_, CALL)                               \
+#define FFK_ROW_DISPATCH_SMALL(EPT_, LANES_, CALL)                             \
   do {                                                                         \
-    if ((WPR_) == 1) {                                                         \
-      if ((EPT_) == 1) { CALL(1, 1); }                                         \
-      else { CALL(2, 1); }                                                     \
+    if ((LANES_) == 16) {                                                      \
+      CALL(1, 16);                                                             \
+    } else if ((LANES_) == 32) {                                               \
+      CALL(1, 32);                                                             \
+    } else if ((LANES_) == 64) {                                               \
+      if ((EPT_) == 1) { CALL(1, 64); }                                        \
+      else { CALL(2, 64); }                                                    \
     } else {                                                                   \
-      if ((EPT_) == 1) { CALL(1, 4); }                                         \
-      else if ((EPT_) == 2) { CALL(2, 4); }                                    \
-      else if ((EPT_) == 4) { CALL(4, 4); }                                    \
-      else { CALL(8, 4); }                                                     \
+      if ((EPT_) == 1) { CALL(1, 256); }                                       \
+      else if ((EPT_) == 2) { CALL(2, 256); }                                  \
+      else if ((EPT_) == 4) { CALL(4, 256); }                                  \
+      else { CALL(8, 256); }                                                   \
     }                                                                          \
   } while (0)
 
-#define FFK_ROW_DISPATCH(EPT_, WPR_, CALL)                                     \
+#define FFK_ROW_DISPATCH(EPT_, LANES_, CALL)                                   \
   do {                                                                         \
-    if ((WPR_) == 1) {                                                         \
-      if ((EPT_) == 1) { CALL(1, 1); }                                         \
-      else if ((EPT_) == 2) { CALL(2, 1); }                                    \
-      else if ((EPT_) == 4) { CALL(4, 1); }                                    \
-      else { CALL(8, 1); }                                                     \
+    if ((LANES_) == 16) {                                                      \
+      CALL(1, 16);                                                             \
+    } else if ((LANES_) == 32) {                                               \
+      CALL(1, 32);                                                             \
+    } else if ((LANES_) == 64) {                                               \
+      if ((EPT_) == 1) { CALL(1, 64); }                                        \
+      else if ((EPT_) == 2) { CALL(2, 64); }                                   \
+      else if ((EPT_) == 4) { CALL(4, 64); }                                   \
+      else { CALL(8, 64); }                                                    \
     } else {                                                                   \
-      if ((EPT_) == 4) { CALL(4, 4); }                                         \
-      else { CALL(8, 4); }                                                     \
+      if ((EPT_) == 4) { CALL(4, 256); }                                       \
+      else { CALL(8, 256); }                                                   \
     }                                                                          \
   } while (0)
 

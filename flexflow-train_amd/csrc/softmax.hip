@@ -11,19 +11,17 @@
 
 namespace ffk {
 
-// ANY: any row length at any address (RowVec).
-template <typename T, int EPT, int WPR, bool STREAM, bool ANY = false>
+// ANY: any row length at any address (LaneRow).
+template <typename T, int EPT, int LANES, bool STREAM, bool ANY = false>
 __global__ __launch_bounds__(kRowThreads) void softmax_fwd_kernel(
     T const *__restrict__ X, T *__restrict__ Y, int64_t rows, int N) {
   constexpr int V = VecIO<T>::kVec;
-  using RV = RowVec<T, ANY>;
-  constexpr int RPB = 4 / WPR;
-  constexpr int LANES = 64 * WPR;
+  using RV = LaneRow<T, ANY, EPT, LANES>;
   __shared__ float smem[2][4][2];
-  RowReducer<WPR> red(smem);
+  RowReducer<LANES> red(smem);
   int const nvec = RV::count(N);
-  int const lane = WPR == 1 ? (threadIdx.x & 63) : threadIdx.x;
-  int64_t const row = (int64_t)blockIdx.x * RPB + (WPR == 1 ? (threadIdx.x >> 6) : 0);
+  int const lane = threadIdx.x % LANES;
+  int64_t const row = (int64_t)blockIdx.x * (kRowThreads / LANES) + threadIdx.x / LANES;
   bool const row_ok = row < rows;
   T const *xr = X + (row_ok ? row : 0) * (int64_t)N;
   float x[EPT][V];
@@ -31,11 +29,11 @@ __global__ __launch_bounds__(kRowThreads) void softmax_fwd_kernel(
 #pragma unroll
   for (int j = 0; j < EPT; j++) {
     int v = lane + j * LANES;
-    if (v < nvec) {
+    if (ANY || v < nvec) {
       RV::template load<STREAM>(xr, v, N, x[j]);
-      if constexpr (ANY) {
+      if (RV::kMayBeShort && N < V) {
 #pragma unroll
-        for (int e = 0; e < V; e++) x[j][e] = e < RV::elems(v, N) ? x[j][e] : -INFINITY;
+        for (int e = 0; e < V; e++) x[j][e] = e < RV::spare(v, N) ? -INFINITY : x[j][e];
       }
 #pragma unroll
       for (int e = 0; e < V; e++) mx = fmaxf(mx, x[j][e]);
@@ -52,7 +50,7 @@ __global__ __launch_bounds__(kRowThreads) void softmax_fwd_kernel(
     for (int e = 0; e < V; e++) {
       float p = __expf(x[j][e] - mx);
       x[j][e] = p;
-      s += p;
+      s += RV::ragged(j, N) && e < RV::spare(lane + j * LANES, N) ? 0.0f : p;
     }
   }
   s = red.sum(s);
@@ -71,20 +69,18 @@ __global__ __launch_bounds__(kRowThreads) void softmax_fwd_kernel(
   }
 }
 
-// ANY: any row length at any address (RowVec).
-template <typename T, int EPT, int WPR, bool STREAM, bool ANY = false>
+// ANY: any row length at any address (LaneRow).
+template <typename T, int EPT, int LANES, bool STREAM, bool ANY = false>
 __global__ __launch_bounds__(kRowThreads) void softmax_bwd_kernel(
     T const *__restrict__ Y, T const *__restrict__ dY, T *__restrict__ dX,
     int64_t rows, int N) {
   constexpr int V = VecIO<T>::kVec;
-  using RV = RowVec<T, ANY>;
-  constexpr int RPB = 4 / WPR;
-  constexpr int LANES = 64 * WPR;
+  using RV = LaneRow<T, ANY, EPT, LANES>;
   __shared__ float smem[2][4][2];
-  RowReducer<WPR> red(smem);
+  RowReducer<LANES> red(smem);
   int const nvec = RV::count(N);
-  int const lane = WPR == 1 ? (threadIdx.x & 63) : threadIdx.x;
-  int64_t const row = (int64_t)blockIdx.x * RPB + (WPR == 1 ? (threadIdx.x >> 6) : 0);
+  int const lane = threadIdx.x % LANES;
+  int64_t const row = (int64_t)blockIdx.x * (kRowThreads / LANES) + threadIdx.x / LANES;
   bool const row_ok = row < rows;
   int64_t const r = row_ok ? row : 0;
   float y[EPT][V], dy[EPT][V];
@@ -92,12 +88,10 @@ __global__ __launch_bounds__(kRowThreads) void softmax_bwd_kernel(
 #pragma unroll
   for (int j = 0; j < EPT; j++) {
     int v = lane + j * LANES;
-    if (v < nvec) {
-      RV::template load<STREAM>(Y + r * (int64_t)N, v, N, y[j]);
-      RV::template load<STREAM>(dY + r * (int64_t)N, v, N, dy[j]);
+    RV::template load<STREAM>(Y + r * (int64_t)N, v, N, y[j]);
+    RV::template load<STREAM>(dY + r * (int64_t)N, v, N, dy[j]);
 #pragma unroll
-      for (int e = 0; e < V; e++) dot += y[j][e] * dy[j][e];
-    }
+    for (int e = 0; e < V; e++) dot += RV::ragged(j, N) && e < RV::spare(v, N) ? 0.0f : y[j][e] * dy[j][e];
   }
   dot = red.sum(dot);
   if (!row_ok) return;
@@ -160,7 +154,7 @@ template <typename T>
 __global__ __launch_bounds__(kRowThreads) void softmax_fwd_longrow_kernel(
     T const *__restrict__ X, T *__restrict__ Y, int64_t N) {
   __shared__ float smem[2][4][2];
-  RowReducer<4> red(smem);
+  RowReducer<256> red(smem);
   T const *xr = X + (int64_t)blockIdx.x * N;
   T *yr = Y + (int64_t)blockIdx.x * N;
   float mx = -INFINITY;
@@ -179,7 +173,7 @@ __global__ __launch_bounds__(kRowThreads) void softmax_bwd_longrow_kernel(
     T const *__restrict__ Y, T const *__restrict__ dY, T *__restrict__ dX,
     int64_t N) {
   __shared__ float smem[2][4][2];
-  RowReducer<4> red(smem);
+  RowReducer<256> red(smem);
   int64_t const base = (int64_t)blockIdx.x * N;
   float dot = 0.0f;
   for (int64_t j = threadIdx.x; j < N; j += kRowThreads) {
@@ -199,21 +193,21 @@ static int softmax_fwd(hipStream_t st, void const *x, void *y, int64_t outer,
   T const *X = static_cast<T const *>(x);
   T *Y = static_cast<T *>(y);
   if (inner == 1) {
-    int ept = 0, wpr = 0;
-    if (pick_row_config(ceil_div(dim, V), ept, wpr)) {
-      int64_t blocks = ceil_div(outer, 4 / wpr);
+    int ept = 0, lanes = 0;
+    if (pick_row_config(ceil_div(dim, V), ept, lanes)) {
+      int64_t blocks = ceil_div(outer, kRowThreads / lanes);
       bool const vec = dim % V == 0 && aligned16(x) && aligned16(y);
       bool const stream = stream_past_caches(outer * dim, sizeof(T));
-#define CALL(E, W)                                                             \
+#define CALL(E, L)                                                             \
   do {                                                                         \
     if (!vec)                                                                  \
-      softmax_fwd_kernel<T, E, W, false, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(X, Y, outer, (int)dim); \
+      softmax_fwd_kernel<T, E, L, false, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(X, Y, outer, (int)dim); \
     else if (stream)                                                           \
-      softmax_fwd_kernel<T, E, W, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(X, Y, outer, (int)dim); \
+      softmax_fwd_kernel<T, E, L, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(X, Y, outer, (int)dim); \
     else                                                                       \
-      softmax_fwd_kernel<T, E, W, false><<<(unsigned)blocks, kRowThreads, 0, st>>>(X, Y, outer, (int)dim); \
+      softmax_fwd_kernel<T, E, L, false><<<(unsigned)blocks, kRowThreads, 0, st>>>(X, Y, outer, (int)dim); \
   } while (0)
-      FFK_ROW_DISPATCH(ept, wpr, CALL);
+      FFK_ROW_DISPATCH(ept, lanes, CALL);
 #undef CALL
     } else {
       softmax_fwd_longrow_kernel<T><<<(unsigned)outer, kRowThreads, 0, st>>>(X, Y, dim);
@@ -234,21 +228,21 @@ static int softmax_bwd(hipStream_t st, void const *y, void const *dy, void *dx,
   T const *DY = static_cast<T const *>(dy);
   T *DX = static_cast<T *>(dx);
   if (inner == 1) {
-    int ept = 0, wpr = 0;
-    if (pick_row_config(ceil_div(dim, V), ept, wpr)) {
-      int64_t blocks = ceil_div(outer, 4 / wpr);
+    int ept = 0, lanes = 0;
+    if (pick_row_config(ceil_div(dim, V), ept, lanes)) {
+      int64_t blocks = ceil_div(outer, kRowThreads / lanes);
       bool const vec = dim % V == 0 && aligned16(y) && aligned16(dy) && aligned16(dx);
       bool const stream = three_past_caches(outer * dim, sizeof(T));
-#define CALL(E, W)                                                             \
+#define CALL(E, L)                                                             \
   do {                                                                         \
     if (!vec)                                                                  \
-      softmax_bwd_kernel<T, E, W, false, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(Y, DY, DX, outer, (int)dim); \
+      softmax_bwd_kernel<T, E, L, false, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(Y, DY, DX, outer, (int)dim); \
     else if (stream)                                                           \
-      softmax_bwd_kernel<T, E, W, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(Y, DY, DX, outer, (int)dim); \
+      softmax_bwd_kernel<T, E, L, true><<<(unsigned)blocks, kRowThreads, 0, st>>>(Y, DY, DX, outer, (int)dim); \
     else                                                                       \
-      softmax_bwd_kernel<T, E, W, false><<<(unsigned)blocks, kRowThreads, 0, st>>>(Y, DY, DX, outer, (int)dim); \
+      softmax_bwd_kernel<T, E, L, false><<<(unsigned)blocks, kRowThreads, 0, st>>>(Y, DY, DX, outer, (int)dim); \
   } while (0)
-      FFK_ROW_DISPATCH(ept, wpr, CALL);
+      FFK_ROW_DISPATCH(ept, lanes, CALL);
 #undef CALL
     } else {
       softmax_bwd_longrow_kernel<T><<<(unsigned)outer, kRowThreads, 0, st>>>(Y, DY, DX, dim);
