@@ -633,7 +633,8 @@ def embedding_backward(indices, out_grad, weight_grad, aggr=AGGR_NONE, determini
         num_bags = indices.numel() // bag
     ws = None
     ws_bytes = 0
-    if workspace or deterministic:
+    # (few lookups are added without a sort: embedding_match_takes in csrc/embedding_match.h)
+    if deterministic or (workspace and (num_bags * bag * -(-D // 512) > 8192 or D % 4)):
         ws_bytes = _call.ffk_embedding_backward_workspace_bytes(num_bags * bag, V)
         if ws_bytes:
             ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=weight_grad.device)

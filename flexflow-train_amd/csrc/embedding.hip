@@ -5,13 +5,16 @@
 //           int64 offsets throughout (the reference does one element per
 //           thread with `int` offsets and re-reads the index per element,
 //           lib/kernels/src/cuda/embedding_kernels.cu:48-125).
-// backward: weight_grad[indices[b,j],:] += output_grad[b,:] with hardware fp32
-//           atomics, one wave instruction covering 64 consecutive floats of a
-//           row (reference: atomicAdd per element, embedding_kernels.cu:128-317).
+// backward: weight_grad[indices[b,j],:] += output_grad[b,:]: few lookups by one launch that compares all
+//           ids (embedding_match.h), more of them sorted by row (radix_sort.h) and walked
+//           (embedding_walk.h), and without the sort's scratch memory, or where rows are no whole
+//           16 bytes, with hardware fp32 atomics, one wave instruction covering 64 consecutive floats of
+//           a row (reference: atomicAdd per element, embedding_kernels.cu:128-317).
 // Indices outside [0, num_entries) are skipped (the reference reads or writes
 // out of bounds for them).
 #include "ffk_common.h"
 #include "embedding_walk.h"
+#include "embedding_match.h"
 #include "radix_sort.h"
 #include <algorithm>
 #include <cstdlib>
@@ -630,6 +633,11 @@ static int emb_backward(hipStream_t st, void const *indices, void const *dy,
                         int64_t num_entries, float scale, void *workspace,
                         size_t workspace_bytes, bool deterministic) {
   int64_t const lookups = num_bags * bag;
+  if (!deterministic && dim % 4 == 0 && aligned16(dy) && aligned16(dw) && embedding_match_takes(lookups, dim, num_entries)) {
+    FFK_HIP(embedding_match<IT>(st, static_cast<IT const *>(indices), static_cast<GT const *>(dy), dw, (int)lookups, (int)bag,
+                                (int)dim, num_entries, scale));
+    return FFK_OK;
+  }
   EmbSortLayout L;
   bool const sorted = workspace != nullptr && dim % 4 == 0 &&
                       (deterministic || dim <= 65535 * 256) &&  // the walk's grid takes 256 columns a row
