@@ -404,16 +404,24 @@ int attention_f32_backward(hipStream_t st, ffk_attention_desc_t const *d, void c
                            void const *v, void const *o, void const *d_o, float const *lse, float *delta,
                            void *dq, void *dk, void *dv);
 
-// any multiple of 8 up to 256 for either head size (attention_gen.hip)
+// any multiple of 8 up to 256 for either head size (attention_gen.hip); what: bit 0 dQ and delta, bit 1 dK and dV
 int attention_bf16_general_forward(hipStream_t st, ffk_attention_desc_t const *d, void const *q, void const *k,
                                    void const *v, void *o, float *lse);
 int attention_bf16_general_backward(hipStream_t st, ffk_attention_desc_t const *d, void const *q, void const *k,
                                     void const *v, void const *o, void const *d_o, float const *lse,
-                                    float *delta, void *dq, void *dk, void *dv);
+                                    float *delta, void *dq, void *dk, void *dv, int what);
 
 // the kernels of this file and of attention_fwd.hip / attention_bwd.hip: one head size, 64 or 128
 static bool tuned_head_size(ffk_attention_desc_t const *d) {
   return (d->head_dim == 64 || d->head_dim == 128) && (d->v_head_dim == 0 || d->v_head_dim == d->head_dim);
+}
+
+// Whether a kernel of 128 rows a workgroup leaves half of the CUs idle over more than `least` streamed rows: the general kernels, whose waves share out the streamed rows, are then ahead at these head sizes too ([2,
+// 1198] x 4 heads of 64, 80 workgroups: forward 23.4 and 18.7 us, dQ 26.8 and 22.5, dK and dV 50 and 30; heads of
+// 128: 33 and 26, 39 and 33, 62 and 46).  Over fewer rows, or with more workgroups, they are not (48 workgroups of 64,
+// 135 rows: 6.0 and 7.0, 8.0 and 7.4, 11.6 and 9.8; 192 of 128, 385 rows: 18 and 27, 21 and 34, 29 and 35).
+static bool few_workgroups(ffk_attention_desc_t const *d, int64_t rows, int64_t streamed, int64_t least) {
+  return option(FFK_OPTION_ATTENTION_VARIANT) == 0 && streamed > least && ceil_div(rows, 128) * d->heads * d->batch < kNumCU / 2;
 }
 
 static int check_desc(char const *who, int dtype, ffk_attention_desc_t const *d) {
@@ -452,7 +460,7 @@ extern "C" int ffk_attention_forward(ffk_stream_t stream, int dtype,
   if (dtype == FFK_FLOAT) return attention_f32_forward(as_stream(stream), d, q, k, v, o, lse);
   int rc = check_desc("attention_forward", dtype, d);
   if (rc != FFK_OK) return rc;
-  if (!tuned_head_size(d)) return attention_bf16_general_forward(as_stream(stream), d, q, k, v, o, lse);
+  if (!tuned_head_size(d) || few_workgroups(d, d->seq_q, d->seq_kv, 256)) return attention_bf16_general_forward(as_stream(stream), d, q, k, v, o, lse);
   AttnParams p;
   p.q = static_cast<bf16 const *>(q);
   p.k = static_cast<bf16 const *>(k);
@@ -512,7 +520,7 @@ extern "C" int ffk_attention_backward(ffk_stream_t stream, int dtype,
   bool const offsets_fit = d->seq_q * d->q_seq_stride * 2 < lim && d->seq_q * d->o_seq_stride * 2 < lim &&
                            d->seq_kv * d->k_seq_stride * 2 < lim && d->seq_kv * d->v_seq_stride * 2 < lim;
   if (!tuned_head_size(d) || !offsets_fit) {
-    return attention_bf16_general_backward(as_stream(stream), d, q, k, v, o, d_o, lse, delta, dq, dk, dv);
+    return attention_bf16_general_backward(as_stream(stream), d, q, k, v, o, d_o, lse, delta, dq, dk, dv, 3);
   }
   AttnBwdParams p;
   p.q = static_cast<bf16 const *>(q);
@@ -535,14 +543,22 @@ extern "C" int ffk_attention_backward(ffk_stream_t stream, int dtype,
   p.causal = d->causal;
   hipStream_t st = as_stream(stream);
   // dQ first: it computes delta for its rows and leaves it in `delta` for the dK/dV kernel
-  dim3 gq((unsigned)(ceil_div(p.Sq, 128) * p.H * p.B));
-  if (d->head_dim == 64) {
-    attn_bwd_dq_kernel<64><<<gq, 256, 0, st>>>(p);
-  } else {
-    attn_bwd_dq_kernel<128><<<gq, 256, 0, st>>>(p);
+  bool const few_q = few_workgroups(d, d->seq_q, d->seq_kv, 256), few_k = few_workgroups(d, d->seq_kv, d->seq_q, 128);
+  int const general = (few_q ? 1 : 0) | (few_k ? 2 : 0);
+  if (!few_q) {
+    dim3 gq((unsigned)(ceil_div(p.Sq, 128) * p.H * p.B));
+    if (d->head_dim == 64) {
+      attn_bwd_dq_kernel<64><<<gq, 256, 0, st>>>(p);
+    } else {
+      attn_bwd_dq_kernel<128><<<gq, 256, 0, st>>>(p);
+    }
+    FFK_CHECK_LAUNCH();
   }
-  FFK_CHECK_LAUNCH();
-  FFK_HIP(attention_bf16_dkdv(st, p, (int)d->head_dim));
+  if (general != 0) {
+    rc = attention_bf16_general_backward(st, d, q, k, v, o, d_o, lse, delta, dq, dk, dv, general);
+    if (rc != FFK_OK) return rc;
+  }
+  if (!few_k) FFK_HIP(attention_bf16_dkdv(st, p, (int)d->head_dim));
   FFK_CHECK_LAUNCH();
   return FFK_OK;
 }
