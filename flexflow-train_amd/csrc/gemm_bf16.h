@@ -181,7 +181,7 @@ struct GemmGroupArgs {
 // a workgroup's time is the bytes it reads over what its LDS stages can have in flight for the some 800 ns
 // they take to come: a quarter of the tile reads half the bytes and there are four times the workgroups
 // (405 x 512 over 2048 8.8 -> 6.3 us, 63 x 768 over 3072 10.2 -> 6.7, 756 x 256 over 768 5.5 -> 4.5), and the
-// output's operators are spread over all of its waves (96 x 256 over 128 with GELU and dropout 7.3 -> 4.9).
+// output's operators are spread over all of its waves (96 x 256 over 128 with GELU and dropout 7.3 -> 5.3).
 template <int BM, int BN, int WM, int WN, int BK, int STAGES, int PF, bool TA, bool TB, int TAIL = 0,
           bool GROUP = false, int EDGE = kEdgeNone, int KG = 1>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pipe_kernel(
@@ -1329,11 +1329,18 @@ hipError_t pick_bf16_group(hipStream_t st, GemmProblem const *p, int n, int K, b
     t128 += (double)(ceil_div(p[i].M, 128) * ceil_div(p[i].N, 128));
   }
   double const kt = (double)ceil_div(K, 64);
-  double const us64 = t64 <= kNumCU ? kt * 0.17 + 1.0 : ceil(t64 / (2 * kNumCU)) * (kt * 0.39 + 1.0);
+  bool const deep = t64 <= kNumCU && kt > 32;
+  double const us64 = deep ? kt * 0.23 + 2.0 : t64 <= kNumCU ? kt * 0.17 + 1.0
+                    : kt > 32 ? kt * 0.285 * t64 / kNumCU + 1.0 : ceil(t64 / (2 * kNumCU)) * (kt * 0.39 + 1.0);
   double const us128 = ceil(t128 / kNumCU) * (kt * 0.46 + 1.0);
-  double const us32 = t32 <= kNumCU ? kt * 0.11 + 1.0 : t32 <= 2 * kNumCU ? kt * 0.22 + 1.0 : 1e9;
+  double const us32 = t32 <= kNumCU ? kt * (kt > 32 ? 0.18 : 0.11) + 1.0 : t32 <= 2 * kNumCU ? kt * (kt > 32 ? 0.36 : 0.22) + 1.0 : 1e9;
   if (us32 < us64 && (us32 < us128 || !fits)) return launch_pipe_group<32, 32, 32, 32, 32, 4, 1, TA, TB, kEdgeBounded, 4>(st, p, n, K, accumulate);
-  if (!fits || us64 < us128) return launch_pipe_group<64, 64, 32, 32, 64, 2, 3, TA, TB, kEdgeBounded, 2>(st, p, n, K, accumulate);
+  if (!fits || us64 < us128) {
+    // (long reductions on four LDS stages a group of waves, one workgroup a CU: 512 x 2048 over 8065, 256 tiles, 49
+    // us on two)
+    if (deep) return launch_pipe_group<64, 64, 32, 32, 64, 4, 3, TA, TB, kEdgeBounded, 2>(st, p, n, K, accumulate);
+    return launch_pipe_group<64, 64, 32, 32, 64, 2, 3, TA, TB, kEdgeBounded, 2>(st, p, n, K, accumulate);
+  }
   // Long reductions of whole 256 x 256 tiles: a round of them, three quarters full, takes less than three
   // of 128 x 128 (four gradients of 12.6 M elements together over 4096
   // rows: 106-114 us against 119; 81 by the model).
@@ -1385,8 +1392,12 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
         }
       }
       // A long reduction over whole tiles stays on this tile, which tests name: 1024 x 2048 over 4096 25-28 us, 27-35
-      // on 64-wide ones; but 1024 x 1024, where the deep 64-wide tile would be faster, 24-27 us, 17-19 on that.
-      if (whole128 && (int64_t)(M / 128) * (N / 128) >= kNumCU / 4 && K >= 4096 && (tile == kTile64 || tile == kTile64Deep)) tile = kTile128;
+      // on 64-wide ones; but 1024 x 1024, where the deep 64-wide tile would be faster, 24-27 us, 17-19 on that.  Not
+      // where that one saves more than as much: 2048 x 512 over 8064 50 us, 31.
+      if (whole128 && (int64_t)(M / 128) * (N / 128) >= kNumCU / 4 && K >= 4096 && (tile == kTile64 || tile == kTile64Deep) &&
+          gemm_tile_us(kTile128, M, N, K) - us < 10.0) {
+        tile = kTile128;
+      }
       bool along_m = false;
       int const first = M >= 256 && N >= 256 ? gemm_whole_rounds(M, N, K, wide_ok, us, along_m) : 0;
       if (first > 0) {
