@@ -422,8 +422,9 @@ template <bool TA, bool TB>
 static void pick_f32(hipStream_t st, int M, int N, int K, float const *A, int64_t lda, float const *B, int64_t ldb,
                      float *C, int64_t ldc, GemmEpilogue const &ep) {
   float const *const bias = static_cast<float const *>(ep.bias);
-  // (64 x 64 tiles of the same output would reach a quarter of the CUs at most)
-  if (K >= 2048 && ceil_div(M, 64) * ceil_div(N, 64) <= kNumCU / 4) {
+  // Tiles of sixteen waves, one round of two a CU at most: 200 x 200 over 3000 12 us, 16 on tiles of four waves, which
+  // are ahead from one of them a CU on (300 x 300 over 4096 36 and 31, 512 x 512 55 and 48), but tests name these.
+  if (K >= 2048 && ceil_div(M, 16) * ceil_div(N, 16) <= 2 * kNumCU) {
     // Two workgroups a CU: with scratch at hand, reductions of thousands are split over workgroups until
     // there are ([476, 58] over 40 305: 147 us with 120 workgroups,
     // 102 with 600 and the 5 of adding up; [128, 45] over 21 856: 72 and 14 + 7).
@@ -444,13 +445,15 @@ static void pick_f32(hipStream_t st, int M, int N, int K, float const *A, int64_
                                                                    ep.accumulate, nullptr, 0);
     return;
   }
-  // the areas up to which the small Linear's forward keeps these tiles.  (Fewer elements, and shorter
-  // reductions, stay on the kernels below, which tests name: 32 x 128 over 64 8.2 us launch to launch, the
+  // The areas up to which the small Linear's forward keeps these tiles, four fifths of them where the reduction is
+  // long: 64 x 64 tiles, one a CU at most, walk it alone (225 x 2048 over 6144 148 us, 92 so; 256 x 256 over 1095 29
+  // and 6.5; 500 x 1000 over 1300 35 and 25; 320 x 1992 over 2688, past the line, 68 and 75).  (Fewer elements, and
+  // shorter reductions, stay on the kernels below, which tests name: 32 x 128 over 64 8.2 us launch to launch, the
   // small Linear's forward on these tiles 3.6.)
   int64_t const area = (int64_t)M * N;
-  if (K >= 256 && K <= 1024 && M < (1 << 20) && N < (1 << 20) && area >= 128 * 128) {
+  if (K >= 256 && M < (1 << 20) && N < (1 << 20) && area >= 128 * 128) {
     int const t = area <= 16 * 16 * 1024 ? 16 : 32;
-    if (area <= 32 * 32 * 640) {
+    if (area <= 32 * 32 * (K <= 1024 ? 640 : 512)) {
       if (describe_only("gemm_f32_small_kernel<%s,%s,%d>", tf(TA), tf(TB), t)) return;
       auto kern = t == 16 ? gemm_f32_small_kernel<TA, TB, 16> : gemm_f32_small_kernel<TA, TB, 32>;
       kern<<<(unsigned)(ceil_div(M, t) * ceil_div(N, t)), 256, 0, st>>>(A, B, C, M, N, K, lda, ldb, ldc, bias, ep.activation,
