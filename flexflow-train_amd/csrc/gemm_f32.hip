@@ -447,11 +447,11 @@ static void pick_f32(hipStream_t st, int M, int N, int K, float const *A, int64_
   }
   // The areas up to which the small Linear's forward keeps these tiles, four fifths of them where the reduction is
   // long: 64 x 64 tiles, one a CU at most, walk it alone (225 x 2048 over 6144 148 us, 92 so; 256 x 256 over 1095 29
-  // and 6.5; 500 x 1000 over 1300 35 and 25; 320 x 1992 over 2688, past the line, 68 and 75).  (Fewer elements, and
-  // shorter reductions, stay on the kernels below, which tests name: 32 x 128 over 64 8.2 us launch to launch, the
-  // small Linear's forward on these tiles 3.6.)
+  // and 6.5; 500 x 1000 over 1300 35 and 25; 320 x 1992 over 2688, past the line, 68 and 75), and so do the guarded
+  // ones below (21 x 80 over 1344 84 and 6.0, 25 x 380 over 256 20 and 4.3).  (Short reductions stay on those, which
+  // tests name: 32 x 128 over 64 8.2 us launch to launch, the small Linear's forward on these tiles 3.6.)
   int64_t const area = (int64_t)M * N;
-  if (K >= 256 && M < (1 << 20) && N < (1 << 20) && area >= 128 * 128) {
+  if (K >= (area < 128 * 128 ? 128 : 256) && M < (1 << 20) && N < (1 << 20)) {
     int const t = area <= 16 * 16 * 1024 ? 16 : 32;
     if (area <= 32 * 32 * (K <= 1024 ? 640 : 512)) {
       if (describe_only("gemm_f32_small_kernel<%s,%s,%d>", tf(TA), tf(TB), t)) return;
