@@ -471,9 +471,14 @@ static void pick_f32(hipStream_t st, int M, int N, int K, float const *A, int64_
   bool const quads = aligned16(A) && aligned16(B) && lda % 4 == 0 && ldb % 4 == 0 && (TA ? M : K) % 4 == 0 && (TB ? K : N) % 4 == 0 &&
                      M >= 4 && N >= 4;
   // 128 x 128 tiles when they give every CU two workgroups, 128 x 64 when those reach three quarters
-  // of the CUs, 64 x 64 below and where half a 128-row tile would be empty
-  int const tile = M <= 64 ? 2 : ceil_div(M, 128) * ceil_div(N, 128) >= 2 * kNumCU ? 0 :
-                   ceil_div(M, 128) * ceil_div(N, 64) >= kNumCU * 3 / 4 ? 1 : 2;
+  // of the CUs, 64 x 64 below and where half a 128-row tile would be empty.  And 64 x 64 where the CU with the most
+  // of them has less to do than the one with the most of the others: the kernel is bound by the matrix pipe, so an
+  // idle CU is lost (6144 x 512 over 4096, 384 tiles of 128 x 64 or 768 of 64 x 64 on 256 CUs, 263 -> 217 us; 3045 x
+  // 1024 over 3072 202 -> 166; 1500 x 1500 over 1500 103 -> 83; where both have as much, 5% behind).
+  auto busiest = [&](int bm, int bn) { return ceil_div(ceil_div(M, bm) * ceil_div(N, bn), kNumCU) * bm * bn; };
+  int tile = M <= 64 ? 2 : ceil_div(M, 128) * ceil_div(N, 128) >= 2 * kNumCU ? 0 :
+             ceil_div(M, 128) * ceil_div(N, 64) >= kNumCU * 3 / 4 ? 1 : 2;
+  if (tile != 2 && busiest(64, 64) < 0.95 * (double)(tile == 0 ? busiest(128, 128) : busiest(128, 64))) tile = 2;
 #define FFK_F32(BM_, BN_)                                                              \
   do {                                                                                 \
     if (quads)                                                                         \
