@@ -116,13 +116,14 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(
 // MFMA, as in gemm_f32_kernel: the two kernels give the same bits.
 // Rows and columns past the edge are read from the last valid ones and never
 // stored; k past the end is zeroed when the tile is written to LDS.
+// KG: groups of four waves that split the k-tiles, each with LDS buffers of its own, and add up at the end.
 // ANY: lengths and row starts that are no multiple of four elements.  The 16-byte reads then start
 // at any element; a quad that straddles an edge is read element by element from clamped places --
 // of a k-contiguous operand only in the last k-tile, of the others only in the workgroups whose
 // tile reaches past the edge.
 // ---------------------------------------------------------------------------
-template <bool TA, bool TB, int BM, int BN, bool ANY>
-__global__ __launch_bounds__(256, 2) void gemm_f32_tiled_kernel(
+template <bool TA, bool TB, int BM, int BN, bool ANY, int KG>
+__global__ __launch_bounds__(256 * KG, KG == 4 ? 4 : 2) void gemm_f32_tiled_kernel(
     float const *__restrict__ A, float const *__restrict__ B, float *C, int M, int N, int K, int64_t lda,
     int64_t ldb, int64_t ldc, float const *__restrict__ bias, int act, int accumulate) {
   constexpr int BKT = 32;
@@ -132,9 +133,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiled_kernel(
   constexpr int A_SP = 2 * BM + 4, B_SP = 2 * BN + 4;                  // pair-layout row strides
   constexpr int A_FLOATS = A_KC ? (BKT / 2) * A_SP : BKT * BM;
   constexpr int B_FLOATS = B_KC ? (BKT / 2) * B_SP : BKT * BN;
-  __shared__ __attribute__((aligned(16))) float As[2][A_FLOATS];
-  __shared__ __attribute__((aligned(16))) float Bs[2][B_FLOATS];
-  int const t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  __shared__ __attribute__((aligned(16))) float As_all[KG][2][A_FLOATS];
+  __shared__ __attribute__((aligned(16))) float Bs_all[KG][2][B_FLOATS];
+  int const group = KG > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
+  auto &As = As_all[group];
+  auto &Bs = Bs_all[group];
+  int const t = threadIdx.x & 255, lane = t & 63, wave = t >> 6;
   int const h = lane >> 5, l32 = lane & 31;
   int const wm0 = (wave >> 1) * (BM / 2), wn0 = (wave & 1) * (BN / 2);
   int tm, tn;
@@ -159,10 +163,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiled_kernel(
     pg[A_CH + i] = B_KC ? B + (int64_t)min(n0 + c / 8, N - 1) * ldb + 4 * (c % 8)
                         : B + (int64_t)(c / (BN / 4)) * ldb + (ANY ? n0 + 4 * (c % (BN / 4)) : min(n0 + 4 * (c % (BN / 4)), N - 4));
   }
+  // Every group of waves takes as many k-tiles, from `first` on; past the reduction's end they are zeros.
+  int const KT = ((K + BKT - 1) / BKT + KG - 1) / KG, first = group * KT;
   int64_t const step_a = A_KC ? BKT : (int64_t)BKT * lda, step_b = B_KC ? BKT : (int64_t)BKT * ldb;
   // load of chunk i of k-tile kt; pg[i] points at k-tile kt on entry and at kt + 1 on return
   auto gload_chunk = [&](int kt, int i, f32x4 (&rg)[NCH]) __attribute__((always_inline)) {
-    int const k0 = kt * BKT;
+    int const k0 = (first + kt) * BKT;
     bool const is_a = i < A_CH;
     bool const kc = is_a ? A_KC : B_KC;
     // this chunk's tile reaches past the edge along the operand's contiguous index
@@ -200,7 +206,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiled_kernel(
   // chunk i of k-tile kt from its registers into buffer buf, k past the end zeroed
   auto lstore_chunk = [&](int buf, int kt, int i, f32x4 const (&rg)[NCH]) __attribute__((always_inline)) {
     f32x4 const zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    int const k0 = kt * BKT;
+    int const k0 = (first + kt) * BKT;
     bool const is_a = i < A_CH;
     int const c = t + (is_a ? i : i - A_CH) * 256;
     float *dst = is_a ? As[buf] : Bs[buf];
@@ -251,7 +257,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiled_kernel(
 #pragma unroll
       for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
 
-  int const KT = (K + BKT - 1) / BKT;
+  if constexpr (KG > 1) {
+#pragma unroll
+    for (int i = 0; i < NCH; i++) pg[i] += first * (i < A_CH ? step_a : step_b);
+  }
   gload(0, rgs[0]);
   if (KT > 1) gload(1, rgs[1]);
 #pragma unroll
@@ -320,6 +329,35 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiled_kernel(
     tile(kt, T0{}, std::false_type{}, std::false_type{});
   }
 
+  if constexpr (KG > 1) {  // the groups' sums meet in LDS
+    static_assert((KG - 1) * 4 * TMW * TNW * 1024 <= KG * 2 * A_FLOATS, "they fit the tiles' room");
+    float *const sums = &As_all[0][0][0];
+    auto at = [&](int w, int i, int j, int g) {
+      return reinterpret_cast<f32x4 *>(sums) + ((((w * 4 + wave) * TMW + i) * TNW + j) * 4 + g) * 64 + lane;
+    };
+#pragma unroll
+    for (int i = 0; i < TMW; i++)
+#pragma unroll
+      for (int j = 0; j < TNW; j++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          if (group > 0) *at(group - 1, i, j, g) = f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+        }
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int w = 0; w < KG - 1; w++)
+#pragma unroll
+      for (int i = 0; i < TMW; i++)
+#pragma unroll
+        for (int j = 0; j < TNW; j++)
+#pragma unroll
+          for (int g = 0; g < 4; g++) {
+            f32x4 const x = *at(w, i, j, g);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[i][j][4 * g + e] += x[e];
+          }
+  }
   // accumulator element r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of its block
 #pragma unroll
   for (int j = 0; j < TNW; j++) {
@@ -410,11 +448,11 @@ __global__ __launch_bounds__(256) void gemm_f32_splits_kernel(float const *__res
   f32_epilogue(C, ldc, bias, act, accumulate, m, n, v);
 }
 
-template <bool TA, bool TB, int BM, int BN, bool ANY>
+template <bool TA, bool TB, int BM, int BN, bool ANY, int KG>
 static void launch_tiled(hipStream_t st, int M, int N, int K, float const *A, int64_t lda, float const *B, int64_t ldb,
                          float *C, int64_t ldc, GemmEpilogue const &ep) {
-  if (describe_only("gemm_f32_tiled_kernel<%s,%s,%d,%d,%s>", tf(TA), tf(TB), BM, BN, tf(ANY))) return;
-  gemm_f32_tiled_kernel<TA, TB, BM, BN, ANY><<<(int)(ceil_div(M, BM) * ceil_div(N, BN)), 256, 0, st>>>(
+  if (describe_only("gemm_f32_tiled_kernel<%s,%s,%d,%d,%s,%d>", tf(TA), tf(TB), BM, BN, tf(ANY), KG)) return;
+  gemm_f32_tiled_kernel<TA, TB, BM, BN, ANY, KG><<<(int)(ceil_div(M, BM) * ceil_div(N, BN)), 256 * KG, 0, st>>>(
       A, B, C, M, N, K, lda, ldb, ldc, static_cast<float const *>(ep.bias), ep.activation, ep.accumulate);
 }
 
@@ -479,16 +517,27 @@ static void pick_f32(hipStream_t st, int M, int N, int K, float const *A, int64_
   int tile = M <= 64 ? 2 : ceil_div(M, 128) * ceil_div(N, 128) >= 2 * kNumCU ? 0 :
              ceil_div(M, 128) * ceil_div(N, 64) >= kNumCU * 3 / 4 ? 1 : 2;
   if (tile != 2 && busiest(64, 64) < 0.95 * (double)(tile == 0 ? busiest(128, 128) : busiest(128, 64))) tile = 2;
-#define FFK_F32(BM_, BN_)                                                              \
-  do {                                                                                 \
-    if (quads)                                                                         \
-      launch_tiled<TA, TB, BM_, BN_, false>(st, M, N, K, A, lda, B, ldb, C, ldc, ep);  \
-    else                                                                               \
-      launch_tiled<TA, TB, BM_, BN_, true>(st, M, N, K, A, lda, B, ldb, C, ldc, ep);   \
+  // One workgroup a CU: two 64 x 64 tiles a CU become one of 128 x 64, and groups of waves split the reduction, so that
+  // a SIMD has another wave's MFMAs while one waits for its fragments (4096 x 512 over 6144 250 -> 231 us, 1075 x 1024
+  // over 3072 118 -> 104; 1024 x 1024 over 3045 73 -> 62 on two groups, 60 on four, over 752 22.3, 19.8 and 20.0, over
+  // 300 12.3, 11.7 and 13.3, of 1030 x 520 over 200 9.5 and 9.8.  With more workgroups that is so as it is, and the
+  // groups lose: 1866 x 3072 over 1024, 360 tiles of 128 x 64, 104 and 116.)
+  int64_t const t64 = ceil_div(M, 64) * ceil_div(N, 64), t128x64 = ceil_div(M, 128) * ceil_div(N, 64);
+  if (tile == 2 && M > 64 && t64 > kNumCU && t128x64 <= kNumCU) tile = 1;
+  int const kg = K < 256 || (tile == 1 ? t128x64 : t64) > kNumCU ? 1 : tile == 2 && K >= 2048 ? 4 : 2;
+#define FFK_F32(BM_, BN_, KG_)                                                              \
+  do {                                                                                      \
+    if (quads)                                                                              \
+      launch_tiled<TA, TB, BM_, BN_, false, KG_>(st, M, N, K, A, lda, B, ldb, C, ldc, ep);  \
+    else                                                                                    \
+      launch_tiled<TA, TB, BM_, BN_, true, KG_>(st, M, N, K, A, lda, B, ldb, C, ldc, ep);   \
   } while (0)
-  if (tile == 0) FFK_F32(128, 128);
-  else if (tile == 1) FFK_F32(128, 64);
-  else FFK_F32(64, 64);
+  if (tile == 0) FFK_F32(128, 128, 1);
+  else if (tile == 1 && kg == 2) FFK_F32(128, 64, 2);
+  else if (tile == 1) FFK_F32(128, 64, 1);
+  else if (kg == 4) FFK_F32(64, 64, 4);
+  else if (kg == 2) FFK_F32(64, 64, 2);
+  else FFK_F32(64, 64, 1);
 #undef FFK_F32
 }
 
