@@ -25,6 +25,7 @@
 // share their rows (the pair kernels), and tiles go straight to LDS.
 #include "ffk_common.h"
 #include "lds_dma.h"
+#include <type_traits>
 
 namespace ffk {
 
@@ -95,21 +96,21 @@ __device__ __forceinline__ void load_owned_row(float const *row, int D, int h32,
 }
 
 // Streamed tile: global -> registers, registers -> LDS.
-template <int DP>
+template <int DP, int N>
 __device__ __forceinline__ void tile_gload(float const *base, int64_t row_stride, int row0, int last_row, int D,
-                                           int t, f32x4 (&r)[AttnF32Cfg<DP>::kChunks]) {
+                                           int t, f32x4 (&r)[N]) {
 #pragma unroll
-  for (int i = 0; i < AttnF32Cfg<DP>::kChunks; i++) {
+  for (int i = 0; i < N; i++) {
     int const c = t + i * 256;
     int const row = c / (DP / 4), ch = c % (DP / 4);
     int const gr = min(row0 + row, last_row);
     r[i] = load4_or_zero(base + (int64_t)gr * row_stride, ch * 4, D);
   }
 }
-template <int DP, int STRIDE>
-__device__ __forceinline__ void tile_lstore(float *tile, int t, f32x4 const (&r)[AttnF32Cfg<DP>::kChunks]) {
+template <int DP, int STRIDE, int N>
+__device__ __forceinline__ void tile_lstore(float *tile, int t, f32x4 const (&r)[N]) {
 #pragma unroll
-  for (int i = 0; i < AttnF32Cfg<DP>::kChunks; i++) {
+  for (int i = 0; i < N; i++) {
     int const c = t + i * 256;
     int const row = c / (DP / 4), ch = c % (DP / 4);
     *reinterpret_cast<f32x4 *>(tile + row * STRIDE + ch * 4) = r[i];
@@ -181,22 +182,59 @@ __device__ __forceinline__ void contract_rows(float const *tile_lane, float cons
   }
 }
 
+// A wave's accumulators to LDS and back, for the wave that adds them up: 16 bytes a lane, lanes side by side.
+template <int NI>
+__device__ __forceinline__ void acc_put(float *to, f32x16 const (&acc)[NI], int lane) {
+#pragma unroll
+  for (int i = 0; i < NI; i++)
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+      *reinterpret_cast<f32x4 *>(to + ((i * 4 + g) * 64 + lane) * 4) =
+          f32x4{acc[i][4 * g], acc[i][4 * g + 1], acc[i][4 * g + 2], acc[i][4 * g + 3]};
+}
+template <int NI>
+__device__ __forceinline__ void acc_add(float const *from, float factor, f32x16 (&acc)[NI], int lane) {
+#pragma unroll
+  for (int i = 0; i < NI; i++)
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      f32x4 const x = *reinterpret_cast<f32x4 const *>(from + ((i * 4 + g) * 64 + lane) * 4);
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[i][4 * g + e] += x[e] * factor;
+    }
+}
+
 // --------------------------------------------------------------------------
-// forward: workgroup = 128 query rows of one (batch, head), 32 per wave
+// forward: workgroup = 128 / KW query rows of one (batch, head), 32 per group of KW waves, which take the keys of a
+// step of 32 * KW in turn and add up in LDS at the end (for problems that would leave CUs without a workgroup)
 // --------------------------------------------------------------------------
-template <int DP, bool DMA>
+template <int DP, int KW>
+struct AttnF32Fwd {
+  using C = AttnF32Cfg<DP>;
+  static constexpr int kT = 32 * KW, kK = kT * C::kStrideA, kV = kT * C::kStrideB;  // rows of a step, floats of its tiles
+  static constexpr int kBuffers = 2 * (kK + kV) * 4 <= 150 * 1024 ? 2 : 1;
+  static constexpr int kSlot = DP * 32 + 128, kMerge = (KW - 1) * (4 / KW) * kSlot;
+  static constexpr int kFloats = kBuffers * (kK + kV) > kMerge ? kBuffers * (kK + kV) : kMerge;
+  static constexpr int kChunks = kT * DP / 4 / 256;
+};
+template <int DP, bool DMA, int KW>
 __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(AttnF32Params p) {
   using C = AttnF32Cfg<DP>;
-  __shared__ __attribute__((aligned(16))) float Ks[2][C::kTile * C::kStrideA];
-  __shared__ __attribute__((aligned(16))) float Vs[2][C::kTile * C::kStrideB];
+  using F = AttnF32Fwd<DP, KW>;
+  static_assert(KW == 1 || (C::kPrefetch && !DMA), "the split form prefetches into registers");
+  constexpr int T = F::kT, QR = 128 / KW;
+  __shared__ __attribute__((aligned(16))) float pool[F::kFloats];
+  auto Ks = [&](int buf) __attribute__((always_inline)) { return pool + (F::kBuffers == 2 ? buf : 0) * F::kK; };
+  auto Vs = [&](int buf) __attribute__((always_inline)) { return pool + F::kBuffers * F::kK + (F::kBuffers == 2 ? buf : 0) * F::kV; };
   int const t = threadIdx.x, lane = t & 63, h32 = lane >> 5, l32 = lane & 31;
   int const wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  int const nqb = (p.Sq + C::kBlk - 1) / C::kBlk;
+  int const qw = wave / KW, kw = wave % KW;
+  int const nqb = (p.Sq + QR - 1) / QR;
   int const hb = blockIdx.x % (p.H * p.B);
   int const qb = nqb - 1 - blockIdx.x / (p.H * p.B);  // heaviest causal blocks first
   int const head = hb % p.H, b = hb / p.H;
-  int const q0 = qb * C::kBlk;
-  int const qrow = q0 + wave * 32 + l32;
+  int const q0 = qb * QR, qw0 = q0 + qw * 32;
+  int const qrow = qw0 + l32;
   float const *qp = p.q + (int64_t)b * p.q_bs + (int64_t)head * p.Dq;
   float const *kp = p.k + (int64_t)b * p.k_bs + (int64_t)head * p.Dq;
   float const *vp = p.v + (int64_t)b * p.v_bs + (int64_t)head * p.Dv;
@@ -205,8 +243,8 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(AttnF32Params p) {
   load_owned_row<DP>(qp + (int64_t)min(qrow, p.Sq - 1) * p.q_ss, p.Dq, h32, qf);
 
   int kv_end = p.Skv;
-  if (p.causal) kv_end = min(p.Skv, q0 + C::kBlk);
-  int const ntiles = (kv_end + C::kTile - 1) / C::kTile;
+  if (p.causal) kv_end = min(p.Skv, q0 + QR);
+  int const ntiles = (kv_end + T - 1) / T;
 
   f32x16 oacc[DP / 32];
 #pragma unroll
@@ -215,7 +253,7 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(AttnF32Params p) {
     for (int r = 0; r < 16; r++) oacc[i][r] = 0.0f;
   float m_run = -INFINITY, l_run = 0.0f;
 
-  f32x4 rk[C::kChunks], rv[C::kChunks];
+  f32x4 rk[F::kChunks], rv[F::kChunks];
   i32x4 k_rsrc, v_rsrc;
   unsigned k_lane = 0, v_lane = 0;
   if constexpr (DMA) {
@@ -226,8 +264,8 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(AttnF32Params p) {
   }
   auto fetch = [&](int kv0, int buf) {
     if constexpr (DMA) {
-      tile_dma<C::kStrideA>(k_rsrc, k_lane, p.k_ss, kv0, p.Skv - 1, wave, Ks[buf]);
-      tile_dma<C::kStrideB>(v_rsrc, v_lane, p.v_ss, kv0, p.Skv - 1, wave, Vs[buf]);
+      tile_dma<C::kStrideA>(k_rsrc, k_lane, p.k_ss, kv0, p.Skv - 1, wave, Ks(buf));
+      tile_dma<C::kStrideB>(v_rsrc, v_lane, p.v_ss, kv0, p.Skv - 1, wave, Vs(buf));
     } else {
       tile_gload<DP>(kp, p.k_ss, kv0, p.Skv - 1, p.Dq, t, rk);
       tile_gload<DP>(vp, p.v_ss, kv0, p.Skv - 1, p.Dv, t, rv);
@@ -237,8 +275,8 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(AttnF32Params p) {
     if constexpr (DMA) {
       wait_vmcnt<0>();
     } else {
-      tile_lstore<DP, C::kStrideA>(Ks[buf], t, rk);
-      tile_lstore<DP, C::kStrideB>(Vs[buf], t, rv);
+      tile_lstore<DP, C::kStrideA>(Ks(buf), t, rk);
+      tile_lstore<DP, C::kStrideB>(Vs(buf), t, rv);
     }
   };
   fetch(0, 0);
@@ -247,18 +285,18 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(AttnF32Params p) {
   __syncthreads();
   int cur = 0;
   for (int it = 0; it < ntiles; it++) {
-    int const kv0 = it * C::kTile;
+    int const kv0 = it * T + kw * 32;  // this wave's keys
     bool const more = it + 1 < ntiles;
-    if ((DMA || C::kPrefetch) && more) fetch(kv0 + C::kTile, cur ^ 1);
-    // a wave whose rows all lie before this tile (causal) has nothing to add
-    bool const active = !p.causal || kv0 <= q0 + wave * 32 + 31;
+    if ((DMA || C::kPrefetch) && more) fetch((it + 1) * T, cur ^ 1);
+    // a wave whose rows all lie before its keys (causal), or whose keys do not exist, has nothing to add
+    bool const active = (KW == 1 || kv0 < p.Skv) && (!p.causal || kv0 <= qw0 + 31);
     if (active) {
       // S^T: rows = keys of the tile, column = this lane's query
       f32x16 s;
 #pragma unroll
       for (int r = 0; r < 16; r++) s[r] = 0.0f;
-      contract_d<DP>(Ks[cur] + l32 * C::kStrideA + h32 * (DP / 2), qf, s);
-      bool const need_mask = (kv0 + C::kTile > p.Skv) || (p.causal && kv0 + C::kTile - 1 > q0 + wave * 32);
+      contract_d<DP>(Ks(cur) + (kw * 32 + l32) * C::kStrideA + h32 * (DP / 2), qf, s);
+      bool const need_mask = (kv0 + C::kTile > p.Skv) || (p.causal && kv0 + C::kTile - 1 > qw0);
       if (need_mask) {
 #pragma unroll
         for (int r = 0; r < 16; r++) {
@@ -270,14 +308,16 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(AttnF32Params p) {
 #pragma unroll
       for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[r]);
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * p.scale_log2;
-      // finite from the first tile on: key 0 is visible to every query
+      // one wave of a group: finite from the first tile on, key 0 is visible to every query.  Of several, one may so
+      // far have met masked keys alone: its maximum stays -inf, and what it subtracts is 0 instead.
       float const m_new = fmaxf(m_run, mx);
-      float const alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      float const m_sub = KW > 1 && m_new == -INFINITY ? 0.0f : m_new;
+      float const alpha = __builtin_amdgcn_exp2f(m_run - m_sub);
       float sum = 0.0f;
       float pv[16];
 #pragma unroll
       for (int r = 0; r < 16; r++) {
-        pv[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], p.scale_log2, -m_new));
+        pv[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], p.scale_log2, -m_sub));
         sum += pv[r];
       }
       sum += __shfl_xor(sum, 32, 64);
@@ -290,14 +330,43 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(AttnF32Params p) {
           for (int r = 0; r < 16; r++) oacc[i][r] *= alpha;
       }
       // O^T += V^T P^T: A = V^T (row d), B = P^T (column = query), reduction over keys
-      contract_rows<DP / 32, C::kStrideB, true>(Vs[cur] + (4 * h32) * C::kStrideB + l32, pv, oacc);
+      contract_rows<DP / 32, C::kStrideB, true>(Vs(cur) + (kw * 32 + 4 * h32) * C::kStrideB + l32, pv, oacc);
     }
+    if (F::kBuffers == 1) __syncthreads();
     if (more) {
-      if (!DMA && !C::kPrefetch) fetch(kv0 + C::kTile, cur ^ 1);
+      if (!DMA && !C::kPrefetch) fetch((it + 1) * T, cur ^ 1);
       stash(cur ^ 1);
     }
     __syncthreads();
     cur ^= 1;
+  }
+  if constexpr (KW > 1) {
+    float *const slots = pool + qw * (KW - 1) * F::kSlot;
+    if (kw > 0) {
+      float *const mine = slots + (kw - 1) * F::kSlot;
+      acc_put<DP / 32>(mine, oacc, lane);
+      mine[DP * 32 + lane] = m_run;
+      mine[DP * 32 + 64 + lane] = l_run;
+    }
+    __syncthreads();
+    if (kw > 0) return;
+    float m_all = m_run;  // finite: this wave's first keys include key 0
+#pragma unroll
+    for (int w = 0; w < KW - 1; w++) m_all = fmaxf(m_all, slots[w * F::kSlot + DP * 32 + lane]);
+    float const mine = __builtin_amdgcn_exp2f(m_run - m_all);
+    l_run *= mine;
+#pragma unroll
+    for (int i = 0; i < DP / 32; i++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) oacc[i][r] *= mine;
+#pragma unroll
+    for (int w = 0; w < KW - 1; w++) {
+      float const *const other = slots + w * F::kSlot;
+      float const factor = __builtin_amdgcn_exp2f(other[DP * 32 + lane] - m_all);
+      l_run += other[DP * 32 + 64 + lane] * factor;
+      acc_add<DP / 32>(other, factor, oacc, lane);
+    }
+    m_run = m_all;
   }
 
   if (qrow < p.Sq) {
@@ -573,7 +642,8 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dq_kernel(AttnF32Params p) {
 // 64 rows; wave w works on rows 32 * (w % 2) in role w / 2.  Bound by the fp32
 // matrix pipe.  With a wave on its own, dK and dV took two launches (the scores
 // computed in both) and dQ spilled: batch 8 x 8 heads x 512 at
-// head size 256, dK and dV 498 -> 345 us, dQ 309 -> 273.
+// head size 256, dK and dV 498 -> 345 us, dQ 309 -> 273.  KW = 2 (f32_split):
+// both pairs own the same 32 rows and take the streamed rows in turn.
 // --------------------------------------------------------------------------
 struct PairTile {
   f32x4 v[4][64];  // elements 4g .. 4g+3 of each lane's accumulator
@@ -593,17 +663,18 @@ __device__ __forceinline__ void pair_get(PairTile const &x, int lane, float (&e)
 // the waves' LDS writes before it are visible after it; direct loads in flight stay in flight
 __device__ __forceinline__ void pair_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// Streams two operands' 32-row tiles into two buffers each, one tile ahead: by direct loads (DMA), or
+// Streams two operands' tiles of T rows into two buffers each, one tile ahead: by direct loads (DMA), or
 // through registers.
-template <int DP, bool DMA, int STRIDE0, int STRIDE1>
+template <int DP, bool DMA, int STRIDE0, int STRIDE1, int T>
 struct PairStream {
+  static_assert(!DMA || T == 32, "direct loads are written for 32 rows");
   float const *base[2];
   int64_t ss[2];
   int D[2];
   int last, t, lane, wave;
   i32x4 rsrc[2];
   unsigned lane_off[2];
-  f32x4 r0[DMA ? 1 : AttnF32Cfg<DP>::kChunks], r1[DMA ? 1 : AttnF32Cfg<DP>::kChunks];
+  f32x4 r0[DMA ? 1 : T * DP / 4 / 256], r1[DMA ? 1 : T * DP / 4 / 256];
   __device__ __forceinline__ void init() {
     if constexpr (DMA) {
 #pragma unroll
@@ -634,20 +705,22 @@ struct PairStream {
 
 // dK and dV: role 0 computes S and P, hands P over and produces dV; role 1 computes dP and from
 // it and P dS, and produces dK.
-template <int DP, bool DMA>
+template <int DP, bool DMA, int KW>
 __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Params p) {
   using C = AttnF32Cfg<DP>;
-  __shared__ __attribute__((aligned(16))) float Qs[2][C::kTile * C::kStrideB];
-  __shared__ __attribute__((aligned(16))) float Gs[2][C::kTile * C::kStrideB];  // dO
+  constexpr int T = 32 * KW;
+  __shared__ __attribute__((aligned(16))) float Qs[2][T * C::kStrideB];
+  __shared__ __attribute__((aligned(16))) float Gs[2][T * C::kStrideB];  // dO
   __shared__ PairTile Ps[2];
-  __shared__ __attribute__((aligned(16))) float Ls[2][C::kTile], Ds[2][C::kTile];
+  __shared__ __attribute__((aligned(16))) float Ls[2][T], Ds[2][T];
   int const t = threadIdx.x, lane = t & 63, h32 = lane >> 5, l32 = lane & 31;
   int const wave = __builtin_amdgcn_readfirstlane(t >> 6);
   int const blk = wave & 1, role = wave >> 1;
   int const hb = blockIdx.x % (p.H * p.B);
   int const head = hb % p.H, b = hb / p.H;
-  int const kv0 = (blockIdx.x / (p.H * p.B)) * 64 + blk * 32;  // this wave's first key
-  int const kvg = (blockIdx.x / (p.H * p.B)) * 64;             // the workgroup's
+  int const kvg = (blockIdx.x / (p.H * p.B)) * (64 / KW);  // the workgroup's first key
+  int const kv0 = KW == 1 ? kvg + blk * 32 : kvg;           // this wave's
+  int const part = KW == 1 ? 0 : blk * 32;                  // its first query of a step
   int const kvrow = kv0 + l32;
   float const *lsep = p.lse + ((int64_t)b * p.H + head) * p.Sq;
   float const *delp = p.delta + ((int64_t)b * p.H + head) * p.Sq;
@@ -664,9 +737,9 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Para
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[i][r] = 0.0f;
 
-  int const q_begin = p.causal ? (kvg / C::kTile) * C::kTile : 0;
-  int const ntiles = q_begin < p.Sq ? (p.Sq - q_begin + C::kTile - 1) / C::kTile : 0;
-  PairStream<DP, DMA, C::kStrideB, C::kStrideB> st;
+  int const q_begin = p.causal ? (kvg / T) * T : 0;
+  int const ntiles = q_begin < p.Sq ? (p.Sq - q_begin + T - 1) / T : 0;
+  PairStream<DP, DMA, C::kStrideB, C::kStrideB, T> st;
   st.base[0] = p.q + (int64_t)b * p.q_bs + (int64_t)head * p.Dq;
   st.base[1] = p.d_o + (int64_t)b * p.o_bs + (int64_t)head * p.Dv;
   st.ss[0] = p.q_ss; st.ss[1] = p.o_ss;
@@ -675,12 +748,12 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Para
   st.init();
   float rl = 0.0f, rd = 0.0f;
   auto load_row_terms = [&](int qt0) {
-    int const gr = min(qt0 + (t & (C::kTile - 1)), p.Sq - 1);
+    int const gr = min(qt0 + (t & (T - 1)), p.Sq - 1);
     rl = lsep[gr];
     rd = delp[gr];
   };
   auto store_row_terms = [&](int buf) {
-    if (t < C::kTile) {
+    if (t < T) {
       Ls[buf][t] = rl * kLog2eF;
       Ds[buf][t] = rd * p.scale;
     }
@@ -695,27 +768,27 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Para
   __syncthreads();
   int cur = 0;
   for (int it = 0; it < ntiles; it++) {
-    int const qt0 = q_begin + it * C::kTile;
+    int const step0 = q_begin + it * T, qt0 = step0 + part;
     bool const more = it + 1 < ntiles;
     if (more) {
-      load_row_terms(qt0 + C::kTile);
-      st.fetch(qt0 + C::kTile, Qs[cur ^ 1], Gs[cur ^ 1]);
+      load_row_terms(step0 + T);
+      st.fetch(step0 + T, Qs[cur ^ 1], Gs[cur ^ 1]);
     }
-    // waves whose keys all lie after this query tile (causal) contribute nothing
-    bool const active = !p.causal || kv0 <= qt0 + C::kTile - 1;
+    // waves whose keys all lie after their queries (causal), or whose queries do not exist, contribute nothing
+    bool const active = (KW == 1 || qt0 < p.Sq) && (!p.causal || kv0 <= qt0 + 31);
     float ex[16];  // role 0: P, role 1: dS
     f32x16 s;
     if (active) {
       // S = Q K^T or dP = dO V^T: rows = queries of the tile, column = this lane's key
 #pragma unroll
       for (int r = 0; r < 16; r++) s[r] = 0.0f;
-      contract_d<DP>((role == 0 ? Qs[cur] : Gs[cur]) + l32 * C::kStrideB + h32 * (DP / 2), own, s);
+      contract_d<DP>((role == 0 ? Qs[cur] : Gs[cur]) + (part + l32) * C::kStrideB + h32 * (DP / 2), own, s);
       if (role == 0) {
 #pragma unroll
         for (int r = 0; r < 16; r++) {
           int const ql = 8 * (r >> 2) + 4 * h32 + (r & 3);
           int const qg = qt0 + ql;
-          float const e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], p.scale_log2, -Ls[cur][ql]));
+          float const e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], p.scale_log2, -Ls[cur][part + ql]));
           bool const masked = qg >= p.Sq || kvrow >= p.Skv || (p.causal && kvrow > qg);
           ex[r] = masked ? 0.0f : e;
         }
@@ -732,13 +805,13 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Para
           int const qg = qt0 + ql;
           bool const masked = qg >= p.Sq || kvrow >= p.Skv || (p.causal && kvrow > qg);
           // dS = P (dP - delta) scale; Ds holds delta * scale
-          float const ds = ex[r] * __builtin_fmaf(s[r], p.scale, -Ds[cur][ql]);
+          float const ds = ex[r] * __builtin_fmaf(s[r], p.scale, -Ds[cur][part + ql]);
           ex[r] = masked ? 0.0f : ds;
         }
       }
       // dV += P^T dO or dK += dS^T Q: A = the accumulator (row = key), B = rows of the
       // matching query, reduction over the tile's queries
-      contract_rows<DP / 32, C::kStrideB, false>((role == 0 ? Gs[cur] : Qs[cur]) + (4 * h32) * C::kStrideB + l32, ex, acc);
+      contract_rows<DP / 32, C::kStrideB, false>((role == 0 ? Gs[cur] : Qs[cur]) + (part + 4 * h32) * C::kStrideB + l32, ex, acc);
     }
     if (more) {
       st.land(Qs[cur ^ 1], Gs[cur ^ 1]);
@@ -748,6 +821,14 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Para
     cur ^= 1;
   }
 
+  if constexpr (KW > 1) {
+    float *const slot = &Qs[0][0] + role * DP * 32;
+    static_assert(2 * DP * 32 <= 2 * T * C::kStrideB, "the sums fit the tiles' room");
+    if (blk > 0) acc_put<DP / 32>(slot, acc, lane);
+    __syncthreads();
+    if (blk > 0) return;
+    acc_add<DP / 32>(slot, 1.0f, acc, lane);
+  }
   // accumulator element r: key row 8*(r/4) + 4*h + r%4 of this wave's 32, column d = i*32 + l%32
   float *op = role == 0 ? p.dv + (int64_t)b * p.v_bs + (int64_t)head * p.Dv : p.dk + (int64_t)b * p.k_bs + (int64_t)head * p.Dq;
   int64_t const oss = role == 0 ? p.v_ss : p.k_ss;
@@ -765,20 +846,22 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Para
 
 // dQ: role 0 computes S and P, role 1 dP; each hands the other its tile, both form dS, and each
 // produces half of dQ's columns.
-template <int DP, bool DMA>
+template <int DP, bool DMA, int KW>
 __global__ __launch_bounds__(256) void attn_f32_bwd_dq_pair_kernel(AttnF32Params p) {
   using C = AttnF32Cfg<DP>;
-  __shared__ __attribute__((aligned(16))) float Ks[2][C::kTile * C::kStrideB];
-  __shared__ __attribute__((aligned(16))) float Vs[2][C::kTile * C::kStrideA];
+  constexpr int T = 32 * KW, QR = 64 / KW;
+  __shared__ __attribute__((aligned(16))) float Ks[2][T * C::kStrideB];
+  __shared__ __attribute__((aligned(16))) float Vs[2][T * C::kStrideA];
   __shared__ PairTile Xs[2][2];
   int const t = threadIdx.x, lane = t & 63, h32 = lane >> 5, l32 = lane & 31;
   int const wave = __builtin_amdgcn_readfirstlane(t >> 6);
   int const blk = wave & 1, role = wave >> 1;
-  int const nqb = (p.Sq + 63) / 64;
+  int const nqb = (p.Sq + QR - 1) / QR;
   int const hb = blockIdx.x % (p.H * p.B);
   int const qb = nqb - 1 - blockIdx.x / (p.H * p.B);
   int const head = hb % p.H, b = hb / p.H;
-  int const q0 = qb * 64 + blk * 32;  // this wave's first query
+  int const q0 = qb * QR + (KW == 1 ? blk * 32 : 0);  // this wave's first query
+  int const part = KW == 1 ? 0 : blk * 32;             // its first key of a step
   int const qrow = q0 + l32;
   int const rq = min(qrow, p.Sq - 1);
   float own[DP / 2];  // role 0: the row of Q, role 1: of dO
@@ -793,9 +876,9 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dq_pair_kernel(AttnF32Params
     for (int r = 0; r < 16; r++) dq[i][r] = 0.0f;
 
   int kv_end = p.Skv;
-  if (p.causal) kv_end = min(p.Skv, qb * 64 + 64);
-  int const ntiles = (kv_end + C::kTile - 1) / C::kTile;
-  PairStream<DP, DMA, C::kStrideB, C::kStrideA> st;
+  if (p.causal) kv_end = min(p.Skv, qb * QR + QR);
+  int const ntiles = (kv_end + T - 1) / T;
+  PairStream<DP, DMA, C::kStrideB, C::kStrideA, T> st;
   st.base[0] = p.k + (int64_t)b * p.k_bs + (int64_t)head * p.Dq;
   st.base[1] = p.v + (int64_t)b * p.v_bs + (int64_t)head * p.Dv;
   st.ss[0] = p.k_ss; st.ss[1] = p.v_ss;
@@ -808,17 +891,17 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dq_pair_kernel(AttnF32Params
   __syncthreads();
   int cur = 0;
   for (int it = 0; it < ntiles; it++) {
-    int const kt0 = it * C::kTile;
+    int const kt0 = it * T + part;
     bool const more = it + 1 < ntiles;
-    if (more) st.fetch(kt0 + C::kTile, Ks[cur ^ 1], Vs[cur ^ 1]);
-    bool const active = !p.causal || kt0 <= q0 + 31;
+    if (more) st.fetch((it + 1) * T, Ks[cur ^ 1], Vs[cur ^ 1]);
+    bool const active = (KW == 1 || kt0 < p.Skv) && (!p.causal || kt0 <= q0 + 31);
     float ex[16];  // role 0: P, role 1: (dP - delta) scale
     if (active) {
       // S^T = K Q^T or dP^T = V dO^T: rows = keys of the tile, column = this lane's query
       f32x16 s;
 #pragma unroll
       for (int r = 0; r < 16; r++) s[r] = 0.0f;
-      contract_d<DP>(role == 0 ? Ks[cur] + l32 * C::kStrideB + h32 * (DP / 2) : Vs[cur] + l32 * C::kStrideA + h32 * (DP / 2),
+      contract_d<DP>(role == 0 ? Ks[cur] + (part + l32) * C::kStrideB + h32 * (DP / 2) : Vs[cur] + (part + l32) * C::kStrideA + h32 * (DP / 2),
                      own, s);
 #pragma unroll
       for (int r = 0; r < 16; r++) {
@@ -838,13 +921,20 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dq_pair_kernel(AttnF32Params
 #pragma unroll
       for (int r = 0; r < 16; r++) ex[r] *= other[r];
       // dQ^T += K^T dS^T: A = K^T (row d), B = dS^T, reduction over the tile's keys
-      contract_rows<DP / 64, C::kStrideB, true>(Ks[cur] + (4 * h32) * C::kStrideB + role * (DP / 2) + l32, ex, dq);
+      contract_rows<DP / 64, C::kStrideB, true>(Ks[cur] + (part + 4 * h32) * C::kStrideB + role * (DP / 2) + l32, ex, dq);
     }
     if (more) st.land(Ks[cur ^ 1], Vs[cur ^ 1]);
     __syncthreads();
     cur ^= 1;
   }
 
+  if constexpr (KW > 1) {
+    float *const slot = &Ks[0][0] + role * (DP / 2) * 32;
+    if (blk > 0) acc_put<DP / 64>(slot, dq, lane);
+    __syncthreads();
+    if (blk > 0) return;
+    acc_add<DP / 64>(slot, 1.0f, dq, lane);
+  }
   if (qrow < p.Sq) {
     float *dqp = p.dq + (int64_t)b * p.q_bs + (int64_t)qrow * p.q_ss + (int64_t)head * p.Dq;
 #pragma unroll
@@ -910,6 +1000,29 @@ static bool rows_fit_dma(AttnF32Params const &p) {
     else { CALL(256, false); }                                                 \
   } while (0)
 
+// How many waves, or pairs of them, share a group's rows: as many as leave one round of workgroups, two under a causal
+// mask, where half of them are short.  In us by 1, 2, 4 ([B, S, D] x heads; forward, dK and dV by 1, 2):
+//   [3, 305, 128] x 4   60 38 31, 63 38      [5, 219, 64] x 4, causal   27 19 15, 29 20
+//   [5, 215, 128] x 8   45 33 42, 46 60      [2, 600, 128] x 8, causal  101 64 44, 111 69
+//   [2, 376, 64] x 16   44 29 34, 49 55      [5, 609, 128] x 8, causal  111 70 94, 124 131
+static int f32_split(AttnF32Params const &p, int rows_owned, int rows, int streamed, int most) {
+  int64_t const heads = (int64_t)p.H * p.B, limit = p.causal ? 2 * kNumCU : kNumCU;
+  int kw = 1;
+  while (kw < most && heads * ceil_div(rows_owned, rows / (2 * kw)) <= limit && streamed > 32 * kw) kw *= 2;
+  return kw;
+}
+
+template <int DP, bool DMA>
+static void launch_f32_forward(hipStream_t st, AttnF32Params const &p) {
+  int const kw = DP <= 128 ? f32_split(p, p.Sq, 128, p.Skv, 4) : 1;
+  unsigned const grid = (unsigned)(ceil_div(p.Sq, 128 / kw) * p.H * p.B);
+  if constexpr (DP <= 128) {
+    if (kw == 4) return (void)(attn_f32_fwd_kernel<DP, DMA, 4><<<grid, 256, 0, st>>>(p));
+    if (kw == 2) return (void)(attn_f32_fwd_kernel<DP, DMA, 2><<<grid, 256, 0, st>>>(p));
+  }
+  attn_f32_fwd_kernel<DP, DMA, 1><<<grid, 256, 0, st>>>(p);
+}
+
 int attention_f32_forward(hipStream_t st, ffk_attention_desc_t const *d, void const *q, void const *k,
                           void const *v, void *o, float *lse) {
   int rc = check_desc_f32("attention_forward", d);
@@ -920,9 +1033,8 @@ int attention_f32_forward(hipStream_t st, ffk_attention_desc_t const *d, void co
   p.v = static_cast<float const *>(v);
   p.out = static_cast<float *>(o);
   p.lse = lse;
-  unsigned const grid = (unsigned)(ceil_div(p.Sq, 128) * p.H * p.B);
   int const dmax = p.Dq > p.Dv ? p.Dq : p.Dv;
-#define CALL(DP_, DMA_) attn_f32_fwd_kernel<DP_, DMA_><<<grid, 256, 0, st>>>(p)
+#define CALL(DP_, DMA_) launch_f32_forward<DP_, DMA_>(st, p)
   FFK_ATTN_F32_DISPATCH(dmax, CALL);
 #undef CALL
   FFK_CHECK_LAUNCH();
@@ -940,10 +1052,17 @@ static void launch_f32_backward(hipStream_t st, AttnF32Params const &p, int64_t 
     return DP >= 64 && (DP != 128 || ceil_div(rows_owned, 128) * heads < kNumCU);
   };
   if constexpr (DP >= 64) {
-    if (pairs(p.Skv)) {
-      attn_f32_bwd_dkdv_pair_kernel<DP, DMA><<<(unsigned)(ceil_div(p.Skv, 64) * heads), 256, 0, st>>>(p);
-    }
-    if (pairs(p.Sq)) attn_f32_bwd_dq_pair_kernel<DP, DMA><<<(unsigned)(ceil_div(p.Sq, 64) * heads), 256, 0, st>>>(p);
+    auto both = [&](auto split) {
+      constexpr int KW = decltype(split)::value;
+      if (pairs(p.Skv) && f32_split(p, p.Skv, 64, p.Sq, DP <= 128 ? 2 : 1) == KW) {
+        attn_f32_bwd_dkdv_pair_kernel<DP, DMA, KW><<<(unsigned)(ceil_div(p.Skv, 64 / KW) * heads), 256, 0, st>>>(p);
+      }
+      if (pairs(p.Sq) && f32_split(p, p.Sq, 64, p.Skv, DP <= 128 ? 2 : 1) == KW) {
+        attn_f32_bwd_dq_pair_kernel<DP, DMA, KW><<<(unsigned)(ceil_div(p.Sq, 64 / KW) * heads), 256, 0, st>>>(p);
+      }
+    };
+    both(std::integral_constant<int, 1>{});
+    if constexpr (DP <= 128) both(std::integral_constant<int, 2>{});
   }
   if constexpr (DP == 32 || DP == 128) {
     if (!pairs(p.Skv)) attn_f32_bwd_dkdv_kernel<DP><<<(unsigned)(ceil_div(p.Skv, 128) * heads), 256, 0, st>>>(p);
