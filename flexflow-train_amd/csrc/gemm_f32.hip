@@ -521,9 +521,11 @@ static void pick_f32(hipStream_t st, int M, int N, int K, float const *A, int64_
   // a SIMD has another wave's MFMAs while one waits for its fragments (4096 x 512 over 6144 250 -> 231 us, 1075 x 1024
   // over 3072 118 -> 104; 1024 x 1024 over 3045 73 -> 62 on two groups, 60 on four, over 752 22.3, 19.8 and 20.0, over
   // 300 12.3, 11.7 and 13.3, of 1030 x 520 over 200 9.5 and 9.8.  With more workgroups that is so as it is, and the
-  // groups lose: 1866 x 3072 over 1024, 360 tiles of 128 x 64, 104 and 116.)
+  // groups lose: 1866 x 3072 over 1024, 360 tiles of 128 x 64, 104 and 116.)  Not where one column of tiles reads A from
+  // memory just once: half as many workgroups then have fewer reads under way (19253 x 54 over 2048 105 -> 117 us,
+  // 24000 x 56 over 512 25 -> 29; of two columns, 9000 x 112 over 2048, 80 -> 77).
   int64_t const t64 = ceil_div(M, 64) * ceil_div(N, 64), t128x64 = ceil_div(M, 128) * ceil_div(N, 64);
-  if (tile == 2 && M > 64 && t64 > kNumCU && t128x64 <= kNumCU) tile = 1;
+  if (tile == 2 && M > 64 && N > 64 && t64 > kNumCU && t128x64 <= kNumCU) tile = 1;
   int const kg = K < 256 || (tile == 1 ? t128x64 : t64) > kNumCU ? 1 : tile == 2 && K >= 2048 ? 4 : 2;
 #define FFK_F32(BM_, BN_, KG_)                                                              \
   do {                                                                                      \
