@@ -416,10 +416,11 @@ static bool tuned_head_size(ffk_attention_desc_t const *d) {
   return (d->head_dim == 64 || d->head_dim == 128) && (d->v_head_dim == 0 || d->v_head_dim == d->head_dim);
 }
 
-// Whether a kernel of 128 rows a workgroup leaves half of the CUs idle over more than `least` streamed rows: the general kernels, whose waves share out the streamed rows, are then ahead at these head sizes too ([2,
-// 1198] x 4 heads of 64, 80 workgroups: forward 23.4 and 18.7 us, dQ 26.8 and 22.5, dK and dV 50 and 30; heads of
-// 128: 33 and 26, 39 and 33, 62 and 46).  Over fewer rows, or with more workgroups, they are not (48 workgroups of 64,
-// 135 rows: 6.0 and 7.0, 8.0 and 7.4, 11.6 and 9.8; 192 of 128, 385 rows: 18 and 27, 21 and 34, 29 and 35).
+// Whether a kernel of 128 rows a workgroup leaves half of the CUs idle over more than `least` streamed rows: the general
+// kernels, whose waves share out the streamed rows, are then ahead at these head sizes too ([2, 1198] x 4 heads of 64, 80
+// workgroups: forward 23.7 and 22.0 us, dQ 27 and 23, dK and dV 51 and 30; heads of 128: 35 and 31, 41 and 34, 65 and
+// 48).  Over fewer rows, or with more workgroups, they are not (48 workgroups of 64, 135 rows: 6.0 and 7.0, 8.0 and
+// 7.4, 11.6 and 9.8; 192 of 128, 385 rows: 18 and 27, 21 and 34, 29 and 35).
 static bool few_workgroups(ffk_attention_desc_t const *d, int64_t rows, int64_t streamed, int64_t least) {
   return option(FFK_OPTION_ATTENTION_VARIANT) == 0 && streamed > least && ceil_div(rows, 128) * d->heads * d->batch < kNumCU / 2;
 }

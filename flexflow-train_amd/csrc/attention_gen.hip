@@ -133,7 +133,9 @@ template <int DP, int KW>
 __global__ __launch_bounds__(256) void attn_gen_fwd_kernel(AttnGenParams p) {
   using C = GenFwd<DP, KW>;
   constexpr int KS = GenStride<DP>::row, VS = GenStride<DP>::turned, J = C::kJ, QR = 128 / KW;
+  constexpr int NB = KW * J;  // 32-key blocks of a step
   __shared__ __attribute__((aligned(16))) uint8_t pool[C::kBytes];
+  __shared__ float block_max[KW > 1 ? 4 / KW : 1][KW > 1 ? NB : 1][32];
   int const t = threadIdx.x, lane = t & 63, h32 = lane >> 5;
   int const wave = __builtin_amdgcn_readfirstlane(t >> 6);
   int const qw = wave / KW, kw = wave % KW;
@@ -143,6 +145,7 @@ __global__ __launch_bounds__(256) void attn_gen_fwd_kernel(AttnGenParams p) {
   int const head = hb % p.H, b = hb / p.H;
   int const q0 = qb * QR, qw0 = q0 + qw * 32;
   int const qrow = qw0 + (lane & 31);
+  bool const in_pairs = p.Dq == p.Dv && (p.Dq == 64 || p.Dq == 128);
   bf16 const *qp = p.q + (int64_t)b * p.q_bs + (int64_t)head * p.Dq;
   bf16 const *kp = p.k + (int64_t)b * p.k_bs + (int64_t)head * p.Dq;
   bf16 const *vp = p.v + (int64_t)b * p.v_bs + (int64_t)head * p.Dv;
@@ -161,7 +164,7 @@ __global__ __launch_bounds__(256) void attn_gen_fwd_kernel(AttnGenParams p) {
   for (int i = 0; i < DP / 32; i++)
 #pragma unroll
     for (int r = 0; r < 16; r++) oacc[i][r] = 0.0f;
-  float m_run = -INFINITY, l_run = 0.0f;
+  float m_run = -INFINITY, m_own = -INFINITY, l_run = 0.0f;  // largest score of all waves' keys, what P is relative to
 
   GenTile<DP, C::kT> tk, tv;
   auto fetch = [&](int kv0) {
@@ -189,11 +192,13 @@ __global__ __launch_bounds__(256) void attn_gen_fwd_kernel(AttnGenParams p) {
     int const kv0 = it * C::kT + kw * 32 * J;  // this wave's keys
     // a wave whose rows all lie before its keys (causal), or whose keys do not exist, has nothing to add
     bool const active = kv0 < p.Skv && (!p.causal || kv0 <= qw0 + 31);
+    // S^T: rows = keys, column = this lane's query; the largest score of each block of 32 keys
+    f32x16 s[J];
+    float mx[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) mx[j] = -INFINITY;
     if (active) {
       bf16 const *kt = k_tile(cur) + kw * 32 * J * KS + koff;
-      bf16 const *vt = v_tile(cur) + kw * 32 * J * VS + toff;
-      // S^T: rows = keys, column = this lane's query
-      f32x16 s[J];
 #pragma unroll
       for (int j = 0; j < J; j++)
 #pragma unroll
@@ -215,41 +220,70 @@ __global__ __launch_bounds__(256) void attn_gen_fwd_kernel(AttnGenParams p) {
             if (kv >= p.Skv || (p.causal && kv > qrow)) s[j][r] = -INFINITY;
           }
       }
-      float mx = -INFINITY;
 #pragma unroll
-      for (int j = 0; j < J; j++)
+      for (int j = 0; j < J; j++) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[j][r]);
-      mx = max_across_halves(mx) * p.scale_log2;
-      // one wave of a group: finite from the first tile on, key 0 is visible to every query.  Of several, one
-      // may so far have met masked keys alone: its maximum stays -inf, and what it subtracts is 0 instead.
-      float const m_new = fmaxf(m_run, mx);
-      float const m_sub = KW > 1 && m_new == -INFINITY ? 0.0f : m_new;
-      float const alpha = __builtin_amdgcn_exp2f(m_run - m_sub);
-      float sum = 0.0f;
+        for (int r = 0; r < 16; r++) mx[j] = fmaxf(mx[j], s[j][r]);
+        mx[j] = max_across_halves(mx[j]) * p.scale_log2;
+      }
+    }
+    // What P is relative to: the largest score up to its block's end, also of the other waves' blocks, as if one wave
+    // walked them all, blocks of 64 keys at the head sizes of the kernels that step by 64.  P is rounded to bf16, so
+    // with another maximum each of its roundings falls differently, and results of two splits of the rows would be
+    // apart by 1e-3; so they differ in the order of fp32 sums alone (one barrier a step; [2, 1198] x 4 heads of 64, 80
+    // workgroups 22 us, 18.7 with a maximum for each wave, 23.7 without shares).  Finite: key 0 is visible to every
+    // query.
+    float m_block[J], m_step = m_run;
+    if constexpr (KW > 1) {
+      if (lane < 32) {
+#pragma unroll
+        for (int j = 0; j < J; j++) block_max[qw][kw * J + j][lane] = mx[j];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int n = 0; n < NB; n++) {
+        float const now = block_max[qw][n][lane & 31];
+        float const ahead = n % 2 == 0 && in_pairs ? fmaxf(now, block_max[qw][n + 1][lane & 31]) : now;
+        m_step = fmaxf(m_step, ahead);
+#pragma unroll
+        for (int j = 0; j < J; j++)
+          if (n == kw * J + j) m_block[j] = m_step;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < J; j++) {
+        m_step = fmaxf(m_step, j % 2 == 0 && J > 1 && in_pairs ? fmaxf(mx[j], mx[J - 1]) : mx[j]);
+        m_block[j] = m_step;
+      }
+    }
+    m_run = m_step;
+    if (active) {
+      bf16 const *vt = v_tile(cur) + kw * 32 * J * VS + toff;
+      float alpha[J];
       bf16x8 pf[2 * J];
 #pragma unroll
       for (int j = 0; j < J; j++) {
-        float pv[16];
+        alpha[j] = __builtin_amdgcn_exp2f(m_own - m_block[j]);
+        m_own = m_block[j];
+        float sum = 0.0f, pv[16];
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-          pv[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j][r], p.scale_log2, -m_sub));
+          pv[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j][r], p.scale_log2, -m_own));
           sum += pv[r];
         }
         pf[2 * j] = pack8(pv);
         pf[2 * j + 1] = pack8(pv + 8);
+        l_run = l_run * alpha[j] + sum;  // this lane's 16 of every 32 keys; the lane halves meet at the end
       }
-      l_run = l_run * alpha + sum;  // this lane's 16 of every 32 keys; the lane halves meet at the end
-      m_run = m_new;
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
 #pragma unroll
-        for (int i = 0; i < DP / 32; i++)
+      for (int j = 0; j < J; j++) {
+        if (__builtin_amdgcn_ballot_w64(alpha[j] != 1.0f) != 0) {
 #pragma unroll
-          for (int r = 0; r < 16; r++) oacc[i][r] *= alpha;
-      }
-      // O^T += V^T P^T: A = V^T (rows d) through transposing loads, B = P^T
+          for (int i = 0; i < DP / 32; i++)
 #pragma unroll
-      for (int j = 0; j < J; j++)
+            for (int r = 0; r < 16; r++) oacc[i][r] *= alpha[j];
+        }
+        // O^T += V^T P^T: A = V^T (rows d) through transposing loads, B = P^T
 #pragma unroll
         for (int s2 = 0; s2 < 2; s2++)
 #pragma unroll
@@ -257,6 +291,7 @@ __global__ __launch_bounds__(256) void attn_gen_fwd_kernel(AttnGenParams p) {
             bf16x8 const vf = frag_tr_acc(vt, VS, j * 32, s2, i * 32);
             oacc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[2 * j + s2], oacc[i], 0, 0, 0);
           }
+      }
     }
     if (C::kBuffers == 1) __syncthreads();
     if (more) stash(C::kBuffers == 1 ? 0 : cur ^ 1);
@@ -271,15 +306,12 @@ __global__ __launch_bounds__(256) void attn_gen_fwd_kernel(AttnGenParams p) {
     if (kw > 0) {
       float *const mine = slots + (kw - 1) * kSlot;
       gen_put<DP / 32>(mine, oacc, lane);
-      mine[DP * 32 + lane] = m_run;
+      mine[DP * 32 + lane] = m_own;
       mine[DP * 32 + 64 + lane] = l_run;
     }
     __syncthreads();
     if (kw > 0) return;
-    float m_all = m_run;  // finite: this wave's first keys include key 0
-#pragma unroll
-    for (int w = 0; w < KW - 1; w++) m_all = fmaxf(m_all, slots[w * kSlot + DP * 32 + lane]);
-    float const mine = __builtin_amdgcn_exp2f(m_run - m_all);
+    float const mine = __builtin_amdgcn_exp2f(m_own - m_run);  // (m_run is the same in all of them)
     l_run *= mine;
 #pragma unroll
     for (int i = 0; i < DP / 32; i++)
@@ -288,11 +320,10 @@ __global__ __launch_bounds__(256) void attn_gen_fwd_kernel(AttnGenParams p) {
 #pragma unroll
     for (int w = 0; w < KW - 1; w++) {
       float const *const other = slots + w * kSlot;
-      float const factor = __builtin_amdgcn_exp2f(other[DP * 32 + lane] - m_all);
+      float const factor = __builtin_amdgcn_exp2f(other[DP * 32 + lane] - m_run);
       l_run += other[DP * 32 + 64 + lane] * factor;
       gen_add<DP / 32>(other, factor, oacc, lane);
     }
-    m_run = m_all;
   }
   if (qrow < p.Sq) {
     float const inv = 1.0f / l_run;
@@ -875,15 +906,15 @@ static AttnGenParams make_gen_params(ffk_attention_desc_t const *d) {
 //   [2, 1198, 64]  80 WGs   27 19 20 / 34 23 22 / 57 36 30     [3, 390, 80]   96 WGs   15 12 20 / 17 15 16 / 24 18 28
 //   [8, 600, 32]  160 WGs   14  9  8 / 15 11 10 / 18 13 10     [4, 798, 256] 112 WGs   55 39  - / 68 45  -
 //   [16, 403, 80] 256 WGs   17 25 41 / 19 21 31 / 26 36 58     [48, 600, 32] 960 WGs   30 33 38 / 33 39 47 / 48 51 61
-// At a head size of 32 two workgroups a CU are not too many, at 256 one and a half rounds are shorter as three of half
-// the length (360 WGs, dQ, 373 and 338; 448 68 and 90).
+// At a head size of 32 two workgroups a CU are not too many.  ([64, 512, 256] 256 WGs: 45 64 - / 58 76 -, [20, 2297, 256]
+// 360: 305 331 - / 376 360 -.)
 static int gen_split(AttnGenParams const &p, int rows, int streamed, int most, int enough) {
   int kw = 1;
   while (kw < most && (int64_t)p.H * p.B * ceil_div(rows, 128 / kw) < enough && streamed > 32 * kw) kw *= 2;
   return kw;
 }
 template <int DP>
-constexpr int kGenEnough = DP == 32 ? 2 * kNumCU : DP == 256 ? kNumCU * 3 / 2 : kNumCU;
+constexpr int kGenEnough = DP == 32 ? 2 * kNumCU : kNumCU;
 
 template <int DP>
 static void launch_gen_forward(hipStream_t st, AttnGenParams const &p) {
