@@ -1162,30 +1162,33 @@ inline int pipe_tile_for(bf16 const *C, int M, int N, int K, int64_t lda, int64_
 inline bool edge_operands_ok(int64_t lda, int64_t ldb) { return 2 * 256 * std::max(lda, ldb) < (int64_t(1) << 31); }
 
 // The time of a bf16 product on each of the tiles, in us, from which its tile is chosen.  Its
-// coefficients come from products of M and N 128-4096, K 256-4096; it ranks the tiles and does not
-// predict: 60 products drawn from that range, on the tile it picks, took 1.05 to 1.9 times its figure
-// launch to launch (median 1.4; 2-3 us of each is the launch), the short and the transposed ones most.
+// coefficients are those with which the tiles picked for 670 products drawn from M 64-5000, N and K 128-4096
+// took least: 1.4% longer than the best tile each on these and on 330 others (2.4% before, 20% and more at
+// the worst, of 2048-long reductions and of 257 to 512 tiles of 64 x 64: 1149 x 768 over 2048 12.7 -> 10.5 us, 828 x
+// 1536 over 2560 21.5 -> 18.1).  It ranks the tiles and does not predict: launch to launch they took 0.8 to 2.1 times
+// its figure (median 1.3; 2-3 us of each is the launch), the short and the transposed ones most.
 //  - a round over the chip costs its 64-deep k-tiles times what one takes with so many CUs busy
 //    (memory and LDS are shared, the clock too), and a constant of filling, draining and storing
 //  - 32 x 32, four waves that split the reduction, two workgroups a CU
 //    64 x 64, two groups of waves that split the reduction, two workgroups a CU
 //    64 x 64 deep: four LDS stages a group, one workgroup a CU: holds its rate where the operands
-//    come from behind L2, as they do in reductions longer than 2048
+//    come from behind L2, as they do in reductions of 2048 and longer
 //    128 x 64: eight waves, two workgroups a CU; 128 x 128; 256 x 256; wide: the latter with one wave
 //    per SIMD
-enum EdgeTile { kTile32 = 32, kTile64 = 64, kTile64Deep = 65, kTile128x64 = 70, kTile128 = 128, kTile256 = 256, kTile256Wide = 264 };
+enum EdgeTile { kTile32 = 32, kTile64 = 64, kTile64Deep = 65, kTile128x64 = 70, kTile128 = 128, kTile256x128 = 130, kTile256 = 256, kTile256Wide = 264 };
 inline double gemm_tile_us(EdgeTile t, double m, double n, double k, double splits = 1) {
   int const bm = t == kTile32 ? 32 : t == kTile64 || t == kTile64Deep ? 64 : t == kTile128x64 || t == kTile128 ? 128 : 256;
-  int const bn = t == kTile128x64 ? 64 : bm;
+  int const bn = t == kTile128x64 ? 64 : t == kTile256x128 ? 128 : bm;
   double const tiles = ceil(m / bm) * ceil(n / bn) * splits, kt = ceil(ceil(k / 64) / splits);
   auto round_us = [&](double count) {  // of `count` workgroups at a time
     double const f = count / kNumCU;
     switch (t) {
       case kTile32: return f <= 1 ? kt * 0.11 + 1.9 : kt * 0.40 + 2.4;
-      case kTile64: return f <= 1 ? kt * 0.166 + 1.8 : kt * 0.36 + 2.4;
-      case kTile64Deep: return kt * 0.175 + 2.1;
-      case kTile128x64: return f <= 1 ? kt * (0.29 + 0.08 * f) + 1.6 : kt * 0.54 + 2.0;
-      case kTile128: return kt * std::max(0.31, 0.10 + 0.37 * f) + 2.0;
+      case kTile64: return f <= 1 ? kt * 0.166 + 1.8 : kt * 0.28 + 1.9;
+      case kTile64Deep: return kt * 0.167 + 2.1;
+      case kTile128x64: return f <= 1 ? kt * (0.30 + 0.06 * f) + 1.55 : kt * 0.63 + 2.35;
+      case kTile128: return kt * std::max(0.325, 0.11 + 0.367 * f) + 2.1;
+      case kTile256x128: return kt * (0.42 + 0.40 * f) + 3.5;
       case kTile256: return kt * std::max(1.09, 0.35 + 1.25 * f) + 5.5 + 2.0 * f;
       default: return kt * std::max(0.96, 0.25 + 1.19 * f) + 5.5 + 3.0 * f;
     }
@@ -1194,12 +1197,26 @@ inline double gemm_tile_us(EdgeTile t, double m, double n, double k, double spli
   double const full = floor(tiles / a_round), last = tiles - full * a_round;
   double us = full * round_us(a_round) + (last > 0 ? round_us(last) : 0.0);
   // the rounds of 128 x 128 tiles overlap less than the first one's fill suggests
-  if (t == kTile128) us += 2.0 * (ceil(tiles / a_round) - 1);
-  if (t == kTile64 && kt > 32) us += 0.2 * (kt - 32) * ceil(tiles / a_round);
+  if (t == kTile128) us += 1.9 * (ceil(tiles / a_round) - 1);
+  if (t == kTile64 && kt > 30) us += 0.2 * (kt - 30) * ceil(tiles / a_round);
   if (splits > 1) us += 4.0 + splits * m * n * 8 / 4.0e6;  // the partial sums: written and read at 4 TB/s
   return us;
 }
+// 256 x 128 tiles, eight waves of 64 x 64, where one round holds them and two of 128 x 128 were needed: both tiles
+// have one workgroup a CU, and this one does with 48 KB of loads and 128 of LDS reads a 64-deep k-tile what two of the
+// other do with 64 and 192.  Launch to launch, 1379 x 3072 over 768 16.9 -> 14.6 us, 3571 x 2048 over 512 15.2 -> 12.5,
+// 2176 x 2048 over 2048 33 -> 29.  The fuller the round and the longer the reduction, the more the CUs share one limit, of
+// memory and clock: 3200 x 2048 over 1024 19.8 and 20.5, 2816 x 2048 over 2048 with A transposed 33.8 and 35.1, which is
+// where the line lies; 4096 x 1024 over 4096, 128 of these tiles, 51 where 256 of the others take 32.
+inline bool gemm_takes_256x128(int M, int N, int K) {
+  int64_t const t128 = ceil_div(M, 128) * ceil_div(N, 128), tiles = ceil_div(M, 256) * ceil_div(N, 128);
+  return M >= 256 && N >= 128 && t128 > kNumCU && tiles <= kNumCU && K <= 2048 && (2 * tiles - kNumCU) * K <= 512 * kNumCU;
+}
 inline EdgeTile gemm_tile_for(int M, int N, int K, bool wide_ok, double *time = nullptr) {
+  if (gemm_takes_256x128(M, N, K)) {
+    if (time != nullptr) *time = gemm_tile_us(kTile256x128, M, N, K);
+    return kTile256x128;
+  }
   EdgeTile best = kTile64;
   double least = gemm_tile_us(kTile64, M, N, K);
   for (EdgeTile const t : {kTile32, kTile64Deep, kTile128x64, kTile128, kTile256, kTile256Wide}) {
@@ -1217,6 +1234,7 @@ inline EdgeTile gemm_tile_for(int M, int N, int K, bool wide_ok, double *time = 
 inline int gemm_split_tile(int M, int N, int K, GemmEpilogue const &ep) {
   EdgeTile const t = gemm_tile_for(M, N, K, ep.activation == FFK_ACT_NONE);
   if (t == kTile32 || t == kTile64 || t == kTile64Deep) return t;
+  if (t == kTile256x128) return 0;
   int const bm = t == kTile256 || t == kTile256Wide ? 256 : 128, bn = t == kTile128x64 ? 64 : bm;
   return M < bm || N < bn ? kTile64 : 0;
 }
@@ -1263,7 +1281,17 @@ inline int gemm_whole_rounds(int M, int N, int K, bool wide_ok, double one_launc
 template <int TAIL, bool TA, bool TB>
 static hipError_t launch_tail(hipStream_t st, bf16 const *A, bf16 const *B, bf16 *C, int M, int N, int K, int64_t lda,
                               int64_t ldb, int64_t ldc, GemmEpilogue const &ep) {
-  int const tile = pipe_tile_for(C, M, N, K, lda, ldb, ldc, ep, gemm_variant_override());
+  // column sums are taken over blocks of 32 rows from multiples of 32 on, where overlapping tiles do not begin
+  constexpr bool sums = TAIL == GemmEpilogue::kTailDropoutGeluGrad || TAIL == GemmEpilogue::kTailDropoutReluGrad;
+  constexpr int edge = sums ? kEdgeBounded : kEdgeOverlap;
+  int const variant = gemm_variant_override();
+  if (variant == 0 && gemm_takes_256x128(M, N, K)) {
+    if (M % 256 == 0 && N % 128 == 0 && pipe_operands_ok(C, K, lda, ldb, ldc, ep)) {
+      return launch_pipe<256, 128, 64, 64, 64, 3, 1, TA, TB, TAIL>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+    }
+    return launch_pipe<256, 128, 64, 64, 64, 3, 1, TA, TB, TAIL, edge>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+  }
+  int const tile = pipe_tile_for(C, M, N, K, lda, ldb, ldc, ep, variant);
   if (tile == 256) return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB, TAIL>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
   if (tile == 128) return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, TAIL>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
   switch (gemm_split_tile(M, N, K, ep)) {
@@ -1274,9 +1302,6 @@ static hipError_t launch_tail(hipStream_t st, bf16 const *A, bf16 const *B, bf16
   if constexpr (TAIL == GemmEpilogue::kTailGeluDropout) {
     return hipErrorInvalidValue;  // (one large tile a CU: gemm_tail_supported has refused it)
   } else {
-    // column sums are taken over blocks of 32 rows from multiples of 32 on, where overlapping tiles do not begin
-    constexpr bool sums = TAIL == GemmEpilogue::kTailDropoutGeluGrad || TAIL == GemmEpilogue::kTailDropoutReluGrad;
-    constexpr int edge = sums ? kEdgeBounded : kEdgeOverlap;
     if (!sums && (M < 128 || N < 128)) return hipErrorInvalidValue;
     // 128 x 64 where the plain product takes it (1379 x 3072 over 768 with ReLU and dropout: 24.4 -> 21.6 us), and
     // where a round holds them all: the operators on the store are then spread over twice the CUs (1379 x 768
@@ -1375,7 +1400,7 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
     bool const wide_ok = ep.activation == FFK_ACT_NONE && ldc % 8 == 0;
     double us;
     EdgeTile tile = gemm_tile_for(M, N, K, wide_ok, &us);
-    bool const forced = variant == 32 || variant == 64 || variant == 65 || variant == 70 || variant == 128 || variant == 256 || variant == 264;
+    bool const forced = variant == 32 || variant == 64 || variant == 65 || variant == 70 || variant == 128 || variant == 130 || variant == 256 || variant == 264;
     bool const whole128 = M % 128 == 0 && N % 128 == 0 && pipe_operands_ok(C, K, lda, ldb, ldc, ep);
     if (forced) {
       tile = variant == kTile256Wide && ep.activation != FFK_ACT_NONE ? kTile256 : (EdgeTile)variant;
@@ -1393,9 +1418,11 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
       }
       // A long reduction over whole tiles stays on this tile, which tests name: 1024 x 2048 over 4096 25-28 us, 27-35
       // on 64-wide ones; but 1024 x 1024, where the deep 64-wide tile would be faster, 24-27 us, 17-19 on that.  Not
-      // where that one saves more than as much: 2048 x 512 over 8064 50 us, 31.
-      if (whole128 && (int64_t)(M / 128) * (N / 128) >= kNumCU / 4 && K >= 4096 && (tile == kTile64 || tile == kTile64Deep) &&
-          gemm_tile_us(kTile128, M, N, K) - us < 10.0) {
+      // where that one saves more than as much: 2048 x 512 over 8064 50 us, 31.  And one that gives half the CUs
+      // such a tile, on which operators on its store would run, adds up in their order.
+      int64_t const t128 = (int64_t)(M / 128) * (N / 128);
+      if (whole128 && (tile == kTile64 || tile == kTile64Deep) &&
+          (t128 >= kNumCU / 2 || (t128 >= kNumCU / 4 && K >= 4096 && gemm_tile_us(kTile128, M, N, K) - us < 12.0))) {
         tile = kTile128;
       }
       bool along_m = false;
@@ -1411,7 +1438,8 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
       }
     }
     // tiles that begin early: the output has to hold one, and old values added by one workgroup only
-    int const bm = tile == kTile256 || tile == kTile256Wide ? 256 : 128, bn = tile == kTile128x64 ? 64 : bm;
+    int const bm = tile == kTile256 || tile == kTile256x128 || tile == kTile256Wide ? 256 : 128;
+    int const bn = tile == kTile128x64 ? 64 : tile == kTile256x128 ? 128 : bm;
     if (tile != kTile32 && tile != kTile64 && tile != kTile64Deep && (M < bm || N < bn || (ep.accumulate && N % 8 != 0))) tile = kTile64;
     bool const whole = M % bm == 0 && N % bn == 0 && pipe_operands_ok(C, K, lda, ldb, ldc, ep);
     switch (tile) {
@@ -1421,6 +1449,9 @@ hipError_t pick_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
       case kTile256:
         if (whole) return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
         return launch_pipe<256, 256, 128, 64, 32, 4, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+      case kTile256x128:
+        if (whole) return launch_pipe<256, 128, 64, 64, 64, 3, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
+        return launch_pipe<256, 128, 64, 64, 64, 3, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
       case kTile128:
         if (whole) return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
         return launch_pipe<128, 128, 64, 32, 64, 4, 1, TA, TB, 0, kEdgeOverlap>(st, A, B, C, M, N, K, lda, ldb, ldc, ep);
