@@ -34,8 +34,8 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
   __shared__ float smem[2][4][2];
   RowReducer<LANES> red(smem);
   int const nvec = RV::count(N);
-  int const lane = threadIdx.x % LANES;
-  int64_t const row = (int64_t)blockIdx.x * (kRowThreads / LANES) + threadIdx.x / LANES;
+  int const lane = lane_in_row<LANES, kRowThreads>();
+  int64_t const row = (int64_t)blockIdx.x * (kRowThreads / LANES) + row_in_block<LANES, kRowThreads>();
   bool const row_ok = row < M;
   T const *xr = X + (row_ok ? row : 0) * (int64_t)N;
 
@@ -193,8 +193,8 @@ __global__ __launch_bounds__(ln_bwd_threads(EPT, LANES)) void layer_norm_bwd_ker
   __shared__ float smem[2][4][2];
   RowReducer<LANES> red(smem);
   int const nvec = RV::count(N);
-  int const lane = threadIdx.x % LANES;
-  int const sub = threadIdx.x / LANES;
+  int const lane = lane_in_row<LANES, THREADS>();
+  int const sub = row_in_block<LANES, THREADS>();
   float const inv_n = 1.0f / (float)N;
 
   float g[EPT][V], dg[EPT][V], db[EPT][V];

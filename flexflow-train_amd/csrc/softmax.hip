@@ -20,8 +20,8 @@ __global__ __launch_bounds__(kRowThreads) void softmax_fwd_kernel(
   __shared__ float smem[2][4][2];
   RowReducer<LANES> red(smem);
   int const nvec = RV::count(N);
-  int const lane = threadIdx.x % LANES;
-  int64_t const row = (int64_t)blockIdx.x * (kRowThreads / LANES) + threadIdx.x / LANES;
+  int const lane = lane_in_row<LANES, kRowThreads>();
+  int64_t const row = (int64_t)blockIdx.x * (kRowThreads / LANES) + row_in_block<LANES, kRowThreads>();
   bool const row_ok = row < rows;
   T const *xr = X + (row_ok ? row : 0) * (int64_t)N;
   float x[EPT][V];
@@ -79,8 +79,8 @@ __global__ __launch_bounds__(kRowThreads) void softmax_bwd_kernel(
   __shared__ float smem[2][4][2];
   RowReducer<LANES> red(smem);
   int const nvec = RV::count(N);
-  int const lane = threadIdx.x % LANES;
-  int64_t const row = (int64_t)blockIdx.x * (kRowThreads / LANES) + threadIdx.x / LANES;
+  int const lane = lane_in_row<LANES, kRowThreads>();
+  int64_t const row = (int64_t)blockIdx.x * (kRowThreads / LANES) + row_in_block<LANES, kRowThreads>();
   bool const row_ok = row < rows;
   int64_t const r = row_ok ? row : 0;
   float y[EPT][V], dy[EPT][V];
