@@ -376,8 +376,8 @@ __global__ __launch_bounds__(256) void embedding_bwd_sorted_kernel(
   }
 }
 
-// The non-deterministic sorted path of tensors of 4 GB and more, which the walk's 32-bit offsets
-// (embedding_walk.h) do not reach: a wave walks `chunk` consecutive sorted positions, a
+// The non-deterministic sorted path of bags between two ends (the rule in emb_backward) and of tensors of 4 GB and
+// more, which the walk's 32-bit offsets (embedding_walk.h) do not reach: a wave walks `chunk` consecutive sorted positions, a
 // workgroup sixteen such chunks.  Walkers add runs that lie inside their chunk straight to memory;
 // the partial sums of runs that cross a walker border meet in LDS and are merged by the workgroup,
 // so only runs that cross a WORKGROUP border reach memory as atomics.  A row looked up
@@ -667,8 +667,13 @@ static int emb_backward(hipStream_t st, void const *indices, void const *dy,
       FFK_CHECK_LAUNCH();
       return FFK_OK;
     }
-    // 32-bit byte offsets reach all of both tensors
-    if ((uint64_t)num_entries * dim * 4 <= kWalkNowhere && (uint64_t)num_bags * dim * sizeof(GT) <= kWalkNowhere) {
+    // 32-bit byte offsets reach all of both tensors.  Not bags of 65 to 128 columns with 65 536 lookups and
+    // up to four times as many, where the kernel below is ahead (a table's pass, us, that kernel and the walk; 128 columns:
+    // 40 000 lookups 38.0 37.6, 85 700 49.2 52.0, 138 264 58.5 66.3, 200 000 70.9 76.5, 300 000 of 900 000 rows 93.8 90.5,
+    // 524 288 127 116; 96 columns: 138 264 56.5 61.8, 300 000 80.2 76.3; 64 columns: 54.6 56.0 of 50 000 rows, 61.3 58.0 of
+    // 900 000).
+    bool const middling = bag > 1 && dim > 64 && dim <= 128 && lookups >= (1 << 16) && lookups < (1 << 18);
+    if (!middling && (uint64_t)num_entries * dim * 4 <= kWalkNowhere && (uint64_t)num_bags * dim * sizeof(GT) <= kWalkNowhere) {
       WalkArgs const a = {keys_out, vals_out, lookups, 0, (int)bag, (int)dim, (uint32_t)num_entries, scale,
                           (uint32_t)(num_bags * dim * (int64_t)sizeof(GT)), (uint32_t)(num_entries * dim * 4)};
       FFK_HIP(embedding_walk<GT>(st, a, G, dw));
