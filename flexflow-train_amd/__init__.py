@@ -622,8 +622,9 @@ def embedding_forward(indices, weight, aggr=AGGR_NONE, out_dtype=None):
 
 def embedding_backward(indices, out_grad, weight_grad, aggr=AGGR_NONE, deterministic=False,
                        workspace=True):
-    """workspace=True allocates the sort scratch (sorted scatter-add);
-    workspace=False passes none (plain atomics, what a caller without scratch gets)."""
+    """workspace=True allocates the scratch: weight_grad is then this call's alone until it is over
+    (rows are summed in registers and added with loads and stores); workspace=False passes none: plain
+    atomics, beside which other calls may add to weight_grad."""
     torch = _torch()
     V, D = weight_grad.shape
     if aggr == AGGR_NONE:
@@ -633,8 +634,7 @@ def embedding_backward(indices, out_grad, weight_grad, aggr=AGGR_NONE, determini
         num_bags = indices.numel() // bag
     ws = None
     ws_bytes = 0
-    # (few lookups are added without a sort: embedding_match_takes in csrc/embedding_match.h)
-    if deterministic or (workspace and (num_bags * bag * -(-D // 512) > 8192 or D % 4)):
+    if deterministic or workspace:
         ws_bytes = _call.ffk_embedding_backward_workspace_bytes(num_bags * bag, V)
         if ws_bytes:
             ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=weight_grad.device)

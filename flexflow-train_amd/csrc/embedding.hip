@@ -7,7 +7,7 @@
 //           lib/kernels/src/cuda/embedding_kernels.cu:48-125).
 // backward: weight_grad[indices[b,j],:] += output_grad[b,:]: few lookups by one launch that compares all
 //           ids (embedding_match.h), more of them sorted by row (radix_sort.h) and walked
-//           (embedding_walk.h), and without the sort's scratch memory, or where rows are no whole
+//           (embedding_walk.h), and for a caller without the scratch memory, or where rows are no whole
 //           16 bytes, with hardware fp32 atomics, one wave instruction covering 64 consecutive floats of
 //           a row (reference: atomicAdd per element, embedding_kernels.cu:128-317).
 // Indices outside [0, num_entries) are skipped (the reference reads or writes
@@ -633,18 +633,18 @@ static int emb_backward(hipStream_t st, void const *indices, void const *dy,
                         int64_t num_entries, float scale, void *workspace,
                         size_t workspace_bytes, bool deterministic) {
   int64_t const lookups = num_bags * bag;
-  if (!deterministic && dim % 4 == 0 && aligned16(dy) && aligned16(dw) && embedding_match_takes(lookups, dim, num_entries)) {
+  // A caller without the scratch gets atomics whatever the sizes: calls on several streams may then add to one
+  // table at a time.  The kernels behind the scratch add to a row with loads and stores.
+  EmbSortLayout L;
+  bool const alone = workspace != nullptr && reinterpret_cast<uintptr_t>(workspace) % 256 == 0 &&
+                     emb_sort_layout(lookups, num_entries, L) && L.total <= workspace_bytes;
+  bool const vectors = dim % 4 == 0 && aligned16(dy) && aligned16(dw);
+  if (alone && vectors && !deterministic && embedding_match_takes(lookups, dim, num_entries)) {
     FFK_HIP(embedding_match<IT>(st, static_cast<IT const *>(indices), static_cast<GT const *>(dy), dw, (int)lookups, (int)bag,
                                 (int)dim, num_entries, scale));
     return FFK_OK;
   }
-  EmbSortLayout L;
-  bool const sorted = workspace != nullptr && dim % 4 == 0 &&
-                      (deterministic || dim <= 65535 * 256) &&  // the walk's grid takes 256 columns a row
-                      reinterpret_cast<uintptr_t>(dy) % 16 == 0 &&
-                      reinterpret_cast<uintptr_t>(dw) % 16 == 0 &&
-                      reinterpret_cast<uintptr_t>(workspace) % 256 == 0 &&
-                      emb_sort_layout(lookups, num_entries, L) && L.total <= workspace_bytes;
+  bool const sorted = alone && vectors && (deterministic || dim <= 65535 * 256);  // the walk's grid takes 256 columns a row
   if (sorted) {
     uint8_t *ws = static_cast<uint8_t *>(workspace);
     uint32_t *keys_out = nullptr, *vals_out = nullptr;

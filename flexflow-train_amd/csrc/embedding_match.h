@@ -162,7 +162,7 @@ static inline bool embedding_match_takes(int64_t n, int64_t dim, int64_t num_ent
   return n * ceil_div(dim, 512) <= kMatchMax && num_entries < (int64_t)kMatchNone;
 }
 
-// dim % 4 == 0, both tensors 16-byte aligned, embedding_match_takes.
+// dim % 4 == 0, both tensors 16-byte aligned, embedding_match_takes; nothing else adds to dw meanwhile.
 template <typename IT, typename GT>
 static hipError_t embedding_match(hipStream_t st, IT const *idx, GT const *dy, float *dw, int n, int bag, int dim,
                                   int64_t num_entries, float scale) {

@@ -533,11 +533,15 @@ int ffk_layer_norm_backward_residual(
  * backward: weight_grad[indices[b,j],:] += output_grad[b,:] (* 1/bag for AVG),
  *   fp32 accumulators; weight_grad is always accumulated into.
  *   Without workspace: hardware fp32 atomics, one wave instruction per 64
- *   consecutive floats of a row (order, hence rounding, varies run to run).
+ *   consecutive floats of a row (order, hence rounding, varies run to run);
+ *   calls on several streams may add to one weight_grad at the same time.
  *   With workspace of ffk_embedding_backward_workspace_bytes(num_bags*bag,
- *   num_entries) bytes (256-byte aligned) and dim % 4 == 0: lookups are sorted
- *   by row first and runs of equal rows are summed in registers; only runs
- *   that straddle two walkers' chunks still use atomics.
+ *   num_entries) bytes (256-byte aligned) and dim % 4 == 0 the call has
+ *   weight_grad to itself until it is over: it adds to rows with loads and
+ *   stores.  Few lookups (num_bags * bag * ceil(dim / 512) <= 8192) are
+ *   compared with each other in one launch that leaves the workspace alone;
+ *   more are sorted by row first and runs of equal rows summed in registers.
+ *   Atomics remain for rows that many waves or workgroups share.
  *   deterministic == 1 (needs the workspace): every row is summed by one
  *   walker in ascending lookup order, no atomics, bit-reproducible.          */
 /* ------------------------------------------------------------------------ */

@@ -40,3 +40,22 @@ def test_few_lookups(ffk, kind, dim):
             times = torch.bincount(ids[valid], minlength=rows).double()[:, None] + 3
             err = (dw.double() - want).abs()
             assert bool((err <= times * 2.0 ** -24 * size).all()), float((err / size).max())
+
+
+@pytest.mark.parametrize("lookups,dim", [(300, 64), (2000, 128), (8192, 256)])
+def test_calls_without_scratch_add_to_one_table_side_by_side(ffk, lookups, dim):
+    """Atomics: two streams that add to the same rows at a time lose nothing.  Whole numbers, exact in float32."""
+    gen = torch.Generator(device="cuda").manual_seed(lookups)
+    rows, calls = lookups // 3, 40  # three lookups a row: what one wave would load, add to and store back
+    ids = [torch.randint(0, rows, (lookups,), device="cuda", generator=gen) for _ in range(2)]
+    dy = [torch.randint(-4, 5, (lookups, dim), device="cuda", generator=gen).float() for _ in range(2)]
+    dw = torch.zeros(rows, dim, device="cuda")
+    want = calls * sum(torch.zeros(rows, dim, device="cuda").index_add_(0, i, g) for i, g in zip(ids, dy))
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(calls):
+        for s, i, g in zip(streams, ids, dy):
+            with torch.cuda.stream(s):
+                ffk.embedding_backward(i, g, dw, workspace=False)
+    torch.cuda.synchronize()
+    assert torch.equal(dw, want)
