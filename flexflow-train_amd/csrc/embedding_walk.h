@@ -47,9 +47,12 @@ struct WalkShape {
 
 // BAGGED: bags of several entries, whose gradient rows are read once per entry; the weight gradient's then
 // pass by the caches so that those stay (eight tables of 524 288 lookups 1056 us without that, 1036 with it).
-// STREAM: a gradient read once and larger than the caches passes by them itself (316 MB 208 us, 229 without;
-// 134 MB 99 with, 93 without).
-template <typename GT, int LPR, bool BAGGED, bool STREAM>
+// Otherwise a gradient row is read once, and passes by the caches: what it would drive out of them has to be written
+// back first.  Sort and walk, us, with caches full of what another kernel wrote / read / of these tensors, and in
+// brackets with gradient rows that go through the caches: 65 536 x 1024 bf16 82 / 76 / 70 (104 / 76 / 62), 16 384 x 1024
+// bf16 43 / 39 / 34 (48 / 39 / 32), 55 139 x 328 bf16 48 / 46 / 42 (53 / 45 / 39), 21 193 x 1376 fp32 50 / 47 / 43 (72 /
+// 48 / 40).
+template <typename GT, int LPR, bool BAGGED>
 __global__ __launch_bounds__((WalkShape<GT, LPR>::kThreads), (WalkShape<GT, LPR>::kThreads == 1024 ? 8 : 4))
 void embedding_bwd_walk_kernel(WalkArgs a, GT const *dY, float *dW) {
   constexpr int WALKERS = WalkShape<GT, LPR>::kWalkers, NT = WalkShape<GT, LPR>::kThreads, PW = LPR * 4;
@@ -103,7 +106,7 @@ void embedding_bwd_walk_kernel(WalkArgs a, GT const *dY, float *dW) {
     __amdgpu_buffer_rsrc_t const rw = __builtin_amdgcn_make_buffer_rsrc(dW + skip, 0, (int)(a.dw_bytes - skip * 4u), 0x00020000);
     u32x2 const *const mine = meta + (q << a.chunk_shift);
     using Raw = typename std::conditional<sizeof(GT) == 2, u32x2, u32x4>::type;
-    constexpr int aux = STREAM ? kNonTemporal : 0;
+    constexpr int aux = BAGGED ? 0 : kNonTemporal;
     Raw rows[DEPTH];
     u32x4 old[DEPTH];
     uint32_t what[DEPTH];
@@ -191,9 +194,7 @@ static hipError_t embedding_walk_launch(hipStream_t st, WalkArgs a, GT const *dy
     a.chunk_shift++;
   }
   dim3 const grid((unsigned)ceil_div(a.n, (int64_t)Shape::kWalkers << a.chunk_shift), (unsigned)groups);
-  auto kern = a.bag > 1                                                 ? embedding_bwd_walk_kernel<GT, LPR, true, false>
-              : stream_past_caches(a.dy_bytes / sizeof(GT), sizeof(GT)) ? embedding_bwd_walk_kernel<GT, LPR, false, true>
-                                                                        : embedding_bwd_walk_kernel<GT, LPR, false, false>;
+  auto kern = a.bag > 1 ? embedding_bwd_walk_kernel<GT, LPR, true> : embedding_bwd_walk_kernel<GT, LPR, false>;
   kern<<<grid, Shape::kThreads, 0, st>>>(a, dy, dw);
   return hipGetLastError();
 }
