@@ -7,11 +7,11 @@
 // prefix offsets, held in LDS), and then walks the rows.  Forward and the
 // overwriting backward are byte moves (any data type, 16 bytes per lane when
 // every blk_i and pointer allows); the accumulating backward adds in fp32.
+#include "concat_columns.h"
 #include "ffk_common.h"
 
 namespace ffk {
 
-constexpr int kConcatThreads = 256;
 constexpr int kConcatMaxParts = 64;
 
 struct ConcatArgs {
@@ -108,17 +108,7 @@ __global__ __launch_bounds__(kConcatThreads) void concat_kernel(char *cat, Conca
 template <typename U, int MODE>
 static hipError_t concat_launch(hipStream_t st, char *cat, ConcatArgs &a, int64_t window_bytes) {
   a.units_per_row = window_bytes / (int64_t)sizeof(U);
-  // The columns of a workgroup, of which it takes as many rows as it has threads for, so that as few of its
-  // threads as can be are left over (288 columns of 16 bytes, nine parts of 128 floats: 9 x 32, where 256 + 32 had
-  // every other workgroup work with 32 threads; [16384, 9 x 128] 39 us, with four rows of a thread in flight 30,
-  // a copy of that size 25).
-  a.cols_per_wg = 1;
-  int64_t most = 0;
-  for (int cols = (int)(a.units_per_row < kConcatThreads ? a.units_per_row : kConcatThreads); cols >= 1; cols--) {
-    // of 2^20 threads, those with an element
-    int64_t const used = a.units_per_row * (kConcatThreads / cols * cols) * 4096 / (ceil_div(a.units_per_row, cols) * cols);
-    if (used > most + most / 32) most = used, a.cols_per_wg = cols;  // (a few more for shorter pieces of a row are not worth it)
-  }
+  a.cols_per_wg = concat_columns(a.units_per_row, a.num_blocks);
   int const rows_per_wg = kConcatThreads / a.cols_per_wg;
   int64_t const gx = ceil_div(a.units_per_row, a.cols_per_wg);
   int64_t gy = ceil_div(a.num_blocks, rows_per_wg);
