@@ -304,6 +304,13 @@ static int linear_backward_impl(
   }
   bool const act = activation != FFK_ACT_NONE;
   bool const sums = bias_grad != nullptr;
+  // (asked for whichever kernels run: a caller need not know which of them use it)
+  size_t const partial_bytes = sums ? align256((size_t)colsum_partials_elems(batch, out_dim) * sizeof(float)) : 0;
+  auto grad_bytes = [&](int64_t ld) { return align256((size_t)batch * (size_t)ld * dtype_size(dtype)); };
+  size_t const least = partial_bytes + (act ? grad_bytes(out_dim) : 0);
+  if (least > 0 && (workspace == nullptr || workspace_bytes < least)) {
+    return fail(FFK_ERR_WORKSPACE, "linear_backward: workspace of %zu bytes needed, %zu given", least, workspace_bytes);
+  }
   if (dtype == FFK_BF16 && input_tail == nullptr && std::max(std::max(batch, in_dim), out_dim) < (1 << 30) && (input_grad != nullptr || weight_grad != nullptr) &&
       tl_weight_grads == nullptr && option(FFK_OPTION_GEMM_VARIANT) == 0 && option(FFK_OPTION_LAYER_UNFUSED) == 0 &&
       linear_any_takes(batch, in_dim, out_dim, in_dim % 8 == 0 && aligned16(weight) && aligned16(input))) {
@@ -340,12 +347,6 @@ static int linear_backward_impl(
   bool pad = linear_pads_grad(dtype, out_dim) && in_dim % 8 == 0 && input_tail == nullptr && aligned16(weight) &&
              aligned16(input) && (input_grad != nullptr || weight_grad != nullptr) &&
              (sums || act || batch * in_dim * out_dim >= (int64_t(1) << 26));
-  size_t const partial_bytes = sums ? align256((size_t)colsum_partials_elems(batch, out_dim) * sizeof(float)) : 0;
-  auto grad_bytes = [&](int64_t ld) { return align256((size_t)batch * (size_t)ld * dtype_size(dtype)); };
-  size_t const least = partial_bytes + (act ? grad_bytes(out_dim) : 0);
-  if (least > 0 && (workspace == nullptr || workspace_bytes < least)) {
-    return fail(FFK_ERR_WORKSPACE, "linear_backward: workspace of %zu bytes needed, %zu given", least, workspace_bytes);
-  }
   // (a caller that knows the sizes without padding and splits keeps working)
   if (pad && (workspace == nullptr || !aligned16(workspace) ||
               workspace_bytes < partial_bytes + grad_bytes(linear_grad_ld(dtype, out_dim)))) {

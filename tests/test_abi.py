@@ -6,6 +6,9 @@ import random
 import re
 import subprocess
 
+import pytest
+import torch
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
@@ -37,6 +40,24 @@ def test_argument_checks_do_not_need_a_device(ffk):
                                      ffk.AGGR_NONE, 4, 2, 8, 10) == 1
     assert lib.ffk_element_unary_forward(None, ffk.FLOAT, 9999, 0.0, 1, 1, 4) == 3
     assert lib.ffk_gemm(None, ffk.DOUBLE, 0, 0, 4, 4, 4, 1, 1, 1, 0) == 3
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the addresses are made up")
+@pytest.mark.parametrize("shape", [(64, 128, 40), (33, 72, 40), (57, 56, 64), (65, 63, 129), (300, 127, 200)])
+def test_linear_backward_refuses_a_call_without_its_scratch(ffk, shape):
+    """bf16: an activation's gradient and the bias gradient's partial sums need scratch at every size and alignment,
+    whichever kernels run."""
+    batch, in_dim, out_dim = shape
+    y, dy, x, dx, w, dw, db, ws = (ctypes.c_void_p((i + 1) << 24) for i in range(8))
+
+    def call(act, bias, room):
+        return ffk.lib().ffk_linear_backward(None, ffk.BF16, act, 0, y, dy, x, dx, w, dw, db if bias else None, batch,
+                                             in_dim, out_dim, ws if room else None, room, 0)
+
+    for act, bias in ((ffk.ACT_RELU, True), (ffk.ACT_RELU, False), (ffk.ACT_NONE, True)):
+        for room in (0, 64):
+            assert call(act, bias, room) == 4, (act, bias, room)
+            assert b"workspace" in ffk.lib().ffk_last_error()
 
 
 def test_gemm_kernel_name_needs_no_device(ffk):
