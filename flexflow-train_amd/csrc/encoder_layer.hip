@@ -253,6 +253,7 @@ extern "C" int ffk_encoder_layer_backward(ffk_stream_t st, int dtype,
   // one layer: they run as one launch at the end.  Every operand stays as it is until then: they lie in
   // the workspace, but for x in the post-LayerNorm form.
   CollectWeightGrads weight_grads(layer_fusion_enabled());
+  LayerOperators const operators;  // with fusion and without
 
   // ---- tail: y = x1 + f2_drop (pre-LN) or y = LN2(x1 + f2_drop) (post-LN)
   void const *g_sum = dy;  // gradient of (x1 + f2_drop)

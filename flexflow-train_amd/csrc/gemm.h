@@ -106,6 +106,15 @@ struct CollectWeightGrads {
   }
   ~CollectWeightGrads() { tl_weight_grads = saved; }
 };
+// Set while an encoder layer's entry point runs its operators on the calling thread: its Linear backwards then run as
+// a sequence of products, whose bits the fused operators and the sequence of single ones share, and not as the jobs of
+// one launch (linear_any.hip), which add up in another order.
+inline thread_local bool tl_layer_operators = false;
+struct LayerOperators {
+  bool const saved = tl_layer_operators;
+  LayerOperators() { tl_layer_operators = true; }
+  ~LayerOperators() { tl_layer_operators = saved; }
+};
 int weight_grad_dispatch(hipStream_t stream, int dtype, int64_t M, int64_t N, int64_t K, void const *A, int64_t lda,
                          void const *B, int64_t ldb, void *C, int64_t ldc, GemmEpilogue const &ep);
 // Runs what was collected (nothing to do for an empty group) and empties it.

@@ -312,7 +312,7 @@ static int linear_backward_impl(
     return fail(FFK_ERR_WORKSPACE, "linear_backward: workspace of %zu bytes needed, %zu given", least, workspace_bytes);
   }
   if (dtype == FFK_BF16 && input_tail == nullptr && std::max(std::max(batch, in_dim), out_dim) < (1 << 30) && (input_grad != nullptr || weight_grad != nullptr) &&
-      tl_weight_grads == nullptr && option(FFK_OPTION_GEMM_VARIANT) == 0 && option(FFK_OPTION_LAYER_UNFUSED) == 0 &&
+      !tl_layer_operators && option(FFK_OPTION_GEMM_VARIANT) == 0 &&
       linear_any_takes(batch, in_dim, out_dim, in_dim % 8 == 0 && aligned16(weight) && aligned16(input))) {
     size_t const split = linear_split_bytes(dtype, batch, out_dim);
     LinearAnyPlan const plan = linear_any_plan(batch, in_dim, out_dim, split);

@@ -88,3 +88,21 @@ def test_gradient_written_over_the_output_gradient(ffk):
     ffk.linear_backward(y, over, x, w, *got, activation=ffk.ACT_RELU, accumulate=0)
     for a, b, name in zip(apart, got, ("dx", "dw", "db")):
         assert_close(to_np(b), to_np(a), 2.0 ** -7, name)
+
+
+@pytest.mark.parametrize("shape", [(64, 128, 40), (96, 128, 256), (65, 63, 129)])
+def test_the_layer_option_leaves_a_linear_alone(ffk, shape):
+    """What makes an encoder layer run one kernel per operator is no switch of the operators: the same bits either way."""
+    B, I, O = shape
+    gen = torch.Generator(device="cuda").manual_seed(B)
+    x, w, dy = (torch.randn(s, generator=gen, device="cuda").to(BT) for s in ((B, I), (O, I), (B, O)))
+    got = []
+    for value in (0, 1):
+        out = [torch.empty_like(x), torch.empty_like(w), torch.empty(O, dtype=BT, device="cuda")]
+        ffk.set_option(ffk.OPTION_LAYER_UNFUSED, value)
+        try:
+            ffk.linear_backward(None, dy, x, w, *out, accumulate=0)
+        finally:
+            ffk.set_option(ffk.OPTION_LAYER_UNFUSED, 0)
+        got.append(out)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
