@@ -56,8 +56,8 @@ static LayerWs layout(ffk_encoder_layer_desc_t const *d, int dtype) {
   L.mha_reserve = take(a256(ffk_mha_reserve_bytes(&m, dtype)));
   L.ln_ws = take(a256(ffk_layer_norm_backward_workspace_bytes((int64_t)T, d->d_model)));
   L.ln_ws_b = take(a256(ffk_layer_norm_backward_workspace_bytes((int64_t)T, d->d_model)));
-  size_t l1 = ffk_linear_backward_workspace_bytes(dtype, FFK_ACT_RELU, 1, (int64_t)T, d->d_ff);
-  size_t l2 = ffk_linear_backward_workspace_bytes(dtype, FFK_ACT_NONE, 1, (int64_t)T, d->d_model);
+  size_t l1 = linear_sequence_workspace_bytes(dtype, FFK_ACT_RELU, 1, (int64_t)T, d->d_ff);
+  size_t l2 = linear_sequence_workspace_bytes(dtype, FFK_ACT_NONE, 1, (int64_t)T, d->d_model);
   L.lin_ws = take(a256(l1 > l2 ? l1 : l2));
   L.lin_ws_b = take(a256(l1 > l2 ? l1 : l2));
   L.total = off;

@@ -70,6 +70,9 @@ int linear_backward_dropout_gelu(hipStream_t st, int dtype, void const *output_g
                                  // gelu_input, not a GELU with that input
                                  bool relu = false);
 
+// The workspace of a Linear backward that runs as a sequence of products, as an encoder layer's do.
+size_t linear_sequence_workspace_bytes(int dtype, int activation, int use_bias, int64_t batch, int64_t out_dim);
+
 // Linear backward (no activation) whose input gradient is residual + output_grad . weight, the product
 // rounded to the storage type first: what a separate element-wise add of the stored gradient gives.
 // FFK_ERR_UNSUPPORTED as above, before any launch.

@@ -166,20 +166,26 @@ static int64_t linear_grad_ld(int dtype, int64_t out_dim) {
 
 // Room for the partial sums of reductions that are split over workgroups: it lies at the end of the
 // workspace, where it overlaps neither g nor column sums that wait there, and it depends on nothing else
-// the call asks for, so that each gradient has the same bits whatever becomes of the others.
+// the call asks for, so that each gradient has the same bits whatever becomes of the others (but for a bias
+// gradient asked for alone in bf16, whose column sums are a kernel of their own).
 // in_dim is not known here; what the splits can use is bounded all the same.
+//
+// Of the sequence of products, for the input gradient:
 //  fp32: 16 x 16 tiles on two workgroups a CU at most, fewer than 1024 tiles of 1 KB (gemm_f32.hip).
-//  bf16: the jobs of linear_any.hip, on outputs so few that parts of their reductions have to fill the
-//  chip: 512 tiles of 64 x 64 at 16 KB, where a reduction has 512 terms and more.  The input gradient
-//  alone: one round of 256 x 256 tiles in fp32, 64 MB ([2048, 50257] . [50257, 1024] takes all of it: 8
+//  bf16: one round of 256 x 256 tiles in fp32, 64 MB ([2048, 50257] . [50257, 1024] takes all of it: 8
 //  splits, 210 us, 446 without), 16 splits of 2048 columns for few rows.  Shorter reductions, and rows
 //  fewer than a tile's, are not split (gemm_splits_for).
-static size_t linear_split_bytes(int dtype, int64_t batch, int64_t out_dim) {
+static size_t linear_product_split_bytes(int dtype, int64_t batch, int64_t out_dim) {
   if (dtype == FFK_FLOAT) return out_dim >= 2048 ? size_t(1) << 20 : 0;
-  if (dtype != FFK_BF16) return 0;
-  size_t const any = batch >= 512 || out_dim >= 512 ? size_t(8) << 20 : 0;
-  if (out_dim <= 63 * 64 || batch < 128) return any;
-  return std::max(any, batch >= 512 ? size_t(64) << 20 : (size_t)batch << 17);
+  if (dtype != FFK_BF16 || out_dim <= 63 * 64 || batch < 128) return 0;
+  return batch >= 512 ? size_t(64) << 20 : (size_t)batch << 17;
+}
+// Of whichever form the backward takes.  The jobs of one launch (linear_any.hip) cut reductions that are long
+// enough, for outputs so few that parts of them have to fill the chip: 512 parts of 64 x 64 at 16 KB, and where
+// the plan would have more, or larger ones, it makes do.
+static size_t linear_split_bytes(int dtype, int64_t batch, int64_t out_dim) {
+  size_t const any = dtype == FFK_BF16 && linear_any_may_split(batch, out_dim) ? size_t(8) << 20 : 0;
+  return std::max(any, linear_product_split_bytes(dtype, batch, out_dim));
 }
 
 // Whether the two tensors share memory.
@@ -204,10 +210,8 @@ static bool linear_any_takes(int64_t batch, int64_t in_dim, int64_t out_dim, boo
   return k_tiles <= (in_dim <= 128 ? 40000 : 8000);
 }
 
-extern "C" size_t ffk_linear_backward_workspace_bytes(int dtype, int activation,
-                                                      int use_bias,
-                                                      int64_t batch,
-                                                      int64_t out_dim) {
+// g and the column sums
+static size_t linear_gradient_bytes(int dtype, int activation, int use_bias, int64_t batch, int64_t out_dim) {
   size_t bytes = 0;
   if (activation != FFK_ACT_NONE || linear_pads_grad(dtype, out_dim)) {
     bytes += align256((size_t)batch * (size_t)linear_grad_ld(dtype, out_dim) * dtype_size(dtype));
@@ -215,7 +219,14 @@ extern "C" size_t ffk_linear_backward_workspace_bytes(int dtype, int activation,
   if (use_bias) {
     bytes += align256((size_t)colsum_partials_elems(batch, out_dim) * sizeof(float));
   }
-  return bytes + linear_split_bytes(dtype, batch, out_dim);
+  return bytes;
+}
+
+extern "C" size_t ffk_linear_backward_workspace_bytes(int dtype, int activation,
+                                                      int use_bias,
+                                                      int64_t batch,
+                                                      int64_t out_dim) {
+  return linear_gradient_bytes(dtype, activation, use_bias, batch, out_dim) + linear_split_bytes(dtype, batch, out_dim);
 }
 
 extern "C" int ffk_linear_forward(ffk_stream_t stream, int dtype,
@@ -367,7 +378,7 @@ static int linear_backward_impl(
   if (input_grad != nullptr) {
     GemmEpilogue dx = input_tail != nullptr ? *input_tail : ep;
     dx.accumulate = (accumulate & FFK_ACC_INPUT) != 0;
-    size_t const used = partial_bytes + (act || pad ? grad_bytes(ldg) : 0), split = linear_split_bytes(dtype, batch, out_dim);
+    size_t const used = partial_bytes + (act || pad ? grad_bytes(ldg) : 0), split = linear_product_split_bytes(dtype, batch, out_dim);
     if (input_tail == nullptr && split > 0 && aligned16(workspace) && workspace_bytes >= used + split) {
       dx.splitk_ws = ws + ((workspace_bytes - split) & ~(size_t)255);
       // ... of no more partial sums than there are weights: beyond that it depends (4000 x 20 over 2048 in fp32
@@ -421,6 +432,10 @@ extern "C" int ffk_linear_l2_regularizer_grad(ffk_stream_t stream, int dtype, vo
 }
 
 namespace ffk {
+
+size_t linear_sequence_workspace_bytes(int dtype, int activation, int use_bias, int64_t batch, int64_t out_dim) {
+  return linear_gradient_bytes(dtype, activation, use_bias, batch, out_dim) + linear_product_split_bytes(dtype, batch, out_dim);
+}
 
 int linear_gelu_dropout_forward(hipStream_t st, int dtype, void const *input, void *output,
                                 void *dropped, void const *weight, void const *bias, int64_t batch,

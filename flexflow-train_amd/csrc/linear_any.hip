@@ -134,9 +134,8 @@ LinearAnyPlan linear_any_plan(int64_t batch, int64_t in_dim, int64_t out_dim, si
   p.tile = any_tile_for(batch, in_dim, out_dim);
   int64_t const nbn = ceil_div(in_dim, p.tile), tx = ceil_div(batch, p.tile) * nbn, tw = ceil_div(out_dim, p.tile) * nbn;
   int64_t const kx = ceil_div(out_dim, kBK), kw = ceil_div(batch, kBK);
-  // Even shares of the k-tiles for two and a half workgroups a CU (two of the large), but none shorter than
-  // twelve, 5 us: the second launch takes about 4.
-  int64_t const share = std::max<int64_t>(12, ceil_div(tx * kx + tw * kw, p.tile == 64 ? kNumCU * 5 / 2 : kNumCU * 2));
+  // Even shares of the k-tiles for two and a half workgroups a CU (two of the large).
+  int64_t const share = std::max(kLinearAnyShare, ceil_div(tx * kx + tw * kw, p.tile == 64 ? kNumCU * 5 / 2 : kNumCU * 2));
   auto cut = [&](int64_t k, int &splits, int &per) {
     int64_t const s = k * 2 <= share * 3 ? 1 : ceil_div(k, share);
     per = (int)ceil_div(k, s);

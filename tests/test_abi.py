@@ -60,6 +60,25 @@ def test_linear_backward_refuses_a_call_without_its_scratch(ffk, shape):
             assert b"workspace" in ffk.lib().ffk_last_error()
 
 
+def test_linear_backward_asks_for_split_scratch_it_can_use(ffk):
+    """bf16: reductions of up to 18 k-tiles of 64 stay whole, and an encoder layer's Linear backwards are sequences of
+    products, whose reductions of up to 63 tiles do.  Neither has a use for the 8 MB of partial sums."""
+    lib = ffk.lib()
+
+    def linear(batch, out_dim):
+        return lib.ffk_linear_backward_workspace_bytes(ffk.BF16, ffk.ACT_NONE, 0, batch, out_dim)
+
+    assert linear(1152, 1152) == 0
+    assert linear(1153, 64) == linear(64, 1160) == 8 << 20
+
+    def layer(tokens):
+        desc = ffk.EncoderLayerDesc(1, tokens, 256, 4, 1024)
+        return lib.ffk_encoder_layer_workspace_bytes(ctypes.byref(desc), ffk.BF16)
+
+    for tokens in (512, 1153):
+        assert 0 < layer(tokens) - layer(tokens - 1) < 1 << 20, tokens
+
+
 def test_gemm_kernel_name_needs_no_device(ffk):
     """The dispatch answers which kernel a shape runs on without launching anything."""
     big = ffk.gemm_kernel_name(ffk.BF16, False, True, 4096, 4096, 1024, has_bias=True)
