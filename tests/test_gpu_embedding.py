@@ -104,7 +104,11 @@ def test_out_of_range_ids_are_skipped_and_errors(ffk):
 @pytest.mark.parametrize("idt", [torch.int32, torch.int64])
 @pytest.mark.parametrize("gdt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("V,D,B,bag", [(300, 1024, 5000, 1), (50, 64, 2300, 3), (1000, 100, 700, 4),
-                                       (4000, 192, 2049, 2), (7, 256, 4096, 1), (20, 8, 5, 1)])
+                                       (4000, 192, 2049, 2), (7, 256, 4096, 1), (20, 8, 5, 1),
+                                       # past the 8192 lookups that a call with scratch does not sort
+                                       (1000, 100, 2500, 4), (50, 64, 2900, 3), (4000, 192, 4501, 2), (20, 8, 8300, 1),
+                                       # rows of no whole 16 bytes: atomics with scratch and without
+                                       (300, 37, 9000, 1), (40, 7, 500, 3)])
 def test_scatter_add_modes(ffk, oracle, mode, idt, gdt, V, D, B, bag):
     """The three backward paths on the same inputs: plain atomics (no scratch),
     sorted runs summed in registers (scratch given), and the deterministic
@@ -132,6 +136,10 @@ def test_scatter_add_modes(ffk, oracle, mode, idt, gdt, V, D, B, bag):
     kw = dict(atomic=dict(workspace=False), sorted=dict(workspace=True),
               deterministic=dict(deterministic=True))[mode]
     dw = torch.zeros((V, D), device="cuda")
+    if mode == "deterministic" and D % 4 != 0:
+        with pytest.raises(ffk.FFKError, match="deterministic mode needs"):
+            ffk.embedding_backward(to_dev(ids_dev, torch, idt), to_dev(dy, torch, gdt), dw, aggr=aggr, **kw)
+        return
     ffk.embedding_backward(to_dev(ids_dev, torch, idt), to_dev(dy, torch, gdt), dw, aggr=aggr, **kw)
     assert_close(to_np(dw), want, FP32_RTOL, "dW")
     if mode == "deterministic":

@@ -45,8 +45,9 @@ def _case(ffk, n, bag, vocab, dim, index_dtype, grad_dtype, deterministic, skew,
 ])
 @pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])
 def test_sizes_where_the_sort_changes_form(ffk, n, bag, vocab, dim, index_dtype):
-    for skew in (False, True):
-        _case(ffk, n, bag, vocab, dim, index_dtype, torch.float32, False, skew, n + bag)
+    # (up to 8192 lookups only a deterministic call sorts)
+    for skew, deterministic in ((False, False), (True, False), (False, True), (True, True)):
+        _case(ffk, n, bag, vocab, dim, index_dtype, torch.float32, deterministic, skew, n + bag)
 
 
 @pytest.mark.parametrize("dim", [4, 64, 68, 128, 256, 260, 512, 1024, 1600])
@@ -58,7 +59,10 @@ def test_row_lengths_bags_and_modes(ffk, dim, grad_dtype):
 
 
 @pytest.mark.parametrize("dim", [4, 16, 20, 32, 36, 64, 68, 128, 132, 256, 1600])
-@pytest.mark.parametrize("n,bag", [(1, 1), (255, 1), (257, 1), (2049, 1), (683, 3), (70001, 1)])
+@pytest.mark.parametrize("n,bag", [(1, 1), (255, 1), (257, 1), (2049, 1), (683, 3), (70001, 1),
+                                   # past 8192 lookups, which are matched and not walked: a last walker of one
+                                   # position, a workgroup short of one, of one position more, and bags
+                                   (8193, 1), (8447, 1), (8449, 1), (2817, 3)])
 def test_walk_at_its_borders(ffk, dim, n, bag):
     """Walkers of 4 to 64 lanes, the last one short; runs that cross walkers and workgroups (half of the lookups are
     three ids) beside rows looked up once."""
@@ -78,16 +82,30 @@ def test_walk_at_its_borders(ffk, dim, n, bag):
         assert bool((buf[:64] == 1.0).all()) and bool((buf[64 + vocab * dim:] == 1.0).all())
 
 
-def test_table_beyond_32_bit_offsets(ffk):
-    """4.4 GB of weight gradient: row offsets past 2^32 bytes."""
-    vocab, dim, n = 1100000, 1024, 3000
+def _large_table(ffk, vocab, dim, n):
+    """n lookups in the first and the last 700 rows."""
     gen = torch.Generator(device="cuda").manual_seed(3)
     ids = torch.randint(vocab - 700, vocab, (n,), generator=gen, device="cuda")
-    ids[::2] = torch.randint(0, 700, (n // 2,), generator=gen, device="cuda")
-    dy = torch.randint(-4, 5, (n, dim), generator=gen, device="cuda").float()
+    ids[::2] = torch.randint(0, 700, ((n + 1) // 2,), generator=gen, device="cuda")
+    ids[:2] = torch.tensor([vocab - 1, 0], device="cuda")
+    dy = torch.randint(-4, 5, (n, dim), generator=gen, device="cuda", dtype=torch.float32)
     got = torch.zeros((vocab, dim), device="cuda")
     ffk.embedding_backward(ids.view(n, 1), dy, got, aggr=ffk.AGGR_SUM)
     small = torch.zeros((1400, dim), device="cuda")
     small.index_add_(0, torch.where(ids < 700, ids, ids - (vocab - 1400)), dy)
     assert torch.equal(got[:700], small[:700]) and torch.equal(got[-700:], small[700:])
     assert not bool(got[700:-700].any())
+
+
+@pytest.mark.parametrize("n", [3000,   # (rows of 1024 count twice) compared with each other
+                               5000])  # sorted, for the kernel with 64-bit offsets
+def test_table_beyond_32_bit_offsets(ffk, n):
+    """4.4 GB of weight gradient: row offsets past 2^32 bytes."""
+    _large_table(ffk, 1100000, 1024, n)
+
+
+# (0xfffff000 bytes are as far as the walk's offsets reach)
+@pytest.mark.parametrize("vocab,n", [(1048575, 5000), (1048576, 5000),        # the weight gradient's, and one row more
+                                     (3000, 1048575), (3000, 1048576)])       # the output gradient's
+def test_walk_at_the_end_of_its_offsets(ffk, vocab, n):
+    _large_table(ffk, vocab, 1024, n)
