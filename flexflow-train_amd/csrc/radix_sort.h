@@ -544,12 +544,12 @@ static inline RadixSortPlan radix_sort_plan(int64_t n, unsigned key_bits) {
     // with gather and walk; at 28 tiles the counts ahead cost more, 42 -> 47 us for 28 474 ids); beyond 131 072
     // lookups, where each pass has a histogram launch of its own, a third launch adds it up once (524 288 ids
     // below a million: two passes of 18-21 us instead of three of 17).  In between, neither pays.
+    // (Such digits have nine or ten bits, of which the scan's workgroups take 64 at a time.)
     int const wide_passes = (int)((key_bits + 9) / 10);
     p.wide = wide_passes < p.passes && (p.ntiles <= kSortWideTiles || p.items > 1);
     if (p.wide) p.passes = wide_passes;
     p.scanned = p.wide && p.items > 1 && p.ntiles > 1;
     p.bits = (int)((key_bits + p.passes - 1) / p.passes);
-    if (p.scanned && p.bits < 6) p.bits = 6;  // the scan's workgroups take 64 digits
     p.table_bytes = p.scanned ? ((size_t)(p.ntiles + 1) << p.bits) * sizeof(uint32_t)
                               : ((size_t)p.ntiles << p.bits) * (size_t)p.passes * sizeof(uint32_t);
   } else {
