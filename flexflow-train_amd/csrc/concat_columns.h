@@ -9,7 +9,7 @@ constexpr int kConcatThreads = 256;
 // A workgroup takes as many rows, of those there are, as it has threads for.  It takes all columns it can, or, where
 // that leaves more than a 32nd fewer threads over, an even share of one more piece of the row and up to three more, or
 // a power of two down to eight (288 columns of 16 bytes, nine parts of 128 floats: 9 x 32, where 256 + 32 had every
-// other workgroup work with 32 threads; [16384, 9 x 128] 39 us, with four rows of a thread in flight 30, a copy of that
+// other workgroup work with 32 threads; [16384, 9 x 128] 39 us, with four rows of a thread in flight 28, a copy of that
 // size 25).  These widths take 0.04 us of a call's host time, where all 256 took 2.3 and left 2% fewer threads over.
 inline int concat_columns(int64_t units_per_row, int64_t rows) {
   int64_t const fewest = (units_per_row + kConcatThreads - 1) / kConcatThreads;

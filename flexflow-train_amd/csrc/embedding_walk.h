@@ -14,8 +14,9 @@
 // 16 cycles of a 16-byte access all the same: branches around it are cheaper (50 us against 44).
 // Workgroups go from the end of the positions to their beginning: where ids are ranked by how often they come
 // up, the positions at the end are rows looked up once each, which take longest, and there are twice the
-// walkers that the chip holds at a time, so that the others fill in behind them (65 536 x 1024 bf16: 109 us
-// with its sort in the order of the positions, 99 so).
+// walkers that the chip holds at a time, so that the others fill in behind them (65 536 x 1024 bf16
+// with its sort, caches full of what another kernel wrote / read / of these tensors: 93 / 85 / 79 us in the order of the
+// positions, 87 / 78 / 72 so; 55 139 x 328 bf16 50 / 46 / 43 and 53 / 49 / 44).
 //
 // Walkers add runs that lie inside their chunk straight to memory; the partial sums of runs that cross a
 // walker border meet in LDS and are merged by the workgroup, so only runs that cross a WORKGROUP border

@@ -1125,7 +1125,7 @@ static hipError_t launch_bf16(hipStream_t st, bf16 const *A, bf16 const *B,
   return hipGetLastError();
 }
 
-// FFK_OPTION_GEMM_VARIANT = 128|256|1 forces a tile configuration (1 = the
+// FFK_OPTION_GEMM_VARIANT forces a tile (EdgeTile's values, 192, or 1 = the
 // register-staged kernel); 0 = the heuristic.  For tuning runs and tests.
 inline int gemm_variant_override() { return option(FFK_OPTION_GEMM_VARIANT); }
 

@@ -112,8 +112,9 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(
 // of LDS work, the matrix pipe 80% busy).  An operand
 // whose rows are contiguous (A[K,M], B[K,N]) lies as [k][row] with the two
 // 32-float halves of every odd k swapped, which does the same for the read
-// without padding.  Every element's products are added in ascending k, two per
-// MFMA, as in gemm_f32_kernel: the two kernels give the same bits.
+// without padding.  A group of waves (KG below) adds every element's products in
+// ascending k, two per MFMA, as gemm_f32_kernel does: with one group the two
+// kernels give the same bits.
 // Rows and columns past the edge are read from the last valid ones and never
 // stored; k past the end is zeroed when the tile is written to LDS.
 // KG: groups of four waves that split the k-tiles, each with LDS buffers of its own, and add up at the end.

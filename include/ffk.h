@@ -135,11 +135,13 @@ int ffk_probe_mfma_bf16(ffk_stream_t stream, int iterations, uint32_t seed,
  * reference.  All start at 0 and change through ffk_set_option only: the
  * library never reads the environment.
  *   FFK_OPTION_GEMM_VARIANT: 0 = the dispatch heuristic;
- *     128 / 256 force that pipelined bf16 tile (eight waves), 264 the 256 tile
- *     with one wave per SIMD, 1 the register-staged kernel.
+ *     any other value forces a bf16 tile where the operands allow it: 32, 64,
+ *     128 and 256 the square ones, 65 the 64 x 64 one with four LDS stages, 70
+ *     128 x 64, 130 256 x 128, 192 256 x 192 (A and B^T row by row only), 264
+ *     the 256 x 256 one with one wave per SIMD; 1 the register-staged kernel.
  *   FFK_OPTION_LAYER_UNFUSED: != 0 makes the encoder-layer
  *     entry points (and a step-driver instance created while it is set) run
- *     one kernel per operator.
+ *     one kernel per operator.  No other call changes with it.
  *   FFK_OPTION_ATTENTION_VARIANT: which of the two tuned bf16 forward
  *     kernels runs: 0 = 64 query rows per wavefront from 1024 keys on, 32
  *     below; 1 = 32 rows at every size; 2 = 64 rows at every size.          */
@@ -176,11 +178,14 @@ int ffk_get_option(int which, int *value);
  *   bytes; may be NULL when that size is 0.  It holds, one behind the other,
  *   g when there is an activation or when out_dim is no multiple of 8 in bf16
  *   (then with rows padded to whole 16 bytes); the partial column sums of the
- *   bias gradient; and at its end the partial sums of an input_grad whose
- *   reduction over out_dim is split over workgroups.  An activation's g and the
- *   column sums are needed (FFK_ERR_WORKSPACE); without the size of the query,
- *   or 16-byte alignment, the padding and the splits are left out, which costs
- *   time and gives the sums another order, so other last bits.                */
+ *   bias gradient; and at its end the partial sums of reductions that are split
+ *   over workgroups: input_grad's over out_dim and, in bf16, weight_grad's and
+ *   bias_grad's over batch.  Room for an activation's g and for the column sums
+ *   is needed (FFK_ERR_WORKSPACE), also by sizes whose kernels keep neither;
+ *   without the size of the query, or 16-byte alignment, the padding and the
+ *   splits are left out, which costs time and gives the sums another order, so
+ *   other last bits.  In bf16 a layer that is small, or whose rows are no whole
+ *   16 bytes, takes its gradients from one launch, with an order of its own.  */
 /* ------------------------------------------------------------------------ */
 int ffk_linear_forward(ffk_stream_t stream, int dtype, int activation,
                        void const *input, void *output, void const *weight,
