@@ -18,23 +18,42 @@ struct ColreduceJob {
   int accumulate;
 };
 
-template <typename T>
+// The row groups of a workgroup of fewer than 1024 threads (a launch that also does something else,
+// gemm_bf16.h) share its threads; what is added up, and in which order, stays the same.
+template <typename T, int NT = 1024>
 __device__ __forceinline__ void colreduce_block(ColreduceJob const &job, int block, float (&red)[32][33]) {
+  constexpr int G = 1024 / NT;  // row groups of a thread
   int const cx = threadIdx.x & 31, ry = threadIdx.x >> 5;
   int const j = block * 32 + cx;
-  float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+  float s[G][4];
+#pragma unroll
+  for (int g = 0; g < G; g++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) s[g][q] = 0.0f;
   if (j < job.ncols) {
     float const *p = job.partials + j;
-    int r = ry;
-    for (; r + 96 < job.nparts; r += 128) {
-      s0 += p[(int64_t)r * job.ncols];
-      s1 += p[(int64_t)(r + 32) * job.ncols];
-      s2 += p[(int64_t)(r + 64) * job.ncols];
-      s3 += p[(int64_t)(r + 96) * job.ncols];
+    for (int r = 0; r < job.nparts; r += 128) {
+      float v[G][4];
+#pragma unroll
+      for (int g = 0; g < G; g++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          int const row = r + ry + g * (NT / 32) + q * 32;
+          v[g][q] = row < job.nparts ? p[(int64_t)row * job.ncols] : 0.0f;
+        }
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        bool const whole = r + ry + g * (NT / 32) + 96 < job.nparts;  // the last rows are one sum
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          s[g][0] += q == 0 || !whole ? v[g][q] : 0.0f;
+          if (q > 0) s[g][q] += whole ? v[g][q] : 0.0f;
+        }
+      }
     }
-    for (; r < job.nparts; r += 32) s0 += p[(int64_t)r * job.ncols];
   }
-  red[ry][cx] = (s0 + s1) + (s2 + s3);
+#pragma unroll
+  for (int g = 0; g < G; g++) red[ry + g * (NT / 32)][cx] = (s[g][0] + s[g][1]) + (s[g][2] + s[g][3]);
   __syncthreads();
   if (ry == 0 && j < job.ncols) {
     float t = 0.0f;
@@ -70,18 +89,28 @@ struct ColreduceBatch {
 // non-null while a caller on this thread is collecting
 inline thread_local ColreduceBatch *tl_colreduce_batch = nullptr;
 
+template <typename T, int NT>
+__device__ __forceinline__ void colreduce_batch_block(ColreduceBatch const &b, int block, float (&red)[32][33]) {
+  int k = 0;
+  while (k + 1 < b.count && block >= b.first_block[k + 1]) k++;
+  colreduce_block<T, NT>(b.job[k], block - b.first_block[k], red);
+}
+
 template <typename T>
 __global__ __launch_bounds__(1024) void colreduce_batch_kernel(ColreduceBatch b) {
   __shared__ float red[32][33];
-  int k = 0;
-  while (k + 1 < b.count && (int)blockIdx.x >= b.first_block[k + 1]) k++;
-  colreduce_block<T>(b.job[k], (int)blockIdx.x - b.first_block[k], red);
+  colreduce_batch_block<T, 1024>(b, (int)blockIdx.x, red);
+}
+
+// Workgroups of what was collected.
+inline int colreduce_blocks(ColreduceBatch const &b) {
+  return b.count == 0 ? 0 : b.first_block[b.count - 1] + (int)ceil_div(b.job[b.count - 1].ncols, 32);
 }
 
 // Runs what was collected (nothing to do for an empty batch) and empties it.
 inline hipError_t colreduce_flush(hipStream_t st, ColreduceBatch &b) {
   if (b.count == 0) return hipSuccess;
-  int const blocks = b.first_block[b.count - 1] + (int)ceil_div(b.job[b.count - 1].ncols, 32);
+  int const blocks = colreduce_blocks(b);
   b.first_block[b.count] = blocks;
   if (b.dtype == FFK_FLOAT) {
     colreduce_batch_kernel<float><<<(unsigned)blocks, 1024, 0, st>>>(b);

@@ -392,7 +392,7 @@ extern "C" int ffk_encoder_layer_backward(ffk_stream_t st, int dtype,
                                       L.ln_ws - L.mha_reserve, mha_mode));
     if (!added) FFK_TRY(ffk_element_binary_forward(st, dtype, FFK_OP_EW_ADD, dx, g_attn_res, dx, T * E, T * E, T * E));
   }
-  FFK_TRY(weight_grad_flush(as_stream(st), weight_grads.group));
+  FFK_TRY(weight_grad_flush(as_stream(st), weight_grads.group, &reductions));  // in one launch where it can be
   FFK_HIP(colreduce_flush(as_stream(st), reductions));
   return FFK_OK;
 }

@@ -117,8 +117,10 @@ struct LayerOperators {
 };
 int weight_grad_dispatch(hipStream_t stream, int dtype, int64_t M, int64_t N, int64_t K, void const *A, int64_t lda,
                          void const *B, int64_t ldb, void *C, int64_t ldc, GemmEpilogue const &ep);
-// Runs what was collected (nothing to do for an empty group) and empties it.
-int weight_grad_flush(hipStream_t stream, WeightGradGroup &group);
+// Runs what was collected (nothing to do for an empty group) and empties it.  sums: column reductions, complete
+// but for this pass, that may run in the same launch; it empties what it has taken.
+struct ColreduceBatch;
+int weight_grad_flush(hipStream_t stream, WeightGradGroup &group, ColreduceBatch *sums = nullptr);
 
 // out[N] (+)= sum over the M rows of X[M,N] (ldx row stride); `partials` is
 // fp32 scratch of colsum_partials_elems(M, N) floats.

@@ -36,7 +36,7 @@ extern template hipError_t pick_bf16_tail<false, false>(hipStream_t, bf16 const 
                                                         int64_t, int64_t, GemmEpilogue const &);
 extern template hipError_t pick_bf16_tail<false, true>(hipStream_t, bf16 const *, bf16 const *, bf16 *, int, int, int, int64_t,
                                                        int64_t, int64_t, GemmEpilogue const &);
-extern template hipError_t pick_bf16_group<true, false>(hipStream_t, GemmProblem const *, int, int, bool);
+extern template hipError_t pick_bf16_group<true, false>(hipStream_t, GemmProblem const *, int, int, bool, ColreduceBatch *);
 
 // ---------------------------------------------------------------------------
 // Plain kernel for bf16 shapes the tiled kernel cannot take.
@@ -321,7 +321,7 @@ int weight_grad_dispatch(hipStream_t st, int dtype, int64_t M, int64_t N, int64_
   return gemm_dispatch(st, dtype, true, false, M, N, K, A, lda, B, ldb, C, ldc, ep);
 }
 
-int weight_grad_flush(hipStream_t st, WeightGradGroup &g) {
+int weight_grad_flush(hipStream_t st, WeightGradGroup &g, ColreduceBatch *sums) {
   int const n = g.count;
   g.count = 0;
   if (n == 0) return FFK_OK;
@@ -331,7 +331,7 @@ int weight_grad_flush(hipStream_t st, WeightGradGroup &g) {
     ep.accumulate = g.accumulate;
     return gemm_dispatch(st, FFK_BF16, true, false, p.M, p.N, g.K, p.A, p.lda, p.B, p.ldb, p.C, p.ldc, ep);
   }
-  hipError_t const e = pick_bf16_group<true, false>(st, g.p, n, (int)g.K, g.accumulate);
+  hipError_t const e = pick_bf16_group<true, false>(st, g.p, n, (int)g.K, g.accumulate, sums);
   FFK_HIP(e);
   return FFK_OK;
 }

@@ -4,6 +4,7 @@
 #pragma once
 #include "lds_dma.h"
 #include "gemm.h"
+#include "colreduce.h"
 #include "gemm_any.h"
 #include <algorithm>
 #include <stdarg.h>
@@ -158,7 +159,14 @@ struct GemmGroupArgs {
     int first_tile;  // number of tiles (= workgroups) of the problems before it
   } p[kMaxGemmGroup - 1];
   int count;  // of p
+  // Column reductions that ride along: workgroups from first_sum on.  They read what earlier launches left, and
+  // run where the tiles leave CUs idle; a launch of their own is 3 to 7 us of latency (encoder layers forward and
+  // backward, batch x tokens x width: 8 x 512 x 1024 511 -> 504 us, 7 x 197 x 768 247.5 -> 242, 2 x 48 x 128 69 -> 67
+  // replayed from a graph, 88 -> 80 launched one by one).
+  int first_sum;
+  ColreduceBatch sums;
 };
+struct GemmNoGroup {};
 
 // TAIL (GemmEpilogue::Tail): element-wise operators applied to the 8-element
 // pieces of the output tile on their way from LDS to memory.
@@ -188,10 +196,16 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
     bf16 const *__restrict__ A, bf16 const *__restrict__ B, bf16 *C, int M,
     int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
     bf16 const *__restrict__ bias, int act, int accumulate,
-    float *__restrict__ partial, int k_tiles_per_split, GemmTailArgs tail, GemmGroupArgs group) {
+    float *__restrict__ partial, int k_tiles_per_split, GemmTailArgs tail, std::conditional_t<GROUP, GemmGroupArgs, GemmNoGroup> group) {
+  extern __shared__ __attribute__((aligned(16))) bf16 smem[];
   int bid = blockIdx.x;
   if constexpr (GROUP) {
     int const id = bid;
+    if (id >= group.first_sum) {
+      colreduce_batch_block<bf16, (BM / WM) * (BN / WN) * 64 * KG>(group.sums, id - group.first_sum,
+                                                                   *reinterpret_cast<float (*)[32][33]>(smem));
+      return;
+    }
 #pragma unroll
     for (int q = 0; q < kMaxGemmGroup - 1; q++) {
       if (q < group.count && id >= group.p[q].first_tile) {  // uniform over the workgroup
@@ -221,8 +235,6 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   constexpr int CS = WN + 8;               // row stride of a wave's staged output tile
   static_assert(A_ELEMS / 8 % NT == 0 && B_ELEMS / 8 % NT == 0, "tile/threads");
   static_assert(STAGES * LPT <= 63, "vmcnt range");
-
-  extern __shared__ __attribute__((aligned(16))) bf16 smem[];
 
   static_assert(KG == 1 || EDGE == kEdgeBounded, "written for this");
   int const kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
@@ -1072,7 +1084,7 @@ static hipError_t launch_pipe(hipStream_t st, bf16 const *A, bf16 const *B,
     int const k_tiles = (K + BK - 1) / BK, per_split = (k_tiles + splits - 1) / splits;
     splits = (k_tiles + per_split - 1) / per_split;  // none is empty
     kern<<<blocks * splits, NT, kLds, st>>>(A, B, C, M, N, K, lda, ldb, ldc, nullptr, FFK_ACT_NONE, 0, partial, per_split,
-                                            tail, GemmGroupArgs{});
+                                            tail, GemmNoGroup{});
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     int64_t const quads = (int64_t)M * N / 4;
@@ -1083,13 +1095,13 @@ static hipError_t launch_pipe(hipStream_t st, bf16 const *A, bf16 const *B,
   }
   kern<<<blocks, NT, kLds, st>>>(A, B, C, M, N, K, lda, ldb, ldc,
                                      static_cast<bf16 const *>(ep.bias), ep.activation,
-                                     ep.accumulate, nullptr, 0, tail, GemmGroupArgs{});
+                                     ep.accumulate, nullptr, 0, tail, GemmNoGroup{});
   return hipGetLastError();
 }
 
 // Several GEMMs of the same kind and reduction length in one launch.
 template <int BM, int BN, int WM, int WN, int BK, int STAGES, int PF, bool TA, bool TB, int EDGE, int KG>
-static hipError_t launch_pipe_group(hipStream_t st, GemmProblem const *p, int n, int K, bool accumulate) {
+static hipError_t launch_pipe_group(hipStream_t st, GemmProblem const *p, int n, int K, bool accumulate, ColreduceBatch *sums) {
   using Cfg = PipeCfg<BM, BN, WM, WN, BK, STAGES>;
   constexpr int NT = Cfg::NW * 64 * KG;
   constexpr size_t kLds = Cfg::template groups<KG>();
@@ -1106,6 +1118,12 @@ static hipError_t launch_pipe_group(hipStream_t st, GemmProblem const *p, int n,
     tiles += ceil_div(p[i].M, BM) * ceil_div(p[i].N, BN);
   }
   g.count = n - 1;
+  g.first_sum = (int)tiles;
+  if (sums != nullptr && sums->count > 0 && sums->dtype == FFK_BF16) {
+    g.sums = *sums;
+    tiles += colreduce_blocks(*sums);
+    sums->count = 0;
+  }
   kern<<<(unsigned)tiles, NT, kLds, st>>>(static_cast<bf16 const *>(p[0].A), static_cast<bf16 const *>(p[0].B),
                                          static_cast<bf16 *>(p[0].C), (int)p[0].M, (int)p[0].N, K, p[0].lda, p[0].ldb,
                                          p[0].ldc, nullptr, FFK_ACT_NONE, accumulate ? 1 : 0, nullptr, 0, GemmTailArgs{}, g);
@@ -1342,7 +1360,7 @@ hipError_t pick_bf16_tail(hipStream_t st, bf16 const *A, bf16 const *B, bf16 *C,
 // rank the three and do not predict: 432 tiles of 128 x 128 over 1379 rows (the gradients of a 768-wide
 // layer) 37 us, 22 by the formula.
 template <bool TA, bool TB>
-hipError_t pick_bf16_group(hipStream_t st, GemmProblem const *p, int n, int K, bool accumulate) {
+hipError_t pick_bf16_group(hipStream_t st, GemmProblem const *p, int n, int K, bool accumulate, ColreduceBatch *sums) {
   bool exact = K % 64 == 0, fits = true, exact256 = true;
   double t32 = 0, t64 = 0, t128 = 0;
   for (int i = 0; i < n; i++) {
@@ -1359,22 +1377,22 @@ hipError_t pick_bf16_group(hipStream_t st, GemmProblem const *p, int n, int K, b
                     : kt > 32 ? kt * 0.285 * t64 / kNumCU + 1.0 : ceil(t64 / (2 * kNumCU)) * (kt * 0.39 + 1.0);
   double const us128 = ceil(t128 / kNumCU) * (kt * 0.46 + 1.0);
   double const us32 = t32 <= kNumCU ? kt * (kt > 32 ? 0.18 : 0.11) + 1.0 : t32 <= 2 * kNumCU ? kt * (kt > 32 ? 0.36 : 0.22) + 1.0 : 1e9;
-  if (us32 < us64 && (us32 < us128 || !fits)) return launch_pipe_group<32, 32, 32, 32, 32, 4, 1, TA, TB, kEdgeBounded, 4>(st, p, n, K, accumulate);
+  if (us32 < us64 && (us32 < us128 || !fits)) return launch_pipe_group<32, 32, 32, 32, 32, 4, 1, TA, TB, kEdgeBounded, 4>(st, p, n, K, accumulate, sums);
   if (!fits || us64 < us128) {
     // (long reductions on four LDS stages a group of waves, one workgroup a CU: 512 x 2048 over 8065, 256 tiles, 49
     // us on two)
-    if (deep) return launch_pipe_group<64, 64, 32, 32, 64, 4, 3, TA, TB, kEdgeBounded, 2>(st, p, n, K, accumulate);
-    return launch_pipe_group<64, 64, 32, 32, 64, 2, 3, TA, TB, kEdgeBounded, 2>(st, p, n, K, accumulate);
+    if (deep) return launch_pipe_group<64, 64, 32, 32, 64, 4, 3, TA, TB, kEdgeBounded, 2>(st, p, n, K, accumulate, sums);
+    return launch_pipe_group<64, 64, 32, 32, 64, 2, 3, TA, TB, kEdgeBounded, 2>(st, p, n, K, accumulate, sums);
   }
   // Long reductions of whole 256 x 256 tiles: a round of them, three quarters full, takes less than three
   // of 128 x 128 (four gradients of 12.6 M elements together over 4096
   // rows: 106-114 us against 119; 81 by the model).
   if (exact && exact256 && K >= 1024 &&
       gemm_tile_us(kTile256Wide, 64 * t128, 256, K) < gemm_tile_us(kTile128, 128 * t128, 128, K)) {
-    return launch_pipe_group<256, 256, 128, 128, 64, 2, 1, TA, TB, kEdgeNone, 1>(st, p, n, K, accumulate);
+    return launch_pipe_group<256, 256, 128, 128, 64, 2, 1, TA, TB, kEdgeNone, 1>(st, p, n, K, accumulate, sums);
   }
-  if (exact) return launch_pipe_group<128, 128, 64, 32, 64, 4, 1, TA, TB, kEdgeNone, 1>(st, p, n, K, accumulate);
-  return launch_pipe_group<128, 128, 64, 32, 64, 4, 1, TA, TB, kEdgeOverlap, 1>(st, p, n, K, accumulate);
+  if (exact) return launch_pipe_group<128, 128, 64, 32, 64, 4, 1, TA, TB, kEdgeNone, 1>(st, p, n, K, accumulate, sums);
+  return launch_pipe_group<128, 128, 64, 32, 64, 4, 1, TA, TB, kEdgeOverlap, 1>(st, p, n, K, accumulate, sums);
 }
 
 template <bool TA, bool TB>
