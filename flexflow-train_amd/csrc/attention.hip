@@ -27,6 +27,7 @@
 // is then loaded with the same permutation of the reduction index, which the
 // transposing load does for free.
 #include "attention_common.h"
+#include "fused_ops.h"
 #include <type_traits>
 
 namespace ffk {
@@ -402,7 +403,7 @@ int attention_f32_forward(hipStream_t st, ffk_attention_desc_t const *d, void co
                           void const *v, void *o, float *lse);
 int attention_f32_backward(hipStream_t st, ffk_attention_desc_t const *d, void const *q, void const *k,
                            void const *v, void const *o, void const *d_o, float const *lse, float *delta,
-                           void *dq, void *dk, void *dv);
+                           void *dq, void *dk, void *dv, void *scratch, size_t scratch_bytes);
 
 // any multiple of 8 up to 256 for either head size (attention_gen.hip); what: bit 0 dQ and delta, bit 1 dK and dV
 int attention_bf16_general_forward(hipStream_t st, ffk_attention_desc_t const *d, void const *q, void const *k,
@@ -505,6 +506,12 @@ extern "C" int ffk_attention_backward(ffk_stream_t stream, int dtype,
                                       void const *d_o, float const *lse,
                                       float *delta, void *dq, void *dk,
                                       void *dv) {
+  return attention_backward(as_stream(stream), dtype, d, q, k, v, o, d_o, lse, delta, dq, dk, dv, nullptr, 0);
+}
+
+int ffk::attention_backward(hipStream_t st, int dtype, ffk_attention_desc_t const *d, void const *q, void const *k,
+                            void const *v, void const *o, void const *d_o, float const *lse, float *delta, void *dq,
+                            void *dk, void *dv, void *scratch, size_t scratch_bytes) {
   FFK_REQUIRE(d != nullptr, "attention_backward: NULL descriptor");
   FFK_REQUIRE(q && k && v && o && d_o && lse && delta && dq && dk && dv,
               "attention_backward: NULL tensor");
@@ -512,7 +519,7 @@ extern "C" int ffk_attention_backward(ffk_stream_t stream, int dtype,
                   aligned16(dq) && aligned16(dk) && aligned16(dv),
               "attention_backward: tensors must be 16-byte aligned");
   if (dtype == FFK_FLOAT) {
-    return attention_f32_backward(as_stream(stream), d, q, k, v, o, d_o, lse, delta, dq, dk, dv);
+    return attention_f32_backward(st, d, q, k, v, o, d_o, lse, delta, dq, dk, dv, scratch, scratch_bytes);
   }
   int rc = check_desc("attention_backward", dtype, d);
   if (rc != FFK_OK) return rc;
@@ -521,7 +528,7 @@ extern "C" int ffk_attention_backward(ffk_stream_t stream, int dtype,
   bool const offsets_fit = d->seq_q * d->q_seq_stride * 2 < lim && d->seq_q * d->o_seq_stride * 2 < lim &&
                            d->seq_kv * d->k_seq_stride * 2 < lim && d->seq_kv * d->v_seq_stride * 2 < lim;
   if (!tuned_head_size(d) || !offsets_fit) {
-    return attention_bf16_general_backward(as_stream(stream), d, q, k, v, o, d_o, lse, delta, dq, dk, dv, 3);
+    return attention_bf16_general_backward(st, d, q, k, v, o, d_o, lse, delta, dq, dk, dv, 3);
   }
   AttnBwdParams p;
   p.q = static_cast<bf16 const *>(q);
@@ -542,7 +549,6 @@ extern "C" int ffk_attention_backward(ffk_stream_t stream, int dtype,
   p.scale = d->scale;
   p.scale_log2 = d->scale * kLog2e;
   p.causal = d->causal;
-  hipStream_t st = as_stream(stream);
   // dQ first: it computes delta for its rows and leaves it in `delta` for the dK/dV kernel
   bool const few_q = few_workgroups(d, d->seq_q, d->seq_kv, 256), few_k = few_workgroups(d, d->seq_kv, d->seq_q, 128);
   int const general = (few_q ? 1 : 0) | (few_k ? 2 : 0);

@@ -25,6 +25,8 @@
 // share their rows (the pair kernels), and tiles go straight to LDS.
 #include "ffk_common.h"
 #include "lds_dma.h"
+#include "fused_ops.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace ffk {
@@ -42,6 +44,11 @@ struct AttnF32Params {
   int64_t q_bs, q_ss, k_bs, k_ss, v_bs, v_ss, o_bs, o_ss;
   float scale, scale_log2;
   int causal;
+  // The pairs of batch entry and head that a launch of the backward takes, and where dK and dV's kernel leaves dS
+  // for dQ's (nullptr: it does not): [pairs][Sq][ds_ld], rows of whole tiles of 32 keys.
+  int pair0, pairs;
+  float *ds;
+  int64_t ds_ld;
 };
 
 template <int DP>
@@ -416,11 +423,22 @@ __global__ __launch_bounds__(256) void attn_f32_delta_kernel(AttnF32Params p) {
   if (ok && lane % LPR == 0) p.delta[((int64_t)b * p.H + head) * p.Sq + q] = s;
 }
 
+// A 32 x 32 tile of dS to p.ds: rows = queries from qt0 on, column = this lane's key (32 lanes write 128 bytes of a row).
+__device__ __forceinline__ void save_scores(AttnF32Params const &p, int pair, int qt0, int key, int h32, float const (&e)[16]) {
+  float *const to = p.ds + (int64_t)pair * p.Sq * p.ds_ld + (int64_t)qt0 * p.ds_ld;
+  int const left = p.Sq - qt0;  // rows that exist
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    int const ql = 8 * (r >> 2) + 4 * h32 + (r & 3);
+    if (ql < left) to[ql * p.ds_ld + key] = e[r];
+  }
+}
+
 // --------------------------------------------------------------------------
 // backward (A): dK, dV.  Workgroup owns 128 key rows, streams query tiles.
 // Where the pair kernels are not taken (launch_f32_backward).
 // --------------------------------------------------------------------------
-template <int DP>
+template <int DP, bool SAVE>
 __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_kernel(AttnF32Params p) {
   using C = AttnF32Cfg<DP>;
   __shared__ __attribute__((aligned(16))) float Qs[2][C::kTile * C::kStrideB];
@@ -428,9 +446,9 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_kernel(AttnF32Params p)
   __shared__ __attribute__((aligned(16))) float Ls[2][C::kTile], Ds[2][C::kTile];
   int const t = threadIdx.x, lane = t & 63, h32 = lane >> 5, l32 = lane & 31;
   int const wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  int const hb = blockIdx.x % (p.H * p.B);
+  int const pair = blockIdx.x % p.pairs, hb = p.pair0 + pair;
   int const head = hb % p.H, b = hb / p.H;
-  int const kv0 = (blockIdx.x / (p.H * p.B)) * C::kBlk;
+  int const kv0 = (blockIdx.x / p.pairs) * C::kBlk;
   int const kvrow = kv0 + wave * 32 + l32;
   float const *qp = p.q + (int64_t)b * p.q_bs + (int64_t)head * p.Dq;
   float const *gp = p.d_o + (int64_t)b * p.o_bs + (int64_t)head * p.Dv;
@@ -504,6 +522,7 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_kernel(AttnF32Params p)
         // dS = P (dP - delta) scale; Ds holds delta * scale
         dsv[r] = masked ? 0.0f : e * __builtin_fmaf(dp[r], p.scale, -Ds[cur][ql]);
       }
+      if (SAVE && kv0 + wave * 32 < p.Skv) save_scores(p, pair, qt0, kvrow, h32, dsv);
       // dV += P^T dO, dK += dS^T Q: A = the accumulator (row = key), B = dO / Q rows of the
       // matching query, reduction over the tile's queries
       contract_rows<DP / 32, C::kStrideB, false>(Gs[cur] + (4 * h32) * C::kStrideB + l32, pv, dv);
@@ -705,7 +724,7 @@ struct PairStream {
 
 // dK and dV: role 0 computes S and P, hands P over and produces dV; role 1 computes dP and from
 // it and P dS, and produces dK.
-template <int DP, bool DMA, int KW>
+template <int DP, bool DMA, int KW, bool SAVE>
 __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Params p) {
   using C = AttnF32Cfg<DP>;
   constexpr int T = 32 * KW;
@@ -716,9 +735,9 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Para
   int const t = threadIdx.x, lane = t & 63, h32 = lane >> 5, l32 = lane & 31;
   int const wave = __builtin_amdgcn_readfirstlane(t >> 6);
   int const blk = wave & 1, role = wave >> 1;
-  int const hb = blockIdx.x % (p.H * p.B);
+  int const pair = blockIdx.x % p.pairs, hb = p.pair0 + pair;
   int const head = hb % p.H, b = hb / p.H;
-  int const kvg = (blockIdx.x / (p.H * p.B)) * (64 / KW);  // the workgroup's first key
+  int const kvg = (blockIdx.x / p.pairs) * (64 / KW);  // the workgroup's first key
   int const kv0 = KW == 1 ? kvg + blk * 32 : kvg;           // this wave's
   int const part = KW == 1 ? 0 : blk * 32;                  // its first query of a step
   int const kvrow = kv0 + l32;
@@ -808,6 +827,7 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dkdv_pair_kernel(AttnF32Para
           float const ds = ex[r] * __builtin_fmaf(s[r], p.scale, -Ds[cur][part + ql]);
           ex[r] = masked ? 0.0f : ds;
         }
+        if (SAVE && kv0 < p.Skv) save_scores(p, pair, qt0, kvrow, h32, ex);
       }
       // dV += P^T dO or dK += dS^T Q: A = the accumulator (row = key), B = rows of the
       // matching query, reduction over the tile's queries
@@ -951,6 +971,92 @@ __global__ __launch_bounds__(256) void attn_f32_bwd_dq_pair_kernel(AttnF32Params
   }
 }
 
+// dQ from the dS that dK and dV's kernel has left: one product instead of the three that it takes to compute
+// dS again.  A workgroup's four waves own groups of 32 query rows, CW of them share a group and take DP / CW
+// columns each; the waves read dS from memory in the layout of an operand, a tile ahead, and K's tiles from LDS.
+// Bound by the fp32 matrix pipe: batch 8 x 8 heads x 512 at head size 256 274 -> 87 us, 98 TFLOP/s, while the stores of
+// dS (67 MB) lengthen dK and dV's kernel from 351 to 364; 4 x 8 heads x 508 at 64, whole block, 319 -> 296; no size
+// measured, down to 37 rows, got slower.  The products are added up in the order of a kernel whose waves
+// do not share out the keys, to the same bits.
+template <int DP, bool DMA, int CW>
+__global__ __launch_bounds__(256) void attn_f32_bwd_dq_from_scores_kernel(AttnF32Params p) {
+  using C = AttnF32Cfg<DP>;
+  constexpr int ROWS = 128 / CW, T = C::kTile, N = DP / 32 / CW;
+  __shared__ __attribute__((aligned(16))) float Ks[2][T * C::kStrideB];
+  int const t = threadIdx.x, lane = t & 63, h32 = lane >> 5, l32 = lane & 31;
+  int const wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  int const blk = wave % (4 / CW), part = wave / (4 / CW);
+  int const nqb = (p.Sq + ROWS - 1) / ROWS;
+  int const pair = blockIdx.x % p.pairs, hb = p.pair0 + pair;
+  int const qb = nqb - 1 - blockIdx.x / p.pairs;  // heaviest causal blocks first
+  int const head = hb % p.H, b = hb / p.H;
+  int const q0 = qb * ROWS + blk * 32, qrow = q0 + l32;
+  float const *kp = p.k + (int64_t)b * p.k_bs + (int64_t)head * p.Dq;
+  float const *const scores = p.ds + ((int64_t)pair * p.Sq + min(qrow, p.Sq - 1)) * p.ds_ld + 4 * h32;
+  f32x16 dq[N];
+#pragma unroll
+  for (int i = 0; i < N; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) dq[i][r] = 0.0f;
+
+  int kv_end = p.Skv;
+  if (p.causal) kv_end = min(p.Skv, qb * ROWS + ROWS);
+  int const ntiles = (kv_end + T - 1) / T;
+  // the tiles that this wave's rows see, and that dK and dV's kernel has written: keys up to the rows' own
+  int const mine = p.causal ? min(ntiles, q0 / T + 1) : ntiles;
+  f32x4 rk[C::kChunks], next[4];
+  i32x4 rsrc;
+  unsigned lane_off = 0;
+  if constexpr (DMA) {
+    rsrc = buffer_resource(kp, kRowsBound);
+    lane_off = row_lane_offset(lane, p.Dq);
+  }
+  auto fetch = [&](int it, int buf) __attribute__((always_inline)) {
+    if constexpr (DMA) tile_dma<C::kStrideB>(rsrc, lane_off, p.k_ss, it * T, p.Skv - 1, wave, Ks[buf]);
+    else tile_gload<DP>(kp, p.k_ss, it * T, p.Skv - 1, p.Dq, t, rk);
+    if (it < mine) {
+#pragma unroll
+      for (int g = 0; g < 4; g++) next[g] = *reinterpret_cast<f32x4 const *>(scores + it * T + 8 * g);
+    }
+  };
+  float ds[16];
+  auto land = [&](int buf) __attribute__((always_inline)) {
+    if constexpr (DMA) wait_vmcnt<0>();
+    else tile_lstore<DP, C::kStrideB>(Ks[buf], t, rk);
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) ds[4 * g + e] = next[g][e];
+  };
+#pragma unroll
+  for (int g = 0; g < 4; g++) next[g] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  fetch(0, 0);
+  land(0);
+  if constexpr (DMA) wait_all_vmem_known_to_compiler();
+  __syncthreads();
+  int cur = 0;
+  for (int it = 0; it < ntiles; it++) {
+    bool const more = it + 1 < ntiles;
+    if (more) fetch(it + 1, cur ^ 1);
+    // dQ^T += K^T dS^T: A = K^T (row d), B = dS^T, reduction over the tile's keys
+    if (it < mine) contract_rows<N, C::kStrideB, true>(Ks[cur] + 4 * h32 * C::kStrideB + part * (DP / CW) + l32, ds, dq);
+    if (more) land(cur ^ 1);
+    __syncthreads();
+    cur ^= 1;
+  }
+  if (qrow < p.Sq) {
+    float *dqp = p.dq + (int64_t)b * p.q_bs + (int64_t)qrow * p.q_ss + (int64_t)head * p.Dq;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        int const d = part * (DP / CW) + i * 32 + 8 * g + 4 * h32;
+        if (d < p.Dq) *reinterpret_cast<f32x4 *>(dqp + d) = f32x4{dq[i][4 * g], dq[i][4 * g + 1], dq[i][4 * g + 2], dq[i][4 * g + 3]};
+      }
+    }
+  }
+}
+
 static int check_desc_f32(char const *who, ffk_attention_desc_t const *d) {
   int64_t const dq = d->head_dim, dv = d->v_head_dim > 0 ? d->v_head_dim : d->head_dim;
   FFK_REQUIRE(dq > 0 && dq <= 256 && dq % 4 == 0 && dv <= 256 && dv % 4 == 0,
@@ -982,6 +1088,7 @@ static AttnF32Params make_params(ffk_attention_desc_t const *d) {
   p.scale = d->scale;
   p.scale_log2 = d->scale * kLog2eF;
   p.causal = d->causal;
+  p.pairs = p.B * p.H;
   return p;
 }
 
@@ -1041,8 +1148,26 @@ int attention_f32_forward(hipStream_t st, ffk_attention_desc_t const *d, void co
   return FFK_OK;
 }
 
+// Scratch for dS, which lets dQ's kernel skip two of its three products, and how many pairs of batch entry and head
+// go into it at a time: all of them, or in several launches where those still fill the chip twice over; 0: no use of it.
+// Half a GB holds dS of every block of up to 700 rows that was measured; where it does not, a launch for a part of the
+// heads still has two workgroups a CU.
+constexpr size_t kMostScores = (size_t)512 << 20;
+static int64_t f32_scores_row(int64_t seq_kv) { return ceil_div(seq_kv, 32) * 32; }
+size_t attention_f32_scores_bytes(int64_t pairs, int64_t seq_q, int64_t seq_kv) {
+  if (pairs <= 0 || seq_q <= 0 || seq_kv <= 0 || seq_q >= (1 << 30) || seq_kv >= (1 << 30)) return 0;
+  size_t const one = (size_t)seq_q * f32_scores_row(seq_kv) * sizeof(float), most = kMostScores / one;
+  return one * std::min<size_t>((size_t)pairs, most);
+}
+static int64_t f32_pairs_at_a_time(AttnF32Params const &p, size_t bytes) {
+  int64_t const all = (int64_t)p.H * p.B;
+  int64_t const most = (int64_t)(std::min(bytes, kMostScores) / ((size_t)p.Sq * f32_scores_row(p.Skv) * sizeof(float)));
+  if (most >= all) return all;
+  return most * ceil_div(std::min(p.Sq, p.Skv), 128) >= 2 * kNumCU ? most : 0;
+}
+
 template <int DP, bool DMA>
-static void launch_f32_backward(hipStream_t st, AttnF32Params const &p, int64_t rows) {
+static void launch_f32_backward(hipStream_t st, AttnF32Params const &p, int64_t rows, void *scratch, size_t scratch_bytes) {
   attn_f32_delta_kernel<DP><<<(unsigned)ceil_div(rows, 4 * (64 / (DP / 4))), 256, 0, st>>>(p);
   int64_t const heads = (int64_t)p.H * p.B;
   // Pairs always at 256 (see above) and at 64, where they leave registers for twice the waves (batch 6 x 32
@@ -1051,28 +1176,58 @@ static void launch_f32_backward(hipStream_t st, AttnF32Params const &p, int64_t 
   auto pairs = [&](int64_t rows_owned) {
     return DP >= 64 && (DP != 128 || ceil_div(rows_owned, 128) * heads < kNumCU);
   };
+  auto launch_dkdv = [&](AttnF32Params const &q, auto save) {
+    constexpr bool SAVE = decltype(save)::value;
+    int64_t const n = q.pairs;
+    if constexpr (DP >= 64) {
+      if (pairs(p.Skv)) {
+        int const kw = f32_split(p, p.Skv, 64, p.Sq, DP <= 128 ? 2 : 1);
+        if constexpr (DP <= 128) {
+          if (kw == 2) return (void)(attn_f32_bwd_dkdv_pair_kernel<DP, DMA, 2, SAVE><<<(unsigned)(ceil_div(p.Skv, 32) * n), 256, 0, st>>>(q));
+        }
+        attn_f32_bwd_dkdv_pair_kernel<DP, DMA, 1, SAVE><<<(unsigned)(ceil_div(p.Skv, 64) * n), 256, 0, st>>>(q);
+        return;
+      }
+    }
+    if constexpr (DP == 32 || DP == 128) {
+      attn_f32_bwd_dkdv_kernel<DP, SAVE><<<(unsigned)(ceil_div(p.Skv, 128) * n), 256, 0, st>>>(q);
+    }
+  };
+  if (int64_t const at_a_time = f32_pairs_at_a_time(p, scratch_bytes); scratch != nullptr && at_a_time > 0) {
+    AttnF32Params q = p;
+    q.ds = static_cast<float *>(scratch);
+    q.ds_ld = f32_scores_row(p.Skv);
+    for (q.pair0 = 0; q.pair0 < heads; q.pair0 += q.pairs) {
+      q.pairs = (int)std::min<int64_t>(at_a_time, heads - q.pair0);
+      launch_dkdv(q, std::true_type{});
+      // few columns a wave where so many rows a workgroup leave CUs without one (3 x 4 heads x 633 of 64, causal, whole
+      // block: 183 us by the kernel that computes dS again, 186 with 128 rows a workgroup, 176 with 64)
+      constexpr int CW = DP <= 64 ? 1 : 2, MORE = DP >= 64 ? 2 * CW : CW;
+      if (MORE > CW && ceil_div(p.Sq, 128 / CW) * q.pairs < kNumCU) {
+        attn_f32_bwd_dq_from_scores_kernel<DP, DMA, MORE><<<(unsigned)(ceil_div(p.Sq, 128 / MORE) * q.pairs), 256, 0, st>>>(q);
+      } else {
+        attn_f32_bwd_dq_from_scores_kernel<DP, DMA, CW><<<(unsigned)(ceil_div(p.Sq, 128 / CW) * q.pairs), 256, 0, st>>>(q);
+      }
+    }
+    return;
+  }
+  launch_dkdv(p, std::false_type{});
   if constexpr (DP >= 64) {
-    auto both = [&](auto split) {
-      constexpr int KW = decltype(split)::value;
-      if (pairs(p.Skv) && f32_split(p, p.Skv, 64, p.Sq, DP <= 128 ? 2 : 1) == KW) {
-        attn_f32_bwd_dkdv_pair_kernel<DP, DMA, KW><<<(unsigned)(ceil_div(p.Skv, 64 / KW) * heads), 256, 0, st>>>(p);
+    if (pairs(p.Sq)) {
+      int const kw = f32_split(p, p.Sq, 64, p.Skv, DP <= 128 ? 2 : 1);
+      if constexpr (DP <= 128) {
+        if (kw == 2) return (void)(attn_f32_bwd_dq_pair_kernel<DP, DMA, 2><<<(unsigned)(ceil_div(p.Sq, 32) * heads), 256, 0, st>>>(p));
       }
-      if (pairs(p.Sq) && f32_split(p, p.Sq, 64, p.Skv, DP <= 128 ? 2 : 1) == KW) {
-        attn_f32_bwd_dq_pair_kernel<DP, DMA, KW><<<(unsigned)(ceil_div(p.Sq, 64 / KW) * heads), 256, 0, st>>>(p);
-      }
-    };
-    both(std::integral_constant<int, 1>{});
-    if constexpr (DP <= 128) both(std::integral_constant<int, 2>{});
+      attn_f32_bwd_dq_pair_kernel<DP, DMA, 1><<<(unsigned)(ceil_div(p.Sq, 64) * heads), 256, 0, st>>>(p);
+      return;
+    }
   }
-  if constexpr (DP == 32 || DP == 128) {
-    if (!pairs(p.Skv)) attn_f32_bwd_dkdv_kernel<DP><<<(unsigned)(ceil_div(p.Skv, 128) * heads), 256, 0, st>>>(p);
-    if (!pairs(p.Sq)) attn_f32_bwd_dq_kernel<DP><<<(unsigned)(ceil_div(p.Sq, 128) * heads), 256, 0, st>>>(p);
-  }
+  if constexpr (DP == 32 || DP == 128) attn_f32_bwd_dq_kernel<DP><<<(unsigned)(ceil_div(p.Sq, 128) * heads), 256, 0, st>>>(p);
 }
 
 int attention_f32_backward(hipStream_t st, ffk_attention_desc_t const *d, void const *q, void const *k,
                            void const *v, void const *o, void const *d_o, float const *lse, float *delta,
-                           void *dq, void *dk, void *dv) {
+                           void *dq, void *dk, void *dv, void *scratch, size_t scratch_bytes) {
   int rc = check_desc_f32("attention_backward", d);
   if (rc != FFK_OK) return rc;
   AttnF32Params p = make_params(d);
@@ -1088,7 +1243,7 @@ int attention_f32_backward(hipStream_t st, ffk_attention_desc_t const *d, void c
   p.dv = static_cast<float *>(dv);
   int64_t const rows = (int64_t)p.B * p.H * p.Sq;
   int const dmax = p.Dq > p.Dv ? p.Dq : p.Dv;
-#define CALL(DP_, DMA_) launch_f32_backward<DP_, DMA_>(st, p, rows)
+#define CALL(DP_, DMA_) launch_f32_backward<DP_, DMA_>(st, p, rows, scratch, scratch_bytes)
   FFK_ATTN_F32_DISPATCH(dmax, CALL);
 #undef CALL
   FFK_CHECK_LAUNCH();

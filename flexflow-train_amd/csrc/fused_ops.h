@@ -87,6 +87,13 @@ int mha_backward_add_residual(hipStream_t st, int dtype, ffk_mha_desc_t const *d
                               void const *residual, bool *added, void const *weight, void *weight_grad,
                               void const *output_grad, void *reserve, size_t reserve_bytes, int accumulate);
 
+// ffk_attention_backward, with scratch (16-byte aligned, nullptr: none) that lets it compute dS once instead of
+// twice.  attention_scores_bytes: what it can use of it; less, or none, is as good as the entry point.
+int attention_backward(hipStream_t st, int dtype, ffk_attention_desc_t const *d, void const *q, void const *k, void const *v,
+                       void const *o, void const *d_o, float const *lse, float *delta, void *dq, void *dk, void *dv,
+                       void *scratch, size_t scratch_bytes);
+size_t attention_f32_scores_bytes(int64_t pairs, int64_t seq_q, int64_t seq_kv);
+
 // summed = residual + dropout(in); y = LayerNorm(summed), statistics kept as the separate
 // LayerNorm would.  Returns FFK_ERR_UNSUPPORTED (without setting an error
 // message) when the row length or the alignment has no vector kernel.

@@ -14,7 +14,9 @@
 // attention_gen.hip.
 //
 // Reserve space layout (bytes, each region 256-byte aligned):
-//   QKV projections | context | lse | delta | d(context) | d(QKV projections)
+//   QKV projections | context | lse | delta | d(context) | d(QKV projections) | dS
+// The last one is room that the backward makes use of where the caller has it (FLOAT); a reserve space
+// without it does as well.
 #include "gemm.h"
 #include "fused_ops.h"
 
@@ -23,7 +25,7 @@ namespace ffk {
 struct MhaLayout {
   int64_t TQ, TK;                 // tokens: B*Sq, B*Skv
   int64_t nQ, nK, nV, nC;         // elements of each projected tensor / context
-  size_t off_qkv, off_ctx, off_lse, off_delta, off_dctx, off_dqkv, total;
+  size_t off_qkv, off_ctx, off_lse, off_delta, off_dctx, off_dqkv, total, with_scores;
   int64_t wq, wk, wv, wo;         // weight offsets (elements)
 };
 
@@ -45,6 +47,7 @@ static MhaLayout make_layout(ffk_mha_desc_t const *d, size_t es) {
   L.off_dctx = off;  off += align256((size_t)L.nC * es);
   L.off_dqkv = off;  off += align256((size_t)(L.nQ + L.nK + L.nV) * es);
   L.total = off;
+  L.with_scores = off + (es == sizeof(float) ? attention_f32_scores_bytes(d->num_samples * d->num_heads, d->qo_seq_length, d->kv_seq_length) : 0);
   L.wq = 0;
   L.wk = L.wq + d->num_heads * d->q_proj_size * d->q_size;
   L.wv = L.wk + d->num_heads * d->k_proj_size * d->k_size;
@@ -115,7 +118,7 @@ extern "C" size_t ffk_mha_weight_elements(ffk_mha_desc_t const *d) {
 
 extern "C" size_t ffk_mha_reserve_bytes(ffk_mha_desc_t const *d, int dtype) {
   if (d == nullptr || dtype_size(dtype) == 0) return 0;
-  return make_layout(d, dtype_size(dtype)).total;
+  return make_layout(d, dtype_size(dtype)).with_scores;
 }
 
 extern "C" int ffk_mha_forward(ffk_stream_t stream, int dtype,
@@ -241,9 +244,9 @@ static int mha_backward_impl(ffk_stream_t stream, int dtype, ffk_mha_desc_t cons
     dqp = dqkv; dkp = dqkv + L.nQ * es; dvp = dqkv + (L.nQ + L.nK) * es;
   }
   // The core writes dQ/dK/dV with the same strides it reads Q/K/V with.
-  rc = ffk_attention_backward(stream, dtype, &a, qp, kp, vp, ctx, dctx,
-                              reinterpret_cast<float const *>(rs + L.off_lse),
-                              reinterpret_cast<float *>(rs + L.off_delta), dqp, dkp, dvp);
+  size_t const more = reserve_bytes - L.total;
+  rc = attention_backward(st, dtype, &a, qp, kp, vp, ctx, dctx, reinterpret_cast<float const *>(rs + L.off_lse),
+                          reinterpret_cast<float *>(rs + L.off_delta), dqp, dkp, dvp, aligned16(rs + L.total) ? rs + L.total : nullptr, more);
   if (rc != FFK_OK) return rc;
 
   if (folded) {

@@ -637,7 +637,9 @@ int ffk_attention_backward(ffk_stream_t stream, int dtype,
  *   pre-projection context and the log-sum-exp between forward and backward
  *   plus backward scratch, like MHAPerDeviceState.reserveSpace.  Its layout
  *   follows from the descriptor alone, so backward needs the descriptor forward
- *   had and nothing else.
+ *   had and nothing else.  For FLOAT the size asked for includes up to 512 MB
+ *   behind that in which backward keeps dS, so that it is computed once; a
+ *   reserve space without this part is taken as well.
  * backward: query_grad/key_grad/value_grad are overwritten unless accumulate
  *   (cudnnMultiHeadAttnBackwardData stores them);
  *   key_grad/value_grad may be NULL when key/value alias query (their
