@@ -11,6 +11,7 @@
 #include <stdio.h>
 #include <string.h>
 #include <type_traits>
+#include <utility>
 
 namespace ffk {
 
@@ -85,6 +86,34 @@ __device__ __forceinline__ u32x2 load_any8(bf16 const *p) { return reinterpret_c
 __device__ __forceinline__ u32x2 load_first4(bf16 const *p, int n) {
   u32x4 const v = load_raw_first(p, n);
   return u32x2{v[0], v[1]};
+}
+
+// f of 0, 1, ..., as constants (a loop of this many long bodies is not unrolled)
+template <int... I, typename F>
+__device__ __forceinline__ void unroll_for(std::integer_sequence<int, I...>, F f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+// acc += a . b with the accumulator in accumulation registers.  Written as an instruction: of 256 accumulator and 128
+// fragment registers the compiler keeps some of each kind in the other kind's place, and then moves 108 of them
+// there and back in every k-tile ([16384, 4096] . [12288, 4096]^T 1473 us, 1194 so).  It does not see
+// that these results take time: mfma16_settled has to stand between the last of them and their first use.
+__device__ __forceinline__ void mfma16_in_place(f32x4 &acc, bf16x8 a, bf16x8 b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+// ... and a direct load behind it: the MFMA stands between the write of M0 and the load that reads it, where lds_dma16 has
+// a wait state.
+__device__ __forceinline__ void mfma16_in_place_and_load(f32x4 &acc, bf16x8 a, bf16x8 b, i32x4 rsrc, unsigned lane_byte_off,
+                                                         unsigned uniform_byte_off, unsigned lds_byte_addr) {
+  asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\tbuffer_load_dwordx4 %4, %5, %6 offen lds"
+               : "+a"(acc)
+               : "v"(a), "v"(b), "s"(lds_byte_addr), "v"(lane_byte_off), "s"(rsrc), "s"(uniform_byte_off)
+               : "memory");
+}
+template <int N>
+__device__ __forceinline__ void mfma16_settled(f32x4 (&acc)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; i++) asm volatile("s_nop 7" : "+a"(acc[i]));
 }
 
 enum { kEdgeNone = 0, kEdgeOverlap = 1, kEdgeBounded = 2 };
@@ -224,7 +253,18 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   constexpr int NT = NW * 64;
   // a group is one wave: nobody but the wave itself reads its stages, and no barrier stands in its loop
   constexpr bool ALONE = NW == 1 && KG > 1;
-  constexpr int TM = WM / 32, TN = WN / 32;
+  // One wave per SIMD and two stages: see the k-loop.
+  constexpr bool WIDE2 = WM == 128 && (WN == 128 || WN == 96) && STAGES == 2;
+  // M16: on v_mfma_f32_16x16x32_bf16 instead of v_mfma_f32_32x32x16_bf16: the same bits (measured over reductions of 32
+  // to 4096) for less power.  With operands in registers alone, all CUs busy and normally distributed values, the
+  // first runs at 2.04 PFLOP/s and the second at 1.80, both at the clock that power leaves them.
+  // (The wide tile, launch to launch, and with what the k-loop says of the order of its loads: [16384, 4096] . [12288,
+  // 4096]^T 1242 -> 1143 us, [16384, 12288] . [12288, 4096] 1320 -> 1214, [12288, 16384] . [16384, 4096] with A transposed
+  // 1271 -> 1215, [4096, 1024] . [4096, 1024]^T 40 -> 36-37.)
+  constexpr bool M16 = WIDE2;
+  constexpr int MB = M16 ? 16 : 32, MK = M16 ? 32 : 16;  // rows and columns, and k's, of a matrix instruction
+  using Acc = std::conditional_t<M16, f32x4, f32x16>;
+  constexpr int TM = WM / MB, TN = WN / MB;
   constexpr bool TBL = (TB == false);  // B tile lies as [BK][BN]
   constexpr int A_ELEMS = BM * BK, B_ELEMS = BN * BK;
   constexpr int A_LOADS = A_ELEMS / 8 / NT, B_LOADS = B_ELEMS / 8 / NT;
@@ -271,7 +311,12 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   // chunk pc ^ ((row / RPW) % CPRK).  Tile lying as [BK][cols]: the 64-byte
   // segment s of row k sits at segment s ^ (k % 4) (with 64 columns, whose rows are
   // half a bank window, at s ^ ((k / 2) % 2); with 32 there is one).
+  // For M16, whose transposing reads take rows k and k + 8 side by side, 32 bytes of each: the 32-byte piece p of row k
+  // sits at p ^ (2 (k % 4) + (k / 8) % 2).
   auto tr_swizzle = [](int krow, int cols) { return cols == 32 ? 0 : cols == 64 ? (krow >> 1) & 1 : krow & 3; };
+  auto tr_chunk = [&](int krow, int pc, int cols) {  // the 16-byte chunk of the row that lies at chunk pc
+    return M16 ? pc ^ ((((krow & 3) << 1) | ((krow >> 3) & 1)) << 1) : (((pc >> 2) ^ tr_swizzle(krow, cols)) << 2) | (pc & 3);
+  };
   constexpr int ROWS_PER_LOAD_KC = NT / CPRK;     // rows covered by one load of all threads
   static_assert((ROWS_PER_LOAD_KC / RPW) % CPRK == 0, "swizzle must repeat per load");
   static_assert((!TA || (NT * 8 % BM == 0 && (NT * 8 / BM) % 4 == 0)) && (!TBL || (NT * 8 % BN == 0 && (NT * 8 / BN) % 4 == 0)),
@@ -286,7 +331,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
     } else {
       constexpr int CPR = BM / 8;
       int krow = c / CPR, pc = c % CPR;
-      int lc = ((((pc >> 2) ^ tr_swizzle(krow, BM)) << 2) | (pc & 3));
+      int lc = tr_chunk(krow, pc, BM);
       voff_a = (unsigned)(krow * lda + lc * 8) * 2u;
     }
     if (!TBL) {
@@ -296,7 +341,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
     } else {
       constexpr int CPR = BN / 8;
       int krow = c / CPR, pc = c % CPR;
-      int lc = ((((pc >> 2) ^ tr_swizzle(krow, BN)) << 2) | (pc & 3));
+      int lc = tr_chunk(krow, pc, BN);
       voff_b = (unsigned)(krow * ldb + lc * 8) * 2u;
     }
   }
@@ -308,7 +353,11 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   // (kEdgeBounded) lanes whose rows or columns lie past the operand ask for what no descriptor covers and get
   // zeros: of a K-contiguous panel each load has rows of its own, of one lying [BK][cols] all have the lane's columns
   constexpr bool ROWS_A = EDGE == kEdgeBounded && !TA, ROWS_B = EDGE == kEdgeBounded && !TBL;
-  unsigned off_a[ROWS_A ? A_LOADS : 1], off_b[ROWS_B ? B_LOADS : 1];
+  // (M16) loads of 8 rows of a panel lying [BK][cols] take turns between two offsets, 32 bytes apart
+  constexpr bool TURN_A = M16 && TA && NT * 8 / BM == 8, TURN_B = M16 && TBL && NT * 8 / BN == 8;
+  static_assert(!M16 || (EDGE != kEdgeBounded && (!TA || TURN_A || NT * 8 / BM % 16 == 0) && (!TBL || TURN_B || NT * 8 / BN % 16 == 0)),
+                "written for these loads");
+  unsigned off_a[ROWS_A ? A_LOADS : TURN_A ? 2 : 1], off_b[ROWS_B ? B_LOADS : TURN_B ? 2 : 1];
   {
     int const c = wave * 64 + lane;
     auto columns_from = [&](int cols) {  // of the lane's pieces (see the swizzle above)
@@ -326,9 +375,20 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
       off_b[q] = there ? voff_b : 0x80000000u;
     }
   }
-  auto lane_a = [&](int q) __attribute__((always_inline)) { return off_a[ROWS_A ? q : 0]; };
-  auto lane_b = [&](int q) __attribute__((always_inline)) { return off_b[ROWS_B ? q : 0]; };
+  if constexpr (TURN_A) {
+    int const c = wave * 64 + lane;
+    off_a[1] = (unsigned)(c / (BM / 8) * lda + tr_chunk(c / (BM / 8) + 8, c % (BM / 8), BM) * 8) * 2u;
+  }
+  if constexpr (TURN_B) {
+    int const c = wave * 64 + lane;
+    off_b[1] = (unsigned)(c / (BN / 8) * ldb + tr_chunk(c / (BN / 8) + 8, c % (BN / 8), BN) * 8) * 2u;
+  }
+  auto lane_a = [&](int q) __attribute__((always_inline)) { return off_a[ROWS_A ? q : TURN_A ? q & 1 : 0]; };
+  auto lane_b = [&](int q) __attribute__((always_inline)) { return off_b[ROWS_B ? q : TURN_B ? q & 1 : 0]; };
 
+  // WIDE2: a ring of five panels, A's and B's of the k-tiles in turn (see the k-loop); `stage` is where a tile's A lies.
+  constexpr int RING = 5, PANEL = A_ELEMS > B_ELEMS ? A_ELEMS : B_ELEMS;
+  auto ring_at = [](int at, int d) __attribute__((always_inline)) { return at + d >= RING ? at + d - RING : at + d; };
   // LDS destinations of the direct loads are scalar byte addresses: base + stage + chunk row
   bf16 *const stages = smem + (KG == 1 ? 0 : kg * (STAGES * STAGE_ELEMS));
   unsigned const smem_addr = lds_address_of(stages);
@@ -337,8 +397,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   // (first and count are constants once the caller's loops are unrolled)
   // (maybe_last: the k-tile may be the last one of the reduction)
   auto issue_some = [&](int kt, int stage, int first, int count, bool maybe_last) __attribute__((always_inline)) {
-    unsigned const sa = smem_addr + (unsigned)(stage * STAGE_ELEMS) * 2u;
-    unsigned const sb = sa + (unsigned)A_ELEMS * 2u;
+    unsigned const sa = smem_addr + (unsigned)(WIDE2 ? stage * PANEL : stage * STAGE_ELEMS) * 2u;
+    unsigned const sb = WIDE2 ? smem_addr + (unsigned)(ring_at(stage, 1) * PANEL) * 2u : sa + (unsigned)A_ELEMS * 2u;
     unsigned const bound = EDGE == kEdgeBounded ? 0x80000000u : 0xffffffffu;
     if constexpr (EDGE != kEdgeNone) {
       if (maybe_last && kt0 + kt >= KT_all - 1 && (K % BK != 0 || kt0 + kt >= KT_all)) {  // uniform over the wave
@@ -376,6 +436,19 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
       }
     }
   };
+  // (WIDE2) f(descriptor, lane offset, uniform offset, LDS address) of load q of a k-tile that is not the last one;
+  // panel: where in the ring what it is part of goes
+  auto load_operands = [&](int kt, int panel, int q, auto f) __attribute__((always_inline)) {
+    static_assert(EDGE != kEdgeBounded || !M16, "no bound in the descriptor");
+    if (q < A_LOADS) {
+      f(buffer_resource(panel_a + (TA ? (int64_t)(kt0 + kt) * BK * lda : (int64_t)(kt0 + kt) * BK)), lane_a(q),
+        (unsigned)(q * step_a) * 2u, smem_addr + (unsigned)(panel * PANEL) * 2u + (unsigned)(q * NW + wave_s) * 1024u);
+    } else {
+      int const i = q - A_LOADS;
+      f(buffer_resource(panel_b + (TBL ? (int64_t)(kt0 + kt) * BK * ldb : (int64_t)(kt0 + kt) * BK)), lane_b(i),
+        (unsigned)(i * step_b) * 2u, smem_addr + (unsigned)(panel * PANEL) * 2u + (unsigned)(i * NW + wave_s) * 1024u);
+    }
+  };
   auto issue = [&](int kt, int stage) {
     issue_some(kt, stage, 0, LPT, true);
   };
@@ -384,15 +457,16 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   // an LDS address is tabulated once here; inside the loop an address is
   // stage base + table entry + a compile-time constant that folds into the
   // instruction's offset field, so the k-loop carries almost no address math.
-  constexpr int KS = BK / 16;  // MFMA k-steps per tile
-  // K-contiguous tile: lane l reads row (row0 + l%32), logical chunk 2 kk + l/32.
-  // row0 is a multiple of 32, so the swizzle term depends on the lane only.
+  constexpr int KS = BK / MK;  // MFMA k-steps per tile
+  // K-contiguous tile: lane l reads row (row0 + l%32), logical chunk 2 kk + l/32 (M16: l%16, 4 kk + l/16).
+  // row0 is a multiple of 32 (16), so the swizzle term depends on the lane only.
   int kc_off[KS];
   {
-    int const sw = ((lane & 31) / RPW) & (CPRK - 1);
+    int const sw = ((lane & (MB - 1)) / RPW) & (CPRK - 1);
+    static_assert(!M16 || 16 / RPW % CPRK == 0, "the swizzle repeats every 16 rows");
 #pragma unroll
     for (int kk = 0; kk < KS; kk++) {
-      kc_off[kk] = (lane & 31) * BK + (((2 * kk + (lane >> 5)) ^ sw) << 3);
+      kc_off[kk] = (lane & (MB - 1)) * BK + (((MK / 8 * kk + lane / MB) ^ sw) << 3);
     }
   }
   auto frag_kc = [&](bf16 const *tile, int row0, int kk) -> bf16x8 {
@@ -401,9 +475,19 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   // Tile lying as [BK][cols]: lane reads rows kk*16 + 8 (l/32) + (l%16)/4 (+4),
   // columns col0 + 16 ((l/16)%2) + 4 (l%4); the 64-byte segment index is
   // XOR-ed with tr_swizzle(row), which touches only its two low bits (its one bit).
-  // One entry per 32-wide block of the wave's tile.
+  // One entry per 32-wide block of the wave's tile.  M16: rows kk*32 + 8 (l/16) + (l%16)/4 (+4), columns
+  // col0 + 4 (l%4), one entry per 16-wide block.
   int tr_tab_a[TM], tr_tab_b[TN];
-  {
+  if constexpr (M16) {
+    int const krow = (lane >> 4) * 8 + ((lane & 15) >> 2);
+    auto offset = [&](int cols, int block) {
+      return krow * cols + ((block ^ (((krow & 3) << 1) | ((krow >> 3) & 1))) << 4) + (lane & 3) * 4;
+    };
+#pragma unroll
+    for (int i = 0; i < TM; i++) tr_tab_a[i] = offset(BM, (wm0 >> 4) + i);
+#pragma unroll
+    for (int j = 0; j < TN; j++) tr_tab_b[j] = offset(BN, (wn0 >> 4) + j);
+  } else {
     int const i16 = lane & 15;
     int const q = i16 >> 2;
     int const inseg = ((lane >> 4) & 1) * 16 + (i16 & 3) * 4;
@@ -417,7 +501,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
     for (int j = 0; j < TN; j++) tr_tab_b[j] = offset(BN, (wn0 >> 5) + j);
   }
   auto frag_tr = [&](bf16 const *tile, int rowlen, int tab, int kk) -> bf16x8 {
-    bf16 const *p = tile + tab + kk * 16 * rowlen;
+    bf16 const *p = tile + tab + kk * MK * rowlen;
     typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
     s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p));
     s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p + 4 * rowlen));
@@ -430,13 +514,13 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
     return u.v;
   };
 
-  f32x16 acc[TM][TN];
+  Acc acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; i++)
 #pragma unroll
     for (int j = 0; j < TN; j++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+      for (int r = 0; r < (M16 ? 4 : 16); r++) acc[i][j][r] = 0.0f;
 
   int const KT = KG > 1 ? (KT_all + KG - 1) / KG : partial != nullptr ? (EDGE ? min(k_tiles_per_split, KT_all - kt0) : k_tiles_per_split) : KT_all;
   constexpr int NB = PF + 1;  // fragment buffers
@@ -449,17 +533,15 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   // a wave that cannot issue its next load cannot issue its next MFMA either.
   constexpr bool SPREAD = STAGES >= 3 && LPT % KS == 0;
   constexpr int PART = SPREAD ? LPT / KS : LPT;
-  // One wave per SIMD and two stages: a refill goes out in two halves, the first behind the
-  // barrier that frees its stage, the second in the first k-step of the following tile.
-  constexpr bool WIDE2 = WM == 128 && (WN == 128 || WN == 96) && STAGES == 2;
-  constexpr int PRO_PART = WIDE2 ? LPT / 2 : PART;  // of the last tile the prologue starts
+  // (One wave per SIMD and two stages: a refill goes out behind the barrier that frees its stage.)
+  constexpr int PRO_PART = WIDE2 ? LPT : PART;  // of the last tile the prologue starts
 #pragma unroll
   for (int s = 0; s < STAGES; s++) {
     if (s < KT) {
-      if ((SPREAD || WIDE2) && s == STAGES - 1) {
+      if (SPREAD && s == STAGES - 1) {
         issue_some(s, s, 0, PRO_PART, true);  // tile 0's steps issue the rest
       } else {
-        issue(s, s);
+        issue(s, WIDE2 ? 2 * s : s);
       }
     }
   }
@@ -479,6 +561,16 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
       bfr[buf][j] = TBL ? frag_tr(sb, BN, tr_tab_b[j], kk) : frag_kc(sb, wn0 + j * 32, kk);
     }
   };
+  // (M16, one wave per SIMD) one fragment of k-step kk of the panel at `at` in the ring
+  auto read_a16 = [&](int at, int i, int kk) __attribute__((always_inline)) {
+    bf16 const *sa = smem + at * PANEL;
+    af[kk][i] = TA ? frag_tr(sa, BM, tr_tab_a[i], kk) : frag_kc(sa, wm0 + i * 16, kk);
+  };
+  auto read_b16 = [&](int at, int j, int kk) __attribute__((always_inline)) {
+    bf16 const *sb = smem + at * PANEL;
+    bfr[kk][j] = TBL ? frag_tr(sb, BN, tr_tab_b[j], kk) : frag_kc(sb, wn0 + j * 16, kk);
+  };
+  constexpr int EARLY = 3;  // A's fragments of a tile's first step that are read before it begins
   // Tile 0 must have landed (STAGES-1 younger tiles may still be in flight).
   if (STAGES - 1 < KT) {
     wait_vmcnt<(STAGES - 2) * LPT + PRO_PART>();
@@ -488,8 +580,15 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   // Barrier without a memory fence: a fence would wait for every direct load
   // still in flight; the vmcnt waits already cover the tile that is needed.
   if constexpr (!ALONE) asm volatile("s_barrier" ::: "memory");
+  if constexpr (M16) {
 #pragma unroll
-  for (int kk = 0; kk < PF; kk++) read_frags(kk, 0, kk);
+    for (int j = 0; j < TN; j++) read_b16(1, j, 0);
+#pragma unroll
+    for (int i = 0; i < EARLY; i++) read_a16(0, i, 0);
+  } else {
+#pragma unroll
+    for (int kk = 0; kk < PF; kk++) read_frags(kk, 0, kk);
+  }
   // One k-tile.  STEADY: every condition of the generic body is known true
   // (next tile exists, a refill is due, STAGES-2 younger tiles in flight), so
   // the steady-state loop is branch-free.
@@ -497,82 +596,92 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   // otherwise.  With the stage a constant every LDS address of the tile is a loop-invariant
   // register plus an immediate; computed from kt it costs three vector instructions per k-step,
   // which two waves on a SIMD do not get for free.
-  auto tile_step = [&](int kt, auto steady_tag, auto stage_tag) {
+  [[maybe_unused]] int ring = 0;  // (WIDE2) where the tile's A lies
+  auto tile_step = [&](int kt, auto steady_tag, auto stage_tag) __attribute__((always_inline)) {
     constexpr bool STEADY = decltype(steady_tag)::value;
     constexpr int SST = decltype(stage_tag)::value;
     auto stage_at = [&](int d) { return SST >= 0 ? (SST + d) % STAGES : (kt + d) % STAGES; };
     int const stage = stage_at(0);
     if constexpr (WIDE2) {
       // One wave per SIMD: nothing but this wave's own instruction order hides a latency, so
-      // the order is written out.  A k-step is 16 MFMAs.  Behind each of them sits one of the 8
-      // fragment reads of the next step or one of up to 8 direct loads, alternating, fenced so
-      // that the compiler keeps them there.  The refill of a stage goes out in two halves: the
-      // first behind the barrier that frees the stage (last step of its tile), the second in
-      // step 0 of the following tile; the steps in between carry fragment reads only.
-      static_assert(PF == 1 && TM == 4 && (TN == 4 || TN == 3) && LPT % 2 == 0 && KS >= 2, "written for these shapes");
-      // A k-step has NS = TM * TN MFMAs; behind them go the NR = TM + TN fragment reads of the
-      // next step and, in the two steps that carry them, NL = LPT / 2 direct loads, each kind
-      // spread evenly over the slots with the loads half a spacing behind the reads (4 x 4
-      // blocks: reads in the even slots, loads in the odd ones; 4 x 3: twelve slots for seven
-      // reads and seven loads).
-      constexpr int NS = TM * TN, NR = TM + TN, NL = LPT / 2;
-#pragma unroll
-      for (int kk = 0; kk < KS; kk++) {
-        int const cur = kk % NB, nxt = (kk + PF) % NB;
-        bool const within = kk + PF < KS;            // the next step lies in this tile
-        bool const reads = within || STEADY || kt + 1 < KT;
-        int const rstage = within ? stage : stage_at(1);
-        int const rkk = within ? kk + PF : kk + PF - KS;
-        bf16 const *ra = smem + rstage * STAGE_ELEMS;
-        bf16 const *rb = ra + A_ELEMS;
-        bool const loads = kk == 0 ? (STEADY || kt + 1 < KT) : !within ? (STEADY || kt + 2 < KT) : false;
-        int const ltile = kk == 0 ? kt + 1 : kt + 2;
-        int const lstage = kk == 0 ? stage_at(1) : stage;
-        int const lfirst = kk == 0 ? LPT / 2 : 0;
-        // slot p follows MFMA p.  Even slots: a fragment read, in the order in which the next
-        // step's MFMAs (row block by row block) first use the fragments: A0, B0..B3, A1, A2, A3.
-        // Odd slots: a direct load.
-        auto aux = [&](int p) __attribute__((always_inline)) {
-          // (all reads first, then the loads, measured 2-7% slower: the four waves' reads then
-          // meet in the LDS pipeline in bursts)
-#pragma unroll
-          for (int r = 0; r < NR; r++) {
-            if (r * NS / NR != p || !reads) continue;
-            if (r == 0 || r > TN) {
-              int const i = r == 0 ? 0 : r - TN;
-              af[nxt][i] = TA ? frag_tr(ra, BM, tr_tab_a[i], rkk) : frag_kc(ra, wm0 + i * 32, rkk);
-            } else {
-              int const j = r - 1;
-              bfr[nxt][j] = TBL ? frag_tr(rb, BN, tr_tab_b[j], rkk) : frag_kc(rb, wn0 + j * 32, rkk);
-            }
-          }
-#pragma unroll
-          for (int l = 0; l < NL; l++) {
-            if ((2 * l + 1) * NS / (2 * NL) != p || !loads) continue;
-            issue_some(ltile, lstage, lfirst + l, 1, !STEADY);
-          }
-        };
-        __builtin_amdgcn_sched_barrier(0);
-        acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[cur][0], af[cur][0], acc[0][0], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (!within && reads) {
-          // the next tile must have landed (nothing younger is in flight with two stages) and
-          // every wave must be done reading this one
-          wait_vmcnt<0>();
-          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      // the order is written out.  A tile is two k-steps of TM * TN MFMAs, row block by row block; behind an MFMA
+      // sits at most one fragment read or one direct load, fenced so that the compiler keeps them there.
+      //   step 0   reads the rest of its own A fragments, each some 20 MFMAs ahead of its use, and all of step 1's;
+      //            A's panel of the tile after the next goes out
+      //   step 1   after BARRIER MFMAs every wave has what it needs of this tile, and the next one has landed: from
+      //            there on the next tile's B fragments and the first of A's are read, and B's panel of the
+      //            tile after it goes out
+      // LDS holds five panels: this tile's two, the next one's, and A's of the one after that, which takes the place of B's of
+      // the tile before.  So loads go out evenly over the whole tile (a CU takes in 64 bytes a cycle, 1024 of the
+      // 2048 cycles; all of them behind the barrier, and the waves waited to get theirs in: [12288,
+      // 16384] . [16384, 4096] with A transposed 1384 us, 1228 so) and have 85 MFMAs' time and more, 1360 cycles, to land.
+      static_assert(PF == 1 && KS == 2 && TM == 8 && TN % 2 == 0, "written for these shapes");
+      constexpr int NS = TM * TN, BARRIER = NS / 4;
+      constexpr int R0 = TM - EARLY + TN + TM, R1 = TN + EARLY;  // reads of the two steps, in even slots; loads in odd ones
+      static_assert(2 * R0 <= NS && 2 * R1 <= NS - BARRIER && 2 * A_LOADS <= NS && 2 * B_LOADS <= NS - BARRIER, "slots");
+      bool const next = STEADY || kt + 1 < KT, after = STEADY || kt + 2 < KT;
+      int const own_b = ring_at(ring, 1), next_a = ring_at(ring, 2), next_b = ring_at(ring, 3), after_a = ring_at(ring, 4);
+      // step 0's read r: A3, B0, B1, A4, B2, B3, ... (A's of this step, B's of the next one), then the other B's and all A's of the next
+      auto read0 = [&](int r) __attribute__((always_inline)) {
+        constexpr int OWN = TM - EARLY;
+        if (r < 2 * OWN) {
+          if (r % 2 == 0) read_a16(ring, EARLY + r / 2, 0);
+          else read_b16(own_b, r / 2, 1);
+        } else if (r < OWN + TN) {
+          read_b16(own_b, r - OWN, 1);
+        } else {
+          read_a16(ring, r - OWN - TN, 1);
         }
-#pragma unroll
-        for (int m = 1; m < TM * TN; m++) {
-          aux(m - 1);
-          __builtin_amdgcn_sched_barrier(0);
-          acc[m / TN][m % TN] =
-              __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[cur][m % TN], af[cur][m / TN], acc[m / TN][m % TN], 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
+      };
+      auto read1 = [&](int r) __attribute__((always_inline)) {
+        if (r == 0 || r > TN) read_a16(next_a, r == 0 ? 0 : r - TN, 0);
+        else read_b16(next_b, r - 1, 0);
+      };
+      // which of `count`, spread over every other slot from `first` on, sits behind MFMA m (-1: none)
+      auto behind = [](int m, int first, int count) constexpr {
+        for (int i = 0; i < count; i++) {
+          if (first + 2 * (i * ((NS - first) / 2) / count) == m) return i;
         }
-        aux(TM * TN - 1);
-      }
+        return -1;
+      };
+      auto mfma = [&](auto kk_tag, auto m_tag) __attribute__((always_inline)) {
+        constexpr int kk = decltype(kk_tag)::value, m = decltype(m_tag)::value;
+        constexpr int r = behind(m, kk == 0 ? 0 : BARRIER, kk == 0 ? R0 : R1);
+        constexpr int l = behind(m, kk == 0 ? 1 : BARRIER + 1, kk == 0 ? A_LOADS : B_LOADS);
+        Acc &d = acc[m / TN][m % TN];
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (l >= 0 && STEADY) {
+          load_operands(kt + 2, kk == 0 ? after_a : ring, kk == 0 ? l : A_LOADS + l,
+                        [&](i32x4 rsrc, unsigned off, unsigned uniform, unsigned lds) __attribute__((always_inline)) {
+            mfma16_in_place_and_load(d, bfr[kk][m % TN], af[kk][m / TN], rsrc, off, uniform, lds);
+          });
+        } else {
+          mfma16_in_place(d, bfr[kk][m % TN], af[kk][m / TN]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (l >= 0 && !STEADY) {
+          if (after) issue_some(kt + 2, after_a, kk == 0 ? l : A_LOADS + l, 1, true);
+        }
+        if constexpr (kk == 1 && m == BARRIER - 1) {
+          if (next) {
+            // younger than the next tile's panels is A's of the one after it
+            if (after) wait_vmcnt<A_LOADS>();
+            else wait_vmcnt<0>();
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          }
+        }
+        if constexpr (r >= 0) {
+          if constexpr (kk == 0) read0(r);
+          else if (next) read1(r);
+        }
+      };
+      unroll_for(std::make_integer_sequence<int, NS>{}, [&](auto m) __attribute__((always_inline)) { mfma(std::integral_constant<int, 0>{}, m); });
+      unroll_for(std::make_integer_sequence<int, NS>{}, [&](auto m) __attribute__((always_inline)) { mfma(std::integral_constant<int, 1>{}, m); });
+      __builtin_amdgcn_sched_barrier(0);
+      ring = ring_at(ring, 2);
       return;
     }
+    if constexpr (!WIDE2) {
 #pragma unroll
     for (int kk = 0; kk < KS; kk++) {
       int const cur = kk % NB;
@@ -623,6 +732,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[cur][j], af[cur][i], acc[i][j], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
+    }
   };
   using Dyn = std::integral_constant<int, -1>;
   int kt = 0;
@@ -645,17 +755,19 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
     tile_step(kt, std::false_type{}, Dyn{});
   }
   // acc[i][j][r]: output row m = wm0 + 32 i + lane % 32,
-  //               column n = wn0 + 32 j + 8 (r / 4) + 4 (lane / 32) + r % 4.
-  // The plain store (no tail, nothing to add to): straight from the registers.  A lane holds
-  // columns 8 g + 4 h .. + 3 of every group g of 8 (h = its lane half); one swap of the lane
-  // halves per pair of groups gives the lower half the 8 columns of group g and the upper half
-  // those of group g + 1, so that every lane stores 16 bytes and the two halves together 32
-  // contiguous bytes of a row.  No LDS, so no barrier either: a wave writes its tile as soon as
-  // its own loop is done.  Used by the one-wave-per-SIMD kernel, where it is 4-6% of a launch at
-  // reductions up to 2048 (FFN-up shape 37.6 -> 36.0 us); with two waves per SIMD the staged
-  // epilogue below, whose stores are whole 128-byte lines, is 2-5% ahead.  (The 32-byte pieces
-  // cost memory traffic: 49 MB written per 32 MB tile set by the write counter, whatever the
-  // order of the stores; going row by row instead of column block by column block is 3% slower.)
+  //               column n = wn0 + 32 j + 8 (r / 4) + 4 (lane / 32) + r % 4;
+  // M16:          row m = wm0 + 16 i + lane % 16, column n = wn0 + 16 j + 4 (lane / 16) + r.
+  // Both are groups of four consecutive columns (GROUPS to a block).
+  constexpr int GROUPS = M16 ? 1 : 4;
+  if constexpr (M16) mfma16_settled(acc[TM - 1]);
+  auto row_of = [&](int i) __attribute__((always_inline)) { return i * MB + (lane & (MB - 1)); };
+  auto col_of = [&](int j, int g) __attribute__((always_inline)) { return j * MB + 8 * g + 4 * (lane / MB); };
+  // The plain store (no tail, nothing to add to): straight from the registers.  A lane holds four columns of a
+  // block; swapping every other row of 16 lanes between a pair of blocks gives each lane 8 columns of one of the two,
+  // so that every lane stores 16 bytes and four lanes together 64 contiguous bytes of a row.  No LDS, so no barrier either:
+  // a wave writes its tile as soon as its own loop is done.  Used by the one-wave-per-SIMD kernel, where it
+  // was 4-6% of a launch at reductions up to 2048; with two waves per SIMD the staged
+  // epilogue below, whose stores are whole 128-byte lines, is 2-5% ahead.
   // Eight columns from column n of row m on (EDGE: those that exist).
   auto store8 = [&](int m, int n, u32x4 v) __attribute__((always_inline)) {
     bf16 *const to = C + (int64_t)m * ldc + n;
@@ -691,29 +803,27 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
     if (partial == nullptr && accumulate == 0) {  // uniform over the launch
       auto direct = [&](auto actf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-          float bv[4][4];
+        for (int j = 0; j < TN; j += 2) {
+          float bv[2][4];
 #pragma unroll
-          for (int g = 0; g < 4; g++) bias4(n0 + wn0 + j * 32 + 8 * g + 4 * (lane >> 5), bv[g]);
+          for (int jj = 0; jj < 2; jj++) bias4(n0 + wn0 + col_of(j + jj, 0), bv[jj]);
+          int const h = lane >> 4, n = (j + (h & 1)) * 16 + (h >> 1) * 8;
 #pragma unroll
           for (int i = 0; i < TM; i++) {
+            uint32_t w[2][2];
 #pragma unroll
-            for (int g = 0; g < 4; g += 2) {
-              uint32_t w[2][2];
+            for (int jj = 0; jj < 2; jj++) {
+              float v[4];
 #pragma unroll
-              for (int gg = 0; gg < 2; gg++) {
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = actf(acc[i][j][4 * (g + gg) + e] + bv[g + gg][e]);
-                w[gg][0] = pack_bf16x2(v[0], v[1]);
-                w[gg][1] = pack_bf16x2(v[2], v[3]);
-              }
-              // swaps the upper lane half of the first operand with the lower half of the second
-              auto const lo = __builtin_amdgcn_permlane32_swap(w[0][0], w[1][0], false, false);
-              auto const hi = __builtin_amdgcn_permlane32_swap(w[0][1], w[1][1], false, false);
-              u32x4 const out = {lo[0], hi[0], lo[1], hi[1]};
-              store8(m0 + wm0 + i * 32 + (lane & 31), n0 + wn0 + j * 32 + 8 * (lane >> 5) + 8 * g, out);
+              for (int e = 0; e < 4; e++) v[e] = actf(acc[i][j + jj][e] + bv[jj][e]);
+              w[jj][0] = pack_bf16x2(v[0], v[1]);
+              w[jj][1] = pack_bf16x2(v[2], v[3]);
             }
+            // swaps the odd rows of 16 lanes of the first operand with the even rows of the second
+            auto const lo = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+            auto const hi = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+            u32x4 const out = {lo[0], hi[0], lo[1], hi[1]};
+            store8(m0 + wm0 + row_of(i), n0 + wn0 + n, out);
           }
         }
       };
@@ -923,13 +1033,13 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
 #pragma unroll
     for (int j = 0; j < TN; j++) {
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        int const n = j * 32 + 8 * g + 4 * (lane >> 5);
+      for (int g = 0; g < GROUPS; g++) {
+        int const n = col_of(j, g);
         float bv[4];
         bias4(n0 + wn0 + n, bv);
 #pragma unroll
         for (int i = half * TMH; i < (half + 1) * TMH; i++) {
-          int const m = i * 32 + (lane & 31);
+          int const m = row_of(i);
           float v[4];
 #pragma unroll
           for (int e = 0; e < 4; e++) v[e] = acc[i][j][4 * g + e] + bv[e];
@@ -977,12 +1087,12 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
     float *dst = partial + (int64_t)split * M * N;
 #pragma unroll
     for (int i = 0; i < TM; i++) {
-      int64_t const m = m0 + wm0 + i * 32 + (lane & 31);
+      int64_t const m = m0 + wm0 + row_of(i);
 #pragma unroll
       for (int j = 0; j < TN; j++) {
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-          int const n = n0 + wn0 + j * 32 + 8 * g + 4 * (lane >> 5);
+        for (int g = 0; g < GROUPS; g++) {
+          int const n = n0 + wn0 + col_of(j, g);
           if (EDGE != kEdgeNone && m >= M) continue;
           if (EDGE == kEdgeBounded && n >= N) continue;  // (N % 4 == 0 where a reduction is split)
           f32x4 v = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
@@ -1044,7 +1154,8 @@ static __global__ __launch_bounds__(256) void splitk_reduce_kernel(
 template <int BM, int BN, int WM, int WN, int BK, int STAGES>
 struct PipeCfg {
   static constexpr int NW = (BM / WM) * (BN / WN);
-  static constexpr size_t kStageBytes = (size_t)STAGES * (BM + BN) * BK * sizeof(bf16);
+  // (one wave per SIMD: five panels)
+  static constexpr size_t kStageBytes = (size_t)(WM == 128 && STAGES == 2 ? 5 * (BM > BN ? BM : BN) : STAGES * (BM + BN)) * BK * sizeof(bf16);
   static constexpr size_t kOutBytes = (size_t)NW * WM * (WN + 8) * sizeof(bf16);
   static constexpr size_t kLds = kStageBytes > kOutBytes ? kStageBytes : kOutBytes;
   static_assert(kLds <= 160 * 1024, "LDS budget");
