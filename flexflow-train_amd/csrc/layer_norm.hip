@@ -41,11 +41,11 @@ __global__ __launch_bounds__(kRowThreads) void layer_norm_fwd_kernel(
 
   float x[EPT][V];
   float s = 0.0f;
-  // Short rows (up to two vectors per lane): gamma and beta are asked for before the row's two
+  // Short rows (up to two vectors per lane, or twelve elements): gamma and beta are asked for before the row's two
   // reductions, not after them: such a kernel is one chain of memory round trips, and this one
   // then runs under the others.  Longer rows load them where they are used; their registers
   // are better spent on resident waves.
-  constexpr bool kEarly = EPT <= 2;
+  constexpr bool kEarly = EPT <= 2 || EPT * V <= 12;
   float g[EPT][V], b[EPT][V];
   auto load_params = [&](int j) __attribute__((always_inline)) {
     int v = lane + j * LANES;
@@ -457,7 +457,7 @@ static int ln_forward(hipStream_t st, void const *x, void *y, void const *gamma,
   int ept = 0, lanes = 0;
   bool const vec = (N % V == 0) && aligned16(x) && aligned16(y) && (gamma == nullptr || aligned16(gamma)) &&
                    (beta == nullptr || aligned16(beta));
-  if (!pick_row_config_small(ceil_div(N, V), ept, lanes)) {
+  if (!pick_row_config_small(ceil_div(N, V), ln_fwd_wave_vectors<T>(), ept, lanes)) {
     layer_norm_fwd_generic_kernel<T><<<(unsigned)M, kRowThreads, 0, st>>>(
         X, Y, G, Bt, mean, rstd, M, (int)N, eps);
   } else if (vec) {
@@ -472,14 +472,14 @@ static int ln_forward(hipStream_t st, void const *x, void *y, void const *gamma,
       layer_norm_fwd_kernel<T, E, L><<<(unsigned)blocks, kRowThreads, 0, st>>>( \
           X, Y, G, Bt, mean, rstd, M, (int)N, eps);                            \
   } while (0)
-    FFK_ROW_DISPATCH_SMALL(ept, lanes, CALL);
+    FFK_ROW_DISPATCH_FORWARD(ept, lanes, CALL);
 #undef CALL
   } else {
     // [3001, 1001] fp32: 11.3 us with the scalar kernel, which reads a row three times
 #define CALL(E, L)                                                                                             \
   layer_norm_fwd_kernel<T, E, L, false, false, true><<<(unsigned)ceil_div(M, kRowThreads / lanes), kRowThreads, 0, st>>>( \
       X, Y, G, Bt, mean, rstd, M, (int)N, eps)
-    FFK_ROW_DISPATCH_SMALL(ept, lanes, CALL);
+    FFK_ROW_DISPATCH_FORWARD(ept, lanes, CALL);
 #undef CALL
   }
   FFK_CHECK_LAUNCH();
@@ -505,7 +505,7 @@ static int ln_backward(hipStream_t st, void const *dy, void const *x,
   T const *G = static_cast<T const *>(gamma);
   T *DX = static_cast<T *>(dx);
   int ept = 0, lanes = 0;
-  bool const fits = pick_row_config_small(ceil_div(N, V), ept, lanes);
+  bool const fits = pick_row_config_small(ceil_div(N, V), ln_bwd_wave_vectors(M), ept, lanes);
   bool const vec = (N % V == 0) && aligned16(dy) && aligned16(x) && (dx == nullptr || aligned16(dx)) &&
                    aligned16(residual) && (gamma == nullptr || aligned16(gamma)) && fits;
   if (!vec && RES != nullptr) {
@@ -591,7 +591,7 @@ static int ln_forward_pre(hipStream_t st, void const *in, void const *residual, 
   int ept = 0, lanes = 0;
   bool vec = (N % 8 == 0) && (drop.offset & 7) == 0 && aligned16(in) && aligned16(residual) && aligned16(summed) &&
              aligned16(y) && (gamma == nullptr || aligned16(gamma)) && (beta == nullptr || aligned16(beta)) &&
-             pick_row_config_small(N / V, ept, lanes);
+             pick_row_config_small(N / V, ln_fwd_wave_vectors<T>(), ept, lanes);
   if (!vec) return FFK_ERR_UNSUPPORTED;
   int64_t blocks = ceil_div(M, kRowThreads / lanes);
 #define CALL(E, L)                                                                                  \
@@ -599,7 +599,7 @@ static int ln_forward_pre(hipStream_t st, void const *in, void const *residual, 
       static_cast<T const *>(in), static_cast<T *>(y), static_cast<T const *>(gamma),             \
       static_cast<T const *>(beta), mean, rstd, M, (int)N, eps, static_cast<T const *>(residual), \
       static_cast<T *>(summed), drop)
-  FFK_ROW_DISPATCH_SMALL(ept, lanes, CALL);
+  FFK_ROW_DISPATCH_FORWARD(ept, lanes, CALL);
 #undef CALL
   FFK_CHECK_LAUNCH();
   return FFK_OK;

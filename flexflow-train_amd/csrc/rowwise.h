@@ -155,13 +155,13 @@ static inline bool pick_row_config(int64_t nvec, int &ept, int &lanes) {
   return false;
 }
 
-// The LayerNorm kernels': at most one wave per row up to 128 vectors,
+// The LayerNorm kernels': at most one wave per row up to 128 vectors, or up to 64 * wave_vectors of them,
 // one workgroup per row beyond (few vectors per lane keeps register use low and
 // measured 76% vs 59% of HBM peak for a [16384, 4096] bf16 LayerNorm forward).
-static inline bool pick_row_config_small(int64_t nvec, int &ept, int &lanes) {
-  if (nvec <= 128) {
+static inline bool pick_row_config_small(int64_t nvec, int wave_vectors, int &ept, int &lanes) {
+  if (nvec <= 64 * wave_vectors) {
     lanes = nvec <= 16 ? 16 : nvec <= 32 ? 32 : 64;
-    ept = nvec <= 64 ? 1 : 2;
+    ept = nvec <= 64 ? 1 : (int)((nvec + 63) / 64);
     return true;
   }
   if (nvec <= 256 * 8) {
@@ -172,6 +172,20 @@ static inline bool pick_row_config_small(int64_t nvec, int &ept, int &lanes) {
   return false;
 }
 
+// Rows of 129 to 256 vectors leave up to half of a workgroup's lanes idle, and pass a barrier for each sum, where a
+// wave takes them in three or four vectors a lane.  The wave's form and, in brackets, the workgroup's:
+//   forward, 129-192 vectors: [60000, 513] fp32 46 us (67), [32768, 768] 41 (42), [3001, 640] 5.1 (5.8); bf16
+//     [60000, 1025] 61 (106), [32768, 1536] 43 (56), [4096, 1280] 6.4 (7.8)
+//   forward, 193-256 vectors: bf16 [32768, 1800] 54 (61), [16384, 2048] 30 (34), [3001, 2048] 7.7 (7.6); but fp32
+//     [32768, 1000] 54 (48), whose workgroup has fewer idle lanes than its rows have bytes
+template <typename T>
+constexpr int ln_fwd_wave_vectors() { return sizeof(T) == 2 ? 4 : 3; }
+//   backward, 129-192 vectors: [60000, 513] fp32 74 (126), [16384, 768] 35 (42), [6000, 768] 15.0 (15.2); bf16 [60000, 1025]
+//     76 (148), [16384, 1280] 32 (44), [6000, 1536] 17.1 (17.4); but [4096, 768] 12.9 (12.4), bf16 [4096, 1280] 14.7
+//     (13.5): waves of few rows each, whose sums of the parameters' gradients have yet to be folded
+//   backward, 193-256 vectors: bf16 [16384, 2048] 52 (47), fp32 [4096, 1024] 15 (14): registers
+inline int ln_bwd_wave_vectors(int64_t rows) { return rows >= 6000 ? 3 : 2; }
+
 #define FFK_ROW_DISPATCH_SMALL(EPT_, LANES_, CALL)                             \
   do {                                                                         \
     if ((LANES_) == 16) {                                                      \
@@ -180,12 +194,23 @@ static inline bool pick_row_config_small(int64_t nvec, int &ept, int &lanes) {
       CALL(1, 32);                                                             \
     } else if ((LANES_) == 64) {                                               \
       if ((EPT_) == 1) { CALL(1, 64); }                                        \
-      else { CALL(2, 64); }                                                    \
+      else if ((EPT_) == 2) { CALL(2, 64); }                                   \
+      else { CALL(3, 64); }                                                    \
     } else {                                                                   \
       if ((EPT_) == 1) { CALL(1, 256); }                                       \
       else if ((EPT_) == 2) { CALL(2, 256); }                                  \
       else if ((EPT_) == 4) { CALL(4, 256); }                                  \
       else { CALL(8, 256); }                                                   \
+    }                                                                          \
+  } while (0)
+
+// (and of T where a wave takes four vectors a lane)
+#define FFK_ROW_DISPATCH_FORWARD(EPT_, LANES_, CALL)                           \
+  do {                                                                         \
+    if ((LANES_) == 64 && (EPT_) == 4) {                                       \
+      if constexpr (ln_fwd_wave_vectors<T>() == 4) { CALL(4, 64); }            \
+    } else {                                                                   \
+      FFK_ROW_DISPATCH_SMALL(EPT_, LANES_, CALL);                              \
     }                                                                          \
   } while (0)
 
