@@ -32,7 +32,23 @@ __device__ __forceinline__ void colreduce_block(ColreduceJob const &job, int blo
     for (int q = 0; q < 4; q++) s[g][q] = 0.0f;
   if (j < job.ncols) {
     float const *p = job.partials + j;
-    for (int r = 0; r < job.nparts; r += 128) {
+    int r = 0;
+    // Whole blocks of rows, four of them in flight where a thread has one row group of each: the loads are the time.
+    // (All rows guarded, one block in flight: LayerNorm backward 0.4 us longer, [4096, 1024] fp32 15.0 us and 14.4.)
+    constexpr int kBlocks = G == 1 ? 4 : 1;
+#pragma unroll kBlocks
+    for (; r + 128 <= job.nparts; r += 128) {
+      float v[G][4];
+#pragma unroll
+      for (int g = 0; g < G; g++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[g][q] = p[(int64_t)(r + ry + g * (NT / 32) + q * 32) * job.ncols];
+#pragma unroll
+      for (int g = 0; g < G; g++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) s[g][q] += v[g][q];
+    }
+    if (r < job.nparts) {
       float v[G][4];
 #pragma unroll
       for (int g = 0; g < G; g++)
