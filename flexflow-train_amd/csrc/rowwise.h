@@ -141,7 +141,17 @@ __device__ __forceinline__ int lane_in_row() {
 
 // Picks (EPT, LANES) for a row of `nvec` 16-byte vectors; returns false when the
 // row does not fit in registers (nvec > 256 * 8).
-static inline bool pick_row_config(int64_t nvec, int &ept, int &lanes) {
+// whole: rows of whole aligned vectors.  A workgroup, two vectors a lane, takes rows that a wave would need eight a
+// lane for, where it has few idle lanes.  Softmax forward / backward, us, and in brackets by waves: bf16 [16384, 4096] 47 / 62
+// (51 / 67), [16384, 3600] 43 / 59 (51 / 59), [3001, 3600] 8.9 / 10.6 (9.6 / 10.5), fp32 [16384, 1800] 43 / 59 (54 / 60), [8192,
+// 1537] 18.5 / 28.5 (19.3 / 29.5).  Not fp32 rows that fill the wave ([8192, 2048] 24.9 / 36.7 (23.2 / 39.8)), nor bf16 rows at any
+// address ([16384, 3073] 41 / 62 (38 / 55)), nor rows of few more vectors than 256 (bf16 [16384, 2060] 29.3 / 36.9 (27.1 / 38.3)).
+static inline bool pick_row_config(int64_t nvec, size_t elem_size, bool whole, int &ept, int &lanes) {
+  if (nvec > 320 && (elem_size == 2 ? whole && nvec <= 512 : nvec <= 480)) {
+    lanes = 256;
+    ept = 2;
+    return true;
+  }
   if (nvec <= 64 * 8) {
     lanes = nvec <= 16 ? 16 : nvec <= 32 ? 32 : 64;
     ept = nvec <= 64 ? 1 : nvec <= 128 ? 2 : nvec <= 256 ? 4 : 8;
@@ -226,7 +236,8 @@ inline int ln_bwd_wave_vectors(int64_t rows) { return rows >= 6000 ? 3 : 2; }
       else if ((EPT_) == 4) { CALL(4, 64); }                                   \
       else { CALL(8, 64); }                                                    \
     } else {                                                                   \
-      if ((EPT_) == 4) { CALL(4, 256); }                                       \
+      if ((EPT_) == 2) { CALL(2, 256); }                                       \
+      else if ((EPT_) == 4) { CALL(4, 256); }                                  \
       else { CALL(8, 256); }                                                   \
     }                                                                          \
   } while (0)

@@ -194,9 +194,9 @@ static int softmax_fwd(hipStream_t st, void const *x, void *y, int64_t outer,
   T *Y = static_cast<T *>(y);
   if (inner == 1) {
     int ept = 0, lanes = 0;
-    if (pick_row_config(ceil_div(dim, V), ept, lanes)) {
+    bool const vec = dim % V == 0 && aligned16(x) && aligned16(y);
+    if (pick_row_config(ceil_div(dim, V), sizeof(T), vec, ept, lanes)) {
       int64_t blocks = ceil_div(outer, kRowThreads / lanes);
-      bool const vec = dim % V == 0 && aligned16(x) && aligned16(y);
       bool const stream = stream_past_caches(outer * dim, sizeof(T));
 #define CALL(E, L)                                                             \
   do {                                                                         \
@@ -229,9 +229,9 @@ static int softmax_bwd(hipStream_t st, void const *y, void const *dy, void *dx,
   T *DX = static_cast<T *>(dx);
   if (inner == 1) {
     int ept = 0, lanes = 0;
-    if (pick_row_config(ceil_div(dim, V), ept, lanes)) {
+    bool const vec = dim % V == 0 && aligned16(y) && aligned16(dy) && aligned16(dx);
+    if (pick_row_config(ceil_div(dim, V), sizeof(T), vec, ept, lanes)) {
       int64_t blocks = ceil_div(outer, kRowThreads / lanes);
-      bool const vec = dim % V == 0 && aligned16(y) && aligned16(dy) && aligned16(dx);
       bool const stream = three_past_caches(outer * dim, sizeof(T));
 #define CALL(E, L)                                                             \
   do {                                                                         \
