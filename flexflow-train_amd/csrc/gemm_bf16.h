@@ -102,7 +102,7 @@ __device__ __forceinline__ void mfma16_in_place(f32x4 &acc, bf16x8 a, bf16x8 b) 
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
 // ... and a direct load behind it: the MFMA stands between the write of M0 and the load that reads it, where lds_dma16 has
-// a wait state.
+// a wait state.  (The descriptor needs more of them: uniform_pointer in lds_dma.h.)
 __device__ __forceinline__ void mfma16_in_place_and_load(f32x4 &acc, bf16x8 a, bf16x8 b, i32x4 rsrc, unsigned lane_byte_off,
                                                          unsigned uniform_byte_off, unsigned lds_byte_addr) {
   asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\tbuffer_load_dwordx4 %4, %5, %6 offen lds"
@@ -348,8 +348,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64 * KG) void gemm_bf16_pip
   int const KT_all = EDGE ? (K + BK - 1) / BK : K / BK;  // k-tiles of the whole reduction
   int64_t const step_a = TA ? (int64_t)(NT * 8 / BM) * lda : (int64_t)ROWS_PER_LOAD_KC * lda;
   int64_t const step_b = TBL ? (int64_t)(NT * 8 / BN) * ldb : (int64_t)ROWS_PER_LOAD_KC * ldb;
-  bf16 const *const panel_a = TA ? A + m0 : A + (int64_t)m0 * lda;
-  bf16 const *const panel_b = TBL ? B + n0 : B + (int64_t)n0 * ldb;
+  bf16 const *const panel_a = uniform_pointer(TA ? A + m0 : A + (int64_t)m0 * lda);
+  bf16 const *const panel_b = uniform_pointer(TBL ? B + n0 : B + (int64_t)n0 * ldb);
   // (kEdgeBounded) lanes whose rows or columns lie past the operand ask for what no descriptor covers and get
   // zeros: of a K-contiguous panel each load has rows of its own, of one lying [BK][cols] all have the lane's columns
   constexpr bool ROWS_A = EDGE == kEdgeBounded && !TA, ROWS_B = EDGE == kEdgeBounded && !TBL;

@@ -71,6 +71,19 @@ __device__ __forceinline__ i32x4 buffer_resource(void const *base, unsigned num_
   r[3] = 0x00020000;
   return r;
 }
+// A pointer that all lanes of a wave share, as a scalar.  What a division by a run-time value went into is computed
+// in vector registers, and so is every address made of it: buffer_resource then moves the address over right in front of the
+// direct load, which reads it fewer than the five wait states later that a scalar register written by a vector
+// instruction needs before a vector-memory instruction (the compiler keeps that distance, but not from instructions written
+// out).  A kernel whose loop forms descriptors makes their base a scalar once, and adds to it in scalar registers.
+// tests/test_wait_states.py looks at every direct load of the built library.
+template <typename T>
+__device__ __forceinline__ T *uniform_pointer(T *p) {
+  uint64_t const a = reinterpret_cast<uint64_t>(p);
+  // (unsigned: the builtin returns an int, whose sign would fill the upper half)
+  unsigned const lo = __builtin_amdgcn_readfirstlane((unsigned)a), hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+  return reinterpret_cast<T *>((uint64_t)hi << 32 | lo);
+}
 // The LDS byte address of a __shared__ object, as a scalar.
 __device__ __forceinline__ unsigned lds_address_of(void *p) {
   return __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)p);
