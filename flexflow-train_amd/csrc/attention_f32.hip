@@ -1148,22 +1148,20 @@ int attention_f32_forward(hipStream_t st, ffk_attention_desc_t const *d, void co
   return FFK_OK;
 }
 
-// Scratch for dS, which lets dQ's kernel skip two of its three products, and how many pairs of batch entry and head
-// go into it at a time: all of them, or in several launches where those still fill the chip twice over; 0: no use of it.
-// Half a GB holds dS of every block of up to 700 rows that was measured; where it does not, a launch for a part of the
-// heads still has two workgroups a CU.
+// Scratch for dS, which lets dQ's kernel skip two of its three products: how many pairs of batch entry and head go into
+// `bytes` of it at a time, all of them, or as many in several launches where those still fill the chip twice over; 0: no use
+// of it.  Half a GB holds dS of every block of up to 700 rows that was measured; where it does not, a launch for a
+// part of the heads still has two workgroups a CU.  What is asked for is what is used: by this rule too.
 constexpr size_t kMostScores = (size_t)512 << 20;
 static int64_t f32_scores_row(int64_t seq_kv) { return ceil_div(seq_kv, 32) * 32; }
-size_t attention_f32_scores_bytes(int64_t pairs, int64_t seq_q, int64_t seq_kv) {
+static int64_t f32_pairs_at_a_time(int64_t pairs, int64_t seq_q, int64_t seq_kv, size_t bytes) {
   if (pairs <= 0 || seq_q <= 0 || seq_kv <= 0 || seq_q >= (1 << 30) || seq_kv >= (1 << 30)) return 0;
-  size_t const one = (size_t)seq_q * f32_scores_row(seq_kv) * sizeof(float), most = kMostScores / one;
-  return one * std::min<size_t>((size_t)pairs, most);
+  int64_t const most = (int64_t)(std::min(bytes, kMostScores) / ((size_t)seq_q * f32_scores_row(seq_kv) * sizeof(float)));
+  if (most >= pairs) return pairs;
+  return most * ceil_div(std::min(seq_q, seq_kv), 128) >= 2 * kNumCU ? most : 0;
 }
-static int64_t f32_pairs_at_a_time(AttnF32Params const &p, size_t bytes) {
-  int64_t const all = (int64_t)p.H * p.B;
-  int64_t const most = (int64_t)(std::min(bytes, kMostScores) / ((size_t)p.Sq * f32_scores_row(p.Skv) * sizeof(float)));
-  if (most >= all) return all;
-  return most * ceil_div(std::min(p.Sq, p.Skv), 128) >= 2 * kNumCU ? most : 0;
+size_t attention_f32_scores_bytes(int64_t pairs, int64_t seq_q, int64_t seq_kv) {
+  return (size_t)f32_pairs_at_a_time(pairs, seq_q, seq_kv, kMostScores) * (size_t)seq_q * f32_scores_row(seq_kv) * sizeof(float);
 }
 
 template <int DP, bool DMA>
@@ -1193,7 +1191,7 @@ static void launch_f32_backward(hipStream_t st, AttnF32Params const &p, int64_t 
       attn_f32_bwd_dkdv_kernel<DP, SAVE><<<(unsigned)(ceil_div(p.Skv, 128) * n), 256, 0, st>>>(q);
     }
   };
-  if (int64_t const at_a_time = f32_pairs_at_a_time(p, scratch_bytes); scratch != nullptr && at_a_time > 0) {
+  if (int64_t const at_a_time = f32_pairs_at_a_time(heads, p.Sq, p.Skv, scratch_bytes); scratch != nullptr && at_a_time > 0) {
     AttnF32Params q = p;
     q.ds = static_cast<float *>(scratch);
     q.ds_ld = f32_scores_row(p.Skv);

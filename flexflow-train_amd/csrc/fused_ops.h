@@ -88,7 +88,7 @@ int mha_backward_add_residual(hipStream_t st, int dtype, ffk_mha_desc_t const *d
                               void const *output_grad, void *reserve, size_t reserve_bytes, int accumulate);
 
 // ffk_attention_backward, with scratch (16-byte aligned, nullptr: none) that lets it compute dS once instead of
-// twice.  attention_scores_bytes: what it can use of it; less, or none, is as good as the entry point.
+// twice.  attention_f32_scores_bytes: what it makes use of, none for some shapes; less, or none, is taken too.
 int attention_backward(hipStream_t st, int dtype, ffk_attention_desc_t const *d, void const *q, void const *k, void const *v,
                        void const *o, void const *d_o, float const *lse, float *delta, void *dq, void *dk, void *dv,
                        void *scratch, size_t scratch_bytes);

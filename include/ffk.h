@@ -638,8 +638,9 @@ int ffk_attention_backward(ffk_stream_t stream, int dtype,
  *   plus backward scratch, like MHAPerDeviceState.reserveSpace.  Its layout
  *   follows from the descriptor alone, so backward needs the descriptor forward
  *   had and nothing else.  For FLOAT the size asked for includes up to 512 MB
- *   behind that in which backward keeps dS, so that it is computed once; a
- *   reserve space without this part is taken as well.
+ *   behind that, for shapes where backward makes use of it: it keeps dS there,
+ *   so that it is computed once.  A reserve space without this part is taken as
+ *   well.
  * backward: query_grad/key_grad/value_grad are overwritten unless accumulate
  *   (cudnnMultiHeadAttnBackwardData stores them);
  *   key_grad/value_grad may be NULL when key/value alias query (their
