@@ -186,6 +186,9 @@ SIGNATURES = {
                                 c_p, c_sz]),
     "ffk_mha_backward": (c_int, [c_p, c_int, ctypes.POINTER(MHADesc), c_p, c_p, c_p, c_p, c_p,
                                  c_p, c_p, c_p, c_p, c_p, c_sz, c_int]),
+    "ffk_mha_backward_workspace_bytes": (c_sz, [ctypes.POINTER(MHADesc), c_int]),
+    "ffk_mha_backward_with_workspace": (c_int, [c_p, c_int, ctypes.POINTER(MHADesc), c_p, c_p, c_p, c_p, c_p,
+                                                c_p, c_p, c_p, c_p, c_p, c_sz, c_p, c_sz, c_int]),
     "ffk_encoder_layer_workspace_bytes": (c_sz, [ctypes.POINTER(EncoderLayerDesc), c_int]),
     "ffk_encoder_layer_forward": (c_int, [c_p, c_int, ctypes.POINTER(EncoderLayerDesc),
                                           ctypes.POINTER(EncoderLayerParams), c_p, c_p, c_p, c_sz]),
@@ -694,10 +697,18 @@ def mha_desc(num_samples, num_heads, q_size, k_size, v_size, q_proj, k_proj, v_p
 MHA_ACC_INPUT_GRADS, MHA_OVERWRITE_WEIGHT_GRAD = 1, 2
 
 
-def mha_reserve(desc, dtype, device="cuda"):
+def mha_reserve(desc, dtype, device="cuda", backward_scratch=True):
+    """backward_scratch=False: without the part that is scratch of the backward alone, which layers can share
+    (mha_backward_workspace)."""
     torch = _torch()
     n = _call.ffk_mha_reserve_bytes(desc, dtype)
+    if not backward_scratch:
+        n -= _call.ffk_mha_backward_workspace_bytes(desc, dtype)
     return torch.empty((n,), dtype=torch.uint8, device=device)
+
+
+def mha_backward_workspace(desc, dtype, device="cuda"):
+    return _torch().empty((_call.ffk_mha_backward_workspace_bytes(desc, dtype),), dtype=_torch().uint8, device=device)
 
 
 def mha_forward(desc, query, key, value, weight, reserve, out=None):
@@ -710,8 +721,12 @@ def mha_forward(desc, query, key, value, weight, reserve, out=None):
 
 
 def mha_backward(desc, query, dquery, key, dkey, value, dvalue, weight, dweight, out_grad,
-                 reserve, accumulate=False):
-    _call.ffk_mha_backward(dtype_of(query), desc, query, dquery, key, dkey, value, dvalue, weight, dweight, out_grad, reserve, reserve.numel(), int(accumulate))
+                 reserve, accumulate=False, workspace=None):
+    if workspace is None:
+        _call.ffk_mha_backward(dtype_of(query), desc, query, dquery, key, dkey, value, dvalue, weight, dweight, out_grad, reserve, reserve.numel(), int(accumulate))
+    else:
+        _call.ffk_mha_backward_with_workspace(dtype_of(query), desc, query, dquery, key, dkey, value, dvalue, weight, dweight,
+                                              out_grad, reserve, reserve.numel(), workspace, workspace.numel(), int(accumulate))
     return dquery, dkey, dvalue, dweight
 
 

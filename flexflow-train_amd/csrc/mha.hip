@@ -15,8 +15,8 @@
 //
 // Reserve space layout (bytes, each region 256-byte aligned):
 //   QKV projections | context | lse | delta | d(context) | d(QKV projections) | dS
-// The last one is room that the backward makes use of where the caller has it (FLOAT); a reserve space
-// without it does as well.
+// The last one is scratch that the backward makes use of where the caller has it (FLOAT), here or in memory that it
+// shares between layers; a reserve space without it does as well.
 #include "gemm.h"
 #include "fused_ops.h"
 
@@ -121,6 +121,12 @@ extern "C" size_t ffk_mha_reserve_bytes(ffk_mha_desc_t const *d, int dtype) {
   return make_layout(d, dtype_size(dtype)).with_scores;
 }
 
+extern "C" size_t ffk_mha_backward_workspace_bytes(ffk_mha_desc_t const *d, int dtype) {
+  if (d == nullptr || dtype_size(dtype) == 0) return 0;
+  MhaLayout const L = make_layout(d, dtype_size(dtype));
+  return L.with_scores - L.total;
+}
+
 extern "C" int ffk_mha_forward(ffk_stream_t stream, int dtype,
                                ffk_mha_desc_t const *d, void const *query,
                                void const *key, void const *value,
@@ -175,11 +181,11 @@ extern "C" int ffk_mha_forward(ffk_stream_t stream, int dtype,
 }
 
 // residual != nullptr (self-attention on one tensor): query_grad = residual + gradient where the library
-// has that kernel (*added says so).
+// has that kernel (*added says so).  scratch: for dS; nullptr: what the reserve space has room for.
 static int mha_backward_impl(ffk_stream_t stream, int dtype, ffk_mha_desc_t const *d, void const *query, void *query_grad,
                              void const *key, void *key_grad, void const *value, void *value_grad, void const *weight,
-                             void *weight_grad, void const *output_grad, void *reserve, size_t reserve_bytes, int accumulate,
-                             void const *residual, bool *added) {
+                             void *weight_grad, void const *output_grad, void *reserve, size_t reserve_bytes, void *scratch,
+                             size_t scratch_bytes, int accumulate, void const *residual, bool *added) {
   int rc = check_mha("mha_backward", dtype, d);
   if (rc != FFK_OK) return rc;
   FFK_REQUIRE(query && key && value && weight && output_grad, "mha_backward: NULL tensor");
@@ -244,9 +250,12 @@ static int mha_backward_impl(ffk_stream_t stream, int dtype, ffk_mha_desc_t cons
     dqp = dqkv; dkp = dqkv + L.nQ * es; dvp = dqkv + (L.nQ + L.nK) * es;
   }
   // The core writes dQ/dK/dV with the same strides it reads Q/K/V with.
-  size_t const more = reserve_bytes - L.total;
+  if (scratch == nullptr) {
+    scratch = rs + L.total;
+    scratch_bytes = reserve_bytes - L.total;
+  }
   rc = attention_backward(st, dtype, &a, qp, kp, vp, ctx, dctx, reinterpret_cast<float const *>(rs + L.off_lse),
-                          reinterpret_cast<float *>(rs + L.off_delta), dqp, dkp, dvp, aligned16(rs + L.total) ? rs + L.total : nullptr, more);
+                          reinterpret_cast<float *>(rs + L.off_delta), dqp, dkp, dvp, aligned16(scratch) ? scratch : nullptr, scratch_bytes);
   if (rc != FFK_OK) return rc;
 
   if (folded) {
@@ -303,7 +312,16 @@ extern "C" int ffk_mha_backward(ffk_stream_t stream, int dtype, ffk_mha_desc_t c
                                 void *value_grad, void const *weight, void *weight_grad, void const *output_grad,
                                 void *reserve, size_t reserve_bytes, int accumulate) {
   return mha_backward_impl(stream, dtype, d, query, query_grad, key, key_grad, value, value_grad, weight, weight_grad,
-                           output_grad, reserve, reserve_bytes, accumulate, nullptr, nullptr);
+                           output_grad, reserve, reserve_bytes, nullptr, 0, accumulate, nullptr, nullptr);
+}
+
+extern "C" int ffk_mha_backward_with_workspace(ffk_stream_t stream, int dtype, ffk_mha_desc_t const *d, void const *query,
+                                               void *query_grad, void const *key, void *key_grad, void const *value,
+                                               void *value_grad, void const *weight, void *weight_grad,
+                                               void const *output_grad, void *reserve, size_t reserve_bytes, void *workspace,
+                                               size_t workspace_bytes, int accumulate) {
+  return mha_backward_impl(stream, dtype, d, query, query_grad, key, key_grad, value, value_grad, weight, weight_grad,
+                           output_grad, reserve, reserve_bytes, workspace, workspace_bytes, accumulate, nullptr, nullptr);
 }
 
 namespace ffk {
@@ -313,7 +331,7 @@ int mha_backward_add_residual(hipStream_t st, int dtype, ffk_mha_desc_t const *d
                               void const *output_grad, void *reserve, size_t reserve_bytes, int accumulate) {
   *added = false;
   return mha_backward_impl(st, dtype, d, x, x_grad, x, nullptr, x, nullptr, weight, weight_grad, output_grad, reserve,
-                           reserve_bytes, accumulate, residual, added);
+                           reserve_bytes, nullptr, 0, accumulate, residual, added);
 }
 
 }  // namespace ffk

@@ -182,6 +182,7 @@ PyMethodDef methods[] = {
     ENTRY(ffk_linear_backward_dropout_gelu_bias_grad), ENTRY(ffk_embedding_forward), ENTRY(ffk_embedding_backward),
     ENTRY(ffk_embedding_backward_workspace_bytes), ENTRY(ffk_embedding_backward_typed), ENTRY(ffk_attention_forward),
     ENTRY(ffk_attention_backward), ENTRY(ffk_mha_reserve_bytes), ENTRY(ffk_mha_forward), ENTRY(ffk_mha_backward),
+    ENTRY(ffk_mha_backward_workspace_bytes), ENTRY(ffk_mha_backward_with_workspace),
     ENTRY(ffk_encoder_layer_workspace_bytes), ENTRY(ffk_encoder_layer_forward), ENTRY(ffk_encoder_layer_backward),
     ENTRY(ffk_sgd_update), ENTRY(ffk_adam_update), ENTRY(ffk_sparse_categorical_crossentropy_loss_backward),
     ENTRY(ffk_categorical_crossentropy_loss_backward), ENTRY(ffk_mean_squared_error_avg_loss_backward),

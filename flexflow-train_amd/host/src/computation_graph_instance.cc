@@ -298,7 +298,10 @@ ComputationGraphInstance create_computation_graph_instance(
       p.own_scratch = !layer.weights.empty();
     } else if (auto const *a = std::get_if<MultiHeadAttentionAttrs>(&oa)) {
       ffk_mha_desc_t d = mha_desc(*a, shape_of(layer.inputs[0]), shape_of(layer.inputs[1]), shape_of(layer.inputs[2]));
-      p.saved = saved_planner.take(ffk_mha_reserve_bytes(&d, dt(shape_of(layer.inputs[0]).data_type)));
+      int const type = dt(shape_of(layer.inputs[0]).data_type);
+      size_t const shared = ffk_mha_backward_workspace_bytes(&d, type);  // scratch of the backward, not kept per layer
+      p.saved = saved_planner.take(ffk_mha_reserve_bytes(&d, type) - shared);
+      if (p.bwd.has_backward) p.scratch_bytes = shared;
       // key == value but not the query: both gradients land in one tensor
       if (layer.inputs[1] == layer.inputs[2] && layer.inputs[0] != layer.inputs[1]) acc = true;
       if (layer.inputs[0] == layer.inputs[1] && layer.inputs[0] != layer.inputs[2]) acc = true;
@@ -898,7 +901,8 @@ ComputationGraphInstance create_computation_graph_instance(
         check_ffk(ffk_mha_forward(s.require_gpu(), type, &d, qp, kp, vp, w, y, reserve, reserve_bytes), "MultiHeadAttention forward");
       };
       b = [=](device_stream_t const &s) {
-        check_ffk(ffk_mha_backward(s.require_gpu(), type, &d, qp, dq, kp, dk, vp, dv, w, dw, dy, reserve, reserve_bytes, accumulate),
+        check_ffk(ffk_mha_backward_with_workspace(s.require_gpu(), type, &d, qp, dq, kp, dk, vp, dv, w, dw, dy, reserve, reserve_bytes,
+                                                  ws_bytes ? scratch : nullptr, ws_bytes, accumulate),
                   "MultiHeadAttention backward");
       };
     } else if (auto const *a = std::get_if<DropoutAttrs>(&oa)) {

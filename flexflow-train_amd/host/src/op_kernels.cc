@@ -135,7 +135,8 @@ std::optional<MHAPerDeviceState> init_kernel(DeviceType device_type, device_hand
                       nullptr, allocator};
   ffk_mha_desc_t d = make_desc(s);
   s.weightSize = ffk_mha_weight_elements(&d) * size_of_datatype(data_type);
-  s.reserveSpaceSize = ffk_mha_reserve_bytes(&d, dt(data_type));
+  // what forward leaves for backward: a state lives as long as its operator, the backward's scratch would too
+  s.reserveSpaceSize = ffk_mha_reserve_bytes(&d, dt(data_type)) - ffk_mha_backward_workspace_bytes(&d, dt(data_type));
   s.reserveSpace = allocator.allocate(s.reserveSpaceSize);
   return s;
 }

@@ -1375,6 +1375,57 @@ static void gpu_tests() {
     }
   });
 
+  run("fp32 attention layers of a graph share the scratch of their backward; an operator's state holds none", [&] {
+    struct Counting : IAllocator {
+      Allocator inner = create_local_cuda_memory_allocator();
+      size_t bytes = 0;
+      void *allocate(size_t n) override { bytes += n; return inner.allocate(n); }
+      void deallocate(void *p) override { inner.deallocate(p); }
+      DeviceType get_allocation_device_type() const override { return DeviceType::GPU; }
+    };
+    int const B = 2, S = 512, E = 64, H = 8, D = 32;
+    ffk_mha_desc_t const d{B, H, E, E, E, D, D, D, E, S, S, 1.0f, 0};
+    size_t const scratch = ffk_mha_backward_workspace_bytes(&d, FFK_FLOAT), reserve = ffk_mha_reserve_bytes(&d, FFK_FLOAT);
+    CHECK(scratch == (size_t)B * H * S * S * 4);
+    device_id_t dev = make_device_id_t_from_idx(0, DeviceType::GPU);
+    auto label = random_vec((size_t)B * S * E, 701);
+    auto LABEL = device_accessor(gpu, shape({B, S, E}, DataType::FLOAT), label);
+    std::vector<size_t> bytes;
+    for (int layers = 1; layers <= 3; layers++) {
+      auto counting = std::make_shared<Counting>();
+      Allocator alloc(counting);
+      ComputationGraphBuilder cgb;
+      tensor_guid_t const x = cgb.create_input(shape({B, S, E}, DataType::FLOAT), CreateGrad::YES);
+      tensor_guid_t t = x;
+      for (int l = 0; l < layers; l++) t = cgb.multihead_attention(t, t, t, E, H, D, D, 0.0f, false);
+      ComputationGraphInstance inst = create_computation_graph_instance(
+          cgb.computation_graph, OptimizerAttrs{SGDOptimizerAttrs{0.05, 0.0, false, 0.0}},
+          LossConfig{NonconfigurableLossAttrs{LossFunction::MEAN_SQUARED_ERROR_AVG_REDUCE}, LABEL, t}, {}, alloc,
+          ProfilingSettings{0, 0}, handle, dev);
+      bytes.push_back(counting->bytes);
+      unsigned seed = 710;
+      for (size_t g = 0; g < cgb.computation_graph.tensors.size(); g++) {
+        auto const &src = cgb.computation_graph.layers.at(cgb.computation_graph.tensors[g].source.raw);
+        tensor_guid_t const guid{(int)g};
+        if (!std::holds_alternative<WeightAttrs>(src.attrs.op_attrs) && !(guid == x)) continue;
+        TensorShape const ts = cgb.computation_graph.tensors[g].shape;
+        copy_accessor_data_to_l_from_r(inst.get_tensor_accessor(guid),
+                                       device_accessor(gpu, ts, random_vec((size_t)get_num_elements(ts.dims), seed++, -0.2f, 0.2f)));
+      }
+      perform_all_passes_for_computation_graph_instance(inst, ProfilingSettings{0, 0}, handle, dev);
+      auto const dx = to_host(*inst.get_gradient_accessor(x));
+      CHECK(contains_non_zero(dx));
+      for (float v : dx) CHECK(std::isfinite(v));
+    }
+    // a layer more: its output and its weight with their gradients, and what its forward keeps
+    size_t const layer = 2 * (size_t)B * S * E * 4 + 2 * ffk_mha_weight_elements(&d) * 4 + reserve - scratch;
+    for (int i = 0; i < 2; i++) CHECK(bytes[i + 1] - bytes[i] <= layer + 8 * 256);
+    CHECK(bytes[0] >= layer + scratch);
+    auto state = Kernels::MultiHeadAttention::init_kernel(DeviceType::GPU, handle, gpu, B, H, E, E, E, D, D, D, E, S, S, false);
+    CHECK(state->reserveSpaceSize == reserve - scratch);
+    Kernels::MultiHeadAttention::cleanup_kernel(DeviceType::GPU, gpu, state);
+  });
+
   // Token embedding -> encoder layer -> vocabulary projection -> softmax -> sparse cross entropy:
   // the shape of the reference's BERT builder (lib/models/src/models/bert/bert.cc) at toy size.
   // Two instances, one created with one kernel per operator: the planner's fusions must not change

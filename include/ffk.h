@@ -639,8 +639,12 @@ int ffk_attention_backward(ffk_stream_t stream, int dtype,
  *   follows from the descriptor alone, so backward needs the descriptor forward
  *   had and nothing else.  For FLOAT the size asked for includes up to 512 MB
  *   behind that, for shapes where backward makes use of it: it keeps dS there,
- *   so that it is computed once.  A reserve space without this part is taken as
- *   well.
+ *   so that it is computed once.  This part (ffk_mha_backward_workspace_bytes of
+ *   it, 0: none) is scratch of backward alone, and a reserve space without it is
+ *   taken as well: a caller that holds the reserve spaces of many layers leaves
+ *   it out of them, and lends ffk_mha_backward_with_workspace memory that the
+ *   layers share (workspace: 16-byte aligned; NULL, less, or unaligned is taken
+ *   too, then as far as it goes).
  * backward: query_grad/key_grad/value_grad are overwritten unless accumulate
  *   (cudnnMultiHeadAttnBackwardData stores them);
  *   key_grad/value_grad may be NULL when key/value alias query (their
@@ -675,6 +679,16 @@ int ffk_mha_backward(ffk_stream_t stream, int dtype, ffk_mha_desc_t const *desc,
                      void const *weight, void *weight_grad,
                      void const *output_grad, void *reserve,
                      size_t reserve_bytes, int accumulate);
+size_t ffk_mha_backward_workspace_bytes(ffk_mha_desc_t const *desc, int dtype);
+int ffk_mha_backward_with_workspace(ffk_stream_t stream, int dtype,
+                                    ffk_mha_desc_t const *desc, void const *query,
+                                    void *query_grad, void const *key,
+                                    void *key_grad, void const *value,
+                                    void *value_grad, void const *weight,
+                                    void *weight_grad, void const *output_grad,
+                                    void *reserve, size_t reserve_bytes,
+                                    void *workspace, size_t workspace_bytes,
+                                    int accumulate);
 
 /* ------------------------------------------------------------------------ */
 /* One transformer encoder layer, forward and backward, sequenced over the

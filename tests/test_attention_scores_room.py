@@ -26,6 +26,8 @@ def test_room_for_scores_is_asked_for_where_it_is_used(ffk, B, H, Sq, Skv, pairs
     desc = ffk.mha_desc(B, H, E, E, E, D, D, D, E, Sq, Skv)
     asked = ffk.lib().ffk_mha_reserve_bytes(ctypes.byref(desc), ffk.FLOAT) - kept(B, H, E, D, Sq, Skv)
     assert asked == pairs * Sq * ((Skv + 31) // 32 * 32) * 4
+    assert ffk.lib().ffk_mha_backward_workspace_bytes(ctypes.byref(desc), ffk.FLOAT) == asked
+    assert ffk.lib().ffk_mha_backward_workspace_bytes(ctypes.byref(desc), ffk.BF16) == 0
     # in parts: two workgroups of 128 rows a CU, in half a GB
     most = (512 << 20) // (Sq * ((Skv + 31) // 32 * 32) * 4)
     assert pairs == (B * H if most >= B * H else most if most * (-(-min(Sq, Skv) // 128)) >= 512 else 0)

@@ -55,3 +55,23 @@ def test_backward_with_room_for_half_of_the_heads(ffk):
     want = backward(ffk, desc, x, x, w, dout, full)
     for a, b in zip(backward(ffk, desc, x, x, w, dout, full - scores // 2), want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("D,causal", [(64, True), (256, False)])
+def test_backward_with_room_that_layers_share(ffk, D, causal):
+    """dS in memory of its own: the bits of dS behind what is kept; lent unaligned, the bits without any."""
+    B, H, S, E = 2, 3, 97, 64
+    print("mha fp32, shared workspace", D, flush=True)
+    desc = ffk.mha_desc(B, H, E, E, E, D, D, D, E, S, S, D ** -0.5, causal)
+    gen = torch.Generator(device="cuda").manual_seed(D)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)  # noqa: E731
+    x, w, dout = mk(B, S, E), mk(ffk.lib().ffk_mha_weight_elements(desc)) * 0.2, mk(B, S, E)
+    reserve, ws = ffk.mha_reserve(desc, ffk.FLOAT, backward_scratch=False), ffk.mha_backward_workspace(desc, ffk.FLOAT)
+    full = ffk.mha_reserve(desc, ffk.FLOAT).numel()
+    assert reserve.numel() + ws.numel() == full and ws.numel() == 4 * B * H * S * 128
+    ffk.mha_forward(desc, x, x, x, w, reserve)
+    for lent, same_as in ((ws, full), (ws[4:], reserve.numel())):
+        dx, dw = torch.empty_like(x), torch.zeros_like(w)
+        ffk.mha_backward(desc, x, dx, x, None, x, None, w, dw, dout, reserve, ffk.MHA_OVERWRITE_WEIGHT_GRAD, workspace=lent)
+        for a, b in zip((dx, dw), backward(ffk, desc, x, x, w, dout, same_as)):
+            assert torch.equal(a, b)
