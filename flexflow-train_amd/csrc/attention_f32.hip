@@ -48,7 +48,7 @@ struct AttnF32Params {
   // for dQ's (nullptr: it does not): [pairs][Sq][ds_ld], rows of whole tiles of 32 keys.
   int pair0, pairs;
   float *ds;
-  int64_t ds_ld;
+  int ds_ld;
 };
 
 template <int DP>
@@ -424,13 +424,19 @@ __global__ __launch_bounds__(256) void attn_f32_delta_kernel(AttnF32Params p) {
 }
 
 // A 32 x 32 tile of dS to p.ds: rows = queries from qt0 on, column = this lane's key (32 lanes write 128 bytes of a row).
+// The descriptor of a pair's dS drops rows that do not exist (of up to 96 past the last, f32_pairs_at_a_time), and
+// a row is a scalar multiple away from one offset, formed anew for each tile: no register more than without dS.  (With an
+// address and a guard for each row, 48 registers, the kernels spilled at head size 128 and in the form for 132 to 252, and two
+// waves ran on a SIMD at 32 instead of three; whole backward 1.5 to 5% longer by head size, more for the guards than for the
+// spills, and with 6 x 32 heads x 333 of 20 1% longer than where dS is computed twice.)
 __device__ __forceinline__ void save_scores(AttnF32Params const &p, int pair, int qt0, int key, int h32, float const (&e)[16]) {
-  float *const to = p.ds + (int64_t)pair * p.Sq * p.ds_ld + (int64_t)qt0 * p.ds_ld;
-  int const left = p.Sq - qt0;  // rows that exist
+  unsigned const step = (unsigned)p.ds_ld * 4u;  // bytes; a pair has 512 MB of them at most
+  __amdgpu_buffer_rsrc_t const rsrc = __builtin_amdgcn_make_buffer_rsrc(p.ds + (int64_t)pair * p.Sq * p.ds_ld, 0, p.Sq * (int)step, 0x00020000);
+  unsigned off = (unsigned)(qt0 + 4 * h32) * step + 4u * key;
+  asm("" : "+v"(off));  // keeps the sixteen offsets of a tile from being kept instead of this one
 #pragma unroll
   for (int r = 0; r < 16; r++) {
-    int const ql = 8 * (r >> 2) + 4 * h32 + (r & 3);
-    if (ql < left) to[ql * p.ds_ld + key] = e[r];
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, e[r]), rsrc, off + (8 * (r >> 2) + (r & 3)) * step, 0, 0);
   }
 }
 
@@ -1156,6 +1162,7 @@ constexpr size_t kMostScores = (size_t)512 << 20;
 static int64_t f32_scores_row(int64_t seq_kv) { return ceil_div(seq_kv, 32) * 32; }
 static int64_t f32_pairs_at_a_time(int64_t pairs, int64_t seq_q, int64_t seq_kv, size_t bytes) {
   if (pairs <= 0 || seq_q <= 0 || seq_kv <= 0 || seq_q >= (1 << 30) || seq_kv >= (1 << 30)) return 0;
+  if ((seq_q + 96) * f32_scores_row(seq_kv) * (int64_t)sizeof(float) > (int64_t)1 << 32) return 0;  // 32-bit offsets (save_scores)
   int64_t const most = (int64_t)(std::min(bytes, kMostScores) / ((size_t)seq_q * f32_scores_row(seq_kv) * sizeof(float)));
   if (most >= pairs) return pairs;
   return most * ceil_div(std::min(seq_q, seq_kv), 128) >= 2 * kNumCU ? most : 0;
@@ -1194,7 +1201,7 @@ static void launch_f32_backward(hipStream_t st, AttnF32Params const &p, int64_t 
   if (int64_t const at_a_time = f32_pairs_at_a_time(heads, p.Sq, p.Skv, scratch_bytes); scratch != nullptr && at_a_time > 0) {
     AttnF32Params q = p;
     q.ds = static_cast<float *>(scratch);
-    q.ds_ld = f32_scores_row(p.Skv);
+    q.ds_ld = (int)f32_scores_row(p.Skv);
     for (q.pair0 = 0; q.pair0 < heads; q.pair0 += q.pairs) {
       q.pairs = (int)std::min<int64_t>(at_a_time, heads - q.pair0);
       launch_dkdv(q, std::true_type{});

@@ -20,6 +20,7 @@ def kept(B, H, E, D, Sq, Skv):
     (4, 8, 2500, 2500, 0), (6, 32, 2200, 2200, 0), (4, 32, 4096, 4096, 0), (1, 8, 5000, 5000, 0),
     (64, 16, 4096, 64, 512), (64, 16, 5000, 60, 0),             # one workgroup a pair
     (1, 1, 20000, 20000, 0),                                    # not even one pair fits
+    (1, 1, 1, 1 << 23, 1), (1, 1, 1, 1 << 24, 0), (1, 1, 10, 9 << 20, 1), (1, 1, 10, 11 << 20, 0),  # a tile's rows past 4 GB
 ])
 def test_room_for_scores_is_asked_for_where_it_is_used(ffk, B, H, Sq, Skv, pairs):
     E, D = 64, 32
@@ -30,4 +31,6 @@ def test_room_for_scores_is_asked_for_where_it_is_used(ffk, B, H, Sq, Skv, pairs
     assert ffk.lib().ffk_mha_backward_workspace_bytes(ctypes.byref(desc), ffk.BF16) == 0
     # in parts: two workgroups of 128 rows a CU, in half a GB
     most = (512 << 20) // (Sq * ((Skv + 31) // 32 * 32) * 4)
+    if (Sq + 96) * ((Skv + 31) // 32 * 32) * 4 > 1 << 32:  # offsets of 32 bits
+        most = 0
     assert pairs == (B * H if most >= B * H else most if most * (-(-min(Sq, Skv) // 128)) >= 512 else 0)
