@@ -1,5 +1,7 @@
 """fp32 MultiHeadAttention backward with room for dS in its reserve space (dQ is then one product of it), with room for a
 part of the heads at a time, and without: the same gradients, from reserve space that holds NaN where nothing was written."""
+import ctypes
+
 import pytest
 import torch
 
@@ -35,7 +37,7 @@ def test_backward_with_and_without_room_for_scores(ffk, D, Dv, causal):
         full = ffk.mha_reserve(desc, ffk.FLOAT).numel()
         scores = 4 * B * H * Sq * ((Sk + 31) // 32 * 32)
         want = backward(ffk, desc, x, kv, w, dout, full - scores)
-        for room in (full, full - 16):  # the second is room for all heads but one
+        for room in (full, full - 16):  # the second: a part too small for a launch of its own, as without room
             for name, a, b in zip(("dx", "dk", "dv", "dw"), backward(ffk, desc, x, kv, w, dout, room), want):
                 # two orders of the same fp32 sums
                 assert float((a - b).double().norm() / b.double().norm()) <= 8 * 2.0 ** -24 * max(Sq, Sk) ** 0.5, (name, room)
@@ -54,6 +56,23 @@ def test_backward_with_room_for_half_of_the_heads(ffk):
     full, scores = ffk.mha_reserve(desc, ffk.FLOAT).numel(), 4 * B * H * S * S
     want = backward(ffk, desc, x, x, w, dout, full)
     for a, b in zip(backward(ffk, desc, x, x, w, dout, full - scores // 2), want):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("D", [32, 64, 80, 128, 132, 256])
+@pytest.mark.parametrize("causal", [False, True])
+def test_backward_with_room_for_a_part_of_the_heads(ffk, D, causal):
+    """700 heads of 128 or 121 rows, 520 at a time and then the 180 left, whose products of dS are shared out among more workgroups."""
+    B, H, S, E = 10, 70, 128 if D > 128 else 121, 16
+    print("mha fp32, 520 and 180 of 700 heads", D, causal, flush=True)
+    desc = ffk.mha_desc(B, H, E, E, E, D, D, D, E, S, S, D ** -0.5, causal)
+    gen = torch.Generator(device="cuda").manual_seed(D)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)  # noqa: E731
+    x, w, dout = mk(B, S, E), mk(ffk.lib().ffk_mha_weight_elements(desc)) * 0.2, mk(B, S, E)
+    full, one = ffk.mha_reserve(desc, ffk.FLOAT).numel(), 4 * S * 128
+    assert ffk.lib().ffk_mha_backward_workspace_bytes(ctypes.byref(desc), ffk.FLOAT) == 700 * one
+    want = backward(ffk, desc, x, x, w, dout, full)
+    for a, b in zip(backward(ffk, desc, x, x, w, dout, full - 179 * one - 16), want):
         assert torch.equal(a, b)
 
 

@@ -32,6 +32,11 @@ def test_column_sums_beside_the_weight_gradients(ffk, batch, seq, d_model, heads
     finally:
         ffk.set_option(ffk.OPTION_LAYER_UNFUSED, 0)
     for k in alone:
+        assert np.abs(alone[k]).max() > 0
         if k not in ("attn_weight", "w1", "w2"):
-            assert np.abs(alone[k]).max() > 0
             assert np.array_equal(along[k], alone[k]), k
+        else:
+            # the products of that launch, on tiles that may add up in another order: two roundings to bf16, of at most
+            # 2^-9 of each element, and the fp32 sums' own differences far below that
+            a, b = along[k].astype(np.float64), alone[k].astype(np.float64)
+            assert np.linalg.norm(a - b) <= 2.0 ** -8 * np.linalg.norm(b), k

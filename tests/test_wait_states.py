@@ -3,6 +3,7 @@ compiler neither sees what they do nor puts wait states in front of them.
 
   * direct loads (csrc/lds_dma.h): five wait states between a vector instruction that writes a scalar register and a
     vector-memory instruction that reads it; one between a write of M0 and the direct load behind it
+  * matrix instructions with the accumulator in place (csrc/gemm_bf16.h): see the second test
 """
 import functools
 import glob
@@ -82,21 +83,25 @@ class Code:
         return found
 
 
-def kernels(lib, tmp_path, wanted):
-    """(name, disassembly) of the library's kernels whose text `wanted` finds something in."""
-    shutil.copy(lib, tmp_path / "lib.so")
-    subprocess.run([LLVM + "llvm-objdump", "--offloading", "lib.so"], cwd=tmp_path, check=True, capture_output=True)
-    for path in sorted(glob.glob(str(tmp_path / "lib.so.*gfx950"))):
+def disassembled(lib, where):
+    """(name, instructions) of the library's kernels that have direct loads."""
+    shutil.copy(lib, where / "lib.so")
+    subprocess.run([LLVM + "llvm-objdump", "--offloading", "lib.so"], cwd=where, check=True, capture_output=True)
+    for path in sorted(glob.glob(str(where / "lib.so.*gfx950"))):
         text = subprocess.run([LLVM + "llvm-objdump", "-d", "--no-show-raw-insn", path], check=True, capture_output=True, text=True).stdout
         for name, body in KERNEL.findall(text):
-            if wanted(body):
-                yield name, body
+            if " lds" in body:
+                yield name, Code(body)
 
 
-def test_direct_loads_read_settled_scalars(ffk, tmp_path):
+@pytest.fixture(scope="module")
+def kernels(ffk, tmp_path_factory):
+    return list(disassembled(ffk.LIB_PATH, tmp_path_factory.mktemp("library")))
+
+
+def test_direct_loads_read_settled_scalars(kernels):
     checked, wrong = 0, {}
-    for name, body in kernels(ffk.LIB_PATH, tmp_path, lambda b: " lds" in b):
-        code = Code(body)
+    for name, code in kernels:
         for i, op in enumerate(code.op):
             if not op.startswith("buffer_load") or not code.args[i][-1].endswith("lds"):
                 continue
@@ -109,3 +114,42 @@ def test_direct_loads_read_settled_scalars(ffk, tmp_path):
     assert checked > 1000
     assert not wrong, "%d of %d loads, in %d kernels, for instance %s" % (
         sum(map(len, wrong.values())), checked, len(wrong), [(k, v[0]) for k, v in wrong.items()][:4])
+
+
+def test_accumulators_written_out_are_settled(kernels):
+    """csrc/gemm_bf16.h's matrix instructions with the accumulator in place (v_mfma_f32_16x16x32_bf16, four passes): eight wait
+    states before anything but another of them touches a result, two behind a vector instruction that writes an operand.
+    Twice as many are asked for here, and kept."""
+    op_name, settles, operands = "v_mfma_f32_16x16x32_bf16", 16, 4
+    checked, wrong = 0, []
+    for name, code in kernels:
+        if not any(op == op_name and args[0].startswith("a[") for op, args in zip(code.op, code.args)):
+            continue
+        used = [frozenset().union(*map(registers, args)) for args in code.args]
+        results = {i: registers(code.args[i][0]) for i, op in enumerate(code.op) if op == op_name}
+        touches = frozenset().union(*results.values())
+        for i, op in enumerate(code.op):
+            matrix = op == op_name
+            if matrix:
+                # what its operands or its accumulator were written by
+                wanted, states = frozenset().union(*(registers(a) for a in code.args[i][1:4])), operands
+            elif not op.startswith("s_") and used[i] & touches:
+                wanted, states = used[i] & touches, settles
+            else:
+                continue
+            checked += 1
+            work, seen = [(p, 0) for p in code.before[i]], set()
+            while work:
+                at, passed = work.pop()
+                if (at, passed) in seen or passed >= states:
+                    continue
+                seen.add((at, passed))
+                if matrix:
+                    bad = code.op[at].startswith("v_") and not code.op[at].startswith("v_mfma") and registers(code.args[at][0]) & wanted
+                else:
+                    bad = at in results and results[at] & wanted
+                if bad:
+                    wrong.append((name, code.op[at], code.args[at], op, code.args[i], passed))
+                work += [(p, passed + code.wait_states(at)) for p in code.before[at]]
+    assert checked > 10000
+    assert not wrong, "%d of %d, for instance %s" % (len(wrong), checked, wrong[:3])
