@@ -247,13 +247,13 @@ def time_dominant_kernel(ffk, torch, cfg, iters=50, calibration_copy=False):
 
 
 def measure_mfma_loop(ffk, torch):
-    """The library's probe: every SIMD issues bf16 32x32x16 matrix instructions back to back from
+    """The library's probe: every SIMD issues bf16 16x16x32 matrix instructions back to back from
     registers.  What it reaches is the ceiling for a GEMM on this card at the clock it sustains."""
     out = torch.empty((256 * 256,), device="cuda")
     flops = ffk.probe_mfma_bf16(2000, out)
     us = event_timer(ffk)(lambda: ffk.probe_mfma_bf16(2000, out), 20)
     return {"TFLOP/s": flops / us / 1e6, "vendor_peak_TFLOP/s": MFMA_BF16_PEAK_TFLOPS,
-            "what": "256 CUs x 4 waves, 32000 back-to-back 32x32x16 bf16 MFMAs each on random operands in registers"}
+            "what": "256 CUs x 4 waves, 64000 back-to-back 16x16x32 bf16 MFMAs each on random operands in registers"}
 
 
 def measure_device_copy(ffk, torch):

@@ -191,7 +191,7 @@ struct GemmGroupArgs {
   // Column reductions that ride along: workgroups from first_sum on.  They read what earlier launches left, and
   // run where the tiles leave CUs idle; a launch of their own is 3 to 7 us of latency (encoder layers forward and
   // backward, batch x tokens x width: 8 x 512 x 1024 511 -> 504 us, 7 x 197 x 768 247.5 -> 242, 2 x 48 x 128 69 -> 67
-  // replayed from a graph, 88 -> 80 launched one by one).
+  // replayed from a graph, within noise launched one by one).
   int first_sum;
   ColreduceBatch sums;
 };
@@ -1296,6 +1296,10 @@ inline bool edge_operands_ok(int64_t lda, int64_t ldb) { return 2 * 256 * std::m
 // the worst, of 2048-long reductions and of 257 to 512 tiles of 64 x 64: 1149 x 768 over 2048 12.7 -> 10.5 us, 828 x
 // 1536 over 2560 21.5 -> 18.1).  It ranks the tiles and does not predict: launch to launch they took 0.8 to 2.1 times
 // its figure (median 1.3; 2-3 us of each is the launch), the short and the transposed ones most.
+// The fit is of the 256-wide tiles on 32x32x16 matrix instructions; on 16x16x32 they take some 8% less.  Of 240 other
+// products drawn from M 64-5000, N and K 128-4096 on the present kernels, the tile picked takes 2.4% longer than the best
+// one, and of the 52 with 4 M outputs and reductions of 1024 and more 5.3%: never where the wide tile is the best (13
+// products), most where 256 x 128 tiles would be and gemm_takes_256x128 does not hold (1432 x 3152 over 3528 72 us, 52 on those).
 //  - a round over the chip costs its 64-deep k-tiles times what one takes with so many CUs busy
 //    (memory and LDS are shared, the clock too), and a constant of filling, draining and storing
 //  - 32 x 32, four waves that split the reduction, two workgroups a CU

@@ -1,13 +1,14 @@
 // Measurement aid: what the matrix pipes of the whole chip deliver when nothing else limits them.
-// One workgroup per CU, one wave per SIMD; every wave issues 32x32x16 bf16 MFMAs back to back on
-// four independent accumulators, operands in registers, no memory access inside the loop.  The rate
+// One workgroup per CU, one wave per SIMD; every wave issues 16x16x32 bf16 MFMAs back to back on
+// sixteen independent accumulators, operands in registers, no memory access inside the loop: the instruction of the
+// GEMM's 256-wide tiles, which takes less power than 32x32x16 and so leaves the chip a higher clock.  The rate
 // measured this way is the ceiling a GEMM kernel can approach on this card (its sustained clock
 // under matrix load included), next to the vendor's 2.5 PFLOP/s figure for a fixed clock.
 #include "ffk_common.h"
 
 namespace ffk {
 
-constexpr int kProbeMfmasPerIteration = 16;
+constexpr int kProbeMfmasPerIteration = 32, kProbeAccumulators = 16;
 
 __global__ __launch_bounds__(256) void mfma_probe_kernel(float *__restrict__ out, int iterations, uint32_t seed) {
   // operand bits from a hash of (lane, seed): values in [-1, 1), never NaN or infinite, so the
@@ -21,23 +22,30 @@ __global__ __launch_bounds__(256) void mfma_probe_kernel(float *__restrict__ out
     h = h * 1664525u + 1013904223u;
     b[i] = (__bf16)((float)(int)(h >> 8 & 0xffff) * (1.0f / 32768.0f) - 1.0f);
   }
-  f32x16 acc[4];
+  f32x4 acc[kProbeAccumulators];
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
+  for (int j = 0; j < kProbeAccumulators; j++) {
 #pragma unroll
-    for (int i = 0; i < 16; i++) acc[j][i] = 0.0f;
+    for (int i = 0; i < 4; i++) acc[j][i] = 0.0f;
   }
+  // Written as instructions, in place: the compiler moves accumulators about between them.  It does not see what time
+  // operands and results take, hence the wait states on either side of the loop.
+  asm volatile("s_nop 15" : "+v"(a), "+v"(b));
+#pragma unroll
+  for (int j = 0; j < kProbeAccumulators; j++) asm volatile("s_nop 15" : "+v"(acc[j]));
   for (int it = 0; it < iterations; it++) {
 #pragma unroll
     for (int j = 0; j < kProbeMfmasPerIteration; j++) {
-      acc[j % 4] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[j % 4], 0, 0, 0);
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[j % kProbeAccumulators]) : "v"(a), "v"(b));
     }
   }
+#pragma unroll
+  for (int j = 0; j < kProbeAccumulators; j++) asm volatile("s_nop 15" : "+v"(acc[j]));
   float s = 0.0f;
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
+  for (int j = 0; j < kProbeAccumulators; j++) {
 #pragma unroll
-    for (int i = 0; i < 16; i++) s += acc[j][i];
+    for (int i = 0; i < 4; i++) s += acc[j][i];
   }
   out[(size_t)blockIdx.x * 256 + threadIdx.x] = s;
 }
@@ -53,7 +61,7 @@ extern "C" int ffk_probe_mfma_bf16(ffk_stream_t stream, int iterations, uint32_t
               "probe_mfma_bf16: out must hold %d floats", kNumCU * 256);
   mfma_probe_kernel<<<kNumCU, 256, 0, as_stream(stream)>>>(out, iterations, seed);
   FFK_CHECK_LAUNCH();
-  // per wave and iteration: 16 MFMAs of 32 x 32 x 16 multiply-adds
-  if (flops) *flops = (double)kNumCU * 4.0 * iterations * kProbeMfmasPerIteration * (2.0 * 32 * 32 * 16);
+  // per wave and iteration: 32 MFMAs of 16 x 16 x 32 multiply-adds
+  if (flops) *flops = (double)kNumCU * 4.0 * iterations * kProbeMfmasPerIteration * (2.0 * 16 * 16 * 32);
   return FFK_OK;
 }

@@ -122,7 +122,7 @@ int ffk_event_synchronize(ffk_event_t ev);
 int ffk_event_elapsed_ms(ffk_event_t start, ffk_event_t stop, float *ms);
 
 /* Measurement aid; no counterpart in the reference.  One launch in which
- * every SIMD of the chip issues `iterations` x 16 bf16 32x32x16 matrix
+ * every SIMD of the chip issues `iterations` x 32 bf16 16x16x32 matrix
  * instructions back to back from registers (no memory traffic): timed by the
  * caller, *flops / time is the matrix rate this card sustains, the ceiling a
  * GEMM kernel here can approach (the vendor's 2.5 PFLOP/s assumes a clock the
